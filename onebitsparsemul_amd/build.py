@@ -26,11 +26,17 @@ def _run(cmd):
 
 
 def build_library():
-    objs = []
-    for src in ("onebit_kernels.hip", "onebit_capi.hip", "onebit_diag.hip"):
+    # one compiler per source, side by side
+    objs, compilers = [], []
+    for src in ("onebit_kernels.hip", "onebit_format.hip", "onebit_capi.hip", "onebit_diag.hip"):
         obj = os.path.join(CSRC, src.replace(".hip", ".o"))
-        _run([HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, src), "-o", obj])
+        cmd = [HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
+        print("+", " ".join(cmd), flush=True)
+        compilers.append((cmd, subprocess.Popen(cmd)))
         objs.append(obj)
+    failed = [cmd for cmd, compiler in compilers if compiler.wait() != 0]
+    if failed:
+        raise subprocess.CalledProcessError(1, failed[0])
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs])
     if os.path.exists(STATIC_LIB):
         os.remove(STATIC_LIB)
