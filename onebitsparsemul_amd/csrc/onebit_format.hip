@@ -6,6 +6,19 @@
 
 namespace onebit {
 
+// Position of a workgroup in a two-dimensional list that is walked in strips: `along` runs over [0, length), `across` over
+// the strips' widths. Workgroup b runs on XCD b % 8, so each XCD is given a contiguous range of the list: strip after
+// strip, inside a strip `along` slowest, its `width` workgroups side by side. The grid holds whole strips.
+struct StripPosition {
+  int along, across;
+};
+__device__ __forceinline__ StripPosition strip_position(int width, int length) {
+  const int per = gridDim.x / 8, rem = gridDim.x % 8, xcd = blockIdx.x % 8;
+  const int v = xcd * per + (xcd < rem ? xcd : rem) + blockIdx.x / 8;
+  const int strip = v / (width * length), w = v % (width * length);
+  return StripPosition{w / width, strip * width + w % width};
+}
+
 // =====================================================================================================
 // 32 x 32 bit transpose across each half of a wavefront: on entry bit b of lane 32 h + r is element (r, b), on return
 // element (b, r). Five exchange steps (xor 16, 8, 4, 2, 1), each one lane exchange, one rotate, one bit select; the
@@ -65,12 +78,9 @@ __global__ __launch_bounds__(64 * kPreparePairs) void prepare_kernel(const uint8
                                                                      uint8_t* __restrict__ prep, int m, int k,
                                                                      int kc_total, int layout) {
   const int lane = threadIdx.x & 63;
-  // workgroup b runs on XCD b % 8: each XCD takes a contiguous range of the list ordered row groups fastest
-  const int per = gridDim.x / 8, rem = gridDim.x % 8, xcd = blockIdx.x % 8;
-  const int v = xcd * per + (xcd < rem ? xcd : rem) + blockIdx.x / 8;
-  const int strip = v / (kPrepareStrip * kc_total), w = v % (kPrepareStrip * kc_total);
-  const int kc = w / kPrepareStrip;
-  const int pair = (strip * kPrepareStrip + w % kPrepareStrip) * kPreparePairs + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const StripPosition at = strip_position(kPrepareStrip, kc_total);
+  const int kc = at.along;
+  const int pair = at.across * kPreparePairs + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (pair >= m / 64) return;  // m % 64 == 0: every row of a pair exists
   const int i = lane & 31, ga = lane >> 5;
   const int ncols = k / 16;
@@ -147,79 +157,151 @@ __global__ __launch_bounds__(64 * kPreparePairs) void prepare_kernel(const uint8
 // pruned first), compression to kept values + nibbles (:126-159, including the fixed encodings of groups
 // with fewer or more than two non-zeros), sign quantisation (value > 0 -> 1, __init__.py:22-23), transposed
 // bit packing (__init__.py:25-34,142-143) and the metadata reorder (:21-48).
-// One wavefront = 64 consecutive rows x four metadata columns (64 dense K, one 128-byte line per row); the eight
-// sign bits of a row and column are gathered across the wavefront with ballots, so every store of `a` is 8 bytes
-// of 64 consecutive rows.
+//
+// One wavefront = 64 rows x 64 K. Lines of 128 bytes come in by asynchronous copies (eight lanes per row) and are
+// turned in LDS, after which lane r holds row r: sixteen groups of four. Everything that decides about a group is one bit
+// per value or per pair of values (which of two magnitudes is smaller, zero or not, the sign), so these bits are shifted
+// into slices of sixteen groups, two values per 32-bit register, and the rules are then evaluated once for all sixteen
+// groups with bitwise instructions. Slice bit 4 g + c belongs to group g of metadata column c: the four nibbles of a column
+// are then four bits apart, as in its word. About 32 vector instructions per group where comparing floats group by
+// group took about 110.
+// Bound: memory (2 m k bytes in, m k 3/16 out). The workgroups of an XCD walk in strips of sixteen row tiles, as in
+// prepare_kernel, so that the eight-byte pieces of a line of `a` meet in its L2. Row tiles per workgroup / workgroups of a
+// strip, us inside a HIP graph at 11008 x 4096: 2 / 8 20.2, 4 / 4 20.6, 8 / 2 21.9, 16 / 1 24.2. Against 64-row wavefronts
+// that read their own row's line lane by lane and compared floats: 4096 x 4096 26.2 -> 10.1 us, 11008 x 4096 68.4 -> 20.6
+// (98 MB: 4.8 TB/s, the rate of a 2 GiB copy), 28672 x 8192 316 -> 105.
 // =====================================================================================================
-__device__ __constant__ uint8_t kNibbleOfPattern[16] = {0xE, 0x8, 0x9, 0x4, 0xE, 0x8, 0x9, 0x4,
-                                                        0xE, 0xC, 0xD, 0x4, 0xE, 0xC, 0xD, 0x4};
+constexpr int kPackTiles = 4, kPackStrip = 4;  // row tiles (wavefronts) per workgroup, workgroups side by side in a strip
 
-__global__ __launch_bounds__(64) void pack_kernel(const _Float16* __restrict__ w, uint8_t* __restrict__ a,
-                                                  uint16_t* __restrict__ e, int m, int k, int prune, int layout) {
-  const int64_t r = (int64_t)blockIdx.y * 64 + threadIdx.x;  // m % 64 == 0: always a valid row
-  const int ncols = k / 16;
-  // four metadata columns (64 weights = 128 consecutive bytes of the lane's row) per wavefront: requests of whole
-  // 128-byte lines; the last group of a row may hold two columns only (k % 32 == 0)
-  const int c_first = blockIdx.x * 4;
-  const int c_count = ncols - c_first < 4 ? ncols - c_first : 4;
-  u32x4_t line[8];
+typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t packed_sub(uint32_t x, uint32_t y) {
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2_t, x) - __builtin_bit_cast(u16x2_t, y));
+}
+__device__ __forceinline__ uint32_t packed_add(uint32_t x, uint32_t y) {
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2_t, x) + __builtin_bit_cast(u16x2_t, y));
+}
+__device__ __forceinline__ uint32_t majority(uint32_t x, uint32_t y, uint32_t z) { return ((x ^ y) & (z ^ x)) ^ x; }
+
+__global__ __launch_bounds__(64 * kPackTiles) void pack_kernel(const _Float16* __restrict__ w, uint8_t* __restrict__ a,
+                                                               uint16_t* __restrict__ e, int m, int k, int prune,
+                                                               int layout, int k_tiles) {
+  __shared__ __attribute__((aligned(16))) char lds[kPackTiles * 8192];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const StripPosition at = strip_position(kPackStrip, k_tiles);
+  const int tile = at.across * kPackTiles + wave;
+  if (tile >= m / 64) return;  // m % 64 == 0: every row of a tile exists; wavefronts do not meet at barriers
+  const int64_t row0 = (int64_t)tile * 64;
+  const int ncols = k / 16, c_first = at.along * 4;
+  const int c_count = ncols - c_first < 4 ? ncols - c_first : 4;  // the last tile may hold two columns only (k % 32 == 0)
+
+  // ---- 64 rows x 128 bytes into LDS: copy i carries rows 8 i ... 8 i + 7; piece q of row r goes to position q ^ (r % 8)
+  char* const image = lds + wave * 8192;
+  {
+    const int piece = (lane & 7) ^ (lane >> 3);
+    const int from = piece < 2 * c_count ? piece : 0;  // past K: any valid address will do, the results are not stored
+    const char* src = reinterpret_cast<const char*>(w + (row0 + (lane >> 3)) * k + 16 * c_first) + 16 * from;
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
-    if (i < 2 * c_count) line[i] = reinterpret_cast<const u32x4_t*>(w + r * k + 16 * c_first)[i];
+    for (int i = 0; i < 8; ++i) lds_dma16(src + (size_t)i * 16 * k, lds_offset_of(image) + i * 1024);
+  }
+  wait_vmcnt<0>();
+  uint32_t d[32];  // dword 2 q: values 0 and 1 of group q, dword 2 q + 1: values 2 and 3
 #pragma unroll
-  for (int ci = 0; ci < 4; ++ci) {
-    if (ci >= c_count) break;  // wave-uniform
-    const int c = c_first + ci;                       // metadata column
-    u32x4_t raw[2] = {line[2 * ci], line[2 * ci + 1]};
-    _Float16 v[16];
-    __builtin_memcpy(v, raw, 32);
-    uint32_t word = 0, bits = 0;  // bits: bit t = kept value t of this metadata element is > 0
+  for (int q = 0; q < 8; ++q) {
+    const u32x4_t v = *reinterpret_cast<const u32x4_t*>(image + lane * 128 + ((q ^ (lane & 7)) << 4));
+    d[4 * q] = v.x; d[4 * q + 1] = v.y; d[4 * q + 2] = v.z; d[4 * q + 3] = v.w;
+  }
+
+  // ---- slices. less_ij: magnitude j < magnitude i (i < j), i.e. i outranks j; otherwise j outranks i (ties: the higher
+  // index). Low half | high half of a register: 02|13, 03|12, 01|23 for pairs, 0|1 and 2|3 for single values.
+  uint32_t less_02_13 = 0, less_03_12 = 0, less_01_23 = 0, nonzero_01 = 0, nonzero_23 = 0, nan_01 = 0, nan_23 = 0,
+           minus_01 = 0, minus_23 = 0;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      float x[4], mag[4];
+  for (int t = 0; t < 16; ++t) {
+    const int q = 4 * (t & 3) + (t >> 2);  // group t / 4 of column t % 4
+    const uint32_t d0 = d[2 * q], d1 = d[2 * q + 1];
+    const uint32_t m0 = d0 & 0x7FFF7FFFu, m1 = d1 & 0x7FFF7FFFu;  // magnitudes order like their bits
+    auto push = [](uint32_t& slice, uint32_t x) __attribute__((always_inline)) {  // bits 15 and 31 of x
+      slice = (x & 0x80008000u) | ((slice >> 1) & 0x7FFF7FFFu);
+    };
+    push(less_02_13, packed_sub(m1, m0));
+    push(less_03_12, packed_sub(__builtin_amdgcn_alignbit(m1, m1, 16), m0));
+    push(less_01_23, packed_sub(__builtin_amdgcn_perm(m1, m0, 0x07060302u), __builtin_amdgcn_perm(m1, m0, 0x05040100u)));
+    push(nonzero_01, packed_add(m0, 0x7FFF7FFFu));
+    push(nonzero_23, packed_add(m1, 0x7FFF7FFFu));
+    push(nan_01, packed_add(m0, 0x03FF03FFu));  // magnitude > infinity's bits 0x7C00
+    push(nan_23, packed_add(m1, 0x03FF03FFu));
+    push(minus_01, d0);
+    push(minus_23, d1);
+  }
+
+  // ---- the rules, on 16-bit slices (the upper halves of these registers hold other slices and are masked at the end)
+  const uint32_t nan0 = nan_01, nan1 = nan_01 >> 16, nan2 = nan_23, nan3 = nan_23 >> 16;
+  uint32_t keep0 = ~0u, keep1 = ~0u, keep2 = ~0u, keep3 = ~0u;
+  if (prune) {
+    // a comparison with NaN is false both ways
+    const uint32_t ok01 = ~(nan0 | nan1), ok02 = ~(nan0 | nan2), ok03 = ~(nan0 | nan3), ok12 = ~(nan1 | nan2),
+                   ok13 = ~(nan1 | nan3), ok23 = ~(nan2 | nan3);
+    const uint32_t l01 = less_01_23, l23 = less_01_23 >> 16, l02 = less_02_13, l13 = less_02_13 >> 16, l03 = less_03_12,
+                   l12 = less_03_12 >> 16;
+    // a value goes when two of the other three outrank it
+    keep0 = ~majority(~l01 & ok01, ~l02 & ok02, ~l03 & ok03);
+    keep1 = ~majority(l01 & ok01, ~l12 & ok12, ~l13 & ok13);
+    keep2 = ~majority(l02 & ok02, l12 & ok12, ~l23 & ok23);
+    keep3 = ~majority(l03 & ok03, l13 & ok13, l23 & ok23);
+  }
+  const uint32_t p0 = keep0 & nonzero_01, p1 = keep1 & (nonzero_01 >> 16), p2 = keep2 & nonzero_23,
+                 p3 = keep3 & (nonzero_23 >> 16);
+  const uint32_t plus0 = p0 & ~minus_01 & ~nan0, plus1 = p1 & ~(minus_01 >> 16) & ~nan1, plus2 = p2 & ~minus_23 & ~nan2,
+                 plus3 = p3 & ~(minus_23 >> 16) & ~nan3;
+  // Bits of the nibble idx0 | idx1 << 2 for the pattern of non-zeros (p0 p1 p2 p3). With p0 and p1 it names 0 and 1; with
+  // one of them, that one and 3 if p3, else 2; with neither, 2 and 3. (Which also gives the reference's fixed encodings
+  // of groups with other than two non-zeros.)
+  const uint32_t n0 = ~p0 & p1, n1 = ~(p0 | p1), n2 = ~(p0 ^ p1) | p3, n3 = ~(p0 & p1);
+  // signs of the two kept values, one bit per group: the first in the low half, the second in the high half
+  const uint32_t first = plus0 | (~p0 & (plus1 | (~p1 & plus2)));
+  const uint32_t second = (~n3 & plus1) | (n3 & ((n2 & plus3) | (~n2 & plus2)));
+
+  // ---- a: lane (half h, bit b) of the transposed slices holds rows 32 h ... 32 h + 31 of bit b, which is kept value
+  // 2 g + b / 16 of column c (b % 16 = 4 g + c)
+  const BitTranspose transpose(lane);
+  const uint32_t rows = transpose((first & 0xFFFFu) | (second << 16));
+  {
+    const int b = lane & 31, c = b & 3;
+    const int64_t column = 8 * (c_first + c) + 2 * ((b >> 2) & 3) + (b >> 4);
+    if (c < c_count) *reinterpret_cast<uint32_t*>(a + ((row0 + 32 * (lane >> 5) + column * m) >> 3)) = rows;
+  }
+
+  // ---- e: the words of the four columns
+  uint32_t word[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        x[i] = (float)v[4 * g + i];
-        mag[i] = x[i] < 0.f ? -x[i] : x[i];
-      }
-      int pattern = 0;
+  for (int c = 0; c < 4; ++c) {
+    const uint32_t b0 = n0 >> c, b1 = c < 1 ? n1 << 1 : n1 >> (c - 1), b2 = c < 2 ? n2 << (2 - c) : n2 >> (c - 2),
+                   b3 = c < 3 ? n3 << (3 - c) : n3;
+    word[c] = (b0 & 0x1111u) | (b1 & 0x2222u) | (b2 & 0x4444u) | (b3 & 0x8888u);
+  }
+  if (layout == 0 && (reinterpret_cast<uintptr_t>(e) & 3) == 0) {
+    // Rows r and r + 4 of one column share a dword, and the dwords of an even and the next odd column are neighbours: the
+    // lane of row r stores the even column's, the lane of row r + 4 the odd column's; 256 consecutive bytes per pair.
+    const bool upper = (lane >> 2) & 1;
+    uint32_t* const dst = reinterpret_cast<uint32_t*>(e) + row0 +
+                          ((((lane >> 1) & 1) << 5) | ((lane >> 3) << 2) | ((lane & 1) << 1) | ((lane >> 2) & 1));
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        bool keep = true;
-        if (prune) {
-          int beaten = 0;  // elements that outrank i: larger magnitude, or equal magnitude and higher index
-#pragma unroll
-          for (int j = 0; j < 4; ++j) beaten += (j != i) && (mag[j] > mag[i] || (mag[j] == mag[i] && j > i));
-          keep = beaten < 2;
-        }
-        if (!keep) x[i] = 0.f;
-        pattern |= (x[i] != 0.f) << i;
-      }
-      const int nib = kNibbleOfPattern[pattern];
-      const int i0 = nib & 3, i1 = nib >> 2;
-      word |= (uint32_t)nib << (4 * g);
-      float k0 = x[0], k1 = x[0];
-#pragma unroll
-      for (int i = 1; i < 4; ++i) {
-        if (i0 == i) k0 = x[i];
-        if (i1 == i) k1 = x[i];
-      }
-      bits |= (uint32_t)(k0 > 0.f) << (2 * g);
-      bits |= (uint32_t)(k1 > 0.f) << (2 * g + 1);
+    for (int c = 0; c < 4; c += 2) {
+      const uint32_t other = __builtin_amdgcn_ds_swizzle(upper ? word[c] : word[c + 1], (4 << 10) | 0x1F);
+      const uint32_t pair = upper ? other | (word[c + 1] << 16) : word[c] | (other << 16);
+      if (c < c_count) dst[(size_t)((c_first + c) >> 1) * m] = pair;
     }
-    int64_t off;
-    if (layout == 0) off = meta_offset_reference(r, c, m);
-    else if (layout == 1) off = meta_offset_cutlass(r, c, m);
-    else off = r * ncols + c;
-    e[off] = (uint16_t)word;
-    const int64_t row0 = (int64_t)blockIdx.y * 64;
+  } else {
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const uint64_t mask = __ballot((bits >> t) & 1u);  // bit l = row row0 + l, compressed column 8c + t
-      if (threadIdx.x == 0) {
-        const int64_t pos = row0 + (int64_t)(8 * c + t) * m;  // multiple of 64
-        *reinterpret_cast<uint64_t*>(a + (pos >> 3)) = mask;
-      }
+    for (int c = 0; c < 4; ++c) {
+      if (c >= c_count) break;  // wave-uniform
+      const int64_t r = row0 + lane;
+      const int64_t off = layout == 0   ? meta_offset_reference(r, c_first + c, m)
+                          : layout == 1 ? meta_offset_cutlass(r, c_first + c, m)
+                                        : r * ncols + c_first + c;
+      e[off] = (uint16_t)word[c];
     }
   }
 }
@@ -236,8 +318,11 @@ hipError_t launch_prepare(const void* a, const void* e, void* prep, int m, int k
 }
 
 hipError_t launch_pack(const void* w, void* a, void* e, int m, int k, int prune, int layout, hipStream_t stream) {
-  hipLaunchKernelGGL(pack_kernel, dim3((k / 16 + 3) / 4, m / 64), dim3(64), 0, stream, (const _Float16*)w, (uint8_t*)a,
-                     (uint16_t*)e, m, k, prune, layout);
+  const int k_tiles = (k / 16 + 3) / 4;
+  constexpr int kStripTiles = kPackTiles * kPackStrip;
+  const dim3 grid(k_tiles * kPackStrip * ((m / 64 + kStripTiles - 1) / kStripTiles));
+  hipLaunchKernelGGL(pack_kernel, grid, dim3(64 * kPackTiles), 0, stream, (const _Float16*)w, (uint8_t*)a, (uint16_t*)e,
+                     m, k, prune, layout, k_tiles);
   return hipGetLastError();
 }
 

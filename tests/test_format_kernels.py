@@ -58,3 +58,33 @@ def test_prepared_operand_bytes(m, k, a_shift, e_shift, layout):
     got = _native.prepare(a_gpu[a_shift:a_shift + count], e_gpu[e_shift:e_shift + count], m, k, layout)
     torch.cuda.synchronize()
     assert np.array_equal(got.cpu().numpy(), prepared_by_definition(a, e, m, k, layout))
+
+
+def stored_by_oracle(w, prune, layout):
+    """mask -> compress -> quantise -> pack of the dense weight w (float32 values), as the oracle does it."""
+    if prune:
+        w = np.where(oracle.mask_creator(w) != 0, w, 0).astype(np.float32)
+    sparse, meta = oracle.sparse_from_dense(w, layout)
+    return oracle.pack_binary(np.ascontiguousarray(oracle.binary_quant(sparse).T)), meta
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prune", [True, False])
+@pytest.mark.parametrize("m,k,layout", [
+    (64, 32, _native.META_REFERENCE),     # one row tile, half a K tile
+    (320, 96, _native.META_REFERENCE),    # more row tiles than a workgroup holds, a K tail of half a tile
+    (1088, 192, _native.META_REFERENCE),  # more than one strip of sixteen row tiles
+    (128, 160, _native.META_CUTLASS),
+])
+def test_packed_weight_bytes(m, k, layout, prune):
+    rng = np.random.default_rng(m + k)
+    # few distinct magnitudes (ties), zeros of both signs, the smallest half-precision number, infinities
+    values = np.array([0.0, -0.0, 1.0, -1.0, 0.5, -0.5, 2.0**-24, -2.0**-24, np.inf, -np.inf], dtype=np.float32)
+    w = rng.normal(0, 0.02, (m, k)).astype(np.float16).astype(np.float32)
+    picked = rng.random((m, k)) < 0.6
+    w[picked] = rng.choice(values, picked.sum())
+    a, meta = _native.pack_weight(torch.from_numpy(w).cuda().half(), prune=prune, layout=layout)
+    torch.cuda.synchronize()
+    want_a, want_meta = stored_by_oracle(w, prune, layout)
+    assert np.array_equal(a.cpu().numpy().ravel(), want_a.ravel())
+    assert np.array_equal(meta.cpu().numpy().ravel(), want_meta.ravel())
