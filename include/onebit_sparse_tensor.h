@@ -28,9 +28,11 @@
 extern "C" {
 #endif
 
-/* dtype codes for c / d */
+/* dtype codes (of c and d, unless said otherwise) */
 #define ONEBIT_DTYPE_F32 0
 #define ONEBIT_DTYPE_F16 1
+/* further dtype code, where an entry point says that it takes it */
+#define ONEBIT_DTYPE_BF16 2
 
 /* metadata layouts of e */
 #define ONEBIT_META_REFERENCE 0 /* onebit_sparse_mul/_semi_structured_conversions.py:21-48 (default) */
@@ -141,6 +143,14 @@ int onebit_sparse_linear_prepared_grouped(const onebit_linear_problem *problems,
  * pruned), prune == 0 takes the weight's non-zero pattern as it is.
  */
 int onebit_sparse_pack(const void *weight, int m, int k, int prune, void *a, void *e, int meta_layout, void *stream);
+
+/*
+ * The same for a weight of type fp32, fp16 or bf16 (weight_dtype, any of the three codes). bf16 and fp32 weights give
+ * what the reference's pipeline gives for them: fp32 values are rounded to fp16 after the pruning (so |w| <= 2^-25 counts
+ * as zero), NaN ranks as the largest magnitude.
+ */
+int onebit_sparse_pack_typed(const void *weight, int weight_dtype, int m, int k, int prune, void *a, void *e,
+                             int meta_layout, void *stream);
 
 /* Message of the last failure on the calling thread ("" if none). Host pointer, valid until the next call. */
 const char *onebit_sparse_last_error(void);

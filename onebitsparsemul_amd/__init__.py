@@ -160,9 +160,12 @@ class BinaryLinear_2_4(nn.Module):
         Reference: onebit_sparse_mul/__init__.py:130-145."""
         if tuple(weight.shape) != (self.outfeatures, self.infeatures):
             raise ValueError(f"weight must have shape ({self.outfeatures}, {self.infeatures})")
-        if weight.is_cuda and weight.dtype == torch.float16:
+        if weight.is_cuda and weight.dtype in (torch.float16, torch.bfloat16, torch.float32):
             # one fused HIP kernel (mask, compress, quantise, transpose-pack, reorder); same result as below
-            self.packed_binary_sparse, self.meta = _native.pack_weight(weight.contiguous(), prune=True)
+            weight = weight.contiguous()
+            if weight.data_ptr() % 16:
+                weight = weight.clone()  # a view that starts inside a 16-byte unit
+            self.packed_binary_sparse, self.meta = _native.pack_weight(weight, prune=True)
             self.vaild = True
             self._prepared = None
             return

@@ -8,7 +8,7 @@ import torch
 _DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_DIR, "libonebitmul.so")
 
-F32, F16 = 0, 1
+F32, F16, BF16 = 0, 1, 2
 META_REFERENCE, META_CUTLASS, META_LOGICAL = 0, 1, 2
 
 EXPORTS = (
@@ -17,7 +17,7 @@ EXPORTS = (
     "onebit_sparse_set_skinny_enabled", "onebit_sparse_set_skinny_rows", "onebit_sparse_set_split_k", "onebit_sparse_set_pad_b", "onebit_sparse_describe_launch", "onebit_sparse_set_weight_cache", "onebit_sparse_clear_weight_cache", "onebit_sparse_release_buffers",
     "onebit_sparse_measure_smfmac_rate", "onebit_sparse_device_info",
     "onebit_sparse_describe_launch_for", "onebit_sparse_measure_smfmac_rate_shape",
-    "onebit_sparse_linear_prepared_grouped",
+    "onebit_sparse_linear_prepared_grouped", "onebit_sparse_pack_typed",
 )
 
 
@@ -54,6 +54,8 @@ def lib():
         L.onebit_sparse_linear_prepared_grouped.argtypes = [ctypes.POINTER(LinearProblem), i32, i32, i32, i32, vp]
         L.onebit_sparse_pack.restype = i32
         L.onebit_sparse_pack.argtypes = [vp, i32, i32, i32, vp, vp, i32, vp]
+        L.onebit_sparse_pack_typed.restype = i32
+        L.onebit_sparse_pack_typed.argtypes = [vp, i32, i32, i32, i32, vp, vp, i32, vp]
         L.onebit_sparse_last_error.restype = ctypes.c_char_p
         L.onebit_sparse_last_error.argtypes = []
         L.onebit_sparse_set_tile_config.restype = None
@@ -299,17 +301,20 @@ def measure_smfmac_rate(random_operands=True, iterations=50000, shape=SMFMAC_32X
     return out.value
 
 
+_WEIGHT_CODES = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
+
+
 def pack_weight(weight, prune=True, layout=META_REFERENCE):
-    """dense fp16 (m, k) on the GPU -> (a uint8 (k/2, m/8), meta int16 (m, k/16)), the stored operands."""
+    """dense fp16, bf16 or fp32 (m, k) on the GPU -> (a uint8 (k/2, m/8), meta int16 (m, k/16)), the stored operands."""
     dev = _require_cuda(weight)
-    if weight.dtype != torch.float16 or weight.dim() != 2:
-        raise TypeError("weight must be a 2-dimensional float16 tensor")
+    if weight.dtype not in _WEIGHT_CODES or weight.dim() != 2:
+        raise TypeError("weight must be a 2-dimensional float16, bfloat16 or float32 tensor")
     m, k = weight.shape
     a = torch.empty((k // 2, m // 8), dtype=torch.uint8, device=dev)
     meta = torch.empty((m, k // 16), dtype=torch.int16, device=dev)
     with _on_device(dev):
-        _check(lib().onebit_sparse_pack(weight.data_ptr(), m, k, 1 if prune else 0, a.data_ptr(), meta.data_ptr(), layout,
-                                        _stream(weight)))
+        _check(lib().onebit_sparse_pack_typed(weight.data_ptr(), _WEIGHT_CODES[weight.dtype], m, k, 1 if prune else 0,
+                                              a.data_ptr(), meta.data_ptr(), layout, _stream(weight)))
     return a, meta
 
 

@@ -476,16 +476,23 @@ int onebit_sparse_prepare(const void* a, const void* e, int m, int k, int meta_l
 }
 
 int onebit_sparse_pack(const void* weight, int m, int k, int prune, void* a, void* e, int meta_layout, void* stream) {
+  return onebit_sparse_pack_typed(weight, ONEBIT_DTYPE_F16, m, k, prune, a, e, meta_layout, stream);
+}
+
+int onebit_sparse_pack_typed(const void* weight, int weight_dtype, int m, int k, int prune, void* a, void* e,
+                             int meta_layout, void* stream) {
   g_last_error.clear();
   if (int rc = check_shape(m, 1, k)) return rc;
   if (!weight || !a || !e) return fail(ONEBIT_ERR_ARGUMENT, "null operand pointer");
+  if (weight_dtype < ONEBIT_DTYPE_F32 || weight_dtype > ONEBIT_DTYPE_BF16)
+    return fail(ONEBIT_ERR_ARGUMENT, "weight dtype code must be 0 (fp32), 1 (fp16) or 2 (bf16), got %d", weight_dtype);
   if ((reinterpret_cast<uintptr_t>(weight) & 15) != 0)
     return fail(ONEBIT_ERR_ARGUMENT, "the dense weight must be 16-byte aligned");
   if ((reinterpret_cast<uintptr_t>(a) & 7) != 0 || (reinterpret_cast<uintptr_t>(e) & 1) != 0)
     return fail(ONEBIT_ERR_ARGUMENT, "a must be 8-byte aligned and e 2-byte aligned");
   if (meta_layout < ONEBIT_META_REFERENCE || meta_layout > ONEBIT_META_LOGICAL)
     return fail(ONEBIT_ERR_ARGUMENT, "unknown metadata layout %d", meta_layout);
-  ONEBIT_HIP(onebit::launch_pack(weight, a, e, m, k, prune, meta_layout, static_cast<hipStream_t>(stream)));
+  ONEBIT_HIP(onebit::launch_pack(weight, weight_dtype, a, e, m, k, prune, meta_layout, static_cast<hipStream_t>(stream)));
   return ONEBIT_OK;
 }
 

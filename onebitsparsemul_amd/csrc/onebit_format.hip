@@ -1,6 +1,6 @@
 // gfx950 kernels that bring a weight into the stored format and into the operand the GEMM kernels consume.
 //   prepare_kernel  : reference operands (1-bit values, reordered 2-bit-index metadata) -> prepared operand
-//   pack_kernel     : dense fp16 weight -> the reference operands (2:4 magnitude mask, compression, one-bit values)
+//   pack_kernel     : dense fp16, bf16 or fp32 weight -> the reference operands (2:4 magnitude mask, compression, one-bit values)
 #include "onebit_device.h"
 #include "onebit_launch.h"
 
@@ -151,15 +151,15 @@ __global__ __launch_bounds__(64 * kPreparePairs) void prepare_kernel(const uint8
 }
 
 // =====================================================================================================
-// pack_kernel: dense fp16 weight (m x k, row-major) -> the reference's stored operands (a bits, e metadata).
+// pack_kernel: dense weight (m x k, row-major; fp16, bf16 or fp32) -> the reference's stored operands (a bits, e metadata).
 // Fuses the steps of BinaryLinear_2_4.pack (onebit_sparse_mul/__init__.py:130-145): optional 2:4 magnitude
 // pruning (mask_creator, _semi_structured_conversions.py:286-314; among equal magnitudes the lower index is
 // pruned first), compression to kept values + nibbles (:126-159, including the fixed encodings of groups
 // with fewer or more than two non-zeros), sign quantisation (value > 0 -> 1, __init__.py:22-23), transposed
 // bit packing (__init__.py:25-34,142-143) and the metadata reorder (:21-48).
 //
-// One wavefront = 64 rows x 64 K. Lines of 128 bytes come in by asynchronous copies (eight lanes per row) and are
-// turned in LDS, after which lane r holds row r: sixteen groups of four. Everything that decides about a group is one bit
+// One wavefront = 64 rows x 64 K. The rows' 128 (fp32: 256) bytes come in by asynchronous copies and are turned in LDS,
+// after which lane r holds row r: sixteen groups of four. Everything that decides about a group is one bit
 // per value or per pair of values (which of two magnitudes is smaller, zero or not, the sign), so these bits are shifted
 // into slices of sixteen groups, two values per 32-bit register, and the rules are then evaluated once for all sixteen
 // groups with bitwise instructions. Slice bit 4 g + c belongs to group g of metadata column c: the four nibbles of a column
@@ -169,7 +169,8 @@ __global__ __launch_bounds__(64 * kPreparePairs) void prepare_kernel(const uint8
 // prepare_kernel, so that the eight-byte pieces of a line of `a` meet in its L2. Row tiles per workgroup / workgroups of a
 // strip, us inside a HIP graph at 11008 x 4096: 2 / 8 20.2, 4 / 4 20.6, 8 / 2 21.9, 16 / 1 24.2. Against 64-row wavefronts
 // that read their own row's line lane by lane and compared floats: 4096 x 4096 26.2 -> 10.1 us, 11008 x 4096 68.4 -> 20.6
-// (98 MB: 4.8 TB/s, the rate of a 2 GiB copy), 28672 x 8192 316 -> 105.
+// (98 MB: 4.8 TB/s, the rate of a 2 GiB copy), 28672 x 8192 316 -> 105. bf16 and fp32 weights, which took the tensor route
+// before (a sort of every group, some fifty launches): 11008 x 4096 15.4 ms -> 22 us and 27.8 ms -> 34 us.
 // =====================================================================================================
 constexpr int kPackTiles = 4, kPackStrip = 4;  // row tiles (wavefronts) per workgroup, workgroups side by side in a strip
 
@@ -181,12 +182,41 @@ __device__ __forceinline__ uint32_t packed_sub(uint32_t x, uint32_t y) {
 __device__ __forceinline__ uint32_t packed_add(uint32_t x, uint32_t y) {
   return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2_t, x) + __builtin_bit_cast(u16x2_t, y));
 }
+__device__ __forceinline__ uint32_t packed_min(uint32_t x, uint32_t y) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2_t, x), __builtin_bit_cast(u16x2_t, y)));
+}
 __device__ __forceinline__ uint32_t majority(uint32_t x, uint32_t y, uint32_t z) { return ((x ^ y) & (z ^ x)) ^ x; }
 
-__global__ __launch_bounds__(64 * kPackTiles) void pack_kernel(const _Float16* __restrict__ w, uint8_t* __restrict__ a,
-                                                               uint16_t* __restrict__ e, int m, int k, int prune,
-                                                               int layout, int k_tiles) {
-  __shared__ __attribute__((aligned(16))) char lds[kPackTiles * 8192];
+// Bits of the weight's type. bf16 and fp32 weights follow the unfused route, w * mask and then (fp32) a rounding to half
+// precision: what the mask removes from an infinite or NaN weight is NaN, which is not zero, and NaN counts as the
+// largest magnitude; fp32 values up to 2^-25 become zero. fp16 weights keep the rule that NaN outranks nothing.
+template <int DTYPE>
+struct PackType;
+template <>
+struct PackType<kPackF16> {
+  typedef _Float16 type;
+  static constexpr uint32_t kInfinity = 0x7C00, kLargestZero = 0, kMagnitude = 0x7FFF7FFFu;
+};
+template <>
+struct PackType<kPackBF16> {
+  typedef uint16_t type;
+  static constexpr uint32_t kInfinity = 0x7F80, kLargestZero = 0, kMagnitude = 0x7FFF7FFFu;
+};
+template <>
+struct PackType<kPackF32> {
+  typedef float type;
+  static constexpr uint32_t kInfinity = 0x7F800000u, kLargestZero = 0x33000000u, kMagnitude = 0x7FFFFFFFu;
+};
+
+template <int DTYPE>
+__global__ __launch_bounds__(64 * kPackTiles) void pack_kernel(const typename PackType<DTYPE>::type* __restrict__ w,
+                                                               uint8_t* __restrict__ a, uint16_t* __restrict__ e, int m,
+                                                               int k, int prune, int layout, int k_tiles) {
+  using Type = PackType<DTYPE>;
+  constexpr int SIZE = sizeof(typename Type::type);
+  constexpr int ROW_BYTES = 64 * SIZE, PIECES = ROW_BYTES / 16, ROWS_PER_COPY = 64 / PIECES;
+  constexpr bool NAN_RANKS = DTYPE != kPackF16;
+  __shared__ __attribute__((aligned(16))) char lds[kPackTiles * 64 * ROW_BYTES];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const StripPosition at = strip_position(kPackStrip, k_tiles);
@@ -196,53 +226,85 @@ __global__ __launch_bounds__(64 * kPackTiles) void pack_kernel(const _Float16* _
   const int ncols = k / 16, c_first = at.along * 4;
   const int c_count = ncols - c_first < 4 ? ncols - c_first : 4;  // the last tile may hold two columns only (k % 32 == 0)
 
-  // ---- 64 rows x 128 bytes into LDS: copy i carries rows 8 i ... 8 i + 7; piece q of row r goes to position q ^ (r % 8)
-  char* const image = lds + wave * 8192;
+  // ---- 64 rows into LDS, whole rows per copy; piece q (16 bytes) of row r goes to position q ^ (r % PIECES)
+  char* const image = lds + wave * (64 * ROW_BYTES);
   {
-    const int piece = (lane & 7) ^ (lane >> 3);
-    const int from = piece < 2 * c_count ? piece : 0;  // past K: any valid address will do, the results are not stored
-    const char* src = reinterpret_cast<const char*>(w + (row0 + (lane >> 3)) * k + 16 * c_first) + 16 * from;
+    const char* src = reinterpret_cast<const char*>(w + (row0 + lane / PIECES) * k + 16 * c_first);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) lds_dma16(src + (size_t)i * 16 * k, lds_offset_of(image) + i * 1024);
+    for (int i = 0; i < PIECES; ++i) {
+      const int piece = (lane % PIECES) ^ ((i * ROWS_PER_COPY + lane / PIECES) % PIECES);
+      const int from = piece < SIZE * c_count ? piece : 0;  // past K: any valid address will do, the results are not stored
+      lds_dma16(src + (size_t)i * ROWS_PER_COPY * SIZE * k + 16 * from, lds_offset_of(image) + i * 1024);
+    }
   }
   wait_vmcnt<0>();
-  uint32_t d[32];  // dword 2 q: values 0 and 1 of group q, dword 2 q + 1: values 2 and 3
+  uint32_t d[ROW_BYTES / 4];  // the row; group q (four values): two dwords of two values, or (fp32) four dwords
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const u32x4_t v = *reinterpret_cast<const u32x4_t*>(image + lane * 128 + ((q ^ (lane & 7)) << 4));
+  for (int q = 0; q < PIECES; ++q) {
+    const u32x4_t v = *reinterpret_cast<const u32x4_t*>(image + lane * ROW_BYTES + ((q ^ (lane % PIECES)) << 4));
     d[4 * q] = v.x; d[4 * q + 1] = v.y; d[4 * q + 2] = v.z; d[4 * q + 3] = v.w;
   }
 
   // ---- slices. less_ij: magnitude j < magnitude i (i < j), i.e. i outranks j; otherwise j outranks i (ties: the higher
   // index). Low half | high half of a register: 02|13, 03|12, 01|23 for pairs, 0|1 and 2|3 for single values.
   uint32_t less_02_13 = 0, less_03_12 = 0, less_01_23 = 0, nonzero_01 = 0, nonzero_23 = 0, nan_01 = 0, nan_23 = 0,
-           minus_01 = 0, minus_23 = 0;
+           minus_01 = 0, minus_23 = 0, huge_01 = 0, huge_23 = 0;
 #pragma unroll
   for (int t = 0; t < 16; ++t) {
     const int q = 4 * (t & 3) + (t >> 2);  // group t / 4 of column t % 4
-    const uint32_t d0 = d[2 * q], d1 = d[2 * q + 1];
-    const uint32_t m0 = d0 & 0x7FFF7FFFu, m1 = d1 & 0x7FFF7FFFu;  // magnitudes order like their bits
     auto push = [](uint32_t& slice, uint32_t x) __attribute__((always_inline)) {  // bits 15 and 31 of x
       slice = (x & 0x80008000u) | ((slice >> 1) & 0x7FFF7FFFu);
     };
-    push(less_02_13, packed_sub(m1, m0));
-    push(less_03_12, packed_sub(__builtin_amdgcn_alignbit(m1, m1, 16), m0));
-    push(less_01_23, packed_sub(__builtin_amdgcn_perm(m1, m0, 0x07060302u), __builtin_amdgcn_perm(m1, m0, 0x05040100u)));
-    push(nonzero_01, packed_add(m0, 0x7FFF7FFFu));
-    push(nonzero_23, packed_add(m1, 0x7FFF7FFFu));
-    push(nan_01, packed_add(m0, 0x03FF03FFu));  // magnitude > infinity's bits 0x7C00
-    push(nan_23, packed_add(m1, 0x03FF03FFu));
-    push(minus_01, d0);
-    push(minus_23, d1);
+    if constexpr (SIZE == 2) {
+      const uint32_t d0 = d[2 * q], d1 = d[2 * q + 1];
+      uint32_t m0 = d0 & Type::kMagnitude, m1 = d1 & Type::kMagnitude;  // magnitudes order like their bits
+      if constexpr (NAN_RANKS) m0 = packed_min(m0, (Type::kInfinity + 1) * 0x10001u), m1 = packed_min(m1, (Type::kInfinity + 1) * 0x10001u);
+      push(less_02_13, packed_sub(m1, m0));
+      push(less_03_12, packed_sub(__builtin_amdgcn_alignbit(m1, m1, 16), m0));
+      push(less_01_23, packed_sub(__builtin_amdgcn_perm(m1, m0, 0x07060302u), __builtin_amdgcn_perm(m1, m0, 0x05040100u)));
+      // magnitude > limit sets bit 15 of magnitude + (0x7FFF - limit)
+      constexpr uint32_t kNonzero = 0x7FFFu * 0x10001u, kNan = (0x7FFFu - Type::kInfinity) * 0x10001u;
+      push(nonzero_01, packed_add(m0, kNonzero));
+      push(nonzero_23, packed_add(m1, kNonzero));
+      push(nan_01, packed_add(m0, kNan));
+      push(nan_23, packed_add(m1, kNan));
+      if constexpr (NAN_RANKS) push(huge_01, packed_add(m0, kNan + 0x10001u)), push(huge_23, packed_add(m1, kNan + 0x10001u));
+      push(minus_01, d0);
+      push(minus_23, d1);
+    } else {
+      uint32_t mag[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        mag[i] = d[4 * q + i] & Type::kMagnitude;
+        mag[i] = mag[i] < Type::kInfinity + 1 ? mag[i] : Type::kInfinity + 1;  // every NaN alike
+      }
+      // bits 31 of two words to bits 15 and 31
+      auto tops = [](uint32_t low, uint32_t high) __attribute__((always_inline)) {
+        return __builtin_amdgcn_perm(high, low, 0x07060302u);
+      };
+      push(less_02_13, tops(mag[2] - mag[0], mag[3] - mag[1]));
+      push(less_03_12, tops(mag[3] - mag[0], mag[2] - mag[1]));
+      push(less_01_23, tops(mag[1] - mag[0], mag[3] - mag[2]));
+      constexpr uint32_t kNonzero = 0x7FFFFFFFu - Type::kLargestZero, kNan = 0x7FFFFFFFu - Type::kInfinity;
+      push(nonzero_01, tops(mag[0] + kNonzero, mag[1] + kNonzero));
+      push(nonzero_23, tops(mag[2] + kNonzero, mag[3] + kNonzero));
+      push(nan_01, tops(mag[0] + kNan, mag[1] + kNan));
+      push(nan_23, tops(mag[2] + kNan, mag[3] + kNan));
+      push(huge_01, tops(mag[0] + (kNan + 1), mag[1] + (kNan + 1)));
+      push(huge_23, tops(mag[2] + (kNan + 1), mag[3] + (kNan + 1)));
+      push(minus_01, tops(d[4 * q], d[4 * q + 1]));
+      push(minus_23, tops(d[4 * q + 2], d[4 * q + 3]));
+    }
   }
 
   // ---- the rules, on 16-bit slices (the upper halves of these registers hold other slices and are masked at the end)
   const uint32_t nan0 = nan_01, nan1 = nan_01 >> 16, nan2 = nan_23, nan3 = nan_23 >> 16;
   uint32_t keep0 = ~0u, keep1 = ~0u, keep2 = ~0u, keep3 = ~0u;
   if (prune) {
-    // a comparison with NaN is false both ways
-    const uint32_t ok01 = ~(nan0 | nan1), ok02 = ~(nan0 | nan2), ok03 = ~(nan0 | nan3), ok12 = ~(nan1 | nan2),
-                   ok13 = ~(nan1 | nan3), ok23 = ~(nan2 | nan3);
+    // fp16: a comparison with NaN is false both ways
+    auto comparable = [](uint32_t x, uint32_t y) __attribute__((always_inline)) { return NAN_RANKS ? ~0u : ~(x | y); };
+    const uint32_t ok01 = comparable(nan0, nan1), ok02 = comparable(nan0, nan2), ok03 = comparable(nan0, nan3),
+                   ok12 = comparable(nan1, nan2), ok13 = comparable(nan1, nan3), ok23 = comparable(nan2, nan3);
     const uint32_t l01 = less_01_23, l23 = less_01_23 >> 16, l02 = less_02_13, l13 = less_02_13 >> 16, l03 = less_03_12,
                    l12 = less_03_12 >> 16;
     // a value goes when two of the other three outrank it
@@ -251,10 +313,11 @@ __global__ __launch_bounds__(64 * kPackTiles) void pack_kernel(const _Float16* _
     keep2 = ~majority(l02 & ok02, l12 & ok12, ~l23 & ok23);
     keep3 = ~majority(l03 & ok03, l13 & ok13, l23 & ok23);
   }
-  const uint32_t p0 = keep0 & nonzero_01, p1 = keep1 & (nonzero_01 >> 16), p2 = keep2 & nonzero_23,
-                 p3 = keep3 & (nonzero_23 >> 16);
+  uint32_t p0 = keep0 & nonzero_01, p1 = keep1 & (nonzero_01 >> 16), p2 = keep2 & nonzero_23,
+           p3 = keep3 & (nonzero_23 >> 16);
   const uint32_t plus0 = p0 & ~minus_01 & ~nan0, plus1 = p1 & ~(minus_01 >> 16) & ~nan1, plus2 = p2 & ~minus_23 & ~nan2,
                  plus3 = p3 & ~(minus_23 >> 16) & ~nan3;
+  if (NAN_RANKS && prune) p0 |= huge_01, p1 |= huge_01 >> 16, p2 |= huge_23, p3 |= huge_23 >> 16;  // 0 * infinity
   // Bits of the nibble idx0 | idx1 << 2 for the pattern of non-zeros (p0 p1 p2 p3). With p0 and p1 it names 0 and 1; with
   // one of them, that one and 3 if p3, else 2; with neither, 2 and 3. (Which also gives the reference's fixed encodings
   // of groups with other than two non-zeros.)
@@ -317,12 +380,22 @@ hipError_t launch_prepare(const void* a, const void* e, void* prep, int m, int k
   return hipGetLastError();
 }
 
-hipError_t launch_pack(const void* w, void* a, void* e, int m, int k, int prune, int layout, hipStream_t stream) {
+template <int DTYPE>
+static void launch_pack_type(const void* w, void* a, void* e, int m, int k, int prune, int layout, hipStream_t stream) {
   const int k_tiles = (k / 16 + 3) / 4;
   constexpr int kStripTiles = kPackTiles * kPackStrip;
   const dim3 grid(k_tiles * kPackStrip * ((m / 64 + kStripTiles - 1) / kStripTiles));
-  hipLaunchKernelGGL(pack_kernel, grid, dim3(64 * kPackTiles), 0, stream, (const _Float16*)w, (uint8_t*)a, (uint16_t*)e,
-                     m, k, prune, layout, k_tiles);
+  hipLaunchKernelGGL(pack_kernel<DTYPE>, grid, dim3(64 * kPackTiles), 0, stream,
+                     (const typename PackType<DTYPE>::type*)w, (uint8_t*)a, (uint16_t*)e, m, k, prune, layout, k_tiles);
+}
+
+hipError_t launch_pack(const void* w, int dtype, void* a, void* e, int m, int k, int prune, int layout, hipStream_t stream) {
+  switch (dtype) {
+    case kPackF32: launch_pack_type<kPackF32>(w, a, e, m, k, prune, layout, stream); break;
+    case kPackF16: launch_pack_type<kPackF16>(w, a, e, m, k, prune, layout, stream); break;
+    case kPackBF16: launch_pack_type<kPackBF16>(w, a, e, m, k, prune, layout, stream); break;
+    default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 

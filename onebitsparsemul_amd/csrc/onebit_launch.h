@@ -72,8 +72,10 @@ hipError_t launch_gemm(GemmArgs args, int tile_config, hipStream_t stream);
 // m), y = x W^T + bias; c, alpha, beta and the padded copy of B are not used, splits / chunks_per_split / split_ws as in
 // launch_gemm. Tiles 4, 6, 9, 10, 11, 12, 13, 14, 15.
 hipError_t launch_gemm_tokens(GemmArgs args, int tile_config, hipStream_t stream);
-// dense fp16 (m x k) -> one-bit values `a` and metadata `e`; prune != 0 applies the 2:4 magnitude mask first
-hipError_t launch_pack(const void* w, void* a, void* e, int m, int k, int prune, int layout, hipStream_t stream);
+// dense (m x k) -> one-bit values `a` and metadata `e`; prune != 0 applies the 2:4 magnitude mask first. dtype: the codes
+// of the C ABI.
+enum PackDtype { kPackF32 = 0, kPackF16 = 1, kPackBF16 = 2 };
+hipError_t launch_pack(const void* w, int dtype, void* a, void* e, int m, int k, int prune, int layout, hipStream_t stream);
 
 // Split-K kernel for n <= 64; rows_per_group (32, 64 or 128) = weight rows one workgroup covers (n > 32: at most 64).
 constexpr int kSkinnyMaxN = 64;

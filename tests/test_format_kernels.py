@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import oracle
+import onebitsparsemul_amd as ob
 from onebitsparsemul_amd import _native
 
 
@@ -88,3 +89,24 @@ def test_packed_weight_bytes(m, k, layout, prune):
     want_a, want_meta = stored_by_oracle(w, prune, layout)
     assert np.array_equal(a.cpu().numpy().ravel(), want_a.ravel())
     assert np.array_equal(meta.cpu().numpy().ravel(), want_meta.ravel())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m,k", [(64, 32), (320, 96), (1088, 192)])
+def test_pack_of_bf16_and_fp32_weights(m, k, dtype):
+    """The fused kernel against the layer's tensor route on the CPU, with ties, zeros, the values around the smallest
+    half-precision number, infinities and NaN (w * mask makes a NaN of an infinity that the mask removes)."""
+    rng = np.random.default_rng(m + k)
+    values = np.array([0.0, -0.0, 1.0, -1.0, 0.5, -0.5, 2.0**-24, -2.0**-24, 2.0**-25, -2.0**-25, 2.0**-25 * 1.01, 2.0**-130,
+                       7e4, np.inf, -np.inf, np.nan], dtype=np.float32)
+    w = rng.normal(0, 0.02, (m, k)).astype(np.float32)
+    picked = rng.random((m, k)) < 0.6
+    w[picked] = rng.choice(values, picked.sum())
+    w = torch.from_numpy(w).to(dtype)
+    on_cpu, on_gpu = ob.BinaryLinear_2_4(k, m), ob.BinaryLinear_2_4(k, m)
+    on_cpu.pack(w)
+    on_gpu.pack(w.cuda())
+    torch.cuda.synchronize()
+    assert torch.equal(on_gpu.packed_binary_sparse.cpu(), on_cpu.packed_binary_sparse)
+    assert torch.equal(on_gpu.meta.cpu(), on_cpu.meta)
