@@ -29,6 +29,9 @@ typedef float float4v_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x8_t __attribute__((ext_vector_type(8)));
+// the same, for memory that is aligned to its elements only (gfx950 loads and stores 16 bytes at any address)
+typedef u32x4_t u32x4_any_t __attribute__((aligned(2)));
+typedef u32x2_t u32x2_any_t __attribute__((aligned(2)));
 typedef __fp16 fp16x4_t __attribute__((__vector_size__(8)));
 
 // ---- prepared A operand ---------------------------------------------------------------------------

@@ -955,229 +955,253 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
   }
   // ---- epilogue: D = alpha * acc + beta * C (csrc/kernel.h:27-31), fp16 (RNE) or fp32 output ----
   if constexpr (DMA) {
-    if (p.vector_epilogue) {
-      // Coalesced form: each wavefront turns one 32-row block of its tile at a time through a private LDS
-      // scratch (fp32, row-major) so that every lane then handles 16 bytes of one output row: C is read and D
-      // written in full 128-byte segments instead of 64-byte (fp16) pieces per accumulator register.
-      __syncthreads();  // every wavefront is done with the stage ring, which becomes the scratch
-      constexpr int WCOLS = FN * 32;                   // columns of the wavefront's tile
-      float* scratch = reinterpret_cast<float*>(smem) + wave * (32 * WCOLS);
-      const int col_lane = lane & 31, row_lane = 4 * (lane >> 5);
-      // Column swizzle of the scratch against bank conflicts, the same for rows of floats and for row pairs of packed
-      // halves: line L keeps its 16-byte slots swapped in pairs when L is odd (two consecutive lines are read by one
-      // group of sixteen lanes: they then touch different banks), and, with lines of 256 bytes or more, its two halves of
-      // 128 bytes swapped when bit 2 (rows) or bit 1 (row pairs) of L is set (the upper half-wavefront writes the line
-      // that many below the lower half's).
-      constexpr int kHalfSwap = WCOLS >= 64 ? 32 : 0;
-      // The accumulators of 32-row block fm into the scratch. 32x32x32 form: register v of fragment fn is row
-      // 8 (v / 4) + 4 (lane / 32) + v % 4, column 32 fn + lane % 32; 16x16x64 form: register v of tile (2 fm + rh, ct) is
-      // row 16 rh + 4 (lane / 16) + v, column 16 ct + lane % 16. In both, bit 2 of the row is one bit of the lane
-      // (the writer's own half swap) and bit 0 of the row is bit 0 of v.
-      const int g16 = lane >> 4, c16 = lane & 15;
-      const int half_write = (M16 ? (g16 & 1) : (lane >> 5)) * kHalfSwap;
-      auto store_rows = [&](int fm) __attribute__((always_inline)) {
+    // Coalesced form: each wavefront turns one 32-row block of its tile at a time through a private LDS
+    // scratch (fp32, row-major) so that every lane then handles 16 bytes of one output row: C is read and D
+    // written in full 128-byte segments instead of 64-byte (fp16) pieces per accumulator register.
+    __syncthreads();  // every wavefront is done with the stage ring, which becomes the scratch
+    constexpr int WCOLS = FN * 32;                   // columns of the wavefront's tile
+    float* scratch = reinterpret_cast<float*>(smem) + wave * (32 * WCOLS);
+    const int col_lane = lane & 31, row_lane = 4 * (lane >> 5);
+    // Column swizzle of the scratch against bank conflicts, the same for rows of floats and for row pairs of packed
+    // halves: line L keeps its 16-byte slots swapped in pairs when L is odd (two consecutive lines are read by one
+    // group of sixteen lanes: they then touch different banks), and, with lines of 256 bytes or more, its two halves of
+    // 128 bytes swapped when bit 2 (rows) or bit 1 (row pairs) of L is set (the upper half-wavefront writes the line
+    // that many below the lower half's).
+    constexpr int kHalfSwap = WCOLS >= 64 ? 32 : 0;
+    // The accumulators of 32-row block fm into the scratch. 32x32x32 form: register v of fragment fn is row
+    // 8 (v / 4) + 4 (lane / 32) + v % 4, column 32 fn + lane % 32; 16x16x64 form: register v of tile (2 fm + rh, ct) is
+    // row 16 rh + 4 (lane / 16) + v, column 16 ct + lane % 16. In both, bit 2 of the row is one bit of the lane
+    // (the writer's own half swap) and bit 0 of the row is bit 0 of v.
+    const int g16 = lane >> 4, c16 = lane & 15;
+    const int half_write = (M16 ? (g16 & 1) : (lane >> 5)) * kHalfSwap;
+    auto store_rows = [&](int fm) __attribute__((always_inline)) {
+      if constexpr (M16) {
+#pragma unroll
+        for (int rh = 0; rh < 2; ++rh)
+#pragma unroll
+          for (int ct = 0; ct < 2 * FN; ++ct)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+              scratch[(16 * rh + 4 * g16 + v) * WCOLS + ((ct * 16 + c16) ^ half_write ^ ((v & 1) << 2))] =
+                  acc16[2 * fm + rh][ct][v];
+      } else {
+#pragma unroll
+        for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            scratch[(8 * (v / 4) + row_lane + (v % 4)) * WCOLS + ((fn * 32 + col_lane) ^ half_write ^ ((v & 1) << 2))] =
+                acc[fm][fn][v];
+      }
+    };
+    auto read_swizzle = [&](int line, int half_bit) __attribute__((always_inline)) {
+      return ((line & 1) << 2) ^ (((line >> half_bit) & 1) * kHalfSwap);
+    };
+    // Rows of C and D may start at any element (n is any number). Whole pieces of 8 halves or 4 floats are moved as
+    // vectors at any alignment; what is left of the rows behind their last whole piece, element by element from the
+    // scratch: sum_at(r, c) is the alpha-scaled sum of row r, column c of the block.
+    auto cut_rows = [&](int row_base, int piece, auto&& sum_at) __attribute__((always_inline)) {
+      const int tail = p.n - p.n % piece;
+      if (tail == p.n || tail < col0 || tail >= col0 + WCOLS) return;  // wave-uniform
+#pragma unroll 1
+      for (int i = lane; i < 32 * 8; i += 64) {
+        const int r = i >> 3, row = row_base + r, col = tail + (i & 7);
+        if (row < row_limit && col < p.n) {
+          const size_t o = (size_t)row * p.n + col;
+          float x = sum_at(r, col - col0);
+          if (p.beta != 0.f)
+            x = x + p.beta * (p.c_f16 ? (float)reinterpret_cast<const _Float16*>(p.c)[o] : reinterpret_cast<const float*>(p.c)[o]);
+          if (p.d_f16) reinterpret_cast<_Float16*>(d_out)[o] = (_Float16)x;
+          else reinterpret_cast<float*>(d_out)[o] = x;
+        }
+      }
+    };
+    // The pieces of C that a lane will need for one 32-row block are requested together, before the block's sums
+    // travel through the scratch, so that one memory latency per block is paid instead of one per piece.
+    const bool use_c = p.beta != 0.f;
+    if (p.d_f16 && !use_c && WCOLS >= 8) {
+      // fp16 result without C: alpha * sum is rounded in the accumulator layout, where registers v and v + 1 (v even)
+      // of a lane are rows r and r + 1 of one column; the two halves go through the scratch as one word (a quarter of
+      // the LDS traffic of the fp32 form). A lane then reads eight such words (columns c .. c + 7 of a row pair),
+      // separates low and high halves and stores 16 bytes of row r and 16 bytes of row r + 1.
+      uint32_t* const words = reinterpret_cast<uint32_t*>(scratch);  // [16 row pairs][WCOLS]
+      typedef float float2v __attribute__((ext_vector_type(2)));
+      typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+      constexpr int PER_PAIR = WCOLS / 8;            // 8-column pieces per row pair
+      constexpr int TASKS = 16 * PER_PAIR;           // (row pair, piece) per 32-row block
+      constexpr int ITERS = (TASKS + 63) / 64;
+      // alpha == 1 is tested once per wavefront, not per value: two copies of the loop
+      auto packed_turn = [&](auto scale_tag) __attribute__((always_inline)) {
+      constexpr bool SCALE = decltype(scale_tag)::value;
+#pragma unroll
+      for (int fm = 0; fm < FM; ++fm) {
+        if (!finishes(fm)) continue;  // the other K group stores this fragment
+        const int row_base = row0 + fm * 32;
+        auto pack = [&](float x0, float x1) __attribute__((always_inline)) {  // one packed conversion per register pair
+          float2v x = {x0, x1};
+          if constexpr (SCALE) x = float2v{p.alpha * x.x, p.alpha * x.y};
+          return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, half2v));
+        };
         if constexpr (M16) {
+          // registers (0, 1) and (2, 3) of a tile: rows 16 rh + 4 (lane / 16) + 2 h and the next, row pair
+          // 8 rh + 2 (lane / 16) + h
 #pragma unroll
           for (int rh = 0; rh < 2; ++rh)
 #pragma unroll
             for (int ct = 0; ct < 2 * FN; ++ct)
 #pragma unroll
-              for (int v = 0; v < 4; ++v)
-                scratch[(16 * rh + 4 * g16 + v) * WCOLS + ((ct * 16 + c16) ^ half_write ^ ((v & 1) << 2))] =
-                    acc16[2 * fm + rh][ct][v];
+              for (int h = 0; h < 2; ++h)
+                words[(8 * rh + 2 * g16 + h) * WCOLS + ((ct * 16 + c16) ^ half_write ^ (h << 2))] =
+                    pack(acc16[2 * fm + rh][ct][2 * h], acc16[2 * fm + rh][ct][2 * h + 1]);
         } else {
 #pragma unroll
           for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
-            for (int v = 0; v < 16; ++v)
-              scratch[(8 * (v / 4) + row_lane + (v % 4)) * WCOLS + ((fn * 32 + col_lane) ^ half_write ^ ((v & 1) << 2))] =
-                  acc[fm][fn][v];
+            for (int q = 0; q < 8; ++q)
+              // rows 8 (q / 2) + 4 (lane / 32) + 2 (q % 2) and the next: row pair 4 (q / 2) + 2 (lane / 32) + q % 2
+              words[(4 * (q / 2) + (row_lane >> 1) + (q & 1)) * WCOLS + ((fn * 32 + col_lane) ^ half_write ^ ((q & 1) << 2))] =
+                  pack(acc[fm][fn][2 * q], acc[fm][fn][2 * q + 1]);
         }
-      };
-      auto read_swizzle = [&](int line, int half_bit) __attribute__((always_inline)) {
-        return ((line & 1) << 2) ^ (((line >> half_bit) & 1) * kHalfSwap);
-      };
-      // The pieces of C that a lane will need for one 32-row block are requested together, before the block's sums
-      // travel through the scratch, so that one memory latency per block is paid instead of one per piece.
-      const bool use_c = p.beta != 0.f;
-      if (p.d_f16 && !use_c && WCOLS >= 8) {
-        // fp16 result without C: alpha * sum is rounded in the accumulator layout, where registers v and v + 1 (v even)
-        // of a lane are rows r and r + 1 of one column; the two halves go through the scratch as one word (a quarter of
-        // the LDS traffic of the fp32 form). A lane then reads eight such words (columns c .. c + 7 of a row pair),
-        // separates low and high halves and stores 16 bytes of row r and 16 bytes of row r + 1.
-        uint32_t* const words = reinterpret_cast<uint32_t*>(scratch);  // [16 row pairs][WCOLS]
-        typedef float float2v __attribute__((ext_vector_type(2)));
-        typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-        constexpr int PER_PAIR = WCOLS / 8;            // 8-column pieces per row pair
-        constexpr int TASKS = 16 * PER_PAIR;           // (row pair, piece) per 32-row block
-        constexpr int ITERS = (TASKS + 63) / 64;
-        // alpha == 1 is tested once per wavefront, not per value: two copies of the loop
-        auto packed_turn = [&](auto scale_tag) __attribute__((always_inline)) {
-        constexpr bool SCALE = decltype(scale_tag)::value;
 #pragma unroll
-        for (int fm = 0; fm < FM; ++fm) {
-          if (!finishes(fm)) continue;  // the other K group stores this fragment
-          const int row_base = row0 + fm * 32;
-          auto pack = [&](float x0, float x1) __attribute__((always_inline)) {  // one packed conversion per register pair
-            float2v x = {x0, x1};
-            if constexpr (SCALE) x = float2v{p.alpha * x.x, p.alpha * x.y};
-            return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, half2v));
-          };
-          if constexpr (M16) {
-            // registers (0, 1) and (2, 3) of a tile: rows 16 rh + 4 (lane / 16) + 2 h and the next, row pair
-            // 8 rh + 2 (lane / 16) + h
+        for (int it = 0; it < ITERS; ++it) {
+          const int task = it * 64 + lane;
+          if (TASKS % 64 != 0 && task >= TASKS) break;
+          const int pair = task / PER_PAIR, c8 = (task % PER_PAIR) * 8;
+          const int sw = read_swizzle(pair, 1);
+          const u32x4_t lo = *reinterpret_cast<const u32x4_t*>(words + pair * WCOLS + (c8 ^ sw));
+          const u32x4_t hi = *reinterpret_cast<const u32x4_t*>(words + pair * WCOLS + ((c8 + 4) ^ sw));
+          const uint32_t d[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+          u32x4_t even_row, odd_row;
 #pragma unroll
-            for (int rh = 0; rh < 2; ++rh)
-#pragma unroll
-              for (int ct = 0; ct < 2 * FN; ++ct)
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-                  words[(8 * rh + 2 * g16 + h) * WCOLS + ((ct * 16 + c16) ^ half_write ^ (h << 2))] =
-                      pack(acc16[2 * fm + rh][ct][2 * h], acc16[2 * fm + rh][ct][2 * h + 1]);
-          } else {
-#pragma unroll
-            for (int fn = 0; fn < FN; ++fn)
-#pragma unroll
-              for (int q = 0; q < 8; ++q)
-                // rows 8 (q / 2) + 4 (lane / 32) + 2 (q % 2) and the next: row pair 4 (q / 2) + 2 (lane / 32) + q % 2
-                words[(4 * (q / 2) + (row_lane >> 1) + (q & 1)) * WCOLS + ((fn * 32 + col_lane) ^ half_write ^ ((q & 1) << 2))] =
-                    pack(acc[fm][fn][2 * q], acc[fm][fn][2 * q + 1]);
+          for (int j = 0; j < 4; ++j) {
+            even_row[j] = __builtin_amdgcn_perm(d[2 * j + 1], d[2 * j], 0x05040100u);  // low halves
+            odd_row[j] = __builtin_amdgcn_perm(d[2 * j + 1], d[2 * j], 0x07060302u);   // high halves
           }
-#pragma unroll
-          for (int it = 0; it < ITERS; ++it) {
-            const int task = it * 64 + lane;
-            if (TASKS % 64 != 0 && task >= TASKS) break;
-            const int pair = task / PER_PAIR, c8 = (task % PER_PAIR) * 8;
-            const int sw = read_swizzle(pair, 1);
-            const u32x4_t lo = *reinterpret_cast<const u32x4_t*>(words + pair * WCOLS + (c8 ^ sw));
-            const u32x4_t hi = *reinterpret_cast<const u32x4_t*>(words + pair * WCOLS + ((c8 + 4) ^ sw));
-            const uint32_t d[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-            u32x4_t even_row, odd_row;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              even_row[j] = __builtin_amdgcn_perm(d[2 * j + 1], d[2 * j], 0x05040100u);  // low halves
-              odd_row[j] = __builtin_amdgcn_perm(d[2 * j + 1], d[2 * j], 0x07060302u);   // high halves
-            }
-            const int row = row_base + 2 * pair, col = col0 + c8;
-            if (col < p.n) {
-              _Float16* const out = reinterpret_cast<_Float16*>(d_out) + (size_t)row * p.n + col;
-              if (row < row_limit) *reinterpret_cast<u32x4_t*>(out) = even_row;
-              if (row + 1 < row_limit) *reinterpret_cast<u32x4_t*>(out + p.n) = odd_row;
-            }
+          const int row = row_base + 2 * pair, col = col0 + c8;
+          if (col + 8 <= p.n) {
+            _Float16* const out = reinterpret_cast<_Float16*>(d_out) + (size_t)row * p.n + col;
+            if (row < row_limit) *reinterpret_cast<u32x4_any_t*>(out) = even_row;
+            if (row + 1 < row_limit) *reinterpret_cast<u32x4_any_t*>(out + p.n) = odd_row;
           }
         }
-        };
-        if (p.alpha != 1.f) packed_turn(std::true_type{});
-        else packed_turn(std::false_type{});
-        return;
+        cut_rows(row_base, 8, [&](int r, int c) {  // already scaled and rounded: the low half of a word is the even row
+          const uint32_t word = words[(r >> 1) * WCOLS + (c ^ read_swizzle(r >> 1, 1))];
+          return (float)__builtin_bit_cast(_Float16, (uint16_t)(r & 1 ? word >> 16 : word));
+        });
       }
-#pragma unroll
-      for (int fm = 0; fm < FM; ++fm) {
-        if (!finishes(fm)) continue;  // the other K group stores this fragment
-        const int row_base = row0 + fm * 32;
-        if (p.d_f16) {
-          constexpr int PER_ROW = WCOLS / 8;           // 16-byte pieces (8 halves) per row
-          constexpr int ITERS = 32 * PER_ROW / 64;
-          uint32_t c_raw[ITERS][8];                    // fp16 C: one 16-byte load per piece (words 0-3); fp32 C: two
-#pragma unroll
-          for (int it = 0; it < ITERS; ++it) {
-            const int piece = it * 64 + lane;
-            const int row = row_base + piece / PER_ROW, col = col0 + (piece % PER_ROW) * 8;
-            u32x4_t lo = u32x4_t{0, 0, 0, 0}, hi = u32x4_t{0, 0, 0, 0};
-            if (use_c && row < row_limit && col < p.n) {
-              const size_t o = (size_t)row * p.n + col;
-              if (p.c_f16) {
-                lo = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const _Float16*>(p.c) + o);
-              } else {
-                lo = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const float*>(p.c) + o);
-                hi = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const float*>(p.c) + o + 4);
-              }
-            }
-            c_raw[it][0] = lo.x; c_raw[it][1] = lo.y; c_raw[it][2] = lo.z; c_raw[it][3] = lo.w;
-            c_raw[it][4] = hi.x; c_raw[it][5] = hi.y; c_raw[it][6] = hi.z; c_raw[it][7] = hi.w;
-          }
-          store_rows(fm);
-#pragma unroll
-          for (int it = 0; it < ITERS; ++it) {
-            const int piece = it * 64 + lane;
-            const int r = piece / PER_ROW, c8 = (piece % PER_ROW) * 8;
-            const int row = row_base + r, col = col0 + c8;
-            const int sw = read_swizzle(r, 2);
-            const float4 lo = *reinterpret_cast<const float4*>(scratch + r * WCOLS + (c8 ^ sw));
-            const float4 hi = *reinterpret_cast<const float4*>(scratch + r * WCOLS + ((c8 + 4) ^ sw));
-            float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-            if (row < row_limit && col < p.n) {
-              const size_t o = (size_t)row * p.n + col;
-#pragma unroll
-              for (int j = 0; j < 8; ++j) x[j] = p.alpha * x[j];
-              if (use_c) {
-                if (p.c_f16) {
-                  const half8_t cv =
-                      __builtin_bit_cast(half8_t, u32x4_t{c_raw[it][0], c_raw[it][1], c_raw[it][2], c_raw[it][3]});
-#pragma unroll
-                  for (int j = 0; j < 8; ++j) x[j] = x[j] + p.beta * (float)cv[j];
-                } else {
-#pragma unroll
-                  for (int j = 0; j < 8; ++j) x[j] = x[j] + p.beta * __builtin_bit_cast(float, c_raw[it][j]);
-                }
-              }
-              half8_t out;
-#pragma unroll
-              for (int j = 0; j < 8; ++j) out[j] = (_Float16)x[j];
-              *reinterpret_cast<half8_t*>(reinterpret_cast<_Float16*>(d_out) + o) = out;
-            }
-          }
-        } else {
-          constexpr int PER_ROW = WCOLS / 4;           // 16-byte pieces (4 floats) per row
-          constexpr int ITERS = 32 * PER_ROW / 64;
-          uint32_t c_raw[ITERS][4];                    // fp32 C: one 16-byte load per piece; fp16 C: one 8-byte load
-#pragma unroll
-          for (int it = 0; it < ITERS; ++it) {
-            const int piece = it * 64 + lane;
-            const int row = row_base + piece / PER_ROW, col = col0 + (piece % PER_ROW) * 4;
-            u32x4_t lo = u32x4_t{0, 0, 0, 0};
-            if (use_c && row < row_limit && col < p.n) {
-              const size_t o = (size_t)row * p.n + col;
-              if (p.c_f16) {
-                const u32x2_t t = *reinterpret_cast<const u32x2_t*>(reinterpret_cast<const _Float16*>(p.c) + o);
-                lo.x = t.x; lo.y = t.y;
-              } else {
-                lo = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const float*>(p.c) + o);
-              }
-            }
-            c_raw[it][0] = lo.x; c_raw[it][1] = lo.y; c_raw[it][2] = lo.z; c_raw[it][3] = lo.w;
-          }
-          store_rows(fm);
-#pragma unroll
-          for (int it = 0; it < ITERS; ++it) {
-            const int piece = it * 64 + lane;
-            const int r = piece / PER_ROW, c4 = (piece % PER_ROW) * 4;
-            const int row = row_base + r, col = col0 + c4;
-            const float4 a4 = *reinterpret_cast<const float4*>(scratch + r * WCOLS + (c4 ^ read_swizzle(r, 2)));
-            float x[4] = {a4.x, a4.y, a4.z, a4.w};
-            if (row < row_limit && col < p.n) {
-              const size_t o = (size_t)row * p.n + col;
-#pragma unroll
-              for (int j = 0; j < 4; ++j) x[j] = p.alpha * x[j];
-              if (use_c) {
-                if (p.c_f16) {
-                  const half4_t cv = __builtin_bit_cast(half4_t, u32x2_t{c_raw[it][0], c_raw[it][1]});
-#pragma unroll
-                  for (int j = 0; j < 4; ++j) x[j] = x[j] + p.beta * (float)cv[j];
-                } else {
-#pragma unroll
-                  for (int j = 0; j < 4; ++j) x[j] = x[j] + p.beta * __builtin_bit_cast(float, c_raw[it][j]);
-                }
-              }
-              *reinterpret_cast<float4*>(reinterpret_cast<float*>(d_out) + o) = float4{x[0], x[1], x[2], x[3]};
-            }
-          }
-        }
-      }
+      };
+      if (p.alpha != 1.f) packed_turn(std::true_type{});
+      else packed_turn(std::false_type{});
       return;
     }
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm) {
+      if (!finishes(fm)) continue;  // the other K group stores this fragment
+      const int row_base = row0 + fm * 32;
+      if (p.d_f16) {
+        constexpr int PER_ROW = WCOLS / 8;           // 16-byte pieces (8 halves) per row
+        constexpr int ITERS = 32 * PER_ROW / 64;
+        uint32_t c_raw[ITERS][8];                    // fp16 C: one 16-byte load per piece (words 0-3); fp32 C: two
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+          const int piece = it * 64 + lane;
+          const int row = row_base + piece / PER_ROW, col = col0 + (piece % PER_ROW) * 8;
+          u32x4_t lo = u32x4_t{0, 0, 0, 0}, hi = u32x4_t{0, 0, 0, 0};
+          if (use_c && row < row_limit && col + 8 <= p.n) {
+            const size_t o = (size_t)row * p.n + col;
+            if (p.c_f16) {
+              lo = *reinterpret_cast<const u32x4_any_t*>(reinterpret_cast<const _Float16*>(p.c) + o);
+            } else {
+              lo = *reinterpret_cast<const u32x4_any_t*>(reinterpret_cast<const float*>(p.c) + o);
+              hi = *reinterpret_cast<const u32x4_any_t*>(reinterpret_cast<const float*>(p.c) + o + 4);
+            }
+          }
+          c_raw[it][0] = lo.x; c_raw[it][1] = lo.y; c_raw[it][2] = lo.z; c_raw[it][3] = lo.w;
+          c_raw[it][4] = hi.x; c_raw[it][5] = hi.y; c_raw[it][6] = hi.z; c_raw[it][7] = hi.w;
+        }
+        store_rows(fm);
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+          const int piece = it * 64 + lane;
+          const int r = piece / PER_ROW, c8 = (piece % PER_ROW) * 8;
+          const int row = row_base + r, col = col0 + c8;
+          const int sw = read_swizzle(r, 2);
+          const float4 lo = *reinterpret_cast<const float4*>(scratch + r * WCOLS + (c8 ^ sw));
+          const float4 hi = *reinterpret_cast<const float4*>(scratch + r * WCOLS + ((c8 + 4) ^ sw));
+          float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+          if (row < row_limit && col + 8 <= p.n) {
+            const size_t o = (size_t)row * p.n + col;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] = p.alpha * x[j];
+            if (use_c) {
+              if (p.c_f16) {
+                const half8_t cv =
+                    __builtin_bit_cast(half8_t, u32x4_t{c_raw[it][0], c_raw[it][1], c_raw[it][2], c_raw[it][3]});
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x[j] = x[j] + p.beta * (float)cv[j];
+              } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x[j] = x[j] + p.beta * __builtin_bit_cast(float, c_raw[it][j]);
+              }
+            }
+            half8_t out;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) out[j] = (_Float16)x[j];
+            *reinterpret_cast<u32x4_any_t*>(reinterpret_cast<_Float16*>(d_out) + o) = __builtin_bit_cast(u32x4_t, out);
+          }
+        }
+        cut_rows(row_base, 8, [&](int r, int c) { return p.alpha * scratch[r * WCOLS + (c ^ read_swizzle(r, 2))]; });
+      } else {
+        constexpr int PER_ROW = WCOLS / 4;           // 16-byte pieces (4 floats) per row
+        constexpr int ITERS = 32 * PER_ROW / 64;
+        uint32_t c_raw[ITERS][4];                    // fp32 C: one 16-byte load per piece; fp16 C: one 8-byte load
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+          const int piece = it * 64 + lane;
+          const int row = row_base + piece / PER_ROW, col = col0 + (piece % PER_ROW) * 4;
+          u32x4_t lo = u32x4_t{0, 0, 0, 0};
+          if (use_c && row < row_limit && col + 4 <= p.n) {
+            const size_t o = (size_t)row * p.n + col;
+            if (p.c_f16) {
+              const u32x2_t t = *reinterpret_cast<const u32x2_any_t*>(reinterpret_cast<const _Float16*>(p.c) + o);
+              lo.x = t.x; lo.y = t.y;
+            } else {
+              lo = *reinterpret_cast<const u32x4_any_t*>(reinterpret_cast<const float*>(p.c) + o);
+            }
+          }
+          c_raw[it][0] = lo.x; c_raw[it][1] = lo.y; c_raw[it][2] = lo.z; c_raw[it][3] = lo.w;
+        }
+        store_rows(fm);
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+          const int piece = it * 64 + lane;
+          const int r = piece / PER_ROW, c4 = (piece % PER_ROW) * 4;
+          const int row = row_base + r, col = col0 + c4;
+          const float4 a4 = *reinterpret_cast<const float4*>(scratch + r * WCOLS + (c4 ^ read_swizzle(r, 2)));
+          float x[4] = {a4.x, a4.y, a4.z, a4.w};
+          if (row < row_limit && col + 4 <= p.n) {
+            const size_t o = (size_t)row * p.n + col;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x[j] = p.alpha * x[j];
+            if (use_c) {
+              if (p.c_f16) {
+                const half4_t cv = __builtin_bit_cast(half4_t, u32x2_t{c_raw[it][0], c_raw[it][1]});
+#pragma unroll
+                for (int j = 0; j < 4; ++j) x[j] = x[j] + p.beta * (float)cv[j];
+              } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) x[j] = x[j] + p.beta * __builtin_bit_cast(float, c_raw[it][j]);
+              }
+            }
+            *reinterpret_cast<u32x4_any_t*>(reinterpret_cast<float*>(d_out) + o) =
+                __builtin_bit_cast(u32x4_t, float4{x[0], x[1], x[2], x[3]});
+          }
+        }
+        cut_rows(row_base, 4, [&](int r, int c) { return p.alpha * scratch[r * WCOLS + (c ^ read_swizzle(r, 2))]; });
+      }
+    }
+    return;
   }
-  // Direct form (generic variant, or C / D not 16-byte aligned): one element per accumulator register.
+  // Direct form (generic variant): one element per accumulator register.
   auto finish_element = [&](int row, int col, float sum) __attribute__((always_inline)) {
     if (row < row_limit && col < p.n) {
       const size_t o = (size_t)row * p.n + col;
@@ -1191,16 +1215,6 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
       else reinterpret_cast<float*>(d_out)[o] = x;
     }
   };
-  if constexpr (M16) {
-#pragma unroll
-    for (int rt = 0; rt < 2 * FM; ++rt)
-#pragma unroll
-      for (int ct = 0; ct < 2 * FN; ++ct)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          finish_element(row0 + rt * 16 + 4 * (lane >> 4) + v, col0 + ct * 16 + (lane & 15), acc16[rt][ct][v]);
-    return;
-  }
   const int col_lane = lane & 31;
   const int row_lane = 4 * (lane >> 5);
 #pragma unroll
@@ -1820,21 +1834,50 @@ __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_group_kernel
 }
 
 // =====================================================================================================
-// pad_b_kernel: copies B (k x n, row stride n, any alignment) into rows of ldb = round_up(n, 8) halves, zeros in the
-// padding columns, so that every row starts 16-byte aligned for the asynchronous copies of the main kernel.
-// One thread per 16-byte piece of the destination.
+// pad_b_kernel: copies B (k x n, row stride n, any alignment) into rows of ldb = round_up(n, 8) halves, so that every row starts 16-byte aligned for the asynchronous copies of the main kernel.
+// Bound: memory, 2 k n bytes each way (and a few us of launch and latency below about 10 MB). A workgroup takes `rows`
+// whole rows, as many as fit its 1024 pieces, or 1024 pieces of one longer row, so that neighbouring lanes write
+// neighbouring pieces across row ends; the four loads of a thread, 16 bytes at any alignment, come before its first store.
+// Against two-byte loads, one piece per thread (us): 4096 x 1001 9.0 -> 7.0, 20864 x 707 18.3 -> 12.0, 12832 x 3241 41.7 -> 29.3.
 // =====================================================================================================
-__global__ __launch_bounds__(256) void pad_b_kernel(const _Float16* __restrict__ b, _Float16* __restrict__ dst, int k,
-                                                    int n, int ldb) {
-  const int pieces_per_row = ldb / 8;
-  const size_t piece = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (piece >= (size_t)k * pieces_per_row) return;
-  const size_t row = piece / pieces_per_row;
-  const int col0 = (int)(piece % pieces_per_row) * 8;
-  half8_t v;
+constexpr int kPadPieces = 1024;
+
+// The eight halves of v from number `count` on (1 ... 7, or more: none), zeros behind them.
+__device__ __forceinline__ u32x4_t drop_halves(u32x4_t v, int count) {
+  u32x4_t r = u32x4_t{0, 0, 0, 0};
 #pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = col0 + j < n ? b[row * n + col0 + j] : (_Float16)0.f;
-  *reinterpret_cast<half8_t*>(dst + row * ldb + col0) = v;
+  for (int j = 0; j < 8; ++j) {
+#pragma unroll
+    for (int from = 1; from < 8; ++from)
+      if (from > j && from - j == count) r[j / 2] |= ((v[from / 2] >> (16 * (from % 2))) & 0xFFFFu) << (16 * (j % 2));
+  }
+  return r;
+}
+
+// rows > 1: reciprocal = 2^32 / (ldb / 8) + 1, with which the quotients below 2^11 that occur are exact
+__global__ __launch_bounds__(256) void pad_b_kernel(const _Float16* __restrict__ b, _Float16* __restrict__ dst, int k,
+                                                    int n, int ldb, int rows, uint32_t reciprocal) {
+  const int row0 = blockIdx.x * rows, per_row = ldb / 8, piece0 = blockIdx.y * kPadPieces;
+  const size_t last_start = (size_t)k * n - 8;  // k >= 32
+  u32x4_t v[kPadPieces / 256];
+#pragma unroll
+  for (int i = 0; i < kPadPieces / 256; ++i) {
+    const int local = threadIdx.x + 256 * i;
+    const int r = rows > 1 ? (int)__umulhi(local, reciprocal) : 0, col = 8 * (piece0 + local - r * per_row);
+    // a piece that reaches past the end of its row takes the next row's first values along: nothing is made of them, they
+    // only meet columns that are never stored. Past the end of B it is moved back and shifted into place below.
+    const size_t start = (size_t)(row0 + r) * n + col;
+    v[i] = *reinterpret_cast<const u32x4_any_t*>(b + (start <= last_start ? start : last_start));
+  }
+#pragma unroll
+  for (int i = 0; i < kPadPieces / 256; ++i) {
+    const int local = threadIdx.x + 256 * i;
+    const int r = rows > 1 ? (int)__umulhi(local, reciprocal) : 0, col = 8 * (piece0 + local - r * per_row);
+    const int row = row0 + r;
+    if (r >= rows || row >= k || col >= ldb) continue;
+    if (row == k - 1 && col + 8 > n) v[i] = drop_halves(v[i], col + 8 - n);
+    *reinterpret_cast<u32x4_t*>(dst + (size_t)row * ldb + col) = v[i];
+  }
 }
 
 // =====================================================================================================
@@ -1944,9 +1987,6 @@ static hipError_t launch_gemm_cfg(GemmArgs args, hipStream_t stream) {
 
 static hipError_t launch_gemm_pass(GemmArgs args, int tile_config, hipStream_t stream) {
   const bool aligned = (args.ldb % 8 == 0) && ((reinterpret_cast<uintptr_t>(args.b) & 15) == 0);
-  // the coalesced epilogue moves 16 bytes per lane: n % 8 == 0 keeps every row start aligned when the bases are
-  args.vector_epilogue = args.n % 8 == 0 && (reinterpret_cast<uintptr_t>(args.d) & 15) == 0 &&
-                         (args.beta == 0.f || (reinterpret_cast<uintptr_t>(args.c) & 15) == 0);
   if (!aligned) return launch_gemm_cfg<4, 1, 1, 4, false>(args, stream);
   switch (tile_config) {
     case kTile512x128: return launch_gemm_cfg<4, 1, 4, 4, true>(args, stream);
@@ -2017,9 +2057,10 @@ hipError_t launch_gemm(GemmArgs args, int tile_config, hipStream_t stream) {
   const bool aligned = (args.n % 8 == 0) && ((reinterpret_cast<uintptr_t>(args.b) & 15) == 0);
   if (!aligned && args.b_pad) {
     const int ldb = (args.n + 7) / 8 * 8;
-    const size_t pieces = (size_t)args.k * (ldb / 8);
-    hipLaunchKernelGGL(pad_b_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, stream, args.b, args.b_pad,
-                       args.k, args.n, ldb);
+    const int per_row = ldb / 8, rows = per_row > 1 && per_row < kPadPieces ? kPadPieces / per_row : 1;
+    hipLaunchKernelGGL(pad_b_kernel, dim3((args.k + rows - 1) / rows, (per_row + kPadPieces - 1) / kPadPieces), dim3(256), 0,
+                       stream, args.b, args.b_pad, args.k, args.n, ldb, rows,
+                       (uint32_t)((uint64_t(1) << 32) / per_row + 1));
     if (hipError_t st = hipGetLastError(); st != hipSuccess) return st;
     args.b = args.b_pad;
     args.ldb = ldb;

@@ -1,0 +1,46 @@
+"""Products whose number of columns is no multiple of the 16-byte vectors: rows of C and D start at any element, the last
+piece of a row is cut short, the last one of C lies at the end of its memory. Integer operands: bit-exact."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from onebitsparsemul_amd import _native, synthetic
+
+pytestmark = pytest.mark.gpu
+
+
+def guarded(values, shift):
+    """A copy of `values` on the GPU, `shift` elements into a buffer that ends with it exactly; the buffer too."""
+    flat = torch.full((values.numel() + shift,), 7.0, dtype=values.dtype, device="cuda")
+    flat[shift:] = values.reshape(-1).cuda()
+    return flat[shift:].view(values.shape), flat
+
+
+@pytest.mark.parametrize("tile,m,k", [(9, 576, 288), (10, 320, 544), (4, 320, 288), (6, 192, 288), (13, 192, 544), (14, 128, 544),
+                                      (15, 576, 288)])
+@pytest.mark.parametrize("n", [65, 127, 131, 257])
+def test_main_kernel_ragged_rows(tile, m, k, n):
+    _native.set_tile_config(tile)
+    _native.set_skinny_enabled(False)
+    try:
+        a, meta = synthetic.make_weight(m, k, seed=tile + n)
+        prepared = _native.prepare(a.cuda(), meta.cuda(), m, k)
+        b = synthetic.make_b(k, n, seed=n, kind="int")
+        c = torch.from_numpy(np.random.default_rng(n).integers(-8, 9, (m, n))).to(torch.float32)
+        for c_type, out, shift in ((None, torch.float16, 1), (torch.float16, torch.float16, 3), (torch.float32, torch.float16, 0),
+                                   (torch.float16, torch.float32, 1), (torch.float32, torch.float32, 3), (None, torch.float32, 0)):
+            c_gpu = None if c_type is None else guarded(c.to(c_type), shift)[0]
+            d, flat = guarded(torch.zeros((m, n), dtype=out), shift)
+            _native.matmul_prepared(prepared, guarded(b, shift)[0], d, m, n, k, c=c_gpu, alpha=0.5 if c_type else 1.0,
+                                    beta=0.0 if c_type is None else 2.0)
+            torch.cuda.synchronize()
+            want = oracle.reference_matmul(a.numpy(), b.numpy(), meta.numpy(), m, n, k,
+                                           c=None if c_type is None else c.numpy(), alpha=0.5 if c_type else 1.0,
+                                           beta=0.0 if c_type is None else 2.0,
+                                           d_dtype=oracle.F16 if out == torch.float16 else oracle.F32)
+            assert np.array_equal(d.cpu().numpy(), want), (c_type, out, shift)
+            assert bool((flat[:shift] == 7.0).all())
+    finally:
+        _native.set_tile_config(-1)
+        _native.set_skinny_enabled(True)
