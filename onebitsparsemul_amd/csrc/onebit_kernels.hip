@@ -1246,8 +1246,12 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
 // =====================================================================================================
 constexpr int kSkinnyRegion = 8192;  // bytes of one B image
 
-// how B rows reach the image: whole rows are the image rows (n == NC), rows of n % 8 == 0 elements in 16-byte
-// pieces padded to the image row, 8-byte rows (n == 4, NC == 16), or element by element (any n <= NC, any alignment)
+// How B rows reach the image. kSkinnyBFull: n == NC, 16-byte aligned, whole images are consecutive memory. kSkinnyBAny: any
+// n, any alignment: 16-byte pieces, ceil(n / 8) per row, loaded from wherever the row starts (gfx950 loads 16 bytes at any
+// address). A piece that reaches past its row's end takes the next row's first elements along; they land in columns at or
+// past n, whose results are never stored, so nothing has to be cleared or masked. It replaced element copies and two modes
+// of checked pieces (us inside a HIP graph): 14016 x 14 x 7136 43.2 -> 9.2, 11008 x 15 x 4096 23.1 -> 8.5, 4096 x 33 x 4096
+// 27.8 -> 12.1, 11008 x 63 x 4096 51.1 -> 14.5; n % 8 == 0: 11008 x 8 x 4096 5.8 -> 5.2, 28672 x 40 x 8192 40.8 -> 32.6.
 // kSkinnyBTokens: the token-major form of the linear layer. B is x, n rows (tokens) of k consecutive values, and
 // the result is written as y[token][weight row] (+ bias[weight row]). The image is then token-major too: row t holds
 // the image's K range of token t in 16-byte pieces, piece p stored at position p ^ token_swizzle(t) so that lanes
@@ -1257,33 +1261,16 @@ constexpr int kSkinnyRegion = 8192;  // bytes of one B image
 // loaded in 16-byte pieces (32 n of them: at most two load instructions per wavefront and chunk, where the row-wise
 // modes issue eight; the split-K kernel's time is set by the number of load instructions it issues) and spread over the image rows
 // by LDS stores of 2 n bytes.
-enum SkinnyBMode { kSkinnyBFull = 0, kSkinnyB8 = 1, kSkinnyB4 = 2, kSkinnyBScalar = 3, kSkinnyBTokens = 4, kSkinnyBRun = 5 };
+enum SkinnyBMode { kSkinnyBFull = 0, kSkinnyBAny = 1, kSkinnyBTokens = 2, kSkinnyBRun = 3 };
 
-// 16-byte piece q of the image whose first row is B row k_base: image row q / (NC / 8), columns 8 (q % (NC / 8))
-// ... + 7; zero outside B. Vector modes only.
-template <int NC>
-__device__ __forceinline__ u32x4_t skinny_load_piece(const _Float16* __restrict__ b, int n, int mode, int k_base,
-                                                      int rows_valid, int q) {
-  constexpr int PPR = NC / 8;  // pieces per image row
-  const int row = q / PPR, h = q % PPR;
-  const bool ok = row < rows_valid;
-  const char* base = reinterpret_cast<const char*>(b);
-  u32x4_t v = u32x4_t{0, 0, 0, 0};
-  if (mode == kSkinnyBFull) {
-    const char* src = ok ? base + ((size_t)k_base * NC + (size_t)q * 8) * 2 : base;
-    v = *reinterpret_cast<const u32x4_t*>(src);
-    if (!ok) v = u32x4_t{0, 0, 0, 0};
-  } else if (mode == kSkinnyB8) {
-    const bool use = ok && 8 * h < n;
-    const char* src = use ? base + ((size_t)(k_base + row) * n + 8 * h) * 2 : base;
-    v = *reinterpret_cast<const u32x4_t*>(src);
-    if (!use) v = u32x4_t{0, 0, 0, 0};
-  } else {  // kSkinnyB4
-    const bool use = ok && h == 0;
-    const char* src = use ? base + (size_t)(k_base + row) * 8 : base;
-    const u32x2_t t = *reinterpret_cast<const u32x2_t*>(src);
-    if (use) v = u32x4_t{t.x, t.y, 0, 0};
-  }
+// The eight halves of v from number `count` on, zeros behind them (count >= 8: zeros).
+__device__ __forceinline__ u32x4_t drop_halves(u32x4_t v, int count) {
+  if (count >= 8) return u32x4_t{0, 0, 0, 0};
+  if (count & 4) v = u32x4_t{v.z, v.w, 0, 0};
+  if (count & 2) v = u32x4_t{v.y, v.z, v.w, 0};
+  if (count & 1)
+    v = u32x4_t{__builtin_amdgcn_alignbyte(v.y, v.x, 2), __builtin_amdgcn_alignbyte(v.z, v.y, 2),
+                __builtin_amdgcn_alignbyte(v.w, v.z, 2), v.w >> 16};
   return v;
 }
 
@@ -1298,7 +1285,6 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   constexpr int NF = NC <= 32 ? 1 : NC / 32;           // 32-column fragments per image row
   constexpr int TILE_BYTES = kRowBlock * NC * 4;       // one fp32 partial tile
   static_assert(NC == 16 || NC == 32 || NC == 64, "image width");
-  static_assert(MODE != kSkinnyB4 || NC == 16, "the 8-byte-row mode is for 16 columns");
   static_assert(MODE != kSkinnyBRun || NC == 16, "the run mode is for 16 columns");
   // the partial tiles reuse the wavefront's image memory, RT row blocks per round of the final reduction
   constexpr int RT = R * TILE_BYTES <= kSkinnyRegion ? R : kSkinnyRegion / TILE_BYTES;
@@ -1348,7 +1334,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   const int first = kc_begin + wave;  // this wavefront's first chunk
   // Short K (at most two chunks per wavefront, e.g. 11008 x 4096): everything the wavefront will read is requested
   // at once, so the kernel pays one memory latency instead of one per chunk.
-  constexpr bool kShortPath = NW <= 8 && SUB == 1 && MODE != kSkinnyBScalar;
+  constexpr bool kShortPath = NW <= 8 && SUB == 1;
   const bool short_k = kShortPath && kc_end - kc_begin <= 2 * NW;
   // The prepared operand comes from HBM and is what the first SMFMAC waits for longest: the loop form issues its first
   // loads here, before the rest of the set-up (B descriptor, image offsets, fragment addresses), which then runs under
@@ -1366,14 +1352,14 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
     const int rows = k_rows - k_base;
     return rows < 0 ? 0 : (rows > IMG_ROWS ? IMG_ROWS : rows);
   };
-  // element mode: image position of element `lane` of an image's run of IMG_ROWS * n elements, and the step of 64
-  const int elem_col0 = lane % n_cols;
-  const int elem_offset0 = (lane / n_cols) * ROW_BYTES + elem_col0 * 2;
-  const int step_cols = 64 % n_cols;
-  const int step_bytes = (64 / n_cols) * ROW_BYTES + step_cols * 2;
+  // pieces at any alignment: a load instruction covers any_rows whole rows, lane = (row, piece) of them
+  const int any_pieces = (n_cols + 7) / 8, any_rows = 64 / any_pieces;
+  const int any_row = lane / any_pieces, any_piece = lane % any_pieces;
+  const bool any_used = any_row < any_rows;
+  const uint32_t any_load = (uint32_t)(any_row * n_cols + 8 * any_piece) * 2u, any_load_step = (uint32_t)(any_rows * n_cols) * 2u;
+  const uint32_t any_store = (uint32_t)any_row * ROW_BYTES + 16u * any_piece;
   // Image t of this wavefront = B rows [k_base, k_base + IMG_ROWS) with k_base = (wave + NW (t / SUB)) * 256 +
-  // (t % SUB) * IMG_ROWS. Vector modes: the image travels through registers, loaded while the previous image is
-  // multiplied; element mode: loaded and stored in one go when the image is due.
+  // (t % SUB) * IMG_ROWS. The image travels through registers, loaded while the previous image is multiplied.
   // token-major image: piece lane + 64 i = K values [8 p, 8 p + 8) of the image for token token_lane + TPI i
   const int piece_lane = lane % PPT, token_lane = lane / PPT;
   const uint32_t token_load_base = ((uint32_t)token_lane * (uint32_t)k_rows + 8u * piece_lane) * 2u;
@@ -1383,7 +1369,6 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   // run mode: piece q = lane + 64 i of the image's run; pieces at or past 32 n are sent outside the descriptor (zero)
   const uint32_t run_pieces = 32u * (uint32_t)n_cols;
   auto load_b = [&](int k_base, u32x4_t (&v)[8]) __attribute__((always_inline)) {
-    if (MODE == kSkinnyBScalar) return;
     if (MODE == kSkinnyBRun) {
       const uint32_t run_base = (uint32_t)k_base * (uint32_t)n_cols * 2u;  // the launcher checks k n 2 < 2^32
       if (k_base + IMG_ROWS <= k_rows) {
@@ -1426,47 +1411,57 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
       }
       return;
     }
-    if (MODE == kSkinnyBFull && b_fits && k_base + IMG_ROWS <= k_rows) {
-      // the whole image lies inside B (wave-uniform test): 8 KiB of consecutive memory, no per-piece checks
-      const uint32_t image = (uint32_t)k_base * (NC * 2);
+    if (MODE == kSkinnyBFull) {
+      if (b_fits && k_base + IMG_ROWS <= k_rows) {
+        // the whole image lies inside B (wave-uniform test): 8 KiB of consecutive memory, no per-piece checks
+        const uint32_t image = (uint32_t)k_base * (NC * 2);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = buffer_load16(b_buffer, meta_off + 1024u * i, image);
+        for (int i = 0; i < 8; ++i) v[i] = buffer_load16(b_buffer, meta_off + 1024u * i, image);
+        return;
+      }
+      const int rows_valid = rows_valid_of(k_base);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int q = lane + i * 64;
+        const bool ok = q / (NC / 8) < rows_valid;
+        v[i] = *reinterpret_cast<const u32x4_t*>(b_ptr + (ok ? (size_t)k_base * NC + (size_t)q * 8 : 0));
+        if (!ok) v[i] = u32x4_t{0, 0, 0, 0};
+      }
       return;
     }
-    const int rows_valid = rows_valid_of(k_base);
+    // (wave-uniform) rows from the image's first on, as far as they matter: none past the end of K
+    const int rows_left = k_rows - k_base < IMG_ROWS + 8 ? k_rows - k_base : IMG_ROWS + 8;
+    if (rows_left <= 0) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = skinny_load_piece<NC>(b_ptr, n_cols, MODE, k_base, rows_valid, lane + i * 64);
+      for (int i = 0; i < 8; ++i) v[i] = u32x4_t{0, 0, 0, 0};
+      return;
+    }
+    // lane offsets that do not change from image to image; lanes without a piece and pieces that would end past the rows
+    // left (the last image's, k % 32 == 0: at least 32 rows) load the last whole piece instead
+    const char* image = reinterpret_cast<const char*>(b_ptr + (size_t)k_base * n_cols);
+    const uint32_t last = (uint32_t)(rows_left * n_cols - 8) * 2u;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i * any_rows < IMG_ROWS) {
+        const uint32_t offset = any_load + i * any_load_step;
+        v[i] = *reinterpret_cast<const u32x4_any_t*>(image + (offset < last ? offset : last));
+      }
+    if (rows_left < IMG_ROWS + 8) {
+      // last image: what was read from the last whole piece is shifted into place, rows at or past K are zeros
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (i * any_rows < IMG_ROWS) {
+          const uint32_t offset = any_load + i * any_load_step;
+          if (offset > last) v[i] = drop_halves(v[i], (int)(offset - last) / 2);
+        }
+    }
   };
   auto store_b = [&](int k_base, const u32x4_t (&v)[8]) __attribute__((always_inline)) {
-    if (MODE == kSkinnyBScalar) {
-      // the image's rows are one run of IMG_ROWS n elements; rows at or past K are written as zeros, the padding
-      // columns n ... NC - 1 keep the zeros the image was cleared to
-      const int valid = rows_valid_of(k_base) * n_cols, total = IMG_ROWS * n_cols;
-      const _Float16* src = b_ptr + (size_t)k_base * n_cols;
-      constexpr int BATCH = NC >= 32 ? 16 : 4;  // loads in flight per lane
-      int offset = elem_offset0;  // byte offset in the image of element e = lane + 64 i, kept without divisions
-      int col = elem_col0;
-      for (int e0 = lane; e0 < total; e0 += 64 * BATCH) {
-        uint16_t bits[BATCH];
+    if (MODE == kSkinnyBAny) {
 #pragma unroll
-        for (int i = 0; i < BATCH; ++i) {
-          const int e = e0 + i * 64;
-          bits[i] = __builtin_bit_cast(uint16_t, e < valid ? src[e] : b_ptr[0]);
-          if (e >= valid) bits[i] = 0;
-        }
-#pragma unroll
-        for (int i = 0; i < BATCH; ++i) {
-          const int e = e0 + i * 64;
-          if (e < total) *reinterpret_cast<uint16_t*>(region + offset) = bits[i];
-          // e += 64: 64 / n rows further and 64 % n columns, with one carry at most
-          col += step_cols;
-          offset += step_bytes;
-          if (col >= n_cols) {
-            col -= n_cols;
-            offset += ROW_BYTES - n_cols * 2;
-          }
-        }
-      }
+      for (int i = 0; i < 8; ++i)
+        if (i * any_rows < IMG_ROWS && any_used && any_row + i * any_rows < IMG_ROWS)
+          *reinterpret_cast<u32x4_t*>(region + any_store + i * any_rows * ROW_BYTES) = v[i];
       return;
     }
     if (MODE == kSkinnyBRun) {
@@ -1677,8 +1672,8 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   };
 
   // sixteen wavefronts leave 128 registers each: no room to hold the next image (32 registers) during the SMFMACs
-  constexpr bool kPrefetchB = NW <= 8 && MODE != kSkinnyBScalar;
-  if (MODE == kSkinnyBScalar || MODE == kSkinnyBRun) {
+  constexpr bool kPrefetchB = NW <= 8;
+  if (MODE == kSkinnyBRun) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) *reinterpret_cast<u32x4_t*>(region + (lane + i * 64) * 16) = u32x4_t{0, 0, 0, 0};
   }
@@ -1841,18 +1836,6 @@ __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_group_kernel
 // Against two-byte loads, one piece per thread (us): 4096 x 1001 9.0 -> 7.0, 20864 x 707 18.3 -> 12.0, 12832 x 3241 41.7 -> 29.3.
 // =====================================================================================================
 constexpr int kPadPieces = 1024;
-
-// The eight halves of v from number `count` on (1 ... 7, or more: none), zeros behind them.
-__device__ __forceinline__ u32x4_t drop_halves(u32x4_t v, int count) {
-  u32x4_t r = u32x4_t{0, 0, 0, 0};
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-#pragma unroll
-    for (int from = 1; from < 8; ++from)
-      if (from > j && from - j == count) r[j / 2] |= ((v[from / 2] >> (16 * (from % 2))) & 0xFFFFu) << (16 * (j % 2));
-  }
-  return r;
-}
 
 // rows > 1: reciprocal = 2^32 / (ldb / 8) + 1, with which the quotients below 2^11 that occur are exact
 __global__ __launch_bounds__(256) void pad_b_kernel(const _Float16* __restrict__ b, _Float16* __restrict__ dst, int k,
@@ -2095,28 +2078,23 @@ static hipError_t launch_skinny_mode(const SkinnyArgs& args, hipStream_t stream)
 
 template <int NW, int R>
 static hipError_t launch_skinny_cfg(const SkinnyArgs& args, hipStream_t stream) {
-  const uintptr_t address = reinterpret_cast<uintptr_t>(args.b);
+  const bool aligned = (reinterpret_cast<uintptr_t>(args.b) & 15) == 0;
   if (args.n > 32) {  // 64-column images, two column fragments: at most two row blocks fit the registers
     constexpr int R64 = R > 2 ? 2 : R;
-    if (args.n == 64 && (address & 15) == 0) return launch_skinny_mode<NW, R64, kSkinnyBFull, 64>(args, stream);
-    if (args.n % 8 == 0 && (address & 15) == 0) return launch_skinny_mode<NW, R64, kSkinnyB8, 64>(args, stream);
-    return launch_skinny_mode<NW, R64, kSkinnyBScalar, 64>(args, stream);
+    if (args.n == 64 && aligned) return launch_skinny_mode<NW, R64, kSkinnyBFull, 64>(args, stream);
+    return launch_skinny_mode<NW, R64, kSkinnyBAny, 64>(args, stream);
   }
   if (args.n > 16) {  // 32-column images
-    constexpr int R32 = R;
-    if (args.n == 32 && (address & 15) == 0) return launch_skinny_mode<NW, R32, kSkinnyBFull, 32>(args, stream);
-    if (args.n % 8 == 0 && (address & 15) == 0) return launch_skinny_mode<NW, R32, kSkinnyB8, 32>(args, stream);
-    return launch_skinny_mode<NW, R32, kSkinnyBScalar, 32>(args, stream);
+    if (args.n == 32 && aligned) return launch_skinny_mode<NW, R, kSkinnyBFull, 32>(args, stream);
+    return launch_skinny_mode<NW, R, kSkinnyBAny, 32>(args, stream);
   }
-  if (args.n == 16 && (address & 15) == 0) return launch_skinny_mode<NW, R, kSkinnyBFull, 16>(args, stream);
-  if (args.n == 8 && (address & 15) == 0) return launch_skinny_mode<NW, R, kSkinnyB8, 16>(args, stream);
+  if (args.n == 16 && aligned) return launch_skinny_mode<NW, R, kSkinnyBFull, 16>(args, stream);
   // one column: B is a token-major x of one token and D is its y (same memory in both layouts)
-  if (args.n == 1 && (address & 15) == 0 && (size_t)args.k * 64 * 2 < 0xFFFFFF00u)
+  if (args.n == 1 && aligned && (size_t)args.k * 64 * 2 < 0xFFFFFF00u)
     return launch_skinny_mode<NW, R, kSkinnyBTokens, 16>(args, stream);
-  if ((args.n == 2 || args.n == 4) && (address & 15) == 0 && (size_t)args.k * args.n * 2 < 0xFFFFFF00u)
+  if ((args.n == 2 || args.n == 4) && aligned && (size_t)args.k * args.n * 2 < 0xFFFFFF00u)
     return launch_skinny_mode<NW, R, kSkinnyBRun, 16>(args, stream);
-  if (args.n == 4 && (address & 7) == 0) return launch_skinny_mode<NW, R, kSkinnyB4, 16>(args, stream);
-  return launch_skinny_mode<NW, R, kSkinnyBScalar, 16>(args, stream);
+  return launch_skinny_mode<NW, R, kSkinnyBAny, 16>(args, stream);
 }
 
 template <int NW, int R>

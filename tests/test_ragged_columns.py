@@ -44,3 +44,23 @@ def test_main_kernel_ragged_rows(tile, m, k, n):
     finally:
         _native.set_tile_config(-1)
         _native.set_skinny_enabled(True)
+
+
+@pytest.mark.parametrize("rows", [32, 64, 128])
+@pytest.mark.parametrize("n", [1, 3, 4, 7, 8, 9, 15, 17, 24, 25, 33, 40, 49, 63])
+def test_split_k_kernel_any_columns(rows, n):
+    """B rows that start at any element: every count of 16-byte pieces per row, the end of B inside a piece, K tails that leave
+    the last image with 32 rows or end it exactly."""
+    _native.set_skinny_rows(rows)
+    try:
+        for m, k, shift in ((192, 256, 1), (64, 2592, 0), (320, 4128, 3), (128, 512, 2)):
+            a, meta = synthetic.make_weight(m, k, seed=n + k)
+            prepared = _native.prepare(a.cuda(), meta.cuda(), m, k)
+            b = synthetic.make_b(k, n, seed=n, kind="int")
+            d = torch.full((m, n), float("nan"), dtype=torch.float16, device="cuda")
+            _native.matmul_prepared(prepared, guarded(b, shift)[0], d, m, n, k)
+            torch.cuda.synchronize()
+            want = oracle.reference_matmul(a.numpy(), b.numpy(), meta.numpy(), m, n, k)
+            assert np.array_equal(d.cpu().numpy(), want), (m, k, shift)
+    finally:
+        _native.set_skinny_rows(-1)
