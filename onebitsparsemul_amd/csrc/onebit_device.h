@@ -128,6 +128,25 @@ __device__ __forceinline__ u32x2_t lds_read_tr16(const void* lds_ptr) {
   return __builtin_bit_cast(u32x2_t, r);
 }
 
+// Position XOR of the 16-byte pieces of token row t in the token-major images: sixteen consecutive tokens that read the
+// same piece touch sixteen different 16-byte columns of the 256 bytes the LDS banks span (rows of 128 bytes: two rows
+// fill the span, so the XOR changes every second token; rows of 256 bytes or more: every token).
+template <int ROW_BYTES = 128>
+__device__ __forceinline__ constexpr int token_swizzle(int token) {
+  return ROW_BYTES >= 256 ? (token & 15) : ((token >> 1) & 7);
+}
+
+// The eight halves of v from number `count` on, zeros behind them (count >= 8: zeros).
+__device__ __forceinline__ u32x4_t drop_halves(u32x4_t v, int count) {
+  if (count >= 8) return u32x4_t{0, 0, 0, 0};
+  if (count & 4) v = u32x4_t{v.z, v.w, 0, 0};
+  if (count & 2) v = u32x4_t{v.y, v.z, v.w, 0};
+  if (count & 1)
+    v = u32x4_t{__builtin_amdgcn_alignbyte(v.y, v.x, 2), __builtin_amdgcn_alignbyte(v.z, v.y, 2),
+                __builtin_amdgcn_alignbyte(v.w, v.z, 2), v.w >> 16};
+  return v;
+}
+
 // ---- asynchronous global -> LDS copy --------------------------------------------------------------
 // global_load_lds_dwordx4: each lane fetches 16 bytes from its own global address; the wavefront's 1 KiB
 // lands at LDS offset M0 + 16 * lane. Issued through inline assembly so that the compiler does not

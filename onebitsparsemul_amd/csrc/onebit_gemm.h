@@ -1,12 +1,9 @@
-// gfx950 kernels of the one-bit 2:4 sparse GEMM  D = alpha * A * B + beta * C.
-//   gemm_kernel     : main SMFMAC kernel (B staged through LDS, A expanded in registers)
-//   skinny_kernel   : split-K kernel for N <= 64 (decode shapes)
-//   pad_b_kernel, splitk_reduce_kernel : helpers of the main kernel (unaligned B rows; K split over workgroups)
-// The kernels that bring a weight into these kernels' operand format are in onebit_format.hip.
-// The two GEMM kernels also come in a token-major form for the linear layer, y = x W^T + bias with x and y stored
-// token by token (the transposes of B and D).
-// Replaces the CUTLASS specialisations of the reference (csrc/kernel.h:13-72, csrc/threadblock.h:62-233,
-// csrc/warp.h:18-690) with code written for 64-wide wavefronts; nothing is translated from them.
+// The main SMFMAC kernel of the one-bit 2:4 sparse GEMM on gfx950, D = alpha * A * B + beta * C (B staged through LDS, A
+// expanded in registers), in its plain form and in the token-major form of the linear layer, y = x W^T + bias with x and y
+// stored token by token (the transposes of B and D), and the launch of one instantiation. onebit_gemm.hip and
+// onebit_gemm_tokens.hip instantiate it. Replaces the CUTLASS specialisations of the reference (csrc/kernel.h:13-72,
+// csrc/threadblock.h:62-233, csrc/warp.h:18-690) with code written for 64-wide wavefronts; nothing is translated from them.
+#pragma once
 #include "onebit_device.h"
 #include "onebit_launch.h"
 #include <atomic>
@@ -116,14 +113,6 @@ __device__ __forceinline__ void compute_stage(const char* stage_lds, const AChun
 // Token-major stage image (linear-layer form): row t = the stage's 64 K values of token t (128 bytes, eight 16-byte
 // pieces, piece p stored at position p ^ token_swizzle(t)). The operand of K step ks is pieces 4 ks + gb and 4 ks + 2 + gb of
 // the lane's token: two plain 16-byte reads at the precomputed lane offsets piece_off[2 ks + h].
-// Position XOR of the 16-byte pieces of token row t in the token-major images: sixteen consecutive tokens that read the
-// same piece touch sixteen different 16-byte columns of the 256 bytes the LDS banks span (rows of 128 bytes: two rows
-// fill the span, so the XOR changes every second token; rows of 256 bytes or more: every token).
-template <int ROW_BYTES = 128>
-__device__ __forceinline__ constexpr int token_swizzle(int token) {
-  return ROW_BYTES >= 256 ? (token & 15) : ((token >> 1) & 7);
-}
-
 // One packed register (kept values 2p, 2p+1 of K step STEP) of expand_signs. The empty volatile statement keeps the two
 // instructions where they are written: the optimizer otherwise sinks them past the stage's barrier to the block of their
 // first use.
@@ -175,7 +164,7 @@ __device__ __forceinline__ void mfma_frags_fused(const AChunk (&a)[FM], const u3
 }
 
 // Source of zeros for the asynchronous copies of B rows at or past K.
-__device__ __attribute__((aligned(16))) uint32_t g_zero16[4] = {0, 0, 0, 0};
+static __device__ __attribute__((aligned(16))) uint32_t g_zero16[4] = {0, 0, 0, 0};
 
 // TOKENS (with DMA only): the linear-layer form. p.b is x (p.n tokens x p.k, token-major), p.d is y (p.n tokens x
 // p.m), the epilogue is y = acc + bias; a tile column is a token.
@@ -1231,710 +1220,6 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
   }
 }
 
-// =====================================================================================================
-// skinny_kernel: N <= 64 (decode shapes). HBM-bound: every byte of the prepared operand is read once.
-// Workgroup = NW wavefronts that share R row blocks (32 rows each) and split K among themselves: wavefront w
-// takes the K chunks (of 256) w, w + NW, w + 2 NW, ... Each wavefront stages B rows in a private 8 KiB LDS region
-// as a zero-padded fp16 image of NC columns (NC = 16: the 256 rows of a chunk; NC = 32: 128 rows, two images per
-// chunk; NC = 64: 64 rows, four images, two column fragments), feeds them to SMFMAC through transpose reads (one fragment serves the R row blocks) and keeps a 32x32
-// fp32 partial tile per row block (NC = 16: two 16x16 tiles, multiplied with v_smfmac_f32_16x16x64_f16, which has no
-// idle columns at sixteen). The prepared operand and the next image are loaded into registers while the
-// current one is multiplied. Wavefronts never wait for one another inside the K loop (LDS operations of one
-// wavefront execute in order). The NW partial tiles of a row block are added through LDS in wavefront order
-// (deterministic; the tiles take the place of the images, as many row blocks per round as fit the 8 KiB) and the
-// epilogue is applied. grid = M / (32 R) workgroups; no global workspace, no atomics.
-// =====================================================================================================
-constexpr int kSkinnyRegion = 8192;  // bytes of one B image
-
-// How B rows reach the image. kSkinnyBFull: n == NC, 16-byte aligned, whole images are consecutive memory. kSkinnyBAny: any
-// n, any alignment: 16-byte pieces, ceil(n / 8) per row, loaded from wherever the row starts (gfx950 loads 16 bytes at any
-// address). A piece that reaches past its row's end takes the next row's first elements along; they land in columns at or
-// past n, whose results are never stored, so nothing has to be cleared or masked. It replaced element copies and two modes
-// of checked pieces (us inside a HIP graph): 14016 x 14 x 7136 43.2 -> 9.2, 11008 x 15 x 4096 23.1 -> 8.5, 4096 x 33 x 4096
-// 27.8 -> 12.1, 11008 x 63 x 4096 51.1 -> 14.5; n % 8 == 0: 11008 x 8 x 4096 5.8 -> 5.2, 28672 x 40 x 8192 40.8 -> 32.6.
-// kSkinnyBTokens: the token-major form of the linear layer. B is x, n rows (tokens) of k consecutive values, and
-// the result is written as y[token][weight row] (+ bias[weight row]). The image is then token-major too: row t holds
-// the image's K range of token t in 16-byte pieces, piece p stored at position p ^ token_swizzle(t) so that lanes
-// which read the same piece of consecutive tokens fall into different banks; a lane's SMFMAC operand is two plain
-// 16-byte reads (K consecutive inside a piece), no transpose.
-// kSkinnyBRun: n = 2 or 4 with B 16-byte aligned. The 256 rows of a chunk are one run of 512 n consecutive bytes,
-// loaded in 16-byte pieces (32 n of them: at most two load instructions per wavefront and chunk, where the row-wise
-// modes issue eight; the split-K kernel's time is set by the number of load instructions it issues) and spread over the image rows
-// by LDS stores of 2 n bytes.
-enum SkinnyBMode { kSkinnyBFull = 0, kSkinnyBAny = 1, kSkinnyBTokens = 2, kSkinnyBRun = 3 };
-
-// The eight halves of v from number `count` on, zeros behind them (count >= 8: zeros).
-__device__ __forceinline__ u32x4_t drop_halves(u32x4_t v, int count) {
-  if (count >= 8) return u32x4_t{0, 0, 0, 0};
-  if (count & 4) v = u32x4_t{v.z, v.w, 0, 0};
-  if (count & 2) v = u32x4_t{v.y, v.z, v.w, 0};
-  if (count & 1)
-    v = u32x4_t{__builtin_amdgcn_alignbyte(v.y, v.x, 2), __builtin_amdgcn_alignbyte(v.z, v.y, 2),
-                __builtin_amdgcn_alignbyte(v.w, v.z, 2), v.w >> 16};
-  return v;
-}
-
-// The body of the split-K kernel for workgroup (block_x, block_y) of problem p: block_x = row group, block_y = K split.
-template <int NW, int R, int MODE, int NC>
-__device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block_x, const int block_y) {
-  constexpr int NT = 64 * NW;
-  constexpr int IMG_ROWS = kSkinnyRegion / (NC * 2);   // B rows per image: 256, 128 or 64
-  constexpr int SUB = kChunkK / IMG_ROWS;              // images per chunk: 1, 2 or 4
-  constexpr int IMG_STEPS = kStepsPerChunk / SUB;      // 32-wide K steps per image: 8, 4 or 2
-  constexpr int ROW_BYTES = NC * 2;
-  constexpr int NF = NC <= 32 ? 1 : NC / 32;           // 32-column fragments per image row
-  constexpr int TILE_BYTES = kRowBlock * NC * 4;       // one fp32 partial tile
-  static_assert(NC == 16 || NC == 32 || NC == 64, "image width");
-  static_assert(MODE != kSkinnyBRun || NC == 16, "the run mode is for 16 columns");
-  // the partial tiles reuse the wavefront's image memory, RT row blocks per round of the final reduction
-  constexpr int RT = R * TILE_BYTES <= kSkinnyRegion ? R : kSkinnyRegion / TILE_BYTES;
-  static_assert(RT >= 1 && R % RT == 0, "the row blocks must divide into whole reduction rounds");
-  constexpr bool TOKENS = MODE == kSkinnyBTokens;
-  // Sixteen columns fill half of the 32x32x32 SMFMAC's result tile; v_smfmac_f32_16x16x64_f16 has no idle half and
-  // multiplies a row block's chunk in half the matrix-pipe time (eight instructions of four passes).
-  constexpr bool M16 = NC == 16;
-  constexpr int PPT = IMG_ROWS / 8;                    // token-major image: 16-byte pieces per token row
-  constexpr int TPI = 64 / PPT;                        // ... and tokens covered by the 64 pieces of one wavefront load
-  constexpr int TOKEN_ROW_BYTES = IMG_ROWS * 2;
-  __shared__ __attribute__((aligned(16))) char bs[NW * kSkinnyRegion];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int rb_total = p.m / kRowBlock;
-  const int rb_first = block_x * R;
-  char* region = bs + wave * kSkinnyRegion;
-  // kernel arguments the lambdas use, as values (capturing the argument struct would move it to scratch memory)
-  const _Float16* __restrict__ b_ptr = p.b;
-  const uint8_t* __restrict__ prep = p.prep;
-  const int n_cols = p.n, k_rows = p.k, kc_total = p.kc_total;
-
-  // The streaming loads go through buffer descriptors: wave-uniform base and offset in scalar registers, lane
-  // offsets in one vector register, no vector address arithmetic inside the K loop. One descriptor per row block
-  // (its kc_total blocks are consecutive, under 4 GiB for any K the argument checks admit) and one for B.
-  const uint32_t meta_off = (uint32_t)lane * 16u, sign_off = (uint32_t)kSignOffset + (uint32_t)lane * 8u;
-  buffer_t a_buffer[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    int rb = rb_first + r;
-    if (rb >= rb_total) rb = rb_total - 1;  // never stored
-    a_buffer[r] = make_buffer(prep + (size_t)rb * kc_total * kBlockBytes, (uint32_t)kc_total * kBlockBytes);
-  }
-  auto load_a = [&](int kc, AChunk (&a)[R]) __attribute__((always_inline)) {
-    if (kc >= kc_total) kc = kc_total - 1;  // never multiplied
-    const uint32_t block = (uint32_t)kc * kBlockBytes;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      a[r].meta = buffer_load16(a_buffer[r], meta_off, block);
-      a[r].sign = buffer_load8(a_buffer[r], sign_off, block);
-    }
-  };
-  // K split over workgroups (grid.y > 1): this workgroup multiplies the chunks [kc_begin, kc_end) and writes raw fp32
-  // sums to its slice of the partial-sum buffer; a second kernel adds the slices in order and applies the epilogue.
-  const int kc_begin = block_y * p.chunks_per_split;
-  const int kc_end = kc_begin + p.chunks_per_split < kc_total ? kc_begin + p.chunks_per_split : kc_total;
-  const int first = kc_begin + wave;  // this wavefront's first chunk
-  // Short K (at most two chunks per wavefront, e.g. 11008 x 4096): everything the wavefront will read is requested
-  // at once, so the kernel pays one memory latency instead of one per chunk.
-  constexpr bool kShortPath = NW <= 8 && SUB == 1;
-  const bool short_k = kShortPath && kc_end - kc_begin <= 2 * NW;
-  // The prepared operand comes from HBM and is what the first SMFMAC waits for longest: the loop form issues its first
-  // loads here, before the rest of the set-up (B descriptor, image offsets, fragment addresses), which then runs under
-  // their latency (4096 x 4096 x 16: 4.87 -> 4.70 us). The short form keeps B first: loads return in order, and a B image
-  // requested behind the weights would reach LDS only after them (11008 x 4096 x 1: 5.6 -> 6.3 us when tried).
-  AChunk a_cur[R], a_next[R];
-  if (!short_k) {
-    load_a(first, a_cur);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  const size_t b_bytes = (size_t)k_rows * n_cols * 2;
-  const bool b_fits = b_bytes < (size_t(1) << 32);  // else every image takes the general path
-  const buffer_t b_buffer = make_buffer(b_ptr, b_fits ? (uint32_t)b_bytes : 0u);
-  auto rows_valid_of = [&](int k_base) __attribute__((always_inline)) {
-    const int rows = k_rows - k_base;
-    return rows < 0 ? 0 : (rows > IMG_ROWS ? IMG_ROWS : rows);
-  };
-  // pieces at any alignment: a load instruction covers any_rows whole rows, lane = (row, piece) of them
-  const int any_pieces = (n_cols + 7) / 8, any_rows = 64 / any_pieces;
-  const int any_row = lane / any_pieces, any_piece = lane % any_pieces;
-  const bool any_used = any_row < any_rows;
-  const uint32_t any_load = (uint32_t)(any_row * n_cols + 8 * any_piece) * 2u, any_load_step = (uint32_t)(any_rows * n_cols) * 2u;
-  const uint32_t any_store = (uint32_t)any_row * ROW_BYTES + 16u * any_piece;
-  // Image t of this wavefront = B rows [k_base, k_base + IMG_ROWS) with k_base = (wave + NW (t / SUB)) * 256 +
-  // (t % SUB) * IMG_ROWS. The image travels through registers, loaded while the previous image is multiplied.
-  // token-major image: piece lane + 64 i = K values [8 p, 8 p + 8) of the image for token token_lane + TPI i
-  const int piece_lane = lane % PPT, token_lane = lane / PPT;
-  const uint32_t token_load_base = ((uint32_t)token_lane * (uint32_t)k_rows + 8u * piece_lane) * 2u;
-  const uint32_t token_load_step = (uint32_t)TPI * (uint32_t)k_rows * 2u;
-  const uint32_t token_store_base =
-      (uint32_t)token_lane * TOKEN_ROW_BYTES + (uint32_t)((piece_lane ^ token_swizzle<TOKEN_ROW_BYTES>(token_lane)) << 4);
-  // run mode: piece q = lane + 64 i of the image's run; pieces at or past 32 n are sent outside the descriptor (zero)
-  const uint32_t run_pieces = 32u * (uint32_t)n_cols;
-  auto load_b = [&](int k_base, u32x4_t (&v)[8]) __attribute__((always_inline)) {
-    if (MODE == kSkinnyBRun) {
-      const uint32_t run_base = (uint32_t)k_base * (uint32_t)n_cols * 2u;  // the launcher checks k n 2 < 2^32
-      if (k_base + IMG_ROWS <= k_rows) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-          if (64u * i < run_pieces)
-            v[i] = buffer_load16(b_buffer, lane + 64u * i < run_pieces ? meta_off + 1024u * i : 0xFFFFFF00u, run_base);
-        return;
-      }
-      // last image of a K that is no multiple of 256 (or an image past the end that is loaded but never multiplied):
-      // pieces inside B as they are, zeros past its end. K is a multiple of 32, so the valid bytes are a multiple of 16 n
-      // and no piece straddles the end.
-      const uint32_t valid_bytes = (uint32_t)rows_valid_of(k_base) * (uint32_t)n_cols * 2u;
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        if (64u * i < run_pieces)
-          v[i] = buffer_load16(b_buffer, meta_off + 1024u * i + 16u <= valid_bytes ? run_base + meta_off + 1024u * i : 0xFFFFFF00u, 0);
-      return;
-    }
-    if (TOKENS) {
-      // offsets at or past n * k * 2 (tokens >= n) fall outside the descriptor and read as zero; K positions at or
-      // past k are sent there too (the launcher checks that 64 * k * 2 stays well below 2^32)
-      if (k_base + IMG_ROWS <= k_rows) {
-        // the image's whole K range exists (wave-uniform test): lane offsets that do not change from image to image
-        // plus a scalar offset; the range check looks at the lane offset alone, which is what sends tokens >= n to zero
-        // (load i covers tokens TPI i ... TPI i + TPI - 1: nothing to fetch past the last token)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          if (TPI * i < n_cols) v[i] = buffer_load16(b_buffer, token_load_base + i * token_load_step, (uint32_t)k_base * 2u);
-          else v[i] = u32x4_t{0, 0, 0, 0};
-        }
-        return;
-      }
-      const bool inside = k_base + 8 * piece_lane < k_rows;
-      const uint32_t first = token_load_base + (uint32_t)k_base * 2u;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if (TPI * i < n_cols) v[i] = buffer_load16(b_buffer, inside ? first + i * token_load_step : 0xFFFFFF00u, 0);
-        else v[i] = u32x4_t{0, 0, 0, 0};
-      }
-      return;
-    }
-    if (MODE == kSkinnyBFull) {
-      if (b_fits && k_base + IMG_ROWS <= k_rows) {
-        // the whole image lies inside B (wave-uniform test): 8 KiB of consecutive memory, no per-piece checks
-        const uint32_t image = (uint32_t)k_base * (NC * 2);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = buffer_load16(b_buffer, meta_off + 1024u * i, image);
-        return;
-      }
-      const int rows_valid = rows_valid_of(k_base);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int q = lane + i * 64;
-        const bool ok = q / (NC / 8) < rows_valid;
-        v[i] = *reinterpret_cast<const u32x4_t*>(b_ptr + (ok ? (size_t)k_base * NC + (size_t)q * 8 : 0));
-        if (!ok) v[i] = u32x4_t{0, 0, 0, 0};
-      }
-      return;
-    }
-    // (wave-uniform) rows from the image's first on, as far as they matter: none past the end of K
-    const int rows_left = k_rows - k_base < IMG_ROWS + 8 ? k_rows - k_base : IMG_ROWS + 8;
-    if (rows_left <= 0) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = u32x4_t{0, 0, 0, 0};
-      return;
-    }
-    // lane offsets that do not change from image to image; lanes without a piece and pieces that would end past the rows
-    // left (the last image's, k % 32 == 0: at least 32 rows) load the last whole piece instead
-    const char* image = reinterpret_cast<const char*>(b_ptr + (size_t)k_base * n_cols);
-    const uint32_t last = (uint32_t)(rows_left * n_cols - 8) * 2u;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (i * any_rows < IMG_ROWS) {
-        const uint32_t offset = any_load + i * any_load_step;
-        v[i] = *reinterpret_cast<const u32x4_any_t*>(image + (offset < last ? offset : last));
-      }
-    if (rows_left < IMG_ROWS + 8) {
-      // last image: what was read from the last whole piece is shifted into place, rows at or past K are zeros
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (i * any_rows < IMG_ROWS) {
-          const uint32_t offset = any_load + i * any_load_step;
-          if (offset > last) v[i] = drop_halves(v[i], (int)(offset - last) / 2);
-        }
-    }
-  };
-  auto store_b = [&](int k_base, const u32x4_t (&v)[8]) __attribute__((always_inline)) {
-    if (MODE == kSkinnyBAny) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (i * any_rows < IMG_ROWS && any_used && any_row + i * any_rows < IMG_ROWS)
-          *reinterpret_cast<u32x4_t*>(region + any_store + i * any_rows * ROW_BYTES) = v[i];
-      return;
-    }
-    if (MODE == kSkinnyBRun) {
-      // piece q holds the n columns of rows 8 q / n ... : 2 n bytes to each row's start; columns n ... 15 keep the zeros the
-      // image was cleared to
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const uint32_t q = lane + 64u * i;
-        if (q >= run_pieces) continue;
-        if (n_cols == 4) {
-          *reinterpret_cast<u32x2_t*>(region + (2 * q) * ROW_BYTES) = u32x2_t{v[i].x, v[i].y};
-          *reinterpret_cast<u32x2_t*>(region + (2 * q + 1) * ROW_BYTES) = u32x2_t{v[i].z, v[i].w};
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) *reinterpret_cast<uint32_t*>(region + (4 * q + j) * ROW_BYTES) = v[i][j];
-        }
-      }
-      return;
-    }
-    if (TOKENS) {
-      // token = token_lane + TPI i with token_lane < TPI (a power of two): the two terms share no bits, so the swizzle of
-      // piece i differs from that of piece 0 by a compile-time XOR
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        *reinterpret_cast<u32x4_t*>(region + (token_store_base ^ (uint32_t)(token_swizzle<TOKEN_ROW_BYTES>(TPI * i) << 4)) + i * 1024) = v[i];
-      return;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) *reinterpret_cast<u32x4_t*>(region + (lane + i * 64) * 16) = v[i];
-  };
-
-  float16_t acc[R][NF];
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int f = 0; f < NF; ++f)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[r][f][v] = 0.f;
-  float4v_t acc16[R][2];  // M16: rows 0-15 and 16-31 of the row block; register v of lane l = row 4 (l / 16) + v, column l % 16
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) acc16[r][h] = float4v_t{0.f, 0.f, 0.f, 0.f};
-  const uint32_t one = packed_one_in_vgpr();
-  const int i16 = lane & 15, gb = lane >> 5, g16 = lane >> 4;
-  // (32x32x32 form, NC >= 32; sixteen-column images use the 16x16x64 form further down)
-  const int chunk8 = (NC >= 32 ? ((lane & 31) >> 4) * 4 : 0) + (i16 & 3);  // 8-byte piece of the 32-column fragment
-  const char* lane_ptr = region + (8 * gb + (i16 >> 2)) * ROW_BYTES + chunk8 * 8;
-
-  // token-major image: this lane's token row and swizzle; K step s of the image needs pieces 4 s + gb and 4 s + 2 + gb
-  const int token_col = NC >= 32 ? (lane & 31) : i16;
-  const uint32_t token_read_base = (uint32_t)token_col * TOKEN_ROW_BYTES + (uint32_t)((gb ^ token_swizzle<TOKEN_ROW_BYTES>(token_col)) << 4);
-  // ---- 16x16x64 form (M16). The instruction's A lane (row l % 16, group g = l / 16) holds eight kept values and their
-  // 16 index bits for 16 consecutive K positions, as a lane of the prepared block does for one K step: lane
-  // (row, half ga) of the block, step s. Which K positions group g stands for is free as long as B agrees, so the
-  // operands are built with one v_permlane16_swap per register pair instead of a gather: swapping the odd 16-lane
-  // rows of metadata register 2 P with the even rows of register 2 P + 1 leaves in the first register, for
-  // block rows 0-15, the groups (ga 0, steps 4 P + {0, 1}), (ga 0, steps 4 P + {2, 3}), (ga 1, steps 4 P + {0, 1}),
-  // (ga 1, steps 4 P + {2, 3}) and in the second register the same for block rows 16-31; ABID picks the even or the
-  // odd step of each pair. Instruction (P, abid) therefore covers K positions 128 P + 32 abid + [0, 32) and
-  // 128 P + 32 abid + 64 + [0, 32) of the chunk: group g positions 128 P + 32 abid + 64 (g % 2) + 16 (g / 2) + [0, 16).
-  // The sign words travel the same way (a register swapped with its own copy) and are shifted by 8 (g % 2) once, after
-  // which the expansion uses compile-time shifts. B lane (column l % 16, group gb) holds instruction K rows
-  // 8 gb + [0, 8) and 32 + 8 gb + [0, 8), i.e. chunk rows base + [0, 8) and base + 16 + [0, 8) with
-  // base = 128 P + 32 abid + 64 (gb / 2) + 8 (gb % 2).
-  struct A16 {
-    uint32_t idx[2][2];   // [row half][P]
-    uint32_t sign[2][2];
-  };
-  const uint32_t sign_shift16 = 8u * (g16 & 1);
-  auto gather16 = [&](const AChunk& a) __attribute__((always_inline)) {
-    A16 t;
-#pragma unroll
-    for (int P = 0; P < 2; ++P) {
-      const auto m = __builtin_amdgcn_permlane16_swap(a.meta[2 * P], a.meta[2 * P + 1], false, false);
-      const uint32_t w = P == 0 ? a.sign.x : a.sign.y;
-      const auto sg = __builtin_amdgcn_permlane16_swap(w, w, false, false);
-      t.idx[0][P] = m[0];
-      t.idx[1][P] = m[1];
-      t.sign[0][P] = sg[0] << sign_shift16;
-      t.sign[1][P] = sg[1] << sign_shift16;
-    }
-    return t;
-  };
-  const char* lane_ptr16 = region + (64 * (g16 >> 1) + 8 * (g16 & 1) + (i16 >> 2)) * ROW_BYTES + (i16 & 3) * 8;
-  const uint32_t token_read_base16 =
-      (uint32_t)i16 * TOKEN_ROW_BYTES + (uint32_t)(((8 * (g16 >> 1) + (g16 & 1)) ^ token_swizzle<TOKEN_ROW_BYTES>(i16)) << 4);
-  // B operand of instruction F = 2 P + abid
-  auto frag16 = [&](int F) __attribute__((always_inline)) {
-    u32x8_t raw;
-    if (TOKENS) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const u32x4_t t = *reinterpret_cast<const u32x4_t*>(
-            region + (token_read_base16 ^ (uint32_t)((16 * (F >> 1) + 4 * (F & 1) + 2 * h) << 4)));
-        raw[4 * h] = t.x; raw[4 * h + 1] = t.y; raw[4 * h + 2] = t.z; raw[4 * h + 3] = t.w;
-      }
-      return __builtin_bit_cast(half16_t, raw);
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int row_const = 128 * (F >> 1) + 32 * (F & 1) + 4 * (q & 1) + 16 * (q >> 1);
-      const u32x2_t t = lds_read_tr16(lane_ptr16 + row_const * ROW_BYTES);
-      raw[2 * q] = t.x;
-      raw[2 * q + 1] = t.y;
-    }
-    return __builtin_bit_cast(half16_t, raw);
-  };
-  auto compute16 = [&](const AChunk (&a)[R]) __attribute__((always_inline)) {
-    half16_t bf[4];
-#pragma unroll
-    for (int F = 0; F < 4; ++F) bf[F] = frag16(F);
-    A16 t[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) t[r] = gather16(a[r]);
-#pragma unroll
-    for (int F = 0; F < 4; ++F)
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          u32x4_t av;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) av[q] = ((t[r].sign[h][F >> 1] << (4 * (F & 1) + q)) & 0x80008000u) | one;
-          const half8_t a8 = __builtin_bit_cast(half8_t, av);
-          if ((F & 1) == 0)
-            acc16[r][h] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(a8, bf[F], acc16[r][h], (int)t[r].idx[h][F >> 1], 0, 0);
-          else
-            acc16[r][h] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(a8, bf[F], acc16[r][h], (int)t[r].idx[h][F >> 1], 0, 1);
-        }
-  };
-
-  auto frag = [&](int image_step, int f) __attribute__((always_inline)) {
-    u32x8_t raw;
-    if (TOKENS) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const u32x4_t t = *reinterpret_cast<const u32x4_t*>(
-            region + (token_read_base ^ (uint32_t)((4 * image_step + 2 * h) << 4)) + f * 32 * TOKEN_ROW_BYTES);
-        raw[4 * h] = t.x; raw[4 * h + 1] = t.y; raw[4 * h + 2] = t.z; raw[4 * h + 3] = t.w;
-      }
-      return __builtin_bit_cast(half16_t, raw);
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int row_const = image_step * 32 + 4 * (q & 1) + 16 * (q >> 1);
-      const u32x2_t t = lds_read_tr16(lane_ptr + row_const * ROW_BYTES + f * 64);
-      raw[2 * q] = t.x;
-      raw[2 * q + 1] = t.y;
-    }
-    return __builtin_bit_cast(half16_t, raw);
-  };
-  // the SMFMACs of image SUB_INDEX of a chunk: steps SUB_INDEX * IMG_STEPS ... + IMG_STEPS - 1
-  auto compute = [&](const AChunk (&a)[R], auto sub_tag) __attribute__((always_inline)) {
-    if constexpr (M16) {
-      compute16(a);
-      return;
-    }
-    constexpr int FIRST_STEP = decltype(sub_tag)::value * IMG_STEPS;
-    // Fragments are read in groups of FG K steps (4 FG transpose reads per column fragment) into one of two register
-    // sets: while the SMFMACs of a group run, the reads of the next group are already in flight, so only the first
-    // group of an image waits for LDS. The scheduling barriers keep later groups' reads from being hoisted as well
-    // (8 registers per fragment). Sixteen-wavefront workgroups have 128 registers per wavefront and no room for the
-    // second set: they read each group when it is due.
-    constexpr bool kAhead = NW <= 8;
-    constexpr int FG = (R >= 4 || NF > 1) ? 2 : 4;
-    constexpr int GROUPS = IMG_STEPS / FG;
-    static_assert(IMG_STEPS % FG == 0 && GROUPS >= 1 && GROUPS <= 4, "whole groups of K steps per image");
-    half16_t bfrag[kAhead ? 2 : 1][FG][NF];
-    auto read_group = [&](int first_in_image, half16_t (&dst)[FG][NF]) __attribute__((always_inline)) {
-#pragma unroll
-      for (int st = 0; st < FG; ++st)
-#pragma unroll
-        for (int f = 0; f < NF; ++f) dst[st][f] = frag(first_in_image + st, f);
-    };
-    auto group = [&](auto index_tag) __attribute__((always_inline)) {
-      constexpr int G = decltype(index_tag)::value;
-      if constexpr (G < GROUPS) {
-        constexpr int FIRST = FIRST_STEP + G * FG;  // step within the chunk
-        constexpr int SET = kAhead ? (G & 1) : 0;
-        if constexpr (!kAhead) read_group(G * FG, bfrag[0]);
-        else if constexpr (G + 1 < GROUPS) read_group((G + 1) * FG, bfrag[SET ^ 1]);
-        auto step = [&](auto offset_tag) __attribute__((always_inline)) {
-          constexpr int OFFSET = decltype(offset_tag)::value;
-          if constexpr (OFFSET < FG) {
-            constexpr int STEP = FIRST + OFFSET;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-              const half8_t av = expand_signs<STEP>(a[r], one);
-#pragma unroll
-              for (int f = 0; f < NF; ++f)
-                acc[r][f] = smfmac_step<STEP, false>(a[r], av, bfrag[SET][OFFSET][f], acc[r][f]);
-            }
-          }
-        };
-        step(std::integral_constant<int, 0>{});
-        step(std::integral_constant<int, 1>{});
-        step(std::integral_constant<int, 2>{});
-        step(std::integral_constant<int, 3>{});
-        if constexpr (G + 1 < GROUPS) __builtin_amdgcn_sched_barrier(0);
-      }
-    };
-    if constexpr (kAhead) read_group(0, bfrag[0]);
-    group(std::integral_constant<int, 0>{});
-    group(std::integral_constant<int, 1>{});
-    group(std::integral_constant<int, 2>{});
-    group(std::integral_constant<int, 3>{});
-  };
-
-  // sixteen wavefronts leave 128 registers each: no room to hold the next image (32 registers) during the SMFMACs
-  constexpr bool kPrefetchB = NW <= 8;
-  if (MODE == kSkinnyBRun) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) *reinterpret_cast<u32x4_t*>(region + (lane + i * 64) * 16) = u32x4_t{0, 0, 0, 0};
-  }
-  u32x4_t breg[8];
-  char* const d_out = reinterpret_cast<char*>(p.d) + (size_t)block_y * p.m * p.n * (p.d_f16 ? 2 : 4);
-  if (short_k) {
-    u32x4_t breg2[8];
-    load_b(first * kChunkK, breg);
-    load_a(first, a_cur);
-    load_b((first + NW) * kChunkK, breg2);
-    load_a(first + NW, a_next);
-    if (first < kc_end) {
-      store_b(first * kChunkK, breg);
-      compute(a_cur, std::integral_constant<int, 0>{});
-    }
-    if (first + NW < kc_end) {
-      store_b((first + NW) * kChunkK, breg2);
-      compute(a_next, std::integral_constant<int, 0>{});
-    }
-  }
-  if (kPrefetchB && !short_k) load_b(first * kChunkK, breg);
-  for (int kc = short_k ? kc_end : first; kc < kc_end; kc += NW) {
-    const int k_base = kc * kChunkK;
-    // this wavefront has another chunk after this one (wave-uniform): only then is the next chunk requested; a load
-    // past the last chunk would be one more instruction for the memory pipeline, a third of them when a wavefront
-    // has two or three chunks
-    const bool more = kc + NW < kc_end;
-    if (!kPrefetchB) load_b(k_base, breg);
-    store_b(k_base, breg);  // after the previous image's fragment reads: LDS operations of a wavefront execute in order
-    if (kPrefetchB && (SUB > 1 || more)) load_b(SUB > 1 ? k_base + IMG_ROWS : k_base + NW * kChunkK, breg);
-    if (more) load_a(kc + NW, a_next);
-    compute(a_cur, std::integral_constant<int, 0>{});
-    // the chunk's further images (SUB - 1 of them)
-    auto further = [&](auto sub_tag) __attribute__((always_inline)) {
-      constexpr int S = decltype(sub_tag)::value;
-      if constexpr (S < SUB) {
-        const int image_base = k_base + S * IMG_ROWS;
-        if (!kPrefetchB) {
-          __builtin_amdgcn_sched_barrier(0);  // this image's loads stay behind the previous image's SMFMACs
-          load_b(image_base, breg);
-        }
-        store_b(image_base, breg);
-        if (kPrefetchB && (S + 1 < SUB || more)) load_b(S + 1 < SUB ? image_base + IMG_ROWS : k_base + NW * kChunkK, breg);
-        compute(a_cur, sub_tag);
-      }
-    };
-    further(std::integral_constant<int, 1>{});
-    further(std::integral_constant<int, 2>{});
-    further(std::integral_constant<int, 3>{});
-#pragma unroll
-    for (int r = 0; r < R; ++r) a_cur[r] = a_next[r];
-  }
-
-  smfmac_drain();
-  // ---- add the NW partial tiles through LDS: region of wavefront w := its R tiles as [r][32 rows][NC cols] fp32
-  constexpr int ROUND_ROWS = RT * kRowBlock;
-#pragma unroll
-  for (int round = 0; round < R / RT; ++round) {
-    if (round > 0) __syncthreads();  // the previous round's tiles have been read
-    {
-      float* tile = reinterpret_cast<float*>(region);
-      const int col = lane & 31;
-      if (M16) {
-#pragma unroll
-        for (int rr = 0; rr < RT; ++rr)
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-              const int row = 16 * h + 4 * g16 + v;
-              const float value = acc16[round * RT + rr][h][v];
-              if (TOKENS) tile[i16 * ROUND_ROWS + ((rr * 32 + row) ^ i16)] = value;
-              else tile[(rr * 32 + row) * NC + i16] = value;
-            }
-      } else if (col < NC) {
-#pragma unroll
-        for (int rr = 0; rr < RT; ++rr)
-#pragma unroll
-          for (int f = 0; f < NF; ++f)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-              const int row = 8 * (v / 4) + 4 * (lane >> 5) + (v % 4);
-              const float value = acc[round * RT + rr][f][v];
-              // token-major: [token][weight row of the round], the row index XOR-swizzled by the token so that neither
-              // these stores (32 tokens, one row) nor the reads below (one token, consecutive rows) collide in a bank
-              if (TOKENS) tile[(f * 32 + col) * ROUND_ROWS + ((rr * 32 + row) ^ col)] = value;
-              else tile[(rr * 32 + row) * NC + f * 32 + col] = value;
-            }
-      }
-    }
-    __syncthreads();
-    const int round_row0 = rb_first * kRowBlock + round * ROUND_ROWS;
-    if (TOKENS) {
-      for (int idx = tid; idx < ROUND_ROWS * NC; idx += NT) {
-        const int local = idx % ROUND_ROWS, token = idx / ROUND_ROWS;
-        const int pos = token * ROUND_ROWS + (local ^ (token & 31));
-        float sum = 0.f;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) sum += reinterpret_cast<const float*>(bs + w * kSkinnyRegion)[pos];
-        const int row = round_row0 + local;
-        if (token < p.n && row < p.m) {
-          if (p.bias) sum += p.bias_f16 ? (float)reinterpret_cast<const _Float16*>(p.bias)[row]
-                                        : reinterpret_cast<const float*>(p.bias)[row];
-          const size_t o = (size_t)token * p.m + row;
-          // a B of one column is a token-major x of one token and its result column is y: the launcher sends such calls
-          // here with their alpha, beta and C (element o of C in both layouts); the linear layer passes 1, 0, null
-          sum = p.alpha * sum;
-          if (p.beta != 0.f)
-            sum = sum + p.beta * (p.c_f16 ? (float)reinterpret_cast<const _Float16*>(p.c)[o] : reinterpret_cast<const float*>(p.c)[o]);
-          if (p.d_f16) reinterpret_cast<_Float16*>(d_out)[o] = (_Float16)sum;
-          else reinterpret_cast<float*>(d_out)[o] = sum;
-        }
-      }
-    } else {
-      for (int idx = tid; idx < ROUND_ROWS * NC; idx += NT) {
-        float sum = 0.f;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) sum += reinterpret_cast<const float*>(bs + w * kSkinnyRegion)[idx];
-        const int col = idx % NC;
-        const int row = round_row0 + idx / NC;
-        if (col < p.n && row < p.m) {
-          const size_t o = (size_t)row * p.n + col;
-          float x = p.alpha * sum;
-          if (p.beta != 0.f) {
-            const float cv = p.c_f16 ? (float)reinterpret_cast<const _Float16*>(p.c)[o] : reinterpret_cast<const float*>(p.c)[o];
-            x = x + p.beta * cv;
-          }
-          if (p.d_f16) reinterpret_cast<_Float16*>(d_out)[o] = (_Float16)x;
-          else reinterpret_cast<float*>(d_out)[o] = x;
-        }
-      }
-    }
-  }
-}
-
-template <int NW, int R, int MODE, int NC>
-__global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_kernel(SkinnyArgs p) {
-  skinny_body<NW, R, MODE, NC>(p, blockIdx.x, blockIdx.y);
-}
-
-// Grouped form: several independent products y_i = x_i W_i^T + bias_i that share the token count, in one launch. The
-// workgroups are numbered over the concatenated row groups of the problems; a workgroup finds its problem by
-// comparing its number with the problems' first workgroups (wave-uniform, a handful of scalar compares) and then runs
-// the token-major body on that problem's arguments. Decode-sized products take a few microseconds each, of which the
-// launch itself and the ramp of the memory pipeline are a large part: one launch for the q / k / v or gate / up
-// projections of a layer pays them once.
-template <int NW, int R, int NC>
-__global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_group_kernel(SkinnyGroupArgs g) {
-  int which = 0;
-  for (int i = 1; i < g.count; ++i)
-    if ((int)blockIdx.x >= g.first_block[i]) which = i;
-  skinny_body<NW, R, kSkinnyBTokens, NC>(g.problem[which], (int)blockIdx.x - g.first_block[which], 0);
-}
-
-// =====================================================================================================
-// pad_b_kernel: copies B (k x n, row stride n, any alignment) into rows of ldb = round_up(n, 8) halves, so that every row starts 16-byte aligned for the asynchronous copies of the main kernel.
-// Bound: memory, 2 k n bytes each way (and a few us of launch and latency below about 10 MB). A workgroup takes `rows`
-// whole rows, as many as fit its 1024 pieces, or 1024 pieces of one longer row, so that neighbouring lanes write
-// neighbouring pieces across row ends; the four loads of a thread, 16 bytes at any alignment, come before its first store.
-// Against two-byte loads, one piece per thread (us): 4096 x 1001 9.0 -> 7.0, 20864 x 707 18.3 -> 12.0, 12832 x 3241 41.7 -> 29.3.
-// =====================================================================================================
-constexpr int kPadPieces = 1024;
-
-// rows > 1: reciprocal = 2^32 / (ldb / 8) + 1, with which the quotients below 2^11 that occur are exact
-__global__ __launch_bounds__(256) void pad_b_kernel(const _Float16* __restrict__ b, _Float16* __restrict__ dst, int k,
-                                                    int n, int ldb, int rows, uint32_t reciprocal) {
-  const int row0 = blockIdx.x * rows, per_row = ldb / 8, piece0 = blockIdx.y * kPadPieces;
-  const size_t last_start = (size_t)k * n - 8;  // k >= 32
-  u32x4_t v[kPadPieces / 256];
-#pragma unroll
-  for (int i = 0; i < kPadPieces / 256; ++i) {
-    const int local = threadIdx.x + 256 * i;
-    const int r = rows > 1 ? (int)__umulhi(local, reciprocal) : 0, col = 8 * (piece0 + local - r * per_row);
-    // a piece that reaches past the end of its row takes the next row's first values along: nothing is made of them, they
-    // only meet columns that are never stored. Past the end of B it is moved back and shifted into place below.
-    const size_t start = (size_t)(row0 + r) * n + col;
-    v[i] = *reinterpret_cast<const u32x4_any_t*>(b + (start <= last_start ? start : last_start));
-  }
-#pragma unroll
-  for (int i = 0; i < kPadPieces / 256; ++i) {
-    const int local = threadIdx.x + 256 * i;
-    const int r = rows > 1 ? (int)__umulhi(local, reciprocal) : 0, col = 8 * (piece0 + local - r * per_row);
-    const int row = row0 + r;
-    if (r >= rows || row >= k || col >= ldb) continue;
-    if (row == k - 1 && col + 8 > n) v[i] = drop_halves(v[i], col + 8 - n);
-    *reinterpret_cast<u32x4_t*>(dst + (size_t)row * ldb + col) = v[i];
-  }
-}
-
-// =====================================================================================================
-// splitk_reduce_kernel: d = alpha * (sum over splits, in split order, of the fp32 partial sums) + beta * c.
-// Elementwise over the m * n results; VEC = 4 when the element count and the alignment of c and d allow it.
-// Linear-layer form: bias (row_length values, may be null) is added instead, element i taking bias[i % row_length].
-// =====================================================================================================
-template <int VEC>
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws, int splits, size_t stride,
-                                                            const void* __restrict__ c, void* __restrict__ d,
-                                                            size_t total, float alpha, float beta, int c_f16,
-                                                            int d_f16, const void* __restrict__ bias, int bias_f16,
-                                                            int row_length) {
-  const size_t first = ((size_t)blockIdx.x * 256 + threadIdx.x) * VEC;
-  if (first >= total) return;
-  float x[VEC];
-#pragma unroll
-  for (int j = 0; j < VEC; ++j) x[j] = 0.f;
-  for (int s = 0; s < splits; ++s) {
-    const float* src = ws + (size_t)s * stride + first;
-    if (VEC == 4) {
-      const float4 v = *reinterpret_cast<const float4*>(src);
-      x[0] += v.x; x[1 % VEC] += v.y; x[2 % VEC] += v.z; x[3 % VEC] += v.w;
-    } else {
-      x[0] += src[0];
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < VEC; ++j) {
-    x[j] = alpha * x[j];
-    if (beta != 0.f) {
-      const float cv = c_f16 ? (float)reinterpret_cast<const _Float16*>(c)[first + j]
-                             : reinterpret_cast<const float*>(c)[first + j];
-      x[j] = x[j] + beta * cv;
-    }
-  }
-  if (bias) {
-    const size_t at = first % (size_t)row_length;  // row_length is a multiple of 4: a vector never wraps
-#pragma unroll
-    for (int j = 0; j < VEC; ++j)
-      x[j] += bias_f16 ? (float)reinterpret_cast<const _Float16*>(bias)[at + j] : reinterpret_cast<const float*>(bias)[at + j];
-  }
-  if (VEC == 4) {
-    if (d_f16) {
-      *reinterpret_cast<half4_t*>(reinterpret_cast<_Float16*>(d) + first) =
-          half4_t{(_Float16)x[0], (_Float16)x[1 % VEC], (_Float16)x[2 % VEC], (_Float16)x[3 % VEC]};
-    } else {
-      *reinterpret_cast<float4*>(reinterpret_cast<float*>(d) + first) = float4{x[0], x[1 % VEC], x[2 % VEC], x[3 % VEC]};
-    }
-  } else {
-    if (d_f16) reinterpret_cast<_Float16*>(d)[first] = (_Float16)x[0];
-    else reinterpret_cast<float*>(d)[first] = x[0];
-  }
-}
-
-// Second pass of a K split: ordered sum of the partial results and the epilogue (bias and row_length for the
-// token-major form, where element i of y takes bias[i % m]).
-static hipError_t launch_split_reduce(const float* ws, int splits, size_t total, const void* c, void* d, float alpha,
-                                      float beta, int c_f16, int d_f16, const void* bias, int bias_f16, int row_length,
-                                      hipStream_t stream) {
-  const bool vec = total % 4 == 0 && (reinterpret_cast<uintptr_t>(d) & 15) == 0 &&
-                   (beta == 0.f || (reinterpret_cast<uintptr_t>(c) & 15) == 0) && (!bias || row_length % 4 == 0);
-  if (vec)
-    hipLaunchKernelGGL(splitk_reduce_kernel<4>, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream, ws,
-                       splits, total, c, d, total, alpha, beta, c_f16, d_f16, bias, bias_f16, row_length);
-  else
-    hipLaunchKernelGGL(splitk_reduce_kernel<1>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, ws,
-                       splits, total, c, d, total, alpha, beta, c_f16, d_f16, bias, bias_f16, row_length);
-  return hipGetLastError();
-}
-
-// =====================================================================================================
-// Host-side launchers
-// =====================================================================================================
 template <int WM, int WN, int FM, int FN, bool DMA, bool TOKENS = false, int KG = 1, bool M16 = false>
 static hipError_t launch_gemm_cfg(GemmArgs args, hipStream_t stream) {
   using TS = TileShape<WM, WN, FM, FN, KG>;
@@ -1966,230 +1251,6 @@ static hipError_t launch_gemm_cfg(GemmArgs args, hipStream_t stream) {
   args.xcds = xcds;
   hipLaunchKernelGGL(kern, dim3(args.tiles_m * args.tiles_n, args.splits), dim3(64 * TS::NW), lds, stream, args);
   return hipGetLastError();
-}
-
-static hipError_t launch_gemm_pass(GemmArgs args, int tile_config, hipStream_t stream) {
-  const bool aligned = (args.ldb % 8 == 0) && ((reinterpret_cast<uintptr_t>(args.b) & 15) == 0);
-  if (!aligned) return launch_gemm_cfg<4, 1, 1, 4, false>(args, stream);
-  switch (tile_config) {
-    case kTile512x128: return launch_gemm_cfg<4, 1, 4, 4, true>(args, stream);
-    case kTile256x128: return launch_gemm_cfg<4, 1, 2, 4, true>(args, stream);
-    case kTile128x128: return launch_gemm_cfg<4, 1, 1, 4, true>(args, stream);
-    case kTile256x256: return launch_gemm_cfg<2, 2, 4, 4, true>(args, stream);
-    case kTile256x128w: return launch_gemm_cfg<2, 2, 4, 2, true>(args, stream);
-    case kTile512x128t: return launch_gemm_cfg<2, 2, 8, 2, true>(args, stream);
-    case kTile128x128s: return launch_gemm_cfg<2, 2, 2, 2, true>(args, stream);
-    case kTile256x64: return launch_gemm_cfg<2, 2, 4, 1, true>(args, stream);
-    case kTile256x256w8: return launch_gemm_cfg<2, 4, 4, 2, true>(args, stream);
-    case kTile512x128w8: return launch_gemm_cfg<4, 2, 4, 2, true>(args, stream);
-    case kTile256x128w8: return launch_gemm_cfg<4, 2, 2, 2, true>(args, stream);
-    case kTile128x128w8: return launch_gemm_cfg<2, 4, 2, 1, true>(args, stream);
-    case kTile64x128: return launch_gemm_cfg<2, 2, 1, 2, true>(args, stream);
-    case kTile128x128k2: return launch_gemm_cfg<2, 2, 2, 2, true, false, 2>(args, stream);
-    case kTile64x128k2: return launch_gemm_cfg<2, 2, 1, 2, true, false, 2>(args, stream);
-    case kTile512x128m16: return launch_gemm_cfg<4, 1, 4, 4, true, false, 1, true>(args, stream);
-    default: return hipErrorInvalidValue;
-  }
-}
-
-hipError_t launch_gemm_tokens(GemmArgs args, int tile_config, hipStream_t stream) {
-  if (prepared_bytes(args.m, args.k) >= (size_t(1) << 32)) return hipErrorInvalidValue;  // 32-bit copy offsets
-  if ((reinterpret_cast<uintptr_t>(args.b) & 15) != 0 || (size_t)args.k * 256 * 2 >= (size_t(1) << 32))
-    return hipErrorInvalidValue;  // 16-byte copies of x; 32-bit offsets inside a tile's token rows
-  const int chunks = (args.k + kChunkK - 1) / kChunkK;
-  args.ldb = args.k;
-  args.alpha = 1.f;
-  args.beta = 0.f;
-  args.c = nullptr;
-  auto pass = [&](GemmArgs a) {
-    a.vector_epilogue = (reinterpret_cast<uintptr_t>(a.d) & 15) == 0 && a.m % 8 == 0 &&
-                        (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0;
-    switch (tile_config) {
-      case kTile256x128w: return launch_gemm_cfg<2, 2, 4, 2, true, true>(a, stream);
-      case kTile128x128s: return launch_gemm_cfg<2, 2, 2, 2, true, true>(a, stream);
-      case kTile512x128w8: return launch_gemm_cfg<4, 2, 4, 2, true, true>(a, stream);
-      case kTile256x128w8: return launch_gemm_cfg<4, 2, 2, 2, true, true>(a, stream);
-      case kTile128x128w8: return launch_gemm_cfg<2, 4, 2, 1, true, true>(a, stream);
-      case kTile64x128: return launch_gemm_cfg<2, 2, 1, 2, true, true>(a, stream);
-      case kTile128x128k2: return launch_gemm_cfg<2, 2, 2, 2, true, true, 2>(a, stream);
-      case kTile64x128k2: return launch_gemm_cfg<2, 2, 1, 2, true, true, 2>(a, stream);
-      case kTile512x128m16: return launch_gemm_cfg<4, 1, 4, 4, true, true, 1, true>(a, stream);
-      default: return hipErrorInvalidValue;  // the tiles the automatic choice uses
-    }
-  };
-  if (args.splits <= 1) {
-    args.splits = 1;
-    args.chunks_per_split = chunks;
-    return pass(args);
-  }
-  if (args.chunks_per_split < 1 || (long)(args.splits - 1) * args.chunks_per_split >= chunks || !args.split_ws)
-    return hipErrorInvalidValue;  // an empty split would address past the prepared operand
-  // pass 1: raw fp32 partial sums per split, token-major like y; pass 2: ordered sum and bias
-  GemmArgs first = args;
-  first.d = args.split_ws;
-  first.d_f16 = 0;
-  first.bias = nullptr;
-  if (hipError_t st = pass(first); st != hipSuccess) return st;
-  return launch_split_reduce(args.split_ws, args.splits, (size_t)args.m * args.n, nullptr, args.d, 1.f, 0.f, 0, args.d_f16,
-                             args.bias, args.bias_f16, args.m, stream);
-}
-
-hipError_t launch_gemm(GemmArgs args, int tile_config, hipStream_t stream) {
-  if (prepared_bytes(args.m, args.k) >= (size_t(1) << 32)) return hipErrorInvalidValue;  // 32-bit copy offsets
-  args.ldb = args.n;
-  const bool aligned = (args.n % 8 == 0) && ((reinterpret_cast<uintptr_t>(args.b) & 15) == 0);
-  if (!aligned && args.b_pad) {
-    const int ldb = (args.n + 7) / 8 * 8;
-    const int per_row = ldb / 8, rows = per_row > 1 && per_row < kPadPieces ? kPadPieces / per_row : 1;
-    hipLaunchKernelGGL(pad_b_kernel, dim3((args.k + rows - 1) / rows, (per_row + kPadPieces - 1) / kPadPieces), dim3(256), 0,
-                       stream, args.b, args.b_pad, args.k, args.n, ldb, rows,
-                       (uint32_t)((uint64_t(1) << 32) / per_row + 1));
-    if (hipError_t st = hipGetLastError(); st != hipSuccess) return st;
-    args.b = args.b_pad;
-    args.ldb = ldb;
-  }
-  const int chunks = (args.k + kChunkK - 1) / kChunkK;
-  if (args.splits <= 1) {
-    args.splits = 1;
-    args.chunks_per_split = chunks;
-    return launch_gemm_pass(args, tile_config, stream);
-  }
-  if (args.chunks_per_split < 1 || (long)(args.splits - 1) * args.chunks_per_split >= chunks || !args.split_ws)
-    return hipErrorInvalidValue;  // an empty split would address past the prepared operand
-  // pass 1: raw fp32 partial sums per split; pass 2: ordered sum and epilogue
-  GemmArgs pass = args;
-  pass.alpha = 1.f;
-  pass.beta = 0.f;
-  pass.c = nullptr;
-  pass.d = args.split_ws;
-  pass.d_f16 = 0;
-  if (hipError_t st = launch_gemm_pass(pass, tile_config, stream); st != hipSuccess) return st;
-  return launch_split_reduce(args.split_ws, args.splits, (size_t)args.m * args.n, args.c, args.d, args.alpha, args.beta,
-                             args.c_f16, args.d_f16, nullptr, 0, 1, stream);
-}
-
-template <int NW, int R, int MODE, int NC>
-static hipError_t launch_skinny_mode(const SkinnyArgs& args, hipStream_t stream) {
-  const int row_blocks = args.m / kRowBlock;
-  hipLaunchKernelGGL((skinny_kernel<NW, R, MODE, NC>), dim3((row_blocks + R - 1) / R, args.splits), dim3(64 * NW), 0,
-                     stream, args);
-  return hipGetLastError();
-}
-
-template <int NW, int R>
-static hipError_t launch_skinny_cfg(const SkinnyArgs& args, hipStream_t stream) {
-  const bool aligned = (reinterpret_cast<uintptr_t>(args.b) & 15) == 0;
-  if (args.n > 32) {  // 64-column images, two column fragments: at most two row blocks fit the registers
-    constexpr int R64 = R > 2 ? 2 : R;
-    if (args.n == 64 && aligned) return launch_skinny_mode<NW, R64, kSkinnyBFull, 64>(args, stream);
-    return launch_skinny_mode<NW, R64, kSkinnyBAny, 64>(args, stream);
-  }
-  if (args.n > 16) {  // 32-column images
-    if (args.n == 32 && aligned) return launch_skinny_mode<NW, R, kSkinnyBFull, 32>(args, stream);
-    return launch_skinny_mode<NW, R, kSkinnyBAny, 32>(args, stream);
-  }
-  if (args.n == 16 && aligned) return launch_skinny_mode<NW, R, kSkinnyBFull, 16>(args, stream);
-  // one column: B is a token-major x of one token and D is its y (same memory in both layouts)
-  if (args.n == 1 && aligned && (size_t)args.k * 64 * 2 < 0xFFFFFF00u)
-    return launch_skinny_mode<NW, R, kSkinnyBTokens, 16>(args, stream);
-  if ((args.n == 2 || args.n == 4) && aligned && (size_t)args.k * args.n * 2 < 0xFFFFFF00u)
-    return launch_skinny_mode<NW, R, kSkinnyBRun, 16>(args, stream);
-  return launch_skinny_mode<NW, R, kSkinnyBAny, 16>(args, stream);
-}
-
-template <int NW, int R>
-static hipError_t launch_skinny_tokens_cfg(const SkinnyArgs& args, hipStream_t stream) {
-  if (args.n > 32) return launch_skinny_mode<NW, (R > 2 ? 2 : R), kSkinnyBTokens, 64>(args, stream);
-  if (args.n > 16) return launch_skinny_mode<NW, R, kSkinnyBTokens, 32>(args, stream);
-  return launch_skinny_mode<NW, R, kSkinnyBTokens, 16>(args, stream);
-}
-
-// Fills in the K split of a split-K kernel launch: splits <= 1 = one pass straight into d.
-static hipError_t skinny_split_setup(SkinnyArgs& args, SkinnyArgs& first_pass) {
-  if (args.splits <= 1) {
-    args.splits = 1;
-    args.chunks_per_split = args.kc_total;
-    first_pass = args;
-    return hipSuccess;
-  }
-  if (args.chunks_per_split < 1 || (long)(args.splits - 1) * args.chunks_per_split >= args.kc_total || !args.split_ws)
-    return hipErrorInvalidValue;  // an empty split would only add zeros, but it is a planning error
-  first_pass = args;  // raw fp32 partial sums per split, laid out like the result
-  first_pass.alpha = 1.f;
-  first_pass.beta = 0.f;
-  first_pass.c = nullptr;
-  first_pass.bias = nullptr;
-  first_pass.d = args.split_ws;
-  first_pass.d_f16 = 0;
-  return hipSuccess;
-}
-
-hipError_t launch_skinny_tokens(SkinnyArgs args, int rows_per_group, hipStream_t stream) {
-  if (args.n < 1 || args.n > kSkinnyMaxN) return hipErrorInvalidValue;
-  // 16-byte loads of x; lane offsets of up to 64 token rows must stay below the "outside" offset of the kernel
-  if ((reinterpret_cast<uintptr_t>(args.b) & 15) != 0 || (size_t)args.k * 64 * 2 >= 0xFFFFFF00u) return hipErrorInvalidValue;
-  SkinnyArgs pass;
-  if (hipError_t st = skinny_split_setup(args, pass); st != hipSuccess) return st;
-  hipError_t st;
-  switch (rows_per_group) {
-    case 32: st = launch_skinny_tokens_cfg<16, 1>(pass, stream); break;
-    case 64: st = launch_skinny_tokens_cfg<8, 2>(pass, stream); break;
-    case 128: st = launch_skinny_tokens_cfg<8, 4>(pass, stream); break;
-    default: return hipErrorInvalidValue;
-  }
-  if (st != hipSuccess || args.splits <= 1) return st;
-  return launch_split_reduce(args.split_ws, args.splits, (size_t)args.m * args.n, nullptr, args.d, 1.f, 0.f, 0, args.d_f16,
-                             args.bias, args.bias_f16, args.m, stream);
-}
-
-template <int NW, int R>
-static hipError_t launch_skinny_group_cfg(const SkinnyGroupArgs& g, int blocks, int tokens, hipStream_t stream) {
-  if (tokens > 32) hipLaunchKernelGGL((skinny_group_kernel<NW, (R > 2 ? 2 : R), 64>), dim3(blocks), dim3(64 * NW), 0, stream, g);
-  else if (tokens > 16) hipLaunchKernelGGL((skinny_group_kernel<NW, R, 32>), dim3(blocks), dim3(64 * NW), 0, stream, g);
-  else hipLaunchKernelGGL((skinny_group_kernel<NW, R, 16>), dim3(blocks), dim3(64 * NW), 0, stream, g);
-  return hipGetLastError();
-}
-
-hipError_t launch_skinny_group(SkinnyGroupArgs g, int rows_per_group, hipStream_t stream) {
-  if (g.count < 1 || g.count > kSkinnyMaxGroup) return hipErrorInvalidValue;
-  const int tokens = g.problem[0].n;
-  if (tokens < 1 || tokens > kSkinnyMaxN) return hipErrorInvalidValue;
-  if (rows_per_group != 32 && rows_per_group != 64 && rows_per_group != 128) return hipErrorInvalidValue;
-  const int rows = (rows_per_group == 128 && tokens > 32) ? 64 : rows_per_group;  // as launch_skinny_tokens_cfg does
-  int blocks = 0;
-  for (int i = 0; i < g.count; ++i) {
-    SkinnyArgs& p = g.problem[i];
-    if (p.n != tokens || p.m <= 0 || p.k <= 0 || !p.prep || !p.b || !p.d) return hipErrorInvalidValue;
-    // 16-byte loads of x; lane offsets of up to 64 token rows must stay below the "outside" offset of the kernel
-    if ((reinterpret_cast<uintptr_t>(p.b) & 15) != 0 || (size_t)p.k * 64 * 2 >= 0xFFFFFF00u) return hipErrorInvalidValue;
-    p.splits = 1;
-    p.chunks_per_split = p.kc_total;
-    p.split_ws = nullptr;
-    g.first_block[i] = blocks;
-    blocks += (p.m + rows - 1) / rows;
-  }
-  g.first_block[g.count] = blocks;
-  switch (rows_per_group) {
-    case 32: return launch_skinny_group_cfg<16, 1>(g, blocks, tokens, stream);
-    case 64: return launch_skinny_group_cfg<8, 2>(g, blocks, tokens, stream);
-    default: return launch_skinny_group_cfg<8, 4>(g, blocks, tokens, stream);
-  }
-}
-
-hipError_t launch_skinny(SkinnyArgs args, int rows_per_group, hipStream_t stream) {
-  if (args.n < 1 || args.n > kSkinnyMaxN) return hipErrorInvalidValue;
-  SkinnyArgs pass;
-  if (hipError_t st = skinny_split_setup(args, pass); st != hipSuccess) return st;
-  hipError_t st;
-  switch (rows_per_group) {
-    case 32: st = launch_skinny_cfg<16, 1>(pass, stream); break;  // sixteen wavefronts split K: small M
-    case 64: st = launch_skinny_cfg<8, 2>(pass, stream); break;
-    case 128: st = launch_skinny_cfg<8, 4>(pass, stream); break;  // n > 32: 64-row groups
-    default: return hipErrorInvalidValue;
-  }
-  if (st != hipSuccess || args.splits <= 1) return st;
-  return launch_split_reduce(args.split_ws, args.splits, (size_t)args.m * args.n, args.c, args.d, args.alpha, args.beta,
-                             args.c_f16, args.d_f16, nullptr, 0, 1, stream);
 }
 
 }  // namespace onebit

@@ -77,6 +77,12 @@ hipError_t launch_gemm_tokens(GemmArgs args, int tile_config, hipStream_t stream
 enum PackDtype { kPackF32 = 0, kPackF16 = 1, kPackBF16 = 2 };
 hipError_t launch_pack(const void* w, int dtype, void* a, void* e, int m, int k, int prune, int layout, hipStream_t stream);
 
+// Second pass of a K split: ordered sum of the partial results and the epilogue (bias and row_length for the
+// token-major form, where element i of y takes bias[i % m]).
+hipError_t launch_split_reduce(const float* ws, int splits, size_t total, const void* c, void* d, float alpha,
+                                      float beta, int c_f16, int d_f16, const void* bias, int bias_f16, int row_length,
+                                      hipStream_t stream);
+
 // Split-K kernel for n <= 64; rows_per_group (32, 64 or 128) = weight rows one workgroup covers (n > 32: at most 64).
 constexpr int kSkinnyMaxN = 64;
 hipError_t launch_skinny(SkinnyArgs args, int rows_per_group, hipStream_t stream);

@@ -1,0 +1,65 @@
+// Token-major form of the split-K kernel (the linear layer), one product or several per launch.
+#include "onebit_skinny.h"
+
+namespace onebit {
+
+template <int NW, int R>
+static hipError_t launch_skinny_tokens_cfg(const SkinnyArgs& args, hipStream_t stream) {
+  if (args.n > 32) return launch_skinny_mode<NW, (R > 2 ? 2 : R), kSkinnyBTokens, 64>(args, stream);
+  if (args.n > 16) return launch_skinny_mode<NW, R, kSkinnyBTokens, 32>(args, stream);
+  return launch_skinny_mode<NW, R, kSkinnyBTokens, 16>(args, stream);
+}
+
+hipError_t launch_skinny_tokens(SkinnyArgs args, int rows_per_group, hipStream_t stream) {
+  if (args.n < 1 || args.n > kSkinnyMaxN) return hipErrorInvalidValue;
+  // 16-byte loads of x; lane offsets of up to 64 token rows must stay below the "outside" offset of the kernel
+  if ((reinterpret_cast<uintptr_t>(args.b) & 15) != 0 || (size_t)args.k * 64 * 2 >= 0xFFFFFF00u) return hipErrorInvalidValue;
+  SkinnyArgs pass;
+  if (hipError_t st = skinny_split_setup(args, pass); st != hipSuccess) return st;
+  hipError_t st;
+  switch (rows_per_group) {
+    case 32: st = launch_skinny_tokens_cfg<16, 1>(pass, stream); break;
+    case 64: st = launch_skinny_tokens_cfg<8, 2>(pass, stream); break;
+    case 128: st = launch_skinny_tokens_cfg<8, 4>(pass, stream); break;
+    default: return hipErrorInvalidValue;
+  }
+  if (st != hipSuccess || args.splits <= 1) return st;
+  return launch_split_reduce(args.split_ws, args.splits, (size_t)args.m * args.n, nullptr, args.d, 1.f, 0.f, 0, args.d_f16,
+                             args.bias, args.bias_f16, args.m, stream);
+}
+
+template <int NW, int R>
+static hipError_t launch_skinny_group_cfg(const SkinnyGroupArgs& g, int blocks, int tokens, hipStream_t stream) {
+  if (tokens > 32) hipLaunchKernelGGL((skinny_group_kernel<NW, (R > 2 ? 2 : R), 64>), dim3(blocks), dim3(64 * NW), 0, stream, g);
+  else if (tokens > 16) hipLaunchKernelGGL((skinny_group_kernel<NW, R, 32>), dim3(blocks), dim3(64 * NW), 0, stream, g);
+  else hipLaunchKernelGGL((skinny_group_kernel<NW, R, 16>), dim3(blocks), dim3(64 * NW), 0, stream, g);
+  return hipGetLastError();
+}
+
+hipError_t launch_skinny_group(SkinnyGroupArgs g, int rows_per_group, hipStream_t stream) {
+  if (g.count < 1 || g.count > kSkinnyMaxGroup) return hipErrorInvalidValue;
+  const int tokens = g.problem[0].n;
+  if (tokens < 1 || tokens > kSkinnyMaxN) return hipErrorInvalidValue;
+  if (rows_per_group != 32 && rows_per_group != 64 && rows_per_group != 128) return hipErrorInvalidValue;
+  const int rows = (rows_per_group == 128 && tokens > 32) ? 64 : rows_per_group;  // as launch_skinny_tokens_cfg does
+  int blocks = 0;
+  for (int i = 0; i < g.count; ++i) {
+    SkinnyArgs& p = g.problem[i];
+    if (p.n != tokens || p.m <= 0 || p.k <= 0 || !p.prep || !p.b || !p.d) return hipErrorInvalidValue;
+    // 16-byte loads of x; lane offsets of up to 64 token rows must stay below the "outside" offset of the kernel
+    if ((reinterpret_cast<uintptr_t>(p.b) & 15) != 0 || (size_t)p.k * 64 * 2 >= 0xFFFFFF00u) return hipErrorInvalidValue;
+    p.splits = 1;
+    p.chunks_per_split = p.kc_total;
+    p.split_ws = nullptr;
+    g.first_block[i] = blocks;
+    blocks += (p.m + rows - 1) / rows;
+  }
+  g.first_block[g.count] = blocks;
+  switch (rows_per_group) {
+    case 32: return launch_skinny_group_cfg<16, 1>(g, blocks, tokens, stream);
+    case 64: return launch_skinny_group_cfg<8, 2>(g, blocks, tokens, stream);
+    default: return launch_skinny_group_cfg<8, 4>(g, blocks, tokens, stream);
+  }
+}
+
+}  // namespace onebit
