@@ -136,6 +136,16 @@ int onebit_sparse_linear_prepared_grouped(const onebit_linear_problem *problems,
                                           int y_dtype, void *stream);
 
 /*
+ * Both linear-layer forms for 16-bit activations of either type: x_dtype fp16 or bf16, y_dtype fp32 or the type of x,
+ * bias_dtype any of the three codes. bf16 activations are multiplied as they are (v_smfmac bf16, fp32 accumulation); the
+ * result is rounded once.
+ */
+int onebit_sparse_linear_prepared_typed(const void *prepared, const void *x, const void *bias, void *y, int tokens, int m,
+                                        int k, int x_dtype, int bias_dtype, int y_dtype, void *stream);
+int onebit_sparse_linear_prepared_grouped_typed(const onebit_linear_problem *problems, int count, int tokens, int x_dtype,
+                                                int bias_dtype, int y_dtype, void *stream);
+
+/*
  * Packs a dense fp16 weight (m x k, row-major, device) into the stored operands a (m*k/16 bytes) and e
  * (m*k/8 bytes) on the GPU. Replaces the tensor-op pipeline of BinaryLinear_2_4.pack
  * (onebit_sparse_mul/__init__.py:130-145 with _semi_structured_conversions.py:54-179,286-314): prune != 0 first

@@ -131,6 +131,9 @@ class PreparedWeight:
         return _native.linear_prepared(self.buffer, x, out, self.m, self.k, bias=bias)
 
 
+_BIAS_TYPES = (torch.float16, torch.bfloat16, torch.float32)  # the kernels read a bias of any of them
+
+
 class BinaryLinear_2_4(nn.Module):
     """1-bit 2:4 sparse linear layer: y = x @ W.T (+ bias when one has been assigned), W (outfeatures, infeatures)
     stored at 1.5 bits per weight. Reference: onebit_sparse_mul/__init__.py:101-145."""
@@ -138,9 +141,10 @@ class BinaryLinear_2_4(nn.Module):
     def __init__(self, infeatures: int, outfeatures: int, out_dtype=None):
         """out_dtype: dtype of the kernel's result. None (default): float16 for float16 activations (the sums are
         accumulated in fp32 and rounded once; a sum of infeatures/2 terms of +-x can exceed float16's range for large
-        activations) and float32 for every other activation dtype, so that the only precision loss is the cast of x
-        to float16. torch.float32 returns the reference layer's fp32 product for float16 activations as well
-        (onebit_sparse_mul/__init__.py:12-14: cuda_binary_mul returns an fp32 C)."""
+        activations), bfloat16 for bfloat16 activations (which are multiplied as they are) and float32 for every other
+        activation dtype, so that the only precision loss is the cast of x to float16. torch.float32 returns the
+        reference layer's fp32 product for 16-bit activations as well (onebit_sparse_mul/__init__.py:12-14:
+        cuda_binary_mul returns an fp32 C)."""
         super().__init__()
         if infeatures % 32 != 0 or outfeatures % 64 != 0:
             raise ValueError("`infeatures` must be divisible by 32 and `outfeatures` by 64.")
@@ -188,6 +192,12 @@ class BinaryLinear_2_4(nn.Module):
             self.vaild = True
         self._prepared = None
 
+    def _kernel_types(self, x_dtype):
+        """(type the kernel reads, type it writes) for activations of x_dtype: bf16 as it is, everything else as fp16."""
+        if x_dtype == torch.bfloat16 and self.out_dtype != torch.float16:
+            return torch.bfloat16, self.out_dtype or torch.bfloat16
+        return torch.float16, self.out_dtype or (torch.float16 if x_dtype == torch.float16 else torch.float32)
+
     def forward(self, x):
         if not self.vaild:
             raise NotImplementedError("the BinaryLinear_2_4 layer holds no packed weight: call pack() first")
@@ -196,11 +206,14 @@ class BinaryLinear_2_4(nn.Module):
         lead = x.shape[:-1]
         if x.numel() == 0:  # an empty batch: nothing to launch
             return x.new_zeros(*lead, self.outfeatures)
-        tokens = x.reshape(-1, self.infeatures).to(torch.float16).contiguous()
         bias = self.bias
-        if bias is not None and (bias.dtype not in (torch.float16, torch.float32) or bias.device != x.device):
+        if bias is not None and (bias.dtype not in _BIAS_TYPES or bias.device != x.device):
             bias = bias.to(device=x.device, dtype=torch.float32)
-        out_dtype = self.out_dtype or (torch.float16 if x.dtype == torch.float16 else torch.float32)
+        if x.dtype is torch.float16:
+            in_dtype, out_dtype = torch.float16, self.out_dtype or torch.float16
+        else:
+            in_dtype, out_dtype = self._kernel_types(x.dtype)
+        tokens = x.reshape(-1, self.infeatures).to(in_dtype).contiguous()
         # one kernel: reads the tokens where they lie, adds the bias, writes (tokens, outfeatures)
         y = self._prepared.linear(tokens, bias=bias.contiguous() if bias is not None else None, out_dtype=out_dtype)
         y = y.reshape(*lead, self.outfeatures)
@@ -223,18 +236,18 @@ def forward_grouped(layers, xs):
             raise NotImplementedError("a BinaryLinear_2_4 layer holds no packed weight: call pack() first")
         if layer._prepared is None or layer._prepared.buffer.device != x.device:
             layer._prepared = PreparedWeight(layer.packed_binary_sparse.to(x.device), layer.meta.to(x.device))
-        if id(x) not in flat:  # inputs shared by several layers are made contiguous fp16 once
-            t = x.reshape(-1, layer.infeatures).to(torch.float16).contiguous()
-            flat[id(x)] = t.clone() if t.data_ptr() % 16 else t
-        prepared.append(flat[id(x)])
+        in_dtype = layer._kernel_types(x.dtype)[0]
+        if (id(x), in_dtype) not in flat:  # inputs shared by several layers are made contiguous and 16-bit once
+            t = x.reshape(-1, layer.infeatures).to(in_dtype).contiguous()
+            flat[id(x), in_dtype] = t.clone() if t.data_ptr() % 16 else t
+        prepared.append(flat[id(x), in_dtype])
     tokens = prepared[0].shape[0]
-    out_dtypes = {layer.out_dtype or (torch.float16 if x.dtype == torch.float16 else torch.float32)
-                  for layer, x in zip(layers, xs)}
-    bias_dtypes = {layer.bias.dtype if layer.bias.dtype in (torch.float16, torch.float32) else torch.float32
+    types = {layer._kernel_types(x.dtype) for layer, x in zip(layers, xs)}
+    bias_dtypes = {layer.bias.dtype if layer.bias.dtype in _BIAS_TYPES else torch.float32
                    for layer in layers if layer.bias is not None}
-    if tokens == 0 or len(out_dtypes) > 1 or len(bias_dtypes) > 1 or any(t.shape[0] != tokens for t in prepared):
+    if tokens == 0 or len(types) > 1 or len(bias_dtypes) > 1 or any(t.shape[0] != tokens for t in prepared):
         return [layer(x) for layer, x in zip(layers, xs)]  # nothing to share: the layers one by one
-    out_dtype = out_dtypes.pop()
+    out_dtype = types.pop()[1]
     problems, ys = [], []
     for layer, x, t in zip(layers, xs, prepared):
         bias = layer.bias

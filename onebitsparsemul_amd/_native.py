@@ -17,7 +17,8 @@ EXPORTS = (
     "onebit_sparse_set_skinny_enabled", "onebit_sparse_set_skinny_rows", "onebit_sparse_set_split_k", "onebit_sparse_set_pad_b", "onebit_sparse_describe_launch", "onebit_sparse_set_weight_cache", "onebit_sparse_clear_weight_cache", "onebit_sparse_release_buffers",
     "onebit_sparse_measure_smfmac_rate", "onebit_sparse_device_info",
     "onebit_sparse_describe_launch_for", "onebit_sparse_measure_smfmac_rate_shape",
-    "onebit_sparse_linear_prepared_grouped", "onebit_sparse_pack_typed",
+    "onebit_sparse_linear_prepared_grouped", "onebit_sparse_pack_typed", "onebit_sparse_linear_prepared_typed",
+    "onebit_sparse_linear_prepared_grouped_typed",
 )
 
 
@@ -54,6 +55,10 @@ def lib():
         L.onebit_sparse_linear_prepared_grouped.argtypes = [ctypes.POINTER(LinearProblem), i32, i32, i32, i32, vp]
         L.onebit_sparse_pack.restype = i32
         L.onebit_sparse_pack.argtypes = [vp, i32, i32, i32, vp, vp, i32, vp]
+        L.onebit_sparse_linear_prepared_typed.restype = i32
+        L.onebit_sparse_linear_prepared_typed.argtypes = [vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]
+        L.onebit_sparse_linear_prepared_grouped_typed.restype = i32
+        L.onebit_sparse_linear_prepared_grouped_typed.argtypes = [ctypes.POINTER(LinearProblem), i32, i32, i32, i32, i32, vp]
         L.onebit_sparse_pack_typed.restype = i32
         L.onebit_sparse_pack_typed.argtypes = [vp, i32, i32, i32, i32, vp, vp, i32, vp]
         L.onebit_sparse_last_error.restype = ctypes.c_char_p
@@ -95,6 +100,18 @@ def last_error():
 def _check(rc):
     if rc != 0:
         raise RuntimeError(f"libonebitmul: {last_error()} (status {rc})")
+
+
+_TYPE_CODES = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
+LINEAR_TYPES = (torch.float16, torch.bfloat16)  # of the linear layer's activations; its result has x's type or is fp32
+
+
+def _linear_codes(x, y, bias):  # of the grouped form
+    if y.dtype != torch.float32 and y.dtype != x.dtype:
+        raise TypeError(f"y must be float32 or of x's type ({x.dtype}), got {y.dtype}")
+    if bias is not None and bias.dtype not in _TYPE_CODES:
+        raise TypeError(f"bias must be float32, float16 or bfloat16, got {bias.dtype}")
+    return _TYPE_CODES[x.dtype], _TYPE_CODES[bias.dtype] if bias is not None else F16, _TYPE_CODES[y.dtype]
 
 
 def _dtype_code(t):
@@ -184,52 +201,56 @@ def matmul_prepared(prepared, b, d, m, n, k, c=None, alpha=1.0, beta=0.0, static
 
 
 def linear_prepared(prepared, x, y, m, k, bias=None):
-    """y (tokens, m) = x (tokens, k) @ W.T (+ bias), x fp16 and y fp16 / fp32, both token-major and contiguous."""
+    """y (tokens, m) = x (tokens, k) @ W.T (+ bias), x fp16 or bf16 and y of its type or fp32, both token-major and
+    contiguous."""
     dev = _require_cuda(prepared, x, y, bias)
     tokens = x.shape[0]
-    if x.dtype != torch.float16 or tuple(x.shape) != (tokens, k):
-        raise ValueError("x must be float16 of shape (tokens, k)")
+    if x.dtype not in LINEAR_TYPES or tuple(x.shape) != (tokens, k):
+        raise ValueError("x must be float16 or bfloat16 of shape (tokens, k)")
     if tuple(y.shape) != (tokens, m) or (bias is not None and tuple(bias.shape) != (m,)):
         raise ValueError("y must have shape (tokens, m) and bias (m,)")
     if prepared.numel() != _prepared_bytes_fast(m, k):
         raise ValueError("prepared operand does not match m, k")
+    if y.dtype is not x.dtype and y.dtype is not torch.float32:
+        raise TypeError(f"y must be float32 or of x's type ({x.dtype}), got {y.dtype}")
     with _on_device(dev):
-        _check(lib().onebit_sparse_linear_prepared(
+        _check(lib().onebit_sparse_linear_prepared_typed(
             prepared.data_ptr(), x.data_ptr(), bias.data_ptr() if bias is not None else None, y.data_ptr(), tokens, m, k,
-            _dtype_code(bias) if bias is not None else F16, _dtype_code(y), _stream(x)))
+            _TYPE_CODES[x.dtype], _TYPE_CODES[bias.dtype] if bias is not None else F16, _TYPE_CODES[y.dtype], _stream(x)))
     return y
 
 
 def linear_prepared_grouped(problems):
     """Several products y_i = x_i @ W_i.T (+ bias_i) with the same token count in one call (one launch per 16 problems
-    when tokens <= 64). problems: sequence of (prepared, x, y, m, k, bias or None); all y of one dtype, all biases of one."""
+    when tokens <= 64). problems: sequence of (prepared, x, y, m, k, bias or None); all x of one dtype (fp16 or bf16), all y
+    of one, all biases of one."""
     if not problems:
         return
-    tokens = problems[0][1].shape[0]
+    tokens, x_type = problems[0][1].shape[0], problems[0][1].dtype
     table = (LinearProblem * len(problems))()
     dev = None
-    bias_code, y_code = F16, None
+    x_code, bias_code, y_code = None, None, None
     for i, (prepared, x, y, m, k, bias) in enumerate(problems):
         dev = _require_cuda(prepared, x, y, bias)
-        if x.dtype != torch.float16 or tuple(x.shape) != (tokens, k):
-            raise ValueError("every x must be float16 of shape (tokens, k) with the same token count")
+        if x.dtype not in LINEAR_TYPES or x.dtype != x_type or tuple(x.shape) != (tokens, k):
+            raise ValueError("every x must be float16 or bfloat16, all alike, of shape (tokens, k) with the same token count")
         if tuple(y.shape) != (tokens, m) or (bias is not None and tuple(bias.shape) != (m,)):
             raise ValueError("y must have shape (tokens, m) and bias (m,)")
         if prepared.numel() != _prepared_bytes_fast(m, k):
             raise ValueError("prepared operand does not match m, k")
-        if y_code is not None and _dtype_code(y) != y_code:
+        x_code, own_bias_code, own_y_code = _linear_codes(x, y, bias)
+        if y_code is not None and own_y_code != y_code:
             raise TypeError("all results must have the same dtype")
-        y_code = _dtype_code(y)
+        y_code = own_y_code
         if bias is not None:
-            code = _dtype_code(bias)
-            if any(p[5] is not None and _dtype_code(p[5]) != code for p in problems[:i]):
+            if bias_code is not None and own_bias_code != bias_code:
                 raise TypeError("all biases must have the same dtype")
-            bias_code = code
+            bias_code = own_bias_code
         table[i] = LinearProblem(prepared.data_ptr(), x.data_ptr(), bias.data_ptr() if bias is not None else None,
                                  y.data_ptr(), m, k)
     with _on_device(dev):
-        _check(lib().onebit_sparse_linear_prepared_grouped(table, len(problems), tokens, bias_code, y_code,
-                                                           _stream(problems[0][1])))
+        _check(lib().onebit_sparse_linear_prepared_grouped_typed(
+            table, len(problems), tokens, x_code, F16 if bias_code is None else bias_code, y_code, _stream(problems[0][1])))
 
 
 def _check_stored_operands(a, meta, c, d, m, n, k):
@@ -301,19 +322,16 @@ def measure_smfmac_rate(random_operands=True, iterations=50000, shape=SMFMAC_32X
     return out.value
 
 
-_WEIGHT_CODES = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
-
-
 def pack_weight(weight, prune=True, layout=META_REFERENCE):
     """dense fp16, bf16 or fp32 (m, k) on the GPU -> (a uint8 (k/2, m/8), meta int16 (m, k/16)), the stored operands."""
     dev = _require_cuda(weight)
-    if weight.dtype not in _WEIGHT_CODES or weight.dim() != 2:
+    if weight.dtype not in _TYPE_CODES or weight.dim() != 2:
         raise TypeError("weight must be a 2-dimensional float16, bfloat16 or float32 tensor")
     m, k = weight.shape
     a = torch.empty((k // 2, m // 8), dtype=torch.uint8, device=dev)
     meta = torch.empty((m, k // 16), dtype=torch.int16, device=dev)
     with _on_device(dev):
-        _check(lib().onebit_sparse_pack_typed(weight.data_ptr(), _WEIGHT_CODES[weight.dtype], m, k, 1 if prune else 0,
+        _check(lib().onebit_sparse_pack_typed(weight.data_ptr(), _TYPE_CODES[weight.dtype], m, k, 1 if prune else 0,
                                               a.data_ptr(), meta.data_ptr(), layout, _stream(weight)))
     return a, meta
 

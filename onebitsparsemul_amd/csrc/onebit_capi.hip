@@ -140,6 +140,17 @@ int check_dtype(int c_dtype, int d_dtype) {
   return ONEBIT_OK;
 }
 
+// The linear layer's types: 16-bit activations, a result of their type or fp32, any bias.
+int check_linear_dtypes(int x_dtype, int bias_dtype, int y_dtype) {
+  if (x_dtype != ONEBIT_DTYPE_F16 && x_dtype != ONEBIT_DTYPE_BF16)
+    return fail(ONEBIT_ERR_ARGUMENT, "x dtype code must be 1 (fp16) or 2 (bf16), got %d", x_dtype);
+  if (y_dtype != ONEBIT_DTYPE_F32 && y_dtype != x_dtype)
+    return fail(ONEBIT_ERR_ARGUMENT, "y dtype code must be 0 (fp32) or that of x (%d), got %d", x_dtype, y_dtype);
+  if (bias_dtype < ONEBIT_DTYPE_F32 || bias_dtype > ONEBIT_DTYPE_BF16)
+    return fail(ONEBIT_ERR_ARGUMENT, "bias dtype code must be 0 (fp32), 1 (fp16) or 2 (bf16), got %d", bias_dtype);
+  return ONEBIT_OK;
+}
+
 // Tile and number of K splits of the main kernel. The time is rounds of resident workgroups times one workgroup's K
 // loop; the choice among the tiles, and among splits of K that fill idle compute units at the price of a second launch
 // and of writing and re-reading fp32 partial sums, comes from a cost model fitted to measurements on MI355X
@@ -532,9 +543,16 @@ int onebit_sparse_matmul_prepared_static(const void* prepared, const void* b, co
 
 int onebit_sparse_linear_prepared(const void* prepared, const void* x, const void* bias, void* y, int tokens, int m,
                                   int k, int bias_dtype, int y_dtype, void* stream) {
-  g_last_error.clear();
   if (int rc = check_shape(m, tokens, k)) return rc;
   if (int rc = check_dtype(bias_dtype, y_dtype)) return rc;
+  return onebit_sparse_linear_prepared_typed(prepared, x, bias, y, tokens, m, k, ONEBIT_DTYPE_F16, bias_dtype, y_dtype, stream);
+}
+
+int onebit_sparse_linear_prepared_typed(const void* prepared, const void* x, const void* bias, void* y, int tokens, int m,
+                                        int k, int x_dtype, int bias_dtype, int y_dtype, void* stream) {
+  g_last_error.clear();
+  if (int rc = check_shape(m, tokens, k)) return rc;
+  if (int rc = check_linear_dtypes(x_dtype, bias_dtype, y_dtype)) return rc;
   if (!prepared || !x || !y) return fail(ONEBIT_ERR_ARGUMENT, "null operand pointer");
   if ((reinterpret_cast<uintptr_t>(x) & 15) != 0) return fail(ONEBIT_ERR_ARGUMENT, "x must be 16-byte aligned");
   const int kc_total = (k + onebit::kChunkK - 1) / onebit::kChunkK;
@@ -550,9 +568,10 @@ int onebit_sparse_linear_prepared(const void* prepared, const void* x, const voi
     args.m = m; args.n = tokens; args.k = k;
     args.kc_total = kc_total;
     args.alpha = 1.f; args.beta = 0.f;
-    args.d_f16 = y_dtype == ONEBIT_DTYPE_F16;
+    args.d_f16 = y_dtype != ONEBIT_DTYPE_F32;
     args.bias = bias;
-    args.bias_f16 = bias_dtype == ONEBIT_DTYPE_F16;
+    args.bias_type = bias_dtype;
+    args.bf16 = x_dtype == ONEBIT_DTYPE_BF16;
     if (int rc = setup_skinny_split(args, plan.splits, static_cast<hipStream_t>(stream), nullptr); rc != ONEBIT_OK) return rc;
     ONEBIT_HIP(onebit::launch_skinny_tokens(args, plan.rows_or_tile, static_cast<hipStream_t>(stream)));
     return ONEBIT_OK;
@@ -575,9 +594,10 @@ int onebit_sparse_linear_prepared(const void* prepared, const void* x, const voi
   args.d = y;
   args.m = m; args.n = tokens; args.k = k;
   args.kc_total = kc_total;
-  args.d_f16 = y_dtype == ONEBIT_DTYPE_F16;
+  args.d_f16 = y_dtype != ONEBIT_DTYPE_F32;
   args.bias = bias;
-  args.bias_f16 = bias_dtype == ONEBIT_DTYPE_F16;
+  args.bias_type = bias_dtype;
+  args.bf16 = x_dtype == ONEBIT_DTYPE_BF16;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (plan.splits > 1) {
     int device = 0;
@@ -600,9 +620,15 @@ int onebit_sparse_linear_prepared(const void* prepared, const void* x, const voi
 
 int onebit_sparse_linear_prepared_grouped(const onebit_linear_problem* problems, int count, int tokens, int bias_dtype,
                                           int y_dtype, void* stream) {
+  if (int rc = check_dtype(bias_dtype, y_dtype)) return rc;
+  return onebit_sparse_linear_prepared_grouped_typed(problems, count, tokens, ONEBIT_DTYPE_F16, bias_dtype, y_dtype, stream);
+}
+
+int onebit_sparse_linear_prepared_grouped_typed(const onebit_linear_problem* problems, int count, int tokens, int x_dtype,
+                                                int bias_dtype, int y_dtype, void* stream) {
   g_last_error.clear();
   if (!problems || count < 1) return fail(ONEBIT_ERR_ARGUMENT, "problems must point to at least one problem (count = %d)", count);
-  if (int rc = check_dtype(bias_dtype, y_dtype)) return rc;
+  if (int rc = check_linear_dtypes(x_dtype, bias_dtype, y_dtype)) return rc;
   for (int i = 0; i < count; ++i) {
     const onebit_linear_problem& q = problems[i];
     if (int rc = check_shape(q.m, tokens, q.k)) return rc;
@@ -617,7 +643,8 @@ int onebit_sparse_linear_prepared_grouped(const onebit_linear_problem* problems,
   if (tokens > onebit::kSkinnyMaxN || !g_skinny_enabled) {
     for (int i = 0; i < count; ++i) {
       const onebit_linear_problem& q = problems[i];
-      if (int rc = onebit_sparse_linear_prepared(q.prepared, q.x, q.bias, q.y, tokens, q.m, q.k, bias_dtype, y_dtype, stream))
+      if (int rc = onebit_sparse_linear_prepared_typed(q.prepared, q.x, q.bias, q.y, tokens, q.m, q.k, x_dtype, bias_dtype,
+                                                       y_dtype, stream))
         return rc;
     }
     return ONEBIT_OK;
@@ -644,9 +671,10 @@ int onebit_sparse_linear_prepared_grouped(const onebit_linear_problem* problems,
       args.m = q.m; args.n = tokens; args.k = q.k;
       args.kc_total = (q.k + onebit::kChunkK - 1) / onebit::kChunkK;
       args.alpha = 1.f; args.beta = 0.f;
-      args.d_f16 = y_dtype == ONEBIT_DTYPE_F16;
+      args.d_f16 = y_dtype != ONEBIT_DTYPE_F32;
       args.bias = q.bias;
-      args.bias_f16 = bias_dtype == ONEBIT_DTYPE_F16;
+      args.bias_type = bias_dtype;
+      args.bf16 = x_dtype == ONEBIT_DTYPE_BF16;
     }
     ONEBIT_HIP(onebit::launch_skinny_group(group, rows, static_cast<hipStream_t>(stream)));
   }

@@ -21,9 +21,14 @@
 
 namespace onebit {
 
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half16_t __attribute__((ext_vector_type(16)));
+typedef __bf16 bfloat2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bfloat8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bfloat16x_t __attribute__((ext_vector_type(16)));
+typedef float float2v_t __attribute__((ext_vector_type(2)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
 typedef float float4v_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
@@ -76,15 +81,48 @@ __device__ __forceinline__ AChunk load_a_chunk_lds(const char* block, int lane) 
   return r;
 }
 
-// fp16 1.0 in both halves, held in a vector register: v_and_or_b32 can then take the sign mask as its only
+// Codes of element types at run time, as in the C ABI.
+enum ElementType { kF32 = 0, kF16 = 1, kBF16 = 2 };
+
+// The 16-bit floating types. The kernels are fp16 by default; the token-major form also exists for bf16 activations
+// (BF16 = true): the same operand layout and the same instructions with the other operand type, so only the constant that
+// the signs are put on, the SMFMAC itself and the rounding of 16-bit results differ.
+template <bool BF16>
+__device__ __forceinline__ uint32_t round_pair(float low, float high) {  // two packed values, round to nearest even
+  const float2v_t x = {low, high};
+  if constexpr (BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bfloat2_t));
+  else return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, half2_t));
+}
+template <bool BF16>
+__device__ __forceinline__ uint16_t round_one(float x) {
+  if constexpr (BF16) return __builtin_bit_cast(uint16_t, (__bf16)x);
+  else return __builtin_bit_cast(uint16_t, (_Float16)x);
+}
+// element `at` of an array whose type is known at run time
+__device__ __forceinline__ float load_element(const void* p, int type, size_t at) {
+  if (type == kF32) return reinterpret_cast<const float*>(p)[at];
+  const uint16_t bits = reinterpret_cast<const uint16_t*>(p)[at];
+  return type == kF16 ? (float)__builtin_bit_cast(_Float16, bits) : __builtin_bit_cast(float, (uint32_t)bits << 16);
+}
+// the two values of a packed word, fp16 or bf16
+__device__ __forceinline__ float2v_t unpack_pair(uint32_t word, int type) {
+  if (type == kF16) {
+    const half2_t h = __builtin_bit_cast(half2_t, word);
+    return float2v_t{(float)h.x, (float)h.y};
+  }
+  return float2v_t{__builtin_bit_cast(float, word << 16), __builtin_bit_cast(float, word & 0xFFFF0000u)};
+}
+
+// 1.0 in both halves, held in a vector register: v_and_or_b32 can then take the sign mask as its only
 // literal operand (two literals in one instruction are not encodable, and cost a third instruction).
+template <bool BF16 = false>
 __device__ __forceinline__ uint32_t packed_one_in_vgpr() {
-  uint32_t one = 0x3C003C00u;
+  uint32_t one = BF16 ? 0x3F803F80u : 0x3C003C00u;
   asm volatile("" : "+v"(one));
   return one;
 }
 
-// Expand the eight +-1 values of K step `STEP` (0..7, compile time) into four packed fp16 registers:
+// Expand the eight +-1 values of K step `STEP` (0..7, compile time) into four packed registers:
 // two instructions per register (shift, and-or).
 template <int STEP>
 __device__ __forceinline__ half8_t expand_signs(const AChunk& a, uint32_t packed_one) {
@@ -93,7 +131,7 @@ __device__ __forceinline__ half8_t expand_signs(const AChunk& a, uint32_t packed
 #pragma unroll
   for (int p = 0; p < 4; ++p) {
     const int j = 4 * (STEP % 4) + p;
-    v[p] = ((w << j) & 0x80008000u) | packed_one;  // fp16 1.0 with the stored sign
+    v[p] = ((w << j) & 0x80008000u) | packed_one;  // 1.0 with the stored sign
   }
   return __builtin_bit_cast(half8_t, v);
 }
@@ -103,15 +141,35 @@ __device__ __forceinline__ half8_t expand_signs(const AChunk& a, uint32_t packed
 // allocation mixes the two register files and then copies whole accumulator tiles between them behind the SMFMAC
 // that produced them, which serialises the matrix pipe. Consecutive SMFMACs never share an accumulator, so no
 // wait states are needed between them.
-template <int STEP, bool PINNED = true>
+template <int STEP, bool PINNED = true, bool BF16 = false>
 __device__ __forceinline__ float16_t smfmac_step(const AChunk& a, half8_t av, half16_t bv, float16_t acc) {
   const int idx = (int)a.meta[STEP / 2];
   // Kernels whose consecutive SMFMACs update the same accumulator use the builtin, so that the compiler inserts
   // the wait states that dependency needs.
-  if (!PINNED) return __builtin_amdgcn_smfmac_f32_32x32x32_f16(av, bv, acc, idx, 0, STEP % 2);
-  if (STEP % 2 == 0) asm("v_smfmac_f32_32x32x32_f16 %0, %1, %2, %3" : "+a"(acc) : "v"(av), "v"(bv), "v"(idx));
-  else asm("v_smfmac_f32_32x32x32_f16 %0, %1, %2, %3 abid:1" : "+a"(acc) : "v"(av), "v"(bv), "v"(idx));
+  if constexpr (!PINNED && BF16)
+    return __builtin_amdgcn_smfmac_f32_32x32x32_bf16(__builtin_bit_cast(bfloat8_t, av), __builtin_bit_cast(bfloat16x_t, bv),
+                                                     acc, idx, 0, STEP % 2);
+  else if constexpr (!PINNED)
+    return __builtin_amdgcn_smfmac_f32_32x32x32_f16(av, bv, acc, idx, 0, STEP % 2);
+  else if constexpr (BF16 && STEP % 2 == 0)
+    asm("v_smfmac_f32_32x32x32_bf16 %0, %1, %2, %3" : "+a"(acc) : "v"(av), "v"(bv), "v"(idx));
+  else if constexpr (BF16)
+    asm("v_smfmac_f32_32x32x32_bf16 %0, %1, %2, %3 abid:1" : "+a"(acc) : "v"(av), "v"(bv), "v"(idx));
+  else if constexpr (STEP % 2 == 0)
+    asm("v_smfmac_f32_32x32x32_f16 %0, %1, %2, %3" : "+a"(acc) : "v"(av), "v"(bv), "v"(idx));
+  else
+    asm("v_smfmac_f32_32x32x32_f16 %0, %1, %2, %3 abid:1" : "+a"(acc) : "v"(av), "v"(bv), "v"(idx));
   return acc;
+}
+
+// One SMFMAC of the 16x16x64 shape through the builtin, index half ABID.
+template <int ABID, bool BF16 = false>
+__device__ __forceinline__ float4v_t smfmac16(half8_t av, half16_t bv, float4v_t acc, uint32_t idx) {
+  if constexpr (BF16)
+    return __builtin_amdgcn_smfmac_f32_16x16x64_bf16(__builtin_bit_cast(bfloat8_t, av), __builtin_bit_cast(bfloat16x_t, bv),
+                                                     acc, (int)idx, 0, ABID);
+  else
+    return __builtin_amdgcn_smfmac_f32_16x16x64_f16(av, bv, acc, (int)idx, 0, ABID);
 }
 
 // Wait states between the last SMFMAC and the first read of its result by a vector instruction.

@@ -146,7 +146,7 @@ __device__ __forceinline__ void load_b_piece_tokens(const char* wave_lds, int ks
 // The SMFMACs of one K step with the fetch work for the next step placed between them by hand: fetch(slot) runs right
 // behind SMFMAC number `slot`, and scheduling fences keep it there (the compiler would otherwise keep the
 // inline-assembly SMFMACs of the one-wavefront-per-SIMD tiles in one block, and order the rest as it likes).
-template <int STEP, bool PINNED, int FM, int FN, class Fetch>
+template <int STEP, bool PINNED, bool BF16, int FM, int FN, class Fetch>
 __device__ __forceinline__ void mfma_frags_fused(const AChunk (&a)[FM], const u32x4_t (&av)[FM], const u32x8_t (&bv)[FN],
                                                  float16_t (&acc)[FM][FN], Fetch&& fetch) {
 #pragma unroll
@@ -154,7 +154,7 @@ __device__ __forceinline__ void mfma_frags_fused(const AChunk (&a)[FM], const u3
 #pragma unroll
     for (int fn = 0; fn < FN; ++fn) {
       __builtin_amdgcn_s_setprio(1);  // the wavefront that is about to issue an SMFMAC wins the arbitration on its SIMD
-      acc[fm][fn] = smfmac_step<STEP, PINNED>(a[fm], __builtin_bit_cast(half8_t, av[fm]),
+      acc[fm][fn] = smfmac_step<STEP, PINNED, BF16>(a[fm], __builtin_bit_cast(half8_t, av[fm]),
                                               __builtin_bit_cast(half16_t, bv[fn]), acc[fm][fn]);
       __builtin_amdgcn_s_setprio(0);
       __builtin_amdgcn_sched_barrier(0);
@@ -168,9 +168,10 @@ static __device__ __attribute__((aligned(16))) uint32_t g_zero16[4] = {0, 0, 0, 
 
 // TOKENS (with DMA only): the linear-layer form. p.b is x (p.n tokens x p.k, token-major), p.d is y (p.n tokens x
 // p.m), the epilogue is y = acc + bias; a tile column is a token.
-template <int WM, int WN, int FM, int FN, bool DMA, bool TOKENS = false, int KG = 1, bool M16 = false>
+template <int WM, int WN, int FM, int FN, bool DMA, bool TOKENS = false, int KG = 1, bool M16 = false, bool BF16 = false>
 __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gemm_kernel(GemmArgs p) {
   static_assert(!M16 || (DMA && KG == 1 && WN == 1 && FM == 4 && FN == 4), "the 16x16x64 form exists for the 512x128 four-wavefront tile");
+  static_assert(TOKENS || !BF16, "bf16 activations exist for the token-major form");
   static_assert(DMA || !TOKENS, "the token-major form uses the asynchronous copies");
   static_assert(DMA || KG == 1, "the two-group form uses the asynchronous copies");
   using TS = TileShape<WM, WN, FM, FN, KG>;
@@ -221,7 +222,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
   }
   const char* const wave_image = smem + wn * FN * (32 * kStageK * 2);  // first token row of this wavefront in stage 0
 
-  const uint32_t one = packed_one_in_vgpr();
+  const uint32_t one = packed_one_in_vgpr<BF16>();
   // 32x32x32 form: FM x FN tiles of 32 x 32; 16x16x64 form: 2 FM x 2 FN tiles of 16 x 16 (the other array has one element)
   float16_t acc[M16 ? 1 : FM][M16 ? 1 : FN];
   float4v_t acc16[M16 ? 2 * FM : 1][M16 ? 2 * FN : 1];
@@ -467,7 +468,10 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
         const half8_t a8 = __builtin_bit_cast(half8_t, av);
         const half16_t b16 = __builtin_bit_cast(half16_t, bv);
         // accumulators tied to accumulation registers, as in smfmac_step
-        if ((S & 1) == 0) asm("v_smfmac_f32_16x16x64_f16 %0, %1, %2, %3" : "+a"(c) : "v"(a8), "v"(b16), "v"(idx));
+        if constexpr (BF16) {
+          if ((S & 1) == 0) asm("v_smfmac_f32_16x16x64_bf16 %0, %1, %2, %3" : "+a"(c) : "v"(a8), "v"(b16), "v"(idx));
+          else asm("v_smfmac_f32_16x16x64_bf16 %0, %1, %2, %3 abid:1" : "+a"(c) : "v"(a8), "v"(b16), "v"(idx));
+        } else if ((S & 1) == 0) asm("v_smfmac_f32_16x16x64_f16 %0, %1, %2, %3" : "+a"(c) : "v"(a8), "v"(b16), "v"(idx));
         else asm("v_smfmac_f32_16x16x64_f16 %0, %1, %2, %3 abid:1" : "+a"(c) : "v"(a8), "v"(b16), "v"(idx));
       };
 
@@ -583,7 +587,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
 
 #define ONEBIT_FUSED_STAGE(S, WAITCNT, ISSUE_A)                                                                  \
       {                                                                                                            \
-        mfma_frags_fused<2 * (S), PINNED>(a_cur, av0, bv0, acc, [&](int slot) __attribute__((always_inline)) {     \
+        mfma_frags_fused<2 * (S), PINNED, BF16>(a_cur, av0, bv0, acc, [&](int slot) __attribute__((always_inline)) {     \
           ONEBIT_FETCH_SLOT((S), 1, bv1, 2 * (S) + 1, a_cur, av1)                                                  \
         });                                                                                                        \
         wait_vmcnt_lgkm0<(WAITCNT)>(); /* copies of stage S+1 landed; this wavefront's reads of stage S returned */ \
@@ -593,7 +597,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
           _Pragma("unroll") for (int fm = 0; fm < FM; ++fm) a_next[fm] = load_a_chunk_lds(a_frag_lds[fm], lane);   \
           __builtin_amdgcn_sched_barrier(0);                                                                       \
         }                                                                                                          \
-        mfma_frags_fused<2 * (S) + 1, PINNED>(a_cur, av1, bv1, acc, [&](int slot) __attribute__((always_inline)) { \
+        mfma_frags_fused<2 * (S) + 1, PINNED, BF16>(a_cur, av1, bv1, acc, [&](int slot) __attribute__((always_inline)) { \
           ONEBIT_COPY_SLOT(S, ISSUE_A)                                                                             \
           if constexpr ((S) < kStages - 1) {                                                                       \
             ONEBIT_FETCH_SLOT((S) + 1, 0, bv0, 2 * (S) + 2, a_cur, av0)                                            \
@@ -647,7 +651,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
             _Pragma("unroll") for (int fm = 0; fm < FM; ++fm) a_next[fm] = load_a_chunk_lds(a_frag_lds[fm], lane); \
             __builtin_amdgcn_sched_barrier(0);                                                                   \
           }                                                                                                      \
-          mfma_frags_fused<2 * (S) + KGV, false>(a_cur, AV, BV, acc, [&](int slot) __attribute__((always_inline)) { \
+          mfma_frags_fused<2 * (S) + KGV, false, BF16>(a_cur, AV, BV, acc, [&](int slot) __attribute__((always_inline)) { \
             ONEBIT_COPY_SLOT(S, ISSUE_A)                                                                         \
             if constexpr ((S) < kStages - 1) {                                                                   \
               ONEBIT_FETCH_SLOT((S) + 1, KGV, BV_NEXT, 2 * ((S) + 1) + KGV, a_cur, AV_NEXT)                      \
@@ -756,25 +760,21 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
   if constexpr (TOKENS) {
     // ---- epilogue of the linear-layer form: y[token][row] = acc + bias[row], fp16 (RNE) or fp32 ----
     const int token_lane = lane & 31;
-    auto bias_of = [&](int row) __attribute__((always_inline)) {
-      if (!p.bias) return 0.f;
-      return p.bias_f16 ? (float)reinterpret_cast<const _Float16*>(p.bias)[row] : reinterpret_cast<const float*>(p.bias)[row];
-    };
-    // COUNT (4 or 8) consecutive bias values starting at a row that is a multiple of COUNT, by 16-byte loads
+    auto bias_of = [&](int row) __attribute__((always_inline)) { return p.bias ? load_element(p.bias, p.bias_type, row) : 0.f; };
+    // COUNT (4 or 8) consecutive bias values starting at a row that is a multiple of COUNT, by 8- or 16-byte loads
     auto bias_vector = [&](int row, float* out, auto count_tag) __attribute__((always_inline)) {
       constexpr int COUNT = decltype(count_tag)::value;
 #pragma unroll
       for (int e = 0; e < COUNT; ++e) out[e] = 0.f;
       if (!p.bias) return;
-      if (p.bias_f16) {
-        if constexpr (COUNT == 8) {
-          const half8_t v = *reinterpret_cast<const half8_t*>(reinterpret_cast<const _Float16*>(p.bias) + row);
+      if (p.bias_type != kF32) {
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint16_t*>(p.bias) + row);
+        uint32_t words[COUNT / 2];
+        __builtin_memcpy(words, __builtin_assume_aligned(src, COUNT * 2), COUNT * 2);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) out[e] = (float)v[e];
-        } else {
-          const half4_t v = *reinterpret_cast<const half4_t*>(reinterpret_cast<const _Float16*>(p.bias) + row);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) out[e] = (float)v[e];
+        for (int e = 0; e < COUNT; e += 2) {
+          const float2v_t v = unpack_pair(words[e / 2], p.bias_type);
+          out[e] = v.x; out[e + 1] = v.y;
         }
       } else {
 #pragma unroll
@@ -801,12 +801,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
         // 32 rows as halves (64 bytes, four 16-byte pieces; piece j of token t stored at position j ^ ((t / 4) % 4), so
         // that the sixteen lanes that write one slot of sixteen consecutive tokens meet in no bank): half the LDS
         // traffic of the fp32 form below, same bits (one rounding of sum + bias).
-        typedef float float2v __attribute__((ext_vector_type(2)));
-        typedef _Float16 half2v __attribute__((ext_vector_type(2)));
         auto packed_rows = [&](const float* x, const float* b4) __attribute__((always_inline)) {
-          const float2v lo = {x[0] + b4[0], x[1] + b4[1]}, hi = {x[2] + b4[2], x[3] + b4[3]};
-          return u32x2_t{__builtin_bit_cast(uint32_t, __builtin_convertvector(lo, half2v)),
-                         __builtin_bit_cast(uint32_t, __builtin_convertvector(hi, half2v))};
+          return u32x2_t{round_pair<BF16>(x[0] + b4[0], x[1] + b4[1]), round_pair<BF16>(x[2] + b4[2], x[3] + b4[3])};
         };
         // bias of the four rows starting at `row` (a multiple of 4); rows at or past the end are never stored
         auto bias_rows = [&](int row, float* b4) __attribute__((always_inline)) {
@@ -880,10 +876,10 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
             if (token < p.n && row < row_limit) {
               float bias8[8];
               bias_vector(row, bias8, std::integral_constant<int, 8>{});
-              half8_t out;
+              u32x4_t out;
 #pragma unroll
-              for (int e = 0; e < 8; ++e) out[e] = (_Float16)(x[e] + bias8[e]);
-              *reinterpret_cast<half8_t*>(reinterpret_cast<_Float16*>(d_out) + (size_t)token * p.m + row) = out;
+              for (int e = 0; e < 4; ++e) out[e] = round_pair<BF16>(x[2 * e] + bias8[2 * e], x[2 * e + 1] + bias8[2 * e + 1]);
+              *reinterpret_cast<u32x4_t*>(reinterpret_cast<_Float16*>(d_out) + (size_t)token * p.m + row) = out;
             }
           }
         } else {
@@ -916,7 +912,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
             if (token < p.n && row < row_limit) {
               const float x = acc16[rt][ct][v] + bias_of(row);
               const size_t o = (size_t)token * p.m + row;
-              if (p.d_f16) reinterpret_cast<_Float16*>(d_out)[o] = (_Float16)x;
+              if (p.d_f16) reinterpret_cast<uint16_t*>(d_out)[o] = round_one<BF16>(x);
               else reinterpret_cast<float*>(d_out)[o] = x;
             }
           }
@@ -934,7 +930,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
           if (token < p.n && row < row_limit) {
             const float x = acc[fm][fn][v] + bias_of(row);
             const size_t o = (size_t)token * p.m + row;
-            if (p.d_f16) reinterpret_cast<_Float16*>(d_out)[o] = (_Float16)x;
+            if (p.d_f16) reinterpret_cast<uint16_t*>(d_out)[o] = round_one<BF16>(x);
             else reinterpret_cast<float*>(d_out)[o] = x;
           }
         }
@@ -1013,8 +1009,6 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
       // the LDS traffic of the fp32 form). A lane then reads eight such words (columns c .. c + 7 of a row pair),
       // separates low and high halves and stores 16 bytes of row r and 16 bytes of row r + 1.
       uint32_t* const words = reinterpret_cast<uint32_t*>(scratch);  // [16 row pairs][WCOLS]
-      typedef float float2v __attribute__((ext_vector_type(2)));
-      typedef _Float16 half2v __attribute__((ext_vector_type(2)));
       constexpr int PER_PAIR = WCOLS / 8;            // 8-column pieces per row pair
       constexpr int TASKS = 16 * PER_PAIR;           // (row pair, piece) per 32-row block
       constexpr int ITERS = (TASKS + 63) / 64;
@@ -1026,9 +1020,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
         if (!finishes(fm)) continue;  // the other K group stores this fragment
         const int row_base = row0 + fm * 32;
         auto pack = [&](float x0, float x1) __attribute__((always_inline)) {  // one packed conversion per register pair
-          float2v x = {x0, x1};
-          if constexpr (SCALE) x = float2v{p.alpha * x.x, p.alpha * x.y};
-          return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, half2v));
+          if constexpr (SCALE) return round_pair<false>(p.alpha * x0, p.alpha * x1);
+          else return round_pair<false>(x0, x1);
         };
         if constexpr (M16) {
           // registers (0, 1) and (2, 3) of a tile: rows 16 rh + 4 (lane / 16) + 2 h and the next, row pair
@@ -1220,13 +1213,13 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
   }
 }
 
-template <int WM, int WN, int FM, int FN, bool DMA, bool TOKENS = false, int KG = 1, bool M16 = false>
+template <int WM, int WN, int FM, int FN, bool DMA, bool TOKENS = false, int KG = 1, bool M16 = false, bool BF16 = false>
 static hipError_t launch_gemm_cfg(GemmArgs args, hipStream_t stream) {
   using TS = TileShape<WM, WN, FM, FN, KG>;
   args.tiles_m = (args.m + TS::BM - 1) / TS::BM;
   args.tiles_n = (args.n + TS::BN - 1) / TS::BN;
   const int lds = DMA ? TS::LDS_BYTES : TS::STAGE_BYTES;
-  auto kern = gemm_kernel<WM, WN, FM, FN, DMA, TOKENS, KG, M16>;
+  auto kern = gemm_kernel<WM, WN, FM, FN, DMA, TOKENS, KG, M16, BF16>;
   // the dynamic-LDS limit is a per-device attribute of the kernel; threads that race here set the same value
   static std::atomic<bool> attr_done[64] = {};
   int device = 0;

@@ -47,7 +47,7 @@ template <int VEC>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws, int splits, size_t stride,
                                                             const void* __restrict__ c, void* __restrict__ d,
                                                             size_t total, float alpha, float beta, int c_f16,
-                                                            int d_f16, const void* __restrict__ bias, int bias_f16,
+                                                            int d_type, const void* __restrict__ bias, int bias_type,
                                                             int row_length) {
   const size_t first = ((size_t)blockIdx.x * 256 + threadIdx.x) * VEC;
   if (first >= total) return;
@@ -75,35 +75,34 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   if (bias) {
     const size_t at = first % (size_t)row_length;  // row_length is a multiple of 4: a vector never wraps
 #pragma unroll
-    for (int j = 0; j < VEC; ++j)
-      x[j] += bias_f16 ? (float)reinterpret_cast<const _Float16*>(bias)[at + j] : reinterpret_cast<const float*>(bias)[at + j];
+    for (int j = 0; j < VEC; ++j) x[j] += load_element(bias, bias_type, at + j);
   }
   if (VEC == 4) {
-    if (d_f16) {
-      *reinterpret_cast<half4_t*>(reinterpret_cast<_Float16*>(d) + first) =
-          half4_t{(_Float16)x[0], (_Float16)x[1 % VEC], (_Float16)x[2 % VEC], (_Float16)x[3 % VEC]};
-    } else {
+    if (d_type == kF32)
       *reinterpret_cast<float4*>(reinterpret_cast<float*>(d) + first) = float4{x[0], x[1 % VEC], x[2 % VEC], x[3 % VEC]};
-    }
+    else
+      *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(d) + first) =
+          d_type == kF16 ? u32x2_t{round_pair<false>(x[0], x[1 % VEC]), round_pair<false>(x[2 % VEC], x[3 % VEC])}
+                         : u32x2_t{round_pair<true>(x[0], x[1 % VEC]), round_pair<true>(x[2 % VEC], x[3 % VEC])};
   } else {
-    if (d_f16) reinterpret_cast<_Float16*>(d)[first] = (_Float16)x[0];
-    else reinterpret_cast<float*>(d)[first] = x[0];
+    if (d_type == kF32) reinterpret_cast<float*>(d)[first] = x[0];
+    else reinterpret_cast<uint16_t*>(d)[first] = d_type == kF16 ? round_one<false>(x[0]) : round_one<true>(x[0]);
   }
 }
 
 // Second pass of a K split: ordered sum of the partial results and the epilogue (bias and row_length for the
 // token-major form, where element i of y takes bias[i % m]).
 hipError_t launch_split_reduce(const float* ws, int splits, size_t total, const void* c, void* d, float alpha,
-                                      float beta, int c_f16, int d_f16, const void* bias, int bias_f16, int row_length,
+                                      float beta, int c_f16, int d_type, const void* bias, int bias_type, int row_length,
                                       hipStream_t stream) {
   const bool vec = total % 4 == 0 && (reinterpret_cast<uintptr_t>(d) & 15) == 0 &&
                    (beta == 0.f || (reinterpret_cast<uintptr_t>(c) & 15) == 0) && (!bias || row_length % 4 == 0);
   if (vec)
     hipLaunchKernelGGL(splitk_reduce_kernel<4>, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream, ws,
-                       splits, total, c, d, total, alpha, beta, c_f16, d_f16, bias, bias_f16, row_length);
+                       splits, total, c, d, total, alpha, beta, c_f16, d_type, bias, bias_type, row_length);
   else
     hipLaunchKernelGGL(splitk_reduce_kernel<1>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, ws,
-                       splits, total, c, d, total, alpha, beta, c_f16, d_f16, bias, bias_f16, row_length);
+                       splits, total, c, d, total, alpha, beta, c_f16, d_type, bias, bias_type, row_length);
   return hipGetLastError();
 }
 

@@ -3,6 +3,22 @@
 
 namespace onebit {
 
+template <bool BF16>
+static hipError_t launch_tokens_tile(const GemmArgs& a, int tile_config, hipStream_t stream) {
+  switch (tile_config) {
+    case kTile256x128w: return launch_gemm_cfg<2, 2, 4, 2, true, true, 1, false, BF16>(a, stream);
+    case kTile128x128s: return launch_gemm_cfg<2, 2, 2, 2, true, true, 1, false, BF16>(a, stream);
+    case kTile512x128w8: return launch_gemm_cfg<4, 2, 4, 2, true, true, 1, false, BF16>(a, stream);
+    case kTile256x128w8: return launch_gemm_cfg<4, 2, 2, 2, true, true, 1, false, BF16>(a, stream);
+    case kTile128x128w8: return launch_gemm_cfg<2, 4, 2, 1, true, true, 1, false, BF16>(a, stream);
+    case kTile64x128: return launch_gemm_cfg<2, 2, 1, 2, true, true, 1, false, BF16>(a, stream);
+    case kTile128x128k2: return launch_gemm_cfg<2, 2, 2, 2, true, true, 2, false, BF16>(a, stream);
+    case kTile64x128k2: return launch_gemm_cfg<2, 2, 1, 2, true, true, 2, false, BF16>(a, stream);
+    case kTile512x128m16: return launch_gemm_cfg<4, 1, 4, 4, true, true, 1, true, BF16>(a, stream);
+    default: return hipErrorInvalidValue;  // the tiles the automatic choice uses
+  }
+}
+
 hipError_t launch_gemm_tokens(GemmArgs args, int tile_config, hipStream_t stream) {
   if (prepared_bytes(args.m, args.k) >= (size_t(1) << 32)) return hipErrorInvalidValue;  // 32-bit copy offsets
   if ((reinterpret_cast<uintptr_t>(args.b) & 15) != 0 || (size_t)args.k * 256 * 2 >= (size_t(1) << 32))
@@ -15,18 +31,7 @@ hipError_t launch_gemm_tokens(GemmArgs args, int tile_config, hipStream_t stream
   auto pass = [&](GemmArgs a) {
     a.vector_epilogue = (reinterpret_cast<uintptr_t>(a.d) & 15) == 0 && a.m % 8 == 0 &&
                         (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0;
-    switch (tile_config) {
-      case kTile256x128w: return launch_gemm_cfg<2, 2, 4, 2, true, true>(a, stream);
-      case kTile128x128s: return launch_gemm_cfg<2, 2, 2, 2, true, true>(a, stream);
-      case kTile512x128w8: return launch_gemm_cfg<4, 2, 4, 2, true, true>(a, stream);
-      case kTile256x128w8: return launch_gemm_cfg<4, 2, 2, 2, true, true>(a, stream);
-      case kTile128x128w8: return launch_gemm_cfg<2, 4, 2, 1, true, true>(a, stream);
-      case kTile64x128: return launch_gemm_cfg<2, 2, 1, 2, true, true>(a, stream);
-      case kTile128x128k2: return launch_gemm_cfg<2, 2, 2, 2, true, true, 2>(a, stream);
-      case kTile64x128k2: return launch_gemm_cfg<2, 2, 1, 2, true, true, 2>(a, stream);
-      case kTile512x128m16: return launch_gemm_cfg<4, 1, 4, 4, true, true, 1, true>(a, stream);
-      default: return hipErrorInvalidValue;  // the tiles the automatic choice uses
-    }
+    return a.bf16 ? launch_tokens_tile<true>(a, tile_config, stream) : launch_tokens_tile<false>(a, tile_config, stream);
   };
   if (args.splits <= 1) {
     args.splits = 1;
@@ -41,8 +46,8 @@ hipError_t launch_gemm_tokens(GemmArgs args, int tile_config, hipStream_t stream
   first.d_f16 = 0;
   first.bias = nullptr;
   if (hipError_t st = pass(first); st != hipSuccess) return st;
-  return launch_split_reduce(args.split_ws, args.splits, (size_t)args.m * args.n, nullptr, args.d, 1.f, 0.f, 0, args.d_f16,
-                             args.bias, args.bias_f16, args.m, stream);
+  return launch_split_reduce(args.split_ws, args.splits, (size_t)args.m * args.n, nullptr, args.d, 1.f, 0.f, 0,
+                             args.d_f16 && args.bf16 ? kBF16 : args.d_f16, args.bias, args.bias_type, args.m, stream);
 }
 
 }  // namespace onebit

@@ -29,9 +29,11 @@ struct GemmArgs {
   // take the slower element-copy variant. ldb (elements between B rows) is filled by the launcher.
   _Float16* b_pad;
   int ldb;
-  // linear-layer form (launch_gemm_tokens) only: m values added to every token's row of y, may be null
+  // linear-layer form (launch_gemm_tokens) only: m values added to every token's row of y, may be null; its type (ElementType);
+  // bf16 = 1: x is bf16, and so is a 16-bit y (d_f16 = 1)
   const void* bias;
-  int bias_f16;
+  int bias_type;
+  int bf16;
 };
 
 struct SkinnyArgs {
@@ -44,9 +46,11 @@ struct SkinnyArgs {
   float alpha, beta;
   int c_f16, d_f16;
   // token-major form (launch_skinny_tokens) only: b is x (n tokens x k), d is y (n tokens x m), alpha, beta and c are
-  // not used, bias (m values, may be null) is added to every token's row
+  // not used, bias (m values, may be null, of type bias_type) is added to every token's row; bf16 = 1: x is bf16, and so is
+  // a 16-bit y (d_f16 = 1)
   const void* bias;
-  int bias_f16;
+  int bias_type;
+  int bf16;
   // K split over workgroups (grid.y = splits), for few row groups over a long K: split s multiplies the K chunks
   // [s * chunks_per_split, +chunks_per_split) and writes raw fp32 sums to split_ws + s * m * n (laid out like the
   // result); a second kernel adds the splits in order and applies the epilogue. splits <= 1: one pass straight into d.
@@ -80,7 +84,7 @@ hipError_t launch_pack(const void* w, int dtype, void* a, void* e, int m, int k,
 // Second pass of a K split: ordered sum of the partial results and the epilogue (bias and row_length for the
 // token-major form, where element i of y takes bias[i % m]).
 hipError_t launch_split_reduce(const float* ws, int splits, size_t total, const void* c, void* d, float alpha,
-                                      float beta, int c_f16, int d_f16, const void* bias, int bias_f16, int row_length,
+                                      float beta, int c_f16, int d_type, const void* bias, int bias_type, int row_length,
                                       hipStream_t stream);
 
 // Split-K kernel for n <= 64; rows_per_group (32, 64 or 128) = weight rows one workgroup covers (n > 32: at most 64).

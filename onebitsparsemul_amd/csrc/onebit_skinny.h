@@ -40,7 +40,7 @@ constexpr int kSkinnyRegion = 8192;  // bytes of one B image
 enum SkinnyBMode { kSkinnyBFull = 0, kSkinnyBAny = 1, kSkinnyBTokens = 2, kSkinnyBRun = 3 };
 
 // The body of the split-K kernel for workgroup (block_x, block_y) of problem p: block_x = row group, block_y = K split.
-template <int NW, int R, int MODE, int NC>
+template <int NW, int R, int MODE, int NC, bool BF16 = false>
 __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block_x, const int block_y) {
   constexpr int NT = 64 * NW;
   constexpr int IMG_ROWS = kSkinnyRegion / (NC * 2);   // B rows per image: 256, 128 or 64
@@ -270,7 +270,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int h = 0; h < 2; ++h) acc16[r][h] = float4v_t{0.f, 0.f, 0.f, 0.f};
-  const uint32_t one = packed_one_in_vgpr();
+  const uint32_t one = packed_one_in_vgpr<BF16>();
   const int i16 = lane & 15, gb = lane >> 5, g16 = lane >> 4;
   // (32x32x32 form, NC >= 32; sixteen-column images use the 16x16x64 form further down)
   const int chunk8 = (NC >= 32 ? ((lane & 31) >> 4) * 4 : 0) + (i16 & 3);  // 8-byte piece of the 32-column fragment
@@ -352,10 +352,8 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
 #pragma unroll
           for (int q = 0; q < 4; ++q) av[q] = ((t[r].sign[h][F >> 1] << (4 * (F & 1) + q)) & 0x80008000u) | one;
           const half8_t a8 = __builtin_bit_cast(half8_t, av);
-          if ((F & 1) == 0)
-            acc16[r][h] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(a8, bf[F], acc16[r][h], (int)t[r].idx[h][F >> 1], 0, 0);
-          else
-            acc16[r][h] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(a8, bf[F], acc16[r][h], (int)t[r].idx[h][F >> 1], 0, 1);
+          acc16[r][h] = (F & 1) == 0 ? smfmac16<0, BF16>(a8, bf[F], acc16[r][h], t[r].idx[h][F >> 1])
+                                     : smfmac16<1, BF16>(a8, bf[F], acc16[r][h], t[r].idx[h][F >> 1]);
         }
   };
 
@@ -418,7 +416,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
               const half8_t av = expand_signs<STEP>(a[r], one);
 #pragma unroll
               for (int f = 0; f < NF; ++f)
-                acc[r][f] = smfmac_step<STEP, false>(a[r], av, bfrag[SET][OFFSET][f], acc[r][f]);
+                acc[r][f] = smfmac_step<STEP, false, BF16>(a[r], av, bfrag[SET][OFFSET][f], acc[r][f]);
             }
           }
         };
@@ -540,15 +538,14 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
         for (int w = 0; w < NW; ++w) sum += reinterpret_cast<const float*>(bs + w * kSkinnyRegion)[pos];
         const int row = round_row0 + local;
         if (token < p.n && row < p.m) {
-          if (p.bias) sum += p.bias_f16 ? (float)reinterpret_cast<const _Float16*>(p.bias)[row]
-                                        : reinterpret_cast<const float*>(p.bias)[row];
+          if (p.bias) sum += load_element(p.bias, p.bias_type, row);
           const size_t o = (size_t)token * p.m + row;
           // a B of one column is a token-major x of one token and its result column is y: the launcher sends such calls
           // here with their alpha, beta and C (element o of C in both layouts); the linear layer passes 1, 0, null
           sum = p.alpha * sum;
           if (p.beta != 0.f)
             sum = sum + p.beta * (p.c_f16 ? (float)reinterpret_cast<const _Float16*>(p.c)[o] : reinterpret_cast<const float*>(p.c)[o]);
-          if (p.d_f16) reinterpret_cast<_Float16*>(d_out)[o] = (_Float16)sum;
+          if (p.d_f16) reinterpret_cast<uint16_t*>(d_out)[o] = round_one<BF16>(sum);
           else reinterpret_cast<float*>(d_out)[o] = sum;
         }
       }
@@ -574,9 +571,9 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   }
 }
 
-template <int NW, int R, int MODE, int NC>
+template <int NW, int R, int MODE, int NC, bool BF16>
 __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_kernel(SkinnyArgs p) {
-  skinny_body<NW, R, MODE, NC>(p, blockIdx.x, blockIdx.y);
+  skinny_body<NW, R, MODE, NC, BF16>(p, blockIdx.x, blockIdx.y);
 }
 
 // Grouped form: several independent products y_i = x_i W_i^T + bias_i that share the token count, in one launch. The
@@ -585,18 +582,18 @@ __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_kernel(Skinn
 // the token-major body on that problem's arguments. Decode-sized products take a few microseconds each, of which the
 // launch itself and the ramp of the memory pipeline are a large part: one launch for the q / k / v or gate / up
 // projections of a layer pays them once.
-template <int NW, int R, int NC>
+template <int NW, int R, int NC, bool BF16>
 __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_group_kernel(SkinnyGroupArgs g) {
   int which = 0;
   for (int i = 1; i < g.count; ++i)
     if ((int)blockIdx.x >= g.first_block[i]) which = i;
-  skinny_body<NW, R, kSkinnyBTokens, NC>(g.problem[which], (int)blockIdx.x - g.first_block[which], 0);
+  skinny_body<NW, R, kSkinnyBTokens, NC, BF16>(g.problem[which], (int)blockIdx.x - g.first_block[which], 0);
 }
 
-template <int NW, int R, int MODE, int NC>
+template <int NW, int R, int MODE, int NC, bool BF16 = false>
 static hipError_t launch_skinny_mode(const SkinnyArgs& args, hipStream_t stream) {
   const int row_blocks = args.m / kRowBlock;
-  hipLaunchKernelGGL((skinny_kernel<NW, R, MODE, NC>), dim3((row_blocks + R - 1) / R, args.splits), dim3(64 * NW), 0,
+  hipLaunchKernelGGL((skinny_kernel<NW, R, MODE, NC, BF16>), dim3((row_blocks + R - 1) / R, args.splits), dim3(64 * NW), 0,
                      stream, args);
   return hipGetLastError();
 }

@@ -3,11 +3,16 @@
 
 namespace onebit {
 
+template <int NW, int R, bool BF16>
+static hipError_t launch_skinny_tokens_type(const SkinnyArgs& args, hipStream_t stream) {
+  if (args.n > 32) return launch_skinny_mode<NW, (R > 2 ? 2 : R), kSkinnyBTokens, 64, BF16>(args, stream);
+  if (args.n > 16) return launch_skinny_mode<NW, R, kSkinnyBTokens, 32, BF16>(args, stream);
+  return launch_skinny_mode<NW, R, kSkinnyBTokens, 16, BF16>(args, stream);
+}
+
 template <int NW, int R>
 static hipError_t launch_skinny_tokens_cfg(const SkinnyArgs& args, hipStream_t stream) {
-  if (args.n > 32) return launch_skinny_mode<NW, (R > 2 ? 2 : R), kSkinnyBTokens, 64>(args, stream);
-  if (args.n > 16) return launch_skinny_mode<NW, R, kSkinnyBTokens, 32>(args, stream);
-  return launch_skinny_mode<NW, R, kSkinnyBTokens, 16>(args, stream);
+  return args.bf16 ? launch_skinny_tokens_type<NW, R, true>(args, stream) : launch_skinny_tokens_type<NW, R, false>(args, stream);
 }
 
 hipError_t launch_skinny_tokens(SkinnyArgs args, int rows_per_group, hipStream_t stream) {
@@ -24,16 +29,23 @@ hipError_t launch_skinny_tokens(SkinnyArgs args, int rows_per_group, hipStream_t
     default: return hipErrorInvalidValue;
   }
   if (st != hipSuccess || args.splits <= 1) return st;
-  return launch_split_reduce(args.split_ws, args.splits, (size_t)args.m * args.n, nullptr, args.d, 1.f, 0.f, 0, args.d_f16,
-                             args.bias, args.bias_f16, args.m, stream);
+  return launch_split_reduce(args.split_ws, args.splits, (size_t)args.m * args.n, nullptr, args.d, 1.f, 0.f, 0,
+                             args.d_f16 && args.bf16 ? kBF16 : args.d_f16, args.bias, args.bias_type, args.m, stream);
+}
+
+template <int NW, int R, bool BF16>
+static hipError_t launch_skinny_group_type(const SkinnyGroupArgs& g, int blocks, int tokens, hipStream_t stream) {
+  const dim3 grid(blocks), threads(64 * NW);
+  if (tokens > 32) hipLaunchKernelGGL((skinny_group_kernel<NW, (R > 2 ? 2 : R), 64, BF16>), grid, threads, 0, stream, g);
+  else if (tokens > 16) hipLaunchKernelGGL((skinny_group_kernel<NW, R, 32, BF16>), grid, threads, 0, stream, g);
+  else hipLaunchKernelGGL((skinny_group_kernel<NW, R, 16, BF16>), grid, threads, 0, stream, g);
+  return hipGetLastError();
 }
 
 template <int NW, int R>
 static hipError_t launch_skinny_group_cfg(const SkinnyGroupArgs& g, int blocks, int tokens, hipStream_t stream) {
-  if (tokens > 32) hipLaunchKernelGGL((skinny_group_kernel<NW, (R > 2 ? 2 : R), 64>), dim3(blocks), dim3(64 * NW), 0, stream, g);
-  else if (tokens > 16) hipLaunchKernelGGL((skinny_group_kernel<NW, R, 32>), dim3(blocks), dim3(64 * NW), 0, stream, g);
-  else hipLaunchKernelGGL((skinny_group_kernel<NW, R, 16>), dim3(blocks), dim3(64 * NW), 0, stream, g);
-  return hipGetLastError();
+  return g.problem[0].bf16 ? launch_skinny_group_type<NW, R, true>(g, blocks, tokens, stream)
+                           : launch_skinny_group_type<NW, R, false>(g, blocks, tokens, stream);
 }
 
 hipError_t launch_skinny_group(SkinnyGroupArgs g, int rows_per_group, hipStream_t stream) {
@@ -45,7 +57,7 @@ hipError_t launch_skinny_group(SkinnyGroupArgs g, int rows_per_group, hipStream_
   int blocks = 0;
   for (int i = 0; i < g.count; ++i) {
     SkinnyArgs& p = g.problem[i];
-    if (p.n != tokens || p.m <= 0 || p.k <= 0 || !p.prep || !p.b || !p.d) return hipErrorInvalidValue;
+    if (p.n != tokens || p.bf16 != g.problem[0].bf16 || p.m <= 0 || p.k <= 0 || !p.prep || !p.b || !p.d) return hipErrorInvalidValue;
     // 16-byte loads of x; lane offsets of up to 64 token rows must stay below the "outside" offset of the kernel
     if ((reinterpret_cast<uintptr_t>(p.b) & 15) != 0 || (size_t)p.k * 64 * 2 >= 0xFFFFFF00u) return hipErrorInvalidValue;
     p.splits = 1;
