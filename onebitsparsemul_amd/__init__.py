@@ -23,10 +23,17 @@ __all__ = [
 ]
 
 
+_compiled = None
+
+
 def _binding():
-    """The compiled torch binding `onebit_sparse_cuda` (reference: onebit_sparse_mul/torch_kernel_cuda.cpp)."""
-    from . import onebit_sparse_cuda  # noqa: PLC0415  (compiled module, built in-tree)
-    return onebit_sparse_cuda
+    """The compiled torch binding `onebit_sparse_cuda` (reference: onebit_sparse_mul/torch_kernel_cuda.cpp), which also has the
+    host side of this package's own calls."""
+    global _compiled
+    if _compiled is None:
+        from . import onebit_sparse_cuda  # noqa: PLC0415  (compiled module, built in-tree)
+        _compiled = onebit_sparse_cuda
+    return _compiled
 
 
 def set_weight_cache(entries):
@@ -40,22 +47,10 @@ def clear_weight_cache():
     _native.clear_weight_cache()
 
 
-def _problem_shape(A, B, meta):
-    m, k = meta.shape[0], meta.shape[1] * 16
-    if A.dtype != torch.uint8 or A.numel() != m * k // 16:
-        raise ValueError(f"A must be uint8 with m*k/16 = {m * k // 16} bytes (shape (k/2, m/8)), got {tuple(A.shape)}")
-    if B.dim() != 2 or B.shape[0] != k:
-        raise ValueError(f"B must have shape (k={k}, n), got {tuple(B.shape)}")
-    return m, B.shape[1], k
-
-
 def cuda_binary_mul(A, B, meta):
     """C = W @ B with W the one-bit 2:4 weight stored as (A bits, meta); returns fp32 (m, n) on B's device.
     Reference: onebit_sparse_mul/__init__.py:12-15."""
-    m, n, _ = _problem_shape(A, B, meta)
-    C = torch.empty((m, n), dtype=torch.float32, device=B.device)
-    _binding().onebit_mul(A, B, meta, C)
-    return C
+    return _binding().binary_mul(A, B, meta)
 
 
 def cuda_binary_mul_(A, B, C, meta):
@@ -114,13 +109,10 @@ class PreparedWeight:
     def __init__(self, packed_binary_sparse, meta, layout=_native.META_REFERENCE):
         self.m = meta.shape[0]
         self.k = meta.shape[1] * 16
-        self.buffer = _native.prepare(packed_binary_sparse, meta, self.m, self.k, layout)
+        self.buffer = _binding().prepare(packed_binary_sparse, meta, self.m, self.k, layout)
 
     def matmul(self, b, out=None, c=None, alpha=1.0, beta=0.0, out_dtype=torch.float16):
-        n = b.shape[1]
-        if out is None:
-            out = torch.empty((self.m, n), dtype=out_dtype, device=b.device)
-        return _native.matmul_prepared(self.buffer, b, out, self.m, n, self.k, c=c, alpha=alpha, beta=beta)
+        return _binding().matmul_prepared(self.buffer, b, c, out, self.m, self.k, alpha, beta, out_dtype)
 
     def linear(self, x, bias=None, out=None, out_dtype=torch.float16):
         """y (tokens, m) = x (tokens, k) @ W.T (+ bias): the layer's form, x and y token-major, no transposes."""
@@ -129,9 +121,6 @@ class PreparedWeight:
         if out is None:
             out = torch.empty((x.shape[0], self.m), dtype=out_dtype, device=x.device)
         return _native.linear_prepared(self.buffer, x, out, self.m, self.k, bias=bias)
-
-
-_BIAS_TYPES = (torch.float16, torch.bfloat16, torch.float32)  # the kernels read a bias of any of them
 
 
 class BinaryLinear_2_4(nn.Module):
@@ -169,7 +158,7 @@ class BinaryLinear_2_4(nn.Module):
             weight = weight.contiguous()
             if weight.data_ptr() % 16:
                 weight = weight.clone()  # a view that starts inside a 16-byte unit
-            self.packed_binary_sparse, self.meta = _native.pack_weight(weight, prune=True)
+            self.packed_binary_sparse, self.meta = _binding().pack_weight(weight, True, _native.META_REFERENCE)
             self.vaild = True
             self._prepared = None
             return
@@ -192,73 +181,33 @@ class BinaryLinear_2_4(nn.Module):
             self.vaild = True
         self._prepared = None
 
-    def _kernel_types(self, x_dtype):
-        """(type the kernel reads, type it writes) for activations of x_dtype: bf16 as it is, everything else as fp16."""
-        if x_dtype == torch.bfloat16 and self.out_dtype != torch.float16:
-            return torch.bfloat16, self.out_dtype or torch.bfloat16
-        return torch.float16, self.out_dtype or (torch.float16 if x_dtype == torch.float16 else torch.float32)
-
-    def forward(self, x):
+    def _prepared_on(self, device):
         if not self.vaild:
             raise NotImplementedError("the BinaryLinear_2_4 layer holds no packed weight: call pack() first")
-        if self._prepared is None or self._prepared.buffer.device != x.device:
-            self._prepared = PreparedWeight(self.packed_binary_sparse.to(x.device), self.meta.to(x.device))
-        lead = x.shape[:-1]
-        if x.numel() == 0:  # an empty batch: nothing to launch
-            return x.new_zeros(*lead, self.outfeatures)
-        bias = self.bias
-        if bias is not None and (bias.dtype not in _BIAS_TYPES or bias.device != x.device):
-            bias = bias.to(device=x.device, dtype=torch.float32)
-        if x.dtype is torch.float16:
-            in_dtype, out_dtype = torch.float16, self.out_dtype or torch.float16
-        else:
-            in_dtype, out_dtype = self._kernel_types(x.dtype)
-        tokens = x.reshape(-1, self.infeatures).to(in_dtype).contiguous()
+        prepared = self._prepared
+        if prepared is None or prepared.buffer.device != device:
+            prepared = self._prepared = PreparedWeight(self.packed_binary_sparse.to(device), self.meta.to(device))
+        return prepared.buffer
+
+    def forward(self, x):
         # one kernel: reads the tokens where they lie, adds the bias, writes (tokens, outfeatures)
-        y = self._prepared.linear(tokens, bias=bias.contiguous() if bias is not None else None, out_dtype=out_dtype)
-        y = y.reshape(*lead, self.outfeatures)
-        return y if self.out_dtype is not None else y.to(x.dtype)
+        return _binding().layer_forward(self._prepared_on(x.device), x, self.bias, self.outfeatures, self.infeatures,
+                                        self.out_dtype)
 
 
 def forward_grouped(layers, xs):
     """The forward passes of several BinaryLinear_2_4 layers on inputs with the same number of tokens, in one library
     call (one kernel launch per 16 layers for up to 64 tokens): the q / k / v or gate / up projections of a decoder
     layer. xs: one tensor for all layers, or one per layer. Returns the list of outputs, each what layer(x) returns."""
-    if isinstance(xs, torch.Tensor):
-        xs = [xs] * len(layers)
-    if len(xs) != len(layers):
+    layers = list(layers)
+    shared = isinstance(xs, torch.Tensor)
+    xs = [xs] if shared else list(xs)
+    if not shared and len(xs) != len(layers):
         raise ValueError("one input per layer (or one for all)")
     if not layers:
         return []
-    flat, prepared = {}, []
-    for layer, x in zip(layers, xs):
-        if not layer.vaild:
-            raise NotImplementedError("a BinaryLinear_2_4 layer holds no packed weight: call pack() first")
-        if layer._prepared is None or layer._prepared.buffer.device != x.device:
-            layer._prepared = PreparedWeight(layer.packed_binary_sparse.to(x.device), layer.meta.to(x.device))
-        in_dtype = layer._kernel_types(x.dtype)[0]
-        if (id(x), in_dtype) not in flat:  # inputs shared by several layers are made contiguous and 16-bit once
-            t = x.reshape(-1, layer.infeatures).to(in_dtype).contiguous()
-            flat[id(x), in_dtype] = t.clone() if t.data_ptr() % 16 else t
-        prepared.append(flat[id(x), in_dtype])
-    tokens = prepared[0].shape[0]
-    types = {layer._kernel_types(x.dtype) for layer, x in zip(layers, xs)}
-    bias_dtypes = {layer.bias.dtype if layer.bias.dtype in _BIAS_TYPES else torch.float32
-                   for layer in layers if layer.bias is not None}
-    if tokens == 0 or len(types) > 1 or len(bias_dtypes) > 1 or any(t.shape[0] != tokens for t in prepared):
-        return [layer(x) for layer, x in zip(layers, xs)]  # nothing to share: the layers one by one
-    out_dtype = types.pop()[1]
-    problems, ys = [], []
-    for layer, x, t in zip(layers, xs, prepared):
-        bias = layer.bias
-        if bias is not None:
-            bias = bias.to(device=x.device, dtype=bias_dtypes and next(iter(bias_dtypes))).contiguous()
-        y = torch.empty((tokens, layer.outfeatures), dtype=out_dtype, device=x.device)
-        problems.append((layer._prepared.buffer, t, y, layer.outfeatures, layer.infeatures, bias))
-        ys.append(y)
-    _native.linear_prepared_grouped(problems)
-    outs = []
-    for layer, x, y in zip(layers, xs, ys):
-        y = y.reshape(*x.shape[:-1], layer.outfeatures)
-        outs.append(y if layer.out_dtype is not None else y.to(x.dtype))
-    return outs
+    prepared = [layer._prepared_on(xs[0 if shared else i].device) for i, layer in enumerate(layers)]
+    ys = _binding().grouped_forward(prepared, xs, [layer.bias for layer in layers], [layer.outfeatures for layer in layers],
+                                    [layer.infeatures for layer in layers], [layer.out_dtype for layer in layers])
+    # nothing to share (token counts or types differ): the layers one by one
+    return ys or [layer(xs[0 if shared else i]) for i, layer in enumerate(layers)]
