@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -298,6 +299,51 @@ SkinnyPlan plan_skinny(int m, int n, int k, int compute_units) {
   return SkinnyPlan{rows, 1};
 }
 
+// Row group and K splits over workgroups of wide_tokens_kernel (17 to 64 tokens): the plan with the least modelled time.
+// A workgroup's wavefronts each multiply one K chunk per round; a round's time depends on the row group and the number of
+// sixteen-token column tiles and grows with the share of compute units that load at the same time. One workgroup per
+// compute unit; a split pays a second launch and the partial sums. Fitted to m = 1024 ... 28672, k = 1024 ... 16384, n = 20
+// ... 64 inside HIP graphs (us, best plan | 32-row groups unsplit): 28672 x 8192 x 48 21.0 (128 rows) | 36.0; 11008 x 4096 x
+// 48 8.3 (64 rows) | 12.0; 4096 x 11008 x 48 11.6 (64 rows, four splits) | 15.2; 1024 x 16384 x 48 9.3 (four splits) | 15.9.
+// total_groups: workgroups per row-group size of all products of the launch, in the order of kWideRows.
+const int kWideRows[3] = {32, 64, 128};
+SkinnyPlan plan_wide(const long (&total_groups)[3], double results, int n, int k, bool may_split, int compute_units) {
+  static const double kBase[3][3] = {{2.9, 2.9, 3.0}, {3.3, 3.4, 3.6}, {4.3, 5.8, 6.4}};      // [row group][column tiles]
+  static const double kRound[3][3] = {{0.93, 1.48, 1.89}, {1.26, 1.74, 2.24}, {2.4, 2.75, 3.25}};
+  static const double kLoad[3] = {0.55, 0.55, 0.4};
+  static const double kSplitLines[3] = {1.17, 1.17, 1.05};  // k % 64 != 0: every second token's pieces straddle two lines
+  const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
+  const int tiles = n <= 32 ? 0 : n <= 48 ? 1 : 2;
+  SkinnyPlan best{32, 1};
+  double best_us = 1e30;
+  for (int r = 0; r < 3; ++r) {
+    if (g_skinny_rows > 0 && g_skinny_rows != kWideRows[r]) continue;
+    for (int s : {1, 2, 3, 4, 6, 8}) {
+      if (g_split_k >= 1 && may_split) s = std::min(g_split_k, chunks);
+      if (s > 1 && (!may_split || s > chunks)) break;
+      const int per_split = (chunks + s - 1) / s, rounds = (per_split + 7) / 8;
+      const double load = (double)total_groups[r] * s / compute_units;
+      const double batches = std::ceil(std::max(1.0, load));
+      const double round_us = kRound[r][tiles] * (1.0 + kLoad[r] * std::min(1.0, load)) * (k % 64 ? kSplitLines[r] : 1.0);
+      double us = 1.5 + batches * (kBase[r][tiles] - 1.5 + rounds * round_us);
+      if (s > 1) us += 2.6 + 0.15 * s + (s + 1) * 4.0 * results / 5.0e6;
+      if (us < best_us) {
+        best_us = us;
+        best = SkinnyPlan{kWideRows[r], s};
+      }
+      if (g_split_k >= 1) break;
+    }
+  }
+  if (best_us == 1e30) best.rows = g_skinny_rows;  // a forced row group that does not exist: the launch refuses it
+  return best;
+}
+SkinnyPlan plan_wide(int m, int n, int k, int compute_units) {
+  // split only where the split-K kernel would be: a call that needs no buffer can be captured without a warm-up
+  const bool may_split = plan_skinny(m, n, k, compute_units).splits > 1;
+  const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
+  return plan_wide(groups, (double)m * n, n, k, may_split, compute_units);
+}
+
 LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int compute_units = 256) {
   LaunchPlan plan{};
   // 32 < n <= 64: every 64-row workgroup of the split-K kernel stages all of B, which the main kernel's tiles overtake
@@ -556,7 +602,17 @@ int onebit_sparse_linear_prepared_typed(const void* prepared, const void* x, con
   if (!prepared || !x || !y) return fail(ONEBIT_ERR_ARGUMENT, "null operand pointer");
   if ((reinterpret_cast<uintptr_t>(x) & 15) != 0) return fail(ONEBIT_ERR_ARGUMENT, "x must be 16-byte aligned");
   const int kc_total = (k + onebit::kChunkK - 1) / onebit::kChunkK;
-  LaunchPlan plan = choose_launch(m, tokens, k, true, current_compute_units());
+  const int compute_units = current_compute_units();
+  const bool wide = tokens > onebit::kSkinnyTokens && tokens <= onebit::kSkinnyMaxN && g_skinny_enabled;
+  LaunchPlan plan{};
+  if (wide) {
+    const SkinnyPlan w = plan_wide(m, tokens, k, compute_units);
+    plan.split_k_kernel = 1;
+    plan.rows_or_tile = w.rows;
+    plan.splits = w.splits;
+  } else {
+    plan = choose_launch(m, tokens, k, true, compute_units);
+  }
   if ((size_t)k * 256 * 2 >= (size_t(1) << 32))
     return fail(ONEBIT_ERR_ARGUMENT, "the token-major form addresses x with 32-bit offsets inside a tile of 256 tokens: "
                                      "k = %d is beyond its limit of 8388607", k);
@@ -573,7 +629,8 @@ int onebit_sparse_linear_prepared_typed(const void* prepared, const void* x, con
     args.bias_type = bias_dtype;
     args.bf16 = x_dtype == ONEBIT_DTYPE_BF16;
     if (int rc = setup_skinny_split(args, plan.splits, static_cast<hipStream_t>(stream), nullptr); rc != ONEBIT_OK) return rc;
-    ONEBIT_HIP(onebit::launch_skinny_tokens(args, plan.rows_or_tile, static_cast<hipStream_t>(stream)));
+    ONEBIT_HIP(wide ? onebit::launch_wide_tokens(args, plan.rows_or_tile, static_cast<hipStream_t>(stream))
+                    : onebit::launch_skinny_tokens(args, plan.rows_or_tile, static_cast<hipStream_t>(stream)));
     return ONEBIT_OK;
   }
   switch (plan.rows_or_tile) {
@@ -649,16 +706,24 @@ int onebit_sparse_linear_prepared_grouped_typed(const onebit_linear_problem* pro
     }
     return ONEBIT_OK;
   }
-  // Row group of the launch: as for one product with all the weight rows, the largest that still gives about two
-  // workgroups per three compute units.
+  // Row group of the launch: as for one product with all the weight rows; up to sixteen tokens the largest that still gives
+  // about two workgroups per three compute units.
   const int compute_units = current_compute_units();
   for (int first = 0; first < count; first += onebit::kSkinnyMaxGroup) {
     const int in_launch = std::min(count - first, onebit::kSkinnyMaxGroup);
-    long rows_total = 0;
-    for (int i = 0; i < in_launch; ++i) rows_total += problems[first + i].m;
+    const bool wide = tokens > onebit::kSkinnyTokens;
+    long rows_total = 0, groups[3] = {0, 0, 0};
+    int longest_k = 0;
+    for (int i = 0; i < in_launch; ++i) {
+      const onebit_linear_problem& q = problems[first + i];
+      rows_total += q.m;
+      for (int r = 0; r < 3; ++r) groups[r] += (q.m + kWideRows[r] - 1) / kWideRows[r];
+      longest_k = std::max(longest_k, q.k);
+    }
     const int enough = std::max(1, 160 * compute_units / 256);
-    const int rows = g_skinny_rows > 0 ? g_skinny_rows
-                     : (rows_total / 128 >= enough && tokens <= 32) ? 128 : (rows_total / 64 >= enough) ? 64 : 32;
+    const int rows = wide ? plan_wide(groups, 0.0, tokens, longest_k, false, compute_units).rows
+                     : g_skinny_rows > 0 ? g_skinny_rows
+                     : (rows_total / 128 >= enough) ? 128 : (rows_total / 64 >= enough) ? 64 : 32;
     if (rows != 32 && rows != 64 && rows != 128) return fail(ONEBIT_ERR_ARGUMENT, "row group %d: must be 32, 64 or 128", rows);
     onebit::SkinnyGroupArgs group{};
     group.count = in_launch;
@@ -676,7 +741,8 @@ int onebit_sparse_linear_prepared_grouped_typed(const onebit_linear_problem* pro
       args.bias_type = bias_dtype;
       args.bf16 = x_dtype == ONEBIT_DTYPE_BF16;
     }
-    ONEBIT_HIP(onebit::launch_skinny_group(group, rows, static_cast<hipStream_t>(stream)));
+    ONEBIT_HIP(wide ? onebit::launch_wide_tokens_group(group, rows, static_cast<hipStream_t>(stream))
+                    : onebit::launch_skinny_group(group, rows, static_cast<hipStream_t>(stream)));
   }
   return ONEBIT_OK;
 }

@@ -90,10 +90,16 @@ hipError_t launch_split_reduce(const float* ws, int splits, size_t total, const 
 // Split-K kernel for n <= 64; rows_per_group (32, 64 or 128) = weight rows one workgroup covers (n > 32: at most 64).
 constexpr int kSkinnyMaxN = 64;
 hipError_t launch_skinny(SkinnyArgs args, int rows_per_group, hipStream_t stream);
-// The linear layer's form of the same kernel: y[t][r] = sum_k W[r][k] x[t][k] + bias[r] for n <= 64 tokens, x and y
+// The linear layer's form of the same kernel: y[t][r] = sum_k W[r][k] x[t][k] + bias[r] for n <= kSkinnyTokens tokens, x and y
 // token-major (x 16-byte aligned).
+constexpr int kSkinnyTokens = 16;
 hipError_t launch_skinny_tokens(SkinnyArgs args, int rows_per_group, hipStream_t stream);
 // count <= kSkinnyMaxGroup problems of the same form, each with its own weight, x, bias, y, m and k, in one launch.
 hipError_t launch_skinny_group(SkinnyGroupArgs group, int rows_per_group, hipStream_t stream);
+
+// The linear layer's form for n <= 64 tokens whose images asynchronous copies bring to LDS (wide_tokens_kernel); row groups of
+// 32, 64 or 128.
+hipError_t launch_wide_tokens(SkinnyArgs args, int rows_per_group, hipStream_t stream);
+hipError_t launch_wide_tokens_group(SkinnyGroupArgs group, int rows_per_group, hipStream_t stream);
 
 }  // namespace onebit

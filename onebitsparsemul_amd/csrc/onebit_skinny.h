@@ -32,7 +32,7 @@ constexpr int kSkinnyRegion = 8192;  // bytes of one B image
 // the result is written as y[token][weight row] (+ bias[weight row]). The image is then token-major too: row t holds
 // the image's K range of token t in 16-byte pieces, piece p stored at position p ^ token_swizzle(t) so that lanes
 // which read the same piece of consecutive tokens fall into different banks; a lane's SMFMAC operand is two plain
-// 16-byte reads (K consecutive inside a piece), no transpose.
+// 16-byte reads (K consecutive inside a piece), no transpose. Up to sixteen tokens; more go to wide_tokens_kernel.
 // kSkinnyBRun: n = 2 or 4 with B 16-byte aligned. The 256 rows of a chunk are one run of 512 n consecutive bytes,
 // loaded in 16-byte pieces (32 n of them: at most two load instructions per wavefront and chunk, where the row-wise
 // modes issue eight; the split-K kernel's time is set by the number of load instructions it issues) and spread over the image rows
@@ -50,7 +50,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   constexpr int NF = NC <= 32 ? 1 : NC / 32;           // 32-column fragments per image row
   constexpr int TILE_BYTES = kRowBlock * NC * 4;       // one fp32 partial tile
   static_assert(NC == 16 || NC == 32 || NC == 64, "image width");
-  static_assert(MODE != kSkinnyBRun || NC == 16, "the run mode is for 16 columns");
+  static_assert((MODE != kSkinnyBRun && MODE != kSkinnyBTokens) || NC == 16, "the run and token modes are for 16 columns");
   // the partial tiles reuse the wavefront's image memory, RT row blocks per round of the final reduction
   constexpr int RT = R * TILE_BYTES <= kSkinnyRegion ? R : kSkinnyRegion / TILE_BYTES;
   static_assert(RT >= 1 && R % RT == 0, "the row blocks must divide into whole reduction rounds");
@@ -276,9 +276,6 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   const int chunk8 = (NC >= 32 ? ((lane & 31) >> 4) * 4 : 0) + (i16 & 3);  // 8-byte piece of the 32-column fragment
   const char* lane_ptr = region + (8 * gb + (i16 >> 2)) * ROW_BYTES + chunk8 * 8;
 
-  // token-major image: this lane's token row and swizzle; K step s of the image needs pieces 4 s + gb and 4 s + 2 + gb
-  const int token_col = NC >= 32 ? (lane & 31) : i16;
-  const uint32_t token_read_base = (uint32_t)token_col * TOKEN_ROW_BYTES + (uint32_t)((gb ^ token_swizzle<TOKEN_ROW_BYTES>(token_col)) << 4);
   // ---- 16x16x64 form (M16). The instruction's A lane (row l % 16, group g = l / 16) holds eight kept values and their
   // 16 index bits for 16 consecutive K positions, as a lane of the prepared block does for one K step: lane
   // (row, half ga) of the block, step s. Which K positions group g stands for is free as long as B agrees, so the
@@ -359,15 +356,6 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
 
   auto frag = [&](int image_step, int f) __attribute__((always_inline)) {
     u32x8_t raw;
-    if (TOKENS) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const u32x4_t t = *reinterpret_cast<const u32x4_t*>(
-            region + (token_read_base ^ (uint32_t)((4 * image_step + 2 * h) << 4)) + f * 32 * TOKEN_ROW_BYTES);
-        raw[4 * h] = t.x; raw[4 * h + 1] = t.y; raw[4 * h + 2] = t.z; raw[4 * h + 3] = t.w;
-      }
-      return __builtin_bit_cast(half16_t, raw);
-    }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int row_const = image_step * 32 + 4 * (q & 1) + 16 * (q >> 1);
@@ -508,6 +496,8 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
             for (int v = 0; v < 4; ++v) {
               const int row = 16 * h + 4 * g16 + v;
               const float value = acc16[round * RT + rr][h][v];
+              // token-major: [token][weight row of the round], the row index XOR-swizzled by the token so that neither
+              // these stores (16 tokens, one row) nor the reads below (one token, consecutive rows) collide in a bank
               if (TOKENS) tile[i16 * ROUND_ROWS + ((rr * 32 + row) ^ i16)] = value;
               else tile[(rr * 32 + row) * NC + i16] = value;
             }
@@ -520,10 +510,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
             for (int v = 0; v < 16; ++v) {
               const int row = 8 * (v / 4) + 4 * (lane >> 5) + (v % 4);
               const float value = acc[round * RT + rr][f][v];
-              // token-major: [token][weight row of the round], the row index XOR-swizzled by the token so that neither
-              // these stores (32 tokens, one row) nor the reads below (one token, consecutive rows) collide in a bank
-              if (TOKENS) tile[(f * 32 + col) * ROUND_ROWS + ((rr * 32 + row) ^ col)] = value;
-              else tile[(rr * 32 + row) * NC + f * 32 + col] = value;
+              tile[(rr * 32 + row) * NC + f * 32 + col] = value;
             }
       }
     }

@@ -1,12 +1,10 @@
-// Token-major form of the split-K kernel (the linear layer), one product or several per launch.
+// Token-major form of the split-K kernel (the linear layer, up to sixteen tokens), one product or several per launch.
 #include "onebit_skinny.h"
 
 namespace onebit {
 
 template <int NW, int R, bool BF16>
 static hipError_t launch_skinny_tokens_type(const SkinnyArgs& args, hipStream_t stream) {
-  if (args.n > 32) return launch_skinny_mode<NW, (R > 2 ? 2 : R), kSkinnyBTokens, 64, BF16>(args, stream);
-  if (args.n > 16) return launch_skinny_mode<NW, R, kSkinnyBTokens, 32, BF16>(args, stream);
   return launch_skinny_mode<NW, R, kSkinnyBTokens, 16, BF16>(args, stream);
 }
 
@@ -16,7 +14,7 @@ static hipError_t launch_skinny_tokens_cfg(const SkinnyArgs& args, hipStream_t s
 }
 
 hipError_t launch_skinny_tokens(SkinnyArgs args, int rows_per_group, hipStream_t stream) {
-  if (args.n < 1 || args.n > kSkinnyMaxN) return hipErrorInvalidValue;
+  if (args.n < 1 || args.n > kSkinnyTokens) return hipErrorInvalidValue;
   // 16-byte loads of x; lane offsets of up to 64 token rows must stay below the "outside" offset of the kernel
   if ((reinterpret_cast<uintptr_t>(args.b) & 15) != 0 || (size_t)args.k * 64 * 2 >= 0xFFFFFF00u) return hipErrorInvalidValue;
   SkinnyArgs pass;
@@ -34,26 +32,23 @@ hipError_t launch_skinny_tokens(SkinnyArgs args, int rows_per_group, hipStream_t
 }
 
 template <int NW, int R, bool BF16>
-static hipError_t launch_skinny_group_type(const SkinnyGroupArgs& g, int blocks, int tokens, hipStream_t stream) {
+static hipError_t launch_skinny_group_type(const SkinnyGroupArgs& g, int blocks, hipStream_t stream) {
   const dim3 grid(blocks), threads(64 * NW);
-  if (tokens > 32) hipLaunchKernelGGL((skinny_group_kernel<NW, (R > 2 ? 2 : R), 64, BF16>), grid, threads, 0, stream, g);
-  else if (tokens > 16) hipLaunchKernelGGL((skinny_group_kernel<NW, R, 32, BF16>), grid, threads, 0, stream, g);
-  else hipLaunchKernelGGL((skinny_group_kernel<NW, R, 16, BF16>), grid, threads, 0, stream, g);
+  hipLaunchKernelGGL((skinny_group_kernel<NW, R, 16, BF16>), grid, threads, 0, stream, g);
   return hipGetLastError();
 }
 
 template <int NW, int R>
-static hipError_t launch_skinny_group_cfg(const SkinnyGroupArgs& g, int blocks, int tokens, hipStream_t stream) {
-  return g.problem[0].bf16 ? launch_skinny_group_type<NW, R, true>(g, blocks, tokens, stream)
-                           : launch_skinny_group_type<NW, R, false>(g, blocks, tokens, stream);
+static hipError_t launch_skinny_group_cfg(const SkinnyGroupArgs& g, int blocks, hipStream_t stream) {
+  return g.problem[0].bf16 ? launch_skinny_group_type<NW, R, true>(g, blocks, stream)
+                           : launch_skinny_group_type<NW, R, false>(g, blocks, stream);
 }
 
 hipError_t launch_skinny_group(SkinnyGroupArgs g, int rows_per_group, hipStream_t stream) {
   if (g.count < 1 || g.count > kSkinnyMaxGroup) return hipErrorInvalidValue;
   const int tokens = g.problem[0].n;
-  if (tokens < 1 || tokens > kSkinnyMaxN) return hipErrorInvalidValue;
+  if (tokens < 1 || tokens > kSkinnyTokens) return hipErrorInvalidValue;
   if (rows_per_group != 32 && rows_per_group != 64 && rows_per_group != 128) return hipErrorInvalidValue;
-  const int rows = (rows_per_group == 128 && tokens > 32) ? 64 : rows_per_group;  // as launch_skinny_tokens_cfg does
   int blocks = 0;
   for (int i = 0; i < g.count; ++i) {
     SkinnyArgs& p = g.problem[i];
@@ -64,13 +59,13 @@ hipError_t launch_skinny_group(SkinnyGroupArgs g, int rows_per_group, hipStream_
     p.chunks_per_split = p.kc_total;
     p.split_ws = nullptr;
     g.first_block[i] = blocks;
-    blocks += (p.m + rows - 1) / rows;
+    blocks += (p.m + rows_per_group - 1) / rows_per_group;
   }
   g.first_block[g.count] = blocks;
   switch (rows_per_group) {
-    case 32: return launch_skinny_group_cfg<16, 1>(g, blocks, tokens, stream);
-    case 64: return launch_skinny_group_cfg<8, 2>(g, blocks, tokens, stream);
-    default: return launch_skinny_group_cfg<8, 4>(g, blocks, tokens, stream);
+    case 32: return launch_skinny_group_cfg<16, 1>(g, blocks, stream);
+    case 64: return launch_skinny_group_cfg<8, 2>(g, blocks, stream);
+    default: return launch_skinny_group_cfg<8, 4>(g, blocks, stream);
   }
 }
 
