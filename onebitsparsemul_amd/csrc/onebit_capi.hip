@@ -170,6 +170,7 @@ int check_linear_dtypes(int x_dtype, int bias_dtype, int y_dtype) {
 struct GemmPlan {
   int tile;
   int splits;
+  double us;  // modelled; 0 for a forced tile
 };
 
 struct TileCost {
@@ -219,16 +220,16 @@ GemmPlan plan_gemm(int m, int n, int k, int compute_units) {
           }
         }
     if (splits > chunks) splits = chunks;
-    return GemmPlan{forced_tile, splits};
+    return GemmPlan{forced_tile, splits, 0.0};
   }
   const int fixed_splits = forced_splits >= 1 ? (forced_splits > chunks ? chunks : forced_splits) : 0;
-  GemmPlan best{onebit::kTile128x128s, fixed_splits ? fixed_splits : 1};
+  GemmPlan best{onebit::kTile128x128s, fixed_splits ? fixed_splits : 1, 0.0};
   double best_us = 1e30;
   auto consider = [&](const TileCost& t, int s) {
     const double us = model_us(t, m, n, chunks, s, compute_units);
     if (us < best_us) {
       best_us = us;
-      best = GemmPlan{t.tile, s};
+      best = GemmPlan{t.tile, s, us};
     }
   };
   for (const TileCost& t : kTileCosts) {
@@ -258,6 +259,7 @@ struct LaunchPlan {
   int rows_or_tile;    // skinny_kernel: weight rows per workgroup; gemm_kernel: TileConfig
   int splits;          // gemm_kernel: K splits over workgroups (1 = none)
   int pad_b;           // gemm_kernel: B is read through a padded copy
+  double model_us;     // gemm_kernel: what the plan is modelled to take
 };
 
 // Row group and K splits over workgroups of the split-K kernel. Every workgroup of that kernel reads all of B's rows
@@ -299,49 +301,52 @@ SkinnyPlan plan_skinny(int m, int n, int k, int compute_units) {
   return SkinnyPlan{rows, 1};
 }
 
-// Row group and K splits over workgroups of wide_tokens_kernel (17 to 64 tokens): the plan with the least modelled time.
+// Row group, tokens per workgroup and K splits over workgroups of wide_tokens_kernel: the plan with the least modelled time.
 // A workgroup's wavefronts each multiply one K chunk per round; a round's time depends on the row group and the number of
-// sixteen-token column tiles and grows with the share of compute units that load at the same time. One workgroup per
-// compute unit; a split pays a second launch and the partial sums. Fitted to m = 1024 ... 28672, k = 1024 ... 16384, n = 20
-// ... 64 inside HIP graphs (us, best plan | 32-row groups unsplit): 28672 x 8192 x 48 21.0 (128 rows) | 36.0; 11008 x 4096 x
-// 48 8.3 (64 rows) | 12.0; 4096 x 11008 x 48 11.6 (64 rows, four splits) | 15.2; 1024 x 16384 x 48 9.3 (four splits) | 15.9.
-// total_groups: workgroups per row-group size of all products of the launch, in the order of kWideRows.
+// sixteen-token column tiles and grows with the share of compute units that load at the same time. Workgroups beyond one per
+// compute unit pay the rounds again, less where two fit a compute unit (up to two column tiles on up to 64 rows). A split
+// pays a second launch and the partial sums.
+// Fitted to m = 1024 ... 28672, k = 1024 ... 22176, 17 ... 1024 tokens inside HIP graphs. us of the chosen plan | of 64-token
+// workgroups on 32 rows, unsplit: 28672 x 8192 x 48 21.0 (128 rows) | 36.0; 4096 x 11008 x 32 9.0 (32 rows, 16 tokens) | 12.2;
+// 1024 x 4096 x 256 5.3 (32 rows, 32 tokens) | 7.1; 4096 x 4096 x 128 6.3 (64 rows, 32 tokens) | 7.8.
+// total_groups: row groups of all products of the launch, for each of kWideRows.
 const int kWideRows[3] = {32, 64, 128};
-SkinnyPlan plan_wide(const long (&total_groups)[3], double results, int n, int k, bool may_split, int compute_units) {
-  static const double kBase[3][3] = {{2.9, 2.9, 3.0}, {3.3, 3.4, 3.6}, {4.3, 5.8, 6.4}};      // [row group][column tiles]
-  static const double kRound[3][3] = {{0.93, 1.48, 1.89}, {1.26, 1.74, 2.24}, {2.4, 2.75, 3.25}};
-  static const double kLoad[3] = {0.55, 0.55, 0.4};
+struct WidePlan {
+  int rows, splits, tokens;
+  double us;
+};
+WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, bool may_split, int compute_units) {
+  // [row group][column tiles - 1]
+  static const double kBase[3][4] = {{2.75, 2.9, 2.9, 3.0}, {3.1, 3.3, 3.4, 3.6}, {3.7, 4.3, 5.8, 6.4}};
+  static const double kRound[3][4] = {{0.74, 0.93, 1.48, 1.89}, {1.01, 1.26, 1.74, 2.24}, {1.88, 2.4, 2.75, 3.25}};
+  static const double kLoad[3][4] = {{0.55, 0.55, 0.55, 0.55}, {0.23, 0.44, 0.5, 0.5}, {0.14, 0.24, 0.4, 0.4}};
+  static const double kAgain[3][4] = {{0.57, 1.1, 1.0, 1.0}, {0.73, 0.9, 1.0, 1.0}, {1.0, 1.0, 1.0, 1.0}};
   static const double kSplitLines[3] = {1.17, 1.17, 1.05};  // k % 64 != 0: every second token's pieces straddle two lines
   const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
-  const int tiles = n <= 32 ? 0 : n <= 48 ? 1 : 2;
-  SkinnyPlan best{32, 1};
-  double best_us = 1e30;
-  for (int r = 0; r < 3; ++r) {
-    if (g_skinny_rows > 0 && g_skinny_rows != kWideRows[r]) continue;
-    for (int s : {1, 2, 3, 4, 6, 8}) {
-      if (g_split_k >= 1 && may_split) s = std::min(g_split_k, chunks);
-      if (s > 1 && (!may_split || s > chunks)) break;
-      const int per_split = (chunks + s - 1) / s, rounds = (per_split + 7) / 8;
-      const double load = (double)total_groups[r] * s / compute_units;
-      const double batches = std::ceil(std::max(1.0, load));
-      const double round_us = kRound[r][tiles] * (1.0 + kLoad[r] * std::min(1.0, load)) * (k % 64 ? kSplitLines[r] : 1.0);
-      double us = 1.5 + batches * (kBase[r][tiles] - 1.5 + rounds * round_us);
-      if (s > 1) us += 2.6 + 0.15 * s + (s + 1) * 4.0 * results / 5.0e6;
-      if (us < best_us) {
-        best_us = us;
-        best = SkinnyPlan{kWideRows[r], s};
+  WidePlan best{g_skinny_rows > 0 ? g_skinny_rows : 32, 1, std::min(n, onebit::kSkinnyMaxN), 1e30};
+  for (int width = 1; width <= 4; ++width) {
+    const int groups = (n + 16 * width - 1) / (16 * width);
+    const int tokens = ((n + groups - 1) / groups + 7) / 8 * 8, tiles = (tokens + 15) / 16;
+    if (tiles != width) continue;  // the same groups as with narrower ones
+    for (int r = 0; r < 3; ++r) {
+      if (g_skinny_rows > 0 && g_skinny_rows != kWideRows[r]) continue;
+      for (int s : {1, 2, 3, 4, 6, 8}) {
+        if (g_split_k >= 1 && may_split) s = std::min(g_split_k, chunks);
+        if (s > 1 && (!may_split || s > chunks)) break;
+        const int rounds = ((chunks + s - 1) / s + 7) / 8;
+        const double load = (double)total_groups[r] * groups * s / compute_units;
+        const double work = rounds * kRound[r][tiles - 1] * (1.0 + kLoad[r][tiles - 1] * std::min(1.0, load)) *
+                            (k % 64 ? kSplitLines[r] : 1.0);
+        double us = kBase[r][tiles - 1] + work;
+        if (load > 1.0)
+          us += (std::ceil(load) - 1.0) * (work * kAgain[r][tiles - 1] + (kBase[r][tiles - 1] - 1.5) * (r < 2 ? 0.4 : 1.0));
+        if (s > 1) us += 2.6 + 0.15 * s + (s + 1) * 4.0 * results / 5.0e6;
+        if (us < best.us) best = WidePlan{kWideRows[r], s, tokens, us};
+        if (g_split_k >= 1) break;
       }
-      if (g_split_k >= 1) break;
     }
   }
-  if (best_us == 1e30) best.rows = g_skinny_rows;  // a forced row group that does not exist: the launch refuses it
   return best;
-}
-SkinnyPlan plan_wide(int m, int n, int k, int compute_units) {
-  // split only where the split-K kernel would be: a call that needs no buffer can be captured without a warm-up
-  const bool may_split = plan_skinny(m, n, k, compute_units).splits > 1;
-  const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
-  return plan_wide(groups, (double)m * n, n, k, may_split, compute_units);
 }
 
 LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int compute_units = 256) {
@@ -360,10 +365,32 @@ LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int comput
   const GemmPlan gemm = plan_gemm(m, n, k, compute_units);
   plan.rows_or_tile = gemm.tile;
   plan.splits = gemm.splits;
+  plan.model_us = gemm.us;
   // B rows that are not 16-byte aligned: pad a copy (one extra pass over B) unless the problem is too small for that
   // to pay against the element-copy variant of the kernel
   const bool b_in_place = n % 8 == 0 && b_16_byte_aligned;
   plan.pad_b = !b_in_place && (size_t)k * n >= 65536 && g_pad_b;
+  return plan;
+}
+
+// The linear layer's plan: wide = wide_tokens_kernel with `wide_plan`, else `launch` as for a product with an aligned B.
+// Up to sixteen tokens the split-K kernel; beyond 64 whichever of wide_tokens_kernel and the main kernel is modelled faster
+// (the main kernel's model is up to 12 % above its measured times where the two meet). A layer call may split K, i.e. needs
+// a buffer, only where the other kernel's plan would: what can be captured without a warm-up stays so.
+struct LinearPlan {
+  bool wide;
+  WidePlan wide_plan;
+  LaunchPlan launch;
+};
+LinearPlan plan_linear(int m, int tokens, int k, int compute_units) {
+  LinearPlan plan{};
+  plan.launch = choose_launch(m, tokens, k, true, compute_units);
+  if (tokens <= onebit::kSkinnyTokens || !g_skinny_enabled) return plan;
+  const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
+  const bool beyond = tokens > onebit::kSkinnyMaxN;
+  if (beyond && (g_tile_config >= 0 || groups[2] * ((tokens + 63) / 64) > 2L * compute_units)) return plan;
+  plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, plan.launch.splits > 1 || g_split_k >= 1, compute_units);
+  plan.wide = !beyond || plan.wide_plan.us < 0.88 * plan.launch.model_us;
   return plan;
 }
 
@@ -602,21 +629,12 @@ int onebit_sparse_linear_prepared_typed(const void* prepared, const void* x, con
   if (!prepared || !x || !y) return fail(ONEBIT_ERR_ARGUMENT, "null operand pointer");
   if ((reinterpret_cast<uintptr_t>(x) & 15) != 0) return fail(ONEBIT_ERR_ARGUMENT, "x must be 16-byte aligned");
   const int kc_total = (k + onebit::kChunkK - 1) / onebit::kChunkK;
-  const int compute_units = current_compute_units();
-  const bool wide = tokens > onebit::kSkinnyTokens && tokens <= onebit::kSkinnyMaxN && g_skinny_enabled;
-  LaunchPlan plan{};
-  if (wide) {
-    const SkinnyPlan w = plan_wide(m, tokens, k, compute_units);
-    plan.split_k_kernel = 1;
-    plan.rows_or_tile = w.rows;
-    plan.splits = w.splits;
-  } else {
-    plan = choose_launch(m, tokens, k, true, compute_units);
-  }
+  const LinearPlan linear = plan_linear(m, tokens, k, current_compute_units());
+  const LaunchPlan& plan = linear.launch;
   if ((size_t)k * 256 * 2 >= (size_t(1) << 32))
     return fail(ONEBIT_ERR_ARGUMENT, "the token-major form addresses x with 32-bit offsets inside a tile of 256 tokens: "
                                      "k = %d is beyond its limit of 8388607", k);
-  if (plan.split_k_kernel) {
+  if (linear.wide || plan.split_k_kernel) {
     onebit::SkinnyArgs args{};
     args.prep = static_cast<const uint8_t*>(prepared);
     args.b = static_cast<const _Float16*>(x);
@@ -628,9 +646,12 @@ int onebit_sparse_linear_prepared_typed(const void* prepared, const void* x, con
     args.bias = bias;
     args.bias_type = bias_dtype;
     args.bf16 = x_dtype == ONEBIT_DTYPE_BF16;
-    if (int rc = setup_skinny_split(args, plan.splits, static_cast<hipStream_t>(stream), nullptr); rc != ONEBIT_OK) return rc;
-    ONEBIT_HIP(wide ? onebit::launch_wide_tokens(args, plan.rows_or_tile, static_cast<hipStream_t>(stream))
-                    : onebit::launch_skinny_tokens(args, plan.rows_or_tile, static_cast<hipStream_t>(stream)));
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    if (int rc = setup_skinny_split(args, linear.wide ? linear.wide_plan.splits : plan.splits, s, nullptr); rc != ONEBIT_OK)
+      return rc;
+    args.tokens_per_group = linear.wide_plan.tokens;
+    ONEBIT_HIP(linear.wide ? onebit::launch_wide_tokens(args, linear.wide_plan.rows, s)
+                           : onebit::launch_skinny_tokens(args, plan.rows_or_tile, s));
     return ONEBIT_OK;
   }
   switch (plan.rows_or_tile) {
@@ -721,7 +742,9 @@ int onebit_sparse_linear_prepared_grouped_typed(const onebit_linear_problem* pro
       longest_k = std::max(longest_k, q.k);
     }
     const int enough = std::max(1, 160 * compute_units / 256);
-    const int rows = wide ? plan_wide(groups, 0.0, tokens, longest_k, false, compute_units).rows
+    WidePlan wide_plan{};
+    if (wide) wide_plan = plan_wide(groups, 0.0, tokens, longest_k, false, compute_units);
+    const int rows = wide ? wide_plan.rows
                      : g_skinny_rows > 0 ? g_skinny_rows
                      : (rows_total / 128 >= enough) ? 128 : (rows_total / 64 >= enough) ? 64 : 32;
     if (rows != 32 && rows != 64 && rows != 128) return fail(ONEBIT_ERR_ARGUMENT, "row group %d: must be 32, 64 or 128", rows);
@@ -740,6 +763,7 @@ int onebit_sparse_linear_prepared_grouped_typed(const onebit_linear_problem* pro
       args.bias = q.bias;
       args.bias_type = bias_dtype;
       args.bf16 = x_dtype == ONEBIT_DTYPE_BF16;
+      args.tokens_per_group = wide_plan.tokens;
     }
     ONEBIT_HIP(wide ? onebit::launch_wide_tokens_group(group, rows, static_cast<hipStream_t>(stream))
                     : onebit::launch_skinny_group(group, rows, static_cast<hipStream_t>(stream)));

@@ -57,6 +57,8 @@ struct SkinnyArgs {
   int splits;
   int chunks_per_split;
   float* split_ws;
+  // wide_tokens_kernel only: tokens a workgroup multiplies (at most 64), grid.z = ceil(n / tokens_per_group)
+  int tokens_per_group;
 };
 
 // Several token-major products with the same token count in one launch of the split-K kernel (no K split over
@@ -97,8 +99,8 @@ hipError_t launch_skinny_tokens(SkinnyArgs args, int rows_per_group, hipStream_t
 // count <= kSkinnyMaxGroup problems of the same form, each with its own weight, x, bias, y, m and k, in one launch.
 hipError_t launch_skinny_group(SkinnyGroupArgs group, int rows_per_group, hipStream_t stream);
 
-// The linear layer's form for n <= 64 tokens whose images asynchronous copies bring to LDS (wide_tokens_kernel); row groups of
-// 32, 64 or 128.
+// The linear layer's form whose images of x asynchronous copies bring to LDS (wide_tokens_kernel): any number of tokens, in
+// groups of at most 64 per workgroup; row groups of 32, 64 or 128.
 hipError_t launch_wide_tokens(SkinnyArgs args, int rows_per_group, hipStream_t stream);
 hipError_t launch_wide_tokens_group(SkinnyGroupArgs group, int rows_per_group, hipStream_t stream);
 

@@ -34,9 +34,10 @@ struct WideShape {
   static constexpr int LDS_BYTES = kWideWaves * REGION;
 };
 
-// COPIES: 1 KiB copies per image, one per eight tokens (n <= 8 COPIES)
+// COPIES: 1 KiB copies per image, one per eight tokens. A workgroup multiplies up to 8 COPIES tokens from first_token on.
 template <int R, int COPIES, bool BF16>
-__device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x, const int block_y, char* const smem) {
+__device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x, const int block_y, const int first_token,
+                                          char* const smem) {
   using Shape = WideShape<R, COPIES>;
   constexpr int NW = kWideWaves, CT = Shape::CT, RT = Shape::RT;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -45,6 +46,7 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
   char* const region = smem + wave * Shape::REGION;
   const uint32_t region_offset = lds_offset_of(smem) + wave * Shape::REGION;
   const int kc_total = p.kc_total, k_total = p.k;
+  const int tokens = p.n - first_token < 8 * COPIES ? p.n - first_token : 8 * COPIES;
   const int kc_begin = block_y * p.chunks_per_split;
   const int kc_end = kc_begin + p.chunks_per_split < kc_total ? kc_begin + p.chunks_per_split : kc_total;
   const int first = kc_begin + wave;
@@ -77,10 +79,10 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
 #pragma unroll
   for (int i = 0; i < COPIES; ++i) {
     int token = 8 * i + (lane >> 3);
-    if (token >= p.n) token = p.n - 1;
+    if (token >= tokens) token = tokens - 1;
     copy_off[i] = ((uint32_t)token * (uint32_t)k_total + 8u * (piece0 ^ (4 * (i & 1)))) * 2u;
   }
-  const char* const x_bytes = reinterpret_cast<const char*>(p.b);
+  const char* const x_bytes = reinterpret_cast<const char*>(p.b + (size_t)first_token * k_total);
   const char* const zeros = reinterpret_cast<const char*>(g_zero16_wide);
   auto copy_image = [&](int k0, int slot) __attribute__((always_inline)) {
     const uint32_t dst = region_offset + slot * Shape::IMAGE_BYTES;
@@ -246,11 +248,11 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
 #pragma unroll
       for (int w = 0; w < NW; ++w) sum += *reinterpret_cast<const float4v_t*>(smem + w * Shape::REGION + at);
       const int row = (rb_first + round * RT) * kRowBlock + 4 * slot;
-      if (token >= p.n || row >= p.m) continue;
+      if (token >= tokens || row >= p.m) continue;
       if (p.bias)
 #pragma unroll
         for (int e = 0; e < 4; ++e) sum[e] += load_element(p.bias, p.bias_type, row + e);
-      const size_t o = (size_t)token * p.m + row;
+      const size_t o = (size_t)(first_token + token) * p.m + row;
       if (p.d_f16)
         *reinterpret_cast<u32x2_any_t*>(y_out + o * 2) = u32x2_t{round_pair<BF16>(sum[0], sum[1]), round_pair<BF16>(sum[2], sum[3])};
       else
@@ -262,7 +264,7 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
 template <int R, int COPIES, bool BF16>
 __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_tokens_kernel(SkinnyArgs p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  wide_body<R, COPIES, BF16>(p, blockIdx.x, blockIdx.y, smem);
+  wide_body<R, COPIES, BF16>(p, blockIdx.x, blockIdx.y, blockIdx.z * p.tokens_per_group, smem);
 }
 
 // Several products that share the token count, workgroups numbered over their row groups as in skinny_group_kernel.
@@ -272,7 +274,8 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_tokens_group_kernel(S
   int which = 0;
   for (int i = 1; i < g.count; ++i)
     if ((int)blockIdx.x >= g.first_block[i]) which = i;
-  wide_body<R, COPIES, BF16>(g.problem[which], (int)blockIdx.x - g.first_block[which], 0, smem);
+  wide_body<R, COPIES, BF16>(g.problem[which], (int)blockIdx.x - g.first_block[which], 0,
+                             blockIdx.z * g.problem[which].tokens_per_group, smem);
 }
 
 template <int R, int COPIES, class Args>
@@ -336,11 +339,12 @@ static bool wide_operand_fits(const SkinnyArgs& p) {
 }
 
 hipError_t launch_wide_tokens(SkinnyArgs args, int rows_per_group, hipStream_t stream) {
-  if (args.n < 1 || args.n > kSkinnyMaxN || rows_per_group < 1 || !wide_operand_fits(args)) return hipErrorInvalidValue;
+  const int tokens = args.tokens_per_group;
+  if (args.n < 1 || tokens < 1 || tokens > kSkinnyMaxN || rows_per_group < 1 || !wide_operand_fits(args)) return hipErrorInvalidValue;
   SkinnyArgs pass;
   if (hipError_t st = skinny_split_setup(args, pass); st != hipSuccess) return st;
-  const dim3 grid((args.m + rows_per_group - 1) / rows_per_group, args.splits);
-  const hipError_t st = launch_wide_rows(pass, rows_per_group, args.n, args.bf16, grid, stream);
+  const dim3 grid((args.m + rows_per_group - 1) / rows_per_group, args.splits, (args.n + tokens - 1) / tokens);
+  const hipError_t st = launch_wide_rows(pass, rows_per_group, tokens, args.bf16, grid, stream);
   if (st != hipSuccess || args.splits <= 1) return st;
   return launch_split_reduce(args.split_ws, args.splits, (size_t)args.m * args.n, nullptr, args.d, 1.f, 0.f, 0,
                              args.d_f16 && args.bf16 ? kBF16 : args.d_f16, args.bias, args.bias_type, args.m, stream);
@@ -348,12 +352,12 @@ hipError_t launch_wide_tokens(SkinnyArgs args, int rows_per_group, hipStream_t s
 
 hipError_t launch_wide_tokens_group(SkinnyGroupArgs g, int rows_per_group, hipStream_t stream) {
   if (g.count < 1 || g.count > kSkinnyMaxGroup || rows_per_group < 1) return hipErrorInvalidValue;
-  const int tokens = g.problem[0].n;
-  if (tokens < 1 || tokens > kSkinnyMaxN) return hipErrorInvalidValue;
+  const int n = g.problem[0].n, tokens = g.problem[0].tokens_per_group;
+  if (n < 1 || tokens < 1 || tokens > kSkinnyMaxN) return hipErrorInvalidValue;
   int blocks = 0;
   for (int i = 0; i < g.count; ++i) {
     SkinnyArgs& p = g.problem[i];
-    if (p.n != tokens || p.bf16 != g.problem[0].bf16 || p.m <= 0 || p.k <= 0 || !p.prep || !p.b || !p.d || !wide_operand_fits(p))
+    if (p.n != n || p.tokens_per_group != tokens || p.bf16 != g.problem[0].bf16 || p.m <= 0 || p.k <= 0 || !p.prep || !p.b || !p.d || !wide_operand_fits(p))
       return hipErrorInvalidValue;
     p.splits = 1;
     p.chunks_per_split = p.kc_total;
@@ -362,7 +366,7 @@ hipError_t launch_wide_tokens_group(SkinnyGroupArgs g, int rows_per_group, hipSt
     blocks += (p.m + rows_per_group - 1) / rows_per_group;
   }
   g.first_block[g.count] = blocks;
-  return launch_wide_rows(g, rows_per_group, tokens, g.problem[0].bf16, dim3(blocks), stream);
+  return launch_wide_rows(g, rows_per_group, tokens, g.problem[0].bf16, dim3(blocks, 1, (n + tokens - 1) / tokens), stream);
 }
 
 }  // namespace onebit

@@ -68,3 +68,14 @@ def test_values_behind_the_last_token_do_not_matter():
     _native.linear_prepared(PreparedWeight(a, meta).buffer, x[:tokens], y[:tokens], m, k)
     assert torch.equal(y[:tokens].cpu().double(), x[:tokens].cpu().double() @ _dense(a, meta).T)
     assert bool((y[tokens] == 7).all())
+
+
+@pytest.mark.parametrize("m,k,tokens", [(64, 32, 65), (192, 1056, 100), (448, 96, 257), (1024, 512, 129), (512, 4640, 70)])
+def test_more_tokens_than_one_workgroup_takes(m, k, tokens):
+    a, meta = synthetic.make_weight(m, k, 4, device="cuda")
+    x = torch.randint(-4, 5, (tokens, k), generator=torch.Generator().manual_seed(tokens)) / 2
+    want = (x.double() @ _dense(a, meta).T).float()
+    for dtype in (torch.float16, torch.bfloat16):
+        y = torch.full((tokens + 1, m), 7.0, device="cuda")
+        _native.linear_prepared(PreparedWeight(a, meta).buffer, x.to("cuda", dtype), y[:tokens], m, k)
+        assert torch.equal(y[:tokens].cpu(), want) and bool((y[tokens] == 7).all())
