@@ -33,7 +33,8 @@ __global__ __launch_bounds__(256) void pad_b_kernel(const _Float16* __restrict__
     const int r = rows > 1 ? (int)__umulhi(local, reciprocal) : 0, col = 8 * (piece0 + local - r * per_row);
     const int row = row0 + r;
     if (r >= rows || row >= k || col >= ldb) continue;
-    if (row == k - 1 && col + 8 > n) v[i] = drop_halves(v[i], col + 8 - n);
+    const size_t start = (size_t)row * n + col;
+    if (start > last_start) v[i] = drop_halves(v[i], (int)(start - last_start));
     *reinterpret_cast<u32x4_t*>(dst + (size_t)row * ldb + col) = v[i];
   }
 }

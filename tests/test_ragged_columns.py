@@ -64,3 +64,20 @@ def test_split_k_kernel_any_columns(rows, n):
             assert np.array_equal(d.cpu().numpy(), want), (m, k, shift)
     finally:
         _native.set_skinny_rows(-1)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 7, 9])
+@pytest.mark.parametrize("k", [28672, 65536])
+def test_padded_copy_of_rows_shorter_than_a_piece(n, k):
+    """Several of B's last rows end within one 16-byte piece of its end (or all of them, n < 8)."""
+    m = 64
+    a, meta = synthetic.make_weight(m, k, seed=n)
+    b = synthetic.make_b(k, n, seed=n, kind="int")
+    _native.set_skinny_enabled(False)
+    try:
+        d = torch.empty((m, n), dtype=torch.float32, device="cuda")
+        _native.matmul_prepared(_native.prepare(a.cuda(), meta.cuda(), m, k), b.cuda(), d, m, n, k)
+    finally:
+        _native.set_skinny_enabled(True)
+    ref = oracle.reference_matmul(a.numpy(), b.numpy(), meta.numpy(), m, n, k, d_dtype=oracle.F32)
+    assert np.array_equal(d.cpu().numpy(), ref)
