@@ -37,8 +37,9 @@ void onebit_sparse_set_pad_b(int enabled);
  * the compute-unit count of the current device, as the calls themselves do; without a usable device (a host without a
  * GPU) for 256 compute units, the MI355X figure. plan[0] = 1 for the split-K kernel (n <= 64), 0 for the main kernel;
  * plan[1] = weight rows per workgroup (split-K kernel) or the tile code (main kernel); plan[2] = K splits over
- * workgroups (1 = none); plan[3] = 1 if B is read through a padded copy. The linear-layer entry points plan calls of more
- * than 16 tokens by a model of their own on top of this one. onebit_sparse_describe_launch_for does the
+ * workgroups (1 = none); plan[3] = 1 if B is read through a padded copy. Calls of more
+ * than 16 columns or tokens that the split-K kernel with asynchronous copies of B (csrc/onebit_wide.h) is modelled to run
+ * faster than this plan go there instead; a product then splits K only if this plan does. onebit_sparse_describe_launch_for does the
  * same for an explicit compute-unit count and never touches a device. */
 int onebit_sparse_describe_launch(int m, int n, int k, int b_16_byte_aligned, int *plan);
 int onebit_sparse_describe_launch_for(int m, int n, int k, int b_16_byte_aligned, int compute_units, int *plan);

@@ -29,7 +29,7 @@ def build_library():
     # one compiler per source, side by side
     objs, compilers = [], []
     for src in ("onebit_gemm.hip", "onebit_gemm_tokens.hip", "onebit_skinny.hip", "onebit_skinny_tokens.hip",
-                "onebit_wide_tokens.hip", "onebit_format.hip", "onebit_capi.hip", "onebit_diag.hip"):
+                "onebit_wide.hip", "onebit_wide_tokens.hip", "onebit_format.hip", "onebit_capi.hip", "onebit_diag.hip"):
         obj = os.path.join(CSRC, src.replace(".hip", ".o"))
         cmd = [HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
         print("+", " ".join(cmd), flush=True)

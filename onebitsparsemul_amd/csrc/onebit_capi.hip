@@ -301,7 +301,7 @@ SkinnyPlan plan_skinny(int m, int n, int k, int compute_units) {
   return SkinnyPlan{rows, 1};
 }
 
-// Row group, tokens per workgroup and K splits over workgroups of wide_tokens_kernel: the plan with the least modelled time.
+// Row group, tokens per workgroup and K splits over workgroups of wide_kernel: the plan with the least modelled time.
 // A workgroup's wavefronts each multiply one K chunk per round; a round's time depends on the row group and the number of
 // sixteen-token column tiles and grows with the share of compute units that load at the same time. Workgroups beyond one per
 // compute unit pay the rounds again, less where two fit a compute unit (up to two column tiles on up to 64 rows). A split
@@ -315,13 +315,17 @@ struct WidePlan {
   int rows, splits, tokens;
   double us;
 };
-WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, bool may_split, int compute_units) {
+WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, bool plain, int least_splits,
+                   int most_splits, int compute_units) {
   // [row group][column tiles - 1]
   static const double kBase[3][4] = {{2.75, 2.9, 2.9, 3.0}, {3.1, 3.3, 3.4, 3.6}, {3.7, 4.3, 5.8, 6.4}};
   static const double kRound[3][4] = {{0.74, 0.93, 1.48, 1.89}, {1.01, 1.26, 1.74, 2.24}, {1.88, 2.4, 2.75, 3.25}};
   static const double kLoad[3][4] = {{0.55, 0.55, 0.55, 0.55}, {0.23, 0.44, 0.5, 0.5}, {0.14, 0.24, 0.4, 0.4}};
   static const double kAgain[3][4] = {{0.57, 1.1, 1.0, 1.0}, {0.73, 0.9, 1.0, 1.0}, {1.0, 1.0, 1.0, 1.0}};
   static const double kSplitLines[3] = {1.17, 1.17, 1.05};  // k % 64 != 0: every second token's pieces straddle two lines
+  // plain form, several column groups: a group's piece of a row of B is a part of a line, 32 to 128 bytes (4096 x 64 x 4096 in
+  // four groups 11.0 us against 5.8 token-major, in two 7.1 against 5.1)
+  static const double kColumns[4] = {2.3, 1.45, 1.4, 1.1};
   const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
   WidePlan best{g_skinny_rows > 0 ? g_skinny_rows : 32, 1, std::min(n, onebit::kSkinnyMaxN), 1e30};
   for (int width = 1; width <= 4; ++width) {
@@ -331,18 +335,19 @@ WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, 
     for (int r = 0; r < 3; ++r) {
       if (g_skinny_rows > 0 && g_skinny_rows != kWideRows[r]) continue;
       for (int s : {1, 2, 3, 4, 6, 8}) {
-        if (g_split_k >= 1 && may_split) s = std::min(g_split_k, chunks);
-        if (s > 1 && (!may_split || s > chunks)) break;
+        if (g_split_k >= 1) s = g_split_k;
+        s = std::min(std::min(s, most_splits), chunks);
+        if (s < least_splits) continue;
         const int rounds = ((chunks + s - 1) / s + 7) / 8;
         const double load = (double)total_groups[r] * groups * s / compute_units;
         const double work = rounds * kRound[r][tiles - 1] * (1.0 + kLoad[r][tiles - 1] * std::min(1.0, load)) *
-                            (k % 64 ? kSplitLines[r] : 1.0);
+                            (plain ? (groups > 1 ? kColumns[tiles - 1] : 1.0) : k % 64 ? kSplitLines[r] : 1.0);
         double us = kBase[r][tiles - 1] + work;
         if (load > 1.0)
           us += (std::ceil(load) - 1.0) * (work * kAgain[r][tiles - 1] + (kBase[r][tiles - 1] - 1.5) * (r < 2 ? 0.4 : 1.0));
         if (s > 1) us += 2.6 + 0.15 * s + (s + 1) * 4.0 * results / 5.0e6;
         if (us < best.us) best = WidePlan{kWideRows[r], s, tokens, us};
-        if (g_split_k >= 1) break;
+        if (g_split_k >= 1 || s == most_splits) break;
       }
     }
   }
@@ -373,8 +378,8 @@ LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int comput
   return plan;
 }
 
-// The linear layer's plan: wide = wide_tokens_kernel with `wide_plan`, else `launch` as for a product with an aligned B.
-// Up to sixteen tokens the split-K kernel; beyond 64 whichever of wide_tokens_kernel and the main kernel is modelled faster
+// The linear layer's plan: wide = wide_kernel with `wide_plan`, else `launch` as for a product with an aligned B.
+// Up to sixteen tokens the split-K kernel; beyond 64 whichever of wide_kernel and the main kernel is modelled faster
 // (the main kernel's model is up to 12 % above its measured times where the two meet). A layer call may split K, i.e. needs
 // a buffer, only where the other kernel's plan would: what can be captured without a warm-up stays so.
 struct LinearPlan {
@@ -389,8 +394,22 @@ LinearPlan plan_linear(int m, int tokens, int k, int compute_units) {
   const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
   const bool beyond = tokens > onebit::kSkinnyMaxN;
   if (beyond && (g_tile_config >= 0 || groups[2] * ((tokens + 63) / 64) > 2L * compute_units)) return plan;
-  plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, plan.launch.splits > 1 || g_split_k >= 1, compute_units);
+  const int most_splits = g_split_k >= 1 ? g_split_k : plan.launch.splits > 1 ? 8 : 1;
+  plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, false, 1, most_splits, compute_units);
   plan.wide = !beyond || plan.wide_plan.us < 0.88 * plan.launch.model_us;
+  return plan;
+}
+
+// The product's: wide_kernel in the place of `launch` where that reads B in place or through its padded copy, for 17 columns
+// or more and where it is modelled faster. It splits K where `launch` does, into no more parts, and uses the same buffers, so
+// what a call needs, and whether it can be captured, does not depend on the choice.
+WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b_readable, int compute_units) {
+  WidePlan none{0, 1, 0, 0.0};
+  const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
+  if (n <= 16 || !g_skinny_enabled || g_tile_config >= 0 || groups[2] * ((n + 63) / 64) > 2L * compute_units) return none;
+  if (!b_readable) return none;
+  const WidePlan plan = plan_wide(groups, (double)m * n, n, k, true, launch.splits > 1 ? 2 : 1, launch.splits, compute_units);
+  if (plan.us == 1e30 || (!launch.split_k_kernel && plan.us >= 0.85 * launch.model_us)) return none;
   return plan;
 }
 
@@ -430,13 +449,36 @@ int setup_skinny_split(onebit::SkinnyArgs& args, int splits, hipStream_t stream,
   return ONEBIT_OK;
 }
 
+// Whether a padded copy of a small B (the plan does not count on one) can be made without failing a call that went through
+// without it: never inside a capture that would have to allocate, and never in a fixed workspace, whose size the plan is
+// checked against.
+bool small_pad_available(size_t bytes, hipStream_t stream, const FixedScratch* fixed) {
+  int device = 0;
+  if (fixed || hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices) return false;
+  DeviceState& st = g_dev[device];
+  std::lock_guard<std::recursive_mutex> lock(st.mu);
+  Buffer& pb = st.b_pad[stream];
+  if (bytes <= pb.bytes) return true;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
+  return grow(&pb.ptr, &pb.bytes, bytes, stream) == ONEBIT_OK;
+}
+
 int matmul_prepared_impl(const void* prepared, const void* b, const void* c, void* d, int m, int n, int k, float alpha,
                          float beta, int c_dtype, int d_dtype, hipStream_t stream, const FixedScratch* fixed = nullptr) {
   if (!prepared || !b || !d) return fail(ONEBIT_ERR_ARGUMENT, "null operand pointer");
   if (beta != 0.f && !c) return fail(ONEBIT_ERR_ARGUMENT, "c must not be null when beta != 0");
   const int kc_total = (k + onebit::kChunkK - 1) / onebit::kChunkK;
 
-  const LaunchPlan plan = choose_launch(m, n, k, (reinterpret_cast<uintptr_t>(b) & 15) == 0, current_compute_units());
+  const int compute_units = current_compute_units();
+  const bool b_aligned = (reinterpret_cast<uintptr_t>(b) & 15) == 0;
+  const LaunchPlan plan = choose_launch(m, n, k, b_aligned, compute_units);
+  const bool b_in_place = n % 8 == 0 && b_aligned;
+  // A small B that the main kernel cannot read in place is described as read by element copies; a padded copy is many times
+  // faster (1152 x 78 x 640 61 -> 6 us) and is made wherever its buffer is there or can be had.
+  const size_t pad_bytes = (size_t)k * ((size_t)(n + 7) / 8 * 8) * sizeof(_Float16);
+  const bool pad_b = plan.pad_b || (!plan.split_k_kernel && !b_in_place && g_pad_b && small_pad_available(pad_bytes, stream, fixed));
+  const WidePlan wide = plan_wide_product(plan, m, n, k, b_in_place || pad_b, compute_units);
   if (plan.split_k_kernel) {
     onebit::SkinnyArgs args{};
     args.prep = static_cast<const uint8_t*>(prepared);
@@ -448,8 +490,10 @@ int matmul_prepared_impl(const void* prepared, const void* b, const void* c, voi
     args.alpha = alpha; args.beta = beta;
     args.c_f16 = c_dtype == ONEBIT_DTYPE_F16;
     args.d_f16 = d_dtype == ONEBIT_DTYPE_F16;
-    if (int rc = setup_skinny_split(args, plan.splits, stream, fixed); rc != ONEBIT_OK) return rc;
-    ONEBIT_HIP(onebit::launch_skinny(args, plan.rows_or_tile, stream));
+    args.tokens_per_group = wide.tokens;
+    args.ldb = n;
+    if (int rc = setup_skinny_split(args, wide.rows ? wide.splits : plan.splits, stream, fixed); rc != ONEBIT_OK) return rc;
+    ONEBIT_HIP(wide.rows ? onebit::launch_wide(args, wide.rows, stream) : onebit::launch_skinny(args, plan.rows_or_tile, stream));
     return ONEBIT_OK;
   }
 
@@ -468,29 +512,51 @@ int matmul_prepared_impl(const void* prepared, const void* b, const void* c, voi
   args.c_f16 = c_dtype == ONEBIT_DTYPE_F16;
   args.d_f16 = d_dtype == ONEBIT_DTYPE_F16;
   const int tile = plan.rows_or_tile;
-  const int splits = plan.splits;
-  const bool pad_b = plan.pad_b != 0;
+  const int splits = wide.rows ? wide.splits : plan.splits;
+  auto launch = [&]() -> hipError_t {
+    if (!wide.rows) return onebit::launch_gemm(args, tile, stream);
+    onebit::SkinnyArgs w{};
+    w.prep = args.prep;
+    w.b = args.b;
+    w.c = c;
+    w.d = d;
+    w.m = m; w.n = n; w.k = k;
+    w.kc_total = kc_total;
+    w.alpha = alpha; w.beta = beta;
+    w.c_f16 = args.c_f16;
+    w.d_f16 = args.d_f16;
+    w.splits = args.splits;
+    w.chunks_per_split = args.chunks_per_split;
+    w.split_ws = args.split_ws;
+    w.tokens_per_group = wide.tokens;
+    w.ldb = n;
+    if (pad_b) {
+      if (hipError_t st = onebit::launch_pad_b(args.b, args.b_pad, k, n, stream); st != hipSuccess) return st;
+      w.b = args.b_pad;
+      w.ldb = (n + 7) / 8 * 8;
+    }
+    return onebit::launch_wide(w, wide.rows, stream);
+  };
   if (splits > 1 || pad_b) {
-    size_t split_bytes = 0, pad_bytes = 0;
+    size_t split_bytes = 0;
     if (splits > 1) {
       const int cps = (kc_total + splits - 1) / splits;
       args.chunks_per_split = cps;
       args.splits = (kc_total + cps - 1) / cps;  // every split non-empty
       split_bytes = (size_t)args.splits * m * n * sizeof(float);
     }
-    if (pad_b) pad_bytes = (size_t)k * ((size_t)(n + 7) / 8 * 8) * sizeof(_Float16);
     if (fixed) {
       // partial sums first, the padded copy of B behind them on the next 256-byte boundary; both are written in
       // full by this call's own kernels before they are read, so nothing has to start at zero
-      const size_t pad_at = (split_bytes + 255) & ~size_t(255);
-      if (pad_at + pad_bytes > fixed->bytes)
+      const size_t pad_at = (split_bytes + 255) & ~size_t(255), pad_need = pad_b ? pad_bytes : 0;
+      if (pad_at + pad_need > fixed->bytes)
         return fail(ONEBIT_ERR_ARGUMENT,
                     "this shape needs %zu bytes of scratch (%d K splits of %d x %d fp32 partial sums, %zu bytes of "
                     "padded B); the static workspace of the non-allocating entry point holds %zu",
-                    pad_at + pad_bytes, splits > 1 ? args.splits : 0, m, n, pad_bytes, fixed->bytes);
+                    pad_at + pad_need, splits > 1 ? args.splits : 0, m, n, pad_need, fixed->bytes);
       if (splits > 1) args.split_ws = reinterpret_cast<float*>(fixed->base);
       if (pad_b) args.b_pad = reinterpret_cast<_Float16*>(fixed->base + pad_at);
-      ONEBIT_HIP(onebit::launch_gemm(args, tile, stream));
+      ONEBIT_HIP(launch());
       return ONEBIT_OK;
     }
     int device = 0;
@@ -508,10 +574,10 @@ int matmul_prepared_impl(const void* prepared, const void* b, const void* c, voi
       if (int rc = grow(&pb.ptr, &pb.bytes, pad_bytes, stream); rc != ONEBIT_OK) return rc;
       args.b_pad = static_cast<_Float16*>(pb.ptr);
     }
-    ONEBIT_HIP(onebit::launch_gemm(args, tile, stream));
+    ONEBIT_HIP(launch());
     return ONEBIT_OK;
   }
-  ONEBIT_HIP(onebit::launch_gemm(args, tile, stream));
+  ONEBIT_HIP(launch());
   return ONEBIT_OK;
 }
 
@@ -743,7 +809,7 @@ int onebit_sparse_linear_prepared_grouped_typed(const onebit_linear_problem* pro
     }
     const int enough = std::max(1, 160 * compute_units / 256);
     WidePlan wide_plan{};
-    if (wide) wide_plan = plan_wide(groups, 0.0, tokens, longest_k, false, compute_units);
+    if (wide) wide_plan = plan_wide(groups, 0.0, tokens, longest_k, false, 1, 1, compute_units);
     const int rows = wide ? wide_plan.rows
                      : g_skinny_rows > 0 ? g_skinny_rows
                      : (rows_total / 128 >= enough) ? 128 : (rows_total / 64 >= enough) ? 64 : 32;

@@ -131,19 +131,21 @@ static hipError_t launch_gemm_pass(GemmArgs args, int tile_config, hipStream_t s
   }
 }
 
+hipError_t launch_pad_b(const _Float16* b, _Float16* dst, int k, int n, hipStream_t stream) {
+  const int per_row = (n + 7) / 8, rows = per_row > 1 && per_row < kPadPieces ? kPadPieces / per_row : 1;
+  hipLaunchKernelGGL(pad_b_kernel, dim3((k + rows - 1) / rows, (per_row + kPadPieces - 1) / kPadPieces), dim3(256), 0, stream, b,
+                     dst, k, n, 8 * per_row, rows, (uint32_t)((uint64_t(1) << 32) / per_row + 1));
+  return hipGetLastError();
+}
+
 hipError_t launch_gemm(GemmArgs args, int tile_config, hipStream_t stream) {
   if (prepared_bytes(args.m, args.k) >= (size_t(1) << 32)) return hipErrorInvalidValue;  // 32-bit copy offsets
   args.ldb = args.n;
   const bool aligned = (args.n % 8 == 0) && ((reinterpret_cast<uintptr_t>(args.b) & 15) == 0);
   if (!aligned && args.b_pad) {
-    const int ldb = (args.n + 7) / 8 * 8;
-    const int per_row = ldb / 8, rows = per_row > 1 && per_row < kPadPieces ? kPadPieces / per_row : 1;
-    hipLaunchKernelGGL(pad_b_kernel, dim3((args.k + rows - 1) / rows, (per_row + kPadPieces - 1) / kPadPieces), dim3(256), 0,
-                       stream, args.b, args.b_pad, args.k, args.n, ldb, rows,
-                       (uint32_t)((uint64_t(1) << 32) / per_row + 1));
-    if (hipError_t st = hipGetLastError(); st != hipSuccess) return st;
+    if (hipError_t st = launch_pad_b(args.b, args.b_pad, args.k, args.n, stream); st != hipSuccess) return st;
     args.b = args.b_pad;
-    args.ldb = ldb;
+    args.ldb = (args.n + 7) / 8 * 8;
   }
   const int chunks = (args.k + kChunkK - 1) / kChunkK;
   if (args.splits <= 1) {

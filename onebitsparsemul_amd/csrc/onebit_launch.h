@@ -57,8 +57,10 @@ struct SkinnyArgs {
   int splits;
   int chunks_per_split;
   float* split_ws;
-  // wide_tokens_kernel only: tokens a workgroup multiplies (at most 64), grid.z = ceil(n / tokens_per_group)
+  // wide_kernel only: tokens (columns) a workgroup multiplies (at most 64), grid.z = ceil(n / tokens_per_group); ldb: elements
+  // between B rows in the plain form
   int tokens_per_group;
+  int ldb;
 };
 
 // Several token-major products with the same token count in one launch of the split-K kernel (no K split over
@@ -89,6 +91,9 @@ hipError_t launch_split_reduce(const float* ws, int splits, size_t total, const 
                                       float beta, int c_f16, int d_type, const void* bias, int bias_type, int row_length,
                                       hipStream_t stream);
 
+// B with rows padded to a multiple of eight columns (dst: k * round_up(n, 8) halves).
+hipError_t launch_pad_b(const _Float16* b, _Float16* dst, int k, int n, hipStream_t stream);
+
 // Split-K kernel for n <= 64; rows_per_group (32, 64 or 128) = weight rows one workgroup covers (n > 32: at most 64).
 constexpr int kSkinnyMaxN = 64;
 hipError_t launch_skinny(SkinnyArgs args, int rows_per_group, hipStream_t stream);
@@ -99,9 +104,11 @@ hipError_t launch_skinny_tokens(SkinnyArgs args, int rows_per_group, hipStream_t
 // count <= kSkinnyMaxGroup problems of the same form, each with its own weight, x, bias, y, m and k, in one launch.
 hipError_t launch_skinny_group(SkinnyGroupArgs group, int rows_per_group, hipStream_t stream);
 
-// The linear layer's form whose images of x asynchronous copies bring to LDS (wide_tokens_kernel): any number of tokens, in
+// The linear layer's form whose images of x asynchronous copies bring to LDS (wide_kernel): any number of tokens, in
 // groups of at most 64 per workgroup; row groups of 32, 64 or 128.
 hipError_t launch_wide_tokens(SkinnyArgs args, int rows_per_group, hipStream_t stream);
+// The plain form: B 16-byte aligned with ldb % 8 == 0, columns in groups of a multiple of eight, at most 64.
+hipError_t launch_wide(SkinnyArgs args, int rows_per_group, hipStream_t stream);
 hipError_t launch_wide_tokens_group(SkinnyGroupArgs group, int rows_per_group, hipStream_t stream);
 
 }  // namespace onebit

@@ -1,0 +1,334 @@
+// The split-K kernel whose images of B asynchronous copies bring to LDS, plain and token-major, and the launch of one
+// instantiation. onebit_wide.hip and onebit_wide_tokens.hip instantiate it.
+#pragma once
+#include "onebit_skinny.h"
+
+#include <atomic>
+
+namespace onebit {
+
+// =====================================================================================================
+// wide_tokens_kernel: y[t][r] = sum_k W[r][k] x[t][k] + bias[r] for up to 64 tokens.
+// Workgroup = eight wavefronts that share R row blocks (32 rows each) and split K among themselves chunk by chunk, as in
+// skinny_kernel. What differs is how x gets to the matrix cores: every wavefront keeps a ring of two images (64 K values of
+// all tokens, 2 KB per sixteen) in LDS that asynchronous copies fill. No registers hold x on its way, so the tile can be
+// 128 x 64 (R = 4), and with v_smfmac_f32_16x16x64 there are no idle columns at 24 or 48 tokens; one fragment read from LDS
+// serves 2 R SMFMACs.
+// Bound: with many tokens the bytes of x that pass through LDS. skinny_kernel's 64-row groups staged x through registers,
+// 16 KB of LDS writes and reads per 64 x 64 weights; a 128-row group halves that (28672 x 8192 with 48 tokens: 13 us of LDS
+// time, 12 of SMFMACs and 6 of sign expansion that hardly overlapped). us inside a HIP graph, weights from HBM, before ->
+// now: 28672 x 8192 with 24 / 48 / 64 tokens 16.6 / 33.4 / 35.9 -> 16.6 / 21.0 / 24.5; 11008 x 4096 8.0 / 11.0 / 11.7 -> 6.8 /
+// 8.3 / 9.6; 4096 x 4096 5.7 / 8.4 / 8.7 -> 4.7 / 6.0 / 7.1; 1024 x 1024 with 56 5.0 -> 3.5. Up to sixteen tokens there is no
+// gain (11008 x 4096 with 16: 6.4 -> 6.1, with 4: 5.5 -> 5.8; 28672 x 8192 with 16: 13.5 -> 14.0): skinny_kernel keeps those.
+// =====================================================================================================
+// Source of zeros for the copies of K positions at or past K.
+static __device__ __attribute__((aligned(16))) uint32_t g_zero16_wide[4] = {0, 0, 0, 0};
+
+constexpr int kWideWaves = 8;
+constexpr int kWideImageK = 64;
+
+template <int R, int COPIES>
+struct WideShape {
+  static constexpr int CT = (COPIES + 1) / 2;            // column tiles of sixteen tokens
+  static constexpr int IMAGE_BYTES = 16 * CT * kWideImageK * 2;
+  static constexpr int REGION = 2 * IMAGE_BYTES;         // ring of one wavefront; holds the sums of RT row blocks at the end
+  static constexpr int RT = R < 2 ? R : 2;
+  static constexpr int LDS_BYTES = kWideWaves * REGION;
+};
+
+// COPIES: 1 KiB copies per image, one per eight tokens. A workgroup multiplies up to 8 COPIES tokens from first_token on.
+// TOKENS = false is the plain form, D = alpha A B + beta C, a column of B in the place of a token: B's rows start 16-byte
+// aligned (ldb % 8 == 0, first_token % 8 == 0), an image is 64 of them as they lie, COPIES 16-byte pieces each, read through
+// transpose reads; COPIES is even.
+template <int R, int COPIES, bool TOKENS, bool BF16>
+__device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x, const int block_y, const int first_token,
+                                          char* const smem) {
+  using Shape = WideShape<R, COPIES>;
+  constexpr int NW = kWideWaves, CT = Shape::CT, RT = Shape::RT;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rb_total = p.m / kRowBlock, rb_first = block_x * R;
+  char* const region = smem + wave * Shape::REGION;
+  const uint32_t region_offset = lds_offset_of(smem) + wave * Shape::REGION;
+  const int kc_total = p.kc_total, k_total = p.k;
+  const int tokens = p.n - first_token < 8 * COPIES ? p.n - first_token : 8 * COPIES;
+  const int kc_begin = block_y * p.chunks_per_split;
+  const int kc_end = kc_begin + p.chunks_per_split < kc_total ? kc_begin + p.chunks_per_split : kc_total;
+  const int first = kc_begin + wave;
+
+  const uint32_t meta_off = (uint32_t)lane * 16u, sign_off = (uint32_t)kSignOffset + (uint32_t)lane * 8u;
+  buffer_t a_buffer[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    int rb = rb_first + r;
+    if (rb >= rb_total) rb = rb_total - 1;  // never stored
+    a_buffer[r] = make_buffer(p.prep + (size_t)rb * kc_total * kBlockBytes, (uint32_t)kc_total * kBlockBytes);
+  }
+  auto load_a = [&](int kc, AChunk (&a)[R]) __attribute__((always_inline)) {
+    if (kc >= kc_total) kc = kc_total - 1;  // never multiplied
+    const uint32_t block = (uint32_t)kc * kBlockBytes;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      a[r].meta = buffer_load16(a_buffer[r], meta_off, block);
+      a[r].sign = buffer_load8(a_buffer[r], sign_off, block);
+    }
+  };
+  AChunk raw[R], next[R] = {};
+  load_a(first, raw);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // Plain form: piece q of row r lies at position q ^ row_swizzle(r), so that the 32 lanes of one transpose read (rows r ...
+  // r + 3 and r + 8 ... r + 11, 32 bytes each) meet in no bank where the row stride would make them.
+  constexpr int PIECES = 2 * CT;
+  auto row_swizzle = [](int row) __attribute__((always_inline)) {
+    return PIECES == 8 ? (((row >> 1) & 1) << 2) | (((row >> 3) & 1) << 1) : PIECES == 4 ? ((row >> 3) & 1) << 1 : 0;
+  };
+  // copy i of an image: tokens 8 i ... 8 i + 7, eight 16-byte pieces each; piece q of token t lies at position
+  // q ^ token_swizzle(t). Tokens past the end: the last one again, their results are not stored.
+  uint32_t copy_off[COPIES];
+  const int piece0 = (lane & 7) ^ (lane >> 4);
+#pragma unroll
+  for (int i = 0; i < COPIES; ++i) {
+    if constexpr (TOKENS) {
+      int token = 8 * i + (lane >> 3);
+      if (token >= tokens) token = tokens - 1;
+      copy_off[i] = ((uint32_t)token * (uint32_t)k_total + 8u * (piece0 ^ (4 * (i & 1)))) * 2u;
+    } else {
+      const int row = (64 * i + lane) / PIECES;
+      int col = 8 * (((64 * i + lane) % PIECES) ^ row_swizzle(row));
+      if (first_token + col >= p.ldb) col = 0;  // columns past the row's end: the first ones again, never stored
+      copy_off[i] = ((uint32_t)row * (uint32_t)p.ldb + col) * 2u;
+    }
+  }
+  const size_t k_stride = TOKENS ? 2 : (size_t)p.ldb * 2;  // bytes from one K position to the next
+  const char* const x_bytes = reinterpret_cast<const char*>(p.b + (TOKENS ? (size_t)first_token * k_total : (size_t)first_token));
+  const char* const zeros = reinterpret_cast<const char*>(g_zero16_wide);
+  auto copy_image = [&](int k0, int slot) __attribute__((always_inline)) {
+    const uint32_t dst = region_offset + slot * Shape::IMAGE_BYTES;
+    if (k0 + kWideImageK <= k_total) {  // wave-uniform
+#pragma unroll
+      for (int i = 0; i < COPIES; ++i) lds_dma16_base(x_bytes + k0 * k_stride, copy_off[i], dst + i * 1024);
+    } else {
+      // K positions at or past k come from a block of zeros
+#pragma unroll
+      for (int i = 0; i < COPIES; ++i) {
+        uint32_t off = copy_off[i];
+        asm volatile("" : "+v"(off));  // keeps the 64-bit addresses out of the registers of the other path
+        const int k = k0 + (TOKENS ? 8 * (piece0 ^ (4 * (i & 1))) : (64 * i + lane) / PIECES);
+        lds_dma16(k < k_total ? x_bytes + k0 * k_stride + off : zeros, dst + i * 1024);
+      }
+    }
+  };
+
+  const int i16 = lane & 15, g16 = lane >> 4;
+  const uint32_t one = packed_one_in_vgpr<BF16>();
+  float4v_t acc[2 * R][CT];
+#pragma unroll
+  for (int rt = 0; rt < 2 * R; ++rt)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      acc[rt][ct] = float4v_t{0.f, 0.f, 0.f, 0.f};
+      asm volatile("" : "+v"(acc[rt][ct]));
+    }
+
+  // Operands of one chunk. A lane of the prepared block (row l % 32, half ga) holds, per 32-wide step, what a lane of the
+  // instruction (row l % 16, group g) holds for sixteen K positions. With the index halves of two stages' even steps in one
+  // register and those of their odd steps in another, one v_permlane16_swap leaves the groups (even, ga 0), (odd, ga 0),
+  // (even, ga 1), (odd, ga 1) of block rows 0-15 in the first and of rows 16-31 in the second; ABID picks the stage. Group g
+  // thus covers K positions 32 (g % 2) + 16 (g / 2) + [0, 16) of the 64-wide stage.
+  struct ATile {
+    uint32_t idx[2][2], sign[2][2];  // [row half][stage pair]
+  };
+  ATile t[R];
+  const uint32_t sign_shift = 4u * (g16 & 1);
+  auto gather = [&](const AChunk (&a)[R]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const uint32_t even = __builtin_amdgcn_perm(a[r].meta[2 * q + 1], a[r].meta[2 * q], 0x05040100u);
+        const uint32_t odd = __builtin_amdgcn_perm(a[r].meta[2 * q + 1], a[r].meta[2 * q], 0x07060302u);
+        const auto m = __builtin_amdgcn_permlane16_swap(even, odd, false, false);
+        const uint32_t w = q == 0 ? a[r].sign.x : a[r].sign.y;
+        const auto sg = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+        t[r].idx[0][q] = m[0];
+        t[r].idx[1][q] = m[1];
+        t[r].sign[0][q] = sg[0] << sign_shift;
+        t[r].sign[1][q] = sg[1] << sign_shift;
+      }
+  };
+  // B operand of column tile ct: pieces 4 (g / 2) + g % 2 and that + 2 of token 16 ct + l % 16
+  const uint32_t read_base = (uint32_t)i16 * 128u + (uint32_t)(((4 * (g16 >> 1) + (g16 & 1)) ^ token_swizzle(i16)) << 4);
+  // plain form: K rows 32 (g / 2) + 8 (g % 2) + {0 ... 7, 16 ... 23} of column l % 16, four by a transpose read
+  const int lane_row = 32 * (g16 >> 1) + 8 * (g16 & 1) + (i16 >> 2);
+  uint32_t tile_off[CT];
+  if constexpr (!TOKENS)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+      tile_off[ct] = lane_row * PIECES * 16 + (((2 * ct + ((i16 & 3) >> 1)) ^ row_swizzle(lane_row)) << 4) + (i16 & 1) * 8;
+  half16_t frag[CT];
+  auto read_image = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      u32x8_t raw_frag;
+      if constexpr (!TOKENS) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const u32x2_t v = lds_read_tr16(region + slot * Shape::IMAGE_BYTES + tile_off[ct] + (4 * (q & 1) + 16 * (q >> 1)) * PIECES * 16);
+          raw_frag[2 * q] = v.x; raw_frag[2 * q + 1] = v.y;
+        }
+      } else
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(region + (read_base ^ (h << 5)) + slot * Shape::IMAGE_BYTES + ct * 2048);
+        raw_frag[4 * h] = v.x; raw_frag[4 * h + 1] = v.y; raw_frag[4 * h + 2] = v.z; raw_frag[4 * h + 3] = v.w;
+      }
+      frag[ct] = __builtin_bit_cast(half16_t, raw_frag);
+    }
+  };
+  auto compute = [&](auto s_tag) __attribute__((always_inline)) {
+    constexpr int S = decltype(s_tag)::value;
+    // the signs of the next row tile are expanded in front of the SMFMACs of the current one; the fences keep the optimizer
+    // from expanding all of them first, which takes more registers than there are
+    auto expand = [&](int rt) __attribute__((always_inline)) {
+      u32x4_t av;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) av[q] = ((t[rt >> 1].sign[rt & 1][S / 2] << (8 * (S & 1) + q)) & 0x80008000u) | one;
+      return __builtin_bit_cast(half8_t, av);
+    };
+    half8_t av[2];
+    av[0] = expand(0);
+#pragma unroll
+    for (int rt = 0; rt < 2 * R; ++rt) {
+      if (rt + 1 < 2 * R) av[(rt + 1) & 1] = expand(rt + 1);
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+        acc[rt][ct] = smfmac16<S & 1, BF16>(av[rt & 1], frag[ct], acc[rt][ct], t[rt >> 1].idx[rt & 1][S / 2]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  // Requests return in order, and a wait names how many younger ones may be outstanding. Per chunk a wavefront requests its
+  // images 2 and 3, the first two images of its next chunk and the prepared operand of the chunk after that; before the loop
+  // the operand of the first chunk, its first two images, the operand of the second. Nothing is requested past the last
+  // chunk (wave-uniform branches).
+  if (first < kc_end) {
+    copy_image(first * kChunkK, 0);
+    copy_image(first * kChunkK + kWideImageK, 1);
+    if (first + NW < kc_end) load_a(first + NW, next);
+    __builtin_amdgcn_sched_barrier(0);
+    gather(raw);
+    int kc = first;
+#pragma unroll 1
+    do {
+      const bool more = kc + NW < kc_end;
+      auto stage = [&](auto s_tag) __attribute__((always_inline)) {
+        constexpr int S = decltype(s_tag)::value;
+        // all but the requests younger than image S
+        if (more) wait_vmcnt<(S < 2 ? COPIES + 2 * R : COPIES)>();
+        else wait_vmcnt<(S < 3 ? COPIES : 0)>();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        read_image(S & 1);
+        if constexpr (S == 2) {
+          // the wait the compiler puts in front of the operand's first use counts its own loads only and so also waits for
+          // every copy issued by then: here that is one image, which has had a stage's time
+#pragma unroll
+          for (int r = 0; r < R; ++r) asm volatile("" : "+v"(next[r].meta), "+v"(next[r].sign));
+        }
+        if (S < 2 || more) {
+          wait_vmcnt_lgkm0<63>();  // the image is in registers: its place is free
+          asm volatile("" ::: "memory");
+          __builtin_amdgcn_sched_barrier(0);
+          copy_image(S < 2 ? kc * kChunkK + (S + 2) * kWideImageK : (kc + NW) * kChunkK + (S - 2) * kWideImageK, S & 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        compute(s_tag);
+      };
+      stage(std::integral_constant<int, 0>{});
+      stage(std::integral_constant<int, 1>{});
+      stage(std::integral_constant<int, 2>{});
+      stage(std::integral_constant<int, 3>{});
+      gather(next);
+      if (kc + 2 * NW < kc_end) load_a(kc + 2 * NW, next);
+      __builtin_amdgcn_sched_barrier(0);
+      kc += NW;
+    } while (kc < kc_end);
+  }
+
+  // ---- add the eight partial tiles, RT row blocks per round: a token's rows as 16-byte slots of four rows, slot s at
+  // position s ^ (token % slots)
+  constexpr int SLOTS = RT * 8;
+  char* const y_out = reinterpret_cast<char*>(p.d) + (size_t)block_y * p.m * p.n * 4 * (p.splits > 1);
+#pragma unroll
+  for (int round = 0; round < R / RT; ++round) {
+    if (round > 0) __syncthreads();
+#pragma unroll
+    for (int rr = 0; rr < RT; ++rr)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+          const int token = 16 * ct + i16, slot = 8 * rr + 4 * h + g16;
+          *reinterpret_cast<float4v_t*>(region + (token * SLOTS + (slot ^ (token & (SLOTS - 1)))) * 16) =
+              acc[2 * (round * RT + rr) + h][ct];
+        }
+    __syncthreads();
+    for (int idx = tid; idx < SLOTS * 16 * CT; idx += 64 * NW) {
+      const int slot = TOKENS ? idx % SLOTS : idx / (16 * CT), token = TOKENS ? idx / SLOTS : idx % (16 * CT);
+      const int at = (token * SLOTS + (slot ^ (token & (SLOTS - 1)))) * 16;
+      float4v_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < NW; ++w) sum += *reinterpret_cast<const float4v_t*>(smem + w * Shape::REGION + at);
+      const int row = (rb_first + round * RT) * kRowBlock + 4 * slot;
+      if (token >= tokens || row >= p.m) continue;
+      if constexpr (!TOKENS) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const size_t o = (size_t)(row + e) * p.n + first_token + token;
+          float x = p.alpha * sum[e];
+          if (p.beta != 0.f)
+            x = x + p.beta * (p.c_f16 ? (float)reinterpret_cast<const _Float16*>(p.c)[o] : reinterpret_cast<const float*>(p.c)[o]);
+          if (p.d_f16) reinterpret_cast<_Float16*>(y_out)[o] = (_Float16)x;
+          else reinterpret_cast<float*>(y_out)[o] = x;
+        }
+        continue;
+      }
+      if (p.bias)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] += load_element(p.bias, p.bias_type, row + e);
+      const size_t o = (size_t)(first_token + token) * p.m + row;
+      if (p.d_f16)
+        *reinterpret_cast<u32x2_any_t*>(y_out + o * 2) = u32x2_t{round_pair<BF16>(sum[0], sum[1]), round_pair<BF16>(sum[2], sum[3])};
+      else
+        *reinterpret_cast<u32x4_any_t*>(y_out + o * 4) = __builtin_bit_cast(u32x4_t, sum);
+    }
+  }
+}
+
+template <int R, int COPIES, bool TOKENS, bool BF16>
+__global__ __launch_bounds__(64 * kWideWaves, 2) void wide_kernel(SkinnyArgs p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  wide_body<R, COPIES, TOKENS, BF16>(p, blockIdx.x, blockIdx.y, blockIdx.z * p.tokens_per_group, smem);
+}
+
+template <int R, int COPIES, class Args>
+static hipError_t launch_wide(void (*kern)(Args), std::atomic<bool> (&attr_done)[64], const Args& args, dim3 grid, hipStream_t stream) {
+  constexpr int lds = WideShape<R, COPIES>::LDS_BYTES;
+  if (lds > 65536) {
+    // the dynamic-LDS limit is a per-device attribute of the kernel; threads that race here set the same value
+    int device = 0;
+    if (hipError_t st = hipGetDevice(&device); st != hipSuccess) return st;
+    if (device < 0 || device >= 64) return hipErrorInvalidDevice;
+    if (!attr_done[device].load(std::memory_order_acquire)) {
+      if (hipError_t st = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+          st != hipSuccess)
+        return st;
+      attr_done[device].store(true, std::memory_order_release);
+    }
+  }
+  hipLaunchKernelGGL(kern, grid, dim3(64 * kWideWaves), lds, stream, args);
+  return hipGetLastError();
+}
+
+}  // namespace onebit

@@ -1,0 +1,35 @@
+"""Products of 17 columns or more on few weight rows: column groups and their remainders, ends of K inside an image, row groups
+past M, padded copies of B, alpha, beta and C of either type, K splits. Integer operands: results must equal the dense product."""
+import pytest
+import torch
+
+from onebitsparsemul_amd import PreparedWeight, _native, dequant_desparse_tile, synthetic
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def hooks():
+    lib = _native.lib()
+    yield lib
+    lib.onebit_sparse_set_skinny_rows(-1)
+    lib.onebit_sparse_set_split_k(-1)
+
+
+@pytest.mark.parametrize("m,k", [(64, 32), (192, 1056), (448, 96), (320, 4640)])
+@pytest.mark.parametrize("rows", [-1, 32, 64, 128])
+def test_columns_equal_the_dense_product(hooks, m, k, rows):
+    a, meta = synthetic.make_weight(m, k, 3, device="cuda")
+    weight, dense = PreparedWeight(a, meta), dequant_desparse_tile(a.cpu(), meta.cpu()).double()
+    g = torch.Generator().manual_seed(m + k)
+    hooks.onebit_sparse_set_skinny_rows(rows)
+    for i, n in enumerate((24, 32, 40, 48, 56, 64, 65, 72, 99, 104, 136, 200, 257)):
+        b = torch.randint(-4, 5, (k, n), generator=g).half()
+        c = torch.randint(-4, 5, (m, n), generator=g).to((torch.float16, torch.float32)[i % 2])
+        for splits in (-1, 2, 3):
+            hooks.onebit_sparse_set_split_k(splits)
+            d = torch.full((m + 1, n), 7.0, device="cuda")
+            weight.matmul(b.cuda(), out=d[:m], c=c.cuda(), alpha=0.5, beta=2.0)
+            assert torch.equal(d[:m].cpu(), (0.5 * (dense @ b.double()) + 2.0 * c.double()).float()), (n, splits)
+            assert bool((d[m] == 7).all())
+        assert torch.equal(weight.matmul(b.cuda()).cpu(), (dense @ b.double()).half())
