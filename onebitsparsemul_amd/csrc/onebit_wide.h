@@ -51,7 +51,10 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
   char* const region = smem + wave * Shape::REGION;
   const uint32_t region_offset = lds_offset_of(smem) + wave * Shape::REGION;
   const int kc_total = p.kc_total, k_total = p.k;
-  const int tokens = p.n - first_token < 8 * COPIES ? p.n - first_token : 8 * COPIES;
+  // plain form: eight columns fewer than the image holds where the group is an odd number of pieces wide. The next group
+  // stores those eight, and D may be C: each element must be read and written once.
+  const int group = TOKENS ? 8 * COPIES : p.tokens_per_group;
+  const int tokens = p.n - first_token < group ? p.n - first_token : group;
   const int kc_begin = block_y * p.chunks_per_split;
   const int kc_end = kc_begin + p.chunks_per_split < kc_total ? kc_begin + p.chunks_per_split : kc_total;
   const int first = kc_begin + wave;

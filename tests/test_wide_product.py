@@ -33,3 +33,19 @@ def test_columns_equal_the_dense_product(hooks, m, k, rows):
             assert torch.equal(d[:m].cpu(), (0.5 * (dense @ b.double()) + 2.0 * c.double()).float()), (n, splits)
             assert bool((d[m] == 7).all())
         assert torch.equal(weight.matmul(b.cuda()).cpu(), (dense @ b.double()).half())
+
+
+@pytest.mark.parametrize("n", [72, 104, 200])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_result_over_c(n, dtype):
+    """D may be C. Column groups of an odd number of 16-byte pieces (40 of 72 columns) do not reach into the next group, which
+    would add C twice there."""
+    m, k = 1024, 2048
+    a, meta = synthetic.make_weight(m, k, 5, device="cuda")
+    weight, dense = PreparedWeight(a, meta), dequant_desparse_tile(a.cpu(), meta.cpu()).double()
+    g = torch.Generator().manual_seed(n)
+    b = torch.randint(-1, 2, (k, n), generator=g).half()
+    c = torch.randint(-4, 5, (m, n), generator=g).to(dtype)
+    d = c.cuda()
+    weight.matmul(b.cuda(), out=d, c=d, alpha=1.0, beta=1.0)
+    assert torch.equal(d.cpu(), (dense @ b.double() + c.double()).to(dtype))
