@@ -30,7 +30,8 @@ void onebit_sparse_set_split_k(int splits);
 /* B whose rows are not 16-byte aligned (n % 8 != 0 or an unaligned base) and n beyond the split-K kernel's range:
  * 1 (default) = the main kernel reads a copy of B with rows padded to a multiple of 8 columns, made by one extra
  * pass into a library-owned buffer kept per device and stream (same rules as the K-split buffer); 0 = the main
- * kernel's element-copy variant reads B in place (much slower; always used when k * n < 65536). */
+ * kernel's element-copy variant reads B in place (much slower). With k * n < 65536 the copy is made where its buffer is there
+ * or can be allocated: not by the non-allocating entry point, and in a stream capture only after a warm-up. */
 void onebit_sparse_set_pad_b(int enabled);
 
 /* Diagnostic: what a prepared call of this shape would launch under the calling thread's hooks. The plan is made for

@@ -449,6 +449,10 @@ int setup_skinny_split(onebit::SkinnyArgs& args, int splits, hipStream_t stream,
   return ONEBIT_OK;
 }
 
+// Least size of a padded-copy buffer: that of any B below the 65536 values from which the plan pads (rows of one column grow
+// eightfold). Growing frees the old buffer, which a graph captured earlier still reads; a small B never makes one grow.
+constexpr size_t kLeastPadBytes = size_t(65536) * 8 * sizeof(_Float16);
+
 // Whether a padded copy of a small B (the plan does not count on one) can be made without failing a call that went through
 // without it: never inside a capture that would have to allocate, and never in a fixed workspace, whose size the plan is
 // checked against.
@@ -460,8 +464,13 @@ bool small_pad_available(size_t bytes, hipStream_t stream, const FixedScratch* f
   Buffer& pb = st.b_pad[stream];
   if (bytes <= pb.bytes) return true;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
-  return grow(&pb.ptr, &pb.bytes, bytes, stream) == ONEBIT_OK;
+  if (hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone &&
+      grow(&pb.ptr, &pb.bytes, std::max(bytes, kLeastPadBytes), stream) == ONEBIT_OK)
+    return true;
+  // the call goes on without the copy: nothing of the attempt may show in it
+  (void)hipGetLastError();
+  g_last_error.clear();
+  return false;
 }
 
 int matmul_prepared_impl(const void* prepared, const void* b, const void* c, void* d, int m, int n, int k, float alpha,
@@ -571,7 +580,7 @@ int matmul_prepared_impl(const void* prepared, const void* b, const void* c, voi
     }
     if (pad_b) {
       Buffer& pb = st.b_pad[stream];
-      if (int rc = grow(&pb.ptr, &pb.bytes, pad_bytes, stream); rc != ONEBIT_OK) return rc;
+      if (int rc = grow(&pb.ptr, &pb.bytes, std::max(pad_bytes, kLeastPadBytes), stream); rc != ONEBIT_OK) return rc;
       args.b_pad = static_cast<_Float16*>(pb.ptr);
     }
     ONEBIT_HIP(launch());

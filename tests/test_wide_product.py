@@ -49,3 +49,29 @@ def test_result_over_c(n, dtype):
     d = c.cuda()
     weight.matmul(b.cuda(), out=d, c=d, alpha=1.0, beta=1.0)
     assert torch.equal(d.cpu(), (dense @ b.double() + c.double()).to(dtype))
+
+
+def test_small_ragged_b_leaves_the_buffer_of_a_captured_graph():
+    """The padded copy of B (576 x 119, the larger in values) is the smaller in bytes: the second call must not replace the
+    buffer that the graph reads."""
+    stream = torch.cuda.Stream()
+    weights = {k: synthetic.make_weight(256, k, k, device="cuda") for k in (576, 992)}
+    prepared = {k: PreparedWeight(*w) for k, w in weights.items()}
+    dense = {k: dequant_desparse_tile(w[0].cpu(), w[1].cpu()).double() for k, w in weights.items()}
+    g = torch.Generator().manual_seed(1)
+    large, small = (torch.randint(-4, 5, shape, generator=g).half() for shape in ((576, 119), (992, 66)))
+    large_gpu, small_gpu = large.cuda(), small.cuda()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        prepared[576].matmul(large_gpu)
+        stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            d = prepared[576].matmul(large_gpu)
+        for _ in range(3):
+            got = prepared[992].matmul(small_gpu)
+            d.zero_()
+            graph.replay()
+            stream.synchronize()
+            assert torch.equal(got.cpu(), (dense[992] @ small.double()).half())
+            assert torch.equal(d.cpu(), (dense[576] @ large.double()).half())
