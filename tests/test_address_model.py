@@ -3,7 +3,7 @@
 The kernels' addresses depend on shapes, launch plan and pointers only, never on operand contents, so their index
 arithmetic can be restated on the CPU (numpy, one array element per lane) and every access asserted to lie inside its
 operand: the prepared weight, B (or its padded copy), C / D, the K-split partial sums. The model follows
-onebitsparsemul_amd/csrc/onebit_kernels.hip statement by statement (prepare_kernel, skinny_kernel with its five
+onebitsparsemul_amd/csrc/ statement by statement (prepare_kernel, skinny_kernel with its five
 B staging modes, gemm_kernel's asynchronous copy pattern and epilogue ranges, splitk_reduce_kernel, pad_b_kernel) and
 takes the launch plan from the library itself (onebit_sparse_describe_launch, host-only). It covers the benchmark
 configurations and the long-K shapes with 33 to 64 columns (8192 x 28672 with n = 40, 48, 64). No GPU is touched.
