@@ -422,8 +422,12 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
     group(std::integral_constant<int, 3>{});
   };
 
-  // sixteen wavefronts leave 128 registers each: no room to hold the next image (32 registers) during the SMFMACs
-  constexpr bool kPrefetchB = NW <= 8;
+  // The next image is requested while this one is multiplied. Sixteen wavefronts have 128 registers each: no room for an image
+  // of 32 registers with wide columns, and with sixteen its requests crowd out the ones for the weights (4096 x 11008 with 16
+  // tokens 8.45 -> 8.9 us, with 7 columns 9.9 -> 10.3). The two requests of the run mode pay (us inside a HIP graph, weights
+  // from HBM): 4096 x 11008 with 2 / 4 columns 9.6 / 7.45 -> 9.35 / 7.35, 5120 x 13824 11.65 / 9.0 -> 11.2 / 8.6, 8192 x 8192
+  // 8.5 / 6.75 -> 8.2 / 6.75, 4096 x 4096 5.3 / 4.5 -> 5.25 / 4.4.
+  constexpr bool kPrefetchB = NW <= 8 || MODE == kSkinnyBRun;
   if (MODE == kSkinnyBRun) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) *reinterpret_cast<u32x4_t*>(region + (lane + i * 64) * 16) = u32x4_t{0, 0, 0, 0};
