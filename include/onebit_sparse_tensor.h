@@ -64,8 +64,9 @@ void onebit_sparse_matmul(void *a, void *b, void *c, void *d, void *e, int m, in
  * captured before a larger call on the same stream must be captured again, and a call that would have to grow a
  * buffer while its stream is being captured is refused): calls on different streams may overlap on the GPU. On the
  * host, a call holds a per-device lock from taking that workspace until both kernels are enqueued, so threads that
- * submit to one GPU through this entry point take turns (a few microseconds each). The prepared form below skips the
- * reorder pass and holds the lock only while it looks up its own buffers.
+ * submit to one GPU through this entry point take turns (a few microseconds each). The prepared forms below skip the
+ * reorder pass. Those of their calls that need a library-owned buffer (K split over workgroups, padded copy of B) hold the
+ * same lock from looking the buffer up until their kernels are enqueued; the others take no lock.
  */
 int onebit_sparse_matmul_ex(const void *a, const void *b, const void *c, void *d, const void *e, int m, int n, int k,
                             float alpha, float beta, int c_dtype, int d_dtype, int meta_layout, void *stream);

@@ -420,9 +420,13 @@ struct FixedScratch {
   size_t bytes;
 };
 
+using DeviceLock = std::unique_lock<std::recursive_mutex>;
+
 // K split of a split-K kernel launch: the split geometry and the partial-sum buffer (the caller's fixed workspace, or
-// the library-owned buffer of this device and stream).
-int setup_skinny_split(onebit::SkinnyArgs& args, int splits, hipStream_t stream, const FixedScratch* fixed) {
+// the library-owned buffer of this device and stream). With the latter `lock` holds the device's lock on return and the caller
+// keeps it until both kernels are enqueued: another thread's call on the stream must not come between them, and must not
+// replace the buffer before they are enqueued.
+int setup_skinny_split(onebit::SkinnyArgs& args, int splits, hipStream_t stream, const FixedScratch* fixed, DeviceLock& lock) {
   args.splits = 1;
   if (splits <= 1) return ONEBIT_OK;
   const int cps = (args.kc_total + splits - 1) / splits;
@@ -442,7 +446,7 @@ int setup_skinny_split(onebit::SkinnyArgs& args, int splits, hipStream_t stream,
   ONEBIT_HIP(hipGetDevice(&device));
   if (device < 0 || device >= kMaxDevices) return fail(ONEBIT_ERR_ARGUMENT, "device ordinal %d not supported", device);
   DeviceState& st = g_dev[device];
-  std::lock_guard<std::recursive_mutex> lock(st.mu);
+  lock = DeviceLock(st.mu);
   Buffer& ws = st.split_ws[stream];
   if (int rc = grow(&ws.ptr, &ws.bytes, bytes, stream); rc != ONEBIT_OK) return rc;
   args.split_ws = static_cast<float*>(ws.ptr);
@@ -501,7 +505,8 @@ int matmul_prepared_impl(const void* prepared, const void* b, const void* c, voi
     args.d_f16 = d_dtype == ONEBIT_DTYPE_F16;
     args.tokens_per_group = wide.tokens;
     args.ldb = n;
-    if (int rc = setup_skinny_split(args, wide.rows ? wide.splits : plan.splits, stream, fixed); rc != ONEBIT_OK) return rc;
+    DeviceLock lock;
+    if (int rc = setup_skinny_split(args, wide.rows ? wide.splits : plan.splits, stream, fixed, lock); rc != ONEBIT_OK) return rc;
     ONEBIT_HIP(wide.rows ? onebit::launch_wide(args, wide.rows, stream) : onebit::launch_skinny(args, plan.rows_or_tile, stream));
     return ONEBIT_OK;
   }
@@ -722,7 +727,8 @@ int onebit_sparse_linear_prepared_typed(const void* prepared, const void* x, con
     args.bias_type = bias_dtype;
     args.bf16 = x_dtype == ONEBIT_DTYPE_BF16;
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    if (int rc = setup_skinny_split(args, linear.wide ? linear.wide_plan.splits : plan.splits, s, nullptr); rc != ONEBIT_OK)
+    DeviceLock lock;
+    if (int rc = setup_skinny_split(args, linear.wide ? linear.wide_plan.splits : plan.splits, s, nullptr, lock); rc != ONEBIT_OK)
       return rc;
     args.tokens_per_group = linear.wide_plan.tokens;
     ONEBIT_HIP(linear.wide ? onebit::launch_wide_tokens(args, linear.wide_plan.rows, s)

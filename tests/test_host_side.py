@@ -1,0 +1,104 @@
+"""The host side of the C ABI (csrc/onebit_capi.hip) without a GPU: the library's object is linked against tests/host/device_stub.cpp,
+which stands in for the HIP runtime and the kernels, and called from Python threads. ctypes releases the interpreter lock, so the
+threads really meet inside the library."""
+import ctypes
+import os
+import subprocess
+import threading
+
+import pytest
+
+from onebitsparsemul_amd import build as native_build
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+vp, i32, f32 = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+KERNELS = ("gemm_kernel", "skinny_kernel", "wide_kernel")
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("host")
+    obj, out = str(folder / "device_stub.o"), str(folder / "libhost.so")
+    subprocess.run([os.path.join(os.path.dirname(native_build.HIPCC), "..", "llvm", "bin", "clang++"), "-O1", "-std=c++17", "-fPIC",
+                    "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I", native_build.CSRC, "-I", native_build.INCLUDE, "-c",
+                    os.path.join(HERE, "host", "device_stub.cpp"), "-o", obj], check=True)
+    # -Bsymbolic: the stand-ins, not the HIP runtime that torch has loaded
+    subprocess.run(["g++", "-shared", "-Wl,-Bsymbolic", "-o", out, obj, "-Wl,-u,onebit_sparse_prepare", native_build.STATIC_LIB,
+                    "-lpthread"], check=True)
+    lib = ctypes.CDLL(out)
+    lib.onebit_sparse_last_error.restype = ctypes.c_char_p
+    lib.stub_violation.restype = ctypes.c_char_p
+    lib.stub_allocated_bytes.restype = ctypes.c_size_t
+    lib.onebit_sparse_matmul_prepared.argtypes = [vp, vp, vp, vp, i32, i32, i32, f32, f32, i32, i32, vp]
+    lib.onebit_sparse_matmul_prepared_static.argtypes = lib.onebit_sparse_matmul_prepared.argtypes
+    lib.onebit_sparse_linear_prepared.argtypes = [vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]
+    lib.onebit_sparse_matmul_ex.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, f32, f32, i32, i32, i32, vp]
+    return lib
+
+
+@pytest.fixture
+def fresh(host):
+    host.onebit_sparse_release_buffers()
+    host.stub_set(0, 0)
+    host.stub_reset()
+    yield host
+    host.stub_set(0, 0)
+    host.onebit_sparse_set_weight_cache(0)
+
+
+def product(lib, m, n, k, b=0x2000):  # addresses that nobody reads
+    return lib.onebit_sparse_matmul_prepared(0x1000, b, None, 0x3000, m, n, k, 1.0, 0.0, 0, 1, None)
+
+
+def layer(lib, m, tokens, k):
+    return lib.onebit_sparse_linear_prepared(0x1000, 0x2000, None, 0x3000, tokens, m, k, 1, 1, None)
+
+
+def one_call(lib, m, n, k, a=0x4000):
+    return lib.onebit_sparse_matmul_ex(a, 0x2000, None, 0x3000, 0x5000, m, n, k, 1.0, 0.0, 0, 0, 0, None)
+
+
+def last_launch(lib):
+    out = (i32 * 5)()
+    lib.stub_last_launch(out)
+    return dict(kernel=KERNELS[out[0]], rows_or_tile=out[1], splits=out[2], padded=bool(out[3]), columns=out[4])
+
+
+def in_threads(*bodies):
+    failed = []
+
+    def run(body):
+        try:
+            body()
+        except BaseException as err:  # noqa: BLE001  (re-raised below)
+            failed.append(err)
+
+    threads = [threading.Thread(target=run, args=(body,)) for body in bodies]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    if failed:
+        raise failed[0]
+
+
+# (call, m, columns or tokens, k) that split K over workgroups: through skinny_kernel, wide_kernel and the main kernel
+SPLIT_CALLS = [(product, 2048, 16, 28672), (product, 2048, 40, 28672), (product, 4096, 256, 11008), (layer, 4096, 16, 16384),
+               (layer, 2048, 48, 28672), (layer, 2048, 128, 28672), (layer, 512, 96, 28672), (layer, 8192, 520, 28672)]
+
+
+@pytest.mark.parametrize("call,m,n,k", SPLIT_CALLS)
+def test_threads_on_one_stream_do_not_meet_in_a_buffer(fresh, call, m, n, k):
+    """Two threads submit split products of growing size to one stream. Each call's two kernels (partial sums, then their sum) are
+    enqueued before another call's, and no call's buffer is replaced between its look-up and its launch."""
+    assert call(fresh, m, n, k) == 0 and last_launch(fresh)["splits"] > 1
+    fresh.onebit_sparse_release_buffers()
+    fresh.stub_set(2000, 0)
+
+    def body(offset):
+        for i in range(6):
+            rows = m // 2 // 64 * 64 + 64 * (2 * i + offset)  # every call needs a larger buffer than the one before
+            assert call(fresh, rows, n, k) == 0, fresh.onebit_sparse_last_error()
+
+    in_threads(lambda: body(0), lambda: body(1))
+    assert fresh.stub_violations() == 0, fresh.stub_violation().decode()
