@@ -868,53 +868,50 @@ int onebit_sparse_matmul_ex(const void* a, const void* b, const void* c, void* d
   DeviceState& ds = g_dev[device];
   void* prep = nullptr;
   const int cache_entries = g_weight_cache_entries.load();
+  // The lock is kept until the call's kernels are enqueued: a call from another thread that evicts this weight, or has to grow
+  // this stream's buffer, frees the memory they read after a device synchronization, which then covers them.
+  std::lock_guard<std::recursive_mutex> lock(ds.mu);
   if (cache_entries > 0) {
-    {  // the lock ends before the multiplication is launched, which may take it again for its own buffers
-      std::lock_guard<std::recursive_mutex> lock(ds.mu);
-      for (auto& w : ds.weight_cache)
-        if (w.a == a && w.e == e && w.m == m && w.k == k && w.layout == meta_layout) {
-          w.last_use = ++ds.use_counter;
-          if (w.stream != s) ONEBIT_HIP(hipStreamWaitEvent(s, w.ready, 0));  // its reorder kernel ran on another stream
-          prep = w.prep;
-          break;
-        }
-      if (!prep) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        ONEBIT_HIP(hipStreamIsCapturing(s, &capture));
-        if (capture != hipStreamCaptureStatusNone)
-          return fail(ONEBIT_ERR_ARGUMENT, "a weight that is not in the cache yet cannot be added while the stream is "
-                                           "being captured: run the call once outside the capture first");
-        if ((int)ds.weight_cache.size() >= cache_entries) {  // evict the least recently used entry
-          size_t victim = 0;
-          for (size_t i = 1; i < ds.weight_cache.size(); ++i)
-            if (ds.weight_cache[i].last_use < ds.weight_cache[victim].last_use) victim = i;
-          ONEBIT_HIP(hipDeviceSynchronize());  // earlier work on any stream may still read it
-          ONEBIT_HIP(hipFree(ds.weight_cache[victim].prep));
-          ONEBIT_HIP(hipEventDestroy(ds.weight_cache[victim].ready));
-          ds.weight_cache.erase(ds.weight_cache.begin() + victim);
-        }
-        DeviceState::CachedWeight w{a, e, m, k, meta_layout, nullptr, s, nullptr, ++ds.use_counter};
-        ONEBIT_HIP(hipMalloc(&w.prep, onebit::prepared_bytes(m, k)));
-        if (hipError_t st = hipEventCreateWithFlags(&w.ready, hipEventDisableTiming); st != hipSuccess) {
-          (void)hipFree(w.prep);
-          return fail(ONEBIT_ERR_HIP, "HIP error '%s' from hipEventCreateWithFlags", hipGetErrorString(st));
-        }
-        hipError_t st = onebit::launch_prepare(a, e, w.prep, m, k, meta_layout, s);
-        if (st == hipSuccess) st = hipEventRecord(w.ready, s);
-        if (st != hipSuccess) {
-          (void)hipFree(w.prep);
-          (void)hipEventDestroy(w.ready);
-          return fail(ONEBIT_ERR_HIP, "HIP error '%s' while reordering a cached weight", hipGetErrorString(st));
-        }
-        ds.weight_cache.push_back(w);
+    for (auto& w : ds.weight_cache)
+      if (w.a == a && w.e == e && w.m == m && w.k == k && w.layout == meta_layout) {
+        w.last_use = ++ds.use_counter;
+        if (w.stream != s) ONEBIT_HIP(hipStreamWaitEvent(s, w.ready, 0));  // its reorder kernel ran on another stream
         prep = w.prep;
+        break;
       }
+    if (!prep) {
+      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+      ONEBIT_HIP(hipStreamIsCapturing(s, &capture));
+      if (capture != hipStreamCaptureStatusNone)
+        return fail(ONEBIT_ERR_ARGUMENT, "a weight that is not in the cache yet cannot be added while the stream is "
+                                         "being captured: run the call once outside the capture first");
+      if ((int)ds.weight_cache.size() >= cache_entries) {  // evict the least recently used entry
+        size_t victim = 0;
+        for (size_t i = 1; i < ds.weight_cache.size(); ++i)
+          if (ds.weight_cache[i].last_use < ds.weight_cache[victim].last_use) victim = i;
+        ONEBIT_HIP(hipDeviceSynchronize());  // earlier work on any stream may still read it
+        ONEBIT_HIP(hipFree(ds.weight_cache[victim].prep));
+        ONEBIT_HIP(hipEventDestroy(ds.weight_cache[victim].ready));
+        ds.weight_cache.erase(ds.weight_cache.begin() + victim);
+      }
+      DeviceState::CachedWeight w{a, e, m, k, meta_layout, nullptr, s, nullptr, ++ds.use_counter};
+      ONEBIT_HIP(hipMalloc(&w.prep, onebit::prepared_bytes(m, k)));
+      if (hipError_t st = hipEventCreateWithFlags(&w.ready, hipEventDisableTiming); st != hipSuccess) {
+        (void)hipFree(w.prep);
+        return fail(ONEBIT_ERR_HIP, "HIP error '%s' from hipEventCreateWithFlags", hipGetErrorString(st));
+      }
+      hipError_t st = onebit::launch_prepare(a, e, w.prep, m, k, meta_layout, s);
+      if (st == hipSuccess) st = hipEventRecord(w.ready, s);
+      if (st != hipSuccess) {
+        (void)hipFree(w.prep);
+        (void)hipEventDestroy(w.ready);
+        return fail(ONEBIT_ERR_HIP, "HIP error '%s' while reordering a cached weight", hipGetErrorString(st));
+      }
+      ds.weight_cache.push_back(w);
+      prep = w.prep;
     }
     return matmul_prepared_impl(prep, b, c, d, m, n, k, alpha, beta, c_dtype, d_dtype, s);
   }
-  // the lock is kept until both kernels are enqueued: a call from another thread that has to grow this stream's
-  // buffer (which frees the old one) then waits, and its device synchronization covers the work enqueued here
-  std::lock_guard<std::recursive_mutex> lock(ds.mu);
   Buffer& own = ds.prep[s];
   if (int rc = grow(&own.ptr, &own.bytes, onebit::prepared_bytes(m, k), s)) return rc;
   prep = own.ptr;

@@ -102,3 +102,16 @@ def test_threads_on_one_stream_do_not_meet_in_a_buffer(fresh, call, m, n, k):
 
     in_threads(lambda: body(0), lambda: body(1))
     assert fresh.stub_violations() == 0, fresh.stub_violation().decode()
+
+
+def test_cached_weight_is_not_evicted_between_look_up_and_launch(fresh):
+    """A cache of one entry and two threads with a weight each: every call evicts the other thread's copy."""
+    assert fresh.onebit_sparse_set_weight_cache(1) == 0
+    fresh.stub_set(2000, 0)
+
+    def body(a):
+        for _ in range(6):
+            assert one_call(fresh, 512, 16, 512, a=a) == 0, fresh.onebit_sparse_last_error()
+
+    in_threads(lambda: body(0x4000), lambda: body(0x6000))
+    assert fresh.stub_violations() == 0, fresh.stub_violation().decode()
