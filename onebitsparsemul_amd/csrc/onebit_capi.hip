@@ -93,15 +93,18 @@ DeviceState g_dev[kMaxDevices];
 // Grows a library-owned buffer. Growing frees the old memory after a device synchronization: a HIP graph captured
 // earlier on this stream still holds the old address and must be captured again after a larger call. Inside a stream
 // capture neither the synchronization nor the allocation is possible, so a call that would have to grow there is
-// refused instead of invalidating the capture.
-int grow(void** ptr, size_t* have, size_t need, hipStream_t stream) {
-  if (need <= *have) return ONEBIT_OK;
+// refused instead of invalidating the capture. `reserve`: size to grow to, at least `need`, where that is possible.
+int grow(void** ptr, size_t* have, size_t need, hipStream_t stream, size_t reserve = 0) {
+  reserve = std::max(need, reserve);
+  if (reserve <= *have) return ONEBIT_OK;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   ONEBIT_HIP(hipStreamIsCapturing(stream, &capture));
-  if (capture != hipStreamCaptureStatusNone)
+  if (capture != hipStreamCaptureStatusNone) {
+    if (need <= *have) return ONEBIT_OK;
     return fail(ONEBIT_ERR_ARGUMENT,
                 "a library-owned buffer would have to grow to %zu bytes while the stream is being captured: run the "
                 "call once outside the capture first, or use the non-allocating entry point", need);
+  }
   if (*ptr) {
     // earlier work on any stream may still read the old buffer
     ONEBIT_HIP(hipDeviceSynchronize());
@@ -109,7 +112,7 @@ int grow(void** ptr, size_t* have, size_t need, hipStream_t stream) {
     *ptr = nullptr;
     *have = 0;
   }
-  const size_t bytes = (need + 4095) & ~size_t(4095);
+  const size_t bytes = (reserve + 4095) & ~size_t(4095);
   ONEBIT_HIP(hipMalloc(ptr, bytes));
   *have = bytes;
   return ONEBIT_OK;
@@ -380,8 +383,9 @@ LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int comput
 
 // The linear layer's plan: wide = wide_kernel with `wide_plan`, else `launch` as for a product with an aligned B.
 // Up to sixteen tokens the split-K kernel; beyond 64 whichever of wide_kernel and the main kernel is modelled faster
-// (the main kernel's model is up to 12 % above its measured times where the two meet). A layer call may split K, i.e. needs
-// a buffer, only where the other kernel's plan would: what can be captured without a warm-up stays so.
+// (the main kernel's model is up to 12 % above its measured times where the two meet). A layer call splits K into no more parts
+// than the other kernel's plan would and uses the same buffer, so a call needs no more memory than it would there, and what can
+// be captured without a warm-up stays so.
 struct LinearPlan {
   bool wide;
   WidePlan wide_plan;
@@ -394,8 +398,7 @@ LinearPlan plan_linear(int m, int tokens, int k, int compute_units) {
   const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
   const bool beyond = tokens > onebit::kSkinnyMaxN;
   if (beyond && (g_tile_config >= 0 || groups[2] * ((tokens + 63) / 64) > 2L * compute_units)) return plan;
-  const int most_splits = g_split_k >= 1 ? g_split_k : plan.launch.splits > 1 ? 8 : 1;
-  plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, false, 1, most_splits, compute_units);
+  plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, false, 1, plan.launch.splits, compute_units);
   plan.wide = !beyond || plan.wide_plan.us < 0.88 * plan.launch.model_us;
   return plan;
 }
@@ -420,20 +423,29 @@ struct FixedScratch {
   size_t bytes;
 };
 
+// Splits that a plan's `splits` come to: none of them empty.
+int full_splits(int chunks, int splits) {
+  const int per_split = (chunks + splits - 1) / splits;
+  return (chunks + per_split - 1) / per_split;
+}
+
 using DeviceLock = std::unique_lock<std::recursive_mutex>;
 
 // K split of a split-K kernel launch: the split geometry and the partial-sum buffer (the caller's fixed workspace, or
 // the library-owned buffer of this device and stream). With the latter `lock` holds the device's lock on return and the caller
 // keeps it until both kernels are enqueued: another thread's call on the stream must not come between them, and must not
 // replace the buffer before they are enqueued.
-int setup_skinny_split(onebit::SkinnyArgs& args, int splits, hipStream_t stream, const FixedScratch* fixed, DeviceLock& lock) {
+// most_splits: of the plan that wide_kernel's replaces, at least `splits`. The buffer is made large enough for that many: how
+// far wide_kernel splits changes from one column count to the next in both directions, so a call of fewer columns would
+// otherwise replace a buffer that a graph captured with more of them still reads.
+int setup_skinny_split(onebit::SkinnyArgs& args, int splits, int most_splits, hipStream_t stream, const FixedScratch* fixed,
+                       DeviceLock& lock) {
   args.splits = 1;
   if (splits <= 1) return ONEBIT_OK;
-  const int cps = (args.kc_total + splits - 1) / splits;
-  args.chunks_per_split = cps;
-  args.splits = (args.kc_total + cps - 1) / cps;  // every split non-empty
+  args.chunks_per_split = (args.kc_total + splits - 1) / splits;
+  args.splits = full_splits(args.kc_total, splits);
   if (args.splits <= 1) return ONEBIT_OK;
-  const size_t bytes = (size_t)args.splits * args.m * args.n * sizeof(float);
+  const size_t split_bytes = (size_t)args.m * args.n * sizeof(float), bytes = args.splits * split_bytes;
   if (fixed) {
     if (bytes > fixed->bytes)
       return fail(ONEBIT_ERR_ARGUMENT,
@@ -448,7 +460,8 @@ int setup_skinny_split(onebit::SkinnyArgs& args, int splits, hipStream_t stream,
   DeviceState& st = g_dev[device];
   lock = DeviceLock(st.mu);
   Buffer& ws = st.split_ws[stream];
-  if (int rc = grow(&ws.ptr, &ws.bytes, bytes, stream); rc != ONEBIT_OK) return rc;
+  if (int rc = grow(&ws.ptr, &ws.bytes, bytes, stream, full_splits(args.kc_total, most_splits) * split_bytes); rc != ONEBIT_OK)
+    return rc;
   args.split_ws = static_cast<float*>(ws.ptr);
   return ONEBIT_OK;
 }
@@ -506,7 +519,8 @@ int matmul_prepared_impl(const void* prepared, const void* b, const void* c, voi
     args.tokens_per_group = wide.tokens;
     args.ldb = n;
     DeviceLock lock;
-    if (int rc = setup_skinny_split(args, wide.rows ? wide.splits : plan.splits, stream, fixed, lock); rc != ONEBIT_OK) return rc;
+    if (int rc = setup_skinny_split(args, wide.rows ? wide.splits : plan.splits, plan.splits, stream, fixed, lock); rc != ONEBIT_OK)
+      return rc;
     ONEBIT_HIP(wide.rows ? onebit::launch_wide(args, wide.rows, stream) : onebit::launch_skinny(args, plan.rows_or_tile, stream));
     return ONEBIT_OK;
   }
@@ -552,12 +566,12 @@ int matmul_prepared_impl(const void* prepared, const void* b, const void* c, voi
     return onebit::launch_wide(w, wide.rows, stream);
   };
   if (splits > 1 || pad_b) {
-    size_t split_bytes = 0;
+    size_t split_bytes = 0, most_bytes = 0;
     if (splits > 1) {
-      const int cps = (kc_total + splits - 1) / splits;
-      args.chunks_per_split = cps;
-      args.splits = (kc_total + cps - 1) / cps;  // every split non-empty
+      args.chunks_per_split = (kc_total + splits - 1) / splits;
+      args.splits = full_splits(kc_total, splits);
       split_bytes = (size_t)args.splits * m * n * sizeof(float);
+      most_bytes = (size_t)full_splits(kc_total, plan.splits) * m * n * sizeof(float);  // see setup_skinny_split
     }
     if (fixed) {
       // partial sums first, the padded copy of B behind them on the next 256-byte boundary; both are written in
@@ -580,7 +594,7 @@ int matmul_prepared_impl(const void* prepared, const void* b, const void* c, voi
     std::lock_guard<std::recursive_mutex> lock(st.mu);
     if (splits > 1) {
       Buffer& ws = st.split_ws[stream];
-      if (int rc = grow(&ws.ptr, &ws.bytes, split_bytes, stream); rc != ONEBIT_OK) return rc;
+      if (int rc = grow(&ws.ptr, &ws.bytes, split_bytes, stream, most_bytes); rc != ONEBIT_OK) return rc;
       args.split_ws = static_cast<float*>(ws.ptr);
     }
     if (pad_b) {
@@ -728,7 +742,8 @@ int onebit_sparse_linear_prepared_typed(const void* prepared, const void* x, con
     args.bf16 = x_dtype == ONEBIT_DTYPE_BF16;
     const hipStream_t s = static_cast<hipStream_t>(stream);
     DeviceLock lock;
-    if (int rc = setup_skinny_split(args, linear.wide ? linear.wide_plan.splits : plan.splits, s, nullptr, lock); rc != ONEBIT_OK)
+    if (int rc = setup_skinny_split(args, linear.wide ? linear.wide_plan.splits : plan.splits, plan.splits, s, nullptr, lock);
+        rc != ONEBIT_OK)
       return rc;
     args.tokens_per_group = linear.wide_plan.tokens;
     ONEBIT_HIP(linear.wide ? onebit::launch_wide_tokens(args, linear.wide_plan.rows, s)
@@ -764,9 +779,8 @@ int onebit_sparse_linear_prepared_typed(const void* prepared, const void* x, con
     if (device < 0 || device >= kMaxDevices) return fail(ONEBIT_ERR_ARGUMENT, "device ordinal %d not supported", device);
     DeviceState& st = g_dev[device];
     std::lock_guard<std::recursive_mutex> lock(st.mu);
-    const int cps = (kc_total + plan.splits - 1) / plan.splits;
-    args.chunks_per_split = cps;
-    args.splits = (kc_total + cps - 1) / cps;  // every split non-empty
+    args.chunks_per_split = (kc_total + plan.splits - 1) / plan.splits;
+    args.splits = full_splits(kc_total, plan.splits);
     Buffer& ws = st.split_ws[s];
     if (int rc = grow(&ws.ptr, &ws.bytes, (size_t)args.splits * m * tokens * sizeof(float), s); rc != ONEBIT_OK) return rc;
     args.split_ws = static_cast<float*>(ws.ptr);

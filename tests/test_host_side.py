@@ -115,3 +115,14 @@ def test_cached_weight_is_not_evicted_between_look_up_and_launch(fresh):
 
     in_threads(lambda: body(0x4000), lambda: body(0x6000))
     assert fresh.stub_violations() == 0, fresh.stub_violation().decode()
+
+
+@pytest.mark.parametrize("call,m,k", [(layer, 2048, 28672), (layer, 512, 28672), (layer, 1024, 20480), (product, 2048, 28672),
+                                      (product, 512, 16384)])
+def test_fewer_columns_never_replace_the_partial_sum_buffer(fresh, call, m, k):
+    """From 64 columns or tokens down, the range where the split does not depend on them but through wide_kernel's own plan: a
+    graph captured with more columns keeps its buffer, and a call with fewer can be captured after it without a warm-up."""
+    assert call(fresh, m, 64, k) == 0 and last_launch(fresh)["splits"] > 1
+    fresh.stub_set(0, 1)
+    for n in range(63, 16, -1):
+        assert call(fresh, m, n, k) == 0, (n, fresh.onebit_sparse_last_error())
