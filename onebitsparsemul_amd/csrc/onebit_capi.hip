@@ -329,6 +329,11 @@ WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, 
   // plain form, several column groups: a group's piece of a row of B is a part of a line, 32 to 128 bytes (4096 x 64 x 4096 in
   // four groups 11.0 us against 5.8 token-major, in two 7.1 against 5.1)
   static const double kColumns[4] = {2.3, 1.45, 1.4, 1.1};
+  // The row groups that multiply one token group run on different XCDs, and each XCD fetches its own copy of x: with more x
+  // than fits an XCD's L2 (4 MB) that is what a launch of few rows waits for (us measured | modelled without it:
+  // 896 x 24256 x 704 45 | 29, 1088 x 13888 x 1758 62 | 38, 640 x 17536 x 676 30 | 19; the main kernel takes 29, 41 and 21).
+  constexpr double kFetchBytesPerUs = 6.3e6;
+  const double xcds = std::max(1, compute_units / 32);
   const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
   WidePlan best{g_skinny_rows > 0 ? g_skinny_rows : 32, 1, std::min(n, onebit::kSkinnyMaxN), 1e30};
   for (int width = 1; width <= 4; ++width) {
@@ -348,6 +353,7 @@ WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, 
         double us = kBase[r][tiles - 1] + work;
         if (load > 1.0)
           us += (std::ceil(load) - 1.0) * (work * kAgain[r][tiles - 1] + (kBase[r][tiles - 1] - 1.5) * (r < 2 ? 0.4 : 1.0));
+        us = std::max(us, 3.5 + std::min((double)total_groups[r], xcds) * n * k * 2.0 / kFetchBytesPerUs);
         if (s > 1) us += 2.6 + 0.15 * s + (s + 1) * 4.0 * results / 5.0e6;
         if (us < best.us) best = WidePlan{kWideRows[r], s, tokens, us};
         if (g_split_k >= 1 || s == most_splits) break;
@@ -381,9 +387,15 @@ LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int comput
   return plan;
 }
 
+// wide_kernel against the main kernel. Both models err, the main kernel's mostly upwards (by half at worst), so the line lies
+// where calls that cross it are not slower. Measured on 260 layer calls and 188 products of 512 to 65536 rows, k = 512 to 28672
+// and 65 to 2048 columns whose two models lie within a factor of two: the 213 below 0.81 are 1.53 times as fast as on the main
+// kernel in the mean and the slowest within 2 %; of the 56 between 0.81 and 0.88 ten are slower, by up to 21 % (2496 x 19648 with
+// 197 tokens; 20864 x 7616 with 152 columns, at 0.82, 52 us against 48).
+bool wide_is_faster(const WidePlan& wide, const LaunchPlan& launch) { return wide.us < 0.81 * launch.model_us; }
+
 // The linear layer's plan: wide = wide_kernel with `wide_plan`, else `launch` as for a product with an aligned B.
-// Up to sixteen tokens the split-K kernel; beyond 64 whichever of wide_kernel and the main kernel is modelled faster
-// (the main kernel's model is up to 12 % above its measured times where the two meet). A layer call splits K into no more parts
+// Up to sixteen tokens the split-K kernel; beyond 64 wide_kernel where it is faster than the main kernel. A layer call splits K into no more parts
 // than the other kernel's plan would and uses the same buffer, so a call needs no more memory than it would there, and what can
 // be captured without a warm-up stays so.
 struct LinearPlan {
@@ -399,7 +411,7 @@ LinearPlan plan_linear(int m, int tokens, int k, int compute_units) {
   const bool beyond = tokens > onebit::kSkinnyMaxN;
   if (beyond && (g_tile_config >= 0 || groups[2] * ((tokens + 63) / 64) > 2L * compute_units)) return plan;
   plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, false, 1, plan.launch.splits, compute_units);
-  plan.wide = !beyond || plan.wide_plan.us < 0.88 * plan.launch.model_us;
+  plan.wide = !beyond || wide_is_faster(plan.wide_plan, plan.launch);
   return plan;
 }
 
@@ -412,7 +424,7 @@ WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b
   if (n <= 16 || !g_skinny_enabled || g_tile_config >= 0 || groups[2] * ((n + 63) / 64) > 2L * compute_units) return none;
   if (!b_readable) return none;
   const WidePlan plan = plan_wide(groups, (double)m * n, n, k, true, launch.splits > 1 ? 2 : 1, launch.splits, compute_units);
-  if (plan.us == 1e30 || (!launch.split_k_kernel && plan.us >= 0.85 * launch.model_us)) return none;
+  if (plan.us == 1e30 || (!launch.split_k_kernel && !wide_is_faster(plan, launch))) return none;
   return plan;
 }
 

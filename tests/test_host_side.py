@@ -126,3 +126,20 @@ def test_fewer_columns_never_replace_the_partial_sum_buffer(fresh, call, m, k):
     fresh.stub_set(0, 1)
     for n in range(63, 16, -1):
         assert call(fresh, m, n, k) == 0, (n, fresh.onebit_sparse_last_error())
+
+
+@pytest.mark.parametrize("call,m,n,k", [(layer, 896, 704, 24256), (layer, 1088, 1758, 13888), (layer, 704, 1920, 14816),
+                                        (layer, 640, 676, 17536), (layer, 1088, 1694, 5696), (layer, 1344, 969, 9216),
+                                        (layer, 2496, 197, 19648), (product, 20864, 152, 7616), (product, 768, 616, 8192)])
+def test_calls_that_the_main_kernel_multiplies_faster(fresh, call, m, n, k):
+    """Few rows that read a large x, and shapes where the two kernels' models are near each other: 5 to 57 % slower through
+    wide_kernel."""
+    assert call(fresh, m, n, k) == 0
+    assert last_launch(fresh)["kernel"] == "gemm_kernel"
+
+
+@pytest.mark.parametrize("call,m,n,k", [(layer, 4096, 500, 11008), (layer, 5312, 278, 18944), (layer, 1024, 256, 4096),
+                                        (layer, 4096, 128, 4096), (product, 4096, 256, 4096)])
+def test_calls_that_wide_kernel_multiplies_faster(fresh, call, m, n, k):
+    assert call(fresh, m, n, k) == 0
+    assert last_launch(fresh)["kernel"] == "wide_kernel"
