@@ -392,12 +392,21 @@ LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int comput
 // and 65 to 2048 columns whose two models lie within a factor of two: the 213 below 0.81 are 1.53 times as fast as on the main
 // kernel in the mean and the slowest within 2 %; of the 56 between 0.81 and 0.88 ten are slower, by up to 21 % (2496 x 19648 with
 // 197 tokens; 20864 x 7616 with 152 columns, at 0.82, 52 us against 48).
-bool wide_is_faster(const WidePlan& wide, const LaunchPlan& launch) { return wide.us < 0.81 * launch.model_us; }
+// Up to 64 columns the main kernel is the other plan beyond 40960 rows only, where a wavefront of wide_kernel has one short round
+// of work per workgroup and the workgroups come in many rounds, outside what its model was fitted to: the line is the length of
+// K, from which on wide_kernel is faster at 45056 to 262144 rows (us, wide | main, 48 and 64 tokens: 65536 x 1024 17.0 | 12.0 and
+// 19.0 | 12.4, x 4096 28.5 | 31.4 and 32.8 | 31.8, x 8192 44.1 | 60.2 and 50.1 | 60.5; 45056 x 3616 25.4 | 23.9, x 4096
+// 23.5 | 25.1). With k % 64 != 0, where every second token's pieces straddle two lines, it lies twice as far out (45056 x 4128
+// with 48 tokens 28.6 | 26.8, x 8224 43.4 | 47.9).
+bool wide_is_faster(const WidePlan& wide, const LaunchPlan& launch, int n, int k) {
+  if (n <= onebit::kSkinnyMaxN) return (k + onebit::kChunkK - 1) / onebit::kChunkK >= (n <= 48 ? 16 : 32) * (k % 64 ? 2 : 1);
+  return wide.us < 0.81 * launch.model_us;
+}
 
 // The linear layer's plan: wide = wide_kernel with `wide_plan`, else `launch` as for a product with an aligned B.
-// Up to sixteen tokens the split-K kernel; beyond 64 wide_kernel where it is faster than the main kernel. A layer call splits K into no more parts
-// than the other kernel's plan would and uses the same buffer, so a call needs no more memory than it would there, and what can
-// be captured without a warm-up stays so.
+// Up to sixteen tokens the split-K kernel; beyond, wide_kernel in that kernel's place and where it is faster than the main
+// kernel. A layer call splits K into no more parts than the other kernel's plan would and uses the same buffer, so a call needs
+// no more memory than it would there, and what can be captured without a warm-up stays so.
 struct LinearPlan {
   bool wide;
   WidePlan wide_plan;
@@ -408,10 +417,10 @@ LinearPlan plan_linear(int m, int tokens, int k, int compute_units) {
   plan.launch = choose_launch(m, tokens, k, true, compute_units);
   if (tokens <= onebit::kSkinnyTokens || !g_skinny_enabled) return plan;
   const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
-  const bool beyond = tokens > onebit::kSkinnyMaxN;
-  if (beyond && (g_tile_config >= 0 || groups[2] * ((tokens + 63) / 64) > 2L * compute_units)) return plan;
+  if (!plan.launch.split_k_kernel && g_tile_config >= 0) return plan;
+  if (tokens > onebit::kSkinnyMaxN && groups[2] * ((tokens + 63) / 64) > 2L * compute_units) return plan;
   plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, false, 1, plan.launch.splits, compute_units);
-  plan.wide = !beyond || wide_is_faster(plan.wide_plan, plan.launch);
+  plan.wide = plan.launch.split_k_kernel || wide_is_faster(plan.wide_plan, plan.launch, tokens, k);
   return plan;
 }
 
@@ -424,7 +433,7 @@ WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b
   if (n <= 16 || !g_skinny_enabled || g_tile_config >= 0 || groups[2] * ((n + 63) / 64) > 2L * compute_units) return none;
   if (!b_readable) return none;
   const WidePlan plan = plan_wide(groups, (double)m * n, n, k, true, launch.splits > 1 ? 2 : 1, launch.splits, compute_units);
-  if (plan.us == 1e30 || (!launch.split_k_kernel && !wide_is_faster(plan, launch))) return none;
+  if (plan.us == 1e30 || (!launch.split_k_kernel && !wide_is_faster(plan, launch, n, k))) return none;
   return plan;
 }
 

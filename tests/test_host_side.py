@@ -130,16 +130,19 @@ def test_fewer_columns_never_replace_the_partial_sum_buffer(fresh, call, m, k):
 
 @pytest.mark.parametrize("call,m,n,k", [(layer, 896, 704, 24256), (layer, 1088, 1758, 13888), (layer, 704, 1920, 14816),
                                         (layer, 640, 676, 17536), (layer, 1088, 1694, 5696), (layer, 1344, 969, 9216),
-                                        (layer, 2496, 197, 19648), (product, 20864, 152, 7616), (product, 768, 616, 8192)])
+                                        (layer, 2496, 197, 19648), (product, 20864, 152, 7616), (product, 768, 616, 8192),
+                                        (layer, 49152, 33, 1024), (layer, 131072, 64, 1024), (layer, 131072, 56, 2048),
+                                        (layer, 45056, 64, 4096), (layer, 45056, 48, 3616), (layer, 45056, 48, 4128)])
 def test_calls_that_the_main_kernel_multiplies_faster(fresh, call, m, n, k):
-    """Few rows that read a large x, and shapes where the two kernels' models are near each other: 5 to 57 % slower through
-    wide_kernel."""
+    """Few rows that read a large x, shapes where the two kernels' models are near each other, very many rows of short K: 3 to
+    90 % slower through wide_kernel."""
     assert call(fresh, m, n, k) == 0
     assert last_launch(fresh)["kernel"] == "gemm_kernel"
 
 
 @pytest.mark.parametrize("call,m,n,k", [(layer, 4096, 500, 11008), (layer, 5312, 278, 18944), (layer, 1024, 256, 4096),
-                                        (layer, 4096, 128, 4096), (product, 4096, 256, 4096)])
+                                        (layer, 4096, 128, 4096), (product, 4096, 256, 4096), (layer, 131072, 48, 4096),
+                                        (layer, 65536, 64, 8192), (layer, 40960, 64, 512)])
 def test_calls_that_wide_kernel_multiplies_faster(fresh, call, m, n, k):
     assert call(fresh, m, n, k) == 0
     assert last_launch(fresh)["kernel"] == "wide_kernel"
