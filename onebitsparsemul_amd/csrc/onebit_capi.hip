@@ -318,8 +318,8 @@ struct WidePlan {
   int rows, splits, tokens;
   double us;
 };
-WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, bool plain, int least_splits,
-                   int most_splits, int compute_units) {
+WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, bool plain, int most_splits,
+                   int compute_units) {
   // [row group][column tiles - 1]
   static const double kBase[3][4] = {{2.75, 2.9, 2.9, 3.0}, {3.1, 3.3, 3.4, 3.6}, {3.7, 4.3, 5.8, 6.4}};
   static const double kRound[3][4] = {{0.74, 0.93, 1.48, 1.89}, {1.01, 1.26, 1.74, 2.24}, {1.88, 2.4, 2.75, 3.25}};
@@ -345,7 +345,6 @@ WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, 
       for (int s : {1, 2, 3, 4, 6, 8}) {
         if (g_split_k >= 1) s = g_split_k;
         s = std::min(std::min(s, most_splits), chunks);
-        if (s < least_splits) continue;
         const int rounds = ((chunks + s - 1) / s + 7) / 8;
         const double load = (double)total_groups[r] * groups * s / compute_units;
         const double work = rounds * kRound[r][tiles - 1] * (1.0 + kLoad[r][tiles - 1] * std::min(1.0, load)) *
@@ -419,20 +418,22 @@ LinearPlan plan_linear(int m, int tokens, int k, int compute_units) {
   const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
   if (!plan.launch.split_k_kernel && g_tile_config >= 0) return plan;
   if (tokens > onebit::kSkinnyMaxN && groups[2] * ((tokens + 63) / 64) > 2L * compute_units) return plan;
-  plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, false, 1, plan.launch.splits, compute_units);
+  plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, false, plan.launch.splits, compute_units);
   plan.wide = plan.launch.split_k_kernel || wide_is_faster(plan.wide_plan, plan.launch, tokens, k);
   return plan;
 }
 
-// The product's: wide_kernel in the place of `launch` where that reads B in place or through its padded copy, for 17 columns
-// or more and where it is modelled faster. It splits K where `launch` does, into no more parts, and uses the same buffers, so
-// what a call needs, and whether it can be captured, does not depend on the choice.
+// The product's: wide_kernel in the place of `launch` for 17 columns or more where that reads B in place or through its padded
+// copy: always in the place of the split-K kernel, and where it is faster than the main kernel. It splits K into no more parts
+// than `launch` and uses the same buffers, so a call needs no memory that it would not need there, and what can be captured
+// without a warm-up stays so. It may split into fewer or not at all: a split pays a second launch and fp32 sums through memory
+// (us, split in two -> unsplit: 1024 x 128 x 2048 6.1 -> 3.8, 4096 x 96 x 4096 10.8 -> 7.2, 5120 x 128 x 8192 20.0 -> 13.3).
 WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b_readable, int compute_units) {
   WidePlan none{0, 1, 0, 0.0};
   const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
   if (n <= 16 || !g_skinny_enabled || g_tile_config >= 0 || groups[2] * ((n + 63) / 64) > 2L * compute_units) return none;
   if (!b_readable) return none;
-  const WidePlan plan = plan_wide(groups, (double)m * n, n, k, true, launch.splits > 1 ? 2 : 1, launch.splits, compute_units);
+  const WidePlan plan = plan_wide(groups, (double)m * n, n, k, true, launch.splits, compute_units);
   if (plan.us == 1e30 || (!launch.split_k_kernel && !wide_is_faster(plan, launch, n, k))) return none;
   return plan;
 }
@@ -859,7 +860,7 @@ int onebit_sparse_linear_prepared_grouped_typed(const onebit_linear_problem* pro
     }
     const int enough = std::max(1, 160 * compute_units / 256);
     WidePlan wide_plan{};
-    if (wide) wide_plan = plan_wide(groups, 0.0, tokens, longest_k, false, 1, 1, compute_units);
+    if (wide) wide_plan = plan_wide(groups, 0.0, tokens, longest_k, false, 1, compute_units);
     const int rows = wide ? wide_plan.rows
                      : g_skinny_rows > 0 ? g_skinny_rows
                      : (rows_total / 128 >= enough) ? 128 : (rows_total / 64 >= enough) ? 64 : 32;

@@ -146,3 +146,11 @@ def test_calls_that_the_main_kernel_multiplies_faster(fresh, call, m, n, k):
 def test_calls_that_wide_kernel_multiplies_faster(fresh, call, m, n, k):
     assert call(fresh, m, n, k) == 0
     assert last_launch(fresh)["kernel"] == "wide_kernel"
+
+
+@pytest.mark.parametrize("m,n,k", [(1024, 128, 2048), (4096, 96, 4096), (2048, 160, 4096), (5120, 128, 8192), (4096, 32, 11008)])
+def test_product_is_not_split_because_the_plan_it_replaces_is(fresh, m, n, k):
+    """Slower by up to a half when split in two only because the main kernel's or skinny_kernel's plan would split."""
+    fresh.stub_set(0, 1)
+    assert product(fresh, m, n, k) == 0, fresh.onebit_sparse_last_error()
+    assert last_launch(fresh)["kernel"] == "wide_kernel" and last_launch(fresh)["splits"] == 1
