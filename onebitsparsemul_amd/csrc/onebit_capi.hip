@@ -424,13 +424,20 @@ LinearPlan plan_linear(int m, int tokens, int k, int compute_units) {
 }
 
 // The product's: wide_kernel in the place of `launch` for 17 columns or more where that reads B in place or through its padded
-// copy: always in the place of the split-K kernel, and where it is faster than the main kernel. It splits K into no more parts
-// than `launch` and uses the same buffers, so a call needs no memory that it would not need there, and what can be captured
-// without a warm-up stays so. It may split into fewer or not at all: a split pays a second launch and fp32 sums through memory
-// (us, split in two -> unsplit: 1024 x 128 x 2048 6.1 -> 3.8, 4096 x 96 x 4096 10.8 -> 7.2, 5120 x 128 x 8192 20.0 -> 13.3).
+// copy: in the place of the split-K kernel, but for some of 32 columns, and where it is faster than the main kernel. It splits K
+// into no more parts than `launch` and uses the same buffers, so a call needs no memory that it would not need there, and what
+// can be captured without a warm-up stays so. It may split into fewer or not at all: a split pays a second launch and fp32 sums
+// through memory (us, split in two -> unsplit: 1024 x 128 x 2048 6.1 -> 3.8, 4096 x 96 x 4096 10.8 -> 7.2, 5120 x 128 x 8192
+// 20.0 -> 13.3).
 WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b_readable, int compute_units) {
   WidePlan none{0, 1, 0, 0.0};
   const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
+  // 32 columns, whole rows of an image: skinny_kernel is as fast or faster in one round of 128-row groups, and where K is so short
+  // that its chunks do not fill a round of the sixteen wavefronts of its 32-row groups (us, skinny_kernel | wide_kernel:
+  // 20480 x 4096 10.4 | 11.2, 28672 x 5536 14.2 | 15.0, 2048 x 1056 3.71 | 3.85; 4096 x 4096 5.55 | 5.17, 40960 x 4096 19.7 | 16.6)
+  if (n == 32 && g_skinny_rows <= 0 && launch.split_k_kernel && launch.splits == 1 && groups[2] <= compute_units &&
+      (launch.rows_or_tile == 128 || (launch.rows_or_tile == 32 && k <= 5 * onebit::kChunkK)))
+    return none;
   if (n <= 16 || !g_skinny_enabled || g_tile_config >= 0 || groups[2] * ((n + 63) / 64) > 2L * compute_units) return none;
   if (!b_readable) return none;
   const WidePlan plan = plan_wide(groups, (double)m * n, n, k, true, launch.splits, compute_units);

@@ -154,3 +154,10 @@ def test_product_is_not_split_because_the_plan_it_replaces_is(fresh, m, n, k):
     fresh.stub_set(0, 1)
     assert product(fresh, m, n, k) == 0, fresh.onebit_sparse_last_error()
     assert last_launch(fresh)["kernel"] == "wide_kernel" and last_launch(fresh)["splits"] == 1
+
+
+@pytest.mark.parametrize("m,k,kernel", [(20480, 4096, "skinny_kernel"), (28672, 5536, "skinny_kernel"), (2048, 1056, "skinny_kernel"),
+                                        (4096, 4096, "wide_kernel"), (40960, 4096, "wide_kernel"), (11008, 1056, "wide_kernel")])
+def test_kernel_of_32_columns(fresh, m, k, kernel):
+    assert product(fresh, m, 32, k) == 0
+    assert last_launch(fresh)["kernel"] == kernel
