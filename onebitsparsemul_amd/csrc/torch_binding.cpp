@@ -201,10 +201,10 @@ std::vector<torch::Tensor> grouped_forward(const std::vector<torch::Tensor>& pre
   return ys;
 }
 
-// PreparedWeight.matmul: D = alpha A B + beta C into `out`, or into a new tensor of type out_dtype.
+// PreparedWeight.matmul: D = alpha A B + beta C into `out`, or into a new tensor of type out_dtype (None: torch's default).
 torch::Tensor matmul_prepared(const torch::Tensor& prepared, const torch::Tensor& b, const OptionalTensor& c,
                               const OptionalTensor& out, int64_t m, int64_t k, double alpha, double beta,
-                              c10::ScalarType out_dtype) {
+                              std::optional<c10::ScalarType> out_dtype) {
   at::AutoDispatchBelowADInplaceOrView guard_dispatch;
   const c10::Device device = b.device();
   check_placement(b, device);
@@ -221,7 +221,7 @@ torch::Tensor matmul_prepared(const torch::Tensor& prepared, const torch::Tensor
   };
   if (c.has_value()) check_result(*c);
   const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device);
-  torch::Tensor d = out.has_value() ? *out : empty_result({m, n}, out_dtype, device);
+  torch::Tensor d = out.has_value() ? *out : empty_result({m, n}, out_dtype.value_or(c10::get_default_dtype_as_scalartype()), device);
   check_result(d);
   check_status(onebit_sparse_matmul_prepared(prepared.data_ptr(), b.data_ptr(), c.has_value() ? c->data_ptr() : nullptr,
                                              d.data_ptr(), (int)m, (int)n, (int)k, (float)alpha, (float)beta,
