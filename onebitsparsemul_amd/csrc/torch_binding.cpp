@@ -277,11 +277,13 @@ std::tuple<torch::Tensor, torch::Tensor> pack_weight(const torch::Tensor& weight
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  m.def("onebit_mul", &onebit_mul, "A32 = Sparse W1 * A16 matmul.");
-  m.def("layer_forward", &layer_forward);
-  m.def("grouped_forward", &grouped_forward);
-  m.def("matmul_prepared", &matmul_prepared);
-  m.def("binary_mul", &binary_mul);
-  m.def("prepare", &prepare);
-  m.def("pack_weight", &pack_weight);
+  // Without the interpreter lock: a call may wait for another thread's, or for the device when a buffer has to grow.
+  using NoGil = pybind11::call_guard<pybind11::gil_scoped_release>;
+  m.def("onebit_mul", &onebit_mul, "A32 = Sparse W1 * A16 matmul.", NoGil());
+  m.def("layer_forward", &layer_forward, NoGil());
+  m.def("grouped_forward", &grouped_forward, NoGil());
+  m.def("matmul_prepared", &matmul_prepared, NoGil());
+  m.def("binary_mul", &binary_mul, NoGil());
+  m.def("prepare", &prepare, NoGil());
+  m.def("pack_weight", &pack_weight, NoGil());
 }
