@@ -318,8 +318,8 @@ struct WidePlan {
   int rows, splits, tokens;
   double us;
 };
-WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, bool plain, int most_splits,
-                   int compute_units) {
+WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, bool plain, int least_splits,
+                   int most_splits, int compute_units) {
   // [row group][column tiles - 1]
   static const double kBase[3][4] = {{2.75, 2.9, 2.9, 3.0}, {3.1, 3.3, 3.4, 3.6}, {3.7, 4.3, 5.8, 6.4}};
   static const double kRound[3][4] = {{0.74, 0.93, 1.48, 1.89}, {1.01, 1.26, 1.74, 2.24}, {1.88, 2.4, 2.75, 3.25}};
@@ -345,6 +345,7 @@ WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, 
       for (int s : {1, 2, 3, 4, 6, 8}) {
         if (g_split_k >= 1) s = g_split_k;
         s = std::min(std::min(s, most_splits), chunks);
+        if (s < least_splits) continue;
         const int rounds = ((chunks + s - 1) / s + 7) / 8;
         const double load = (double)total_groups[r] * groups * s / compute_units;
         const double work = rounds * kRound[r][tiles - 1] * (1.0 + kLoad[r][tiles - 1] * std::min(1.0, load)) *
@@ -402,6 +403,14 @@ bool wide_is_faster(const WidePlan& wide, const LaunchPlan& launch, int n, int k
   return wide.us < 0.81 * launch.model_us;
 }
 
+// Least K splits of wide_kernel in the place of `launch`: two where that splits K over 128-row groups (10241 to 16384 rows) and
+// the workgroups' copies of x are long. Its model has the unsplit plan on 64-row groups ahead there by up to 10 %, measured it
+// is up to 16 % behind (us, unsplit | split in two: 11008 x 28672 with 24 and 32 tokens 30.1 | 27.4, 34.7 | 29.5, 14336 x 24576
+// with 32 31.0 | 27.3; below the line 11008 x 20480 with 17 19.7 | 21.4, with 24 22.1 | 22.0).
+int wide_least_splits(const LaunchPlan& launch, int n, int k) {
+  return launch.split_k_kernel && launch.splits > 1 && launch.rows_or_tile == 128 && (long)k * n >= 480000 ? 2 : 1;
+}
+
 // The linear layer's plan: wide = wide_kernel with `wide_plan`, else `launch` as for a product with an aligned B.
 // Up to sixteen tokens the split-K kernel; beyond, wide_kernel in that kernel's place and where it is faster than the main
 // kernel. A layer call splits K into no more parts than the other kernel's plan would and uses the same buffer, so a call needs
@@ -418,7 +427,8 @@ LinearPlan plan_linear(int m, int tokens, int k, int compute_units) {
   const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
   if (!plan.launch.split_k_kernel && g_tile_config >= 0) return plan;
   if (tokens > onebit::kSkinnyMaxN && groups[2] * ((tokens + 63) / 64) > 2L * compute_units) return plan;
-  plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, false, plan.launch.splits, compute_units);
+  plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, false, wide_least_splits(plan.launch, tokens, k),
+                             plan.launch.splits, compute_units);
   plan.wide = plan.launch.split_k_kernel || wide_is_faster(plan.wide_plan, plan.launch, tokens, k);
   return plan;
 }
@@ -434,13 +444,14 @@ WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b
   const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
   // 32 columns, whole rows of an image: skinny_kernel is as fast or faster in one round of 128-row groups, and where K is so short
   // that its chunks do not fill a round of the sixteen wavefronts of its 32-row groups (us, skinny_kernel | wide_kernel:
-  // 20480 x 4096 10.4 | 11.2, 28672 x 5536 14.2 | 15.0, 2048 x 1056 3.71 | 3.85; 4096 x 4096 5.55 | 5.17, 40960 x 4096 19.7 | 16.6)
-  if (n == 32 && g_skinny_rows <= 0 && launch.split_k_kernel && launch.splits == 1 && groups[2] <= compute_units &&
-      (launch.rows_or_tile == 128 || (launch.rows_or_tile == 32 && k <= 5 * onebit::kChunkK)))
+  // 20480 x 4096 10.4 | 11.2, 28672 x 5536 14.2 | 15.0, 11008 x 20480 in two splits 22.9 | 23.5, 2048 x 1056 3.71 | 3.85;
+  // 4096 x 4096 5.55 | 5.17, 40960 x 4096 19.7 | 16.6)
+  if (n == 32 && g_skinny_rows <= 0 && launch.split_k_kernel && groups[2] <= compute_units &&
+      (launch.rows_or_tile == 128 || (launch.rows_or_tile == 32 && launch.splits == 1 && k <= 5 * onebit::kChunkK)))
     return none;
   if (n <= 16 || !g_skinny_enabled || g_tile_config >= 0 || groups[2] * ((n + 63) / 64) > 2L * compute_units) return none;
   if (!b_readable) return none;
-  const WidePlan plan = plan_wide(groups, (double)m * n, n, k, true, launch.splits, compute_units);
+  const WidePlan plan = plan_wide(groups, (double)m * n, n, k, true, wide_least_splits(launch, n, k), launch.splits, compute_units);
   if (plan.us == 1e30 || (!launch.split_k_kernel && !wide_is_faster(plan, launch, n, k))) return none;
   return plan;
 }
@@ -867,7 +878,7 @@ int onebit_sparse_linear_prepared_grouped_typed(const onebit_linear_problem* pro
     }
     const int enough = std::max(1, 160 * compute_units / 256);
     WidePlan wide_plan{};
-    if (wide) wide_plan = plan_wide(groups, 0.0, tokens, longest_k, false, 1, compute_units);
+    if (wide) wide_plan = plan_wide(groups, 0.0, tokens, longest_k, false, 1, 1, compute_units);
     const int rows = wide ? wide_plan.rows
                      : g_skinny_rows > 0 ? g_skinny_rows
                      : (rows_total / 128 >= enough) ? 128 : (rows_total / 64 >= enough) ? 64 : 32;

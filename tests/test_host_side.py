@@ -157,7 +157,17 @@ def test_product_is_not_split_because_the_plan_it_replaces_is(fresh, m, n, k):
 
 
 @pytest.mark.parametrize("m,k,kernel", [(20480, 4096, "skinny_kernel"), (28672, 5536, "skinny_kernel"), (2048, 1056, "skinny_kernel"),
+                                        (11008, 28672, "skinny_kernel"),
                                         (4096, 4096, "wide_kernel"), (40960, 4096, "wide_kernel"), (11008, 1056, "wide_kernel")])
 def test_kernel_of_32_columns(fresh, m, k, kernel):
     assert product(fresh, m, 32, k) == 0
     assert last_launch(fresh)["kernel"] == kernel
+
+
+@pytest.mark.parametrize("call,m,n,k,splits", [(layer, 11008, 32, 28672, 2), (layer, 14336, 24, 24576, 2), (product, 14336, 24, 28672, 2),
+                                               (layer, 11008, 17, 20480, 1), (layer, 11008, 24, 11008, 1)])
+def test_long_k_of_many_rows_stays_split(fresh, call, m, n, k, splits):
+    """Up to 15 % slower unsplit on wide_kernel than in the split plan of skinny_kernel that it replaces."""
+    assert call(fresh, m, n, k) == 0
+    launch = last_launch(fresh)
+    assert (launch["kernel"], launch["splits"]) == ("wide_kernel", splits)
