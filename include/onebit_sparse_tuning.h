@@ -13,7 +13,8 @@ extern "C" {
 #endif
 
 /* Tuning / test hooks: force a tile configuration of the main kernel (-1 = automatic) and choose whether
- * shapes with n <= 32 (n <= 64 when m <= 40960) use the split-K kernel (1, default) or the main kernel (0).
+ * shapes with n <= 32 (n <= 64 when m <= 40960) use the split-K kernels (1, default) or the main kernel (0).
+ * A forced tile also keeps products, and layer calls that could take the main kernel, out of the wide split-K kernel.
  * Tile codes 0-15 are the TileConfig values of csrc/onebit_launch.h (the linear-layer form has 4, 6, 9-15).
  * These five hooks act on the calling thread only: the calls that thread makes afterwards. A hook set on one thread
  * does not change what another thread launches (worker threads of a data-parallel wrapper, autograd threads). */
@@ -34,16 +35,21 @@ void onebit_sparse_set_split_k(int splits);
  * or can be allocated: not by the non-allocating entry point, and in a stream capture only after a warm-up. */
 void onebit_sparse_set_pad_b(int enabled);
 
-/* Diagnostic: what a prepared call of this shape would launch under the calling thread's hooks. The plan is made for
+/* Diagnostic: what a prepared product of this shape launches under the calling thread's hooks. The plan is made for
  * the compute-unit count of the current device, as the calls themselves do; without a usable device (a host without a
- * GPU) for 256 compute units, the MI355X figure. plan[0] = 1 for the split-K kernel (n <= 64), 0 for the main kernel;
- * plan[1] = weight rows per workgroup (split-K kernel) or the tile code (main kernel); plan[2] = K splits over
- * workgroups (1 = none); plan[3] = 1 if B is read through a padded copy. Calls of more
- * than 16 columns or tokens that the split-K kernel with asynchronous copies of B (csrc/onebit_wide.h) is modelled to run
- * faster than this plan go there instead; a product then splits K only if this plan does. onebit_sparse_describe_launch_for does the
- * same for an explicit compute-unit count and never touches a device. */
+ * GPU) for 256 compute units, the MI355X figure. plan[0] = ONEBIT_KERNEL_MAIN, _SPLIT_K (n <= 64) or _WIDE (17 columns or more:
+ * the split-K kernel with asynchronous copies of B, csrc/onebit_wide.h); plan[1] = the tile code (main kernel) or weight rows
+ * per workgroup; plan[2] = K splits over workgroups (1 = none); plan[3] = 1 if B is read through a padded copy. With
+ * k * n < 65536 a B that cannot be read in place is described as the non-allocating entry point reads it, without the copy.
+ * onebit_sparse_describe_launch_for does the same for an explicit compute-unit count and never touches a device. */
+#define ONEBIT_KERNEL_MAIN 0
+#define ONEBIT_KERNEL_SPLIT_K 1
+#define ONEBIT_KERNEL_WIDE 2
 int onebit_sparse_describe_launch(int m, int n, int k, int b_16_byte_aligned, int *plan);
 int onebit_sparse_describe_launch_for(int m, int n, int k, int b_16_byte_aligned, int compute_units, int *plan);
+/* The same for either form (token_major = 1: the linear layer's, n tokens) with five values: plan[4] = columns (tokens) a
+ * workgroup of ONEBIT_KERNEL_WIDE multiplies, 0 for the other kernels. compute_units = 0: of the current device. */
+int onebit_sparse_describe_call(int token_major, int m, int n, int k, int b_16_byte_aligned, int compute_units, int *plan);
 
 /* Diagnostic: sustained rate of one SMFMAC instruction in a register-only loop on the current device (one wavefront
  * per SIMD, `iterations` x 16 instructions each on 16 independent accumulator tiles, no LDS or global memory inside

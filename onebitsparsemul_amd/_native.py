@@ -18,7 +18,7 @@ EXPORTS = (
     "onebit_sparse_measure_smfmac_rate", "onebit_sparse_device_info",
     "onebit_sparse_describe_launch_for", "onebit_sparse_measure_smfmac_rate_shape",
     "onebit_sparse_linear_prepared_grouped", "onebit_sparse_pack_typed", "onebit_sparse_linear_prepared_typed",
-    "onebit_sparse_linear_prepared_grouped_typed",
+    "onebit_sparse_linear_prepared_grouped_typed", "onebit_sparse_describe_call",
 )
 
 
@@ -83,6 +83,8 @@ def lib():
         L.onebit_sparse_describe_launch.argtypes = [i32, i32, i32, i32, ctypes.POINTER(ctypes.c_int)]
         L.onebit_sparse_describe_launch_for.restype = i32
         L.onebit_sparse_describe_launch_for.argtypes = [i32, i32, i32, i32, i32, ctypes.POINTER(ctypes.c_int)]
+        L.onebit_sparse_describe_call.restype = i32
+        L.onebit_sparse_describe_call.argtypes = [i32, i32, i32, i32, i32, i32, ctypes.POINTER(ctypes.c_int)]
         L.onebit_sparse_measure_smfmac_rate_shape.restype = i32
         L.onebit_sparse_measure_smfmac_rate_shape.argtypes = [i32, i32, i32, ctypes.POINTER(ctypes.c_double)]
         L.onebit_sparse_device_info.restype = i32
@@ -343,16 +345,18 @@ def device_info():
     return cus.value, khz.value
 
 
-def describe_launch(m, n, k, b_aligned=True, compute_units=256):
-    """What a prepared call of this shape would launch on a GPU with `compute_units` compute units (host-only; None = the
-    current device's count, which is what the calls themselves plan for): dict(kernel, rows or tile, splits, pad_b)."""
-    plan = (ctypes.c_int * 4)()
-    if compute_units is None:
-        _check(lib().onebit_sparse_describe_launch(m, n, k, 1 if b_aligned else 0, plan))
-    else:
-        _check(lib().onebit_sparse_describe_launch_for(m, n, k, 1 if b_aligned else 0, compute_units, plan))
-    if plan[0]:
+def describe_launch(m, n, k, b_aligned=True, compute_units=256, tokens=False):
+    """What a prepared product of this shape (tokens: the layer form with n tokens) launches on a GPU with `compute_units`
+    compute units (host-only; None = the current device's count, which is what the calls themselves plan for):
+    dict(kernel, rows or tile, splits, pad_b where B may be copied, columns per workgroup of wide_kernel)."""
+    plan = (ctypes.c_int * 5)()
+    if compute_units is not None and compute_units <= 0:
+        raise ValueError("compute_units must be positive")
+    _check(lib().onebit_sparse_describe_call(int(tokens), m, n, k, int(b_aligned), compute_units or 0, plan))
+    if plan[0] == 1:
         return dict(kernel="skinny_kernel", rows=plan[1], splits=plan[2])
+    if plan[0] == 2:
+        return dict(kernel="wide_kernel", rows=plan[1], columns=plan[4], splits=plan[2], pad_b=bool(plan[3]))
     return dict(kernel="gemm_kernel", tile=plan[1], splits=plan[2], pad_b=bool(plan[3]))
 
 

@@ -661,16 +661,40 @@ void onebit_sparse_set_skinny_rows(int rows) { g_skinny_rows = rows; }
 void onebit_sparse_set_split_k(int splits) { g_split_k = splits; }
 void onebit_sparse_set_pad_b(int enabled) { g_pad_b = enabled ? 1 : 0; }
 
+int onebit_sparse_describe_call(int token_major, int m, int n, int k, int b_16_byte_aligned, int compute_units, int* plan) {
+  g_last_error.clear();
+  if (!plan) return fail(ONEBIT_ERR_ARGUMENT, "plan must not be null");
+  if (compute_units < 0) return fail(ONEBIT_ERR_ARGUMENT, "compute_units must not be negative (got %d)", compute_units);
+  if (int rc = check_shape(m, n, k)) return rc;
+  const int units = compute_units ? compute_units : current_compute_units();
+  LaunchPlan launch;
+  WidePlan wide{};
+  bool is_wide;
+  if (token_major) {
+    const LinearPlan linear = plan_linear(m, n, k, units);
+    launch = linear.launch;
+    wide = linear.wide_plan;
+    is_wide = linear.wide;
+  } else {
+    launch = choose_launch(m, n, k, b_16_byte_aligned != 0, units);
+    wide = plan_wide_product(launch, m, n, k, (n % 8 == 0 && b_16_byte_aligned) || launch.pad_b, units);
+    is_wide = wide.rows != 0;
+  }
+  plan[0] = is_wide ? ONEBIT_KERNEL_WIDE : launch.split_k_kernel ? ONEBIT_KERNEL_SPLIT_K : ONEBIT_KERNEL_MAIN;
+  plan[1] = is_wide ? wide.rows : launch.rows_or_tile;
+  plan[2] = full_splits((k + onebit::kChunkK - 1) / onebit::kChunkK, is_wide ? wide.splits : launch.splits);
+  plan[3] = !token_major && launch.pad_b;
+  plan[4] = is_wide ? wide.tokens : 0;
+  return ONEBIT_OK;
+}
+
 int onebit_sparse_describe_launch_for(int m, int n, int k, int b_16_byte_aligned, int compute_units, int* plan) {
   g_last_error.clear();
   if (!plan) return fail(ONEBIT_ERR_ARGUMENT, "plan must not be null");
   if (compute_units <= 0) return fail(ONEBIT_ERR_ARGUMENT, "compute_units must be positive (got %d)", compute_units);
-  if (int rc = check_shape(m, n, k)) return rc;
-  const LaunchPlan p = choose_launch(m, n, k, b_16_byte_aligned != 0, compute_units);
-  plan[0] = p.split_k_kernel;
-  plan[1] = p.rows_or_tile;
-  plan[2] = p.splits;
-  plan[3] = p.pad_b;
+  int call[5];
+  if (int rc = onebit_sparse_describe_call(0, m, n, k, b_16_byte_aligned, compute_units, call); rc != ONEBIT_OK) return rc;
+  std::copy(call, call + 4, plan);
   return ONEBIT_OK;
 }
 

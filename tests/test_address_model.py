@@ -3,9 +3,9 @@
 The kernels' addresses depend on shapes, launch plan and pointers only, never on operand contents, so their index
 arithmetic can be restated on the CPU (numpy, one array element per lane) and every access asserted to lie inside its
 operand: the prepared weight, B (or its padded copy), C / D, the K-split partial sums. The model follows
-onebitsparsemul_amd/csrc/ statement by statement (prepare_kernel, skinny_kernel with its five
+onebitsparsemul_amd/csrc/ statement by statement (prepare_kernel, wide_kernel, skinny_kernel with its five
 B staging modes, gemm_kernel's asynchronous copy pattern and epilogue ranges, splitk_reduce_kernel, pad_b_kernel) and
-takes the launch plan from the library itself (onebit_sparse_describe_launch, host-only). It covers the benchmark
+takes the launch plan from the library itself (onebit_sparse_describe_call, host-only). It covers the benchmark
 configurations and the long-K shapes with 33 to 64 columns (8192 x 28672 with n = 40, 48, 64). No GPU is touched.
 """
 import numpy as np
@@ -225,6 +225,132 @@ def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1
         check_reduce(m, n, splits, d_size)
 
 
+WIDE_WAVES, WIDE_IMAGE_K = 8, 64
+
+
+def row_swizzle(row, pieces):
+    return ((((row >> 1) & 1) << 2) | (((row >> 3) & 1) << 1)) if pieces == 8 else ((row >> 3) & 1) << 1 if pieces == 4 else 0 * row
+
+
+def wide_copies(tokens_form, copies, tokens, k, ldb, first_column):
+    """per copy: lane offsets in bytes, K position inside the image and column of the piece a lane brings"""
+    out = []
+    for i in range(copies):
+        if tokens_form:
+            token = np.minimum(8 * i + (LANE >> 3), tokens - 1)
+            piece = (LANE & 7) ^ (LANE >> 4) ^ (4 * (i & 1))
+            out.append(((token * k + 8 * piece) * 2, 8 * piece, 8 * i + (LANE >> 3)))
+        else:
+            slot = 64 * i + LANE
+            row = slot // copies  # `copies` pieces per row
+            col = 8 * ((slot % copies) ^ row_swizzle(row, copies))
+            used = np.where(first_column + col >= ldb, 0, col)
+            out.append(((row * ldb + used) * 2, row, col))
+    return out
+
+
+def check_wide(m, n, k, rows, columns, splits, tokens=False, pad_b=False, d_size=2):
+    """wide_kernel, either form: the launcher's checks, the prepared operand, the copies of x or B into the ring of two images
+    (K tail, last column group), the fragment reads of an image, the results"""
+    R = rows // 32
+    ldb = k if tokens else (n + 7) // 8 * 8 if pad_b else n
+    copies = (columns + 7) // 8 if tokens else 2 * ((columns + 15) // 16)
+    ct_count = (copies + 1) // 2
+    pieces = 2 * ct_count
+    image_bytes = 16 * ct_count * WIDE_IMAGE_K * 2
+    lds = WIDE_WAVES * 2 * image_bytes
+    assert 1 <= columns <= 64 and columns % 8 == 0 and lds <= 160 * 1024
+    assert (k * 64 * 2 if tokens else ldb * 128) < (1 << 32) and (tokens or (ldb % 8 == 0 and ldb >= n))
+    # the reduction's tiles take the place of the ring: min(R, 2) row blocks of 32 rows, sixteen columns per tile, fp32
+    assert min(R, 2) * 32 * 16 * ct_count * 4 <= 2 * image_bytes
+    kc_total, rb_total = (k + 255) // 256, m // 32
+    prep_size, b_size = prepared_bytes(m, k), (n * k if tokens else k * ldb) * 2
+    cps = (kc_total + splits - 1) // splits if splits > 1 else kc_total
+    splits = (kc_total + cps - 1) // cps
+    assert (splits - 1) * cps < kc_total
+    grid, col_groups = (rb_total + R - 1) // R, (n + columns - 1) // columns
+    # ---- an image: every piece of it copied once, a lane's reads find the K positions and columns it multiplies
+    image = {}
+    for i, (_, k_at, col) in enumerate(wide_copies(tokens, copies, 8 * copies, k, max(ldb, 8 * copies), 0)):
+        for lane in range(64):
+            where = i * 64 + lane
+            assert where * 16 + 16 <= image_bytes and where not in image
+            image[where] = (k_at[lane], col[lane])  # eight K positions of a token, or eight columns of a K position
+    i16, g16 = LANE & 15, LANE >> 4
+    for ct in range(ct_count):
+        if tokens:
+            base = i16 * 128 + (((4 * (g16 >> 1) + (g16 & 1)) ^ ((i16 >> 1) & 7)) << 4)
+            for h in range(2):
+                at = (base ^ (h << 5)) + ct * 2048
+                for lane in range(64):
+                    token, want_k = 16 * ct + i16[lane], 32 * (g16[lane] >> 1) + 8 * (g16[lane] & 1) + 16 * h
+                    assert at[lane] % 16 == 0 and at[lane] + 16 <= image_bytes
+                    if token < 8 * copies:  # an odd copy count leaves the last eight tokens of a tile unwritten: never stored
+                        assert image[at[lane] // 16] == (want_k, token)
+        else:
+            lane_row = 32 * (g16 >> 1) + 8 * (g16 & 1) + (i16 >> 2)
+            tile = lane_row * pieces * 16 + (((2 * ct + ((i16 & 3) >> 1)) ^ row_swizzle(lane_row, pieces)) << 4) + (i16 & 1) * 8
+            for q in range(4):
+                step = 4 * (q & 1) + 16 * (q >> 1)
+                at = tile + step * pieces * 16
+                for lane in range(64):  # four columns of a K position per lane of the transpose read
+                    assert at[lane] + 8 <= image_bytes
+                    assert image[at[lane] // 16] == (lane_row[lane] + step, 16 * ct + 8 * ((i16[lane] & 3) >> 1))
+    # ---- addresses
+    for group in sorted({0, col_groups // 2, col_groups - 1}):
+        first_column = group * columns
+        here = min(n - first_column, 8 * copies if tokens else columns)
+        assert here >= 1
+        base0 = first_column * (k if tokens else 1) * 2
+        plan = wide_copies(tokens, copies, here, k, ldb, first_column)
+        for lane_off, _, _ in plan:
+            assert lane_off.max() < (1 << 32)
+        for split in sorted({0, splits // 2, splits - 1}):
+            kc_begin = split * cps
+            kc_end = min(kc_begin + cps, kc_total)
+            for wave in range(WIDE_WAVES):
+                chunks, images, kc = [kc_begin + wave], [], kc_begin + wave
+                if kc < kc_end:
+                    images += [kc * 4, kc * 4 + 1]
+                    if kc + WIDE_WAVES < kc_end:
+                        chunks.append(kc + WIDE_WAVES)
+                while kc < kc_end:
+                    images += [kc * 4 + 2, kc * 4 + 3]
+                    if kc + WIDE_WAVES < kc_end:
+                        images += [(kc + WIDE_WAVES) * 4, (kc + WIDE_WAVES) * 4 + 1]
+                    if kc + 2 * WIDE_WAVES < kc_end:
+                        chunks.append(kc + 2 * WIDE_WAVES)
+                    kc += WIDE_WAVES
+                mine = range(kc_begin + wave, kc_end, WIDE_WAVES)
+                assert images == [c * 4 + s for c in mine for s in range(4)]  # every image of its chunks once, in order
+                assert len(mine) == 0 or chunks == list(mine)
+                for kc in chunks:
+                    for wg in sorted({0, grid // 2, grid - 1}):
+                        for r in range(R):
+                            rb = min(wg * R + r, rb_total - 1)
+                            block = min(kc, kc_total - 1) * BLOCK
+                            for off, width in ((LANE * 16, 16), (SIGN_OFF + LANE * 8, 8)):
+                                inside(block + off, width, kc_total * BLOCK, "wide_kernel: prepared block inside its descriptor")
+                                inside(rb * kc_total * BLOCK + block + off, width, prep_size, "wide_kernel: prepared operand")
+                for at in images:
+                    k0 = at * WIDE_IMAGE_K
+                    for lane_off, k_at, _ in plan:
+                        real = k0 + k_at < k  # the others are copied from the block of zeros
+                        assert real.all() or k0 + WIDE_IMAGE_K > k
+                        inside(base0 + k0 * (2 if tokens else ldb * 2) + lane_off[real], 16, b_size, "wide_kernel: copies")
+        # ---- results of the group: rows below m, this group's columns and no other's
+        cols = first_column + np.arange(here)
+        assert cols.max() < n and (group == col_groups - 1 or here == columns)
+        elem = 4 if splits > 1 else d_size
+        for wg in sorted({0, grid // 2, grid - 1}):
+            out_rows = np.arange(wg * R * 32, min((wg + 1) * R * 32, m))
+            for split in {0, splits - 1}:
+                at = cols[None, :] * m + out_rows[:, None] if tokens else out_rows[:, None] * n + cols[None, :]
+                inside((split * m * n * (splits > 1) + at) * elem, elem, splits * m * n * elem, "wide_kernel: results")
+    if splits > 1:
+        check_reduce(m, n, splits, d_size)
+
+
 def check_reduce(m, n, splits, d_size):
     """splitk_reduce_kernel: one thread per 4 (or 1) results"""
     total = m * n
@@ -358,9 +484,11 @@ def check_gemm(m, n, k, tile, splits, pad_b, tokens=False, b_aligned=True, d_siz
 
 
 def check_call(m, n, k, tokens=False, b_aligned=True):
-    plan = _native.describe_launch(m, n, k, b_aligned=b_aligned or tokens)
+    plan = _native.describe_launch(m, n, k, b_aligned=b_aligned or tokens, tokens=tokens)
     if plan["kernel"] == "skinny_kernel":
         check_skinny(m, n, k, plan["rows"], tokens=tokens, b_aligned=b_aligned, splits=plan["splits"])
+    elif plan["kernel"] == "wide_kernel":
+        check_wide(m, n, k, plan["rows"], plan["columns"], plan["splits"], tokens=tokens, pad_b=plan["pad_b"])
     else:
         check_gemm(m, n, k, plan["tile"], plan["splits"], plan["pad_b"] and not tokens, tokens=tokens, b_aligned=b_aligned)
     return plan
@@ -384,17 +512,34 @@ def test_prepare_kernel_addresses(m, k):
     check_prepare(m, k)
 
 
+@pytest.mark.parametrize("n", [17, 24, 40, 56, 65, 72, 104, 257])
+@pytest.mark.parametrize("m,k", [(64, 32), (192, 1056), (320, 4640), (1024, 8192)])
+def test_wide_kernel_addresses(n, m, k):
+    """every width of the column groups the plan can choose, each row group, K splits; B in place and through its padded copy"""
+    for rows in (32, 64, 128):
+        for columns in {8 * ((min(n, 16 * width) + 7) // 8) for width in (1, 2, 3, 4)}:
+            for splits in (1, 3):
+                splits = min(splits, (k + 255) // 256)
+                check_wide(m, n, k, rows, columns, splits, tokens=True)
+                check_wide(m, n, k, rows, columns, splits, pad_b=n % 8 != 0)
+
+
 @pytest.mark.parametrize("n", [40, 48, 64])
-@pytest.mark.parametrize("rows,skinny", [(32, True), (64, True), (-1, False)])
-def test_long_k_wide_skinny_shapes(hooks, n, rows, skinny):
-    """8192 x 28672 with 33 to 64 columns: the 64-column images of the split-K kernel with 32- and 64-row workgroups, and
-    the main kernel with the K split its plan chooses, plain and token-major."""
+@pytest.mark.parametrize("rows", [32, 64, -1])
+def test_long_k_wide_skinny_shapes(hooks, n, rows):
+    """8192 x 28672 with 33 to 64 columns: wide_kernel and the 64-column images of skinny_kernel with 32- and 64-row
+    workgroups, and the main kernel with the K split its plan chooses, plain and token-major."""
     m, k = 8192, 28672
+    if rows < 0:
+        _native.set_skinny_enabled(False)
+        for tokens in (False, True):
+            assert check_call(m, n, k, tokens=tokens)["kernel"] == "gemm_kernel"
+        return
     _native.set_skinny_rows(rows)
-    _native.set_skinny_enabled(skinny)
     for tokens in (False, True):
-        plan = check_call(m, n, k, tokens=tokens)
-        assert (plan["kernel"] == "skinny_kernel") == skinny
+        assert check_call(m, n, k, tokens=tokens)["kernel"] == "wide_kernel"
+    _native.set_tile_config(0)  # a forced tile keeps products out of wide_kernel
+    assert check_call(m, n, k)["kernel"] == "skinny_kernel"
 
 
 @pytest.mark.parametrize("m,n,k", [(512, 512, 512), (1024, 1024, 1024), (2048, 2048, 2048), (4096, 4096, 4096), (8192, 8192, 8192),
@@ -420,7 +565,10 @@ def test_benchmark_configurations(hooks, m, n, k):
 def test_ragged_and_split_shapes(hooks, m, n, k, b_aligned):
     for rows in (-1, 32, 64, 128):
         _native.set_skinny_rows(rows)
-        check_call(m, n, k, b_aligned=b_aligned)
+        for tile in (-1, 0):  # 0: a forced tile keeps products out of wide_kernel
+            _native.set_tile_config(tile)
+            check_call(m, n, k, b_aligned=b_aligned)
+        _native.set_tile_config(-1)
     _native.set_skinny_rows(-1)
     check_call(m, n, k, tokens=True)
     for splits in (2, 3, 16):  # the split-K kernel's own K split over workgroups (n <= 64), forced
@@ -459,6 +607,8 @@ def test_the_model_catches_an_out_of_range_access():
     try:
         with pytest.raises(AssertionError):
             check_skinny(1024, 16, 4096, 64)
+        with pytest.raises(AssertionError):
+            check_wide(1024, 48, 4096, 64, 48, 1)
         with pytest.raises(AssertionError):
             check_gemm(1024, 512, 1024, 9, 1, False)
     finally:

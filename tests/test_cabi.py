@@ -172,21 +172,29 @@ def test_launch_plan_of_the_benchmark_shapes(_default_hooks):
         assert plan(11008, n, 4096) == dict(kernel="skinny_kernel", rows=64, splits=1)
         assert plan(4096, n, 11008) == dict(kernel="skinny_kernel", rows=32, splits=1)
     assert plan(28672, 16, 8192) == dict(kernel="skinny_kernel", rows=128, splits=1)
+    # 17 columns or more: the split-K kernel with asynchronous copies of B, but for 32 columns in one round of 128-row groups
+    def wide(rows, columns, splits=1, pad_b=False):
+        return dict(kernel="wide_kernel", rows=rows, columns=columns, splits=splits, pad_b=pad_b)
     assert plan(28672, 32, 8192) == dict(kernel="skinny_kernel", rows=128, splits=1)
-    assert plan(16384, 32, 4096) == dict(kernel="skinny_kernel", rows=64, splits=1)
-    assert plan(4096, 64, 4096) == dict(kernel="skinny_kernel", rows=32, splits=1)
-    assert plan(11008, 64, 4096) == dict(kernel="skinny_kernel", rows=64, splits=1)   # 33 ... 64 columns: at most 64 rows
-    assert plan(28672, 64, 8192) == dict(kernel="skinny_kernel", rows=64, splits=1)
+    assert plan(28672, 32, 8192, tokens=True) == wide(128, 32)
+    assert plan(16384, 32, 4096) == wide(64, 32)
+    assert plan(4096, 64, 4096) == wide(32, 32)
+    assert plan(11008, 64, 4096) == wide(64, 64)
+    assert plan(28672, 64, 8192) == wide(128, 64)
     # few row groups over a long K: K split over workgroups as well, one workgroup per compute unit, 64-row groups
     assert plan(4096, 16, 16384) == dict(kernel="skinny_kernel", rows=64, splits=4)
     assert plan(2048, 16, 28672) == dict(kernel="skinny_kernel", rows=64, splits=8)
     assert plan(8192, 16, 28672) == dict(kernel="skinny_kernel", rows=64, splits=2)
-    assert plan(8192, 64, 8192) == dict(kernel="skinny_kernel", rows=64, splits=2)
+    assert plan(8192, 64, 8192) == wide(64, 32)                                         # there unsplit
     assert plan(11008, 32, 28672) == dict(kernel="skinny_kernel", rows=128, splits=2)   # 64 rows: 172 groups, no room
+    assert plan(11008, 32, 28672, tokens=True) == wide(128, 32, splits=2)
+    assert plan(2048, 48, 28672)["splits"] > 1 and plan(2048, 48, 28672)["kernel"] == "wide_kernel"
     assert plan(4096, 16, 11008) == dict(kernel="skinny_kernel", rows=32, splits=1)     # B too small to pay for it
     assert plan(8192, 16, 16384) == dict(kernel="skinny_kernel", rows=32, splits=1)
-    assert plan(65536, 64, 8192)["kernel"] == "gemm_kernel"      # from about 48k rows on the main kernel is faster
-    assert plan(4096, 65, 4096)["kernel"] == "gemm_kernel"
+    assert plan(65536, 64, 4096)["kernel"] == "gemm_kernel"      # from 40960 rows on the main kernel, unless K is long
+    assert plan(65536, 64, 8192)["kernel"] == "wide_kernel"
+    assert plan(4096, 65, 4096) == wide(64, 24, pad_b=True)      # beyond 64 columns by the two kernels' models
+    assert plan(4096, 500, 11008, tokens=True) == wide(128, 64)
     # fewer than 256 tiles of 512 x 128: tile and split from the cost model
     assert plan(4096, 3072, 4096) == dict(kernel="gemm_kernel", tile=9, splits=1, pad_b=False)    # 192 large tiles: eight wavefronts
     assert plan(4096, 1536, 4096) == dict(kernel="gemm_kernel", tile=10, splits=1, pad_b=False)   # 192 of 256 x 128
@@ -194,9 +202,9 @@ def test_launch_plan_of_the_benchmark_shapes(_default_hooks):
     assert plan(4096, 384, 11008) == dict(kernel="gemm_kernel", tile=13, splits=2, pad_b=False)   # 96 tiles, 43 chunks
     assert plan(4096, 512, 4096) == dict(kernel="gemm_kernel", tile=14, splits=1, pad_b=False)    # 64 x 128, two K groups
     # few tiles over a long K: split over workgroups; many tiles: never
-    few = plan(4096, 128, 4096)
+    few = plan(4096, 256, 11008)
     assert few["kernel"] == "gemm_kernel" and few["splits"] > 1
-    assert plan(4096, 256, 11008)["splits"] > 1
+    assert plan(4096, 128, 4096) == wide(64, 32)
     # B rows that are not 16-byte aligned: padded copy, except for tiny operands
     assert plan(4096, 1001, 4096)["pad_b"] is True
     assert plan(4096, 1000, 4096, b_aligned=False)["pad_b"] is True

@@ -287,13 +287,19 @@ def test_one_call_entry_point_on_several_streams_keeps_the_reordered_weights_apa
 
 @pytest.mark.parametrize("m,k,n,rows", [(20480, 1024, 64, 64), (28672, 512, 40, 64), (28672, 1024, 32, 128), (20480, 768, 24, 128)])
 def test_split_k_kernel_large_m_row_groups(m, k, n, rows):
-    """the row groups the C ABI picks for many weight rows: 64 rows at 33 ... 64 columns, 128 rows at 17 ... 32
-    (partial tiles reduced in two rounds); exact on integers against the oracle"""
-    assert _native.describe_launch(m, n, k) == dict(kernel="skinny_kernel", rows=rows, splits=1)
+    """the row groups of skinny_kernel for many weight rows: 64 rows at 33 ... 64 columns, 128 rows at 17 ... 32
+    (partial tiles reduced in two rounds), where wide_kernel does not take the call (a forced tile keeps it out), and the
+    product and the layer as the C ABI launches them by itself; exact on integers against the oracle"""
     a, meta = synthetic.make_weight(m, k, seed=m + n)
     dense = oracle.decompress_operands(a.numpy(), meta.numpy(), m, k)
     bi = synthetic.make_b(k, n, seed=n, kind="int")
     exact = oracle.host_gemm(dense, bi.numpy(), d_dtype=oracle.F32, acc="f32")
+    _native.set_tile_config(0)
+    assert _native.describe_launch(m, n, k) == dict(kernel="skinny_kernel", rows=rows, splits=1)
+    assert np.array_equal(_run_prepared(a, meta, bi, m, n, k, out_dtype=torch.float32), exact)
+    _native.set_tile_config(-1)
+    assert _native.describe_launch(m, n, k)["kernel"] == ("skinny_kernel" if n == 32 else "wide_kernel")
+    assert _native.describe_launch(m, n, k, tokens=True)["kernel"] == "wide_kernel"
     assert np.array_equal(_run_prepared(a, meta, bi, m, n, k, out_dtype=torch.float32), exact)
     prep = _native.prepare(a.cuda(), meta.cuda(), m, k)
     y = torch.full((n, m), float("nan"), dtype=torch.float32, device="cuda")
@@ -304,9 +310,9 @@ def test_split_k_kernel_large_m_row_groups(m, k, n, rows):
 
 @pytest.mark.parametrize("m,k,ns", [(8192, 28672, (40, 48, 64)), (4096, 16384, (16,)), (2048, 20480, (32,))])
 def test_split_k_kernel_long_k(m, k, ns):
-    """long K (64 to 112 chunks of 256) through the split-K kernel's 16-, 32- and 64-column images with 32- and
-    64-row workgroups, through the main kernel with its planned K split, and through the token-major form of both:
-    bit-exact against the oracle on integer operands"""
+    """long K (64 to 112 chunks of 256) through skinny_kernel's 16-, 32- and 64-column images and through wide_kernel with
+    32- and 64-row workgroups, through the main kernel with its planned K split, and through the token-major form of all
+    three: bit-exact against the oracle on integer operands"""
     a, meta = synthetic.make_weight(m, k, seed=m + k)
     dense = oracle.decompress_operands(a.numpy(), meta.numpy(), m, k)
     prep = _native.prepare(a.cuda(), meta.cuda(), m, k)
@@ -318,12 +324,19 @@ def test_split_k_kernel_long_k(m, k, ns):
         for rows, skinny in ((32, True), (64, True), (-1, False)):
             _native.set_skinny_rows(rows)
             _native.set_skinny_enabled(skinny)
-            d = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda")
-            _native.matmul_prepared(prep, bd, d, m, n, k)
+            kernels = ("skinny_kernel",) + ("wide_kernel",) * (n > 16) if skinny else ("gemm_kernel",)
+            for kernel in kernels:
+                _native.set_tile_config(0 if kernel == "skinny_kernel" else -1)  # a forced tile keeps wide_kernel out
+                assert _native.describe_launch(m, n, k)["kernel"] == kernel
+                d = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda")
+                _native.matmul_prepared(prep, bd, d, m, n, k)
+                torch.cuda.synchronize()
+                assert np.array_equal(d.cpu().numpy(), exact), (n, rows, kernel)
+            _native.set_tile_config(-1)
+            assert _native.describe_launch(m, n, k, tokens=True)["kernel"] == kernels[-1]
             y = torch.full((n, m), float("nan"), dtype=torch.float32, device="cuda")
             _native.linear_prepared(prep, xd, y, m, k)
             torch.cuda.synchronize()
-            assert np.array_equal(d.cpu().numpy(), exact), (n, rows, skinny)
             assert np.array_equal(y.cpu().numpy(), exact.T), (n, rows, skinny, "token-major")
     del dense
 
@@ -332,12 +345,13 @@ def test_split_k_kernel_long_k(m, k, ns):
 @pytest.mark.parametrize("m,n,k", [(256, 16, 8192), (192, 5, 4128), (320, 32, 12320), (128, 40, 8224), (1024, 64, 16384),
                                    (4096, 16, 16384), (256, 1, 8224), (192, 2, 8192), (320, 4, 4128)])
 def test_split_k_kernel_with_k_split_over_workgroups(rows, splits, m, n, k):
-    """the split-K kernel with K split over workgroups as well (partial sums + ordered reduction): forced split counts
+    """the split-K kernels with K split over workgroups as well (partial sums + ordered reduction): forced split counts
     that do and do not divide the chunk count, splits with fewer chunks than wavefronts, K tails, every image width,
-    beta != 0, fp16 and fp32 results, plain and token-major form with bias; the last shape splits by the plan's own
-    choice"""
+    beta != 0, fp16 and fp32 results, plain (skinny_kernel, and beyond sixteen columns wide_kernel too) and token-major
+    form with bias; 4096 x 16 x 16384 splits by the plan's own choice"""
     _native.set_skinny_rows(rows)
     _native.set_split_k(splits)
+    _native.set_tile_config(0)  # a forced tile keeps wide_kernel out
     plan = _native.describe_launch(m, n, k)
     assert plan["kernel"] == "skinny_kernel"
     if (m, n, k) == (4096, 16, 16384) and splits == -1:
@@ -351,6 +365,12 @@ def test_split_k_kernel_with_k_split_over_workgroups(rows, splits, m, n, k):
     assert np.array_equal(got, exact)
     plain = oracle.blas_matmul(dense, bi.numpy(), dtype=np.float32)
     assert np.array_equal(_run_prepared(a, meta, bi, m, n, k, out_dtype=torch.float16), plain.astype(np.float16))
+    _native.set_tile_config(-1)
+    if n > 16:
+        route = _native.describe_launch(m, n, k)["kernel"]
+        assert route == "wide_kernel" or (n == 32 and rows == -1)
+        got = _run_prepared(a, meta, bi, m, n, k, c=ci, alpha=2.0, beta=1.0, out_dtype=torch.float32)
+        assert np.array_equal(got, exact)
     # token-major form with a bias
     bias = synthetic.make_b(1, m, seed=n + 2, kind="int").reshape(m)
     prep = _native.prepare(a.cuda(), meta.cuda(), m, k)

@@ -3,6 +3,7 @@ which stands in for the HIP runtime and the kernels, and called from Python thre
 threads really meet inside the library."""
 import ctypes
 import os
+import random
 import subprocess
 import threading
 
@@ -32,6 +33,7 @@ def host(tmp_path_factory):
     lib.onebit_sparse_matmul_prepared.argtypes = [vp, vp, vp, vp, i32, i32, i32, f32, f32, i32, i32, vp]
     lib.onebit_sparse_matmul_prepared_static.argtypes = lib.onebit_sparse_matmul_prepared.argtypes
     lib.onebit_sparse_linear_prepared.argtypes = [vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]
+    lib.onebit_sparse_describe_call.argtypes = [i32] * 6 + [ctypes.POINTER(i32)]
     lib.onebit_sparse_matmul_ex.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, f32, f32, i32, i32, i32, vp]
     return lib
 
@@ -171,3 +173,41 @@ def test_long_k_of_many_rows_stays_split(fresh, call, m, n, k, splits):
     assert call(fresh, m, n, k) == 0
     launch = last_launch(fresh)
     assert (launch["kernel"], launch["splits"]) == ("wide_kernel", splits)
+
+
+def test_description_is_what_is_launched(fresh):
+    """onebit_sparse_describe_call against the launch of the call itself: both forms, ragged and unaligned B, the hooks."""
+    rng = random.Random(1)
+    hooks = (fresh.onebit_sparse_set_tile_config, fresh.onebit_sparse_set_skinny_rows, fresh.onebit_sparse_set_split_k)
+    plan, seen = (i32 * 5)(), set()
+    try:
+        for _ in range(3000):
+            m, k = 64 * int(2 ** rng.uniform(0, 10)), 32 * int(2 ** rng.uniform(0, 9.8))
+            n, tokens, aligned = int(2 ** rng.uniform(0, 11)), rng.random() < 0.5, rng.random() < 0.8
+            if rng.random() < 0.5:
+                n = (n + 7) // 8 * 8
+            settings = (rng.choice((-1, -1, -1, 4, 9)), rng.choice((-1, -1, 32, 64, 128)), rng.choice((-1, -1, -1, 1, 2, 7)))
+            for hook, value in zip(hooks, settings):
+                hook(value)
+            assert fresh.onebit_sparse_describe_call(tokens, m, n, k, aligned, 256, plan) == 0
+            if tokens:
+                rc = layer(fresh, m, n, k)
+            elif k * n < 65536:  # described as the non-allocating entry point reads it
+                rc = fresh.onebit_sparse_matmul_prepared_static(0x1000, 0x2000 if aligned else 0x2002, None, 0x3000, m, n, k, 1.0, 0.0,
+                                                                0, 1, None)
+            else:
+                rc = product(fresh, m, n, k, b=0x2000 if aligned else 0x2002)
+            if rc != 0 and not tokens and k * n < 65536:
+                assert b"static workspace" in fresh.onebit_sparse_last_error()
+                continue
+            assert rc == 0, fresh.onebit_sparse_last_error()
+            got = last_launch(fresh)
+            described = dict(kernel=KERNELS[plan[0]], rows_or_tile=plan[1], splits=plan[2], padded=bool(plan[3]),
+                             columns=plan[4])
+            assert got == described, (m, n, k, tokens, aligned, settings)
+            seen.add((got["kernel"], got["splits"] > 1, got["padded"], tokens))
+    finally:
+        for hook in hooks:
+            hook(-1)
+    assert len(seen) >= 11, seen
+    assert fresh.stub_violations() == 0, fresh.stub_violation().decode()
