@@ -2,11 +2,12 @@
 
 The kernels' addresses depend on shapes, launch plan and pointers only, never on operand contents, so their index
 arithmetic can be restated on the CPU (numpy, one array element per lane) and every access asserted to lie inside its
-operand: the prepared weight, B (or its padded copy), C / D, the K-split partial sums. The model follows
-onebitsparsemul_amd/csrc/ statement by statement (prepare_kernel, wide_kernel, skinny_kernel with its five
-B staging modes, gemm_kernel's asynchronous copy pattern and epilogue ranges, splitk_reduce_kernel, pad_b_kernel) and
-takes the launch plan from the library itself (onebit_sparse_describe_call, host-only). It covers the benchmark
-configurations and the long-K shapes with 33 to 64 columns (8192 x 28672 with n = 40, 48, 64). No GPU is touched.
+operand: the prepared weight, B (or its padded copy), C / D, the K-split partial sums. The model restates the index
+arithmetic of onebitsparsemul_amd/csrc/: prepare_kernel and pack_kernel, skinny_kernel with its four B staging modes, wide_kernel
+in both forms, gemm_kernel's asynchronous copy pattern and epilogue ranges, splitk_reduce_kernel, pad_b_kernel. Where a load
+deliberately reaches past a row (pieces at any alignment, padded copy) the elements that arrive are tracked too. The route of a call
+comes from the library itself (onebit_sparse_describe_call, host-only). It covers the benchmark configurations and the long-K shapes
+with 33 to 64 columns (8192 x 28672 with n = 40, 48, 64). No GPU is touched.
 """
 import numpy as np
 import pytest
@@ -39,27 +40,114 @@ def meta_offset_reference(r, c, m):
 
 
 # ---------------------------------------------------------------------------------------------------------------
+def strip_positions(grid, width, length):
+    """(along, across) of every workgroup of a grid that is walked in strips (strip_position)"""
+    block = np.arange(grid, dtype=np.int64)
+    per, rem, xcd = grid // 8, grid % 8, block % 8
+    v = xcd * per + np.minimum(xcd, rem) + block // 8
+    strip, w = v // (width * length), v % (width * length)
+    return w // width, strip * width + w % width
+
+
+def check_strips(grid, width, length, groups):
+    """every (along, group) once; the workgroups past the last group return"""
+    along, across = strip_positions(grid, width, length)
+    used = across < groups
+    assert along.min() >= 0 and along.max() < length and across.min() >= 0
+    cells = along[used] * groups + across[used]
+    assert np.array_equal(np.sort(cells), np.arange(length * groups))
+
+
 def check_prepare(m, k):
-    kc_total, rb_total, ncols = (k + 255) // 256, m // 32, k // 16
-    a_bytes, e_elems = m * k // 16, m * ncols
+    kc_total, pairs, ncols = (k + 255) // 256, m // 64, k // 16
+    a_bytes, e_bytes = m * k // 16, m * ncols * 2
+    strips = (pairs + 15) // 16
+    check_strips(kc_total * 4 * strips, 4, kc_total, (pairs + 3) // 4)  # four wavefronts (row pairs) per workgroup
     i, ga = LANE & 31, LANE >> 5
-    for kc in {0, kc_total // 2, kc_total - 1}:
-        for rb in {0, rb_total // 2, rb_total - 1}:
-            for half in (0, 1):
-                j = kc * 128 + LANE + 64 * half
-                ok = j < k // 2
-                inside(((rb * ROW_BLOCK + j[ok] * m) >> 3), 4, a_bytes, "prepare: value bits")
-            r, c0 = rb * ROW_BLOCK + i, kc * 16 + ga
-            off = meta_offset_reference(r, c0, m)
+    for kc in sorted({0, kc_total // 2, kc_total - 1}):
+        for pair in sorted({0, pairs // 2, pairs - 1}):
+            # value bits: eight bytes, the 64 rows of one compressed column
+            j = 15 - (i & 15)
+            col0 = kc * 128 + 16 * (j >> 2) + 8 * ga + 2 * (j & 3) + (i >> 4)
+            for h in (0, 1):
+                # bit i of sign word h: kept value t of step s, which is compressed column 8 (2 s + ga) + t of the chunk
+                t, s = 2 * (j & 3) + (i >> 4), 4 * h + (j >> 2)
+                col = col0 + 64 * h
+                assert np.array_equal(col, kc * 128 + 8 * (2 * s + ga) + t)
+                assert np.array_equal(i, np.where(t % 2 == 0, 15, 31) - (4 * (s % 4) + t // 2))
+                ok = col < k // 2
+                at = pair * 64 + col[ok] * m
+                assert (at % 64 == 0).all()
+                inside(at >> 3, 8, a_bytes, "prepare: value bits")
+            # metadata, reference layout: dwords of rows r and r + 4
+            src = kc * 8 * m + pair * 64 + ((((i >> 1) & 1) << 5) | (((i >> 3) & 3) << 2) | ((i & 1) << 1) | ga)
             for s in range(8):
-                c = c0 + 2 * s
-                ok = c < ncols
-                assert np.array_equal(off[ok], meta_offset_reference(r[ok], c[ok], m))  # the running offset is the closed form
-                inside(off[ok] * 2, 2, e_elems * 2, "prepare: metadata")
-                off = off + 2 * m
-            block = (rb * kc_total + kc) * BLOCK
-            inside(block + LANE * 16, 16, prepared_bytes(m, k), "prepare: block metadata")
-            inside(block + SIGN_OFF + LANE * 8, 8, prepared_bytes(m, k), "prepare: block signs")
+                if kc * 16 + 2 * s >= ncols:
+                    continue
+                for blk in (0, 1):
+                    dword = src + s * m + 16 * blk
+                    inside(dword * 4, 4, e_bytes, "prepare: metadata")
+                    row = pair * 64 + 32 * blk + i
+                    assert np.array_equal(2 * dword + ((i >> 2) & 1), meta_offset_reference(row, kc * 16 + 2 * s + ga, m))
+            # metadata, general form: the running offset is the closed form
+            for blk in (0, 1):
+                r, c0 = pair * 64 + 32 * blk + i, kc * 16 + ga
+                off = meta_offset_reference(r, c0, m)
+                for s in range(8):
+                    ok = c0 + 2 * s < ncols
+                    assert np.array_equal(off[ok], meta_offset_reference(r[ok], (c0 + 2 * s)[ok], m))
+                    inside(off[ok] * 2, 2, e_bytes, "prepare: metadata (general form)")
+                    off = off + 2 * m
+                block = ((2 * pair + blk) * kc_total + kc) * BLOCK
+                inside(block + LANE * 16, 16, prepared_bytes(m, k), "prepare: block metadata")
+                inside(block + SIGN_OFF + LANE * 8, 8, prepared_bytes(m, k), "prepare: block signs")
+
+
+def check_pack(m, k, size):
+    """pack_kernel on values of `size` bytes: rows into LDS and back, value bits and metadata out"""
+    row_bytes, pieces = 64 * size, 4 * size
+    rows_per_copy = 64 // pieces
+    k_tiles, tiles, ncols = (k // 16 + 3) // 4, m // 64, k // 16
+    check_strips(k_tiles * 4 * ((tiles + 15) // 16), 4, k_tiles, (tiles + 3) // 4)
+    a_bytes, e_bytes = m * k // 16, m * ncols * 2
+    for along in sorted({0, k_tiles // 2, k_tiles - 1}):
+        c_first = along * 4
+        c_count = min(ncols - c_first, 4)
+        for tile in sorted({0, tiles // 2, tiles - 1}):
+            row0 = tile * 64
+            # copies: LDS piece position -> (row, piece) it holds
+            image = {}
+            for copy in range(pieces):
+                row = copy * rows_per_copy + LANE // pieces
+                piece = (LANE % pieces) ^ (row % pieces)
+                used = np.where(piece < size * c_count, piece, 0)
+                inside(((row0 + row) * k + 16 * c_first) * size + 16 * used, 16, m * k * size, "pack: weights")
+                for lane in range(64):
+                    image[copy * 64 + lane] = (row[lane], piece[lane])
+            assert len(image) == 64 * pieces
+            for q in range(pieces):
+                at = LANE * row_bytes + ((q ^ (LANE % pieces)) << 4)
+                assert (at % 16 == 0).all()
+                assert all(image[at[lane] // 16] == (lane, q) for lane in range(64))
+            # value bits: lane (h, b) stores the 32 rows of half h of kept value 2 g + b / 16 of column c, b % 16 = 4 g + c
+            b, half = LANE & 31, LANE >> 5
+            c = b & 3
+            column = 8 * (c_first + c) + 2 * ((b >> 2) & 3) + (b >> 4)
+            ok = c < c_count
+            bit = row0 + 32 * half + column * m
+            assert (bit % 32 == 0).all() and len(set(bit[ok])) == ok.sum()
+            inside(bit[ok] >> 3, 4, a_bytes, "pack: value bits")
+            # metadata, dword form: the lane of row r the even column of rows r and r + 4, that of row r + 4 the odd one
+            upper = (LANE >> 2) & 1
+            dst = row0 + ((((LANE >> 1) & 1) << 5) | ((LANE >> 3) << 2) | ((LANE & 1) << 1) | upper)
+            for c in range(0, c_count, 2):
+                dword = dst + ((c_first + c) >> 1) * m
+                inside(dword * 4, 4, e_bytes, "pack: metadata")
+                low_row = row0 + (LANE & ~4)
+                assert np.array_equal(2 * dword, meta_offset_reference(low_row, c_first + c + upper, m))
+                assert np.array_equal(2 * dword + 1, meta_offset_reference(low_row + 4, c_first + c + upper, m))
+            for c in range(c_count):
+                inside(meta_offset_reference(row0 + LANE, c_first + c, m) * 2, 2, e_bytes, "pack: metadata (general form)")
 
 
 # ---------------------------------------------------------------------------------------------------------------
@@ -69,22 +157,53 @@ def skinny_variant(n, rows, b_aligned=True, tokens=False):
     if nc == 64:
         r = min(r, 2)
     if tokens:
+        assert n <= 16
         mode = "tokens"
+    elif n == nc and b_aligned:
+        mode = "full"
     elif n == 1 and b_aligned:
         mode = "tokens"   # a k x 1 B is a token-major x of one token
     elif n in (2, 4) and b_aligned:
         mode = "run"      # a chunk's 256 rows as one run of 16-byte pieces
-    elif n == nc and b_aligned:
-        mode = "full"
-    elif nc > 16 and n % 8 == 0 and b_aligned:
-        mode = "b8"
-    elif nc == 16 and n == 8 and b_aligned:
-        mode = "b8"
-    elif nc == 16 and n == 4:
-        mode = "b4"
     else:
-        mode = "scalar"
+        mode = "any"      # 16-byte pieces wherever the rows start
     return nw, r, nc, mode
+
+
+def drop_halves(values, count):
+    """the eight values from number `count` on, zeros (-1) behind them"""
+    return [values[count + j] if count + j < 8 else -1 for j in range(8)]
+
+
+def check_any_image(n, k, nc, k_base):
+    """One image of the pieces at any alignment: every load inside B, and in the image every element below column n is the
+    element of B it stands for, or zero at or past K. An element of B is tracked by its number."""
+    img_rows, pieces = 8192 // (nc * 2), (n + 7) // 8
+    any_rows = 64 >> (pieces - 1) if nc == 16 else 64 // pieces
+    any_row = LANE >> (pieces - 1) if nc == 16 else LANE // pieces
+    any_piece = LANE & (pieces - 1) if nc == 16 else LANE % pieces
+    assert np.array_equal(any_row, LANE // pieces) and any_rows == 64 // pieces and np.array_equal(any_piece, LANE % pieces)
+    rows_left = min(k - k_base, img_rows + 8)
+    image = np.full((img_rows, nc), -2, dtype=np.int64)  # -2: what LDS held before
+    if rows_left <= 0:
+        return
+    last = (rows_left * n - 8) * 2
+    for i in range(8):
+        if i * any_rows >= img_rows:
+            continue
+        offset = (any_row * n + 8 * any_piece) * 2 + i * any_rows * n * 2
+        assert offset.max() < (1 << 32)
+        at = np.minimum(offset, last)
+        inside(k_base * n * 2 + at, 16, k * n * 2, "split-K kernel: B pieces")
+        for lane in range(64):
+            values = [k_base * n + at[lane] // 2 + j for j in range(8)]
+            if rows_left < img_rows + (0 if n % 8 == 0 else 8) and offset[lane] > last:
+                values = [-1] * 8 if n % 8 == 0 else drop_halves(values, (offset[lane] - last) // 2)
+            row = any_row[lane] + i * any_rows
+            if any_row[lane] < any_rows and row < img_rows:
+                image[row, 8 * any_piece[lane]:8 * any_piece[lane] + 8] = values
+    row, col = np.arange(img_rows)[:, None], np.arange(n)[None, :]
+    assert np.array_equal(image[:, :n], np.where(k_base + row < k, (k_base + row) * n + col, -1))
 
 
 def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1):
@@ -94,7 +213,8 @@ def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1
     sub = CHUNK_K // img_rows
     prep_size, b_size = prepared_bytes(m, k), k * n * 2
     grid = (rb_total + R - 1) // R
-    prefetch_b = nw <= 8 and mode != "scalar"
+    prefetch_b = nw <= 8 or mode == "run"
+    images = set()
     cps = (kc_total + splits - 1) // splits if splits > 1 else kc_total
     splits = (kc_total + cps - 1) // cps
     assert (splits - 1) * cps < kc_total  # the launcher's check: no empty split
@@ -108,7 +228,7 @@ def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1
         rb_first = wg * R
         kc_begin = split * cps
         kc_end = min(kc_begin + cps, kc_total)
-        short_k = nw <= 8 and sub == 1 and mode != "scalar" and kc_end - kc_begin <= 2 * nw
+        short_k = nw <= 8 and sub == 1 and kc_end - kc_begin <= 2 * nw
         for wave in range(nw):
             first = kc_begin + wave
             # --- prepared operand through one descriptor per row block
@@ -134,10 +254,12 @@ def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1
             # --- B images
             k_bases = []
             if short_k:
-                k_bases += [first * CHUNK_K, (first + nw) * CHUNK_K]
+                k_bases.append(first * CHUNK_K)
+                if mode != "any" or first + nw < kc_end:
+                    k_bases.append((first + nw) * CHUNK_K)
             else:
                 kc = first
-                if prefetch_b:
+                if prefetch_b and (nw <= 8 or first < kc_end):
                     k_bases.append(first * CHUNK_K)
                 while kc < kc_end:
                     for s in range(sub):
@@ -169,7 +291,6 @@ def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1
                         assert np.array_equal(accessed, (token_lane + tpi * i < n) & (lane_off != 0xFFFFFF00))
                         inside(lane_off[accessed] + scalar_off, 16, b_size, "split-K kernel: x rows")
                     continue
-                q_all = LANE[None, :] + 64 * np.arange(8)[:, None]
                 if mode == "run":
                     # raw buffer loads of 16-byte pieces q = lane + 64 i < 32 n of the run that starts at k_base * n * 2
                     pieces = 32 * n
@@ -194,23 +315,13 @@ def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1
                         inside(k_base * nc * 2 + LANE[None, :] * 16 + 1024 * np.arange(8)[:, None], 16, b_size,
                                "split-K kernel: whole B image")
                     else:
-                        ppr = nc // 8
-                        ok = (q_all // ppr) < rows_valid
-                        inside((k_base * nc + q_all[ok] * 8) * 2, 16, b_size, "split-K kernel: B image pieces")
-                elif mode == "b8":
-                    ppr = nc // 8
-                    row, h = q_all // ppr, q_all % ppr
-                    use = (row < rows_valid) & (8 * h < n)
-                    inside(((k_base + row[use]) * n + 8 * h[use]) * 2, 16, b_size, "split-K kernel: padded B pieces")
-                elif mode == "b4":
-                    ppr = nc // 8
-                    row, h = q_all // ppr, q_all % ppr
-                    use = (row < rows_valid) & (h == 0)
-                    inside((k_base + row[use]) * 8, 8, b_size, "split-K kernel: 8-byte B rows")
-                else:  # element copies
-                    valid = rows_valid * n
-                    e = np.arange(img_rows * n)
-                    inside((k_base * n + e[e < valid]) * 2, 2, b_size, "split-K kernel: B elements")
+                        q = LANE[None, :] + 64 * np.arange(8)[:, None]
+                        ok = (q // (nc // 8)) < rows_valid
+                        inside((k_base * nc + q[ok] * 8) * 2, 16, b_size, "split-K kernel: B image pieces")
+                elif k_base not in images:  # (the same for every row group)
+                    images.add(k_base)
+                    if len(images) <= 24 or k - k_base < 2 * CHUNK_K:
+                        check_any_image(n, k, nc, k_base)
         # --- result: rows of the workgroup's row blocks, columns below n
         rows_out = np.arange(rb_first * 32, min((rb_first + R) * 32, m))
         cols = np.arange(n)
@@ -349,6 +460,42 @@ def check_wide(m, n, k, rows, columns, splits, tokens=False, pad_b=False, d_size
                 inside((split * m * n * (splits > 1) + at) * elem, elem, splits * m * n * elem, "wide_kernel: results")
     if splits > 1:
         check_reduce(m, n, splits, d_size)
+    if pad_b:
+        check_pad_b(n, k)
+
+
+def check_pad_b(n, k):
+    """pad_b_kernel: every load inside B, every piece of the copy written once with the elements it stands for"""
+    per_row = (n + 7) // 8
+    ldb, rows = 8 * per_row, 1024 // per_row if 1 < per_row < 1024 else 1
+    reciprocal = ((1 << 32) // per_row + 1) & 0xFFFFFFFF
+    last_start, local = k * n - 8, np.arange(1024, dtype=np.int64)
+    if rows > 1:
+        assert np.array_equal((local * reciprocal) >> 32, local // per_row)
+    grid_x, grid_y = (k + rows - 1) // rows, (per_row + 1023) // 1024
+    written = 0
+    for x in sorted({0, 1, grid_x // 2, grid_x - 2, grid_x - 1} & set(range(grid_x))):
+        for y in range(grid_y):
+            r = (local * reciprocal) >> 32 if rows > 1 else 0 * local
+            col, row = 8 * (y * 1024 + local - r * per_row), x * rows + r
+            start = row * n + col
+            at = np.minimum(start, last_start)
+            inside(at * 2, 16, k * n * 2, "pad_b: source")
+            stored = (r < rows) & (row < k) & (col < ldb)
+            written += stored.sum()
+            inside((row[stored] * ldb + col[stored]) * 2, 16, k * ldb * 2, "pad_b: destination")
+            assert len(set(row[stored] * ldb + col[stored])) == stored.sum()
+            for j in np.flatnonzero(stored)[[0, -1]] if stored.any() else ():
+                values = [at[j] + e for e in range(8)]
+                if start[j] > last_start:
+                    values = drop_halves(values, start[j] - last_start) if start[j] - last_start < 8 else [-1] * 8
+                assert all(values[e] == row[j] * n + col[j] + e for e in range(min(8, n - col[j])))
+            wide = (start > last_start) & stored  # each of the shifted pieces
+            for j in np.flatnonzero(wide):
+                values = drop_halves([at[j] + e for e in range(8)], min(8, start[j] - last_start))
+                assert all(values[e] == row[j] * n + col[j] + e for e in range(min(8, n - col[j])))
+    if grid_x <= 5:
+        assert written == k * per_row
 
 
 def check_reduce(m, n, splits, d_size):
@@ -473,14 +620,8 @@ def check_gemm(m, n, k, tile, splits, pad_b, tokens=False, b_aligned=True, d_siz
                 inside(slice0 + (rows_out[:, None] * n + cols_out[None, :]) * elem, elem, total, "main kernel: D")
     if splits > 1:
         check_reduce(m, n, splits, d_size)
-    if pad_b:  # pad_b_kernel: one thread per 16-byte piece of the padded copy
-        pieces_per_row = ldb // 8
-        piece = np.arange(k * pieces_per_row, dtype=np.int64)
-        row, col0 = piece // pieces_per_row, (piece % pieces_per_row) * 8
-        for j in (0, 7):
-            ok = col0 + j < n
-            inside((row[ok] * n + col0[ok] + j) * 2, 2, k * n * 2, "pad_b: source")
-        inside((row * ldb + col0) * 2, 16, k * ldb * 2, "pad_b: destination")
+    if pad_b:
+        check_pad_b(n, k)
 
 
 def check_call(m, n, k, tokens=False, b_aligned=True):
@@ -510,6 +651,27 @@ def hooks():
 @pytest.mark.parametrize("m,k", [(64, 32), (512, 512), (8192, 8192), (11008, 4096), (4096, 11008), (8192, 28672), (25600, 25600)])
 def test_prepare_kernel_addresses(m, k):
     check_prepare(m, k)
+
+
+@pytest.mark.parametrize("m,k", [(64, 32), (64, 64), (512, 512), (192, 1056), (11008, 4096), (28672, 8192)])
+@pytest.mark.parametrize("size", [2, 4])
+def test_pack_kernel_addresses(m, k, size):
+    check_pack(m, k, size)
+
+
+@pytest.mark.parametrize("k", [32, 96, 256, 288, 512])
+def test_pieces_at_any_alignment(k):
+    """every column count of the images; K that ends inside an image, at its end and before it"""
+    for n in range(1, 65):
+        nc = 64 if n > 32 else 32 if n > 16 else 16
+        for k_base in range(0, 512, 8192 // (nc * 2)):
+            check_any_image(n, k, nc, k_base)
+
+
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 17, 63, 66, 99, 119, 1001, 8185, 8200])
+@pytest.mark.parametrize("k", [32, 96, 992])
+def test_padded_copy_addresses(n, k):
+    check_pad_b(n, k)
 
 
 @pytest.mark.parametrize("n", [17, 24, 40, 56, 65, 72, 104, 257])
