@@ -403,12 +403,22 @@ bool wide_is_faster(const WidePlan& wide, const LaunchPlan& launch, int n, int k
   return wide.us < 0.81 * launch.model_us;
 }
 
-// Least K splits of wide_kernel in the place of `launch`: two where that splits K over 128-row groups (10241 to 16384 rows) and
-// the workgroups' copies of x are long. Its model has the unsplit plan on 64-row groups ahead there by up to 10 %, measured it
-// is up to 16 % behind (us, unsplit | split in two: 11008 x 28672 with 24 and 32 tokens 30.1 | 27.4, 34.7 | 29.5, 14336 x 24576
-// with 32 31.0 | 27.3; below the line 11008 x 20480 with 17 19.7 | 21.4, with 24 22.1 | 22.0).
-int wide_least_splits(const LaunchPlan& launch, int n, int k) {
-  return launch.split_k_kernel && launch.splits > 1 && launch.rows_or_tile == 128 && (long)k * n >= 480000 ? 2 : 1;
+// Least K splits of wide_kernel in the place of a `launch` that splits K, up to 64 columns: its model, fitted to weights that lie
+// in the Infinity Cache, has the unsplit plan ahead too often when they come from HBM.
+// Plain form (us with weights from HBM, that kernel's split plan | wide_kernel unsplit | in two): 4096 x 11008 with 24 columns
+// 10.9 | 11.2 | 10.6, 2048 x 9600 with 24 and 32 10.2 | 10.5 | 9.6 and 9.6 | 11.3 | 9.2, 4096 x 9600 with 64 14.0 | 14.9 | 13.1,
+// 2048 x 8192 with 32 9.0 | 9.5 | 8.3; unsplit allowed at 8192 x 8192 with 64 16.5 | 14.3 | 15.4, 4096 x 8192 with 24 9.9 | 9.1 | 9.1.
+// Token-major form, whose images cost less: split where that kernel splits over 128-row groups (10241 to 16384 rows) and the
+// workgroups' copies of x are long (11008 x 28672 with 24 and 32 tokens 27.6 | 30.1 | 27.4 and 30.3 | 34.7 | 29.5, not 11008 x
+// 20480 with 17 20.7 | 19.7 | 21.4), and where it splits a very long K three times or more (5120 x 13824 with 17 tokens
+// 11.4 | 12.2 | 11.7, in three 10.8).
+int wide_least_splits(const LaunchPlan& launch, int n, int k, bool plain) {
+  if (launch.splits <= 1 || n > onebit::kSkinnyMaxN) return 1;
+  const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
+  if (plain) return chunks > 32 || (n > 24 && n <= 32) ? 2 : 1;
+  if (!launch.split_k_kernel) return 1;
+  if (launch.rows_or_tile == 128) return (long)k * n >= 480000 ? 2 : 1;
+  return n <= 32 && launch.splits >= 3 && chunks >= 50 ? 2 : 1;
 }
 
 // The linear layer's plan: wide = wide_kernel with `wide_plan`, else `launch` as for a product with an aligned B.
@@ -427,7 +437,7 @@ LinearPlan plan_linear(int m, int tokens, int k, int compute_units) {
   const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
   if (!plan.launch.split_k_kernel && g_tile_config >= 0) return plan;
   if (tokens > onebit::kSkinnyMaxN && groups[2] * ((tokens + 63) / 64) > 2L * compute_units) return plan;
-  plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, false, wide_least_splits(plan.launch, tokens, k),
+  plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, false, wide_least_splits(plan.launch, tokens, k, false),
                              plan.launch.splits, compute_units);
   plan.wide = plan.launch.split_k_kernel || wide_is_faster(plan.wide_plan, plan.launch, tokens, k);
   return plan;
@@ -442,16 +452,19 @@ LinearPlan plan_linear(int m, int tokens, int k, int compute_units) {
 WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b_readable, int compute_units) {
   WidePlan none{0, 1, 0, 0.0};
   const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
-  // 32 columns, whole rows of an image: skinny_kernel is as fast or faster in one round of 128-row groups, and where K is so short
-  // that its chunks do not fill a round of the sixteen wavefronts of its 32-row groups (us, skinny_kernel | wide_kernel:
-  // 20480 x 4096 10.4 | 11.2, 28672 x 5536 14.2 | 15.0, 11008 x 20480 in two splits 22.9 | 23.5, 2048 x 1056 3.71 | 3.85;
-  // 4096 x 4096 5.55 | 5.17, 40960 x 4096 19.7 | 16.6)
+  // 32 columns, whole rows of an image: skinny_kernel is as fast or faster in one round of 128-row groups, in its split plans
+  // from 3073 rows on, and where K is so short that its chunks do not fill a round of the sixteen wavefronts of its 32-row
+  // groups (us, skinny_kernel | wide_kernel: 20480 x 4096 10.4 | 11.2, 28672 x 5536 14.2 | 15.0, 11008 x 20480 22.9 | 23.5;
+  // 4096 x 11008 10.5 | 11.1, 5120 x 8192 10.2 | 10.7, 2048 x 9600 9.5 | 8.3; 2048 x 1056 3.71 | 3.85; 4096 x 4096 5.55 | 5.17,
+  // 40960 x 4096 19.7 | 16.6)
   if (n == 32 && g_skinny_rows <= 0 && launch.split_k_kernel && groups[2] <= compute_units &&
-      (launch.rows_or_tile == 128 || (launch.rows_or_tile == 32 && launch.splits == 1 && k <= 5 * onebit::kChunkK)))
+      (launch.rows_or_tile == 128 || (launch.splits > 1 ? groups[0] * 8 > 3L * compute_units
+                                                        : launch.rows_or_tile == 32 && k <= 5 * onebit::kChunkK)))
     return none;
   if (n <= 16 || !g_skinny_enabled || g_tile_config >= 0 || groups[2] * ((n + 63) / 64) > 2L * compute_units) return none;
   if (!b_readable) return none;
-  const WidePlan plan = plan_wide(groups, (double)m * n, n, k, true, wide_least_splits(launch, n, k), launch.splits, compute_units);
+  const WidePlan plan = plan_wide(groups, (double)m * n, n, k, true, wide_least_splits(launch, n, k, true), launch.splits,
+                                  compute_units);
   if (plan.us == 1e30 || (!launch.split_k_kernel && !wide_is_faster(plan, launch, n, k))) return none;
   return plan;
 }
