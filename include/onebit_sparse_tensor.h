@@ -121,8 +121,10 @@ int onebit_sparse_linear_prepared(const void *prepared, const void *x, const voi
  * gate / up: onebit_sparse_mul/__init__.py:118-128 called once per projection): with tokens <= 64 every 16 problems are
  * one launch of the split-K kernel, whose workgroups are numbered over the concatenated row groups of the problems, so
  * that the launch and the start of the memory stream are paid once instead of per projection (decode-sized products
- * take a few microseconds each, half of which is that). Results are identical to `count` calls of
- * onebit_sparse_linear_prepared without a K split over workgroups (same sums in the same order per element). With
+ * take a few microseconds each, half of which is that). Results are those of `count` calls of
+ * onebit_sparse_linear_prepared up to the order of the fp32 sums: the launch never splits K over workgroups, up to 16
+ * tokens its row group, and with it the number of wavefronts that split K, follows the rows of all its problems, and
+ * beyond 40960 rows a single call of 33 to 64 tokens may run the main kernel. With
  * tokens > 64 it is exactly such a sequence of calls. bias_dtype and y_dtype hold for all problems. No counterpart in
  * the reference (one launch per product, csrc/kernel_lib.cu:86); allocates nothing.
  */

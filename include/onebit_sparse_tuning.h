@@ -20,16 +20,16 @@ extern "C" {
  * does not change what another thread launches (worker threads of a data-parallel wrapper, autograd threads). */
 void onebit_sparse_set_tile_config(int tile_config);
 void onebit_sparse_set_skinny_enabled(int enabled);
-/* Weight rows one workgroup of the split-K kernel covers: 32, 64 or 128; <= 0 = automatic. */
+/* Weight rows one workgroup of the split-K kernels covers: 32, 64 or 128; <= 0 = automatic. */
 void onebit_sparse_set_skinny_rows(int rows);
-/* K splits over workgroups, of the main kernel and of the split-K kernel (which also splits K among the wavefronts
+/* K splits over workgroups, of the main kernel and of the split-K kernels (which also split K among the wavefronts
  * of a workgroup): 1 = never split, N > 1 = N splits (at most one per 256 of K), <= 0 = automatic (few tiles or row
  * groups and a long K). A split call writes fp32 partial sums to a library-owned buffer kept per
  * device and stream (grown with hipMalloc on first use: warm up before capturing the call in a HIP graph) and adds
  * them in split order, so results do not depend on timing. */
 void onebit_sparse_set_split_k(int splits);
 /* B whose rows are not 16-byte aligned (n % 8 != 0 or an unaligned base) and n beyond the split-K kernel's range:
- * 1 (default) = the main kernel reads a copy of B with rows padded to a multiple of 8 columns, made by one extra
+ * 1 (default) = the kernel reads a copy of B with rows padded to a multiple of 8 columns, made by one extra
  * pass into a library-owned buffer kept per device and stream (same rules as the K-split buffer); 0 = the main
  * kernel's element-copy variant reads B in place (much slower). With k * n < 65536 the copy is made where its buffer is there
  * or can be allocated: not by the non-allocating entry point, and in a stream capture only after a warm-up. */

@@ -1,5 +1,5 @@
 // C ABI of libonebitmul (declared in include/onebit_sparse_tensor.h): argument validation, per-device
-// workspaces, kernel selection. Host code only; the kernels live in onebit_gemm*, onebit_skinny* and
+// workspaces, kernel selection. Host code only; the kernels live in onebit_gemm*, onebit_skinny*, onebit_wide* and
 // onebit_format.hip.
 // Counterpart of the reference's host launcher csrc/kernel_lib.cu:23-97.
 #include "onebit_sparse_tuning.h"

@@ -32,7 +32,7 @@ constexpr int kSkinnyRegion = 8192;  // bytes of one B image
 // the result is written as y[token][weight row] (+ bias[weight row]). The image is then token-major too: row t holds
 // the image's K range of token t in 16-byte pieces, piece p stored at position p ^ token_swizzle(t) so that lanes
 // which read the same piece of consecutive tokens fall into different banks; a lane's SMFMAC operand is two plain
-// 16-byte reads (K consecutive inside a piece), no transpose. Up to sixteen tokens; more go to wide_tokens_kernel.
+// 16-byte reads (K consecutive inside a piece), no transpose. Up to sixteen tokens; more go to wide_kernel.
 // kSkinnyBRun: n = 2 or 4 with B 16-byte aligned. The 256 rows of a chunk are one run of 512 n consecutive bytes,
 // loaded in 16-byte pieces (32 n of them: at most two load instructions per wavefront and chunk, where the row-wise
 // modes issue eight; the split-K kernel's time is set by the number of load instructions it issues) and spread over the image rows

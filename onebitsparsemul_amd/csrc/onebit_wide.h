@@ -8,7 +8,9 @@
 namespace onebit {
 
 // =====================================================================================================
-// wide_tokens_kernel: y[t][r] = sum_k W[r][k] x[t][k] + bias[r] for up to 64 tokens.
+// wide_kernel: y[t][r] = sum_k W[r][k] x[t][k] + bias[r] (token-major form) and D = alpha A B + beta C (plain form) for 17
+// tokens or columns and more, in groups of up to 64 per workgroup (grid.z). The plain form differs in how an image lies in LDS
+// and is read (see wide_body) and in the epilogue; below, x and token stand for B and column too.
 // Workgroup = eight wavefronts that share R row blocks (32 rows each) and split K among themselves chunk by chunk, as in
 // skinny_kernel. What differs is how x gets to the matrix cores: every wavefront keeps a ring of two images (64 K values of
 // all tokens, 2 KB per sixteen) in LDS that asynchronous copies fill. No registers hold x on its way, so the tile can be
@@ -20,6 +22,7 @@ namespace onebit {
 // now: 28672 x 8192 with 24 / 48 / 64 tokens 16.6 / 33.4 / 35.9 -> 16.6 / 21.0 / 24.5; 11008 x 4096 8.0 / 11.0 / 11.7 -> 6.8 /
 // 8.3 / 9.6; 4096 x 4096 5.7 / 8.4 / 8.7 -> 4.7 / 6.0 / 7.1; 1024 x 1024 with 56 5.0 -> 3.5. Up to sixteen tokens there is no
 // gain (11008 x 4096 with 16: 6.4 -> 6.1, with 4: 5.5 -> 5.8; 28672 x 8192 with 16: 13.5 -> 14.0): skinny_kernel keeps those.
+// Beyond 64 tokens, and for products, the host's plan compares it with the kernel it would replace (onebit_capi.hip).
 // =====================================================================================================
 // Source of zeros for the copies of K positions at or past K.
 static __device__ __attribute__((aligned(16))) uint32_t g_zero16_wide[4] = {0, 0, 0, 0};
