@@ -397,9 +397,11 @@ LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int comput
 // K, from which on wide_kernel is faster at 45056 to 262144 rows (us, wide | main, 48 and 64 tokens: 65536 x 1024 17.0 | 12.0 and
 // 19.0 | 12.4, x 4096 28.5 | 31.4 and 32.8 | 31.8, x 8192 44.1 | 60.2 and 50.1 | 60.5; 45056 x 3616 25.4 | 23.9, x 4096
 // 23.5 | 25.1). With k % 64 != 0, where every second token's pieces straddle two lines, it lies twice as far out (45056 x 4128
-// with 48 tokens 28.6 | 26.8, x 8224 43.4 | 47.9).
+// with 48 tokens 28.6 | 26.8, x 8224 43.4 | 47.9). Where the main kernel would split K,
+// wide_kernel in any case (41024 x 7936 and x 8160, 56 and 64 tokens: 46.6 to 49.6 against 53.8 to 56).
 bool wide_is_faster(const WidePlan& wide, const LaunchPlan& launch, int n, int k) {
-  if (n <= onebit::kSkinnyMaxN) return (k + onebit::kChunkK - 1) / onebit::kChunkK >= (n <= 48 ? 16 : 32) * (k % 64 ? 2 : 1);
+  if (n <= onebit::kSkinnyMaxN)
+    return launch.splits > 1 || (k + onebit::kChunkK - 1) / onebit::kChunkK >= (n <= 48 ? 16 : 32) * (k % 64 ? 2 : 1);
   return wide.us < 0.81 * launch.model_us;
 }
 
