@@ -456,12 +456,12 @@ WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b
   const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
   // 32 columns, whole rows of an image: skinny_kernel is as fast or faster in one round of 128-row groups, in its split plans
   // from 3073 rows on, and where K is so short that its chunks do not fill a round of the sixteen wavefronts of its 32-row
-  // groups (us, skinny_kernel | wide_kernel: 20480 x 4096 10.4 | 11.2, 28672 x 5536 14.2 | 15.0, 11008 x 20480 22.9 | 23.5;
-  // 4096 x 11008 10.5 | 11.1, 5120 x 8192 10.2 | 10.7, 2048 x 9600 9.5 | 8.3; 2048 x 1056 3.71 | 3.85; 4096 x 4096 5.55 | 5.17,
-  // 40960 x 4096 19.7 | 16.6)
+  // groups, one per compute unit (us, skinny_kernel | wide_kernel: 20480 x 4096 10.4 | 11.2, 28672 x 5536 14.2 | 15.0, 11008 x
+  // 20480 22.9 | 23.5; 4096 x 11008 10.5 | 11.1, 5120 x 8192 10.2 | 10.7, 2048 x 9600 9.5 | 8.3; 2048 x 1056 3.71 | 3.85, but in
+  // two rounds of workgroups 9920 x 992 5.6 | 4.1, 8512 x 1088 6.3 | 4.8; 4096 x 4096 5.55 | 5.17, 40960 x 4096 19.7 | 16.6)
+  const bool one_short_round = launch.rows_or_tile == 32 && k <= 5 * onebit::kChunkK && groups[0] <= compute_units;
   if (n == 32 && g_skinny_rows <= 0 && launch.split_k_kernel && groups[2] <= compute_units &&
-      (launch.rows_or_tile == 128 || (launch.splits > 1 ? groups[0] * 8 > 3L * compute_units
-                                                        : launch.rows_or_tile == 32 && k <= 5 * onebit::kChunkK)))
+      (launch.rows_or_tile == 128 || (launch.splits > 1 ? groups[0] * 8 > 3L * compute_units : one_short_round)))
     return none;
   if (n <= 16 || !g_skinny_enabled || g_tile_config >= 0 || groups[2] * ((n + 63) / 64) > 2L * compute_units) return none;
   if (!b_readable) return none;

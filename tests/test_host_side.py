@@ -162,7 +162,8 @@ def test_product_is_not_split_because_the_plan_it_replaces_is(fresh, m, n, k):
 @pytest.mark.parametrize("m,k,kernel", [(20480, 4096, "skinny_kernel"), (28672, 5536, "skinny_kernel"), (2048, 1056, "skinny_kernel"),
                                         (11008, 28672, "skinny_kernel"), (4096, 11008, "skinny_kernel"), (5120, 8192, "skinny_kernel"),
                                         (2048, 11008, "wide_kernel"),
-                                        (4096, 4096, "wide_kernel"), (40960, 4096, "wide_kernel"), (11008, 1056, "wide_kernel")])
+                                        (4096, 4096, "wide_kernel"), (40960, 4096, "wide_kernel"), (11008, 1056, "wide_kernel"),
+                                        (8192, 992, "skinny_kernel"), (8256, 992, "wide_kernel"), (9920, 992, "wide_kernel")])
 def test_kernel_of_32_columns(fresh, m, k, kernel):
     assert product(fresh, m, 32, k) == 0
     assert last_launch(fresh)["kernel"] == kernel
