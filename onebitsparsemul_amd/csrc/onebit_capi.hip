@@ -329,10 +329,15 @@ WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, 
   // plain form, several column groups: a group's piece of a row of B is a part of a line, 32 to 128 bytes (4096 x 64 x 4096 in
   // four groups 11.0 us against 5.8 token-major, in two 7.1 against 5.1)
   static const double kColumns[4] = {2.3, 1.45, 1.4, 1.1};
+  // and beyond 64 columns, with rows of B that begin inside a line, every round from the third on costs more (512 x 160 x 10112
+  // in five rounds of 32-row groups 15.3 us, with K in three 11.0; up to 64 columns, where B is small, not: 1280 x 56 x 7520 in
+  // two groups 10.4, in one 12.9)
+  static const double kFurther[3] = {0.18, 0.06, 0.0};
+  const bool cut_lines = n > onebit::kSkinnyMaxN && n % 64;
   // The row groups that multiply one token group run on different XCDs, and each XCD fetches its own copy of x: with more x
   // than fits an XCD's L2 (4 MB) that is what a launch of few rows waits for (us measured | modelled without it:
   // 896 x 24256 x 704 45 | 29, 1088 x 13888 x 1758 62 | 38, 640 x 17536 x 676 30 | 19; the main kernel takes 29, 41 and 21).
-  constexpr double kFetchBytesPerUs = 6.3e6;
+  constexpr double kFetchBytesPerUs = 5.6e6;
   const double xcds = std::max(1, compute_units / 32);
   const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
   WidePlan best{g_skinny_rows > 0 ? g_skinny_rows : 32, 1, std::min(n, onebit::kSkinnyMaxN), 1e30};
@@ -349,11 +354,13 @@ WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, 
         const int rounds = ((chunks + s - 1) / s + 7) / 8;
         const double load = (double)total_groups[r] * groups * s / compute_units;
         const double work = rounds * kRound[r][tiles - 1] * (1.0 + kLoad[r][tiles - 1] * std::min(1.0, load)) *
-                            (plain ? (groups > 1 ? kColumns[tiles - 1] : 1.0) : k % 64 ? kSplitLines[r] : 1.0);
+                            (!plain       ? (k % 64 ? kSplitLines[r] : 1.0)
+                             : groups > 1 ? kColumns[tiles - 1] * (cut_lines ? 1.0 + kFurther[r] * std::max(0, rounds - 2) : 1.0)
+                                          : 1.0);
         double us = kBase[r][tiles - 1] + work;
         if (load > 1.0)
           us += (std::ceil(load) - 1.0) * (work * kAgain[r][tiles - 1] + (kBase[r][tiles - 1] - 1.5) * (r < 2 ? 0.4 : 1.0));
-        us = std::max(us, 3.5 + std::min((double)total_groups[r], xcds) * n * k * 2.0 / kFetchBytesPerUs);
+        us = std::max(us, 3.0 + std::min((double)total_groups[r], xcds) * n * k * 2.0 / kFetchBytesPerUs);
         if (s > 1) us += 2.6 + 0.15 * s + (s + 1) * 4.0 * results / 5.0e6;
         if (us < best.us) best = WidePlan{kWideRows[r], s, tokens, us};
         if (g_split_k >= 1 || s == most_splits) break;
@@ -387,11 +394,14 @@ LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int comput
   return plan;
 }
 
-// wide_kernel against the main kernel. Both models err, the main kernel's mostly upwards (by half at worst), so the line lies
-// where calls that cross it are not slower. Measured on 260 layer calls and 188 products of 512 to 65536 rows, k = 512 to 28672
-// and 65 to 2048 columns whose two models lie within a factor of two: the 213 below 0.81 are 1.53 times as fast as on the main
-// kernel in the mean and the slowest within 2 %; of the 56 between 0.81 and 0.88 ten are slower, by up to 21 % (2496 x 19648 with
-// 197 tokens; 20864 x 7616 with 152 columns, at 0.82, 52 us against 48).
+// wide_kernel against the main kernel. Both models err, and by how much depends on the plans. Measured on 13000 calls of 512 to
+// 28672 rows, k = 512 to 28672 and 65 to 2048 columns (measured / modelled, median): the main kernel's 256 x 128 tile 0.80 for
+// layers and 0.90 for products, its others 0.91 to 1.05; wide_kernel 0.8 to 0.95 where K is one round of its wavefronts, 1.0 to
+// 1.1 on longer K, and 1.0 where it splits K. The lines lie where about as few calls are slower on either side: timed again on
+// 4000 other calls whose modelled times are 0.55 to 1.1 of one another, 25 are more than 5 % slower than on the main kernel, and
+// all are 1.23 times as fast in the mean. One line for all does worse: at 0.81 short K loses (3648 x 992 with 181 tokens 5.6 us,
+// 6.6 on the main kernel; 2176 x 512 with 184 3.8 and 5.2), at 0.88 2496 x 19648 with 197 tokens was 21 % slower than there, and
+// 20864 x 7616 with 152 columns 52 us against 48.
 // Up to 64 columns the main kernel is the other plan beyond 40960 rows only, where a wavefront of wide_kernel has one short round
 // of work per workgroup and the workgroups come in many rounds, outside what its model was fitted to: the line is the length of
 // K, from which on wide_kernel is faster at 45056 to 262144 rows (us, wide | main, 48 and 64 tokens: 65536 x 1024 17.0 | 12.0 and
@@ -399,10 +409,15 @@ LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int comput
 // 23.5 | 25.1). With k % 64 != 0, where every second token's pieces straddle two lines, it lies twice as far out (45056 x 4128
 // with 48 tokens 28.6 | 26.8, x 8224 43.4 | 47.9). Where the main kernel would split K,
 // wide_kernel in any case (41024 x 7936 and x 8160, 56 and 64 tokens: 46.6 to 49.6 against 53.8 to 56).
-bool wide_is_faster(const WidePlan& wide, const LaunchPlan& launch, int n, int k) {
-  if (n <= onebit::kSkinnyMaxN)
-    return launch.splits > 1 || (k + onebit::kChunkK - 1) / onebit::kChunkK >= (n <= 48 ? 16 : 32) * (k % 64 ? 2 : 1);
-  return wide.us < 0.81 * launch.model_us;
+bool wide_is_faster(const WidePlan& wide, const LaunchPlan& launch, int n, int k, bool plain) {
+  const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
+  if (n <= onebit::kSkinnyMaxN) return launch.splits > 1 || chunks >= (n <= 48 ? 16 : 32) * (k % 64 ? 2 : 1);
+  const double line = wide.splits > 1                                 ? 0.92
+                      : launch.rows_or_tile == onebit::kTile256x128w8 ? 0.81
+                      : plain                                         ? 0.85
+                      : launch.splits > 1                             ? 0.87
+                                                                      : 0.88;
+  return wide.us < line * launch.model_us;
 }
 
 // Least K splits of wide_kernel in the place of a `launch` that splits K, up to 64 columns: its model, fitted to weights that lie
@@ -441,7 +456,7 @@ LinearPlan plan_linear(int m, int tokens, int k, int compute_units) {
   if (tokens > onebit::kSkinnyMaxN && groups[2] * ((tokens + 63) / 64) > 2L * compute_units) return plan;
   plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, false, wide_least_splits(plan.launch, tokens, k, false),
                              plan.launch.splits, compute_units);
-  plan.wide = plan.launch.split_k_kernel || wide_is_faster(plan.wide_plan, plan.launch, tokens, k);
+  plan.wide = plan.launch.split_k_kernel || wide_is_faster(plan.wide_plan, plan.launch, tokens, k, false);
   return plan;
 }
 
@@ -467,7 +482,7 @@ WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b
   if (!b_readable) return none;
   const WidePlan plan = plan_wide(groups, (double)m * n, n, k, true, wide_least_splits(launch, n, k, true), launch.splits,
                                   compute_units);
-  if (plan.us == 1e30 || (!launch.split_k_kernel && !wide_is_faster(plan, launch, n, k))) return none;
+  if (plan.us == 1e30 || (!launch.split_k_kernel && !wide_is_faster(plan, launch, n, k, true))) return none;
   return plan;
 }
 

@@ -145,7 +145,8 @@ def test_calls_that_the_main_kernel_multiplies_faster(fresh, call, m, n, k):
 @pytest.mark.parametrize("call,m,n,k", [(layer, 4096, 500, 11008), (layer, 5312, 278, 18944), (layer, 1024, 256, 4096),
                                         (layer, 4096, 128, 4096), (product, 4096, 256, 4096), (layer, 131072, 48, 4096),
                                         (layer, 65536, 64, 8192), (layer, 40960, 64, 512), (layer, 41024, 64, 7936),
-                                        (layer, 41024, 56, 8160)])
+                                        (layer, 41024, 56, 8160), (layer, 3648, 181, 992), (layer, 2176, 184, 512),
+                                        (layer, 2304, 536, 5024)])
 def test_calls_that_wide_kernel_multiplies_faster(fresh, call, m, n, k):
     assert call(fresh, m, n, k) == 0
     assert last_launch(fresh)["kernel"] == "wide_kernel"
