@@ -213,9 +213,10 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
         const uint32_t offset = any_load + i * any_load_step;
         v[i] = *reinterpret_cast<const u32x4_any_t*>(image + (offset < last ? offset : last));
       }
-    // whole pieces: every piece of a row that exists ends inside it. Asked with sixteen-column images only: a test at run time
-    // makes the wider ones slower (us, with and without it: 19456 x 20 x 8672 24.9 | 19.6, 896 x 30 x 9152 10.6 | 9.1)
-    const bool whole_pieces = NC == 16 && n_cols % 8 == 0;
+    // whole pieces: every piece of a row that exists ends inside it. Asked with sixteen wavefronts and sixteen-column images
+    // only: a test at run time makes the others slower (us, with and without it: 19456 x 20 x 8672 24.9 | 19.6, 896 x 30 x 9152
+    // 10.6 | 9.1; eight columns on 64-row groups 8 % in the median of long K)
+    const bool whole_pieces = NC == 16 && NW == 16 && n_cols % 8 == 0;
     if (rows_left < IMG_ROWS + (whole_pieces ? 0 : 8)) {
       // last image: what was read from the last whole piece is shifted into place, rows at or past K are zeros
 #pragma unroll
