@@ -278,14 +278,19 @@ struct LaunchPlan {
 struct SkinnyPlan {
   int rows, splits;
 };
-SkinnyPlan plan_skinny(int m, int n, int k, int compute_units) {
+SkinnyPlan plan_skinny(int m, int n, int k, bool pieces, int compute_units) {
   const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
   const int forced_rows = g_skinny_rows, forced_splits = g_split_k;
   // the largest row group that still gives about two workgroups per three compute units (measured: larger groups
   // re-read B less often, but idle compute units cost more)
   // (n > 32: two column fragments per row block, at most two row blocks per wavefront)
+  // pieces: B in pieces at any alignment, up to sixteen columns. A workgroup of that mode has a compute unit to itself, so 64-row
+  // groups beyond one per compute unit wait for a second round: 128-row groups from there on (us, element copies | 64 | 128 rows:
+  // 18688 x 1280 with three columns 5.84 | 7.40 | 5.95, x 1760 6.77 | 7.66 | 6.06, x 8192 18.5 | 17.7 | 13.9; with twelve 9.7 | 7.4
+  // | 6.0)
   const int enough = std::max(1, 160 * compute_units / 256);
-  int rows = forced_rows > 0 ? forced_rows : (m / 128 >= enough && n <= 32) ? 128 : (m / 64 >= enough) ? 64 : 32;
+  const bool second_round = pieces && (m + 63) / 64 > compute_units;
+  int rows = forced_rows > 0 ? forced_rows : ((m / 128 >= enough && n <= 32) || second_round) ? 128 : (m / 64 >= enough) ? 64 : 32;
   if (forced_splits >= 1) return SkinnyPlan{rows, forced_splits > chunks ? chunks : forced_splits};
   const double image_row_bytes = n <= 16 ? 32.0 : n <= 32 ? 64.0 : 128.0;
   const double threshold = 400e3 * std::max(1.0, m / 4096.0);
@@ -370,14 +375,15 @@ WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, 
   return best;
 }
 
-LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int compute_units = 256) {
+LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int compute_units, bool tokens = false) {
   LaunchPlan plan{};
   // 32 < n <= 64: every 64-row workgroup of the split-K kernel stages all of B, which the main kernel's tiles overtake
   // from about 48k rows on (n = 64: 28672 x 8192 32 us against 42; 32768 x 4096 20 against 26; 49152 x 4096 32.5
   // against 34.4; 65536 x 8192 66 against 68, at n = 40 77 against 66; 131072 x 2048 51 against 35)
   const bool skinny_shape = n <= 32 || (n <= onebit::kSkinnyMaxN && m <= 40960);
   if (skinny_shape && g_skinny_enabled) {
-    const SkinnyPlan sk = plan_skinny(m, n, k, compute_units);
+    const bool pieces = !tokens && n <= 16 && !(b_16_byte_aligned && (n == 1 || n == 2 || n == 4 || n == 16));
+    const SkinnyPlan sk = plan_skinny(m, n, k, pieces, compute_units);
     plan.split_k_kernel = 1;
     plan.rows_or_tile = sk.rows;
     plan.splits = sk.splits;
@@ -449,7 +455,7 @@ struct LinearPlan {
 };
 LinearPlan plan_linear(int m, int tokens, int k, int compute_units) {
   LinearPlan plan{};
-  plan.launch = choose_launch(m, tokens, k, true, compute_units);
+  plan.launch = choose_launch(m, tokens, k, true, compute_units, true);
   if (tokens <= onebit::kSkinnyTokens || !g_skinny_enabled) return plan;
   const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
   if (!plan.launch.split_k_kernel && g_tile_config >= 0) return plan;

@@ -170,6 +170,14 @@ def test_kernel_of_32_columns(fresh, m, k, kernel):
     assert last_launch(fresh)["kernel"] == kernel
 
 
+@pytest.mark.parametrize("call,m,n,rows", [(product, 18688, 3, 128), (product, 16448, 12, 128), (product, 16384, 3, 64),
+                                           (product, 18688, 4, 64), (product, 18688, 1, 64), (layer, 18688, 3, 64)])
+def test_pieces_at_any_alignment_in_one_round(fresh, call, m, n, rows):
+    """64-row groups of that mode beyond one per compute unit took up to 22 % longer than the element copies before them."""
+    assert call(fresh, m, n, 1280) == 0
+    assert last_launch(fresh)["rows_or_tile"] == rows
+
+
 @pytest.mark.parametrize("call,m,n,k,split", [(layer, 11008, 32, 28672, True), (layer, 14336, 24, 24576, True),
                                               (product, 14336, 24, 28672, True), (layer, 11008, 17, 20480, False),
                                               (layer, 11008, 24, 11008, False), (layer, 5120, 17, 13824, True),
