@@ -15,9 +15,11 @@ LIB = os.path.join(PKG, "libonebitmul.so")
 STATIC_LIB = os.path.join(PKG, "libonebitmul.a")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-# -packed-fp32-ops is switched off for every device compile of this project.
+# -packed-fp32-ops is switched off for every device compile of this project. Leading scalar arguments of a kernel, up to
+# fourteen dwords, are in registers when a wavefront starts.
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Xclang", "-target-feature", "-Xclang",
-             "-packed-fp32-ops", "-Wno-unused-command-line-argument", "-I", INCLUDE, "-I", CSRC]
+             "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=14", "-Wno-unused-command-line-argument",
+             "-I", INCLUDE, "-I", CSRC]
 
 
 def _run(cmd):

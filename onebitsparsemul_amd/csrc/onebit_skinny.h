@@ -3,6 +3,7 @@
 #pragma once
 #include "onebit_device.h"
 #include "onebit_launch.h"
+#include <climits>
 #include <type_traits>
 
 namespace onebit {
@@ -339,6 +340,11 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
     return __builtin_bit_cast(half16_t, raw);
   };
   auto compute16 = [&](const AChunk (&a)[R]) __attribute__((always_inline)) {
+    // The compute unit serves the older half of the wavefronts first, when their loads are accepted and again when both of a
+    // SIMD's have work; from its first chunk on the younger half goes first, so that the two end closer together (us, without ->
+    // with, token-major form: 11008 x 4096 with 1 / 4 / 16 tokens 5.00 / 5.02 / 5.63 -> 4.87 / 4.88 / 5.56, 8192 x 8192 with 8
+    // 5.92 -> 5.66; the plain form no different, 4096 x 4 x 11008 6.83 -> 6.93).
+    if (TOKENS && wave >= NW / 2) __builtin_amdgcn_s_setprio(1);
     half16_t bf[4];
 #pragma unroll
     for (int F = 0; F < 4; ++F) bf[F] = frag16(F);
@@ -570,8 +576,44 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   }
 }
 
+// A kernel's arguments as three vectors. The hardware puts the first two, twelve dwords, into scalar registers before a
+// wavefront starts (the build asks for that); out of a struct they would have to be loaded, 0.2 us before the first address can
+// be formed. Vectors, because the host pays for every argument of a launch. us inside a HIP graph, weights from HBM, struct ->
+// this: 11008 x 4096 with 1 / 4 / 16 tokens 5.16 / 5.35 / 5.91 -> 5.00 / 5.02 / 5.63, 28672 x 8192 with one 12.5 -> 12.2,
+// 11008 x 3 x 4096 6.35 -> 6.08.
+enum ArgFlags : uint32_t { kArgD16 = 1, kArgC16 = 2, kArgBias = 4 };  // bits 3 and 4: type of the bias
+struct LaunchArgs {
+  u32x8_t operands;  // prep, b; n, k, m, chunks_per_split
+  u32x4_t results;   // d, the bias (token-major form) or C: a call has one of them at most
+  u32x4_t epilogue;  // ArgFlags, alpha, beta
+};
+static LaunchArgs pack_args(const SkinnyArgs& a) {
+  const uint64_t prep = (uint64_t)a.prep, b = (uint64_t)a.b, d = (uint64_t)a.d, extra = (uint64_t)(a.bias ? a.bias : a.c);
+  const uint32_t flags = (a.d_f16 ? kArgD16 : 0) | (a.c_f16 ? kArgC16 : 0) | (a.bias ? kArgBias : 0) | (uint32_t)a.bias_type << 3;
+  return LaunchArgs{u32x8_t{(uint32_t)prep, (uint32_t)(prep >> 32), (uint32_t)b, (uint32_t)(b >> 32), (uint32_t)a.n, (uint32_t)a.k,
+                            (uint32_t)a.m, (uint32_t)a.chunks_per_split},
+                    u32x4_t{(uint32_t)d, (uint32_t)(d >> 32), (uint32_t)extra, (uint32_t)(extra >> 32)},
+                    u32x4_t{flags, __builtin_bit_cast(uint32_t, a.alpha), __builtin_bit_cast(uint32_t, a.beta), 0u}};
+}
+__device__ __forceinline__ SkinnyArgs unpack_args(u32x8_t operands, u32x4_t results, u32x4_t epilogue) {
+  auto pointer = [](uint32_t low, uint32_t high) __attribute__((always_inline)) { return (uint64_t)high << 32 | low; };
+  SkinnyArgs p{};
+  p.prep = reinterpret_cast<const uint8_t*>(pointer(operands[0], operands[1]));
+  p.b = reinterpret_cast<const _Float16*>(pointer(operands[2], operands[3]));
+  p.n = operands[4]; p.k = operands[5]; p.m = operands[6]; p.chunks_per_split = operands[7];
+  p.kc_total = (p.k + kChunkK - 1) / kChunkK;
+  p.d = reinterpret_cast<void*>(pointer(results[0], results[1]));
+  p.c = reinterpret_cast<const void*>(pointer(results[2], results[3]));  // read where beta != 0 only: never with a bias
+  p.bias = epilogue[0] & kArgBias ? p.c : nullptr;
+  p.d_f16 = epilogue[0] & kArgD16; p.c_f16 = epilogue[0] & kArgC16; p.bias_type = epilogue[0] >> 3 & 3;
+  // (values, not elements: the compiler casts the bits of a vector's first element where an element is named)
+  p.alpha = __builtin_bit_cast(float, (uint32_t)epilogue[1]); p.beta = __builtin_bit_cast(float, (uint32_t)epilogue[2]);
+  return p;
+}
+
 template <int NW, int R, int MODE, int NC, bool BF16>
-__global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_kernel(SkinnyArgs p) {
+__global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_kernel(u32x8_t operands, u32x4_t results, u32x4_t epilogue) {
+  const SkinnyArgs p = unpack_args(operands, results, epilogue);
   skinny_body<NW, R, MODE, NC, BF16>(p, blockIdx.x, blockIdx.y);
 }
 
@@ -581,19 +623,80 @@ __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_kernel(Skinn
 // the token-major body on that problem's arguments. Decode-sized products take a few microseconds each, of which the
 // launch itself and the ramp of the memory pipeline are a large part: one launch for the q / k / v or gate / up
 // projections of a layer pays them once.
+// What decides about the problem comes in scalar registers, so that a workgroup of up to four problems waits for one load of 40
+// bytes where it walked through a table of first workgroups and then read its problem (us inside a HIP graph, before -> now:
+// 3 x 4096 x 4096 with eight tokens 6.18 -> 5.35, 4096 + 2 x 1024 4.57 -> 4.09, 2 x 11008 x 4096 with sixteen 9.02 -> 7.97).
+struct GroupProblem {
+  const uint8_t* prep;
+  const _Float16* b;
+  void* d;
+  const void* bias;
+  int m, k;
+};
+struct GroupTable {
+  GroupProblem problem[kSkinnyMaxGroup];
+  int first_block[kSkinnyMaxGroup];
+};
+struct GroupShared {  // the same for all problems (same_group_types)
+  int d_f16, bias_type, tokens_per_group;
+};
+
+// First workgroups of problems 1, 2 and 3 (INT_MAX where there is none), the number of problems, the token count; `problem`: of
+// this workgroup, `block`: its number among that problem's.
+__device__ __forceinline__ SkinnyArgs group_problem(int first1, int first2, int first3, int count, int tokens, const GroupShared& shared,
+                                                    const GroupTable& table, int& block) {
+  block = blockIdx.x;
+  int which = (block >= first1) + (block >= first2) + (block >= first3);
+  int first = block >= first3 ? first3 : block >= first2 ? first2 : block >= first1 ? first1 : 0;
+  for (int i = 4; i < count; ++i)
+    if (block >= table.first_block[i]) which = i, first = table.first_block[i];
+  const GroupProblem& q = table.problem[which];
+  SkinnyArgs p{};
+  p.prep = q.prep; p.b = q.b; p.d = q.d; p.bias = q.bias;
+  p.m = q.m; p.n = tokens; p.k = q.k;
+  p.kc_total = p.chunks_per_split = (q.k + kChunkK - 1) / kChunkK;
+  p.alpha = 1.f;
+  p.d_f16 = shared.d_f16; p.bias_type = shared.bias_type; p.tokens_per_group = shared.tokens_per_group;
+  block -= first;
+  return p;
+}
+
 template <int NW, int R, int NC, bool BF16>
-__global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_group_kernel(SkinnyGroupArgs g) {
-  int which = 0;
-  for (int i = 1; i < g.count; ++i)
-    if ((int)blockIdx.x >= g.first_block[i]) which = i;
-  skinny_body<NW, R, kSkinnyBTokens, NC, BF16>(g.problem[which], (int)blockIdx.x - g.first_block[which], 0);
+__global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_group_kernel(int first1, int first2, int first3, int count,
+                                                                                 int tokens, GroupShared shared, GroupTable table) {
+  int block;
+  const SkinnyArgs p = group_problem(first1, first2, first3, count, tokens, shared, table, block);
+  skinny_body<NW, R, kSkinnyBTokens, NC, BF16>(p, block, 0);
+}
+
+static bool same_group_types(const SkinnyArgs& a, const SkinnyArgs& b) {
+  return a.bf16 == b.bf16 && a.d_f16 == b.d_f16 && a.bias_type == b.bias_type;
+}
+
+// The arguments of a grouped launch from the launcher's (first_block filled in).
+struct GroupLaunch {
+  int first[4];
+  GroupShared shared;
+  GroupTable table;
+};
+static GroupLaunch group_launch(const SkinnyGroupArgs& g) {
+  GroupLaunch l{};
+  for (int i = 0; i < 4; ++i) l.first[i] = i < g.count ? g.first_block[i] : INT_MAX;
+  l.shared = GroupShared{g.problem[0].d_f16, g.problem[0].bias_type, g.problem[0].tokens_per_group};
+  for (int i = 0; i < g.count; ++i) {
+    const SkinnyArgs& p = g.problem[i];
+    l.table.problem[i] = GroupProblem{p.prep, p.b, p.d, p.bias, p.m, p.k};
+    l.table.first_block[i] = g.first_block[i];
+  }
+  return l;
 }
 
 template <int NW, int R, int MODE, int NC, bool BF16 = false>
 static hipError_t launch_skinny_mode(const SkinnyArgs& args, hipStream_t stream) {
   const int row_blocks = args.m / kRowBlock;
+  const LaunchArgs a = pack_args(args);
   hipLaunchKernelGGL((skinny_kernel<NW, R, MODE, NC, BF16>), dim3((row_blocks + R - 1) / R, args.splits), dim3(64 * NW), 0,
-                     stream, args);
+                     stream, a.operands, a.results, a.epilogue);
   return hipGetLastError();
 }
 

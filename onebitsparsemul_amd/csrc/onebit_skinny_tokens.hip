@@ -34,7 +34,9 @@ hipError_t launch_skinny_tokens(SkinnyArgs args, int rows_per_group, hipStream_t
 template <int NW, int R, bool BF16>
 static hipError_t launch_skinny_group_type(const SkinnyGroupArgs& g, int blocks, hipStream_t stream) {
   const dim3 grid(blocks), threads(64 * NW);
-  hipLaunchKernelGGL((skinny_group_kernel<NW, R, 16, BF16>), grid, threads, 0, stream, g);
+  const GroupLaunch l = group_launch(g);
+  hipLaunchKernelGGL((skinny_group_kernel<NW, R, 16, BF16>), grid, threads, 0, stream, l.first[1], l.first[2], l.first[3], g.count,
+                     g.problem[0].n, l.shared, l.table);
   return hipGetLastError();
 }
 
@@ -52,7 +54,7 @@ hipError_t launch_skinny_group(SkinnyGroupArgs g, int rows_per_group, hipStream_
   int blocks = 0;
   for (int i = 0; i < g.count; ++i) {
     SkinnyArgs& p = g.problem[i];
-    if (p.n != tokens || p.bf16 != g.problem[0].bf16 || p.m <= 0 || p.k <= 0 || !p.prep || !p.b || !p.d) return hipErrorInvalidValue;
+    if (p.n != tokens || !same_group_types(p, g.problem[0]) || p.m <= 0 || p.k <= 0 || !p.prep || !p.b || !p.d) return hipErrorInvalidValue;
     // 16-byte loads of x; lane offsets of up to 64 token rows must stay below the "outside" offset of the kernel
     if ((reinterpret_cast<uintptr_t>(p.b) & 15) != 0 || (size_t)p.k * 64 * 2 >= 0xFFFFFF00u) return hipErrorInvalidValue;
     p.splits = 1;
