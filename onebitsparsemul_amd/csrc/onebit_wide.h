@@ -9,18 +9,20 @@ namespace onebit {
 
 // =====================================================================================================
 // wide_kernel: y[t][r] = sum_k W[r][k] x[t][k] + bias[r] (token-major form) and D = alpha A B + beta C (plain form) for 17
-// tokens or columns and more, in groups of up to 64 per workgroup (grid.z). The plain form differs in how an image lies in LDS
+// tokens or columns and more, in groups of up to 64 per workgroup. The plain form differs in how an image lies in LDS
 // and is read (see wide_body) and in the epilogue; below, x and token stand for B and column too.
 // Workgroup = eight wavefronts that share R row blocks (32 rows each) and split K among themselves chunk by chunk, as in
 // skinny_kernel. What differs is how x gets to the matrix cores: every wavefront keeps a ring of two images (64 K values of
 // all tokens, 2 KB per sixteen) in LDS that asynchronous copies fill. No registers hold x on its way, so the tile can be
-// 128 x 64 (R = 4), and with v_smfmac_f32_16x16x64 there are no idle columns at 24 or 48 tokens; one fragment read from LDS
-// serves 2 R SMFMACs.
+// 128 x 64 (R = 4), and with v_smfmac_f32_16x16x64 there are no idle columns at 16 or 48 tokens; one fragment read from LDS
+// serves 2 R SMFMACs (R of the 32x32x32 ones that whole 32-column tiles take).
 // Bound: with many tokens the bytes of x that pass through LDS. skinny_kernel's 64-row groups staged x through registers,
 // 16 KB of LDS writes and reads per 64 x 64 weights; a 128-row group halves that (28672 x 8192 with 48 tokens: 13 us of LDS
-// time, 12 of SMFMACs and 6 of sign expansion that hardly overlapped). us inside a HIP graph, weights from HBM, before ->
-// now: 28672 x 8192 with 24 / 48 / 64 tokens 16.6 / 33.4 / 35.9 -> 16.6 / 21.0 / 24.5; 11008 x 4096 8.0 / 11.0 / 11.7 -> 6.8 /
-// 8.3 / 9.6; 4096 x 4096 5.7 / 8.4 / 8.7 -> 4.7 / 6.0 / 7.1; 1024 x 1024 with 56 5.0 -> 3.5. Up to sixteen tokens there is no
+// time, 12 of SMFMACs and 6 of sign expansion that hardly overlapped). With 128 x 64 per workgroup and every compute unit busy
+// it is the 64 bytes per clock that a compute unit takes in: 76 KB of x and weights per 64 K of its eight wavefronts, 1216 of
+// the 1310 clocks they need (60 KB, 960 of 1250, at 48 tokens). us inside a HIP graph, weights from HBM, skinny_kernel ->
+// now: 28672 x 8192 with 24 / 48 / 64 tokens 16.6 / 33.4 / 35.9 -> 14.3 / 19.4 / 21.4; 11008 x 4096 8.0 / 11.0 / 11.7 -> 5.5 /
+// 7.9 / 9.1; 4096 x 4096 5.7 / 8.4 / 8.7 -> 3.6 / 4.7 / 5.1; 1024 x 1024 with 56 5.0 -> 2.65. Up to sixteen tokens there is no
 // gain (11008 x 4096 with 16: 6.4 -> 6.1, with 4: 5.5 -> 5.8; 28672 x 8192 with 16: 13.5 -> 14.0): skinny_kernel keeps those.
 // Beyond 64 tokens, and for products, the host's plan compares it with the kernel it would replace (onebit_capi.hip).
 // =====================================================================================================
@@ -48,6 +50,11 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
                                           char* const smem) {
   using Shape = WideShape<R, COPIES>;
   constexpr int NW = kWideWaves, CT = Shape::CT, RT = Shape::RT;
+  // Whole 32-column tiles take the 32x32x32 SMFMAC: with two wavefronts per SIMD it runs at 35.8 clocks beside the four sign
+  // expansions it needs at 64 columns (32 alone), the 16x16x64 one at 43.4 for the same work beside its two, and the prepared
+  // operand is used as it is stored (us: 28672 x 8192 with 32 tokens 16.7 -> 16.1, 8192 x 8192 with 128 15.9 -> 15.2, 16384 x 16384
+  // with 64 27.7 -> 26.9; where every compute unit is busy and power sets the clock about 1 % the other way).
+  constexpr bool S32 = CT % 2 == 0;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rb_total = p.m / kRowBlock, rb_first = block_x * R;
@@ -110,7 +117,7 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
   const char* const x_bytes = reinterpret_cast<const char*>(p.b + (TOKENS ? (size_t)first_token * k_total : (size_t)first_token));
   const char* const zeros = reinterpret_cast<const char*>(g_zero16_wide);
   auto copy_image = [&](int k0, int slot) __attribute__((always_inline)) {
-    const uint32_t dst = region_offset + slot * Shape::IMAGE_BYTES;
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(region_offset + slot * Shape::IMAGE_BYTES);
     if (k0 + kWideImageK <= k_total) {  // wave-uniform
 #pragma unroll
       for (int i = 0; i < COPIES; ++i) lds_dma16_base(x_bytes + k0 * k_stride, copy_off[i], dst + i * 1024);
@@ -128,13 +135,22 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
 
   const int i16 = lane & 15, g16 = lane >> 4;
   const uint32_t one = packed_one_in_vgpr<BF16>();
-  float4v_t acc[2 * R][CT];
+  float4v_t acc[S32 ? 1 : 2 * R][S32 ? 1 : CT];
+  float16_t acc32[S32 ? R : 1][S32 ? CT / 2 : 1];
 #pragma unroll
-  for (int rt = 0; rt < 2 * R; ++rt)
+  for (int rt = 0; rt < (S32 ? 1 : 2 * R); ++rt)
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
+    for (int ct = 0; ct < (S32 ? 1 : CT); ++ct) {
       acc[rt][ct] = float4v_t{0.f, 0.f, 0.f, 0.f};
       asm volatile("" : "+v"(acc[rt][ct]));
+    }
+#pragma unroll
+  for (int r = 0; r < (S32 ? R : 1); ++r)
+#pragma unroll
+    for (int f = 0; f < (S32 ? CT / 2 : 1); ++f) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc32[r][f][v] = 0.f;
+      asm volatile("" : "+v"(acc32[r][f]));
     }
 
   // Operands of one chunk. A lane of the prepared block (row l % 32, half ga) holds, per 32-wide step, what a lane of the
@@ -173,7 +189,37 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
     for (int ct = 0; ct < CT; ++ct)
       tile_off[ct] = lane_row * PIECES * 16 + (((2 * ct + ((i16 & 3) >> 1)) ^ row_swizzle(lane_row)) << 4) + (i16 & 1) * 8;
   half16_t frag[CT];
+  // 32x32x32 form: frag[2 f + ks] = K step ks of the columns 32 f ... 32 f + 31
+  const int gb = lane >> 5, col32 = lane & 31;
+  const uint32_t read_base32 = (uint32_t)col32 * 128u + (uint32_t)((gb ^ token_swizzle(col32)) << 4);
+  const int lane_row32 = 8 * gb + (i16 >> 2);
+  const int c8 = (col32 >> 4) * 4 + (i16 & 3);
   auto read_image = [&](int slot) __attribute__((always_inline)) {
+    if constexpr (S32) {
+#pragma unroll
+      for (int f = 0; f < CT / 2; ++f)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          u32x8_t raw_frag;
+          if constexpr (TOKENS) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const u32x4_t v = *reinterpret_cast<const u32x4_t*>(region + (read_base32 ^ ((4 * ks + 2 * h) << 4)) + slot * Shape::IMAGE_BYTES + f * 4096);
+              raw_frag[4 * h] = v.x; raw_frag[4 * h + 1] = v.y; raw_frag[4 * h + 2] = v.z; raw_frag[4 * h + 3] = v.w;
+            }
+          } else {
+            const int lc = 4 * f + (c8 >> 1);
+            const uint32_t off = lane_row32 * PIECES * 16 + ((lc ^ row_swizzle(lane_row32)) << 4) + (c8 & 1) * 8;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const u32x2_t v = lds_read_tr16(region + slot * Shape::IMAGE_BYTES + off + (32 * ks + 4 * (q & 1) + 16 * (q >> 1)) * PIECES * 16);
+              raw_frag[2 * q] = v.x; raw_frag[2 * q + 1] = v.y;
+            }
+          }
+          frag[2 * f + ks] = __builtin_bit_cast(half16_t, raw_frag);
+        }
+      return;
+    }
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
       u32x8_t raw_frag;
@@ -194,6 +240,23 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
   };
   auto compute = [&](auto s_tag) __attribute__((always_inline)) {
     constexpr int S = decltype(s_tag)::value;
+    if constexpr (S32) {
+      half8_t av[2];
+      av[0] = expand_signs<2 * S>(raw[0], one);
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int i = ks * R + r;
+          if (i + 1 < 2 * R) av[(i + 1) & 1] = (i + 1) / R == 0 ? expand_signs<2 * S>(raw[(i + 1) % R], one) : expand_signs<2 * S + 1>(raw[(i + 1) % R], one);
+#pragma unroll
+          for (int f = 0; f < CT / 2; ++f)
+            acc32[r][f] = ks == 0 ? smfmac_step<2 * S, false, BF16>(raw[r], av[i & 1], frag[2 * f + ks], acc32[r][f])
+                                  : smfmac_step<2 * S + 1, false, BF16>(raw[r], av[i & 1], frag[2 * f + ks], acc32[r][f]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      return;
+    }
     // the signs of the next row tile are expanded in front of the SMFMACs of the current one; the fences keep the optimizer
     // from expanding all of them first, which takes more registers than there are
     auto expand = [&](int rt) __attribute__((always_inline)) {
@@ -215,15 +278,28 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
   };
 
   // Requests return in order, and a wait names how many younger ones may be outstanding. Per chunk a wavefront requests its
-  // images 2 and 3, the first two images of its next chunk and the prepared operand of the chunk after that; before the loop
-  // the operand of the first chunk, its first two images, the operand of the second. Nothing is requested past the last
-  // chunk (wave-uniform branches).
+  // image 2, the prepared operand of its next chunk, image 3 and the first two images of the next chunk; before the loop the
+  // operand of the first chunk and its first two images. Nothing is requested past the last chunk (wave-uniform branches).
+  // A compute unit takes 64 bytes of requests per clock, so what stands in front of the first SMFMAC is what all wavefronts
+  // request before it: the second chunk's operand, requested up front too, held that up by 48 KB (28672 x 8192 with 48 tokens:
+  // the first SMFMAC of a workgroup 6000 to 8000 clocks after its start). And the older four wavefronts are served first all the
+  // way, ending 5000 clocks before the younger ones, whose SIMDs then have one wavefront each; the younger ones go first from
+  // here on. us, weights from HBM, both: 28672 x 8192 with 64 23.7 -> 22.9, 16384 x 16384 with 64 26.9 -> 25.6, 4096 x 4096 with
+  // 32 3.93 -> 3.72, 2048 x 8192 with 256 10.4 -> 9.8.
   if (first < kc_end) {
     copy_image(first * kChunkK, 0);
-    copy_image(first * kChunkK + kWideImageK, 1);
-    if (first + NW < kc_end) load_a(first + NW, next);
     __builtin_amdgcn_sched_barrier(0);
-    gather(raw);
+    if constexpr (S32) {
+      // the compiler's wait for the operand counts its own loads only: image 1 goes behind it (4096 x 4096 with 128 tokens
+      // 6.2 -> 6.0; in the other form the operand is first used further down and image 1 is better requested here)
+#pragma unroll
+      for (int r = 0; r < R; ++r) asm volatile("" : "+v"(raw[r].meta), "+v"(raw[r].sign));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    copy_image(first * kChunkK + kWideImageK, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (wave >= NW / 2) __builtin_amdgcn_s_setprio(1);
+    if constexpr (!S32) gather(raw);
     int kc = first;
 #pragma unroll 1
     do {
@@ -231,12 +307,12 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
       auto stage = [&](auto s_tag) __attribute__((always_inline)) {
         constexpr int S = decltype(s_tag)::value;
         // all but the requests younger than image S
-        if (more) wait_vmcnt<(S < 2 ? COPIES + 2 * R : COPIES)>();
+        if (more) wait_vmcnt<(S == 1 || S == 2 ? COPIES + 2 * R : COPIES)>();
         else wait_vmcnt<(S < 3 ? COPIES : 0)>();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         read_image(S & 1);
-        if constexpr (S == 2) {
+        if constexpr (S == 3) {
           // the wait the compiler puts in front of the operand's first use counts its own loads only and so also waits for
           // every copy issued by then: here that is one image, which has had a stage's time
 #pragma unroll
@@ -250,14 +326,21 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
           __builtin_amdgcn_sched_barrier(0);
         }
         compute(s_tag);
+        if constexpr (S == 0) {
+          if (more) load_a(kc + NW, next);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       };
       stage(std::integral_constant<int, 0>{});
       stage(std::integral_constant<int, 1>{});
       stage(std::integral_constant<int, 2>{});
       stage(std::integral_constant<int, 3>{});
-      gather(next);
-      if (kc + 2 * NW < kc_end) load_a(kc + 2 * NW, next);
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (S32) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) raw[r] = next[r];
+      } else {
+        gather(next);
+      }
       kc += NW;
     } while (kc < kc_end);
   }
@@ -265,10 +348,23 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
   // ---- add the eight partial tiles, RT row blocks per round: a token's rows as 16-byte slots of four rows, slot s at
   // position s ^ (token % slots)
   constexpr int SLOTS = RT * 8;
-  char* const y_out = reinterpret_cast<char*>(p.d) + (size_t)block_y * p.m * p.n * 4 * (p.splits > 1);
+  char* const y_out = reinterpret_cast<char*>(p.d) + (size_t)block_y * p.m * p.n * 4;  // a K split's slice: fp32 sums
 #pragma unroll
   for (int round = 0; round < R / RT; ++round) {
     if (round > 0) __syncthreads();
+    if constexpr (S32) {
+#pragma unroll
+      for (int rr = 0; rr < RT; ++rr)
+#pragma unroll
+        for (int f = 0; f < CT / 2; ++f)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int token = 32 * f + col32, slot = 8 * rr + 2 * q + gb;
+            const float16_t& a = acc32[round * RT + rr][f];
+            *reinterpret_cast<float4v_t*>(region + (token * SLOTS + (slot ^ (token & (SLOTS - 1)))) * 16) =
+                float4v_t{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+          }
+    } else
 #pragma unroll
     for (int rr = 0; rr < RT; ++rr)
 #pragma unroll
@@ -312,28 +408,62 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
   }
 }
 
+// Workgroups of several column groups walk the grid in strips of two of them: an XCD is given a contiguous range of the list
+// (workgroup b runs on XCD b % 8), so that what its workgroups read of x and of the weight meets in its L2. In the plain form the
+// column groups share the lines of B's rows, and with the row groups dealt over the XCDs each of those fetched every line (us,
+// row groups dealt -> strips: 2048 x 256 x 4096 9.0 -> 7.3, 4096 x 128 x 4096 7.7 -> 7.3; token-major 4096 x 11008 with 512 tokens
+// 31.2 -> 30.2).
+// Arguments as for skinny_kernel, but: operands[7] holds chunks_per_split and, from bit 24 on, the columns per workgroup; shape[0]
+// ArgFlags and, from bit 5 on, the row groups (0: the grid has the column groups as its third dimension); shape[1] is ldb; rest = 2^32 / (2 row groups) + 1,
+// workgroups, alpha, beta. All but `rest` is in registers from the start, and the token-major form of up to 64 tokens, where a load
+// at the start or in the epilogue would show most, does not need it: its x lies in every L2, strips gain nothing (1024 x 1024 with
+// 24 tokens 2.71 -> 2.81 us, 4096 x 4096 with 64 5.08 -> 5.18).
 template <int R, int COPIES, bool TOKENS, bool BF16>
-__global__ __launch_bounds__(64 * kWideWaves, 2) void wide_kernel(SkinnyArgs p) {
+__global__ __launch_bounds__(64 * kWideWaves, 2) void wide_kernel(u32x8_t operands, u32x4_t results, u32x2_t shape, u32x4_t rest) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  wide_body<R, COPIES, TOKENS, BF16>(p, blockIdx.x, blockIdx.y, blockIdx.z * p.tokens_per_group, smem);
+  SkinnyArgs p = unpack_args(operands, results, u32x4_t{shape[0], rest[2], rest[3], 0u});
+  p.chunks_per_split = operands[7] & 0xFFFFFFu;
+  p.tokens_per_group = operands[7] >> 24;
+  p.ldb = shape[1];
+  int x = blockIdx.x, group = blockIdx.z;
+  if (const int row_groups = shape[0] >> 5; row_groups > 0) {
+    const int total = rest[1], per = total / 8, rem = total % 8, xcd = x % 8;
+    const int v = xcd * per + (xcd < rem ? xcd : rem) + x / 8;
+    int strip = (int)__umulhi((uint32_t)v, rest[0]), w = v - strip * 2 * row_groups;
+    if (w < 0) --strip, w += 2 * row_groups;  // the reciprocal is rounded up
+    const bool pair = 2 * (strip + 1) * row_groups <= total;
+    x = pair ? w >> 1 : w;
+    group = 2 * strip + (pair ? w & 1 : 0);
+  }
+  wide_body<R, COPIES, TOKENS, BF16>(p, x, blockIdx.y, group * p.tokens_per_group, smem);
 }
 
-template <int R, int COPIES, class Args>
-static hipError_t launch_wide(void (*kern)(Args), std::atomic<bool> (&attr_done)[64], const Args& args, dim3 grid, hipStream_t stream) {
+// The dynamic-LDS limit of a kernel, a per-device attribute; threads that race here set the same value.
+static hipError_t wide_lds_limit(const void* kern, int lds, std::atomic<bool> (&attr_done)[64]) {
+  if (lds <= 65536) return hipSuccess;
+  int device = 0;
+  if (hipError_t st = hipGetDevice(&device); st != hipSuccess) return st;
+  if (device < 0 || device >= 64) return hipErrorInvalidDevice;
+  if (attr_done[device].load(std::memory_order_acquire)) return hipSuccess;
+  if (hipError_t st = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds); st != hipSuccess) return st;
+  attr_done[device].store(true, std::memory_order_release);
+  return hipSuccess;
+}
+
+template <int R, int COPIES, bool TOKENS, bool BF16>
+static hipError_t launch_wide_kernel(const SkinnyArgs& args, hipStream_t stream) {
+  static std::atomic<bool> attr_done[64] = {};
   constexpr int lds = WideShape<R, COPIES>::LDS_BYTES;
-  if (lds > 65536) {
-    // the dynamic-LDS limit is a per-device attribute of the kernel; threads that race here set the same value
-    int device = 0;
-    if (hipError_t st = hipGetDevice(&device); st != hipSuccess) return st;
-    if (device < 0 || device >= 64) return hipErrorInvalidDevice;
-    if (!attr_done[device].load(std::memory_order_acquire)) {
-      if (hipError_t st = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-          st != hipSuccess)
-        return st;
-      attr_done[device].store(true, std::memory_order_release);
-    }
-  }
-  hipLaunchKernelGGL(kern, grid, dim3(64 * kWideWaves), lds, stream, args);
+  const auto kern = wide_kernel<R, COPIES, TOKENS, BF16>;
+  if (hipError_t st = wide_lds_limit(reinterpret_cast<const void*>(kern), lds, attr_done); st != hipSuccess) return st;
+  const int rows = (args.m + 32 * R - 1) / (32 * R), groups = (args.n + args.tokens_per_group - 1) / args.tokens_per_group;
+  const bool strips = groups > 1 && (!TOKENS || args.n > kSkinnyMaxN);
+  LaunchArgs a = pack_args(args);
+  a.operands[7] |= (uint32_t)args.tokens_per_group << 24;  // chunks of 256 of an int K: 23 bits
+  const u32x2_t shape = {a.epilogue[0] | (strips ? (uint32_t)rows << 5 : 0u), (uint32_t)args.ldb};
+  const u32x4_t rest = {(uint32_t)((uint64_t(1) << 32) / (2 * rows) + 1), (uint32_t)(rows * groups), a.epilogue[1], a.epilogue[2]};
+  const dim3 grid = strips ? dim3(rows * groups, args.splits) : dim3(rows, args.splits, groups);
+  hipLaunchKernelGGL(kern, grid, dim3(64 * kWideWaves), lds, stream, a.operands, a.results, shape, rest);
   return hipGetLastError();
 }
 

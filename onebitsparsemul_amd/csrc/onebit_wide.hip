@@ -3,19 +3,13 @@
 
 namespace onebit {
 
-template <int R, int COPIES>
-static hipError_t launch_wide_plain(const SkinnyArgs& args, dim3 grid, hipStream_t stream) {
-  static std::atomic<bool> attr_done[64] = {};
-  return launch_wide<R, COPIES>(wide_kernel<R, COPIES, false, false>, attr_done, args, grid, stream);
-}
-
 template <int R>
-static hipError_t launch_wide_columns(const SkinnyArgs& args, dim3 grid, hipStream_t stream) {
+static hipError_t launch_wide_columns(const SkinnyArgs& args, hipStream_t stream) {
   switch ((args.tokens_per_group + 15) / 16) {
-    case 1: return launch_wide_plain<R, 2>(args, grid, stream);
-    case 2: return launch_wide_plain<R, 4>(args, grid, stream);
-    case 3: return launch_wide_plain<R, 6>(args, grid, stream);
-    case 4: return launch_wide_plain<R, 8>(args, grid, stream);
+    case 1: return launch_wide_kernel<R, 2, false, false>(args, stream);
+    case 2: return launch_wide_kernel<R, 4, false, false>(args, stream);
+    case 3: return launch_wide_kernel<R, 6, false, false>(args, stream);
+    case 4: return launch_wide_kernel<R, 8, false, false>(args, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -28,12 +22,11 @@ hipError_t launch_wide(SkinnyArgs args, int rows_per_group, hipStream_t stream) 
     return hipErrorInvalidValue;
   SkinnyArgs pass;
   if (hipError_t st = skinny_split_setup(args, pass); st != hipSuccess) return st;
-  const dim3 grid((args.m + rows_per_group - 1) / rows_per_group, args.splits, (args.n + columns - 1) / columns);
   hipError_t st;
   switch (rows_per_group) {
-    case 32: st = launch_wide_columns<1>(pass, grid, stream); break;
-    case 64: st = launch_wide_columns<2>(pass, grid, stream); break;
-    case 128: st = launch_wide_columns<4>(pass, grid, stream); break;
+    case 32: st = launch_wide_columns<1>(pass, stream); break;
+    case 64: st = launch_wide_columns<2>(pass, stream); break;
+    case 128: st = launch_wide_columns<4>(pass, stream); break;
     default: return hipErrorInvalidValue;
   }
   if (st != hipSuccess || args.splits <= 1) return st;
