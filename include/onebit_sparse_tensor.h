@@ -145,6 +145,12 @@ int onebit_sparse_linear_prepared_grouped(const onebit_linear_problem *problems,
  */
 int onebit_sparse_linear_prepared_typed(const void *prepared, const void *x, const void *bias, void *y, int tokens, int m,
                                         int k, int x_dtype, int bias_dtype, int y_dtype, void *stream);
+/*
+ * The same for fp32 activations of up to sixteen tokens, which the kernel rounds to fp16 (to nearest even) as it reads them: the
+ * result of converting x first and calling onebit_sparse_linear_prepared. More tokens are refused. y: fp16 or fp32.
+ */
+int onebit_sparse_linear_prepared_f32(const void *prepared, const void *x, const void *bias, void *y, int tokens, int m, int k,
+                                      int bias_dtype, int y_dtype, void *stream);
 int onebit_sparse_linear_prepared_grouped_typed(const onebit_linear_problem *problems, int count, int tokens, int x_dtype,
                                                 int bias_dtype, int y_dtype, void *stream);
 

@@ -685,6 +685,79 @@ int matmul_prepared_impl(const void* prepared, const void* b, const void* c, voi
   return ONEBIT_OK;
 }
 
+// The layer's product on 16-bit activations of either type, or up to sixteen tokens of fp32 ones (x_dtype).
+int linear_prepared_impl(const void* prepared, const void* x, const void* bias, void* y, int tokens, int m, int k, int x_dtype,
+                         int bias_dtype, int y_dtype, hipStream_t s) {
+  if (!prepared || !x || !y) return fail(ONEBIT_ERR_ARGUMENT, "null operand pointer");
+  if ((reinterpret_cast<uintptr_t>(x) & 15) != 0) return fail(ONEBIT_ERR_ARGUMENT, "x must be 16-byte aligned");
+  const int kc_total = (k + onebit::kChunkK - 1) / onebit::kChunkK;
+  const LinearPlan linear = plan_linear(m, tokens, k, current_compute_units());
+  const LaunchPlan& plan = linear.launch;
+  if ((size_t)k * 256 * 2 >= (size_t(1) << 32))
+    return fail(ONEBIT_ERR_ARGUMENT, "the token-major form addresses x with 32-bit offsets inside a tile of 256 tokens: "
+                                     "k = %d is beyond its limit of 8388607", k);
+  if (linear.wide || plan.split_k_kernel) {
+    onebit::SkinnyArgs args{};
+    args.prep = static_cast<const uint8_t*>(prepared);
+    args.b = static_cast<const _Float16*>(x);
+    args.d = y;
+    args.m = m; args.n = tokens; args.k = k;
+    args.kc_total = kc_total;
+    args.alpha = 1.f; args.beta = 0.f;
+    args.d_f16 = y_dtype != ONEBIT_DTYPE_F32;
+    args.bias = bias;
+    args.bias_type = bias_dtype;
+    args.bf16 = x_dtype == ONEBIT_DTYPE_BF16;
+    args.x_f32 = x_dtype == ONEBIT_DTYPE_F32;
+    DeviceLock lock;
+    if (int rc = setup_skinny_split(args, linear.wide ? linear.wide_plan.splits : plan.splits, plan.splits, s, nullptr, lock);
+        rc != ONEBIT_OK)
+      return rc;
+    args.tokens_per_group = linear.wide_plan.tokens;
+    ONEBIT_HIP(linear.wide ? onebit::launch_wide_tokens(args, linear.wide_plan.rows, s)
+                           : onebit::launch_skinny_tokens(args, plan.rows_or_tile, s));
+    return ONEBIT_OK;
+  }
+  switch (plan.rows_or_tile) {
+    case onebit::kTile256x128w: case onebit::kTile128x128s: case onebit::kTile512x128w8: case onebit::kTile256x128w8:
+    case onebit::kTile128x128w8: case onebit::kTile64x128: case onebit::kTile128x128k2: case onebit::kTile64x128k2:
+    case onebit::kTile512x128m16: break;
+    default:
+      return fail(ONEBIT_ERR_ARGUMENT, "tile configuration %d has no token-major variant (4, 6, 9 ... 15 have)",
+                  plan.rows_or_tile);
+  }
+  if (onebit::prepared_bytes(m, k) >= (size_t(1) << 32))
+    return fail(ONEBIT_ERR_ARGUMENT,
+                "the main kernel addresses the prepared operand with 32-bit offsets: m x k = %d x %d needs %zu bytes, "
+                "the limit is 4 GiB (about 22.9e9 weights); split the weight by rows", m, k, onebit::prepared_bytes(m, k));
+  onebit::GemmArgs args{};
+  args.prep = static_cast<const uint8_t*>(prepared);
+  args.b = static_cast<const _Float16*>(x);
+  args.d = y;
+  args.m = m; args.n = tokens; args.k = k;
+  args.kc_total = kc_total;
+  args.d_f16 = y_dtype != ONEBIT_DTYPE_F32;
+  args.bias = bias;
+  args.bias_type = bias_dtype;
+  args.bf16 = x_dtype == ONEBIT_DTYPE_BF16;
+  if (plan.splits > 1) {
+    int device = 0;
+    ONEBIT_HIP(hipGetDevice(&device));
+    if (device < 0 || device >= kMaxDevices) return fail(ONEBIT_ERR_ARGUMENT, "device ordinal %d not supported", device);
+    DeviceState& st = g_dev[device];
+    std::lock_guard<std::recursive_mutex> lock(st.mu);
+    args.chunks_per_split = (kc_total + plan.splits - 1) / plan.splits;
+    args.splits = full_splits(kc_total, plan.splits);
+    Buffer& ws = st.split_ws[s];
+    if (int rc = grow(&ws.ptr, &ws.bytes, (size_t)args.splits * m * tokens * sizeof(float), s); rc != ONEBIT_OK) return rc;
+    args.split_ws = static_cast<float*>(ws.ptr);
+    ONEBIT_HIP(onebit::launch_gemm_tokens(args, plan.rows_or_tile, s));
+    return ONEBIT_OK;
+  }
+  ONEBIT_HIP(onebit::launch_gemm_tokens(args, plan.rows_or_tile, s));
+  return ONEBIT_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -820,75 +893,18 @@ int onebit_sparse_linear_prepared_typed(const void* prepared, const void* x, con
   g_last_error.clear();
   if (int rc = check_shape(m, tokens, k)) return rc;
   if (int rc = check_linear_dtypes(x_dtype, bias_dtype, y_dtype)) return rc;
-  if (!prepared || !x || !y) return fail(ONEBIT_ERR_ARGUMENT, "null operand pointer");
-  if ((reinterpret_cast<uintptr_t>(x) & 15) != 0) return fail(ONEBIT_ERR_ARGUMENT, "x must be 16-byte aligned");
-  const int kc_total = (k + onebit::kChunkK - 1) / onebit::kChunkK;
-  const LinearPlan linear = plan_linear(m, tokens, k, current_compute_units());
-  const LaunchPlan& plan = linear.launch;
-  if ((size_t)k * 256 * 2 >= (size_t(1) << 32))
-    return fail(ONEBIT_ERR_ARGUMENT, "the token-major form addresses x with 32-bit offsets inside a tile of 256 tokens: "
-                                     "k = %d is beyond its limit of 8388607", k);
-  if (linear.wide || plan.split_k_kernel) {
-    onebit::SkinnyArgs args{};
-    args.prep = static_cast<const uint8_t*>(prepared);
-    args.b = static_cast<const _Float16*>(x);
-    args.d = y;
-    args.m = m; args.n = tokens; args.k = k;
-    args.kc_total = kc_total;
-    args.alpha = 1.f; args.beta = 0.f;
-    args.d_f16 = y_dtype != ONEBIT_DTYPE_F32;
-    args.bias = bias;
-    args.bias_type = bias_dtype;
-    args.bf16 = x_dtype == ONEBIT_DTYPE_BF16;
-    const hipStream_t s = static_cast<hipStream_t>(stream);
-    DeviceLock lock;
-    if (int rc = setup_skinny_split(args, linear.wide ? linear.wide_plan.splits : plan.splits, plan.splits, s, nullptr, lock);
-        rc != ONEBIT_OK)
-      return rc;
-    args.tokens_per_group = linear.wide_plan.tokens;
-    ONEBIT_HIP(linear.wide ? onebit::launch_wide_tokens(args, linear.wide_plan.rows, s)
-                           : onebit::launch_skinny_tokens(args, plan.rows_or_tile, s));
-    return ONEBIT_OK;
-  }
-  switch (plan.rows_or_tile) {
-    case onebit::kTile256x128w: case onebit::kTile128x128s: case onebit::kTile512x128w8: case onebit::kTile256x128w8:
-    case onebit::kTile128x128w8: case onebit::kTile64x128: case onebit::kTile128x128k2: case onebit::kTile64x128k2:
-    case onebit::kTile512x128m16: break;
-    default:
-      return fail(ONEBIT_ERR_ARGUMENT, "tile configuration %d has no token-major variant (4, 6, 9 ... 15 have)",
-                  plan.rows_or_tile);
-  }
-  if (onebit::prepared_bytes(m, k) >= (size_t(1) << 32))
-    return fail(ONEBIT_ERR_ARGUMENT,
-                "the main kernel addresses the prepared operand with 32-bit offsets: m x k = %d x %d needs %zu bytes, "
-                "the limit is 4 GiB (about 22.9e9 weights); split the weight by rows", m, k, onebit::prepared_bytes(m, k));
-  onebit::GemmArgs args{};
-  args.prep = static_cast<const uint8_t*>(prepared);
-  args.b = static_cast<const _Float16*>(x);
-  args.d = y;
-  args.m = m; args.n = tokens; args.k = k;
-  args.kc_total = kc_total;
-  args.d_f16 = y_dtype != ONEBIT_DTYPE_F32;
-  args.bias = bias;
-  args.bias_type = bias_dtype;
-  args.bf16 = x_dtype == ONEBIT_DTYPE_BF16;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (plan.splits > 1) {
-    int device = 0;
-    ONEBIT_HIP(hipGetDevice(&device));
-    if (device < 0 || device >= kMaxDevices) return fail(ONEBIT_ERR_ARGUMENT, "device ordinal %d not supported", device);
-    DeviceState& st = g_dev[device];
-    std::lock_guard<std::recursive_mutex> lock(st.mu);
-    args.chunks_per_split = (kc_total + plan.splits - 1) / plan.splits;
-    args.splits = full_splits(kc_total, plan.splits);
-    Buffer& ws = st.split_ws[s];
-    if (int rc = grow(&ws.ptr, &ws.bytes, (size_t)args.splits * m * tokens * sizeof(float), s); rc != ONEBIT_OK) return rc;
-    args.split_ws = static_cast<float*>(ws.ptr);
-    ONEBIT_HIP(onebit::launch_gemm_tokens(args, plan.rows_or_tile, s));
-    return ONEBIT_OK;
-  }
-  ONEBIT_HIP(onebit::launch_gemm_tokens(args, plan.rows_or_tile, s));
-  return ONEBIT_OK;
+  return linear_prepared_impl(prepared, x, bias, y, tokens, m, k, x_dtype, bias_dtype, y_dtype, static_cast<hipStream_t>(stream));
+}
+
+int onebit_sparse_linear_prepared_f32(const void* prepared, const void* x, const void* bias, void* y, int tokens, int m, int k,
+                                      int bias_dtype, int y_dtype, void* stream) {
+  g_last_error.clear();
+  if (int rc = check_shape(m, tokens, k)) return rc;
+  if (int rc = check_linear_dtypes(ONEBIT_DTYPE_F16, bias_dtype, y_dtype)) return rc;
+  if (tokens > onebit::kSkinnyTokens || !g_skinny_enabled)
+    return fail(ONEBIT_ERR_ARGUMENT, "fp32 activations are read by the kernel of up to %d tokens only (got %d): convert them to fp16",
+                onebit::kSkinnyTokens, tokens);
+  return linear_prepared_impl(prepared, x, bias, y, tokens, m, k, ONEBIT_DTYPE_F32, bias_dtype, y_dtype, static_cast<hipStream_t>(stream));
 }
 
 int onebit_sparse_linear_prepared_grouped(const onebit_linear_problem* problems, int count, int tokens, int bias_dtype,

@@ -57,6 +57,8 @@ struct SkinnyArgs {
   int splits;
   int chunks_per_split;
   float* split_ws;
+  // launch_skinny_tokens only: b is x in fp32, rounded to fp16 as it is read (bf16 = 0)
+  int x_f32;
   // wide_kernel only: tokens (columns) a workgroup multiplies (at most 64), grid.z = ceil(n / tokens_per_group); ldb: elements
   // between B rows in the plain form
   int tokens_per_group;

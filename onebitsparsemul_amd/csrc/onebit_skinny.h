@@ -38,7 +38,11 @@ constexpr int kSkinnyRegion = 8192;  // bytes of one B image
 // loaded in 16-byte pieces (32 n of them: at most two load instructions per wavefront and chunk, where the row-wise
 // modes issue eight; the split-K kernel's time is set by the number of load instructions it issues) and spread over the image rows
 // by LDS stores of 2 n bytes.
-enum SkinnyBMode { kSkinnyBFull = 0, kSkinnyBAny = 1, kSkinnyBTokens = 2, kSkinnyBRun = 3 };
+// kSkinnyBTokens32: the token-major form on fp32 activations, rounded to fp16 (nearest even) on their way into the image. One load
+// instruction takes a token's 256 K, whole lines, so there are as many as tokens. A conversion in front of the kernel costs a
+// launch and an allocation (us per layer call, conversion in front -> here: 4096 x 4096 with 1 / 16 tokens 9.2 / 9.0 -> 4.8 / 4.9,
+// 28672 x 8192 with 8 / 16 14.0 / 15.5 -> 11.8 / 14.8, 4096 x 11008 with 16 9.0 -> 8.7).
+enum SkinnyBMode { kSkinnyBFull = 0, kSkinnyBAny = 1, kSkinnyBTokens = 2, kSkinnyBRun = 3, kSkinnyBTokens32 = 4 };
 
 // The body of the split-K kernel for workgroup (block_x, block_y) of problem p: block_x = row group, block_y = K split.
 template <int NW, int R, int MODE, int NC, bool BF16 = false>
@@ -51,11 +55,12 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   constexpr int NF = NC <= 32 ? 1 : NC / 32;           // 32-column fragments per image row
   constexpr int TILE_BYTES = kRowBlock * NC * 4;       // one fp32 partial tile
   static_assert(NC == 16 || NC == 32 || NC == 64, "image width");
-  static_assert((MODE != kSkinnyBRun && MODE != kSkinnyBTokens) || NC == 16, "the run and token modes are for 16 columns");
+  static_assert((MODE != kSkinnyBRun && MODE != kSkinnyBTokens && MODE != kSkinnyBTokens32) || NC == 16, "the run and token modes are for 16 columns");
   // the partial tiles reuse the wavefront's image memory, RT row blocks per round of the final reduction
   constexpr int RT = R * TILE_BYTES <= kSkinnyRegion ? R : kSkinnyRegion / TILE_BYTES;
   static_assert(RT >= 1 && R % RT == 0, "the row blocks must divide into whole reduction rounds");
-  constexpr bool TOKENS = MODE == kSkinnyBTokens;
+  constexpr bool X32 = MODE == kSkinnyBTokens32, TOKENS = MODE == kSkinnyBTokens || X32;
+  static_assert(!X32 || !BF16, "fp32 activations are multiplied as fp16");
   // Sixteen columns fill half of the 32x32x32 SMFMAC's result tile; v_smfmac_f32_16x16x64_f16 has no idle half and
   // multiplies a row block's chunk in half the matrix-pipe time (eight instructions of four passes).
   constexpr bool M16 = NC == 16;
@@ -111,7 +116,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
     load_a(first, a_cur);
     __builtin_amdgcn_sched_barrier(0);
   }
-  const size_t b_bytes = (size_t)k_rows * n_cols * 2;
+  const size_t b_bytes = (size_t)k_rows * n_cols * (X32 ? 4 : 2);
   const bool b_fits = b_bytes < (size_t(1) << 32);  // else every image takes the general path
   const buffer_t b_buffer = make_buffer(b_ptr, b_fits ? (uint32_t)b_bytes : 0u);
   auto rows_valid_of = [&](int k_base) __attribute__((always_inline)) {
@@ -136,6 +141,30 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
       (uint32_t)token_lane * TOKEN_ROW_BYTES + (uint32_t)((piece_lane ^ token_swizzle<TOKEN_ROW_BYTES>(token_lane)) << 4);
   // run mode: piece q = lane + 64 i of the image's run; pieces at or past 32 n are sent outside the descriptor (zero)
   const uint32_t run_pieces = 32u * (uint32_t)n_cols;
+  // fp32 activations, eight tokens from first_token on. Load i: the image's K range of one token, four values per lane; K positions
+  // at or past k: outside the descriptor, as below (the launcher checks that 64 * k * 4 stays well below 2^32). Tokens 8 to 15
+  // are requested when the first eight have been stored: 64 registers of loads in flight do not fit beside the rest.
+  auto load_b32 = [&](int k_base, int first_token, u32x4_t (&v)[8]) __attribute__((always_inline)) {
+    const bool whole = k_base + IMG_ROWS <= k_rows;  // wave-uniform
+    const bool inside = k_base + 4 * lane < k_rows;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (first_token + i < n_cols) {
+        const uint32_t offset = meta_off + (uint32_t)(first_token + i) * (uint32_t)k_rows * 4u;
+        v[i] = buffer_load16(b_buffer, whole ? offset : inside ? offset + (uint32_t)k_base * 4u : 0xFFFFFF00u, whole ? (uint32_t)k_base * 4u : 0u);
+      } else {
+        v[i] = u32x4_t{0, 0, 0, 0};
+      }
+  };
+  auto store_b32 = [&](int first_token, const u32x4_t (&v)[8]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float4v_t f = __builtin_bit_cast(float4v_t, v[i]);
+      const int token = first_token + i;
+      *reinterpret_cast<u32x2_t*>(region + token * TOKEN_ROW_BYTES + (((lane >> 1) ^ token_swizzle<TOKEN_ROW_BYTES>(token)) << 4) +
+                                  (lane & 1) * 8) = u32x2_t{round_pair<false>(f[0], f[1]), round_pair<false>(f[2], f[3])};
+    }
+  };
   auto load_b = [&](int k_base, u32x4_t (&v)[8]) __attribute__((always_inline)) {
     if (MODE == kSkinnyBRun) {
       const uint32_t run_base = (uint32_t)k_base * (uint32_t)n_cols * 2u;  // the launcher checks k n 2 < 2^32
@@ -154,6 +183,10 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
       for (int i = 0; i < 2; ++i)
         if (64u * i < run_pieces)
           v[i] = buffer_load16(b_buffer, meta_off + 1024u * i + 16u <= valid_bytes ? run_base + meta_off + 1024u * i : 0xFFFFFF00u, 0);
+      return;
+    }
+    if (X32) {
+      load_b32(k_base, 0, v);
       return;
     }
     if (TOKENS) {
@@ -229,6 +262,15 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
     }
   };
   auto store_b = [&](int k_base, const u32x4_t (&v)[8]) __attribute__((always_inline)) {
+    if (X32) {
+      store_b32(0, v);
+      if (n_cols > 8) {
+        u32x4_t w[8];
+        load_b32(k_base, 8, w);
+        store_b32(8, w);
+      }
+      return;
+    }
     if (MODE == kSkinnyBAny) {
 #pragma unroll
       for (int i = 0; i < 8; ++i)

@@ -10,13 +10,15 @@ static hipError_t launch_skinny_tokens_type(const SkinnyArgs& args, hipStream_t 
 
 template <int NW, int R>
 static hipError_t launch_skinny_tokens_cfg(const SkinnyArgs& args, hipStream_t stream) {
+  if (args.x_f32) return launch_skinny_mode<NW, R, kSkinnyBTokens32, 16>(args, stream);
   return args.bf16 ? launch_skinny_tokens_type<NW, R, true>(args, stream) : launch_skinny_tokens_type<NW, R, false>(args, stream);
 }
 
 hipError_t launch_skinny_tokens(SkinnyArgs args, int rows_per_group, hipStream_t stream) {
   if (args.n < 1 || args.n > kSkinnyTokens) return hipErrorInvalidValue;
   // 16-byte loads of x; lane offsets of up to 64 token rows must stay below the "outside" offset of the kernel
-  if ((reinterpret_cast<uintptr_t>(args.b) & 15) != 0 || (size_t)args.k * 64 * 2 >= 0xFFFFFF00u) return hipErrorInvalidValue;
+  if ((reinterpret_cast<uintptr_t>(args.b) & 15) != 0 || (size_t)args.k * 64 * (args.x_f32 ? 4 : 2) >= 0xFFFFFF00u || (args.x_f32 && args.bf16))
+    return hipErrorInvalidValue;
   SkinnyArgs pass;
   if (hipError_t st = skinny_split_setup(args, pass); st != hipSuccess) return st;
   hipError_t st;
