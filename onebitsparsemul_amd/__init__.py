@@ -9,6 +9,8 @@ host computation.
 import torch
 import torch.nn as nn
 
+from torch.nn.modules.module import _global_buffer_registration_hooks as _buffer_hooks
+
 from . import _native
 from ._semi_structured_conversions import (
     mask_creator,
@@ -158,9 +160,14 @@ class BinaryLinear_2_4(nn.Module):
             weight = weight.contiguous()
             if weight.data_ptr() % 16:
                 weight = weight.clone()  # a view that starts inside a 16-byte unit
-            self.packed_binary_sparse, self.meta = _binding().pack_weight(weight, True, _native.META_REFERENCE)
-            self.vaild = True
-            self._prepared = None
+            a, meta = _binding().pack_weight(weight, True, _native.META_REFERENCE)
+            buffers = self._buffers
+            if "packed_binary_sparse" in buffers and "meta" in buffers and not _buffer_hooks:
+                # where nn.Module.__setattr__ puts a registered buffer, without its 1.5 us per attribute
+                buffers["packed_binary_sparse"], buffers["meta"] = a, meta
+            else:
+                self.packed_binary_sparse, self.meta = a, meta
+            self.__dict__.update(vaild=True, _prepared=None)
             return
         w = weight * mask_creator(weight).to(weight.dtype)
         if w.dtype not in (torch.half, torch.bfloat16, torch.int32):
@@ -191,6 +198,11 @@ class BinaryLinear_2_4(nn.Module):
 
     def forward(self, x):
         # one kernel: reads the tokens where they lie, adds the bias, writes (tokens, outfeatures)
+        prepared = self._prepared
+        if prepared is not None and self.vaild:
+            y = _binding().layer_forward(prepared.buffer, x, self.bias, self.outfeatures, self.infeatures, self.out_dtype)
+            if y is not None:
+                return y  # else x is on another device than the prepared weight
         return _binding().layer_forward(self._prepared_on(x.device), x, self.bias, self.outfeatures, self.infeatures,
                                         self.out_dtype)
 
@@ -206,8 +218,10 @@ def forward_grouped(layers, xs):
         raise ValueError("one input per layer (or one for all)")
     if not layers:
         return []
-    prepared = [layer._prepared_on(xs[0 if shared else i].device) for i, layer in enumerate(layers)]
-    ys = _binding().grouped_forward(prepared, xs, [layer.bias for layer in layers], [layer.outfeatures for layer in layers],
-                                    [layer.infeatures for layer in layers], [layer.out_dtype for layer in layers])
-    # nothing to share (token counts or types differ): the layers one by one
+    ys = _binding().grouped_forward(layers, xs)
+    if ys is None:  # a layer's weight is not prepared yet, or on another device than its input
+        for i, layer in enumerate(layers):
+            layer._prepared_on(xs[0 if shared else i].device)
+        ys = _binding().grouped_forward(layers, xs)
+    # nothing to share (token counts or types differ, or one layer with inputs on two devices): the layers one by one
     return ys or [layer(xs[0 if shared else i]) for i, layer in enumerate(layers)]

@@ -129,9 +129,11 @@ int64_t token_count(const torch::Tensor& x, int64_t k) {
 // Most tokens of fp32 activations that onebit_sparse_linear_prepared_f32 takes.
 constexpr int64_t kF32Tokens = 16;
 
-// BinaryLinear_2_4.forward behind its bookkeeping: y = x W^T (+ bias), shape and type of the layer's result.
-torch::Tensor layer_forward(const torch::Tensor& prepared, const torch::Tensor& x, const OptionalTensor& bias, int64_t m,
+// BinaryLinear_2_4.forward behind its bookkeeping: y = x W^T (+ bias), shape and type of the layer's result. Nothing where x is on
+// another device than the prepared weight: the layer then prepares its weight there.
+OptionalTensor layer_forward(const torch::Tensor& prepared, const torch::Tensor& x, const OptionalTensor& bias, int64_t m,
                             int64_t k, std::optional<c10::ScalarType> out_dtype) {
+  if (prepared.device() != x.device()) return std::nullopt;
   at::AutoDispatchBelowADInplaceOrView guard_dispatch;
   if (x.numel() == 0) return at::zeros(result_sizes(x, m), x.options());  // an empty batch: nothing to launch
   const int64_t tokens = token_count(x, k);
@@ -215,6 +217,42 @@ std::vector<torch::Tensor> grouped_forward(const std::vector<torch::Tensor>& pre
   return ys;
 }
 
+// forward_grouped: the layers' attributes are read here (in Python their lists took as long as the launch). None where a layer has
+// no weight prepared on its input's device.
+py::object grouped_forward_layers(const py::list& layers, const std::vector<torch::Tensor>& xs) {
+  static PyObject* const names[] = {PyUnicode_InternFromString("_prepared"), PyUnicode_InternFromString("vaild"),
+                                    PyUnicode_InternFromString("buffer"), PyUnicode_InternFromString("bias"),
+                                    PyUnicode_InternFromString("outfeatures"), PyUnicode_InternFromString("infeatures"),
+                                    PyUnicode_InternFromString("out_dtype")};
+  auto get = [](const py::handle& object, int name) {
+    PyObject* value = PyObject_GetAttr(object.ptr(), names[name]);
+    if (!value) throw py::error_already_set();
+    return py::reinterpret_steal<py::object>(value);
+  };
+  const size_t count = layers.size();
+  std::vector<torch::Tensor> prepared(count);
+  std::vector<OptionalTensor> biases(count);
+  std::vector<int64_t> ms(count), ks(count);
+  std::vector<std::optional<c10::ScalarType>> out_dtypes(count);
+  for (size_t i = 0; i < count; ++i) {
+    const py::handle layer = layers[i];
+    const py::object own = get(layer, 0);
+    if (own.is_none() || !py::cast<bool>(get(layer, 1))) return py::none();
+    prepared[i] = py::cast<torch::Tensor>(get(own, 2));
+    if (prepared[i].device() != xs[xs.size() == 1 ? 0 : i].device()) return py::none();
+    biases[i] = py::cast<OptionalTensor>(get(layer, 3));
+    ms[i] = py::cast<int64_t>(get(layer, 4));
+    ks[i] = py::cast<int64_t>(get(layer, 5));
+    out_dtypes[i] = py::cast<std::optional<c10::ScalarType>>(get(layer, 6));
+  }
+  std::vector<torch::Tensor> ys;
+  {
+    const py::gil_scoped_release release;
+    ys = grouped_forward(prepared, xs, biases, ms, ks, out_dtypes);
+  }
+  return py::cast(std::move(ys));
+}
+
 // PreparedWeight.matmul: D = alpha A B + beta C into `out`, or into a new tensor of type out_dtype (None: torch's default).
 torch::Tensor matmul_prepared(const torch::Tensor& prepared, const torch::Tensor& b, const OptionalTensor& c,
                               const OptionalTensor& out, int64_t m, int64_t k, double alpha, double beta,
@@ -295,7 +333,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   using NoGil = pybind11::call_guard<pybind11::gil_scoped_release>;
   m.def("onebit_mul", &onebit_mul, "A32 = Sparse W1 * A16 matmul.", NoGil());
   m.def("layer_forward", &layer_forward, NoGil());
-  m.def("grouped_forward", &grouped_forward, NoGil());
+  m.def("grouped_forward", &grouped_forward_layers);
   m.def("matmul_prepared", &matmul_prepared, NoGil());
   m.def("binary_mul", &binary_mul, NoGil());
   m.def("prepare", &prepare, NoGil());
