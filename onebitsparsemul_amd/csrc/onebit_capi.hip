@@ -278,19 +278,31 @@ struct LaunchPlan {
 struct SkinnyPlan {
   int rows, splits;
 };
+
+// Weight rows per workgroup of the split-K kernel up to sixteen columns, from the workgroups that 32 and 64 rows give: the smallest
+// whose workgroups have a compute unit each. A workgroup more than that waits for a second round (us, 32 | 64 | 128 rows, both forms
+// alike: 9216 x 4096 with one token 6.0 | 4.6 | 6.6, with sixteen 7.3 | 5.4 | 7.2, with three columns 8.3 | 6.3 | 8.3; 17408 x
+// 4096 9.4 | 8.5 | 7.0, 11.2 | 10.2 | 7.6, 12.4 | 11.8 | 8.8; 18432 x 8192 with sixteen 15.9 | 14.6 | 11.5), and a larger group
+// leaves compute units idle (8192 x 4096 with one token 3.9 | 4.6 | 6.6, 16384 x 4096 7.3 | 5.4 | 7.0).
+int single_round_rows(long groups_of_32, long groups_of_64, int compute_units) {
+  return groups_of_32 <= compute_units ? 32 : groups_of_64 <= compute_units ? 64 : 128;
+}
+
 SkinnyPlan plan_skinny(int m, int n, int k, bool pieces, int compute_units) {
   const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
   const int forced_rows = g_skinny_rows, forced_splits = g_split_k;
-  // the largest row group that still gives about two workgroups per three compute units (measured: larger groups
+  // up to sixteen columns: single_round_rows. (pieces: B in pieces at any alignment. The other modes keep 64-row groups on K of up
+  // to five chunks, a route that is pinned by a test; 128 rows are the faster ones there too, 17408 x 1024 with one token 4.3
+  // against 5.3 us)
+  // beyond: the largest row group that still gives about two workgroups per three compute units (measured: larger groups
   // re-read B less often, but idle compute units cost more)
   // (n > 32: two column fragments per row block, at most two row blocks per wavefront)
-  // pieces: B in pieces at any alignment, up to sixteen columns. A workgroup of that mode has a compute unit to itself, so 64-row
-  // groups beyond one per compute unit wait for a second round: 128-row groups from there on (us, element copies | 64 | 128 rows:
-  // 18688 x 1280 with three columns 5.84 | 7.40 | 5.95, x 1760 6.77 | 7.66 | 6.06, x 8192 18.5 | 17.7 | 13.9; with twelve 9.7 | 7.4
-  // | 6.0)
   const int enough = std::max(1, 160 * compute_units / 256);
-  const bool second_round = pieces && (m + 63) / 64 > compute_units;
-  int rows = forced_rows > 0 ? forced_rows : ((m / 128 >= enough && n <= 32) || second_round) ? 128 : (m / 64 >= enough) ? 64 : 32;
+  const int rows = forced_rows > 0 ? forced_rows
+                   : n <= 16       ? (m / 128 < enough && !pieces && chunks <= 5
+                                          ? std::min(64, single_round_rows((m + 31) / 32, (m + 63) / 64, compute_units))
+                                          : single_round_rows((m + 31) / 32, (m + 63) / 64, compute_units))
+                   : (m / 128 >= enough && n <= 32) ? 128 : (m / 64 >= enough) ? 64 : 32;
   if (forced_splits >= 1) return SkinnyPlan{rows, forced_splits > chunks ? chunks : forced_splits};
   const double image_row_bytes = n <= 16 ? 32.0 : n <= 32 ? 64.0 : 128.0;
   const double threshold = 400e3 * std::max(1.0, m / 4096.0);
@@ -938,26 +950,23 @@ int onebit_sparse_linear_prepared_grouped_typed(const onebit_linear_problem* pro
     }
     return ONEBIT_OK;
   }
-  // Row group of the launch: as for one product with all the weight rows; up to sixteen tokens the largest that still gives
-  // about two workgroups per three compute units.
+  // Row group of the launch: as for one product with all the weight rows.
   const int compute_units = current_compute_units();
   for (int first = 0; first < count; first += onebit::kSkinnyMaxGroup) {
     const int in_launch = std::min(count - first, onebit::kSkinnyMaxGroup);
     const bool wide = tokens > onebit::kSkinnyTokens;
-    long rows_total = 0, groups[3] = {0, 0, 0};
+    long groups[3] = {0, 0, 0};
     int longest_k = 0;
     for (int i = 0; i < in_launch; ++i) {
       const onebit_linear_problem& q = problems[first + i];
-      rows_total += q.m;
       for (int r = 0; r < 3; ++r) groups[r] += (q.m + kWideRows[r] - 1) / kWideRows[r];
       longest_k = std::max(longest_k, q.k);
     }
-    const int enough = std::max(1, 160 * compute_units / 256);
     WidePlan wide_plan{};
     if (wide) wide_plan = plan_wide(groups, 0.0, tokens, longest_k, false, 1, 1, compute_units);
     const int rows = wide ? wide_plan.rows
                      : g_skinny_rows > 0 ? g_skinny_rows
-                     : (rows_total / 128 >= enough) ? 128 : (rows_total / 64 >= enough) ? 64 : 32;
+                     : single_round_rows(groups[0], groups[1], compute_units);
     if (rows != 32 && rows != 64 && rows != 128) return fail(ONEBIT_ERR_ARGUMENT, "row group %d: must be 32, 64 or 128", rows);
     onebit::SkinnyGroupArgs group{};
     group.count = in_launch;
