@@ -760,180 +760,153 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
   if constexpr (TOKENS) {
     // ---- epilogue of the linear-layer form: y[token][row] = acc + bias[row], fp16 (RNE) or fp32 ----
     const int token_lane = lane & 31;
-    auto bias_of = [&](int row) __attribute__((always_inline)) { return p.bias ? load_element(p.bias, p.bias_type, row) : 0.f; };
-    // COUNT (4 or 8) consecutive bias values starting at a row that is a multiple of COUNT, by 8- or 16-byte loads
-    auto bias_vector = [&](int row, float* out, auto count_tag) __attribute__((always_inline)) {
-      constexpr int COUNT = decltype(count_tag)::value;
-#pragma unroll
-      for (int e = 0; e < COUNT; ++e) out[e] = 0.f;
-      if (!p.bias) return;
+    // the four bias values from a row on that is a multiple of four, any four where the row is past the end (never stored);
+    // p.bias is not null
+    auto bias_vector = [&](int row, float* out) __attribute__((always_inline)) {
+      const size_t at = row < p.m ? row : 0;
       if (p.bias_type != kF32) {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint16_t*>(p.bias) + row);
-        uint32_t words[COUNT / 2];
-        __builtin_memcpy(words, __builtin_assume_aligned(src, COUNT * 2), COUNT * 2);
+        const u32x2_t words = *reinterpret_cast<const u32x2_any_t*>(reinterpret_cast<const uint16_t*>(p.bias) + at);
 #pragma unroll
-        for (int e = 0; e < COUNT; e += 2) {
+        for (int e = 0; e < 4; e += 2) {
           const float2v_t v = unpack_pair(words[e / 2], p.bias_type);
           out[e] = v.x; out[e + 1] = v.y;
         }
       } else {
+        const u32x4_t v = *reinterpret_cast<const u32x4_any_t*>(reinterpret_cast<const float*>(p.bias) + at);
 #pragma unroll
-        for (int e = 0; e < COUNT; e += 4) {
-          const float4 v = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(p.bias) + row + e);
-          out[e] = v.x; out[e + 1] = v.y; out[e + 2] = v.z; out[e + 3] = v.w;
-        }
+        for (int e = 0; e < 4; ++e) out[e] = __builtin_bit_cast(float, (uint32_t)v[e]);
       }
     };
-    if (p.vector_epilogue) {
-      // Each wavefront turns one 32-row block of its tile at a time through a private LDS scratch laid out
-      // [token][32 rows] fp32: a lane's four accumulator registers of one group are four consecutive rows of its token,
-      // one 16-byte slot (slot s = rows 4 s ... 4 s + 3, stored at position s ^ (token % 8) against bank conflicts);
-      // then every lane handles 16 bytes of one token's row of y.
-      __syncthreads();  // every wavefront is done with the stage ring, which becomes the scratch
-      constexpr int WCOLS = FN * 32;
-      char* scratch = smem + wave * (WCOLS * 128);
-      if constexpr (!M16) if (p.d_f16) {
-        // (measured: 1-5 % off the launch for the 32x32x32 tiles, e.g. 4096 x 4096 with 2048 tokens 37.5 -> 36.7 us; the
-        // 16x16x64 tile, whose single wavefront per SIMD has nothing to hide the conversions behind, is 0.5 % slower
-        // with it and keeps the fp32 form)
-        // fp16 result: the bias is added and the sum rounded in the accumulator layout, where a lane's four registers of
-        // one group are four consecutive rows of its token, i.e. 8 bytes of y. The scratch line of a token then holds its
-        // 32 rows as halves (64 bytes, four 16-byte pieces; piece j of token t stored at position j ^ ((t / 4) % 4), so
-        // that the sixteen lanes that write one slot of sixteen consecutive tokens meet in no bank): half the LDS
-        // traffic of the fp32 form below, same bits (one rounding of sum + bias).
-        auto packed_rows = [&](const float* x, const float* b4) __attribute__((always_inline)) {
-          return u32x2_t{round_pair<BF16>(x[0] + b4[0], x[1] + b4[1]), round_pair<BF16>(x[2] + b4[2], x[3] + b4[3])};
-        };
-        // bias of the four rows starting at `row` (a multiple of 4); rows at or past the end are never stored
-        auto bias_rows = [&](int row, float* b4) __attribute__((always_inline)) {
-          if (row < row_limit) bias_vector(row, b4, std::integral_constant<int, 4>{});
-          else b4[0] = b4[1] = b4[2] = b4[3] = 0.f;
-        };
-        auto slot_at = [&](int t, int slot) __attribute__((always_inline)) {  // byte offset of 8-byte slot `slot` of token t
-          return t * 64 + ((((slot >> 1) ^ ((t >> 2) & 3)) << 4) | ((slot & 1) << 3));
-        };
+    // A tile's sums out of the accumulation registers, here: left to itself the compiler moves all 256 in front of the branches
+    // between the forms below, where they do not fit (44 registers spilled).
+    auto take_sums = [&](const float4v_t& sums) __attribute__((always_inline)) {
+      float4v_t v;
 #pragma unroll
-        for (int fm = 0; fm < FM; ++fm) {
-          if (!finishes(fm)) continue;  // the other K group stores this fragment
-          const int row_base = row0 + fm * 32;
-          {
+      for (int e = 0; e < 4; ++e) {
+        float x;
+        asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"((float)sums[e]));
+        v[e] = x;
+      }
+      return v;
+    };
+    // Each wavefront turns its tile through a private LDS scratch, after which every lane stores 16 bytes of one token's
+    // row of y.
+    __syncthreads();  // every wavefront is done with the stage ring, which becomes the scratch
+    constexpr int WCOLS = FN * 32;
+    char* const scratch = smem + wave * (WCOLS * 128);
+    const int g16 = lane >> 4, c16 = lane & 15;
+    if (p.d_f16) {
+      // 16-bit result: the bias is added and the sum rounded in the accumulator layout, where four registers of a lane are
+      // four consecutive rows of its token, 8 bytes of y. A turn takes as many tokens as the scratch holds with all of the
+      // wavefront's rows, up to 256 bytes of a token, so that the stores write whole lines of y; one 32-row block at a time
+      // they wrote halves of lines, of sixteen tokens per instruction. us, that -> this (fp16 | bf16; the 16x16x64 tile went
+      // through the scratch as floats before, and spilled): 8192 x 8192 with 8192 tokens 438 -> 423 | 424 -> 406, 11008 x 4096
+      // with 4096 172 -> 164 | 166 -> 154, 4096 x 4096 with 4096 62.1 -> 57.6 | 59.6 -> 55.3; fewer tiles than compute units
+      // 35.2 -> 34.9 (2048 tokens).
+      constexpr int FRAGS = kSplitEpilogue ? FM / 2 : FM;  // of the rows that this wavefront finishes
+      constexpr int PIECES = 4 * FRAGS;                    // 16-byte pieces of a token's rows
+      constexpr int TURN = FRAGS > 2 ? 2 * WCOLS / FRAGS : WCOLS;
+      static_assert(TURN * PIECES <= WCOLS * 8 && WCOLS % TURN == 0 && TURN % (M16 ? 16 : 32) == 0, "tokens per turn");
+      // byte offset of the 8-byte slot `slot` (four rows) of the turn's token t; lanes of sixteen consecutive tokens that
+      // write one slot, or read one token, meet in no bank
+      auto slot_at = [&](int t, int slot) __attribute__((always_inline)) {
+        return t * (PIECES * 16) + ((((slot >> 1) ^ ((t * PIECES >> 4) & (PIECES - 1))) << 4) | ((slot & 1) << 3));
+      };
+      auto turns = [&](auto bias_tag) __attribute__((always_inline)) {
+        constexpr bool BIAS = decltype(bias_tag)::value;
+        constexpr int GROUPS = M16 ? 2 : 4;  // of four rows, per 32-row block and lane
+        // 32x32x32 form: registers 4 q ... 4 q + 3 are rows 8 q + 4 (lane / 32) on; 16x16x64 form: the registers of tile
+        // (2 fm + q, ct) are rows 16 q + 4 (lane / 16) on of token 16 ct + lane % 16
+        auto slot_of = [&](int q) __attribute__((always_inline)) { return M16 ? 4 * q + g16 : 2 * q + gb; };
+        float bias[BIAS ? FM * GROUPS : 1][4];
+        if constexpr (BIAS) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              float b4[4];
-              bias_rows(row_base + 8 * q + 4 * gb, b4);
+          for (int i = 0; i < FM * GROUPS; ++i)
+            if (finishes(i / GROUPS)) bias_vector(row0 + i / GROUPS * 32 + 4 * slot_of(i % GROUPS), bias[i]);
+        }
+        const int lane_piece = lane % PIECES, lane_token = lane / PIECES;
+        const int row = row0 + (kSplitEpilogue ? kg * FRAGS * 32 : 0) + 8 * lane_piece;
+        const int tokens = row < row_limit ? p.n : 0;
+        int token = col0 + lane_token;
+        _Float16* y = reinterpret_cast<_Float16*>(d_out) + (size_t)token * p.m + row;
+        const size_t step = (size_t)(64 / PIECES) * p.m;
 #pragma unroll
-              for (int fn = 0; fn < FN; ++fn) {
-                const float x[4] = {acc[fm][fn][4 * q], acc[fm][fn][4 * q + 1], acc[fm][fn][4 * q + 2], acc[fm][fn][4 * q + 3]};
-                *reinterpret_cast<u32x2_t*>(scratch + slot_at(fn * 32 + token_lane, 2 * q + gb)) = packed_rows(x, b4);
+        for (int first = 0; first < WCOLS; first += TURN) {
+#pragma unroll
+          for (int fm = 0; fm < FM; ++fm) {
+            if (!finishes(fm)) continue;  // the other K group stores this fragment
+#pragma unroll
+            for (int q = 0; q < GROUPS; ++q) {
+              const int slot = slot_of(q);
+              auto put = [&](int t, float x0, float x1, float x2, float x3) __attribute__((always_inline)) {
+                if constexpr (BIAS) {
+                  const float* const b4 = bias[fm * GROUPS + q];
+                  x0 += b4[0]; x1 += b4[1]; x2 += b4[2]; x3 += b4[3];
+                }
+                *reinterpret_cast<u32x2_t*>(scratch + slot_at(t, 8 * (fm % FRAGS) + slot)) =
+                    u32x2_t{round_pair<BF16>(x0, x1), round_pair<BF16>(x2, x3)};
+              };
+              if constexpr (M16) {
+#pragma unroll
+                for (int ct = first / 16; ct < (first + TURN) / 16; ++ct) {
+                  const float4v_t v = take_sums(acc16[2 * fm + q][ct]);
+                  put(ct * 16 - first + c16, v[0], v[1], v[2], v[3]);
+                }
+              } else {
+#pragma unroll
+                for (int fn = first / 32; fn < (first + TURN) / 32; ++fn)
+                  put(fn * 32 - first + token_lane, acc[fm][fn][4 * q], acc[fm][fn][4 * q + 1], acc[fm][fn][4 * q + 2],
+                      acc[fm][fn][4 * q + 3]);
               }
             }
           }
 #pragma unroll
-          for (int it = 0; it < WCOLS * 4 / 64; ++it) {
-            const int piece = it * 64 + lane;
-            const int t = piece / 4, j = piece % 4;
-            const int token = col0 + t, row = row_base + 8 * j;
-            const u32x4_t v = *reinterpret_cast<const u32x4_t*>(scratch + slot_at(t, 2 * j));
-            if (token < p.n && row < row_limit)
-              *reinterpret_cast<u32x4_t*>(reinterpret_cast<_Float16*>(d_out) + (size_t)token * p.m + row) = v;
+          for (int it = 0; it < TURN * PIECES / 64; ++it) {
+            const u32x4_t v = *reinterpret_cast<const u32x4_t*>(scratch + slot_at(it * (64 / PIECES) + lane_token, 2 * lane_piece));
+            if (token < tokens) *reinterpret_cast<u32x4_any_t*>(y) = v;
+            token += 64 / PIECES;
+            y += step;
           }
+          __builtin_amdgcn_sched_barrier(0);
         }
-        return;
-      }
+      };
+      if (p.bias) turns(std::true_type{});
+      else turns(std::false_type{});
+      return;
+    }
+    // fp32 result, one 32-row block at a time: [token][32 rows], a lane's four registers of one group one 16-byte slot (slot
+    // s = rows 4 s ... 4 s + 3, stored at position s ^ (token % 8) against bank conflicts).
 #pragma unroll
-      for (int fm = 0; fm < FM; ++fm) {
-        if (!finishes(fm)) continue;  // the other K group stores this fragment
-        if constexpr (M16) {
-          // 16x16x64 form: the four registers of tile (2 fm + rh, ct) are rows 16 rh + 4 (lane / 16) ... + 3 of token
-          // 16 ct + lane % 16: slot 4 rh + lane / 16 of that token's line
-          const int g16 = lane >> 4, c16 = lane & 15;
+    for (int fm = 0; fm < FM; ++fm) {
+      if (!finishes(fm)) continue;  // the other K group stores this fragment
+      if constexpr (M16) {
+        // slot 4 rh + lane / 16 of token 16 ct + lane % 16
 #pragma unroll
-          for (int rh = 0; rh < 2; ++rh)
+        for (int rh = 0; rh < 2; ++rh)
 #pragma unroll
-            for (int ct = 0; ct < 2 * FN; ++ct) {
-              const float4v_t v4 = acc16[2 * fm + rh][ct];
-              *reinterpret_cast<float4*>(scratch + (ct * 16 + c16) * 128 + (((4 * rh + g16) ^ token_swizzle(c16)) << 4)) =
-                  float4{v4[0], v4[1], v4[2], v4[3]};
-            }
-        } else {
+          for (int ct = 0; ct < 2 * FN; ++ct) {
+            const float4v_t v4 = take_sums(acc16[2 * fm + rh][ct]);
+            *reinterpret_cast<float4*>(scratch + (ct * 16 + c16) * 128 + (((4 * rh + g16) ^ token_swizzle(c16)) << 4)) =
+                float4{v4[0], v4[1], v4[2], v4[3]};
+          }
+      } else {
 #pragma unroll
         for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
           for (int q = 0; q < 4; ++q)
             *reinterpret_cast<float4*>(scratch + (fn * 32 + token_lane) * 128 + (((2 * q + gb) ^ token_swizzle(token_lane)) << 4)) =
                 float4{acc[fm][fn][4 * q], acc[fm][fn][4 * q + 1], acc[fm][fn][4 * q + 2], acc[fm][fn][4 * q + 3]};
-        }
-        const int row_base = row0 + fm * 32;
-        if (p.d_f16) {
-#pragma unroll
-          for (int it = 0; it < WCOLS * 4 / 64; ++it) {
-            const int piece = it * 64 + lane;
-            const int t = piece / 4, j = piece % 4;
-            const int token = col0 + t, row = row_base + 8 * j;
-            const float4 lo = *reinterpret_cast<const float4*>(scratch + t * 128 + (((2 * j) ^ token_swizzle(t)) << 4));
-            const float4 hi = *reinterpret_cast<const float4*>(scratch + t * 128 + (((2 * j + 1) ^ token_swizzle(t)) << 4));
-            const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-            if (token < p.n && row < row_limit) {
-              float bias8[8];
-              bias_vector(row, bias8, std::integral_constant<int, 8>{});
-              u32x4_t out;
-#pragma unroll
-              for (int e = 0; e < 4; ++e) out[e] = round_pair<BF16>(x[2 * e] + bias8[2 * e], x[2 * e + 1] + bias8[2 * e + 1]);
-              *reinterpret_cast<u32x4_t*>(reinterpret_cast<_Float16*>(d_out) + (size_t)token * p.m + row) = out;
-            }
-          }
-        } else {
-#pragma unroll
-          for (int it = 0; it < WCOLS * 8 / 64; ++it) {
-            const int piece = it * 64 + lane;
-            const int t = piece / 8, j = piece % 8;
-            const int token = col0 + t, row = row_base + 4 * j;
-            const float4 v4 = *reinterpret_cast<const float4*>(scratch + t * 128 + ((j ^ token_swizzle(t)) << 4));
-            if (token < p.n && row < row_limit) {
-              float bias4[4];
-              bias_vector(row, bias4, std::integral_constant<int, 4>{});
-              *reinterpret_cast<float4*>(reinterpret_cast<float*>(d_out) + (size_t)token * p.m + row) =
-                  float4{v4.x + bias4[0], v4.y + bias4[1], v4.z + bias4[2], v4.w + bias4[3]};
-            }
-          }
-        }
       }
-      return;
-    }
-    // y not 16-byte aligned: one element per accumulator register
-    if constexpr (M16) {
+      const int j = lane % 8, row = row0 + fm * 32 + 4 * j;
+      float bias4[4] = {0.f, 0.f, 0.f, 0.f};
+      if (p.bias) bias_vector(row, bias4);
 #pragma unroll
-      for (int rt = 0; rt < 2 * FM; ++rt)
-#pragma unroll
-        for (int ct = 0; ct < 2 * FN; ++ct)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int token = col0 + ct * 16 + (lane & 15), row = row0 + rt * 16 + 4 * (lane >> 4) + v;
-            if (token < p.n && row < row_limit) {
-              const float x = acc16[rt][ct][v] + bias_of(row);
-              const size_t o = (size_t)token * p.m + row;
-              if (p.d_f16) reinterpret_cast<uint16_t*>(d_out)[o] = round_one<BF16>(x);
-              else reinterpret_cast<float*>(d_out)[o] = x;
-            }
-          }
-      return;
-    }
-#pragma unroll
-    for (int fm = 0; fm < FM; ++fm) {
-      if (!finishes(fm)) continue;  // the other K group stores this fragment
-#pragma unroll
-      for (int fn = 0; fn < FN; ++fn) {
-        const int token = col0 + fn * 32 + token_lane;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int row = row0 + fm * 32 + 8 * (v / 4) + 4 * gb + (v % 4);
-          if (token < p.n && row < row_limit) {
-            const float x = acc[fm][fn][v] + bias_of(row);
-            const size_t o = (size_t)token * p.m + row;
-            if (p.d_f16) reinterpret_cast<uint16_t*>(d_out)[o] = round_one<BF16>(x);
-            else reinterpret_cast<float*>(d_out)[o] = x;
-          }
-        }
+      for (int it = 0; it < WCOLS * 8 / 64; ++it) {
+        const int t = it * 8 + lane / 8, token = col0 + t;
+        const float4 v4 = *reinterpret_cast<const float4*>(scratch + t * 128 + ((j ^ token_swizzle(t)) << 4));
+        if (token < p.n && row < row_limit)
+          *reinterpret_cast<u32x4_any_t*>(reinterpret_cast<float*>(d_out) + (size_t)token * p.m + row) =
+              __builtin_bit_cast(u32x4_t, float4{v4.x + bias4[0], v4.y + bias4[1], v4.z + bias4[2], v4.w + bias4[3]});
       }
     }
     return;

@@ -29,8 +29,6 @@ hipError_t launch_gemm_tokens(GemmArgs args, int tile_config, hipStream_t stream
   args.beta = 0.f;
   args.c = nullptr;
   auto pass = [&](GemmArgs a) {
-    a.vector_epilogue = (reinterpret_cast<uintptr_t>(a.d) & 15) == 0 && a.m % 8 == 0 &&
-                        (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0;
     return a.bf16 ? launch_tokens_tile<true>(a, tile_config, stream) : launch_tokens_tile<false>(a, tile_config, stream);
   };
   if (args.splits <= 1) {
