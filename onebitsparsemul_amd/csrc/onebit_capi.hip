@@ -251,7 +251,12 @@ GemmPlan plan_gemm(int m, int n, int k, int compute_units) {
   // idles and the schedule decides (4096 x 3072 x 4096 with 192 tiles: 51.2 against 50.6; 11008 x 768 x 4096: 49 against 41).
   if (best.tile == onebit::kTile512x128w8 && best.splits == 1) {
     const long tiles = (long)((m + 511) / 512) * ((n + 127) / 128);
-    if (tiles * 20 >= 17L * compute_units) best.tile = onebit::kTile512x128m16;  // from 85 % of a round on
+    // From 85 % of a round on; on K from 43 chunks on, where the epilogue of its four wavefronts weighs less, from three quarters on.
+    // us, eight wavefronts | four (layers in fp16 with a bias, layers with fp32 results, products, products with C and fp32 results):
+    // 4096 x 11008 with 3072 125 | 120, 127 | 127, 124 | 120, 136 | 134; 8192 x 16384 with 1600 194 | 185, 195 | 186, 193 | 185, 204 |
+    // 197; bf16 layers 4096 x 11008 with 3072 118 | 114. On K = 8192 what is stored as fp32 or has C is slower (8192 x 8192 with 1408
+    // 94 | 97 and 102 | 104, fp16 layers 92 | 91).
+    if (tiles * 20 >= 17L * compute_units || (chunks >= 43 && tiles * 4 >= 3L * compute_units)) best.tile = onebit::kTile512x128m16;
   }
   return best;
 }
