@@ -17,7 +17,7 @@ EXPORTS = (
     "onebit_sparse_set_skinny_enabled", "onebit_sparse_set_skinny_rows", "onebit_sparse_set_split_k", "onebit_sparse_set_pad_b", "onebit_sparse_describe_launch", "onebit_sparse_set_weight_cache", "onebit_sparse_clear_weight_cache", "onebit_sparse_release_buffers",
     "onebit_sparse_measure_smfmac_rate", "onebit_sparse_device_info",
     "onebit_sparse_describe_launch_for", "onebit_sparse_measure_smfmac_rate_shape",
-    "onebit_sparse_linear_prepared_grouped", "onebit_sparse_pack_typed", "onebit_sparse_linear_prepared_typed", "onebit_sparse_linear_prepared_f32",
+    "onebit_sparse_linear_prepared_grouped", "onebit_sparse_pack_typed", "onebit_sparse_linear_prepared_typed", "onebit_sparse_linear_prepared_f32", "onebit_sparse_linear_reads_f32",
     "onebit_sparse_linear_prepared_grouped_typed", "onebit_sparse_describe_call",
 )
 
@@ -55,6 +55,8 @@ def lib():
         L.onebit_sparse_linear_prepared_grouped.argtypes = [ctypes.POINTER(LinearProblem), i32, i32, i32, i32, vp]
         L.onebit_sparse_pack.restype = i32
         L.onebit_sparse_pack.argtypes = [vp, i32, i32, i32, vp, vp, i32, vp]
+        L.onebit_sparse_linear_reads_f32.restype = i32
+        L.onebit_sparse_linear_reads_f32.argtypes = [i32, i32, i32]
         L.onebit_sparse_linear_prepared_f32.restype = i32
         L.onebit_sparse_linear_prepared_f32.argtypes = [vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]
         L.onebit_sparse_linear_prepared_typed.restype = i32

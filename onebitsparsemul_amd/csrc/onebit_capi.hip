@@ -702,6 +702,9 @@ int matmul_prepared_impl(const void* prepared, const void* b, const void* c, voi
   return ONEBIT_OK;
 }
 
+// Whether fp32 activations of that many tokens go through the kernel that rounds them itself (skinny_kernel).
+bool takes_f32(int tokens) { return tokens <= onebit::kSkinnyTokens && g_skinny_enabled; }
+
 // The layer's product on 16-bit activations of either type, or up to sixteen tokens of fp32 ones (x_dtype).
 int linear_prepared_impl(const void* prepared, const void* x, const void* bias, void* y, int tokens, int m, int k, int x_dtype,
                          int bias_dtype, int y_dtype, hipStream_t s) {
@@ -918,10 +921,15 @@ int onebit_sparse_linear_prepared_f32(const void* prepared, const void* x, const
   g_last_error.clear();
   if (int rc = check_shape(m, tokens, k)) return rc;
   if (int rc = check_linear_dtypes(ONEBIT_DTYPE_F16, bias_dtype, y_dtype)) return rc;
-  if (tokens > onebit::kSkinnyTokens || !g_skinny_enabled)
+  if (!takes_f32(tokens))
     return fail(ONEBIT_ERR_ARGUMENT, "fp32 activations are read by the kernel of up to %d tokens only (got %d): convert them to fp16",
                 onebit::kSkinnyTokens, tokens);
   return linear_prepared_impl(prepared, x, bias, y, tokens, m, k, ONEBIT_DTYPE_F32, bias_dtype, y_dtype, static_cast<hipStream_t>(stream));
+}
+
+int onebit_sparse_linear_reads_f32(int tokens, int m, int k) {
+  g_last_error.clear();
+  return check_shape(m, tokens, k) == ONEBIT_OK && takes_f32(tokens);
 }
 
 int onebit_sparse_linear_prepared_grouped(const onebit_linear_problem* problems, int count, int tokens, int bias_dtype,

@@ -126,9 +126,6 @@ int64_t token_count(const torch::Tensor& x, int64_t k) {
   return tokens;
 }
 
-// Most tokens of fp32 activations that onebit_sparse_linear_prepared_f32 takes.
-constexpr int64_t kF32Tokens = 16;
-
 // BinaryLinear_2_4.forward behind its bookkeeping: y = x W^T (+ bias), shape and type of the layer's result. Nothing where x is on
 // another device than the prepared weight: the layer then prepares its weight there.
 OptionalTensor layer_forward(const torch::Tensor& prepared, const torch::Tensor& x, const OptionalTensor& bias, int64_t m,
@@ -143,24 +140,21 @@ OptionalTensor layer_forward(const torch::Tensor& prepared, const torch::Tensor&
   const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device);
   const LayerTypes types = layer_types(x.scalar_type(), out_dtype);
   // fp32 activations of a few tokens are rounded by the kernel that reads them, all others by a conversion in front of it
-  bool read_f32 = x.scalar_type() == torch::kFloat32 && tokens <= kF32Tokens && x.is_contiguous() &&
-                  reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
-  torch::Tensor in;
-  if (!read_f32) in = kernel_input(x, types.in);
+  const bool read_f32 = x.scalar_type() == torch::kFloat32 && x.is_contiguous() &&
+                        reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+                        onebit_sparse_linear_reads_f32((int)tokens, (int)m, (int)k);
+  const torch::Tensor in = read_f32 ? x : kernel_input(x, types.in);
   OptionalTensor b;
   if (bias.has_value()) b = kernel_bias(*bias, device, m);
   torch::Tensor y = empty_result(result_sizes(x, m), types.out, device);
   const void* const bias_data = b.has_value() ? b->data_ptr() : nullptr;
   const int bias_code = b.has_value() ? dtype_code(b->scalar_type()) : ONEBIT_DTYPE_F16;
-  if (read_f32 && onebit_sparse_linear_prepared_f32(prepared.data_ptr(), x.data_ptr(), bias_data, y.data_ptr(), (int)tokens, (int)m,
-                                                    (int)k, bias_code, dtype_code(types.out), current_stream(device)) != ONEBIT_OK) {
-    read_f32 = false;  // the kernel is switched off
-    in = kernel_input(x, types.in);
-  }
-  if (!read_f32)
-    check_status(onebit_sparse_linear_prepared_typed(prepared.data_ptr(), in.data_ptr(), bias_data, y.data_ptr(), (int)tokens, (int)m,
-                                                     (int)k, dtype_code(types.in), bias_code, dtype_code(types.out),
-                                                     current_stream(device)));
+  check_status(read_f32
+                   ? onebit_sparse_linear_prepared_f32(prepared.data_ptr(), in.data_ptr(), bias_data, y.data_ptr(), (int)tokens,
+                                                       (int)m, (int)k, bias_code, dtype_code(types.out), current_stream(device))
+                   : onebit_sparse_linear_prepared_typed(prepared.data_ptr(), in.data_ptr(), bias_data, y.data_ptr(), (int)tokens,
+                                                         (int)m, (int)k, dtype_code(types.in), bias_code, dtype_code(types.out),
+                                                         current_stream(device)));
   return out_dtype.has_value() || types.out == x.scalar_type() ? y : y.to(x.scalar_type());
 }
 

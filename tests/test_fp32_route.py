@@ -1,0 +1,40 @@
+"""Which fp32 activations of a layer the kernel reads itself, and which are converted in front of it."""
+import pytest
+import torch
+
+from onebitsparsemul_amd import BinaryLinear_2_4, _native, synthetic
+
+
+@pytest.fixture(autouse=True)
+def _defaults():
+    yield
+    _native.set_skinny_rows(-1)
+    _native.set_skinny_enabled(True)
+
+
+def _layer(m, k):
+    a, meta = synthetic.make_weight(m, k, seed=m + k)
+    layer = BinaryLinear_2_4(k, m).cuda()
+    layer.load_state_dict({"packed_binary_sparse": a.cuda(), "meta": meta.cuda()})
+    return layer
+
+
+def test_few_tokens_through_the_kernel_that_is_on():
+    reads = _native.lib().onebit_sparse_linear_reads_f32
+    assert reads(1, 4096, 4096) == 1 and reads(16, 4096, 4096) == 1 and reads(17, 4096, 4096) == 0
+    assert reads(0, 4096, 4096) == 0 and reads(4, 100, 4096) == 0
+    _native.set_skinny_enabled(False)
+    assert reads(1, 4096, 4096) == 0
+
+
+@pytest.mark.gpu
+def test_a_failed_call_is_not_made_again():
+    """A refused call raises where it was refused: no conversion, no second attempt whose success or error would stand for it."""
+    layer = _layer(128, 512)
+    x = torch.randn(4, 512, device="cuda")
+    layer(x)
+    _native.set_skinny_rows(96)  # no such row group: the launch is refused on the host
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    with pytest.raises(RuntimeError):
+        layer(x)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == 1  # the result, no converted copy of x
