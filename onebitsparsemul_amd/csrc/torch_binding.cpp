@@ -126,6 +126,12 @@ int64_t token_count(const torch::Tensor& x, int64_t k) {
   return tokens;
 }
 
+// Whether the values of a contiguous tensor are what lies in its memory: a negated view's sign is applied by the next operation on it
+// (here a conversion), and a subclass that handles operations itself may keep its values elsewhere.
+bool values_in_memory(const torch::Tensor& x) {
+  return !x.is_neg() && !x._is_zerotensor() && !x.unsafeGetTensorImpl()->is_python_dispatch();
+}
+
 // BinaryLinear_2_4.forward behind its bookkeeping: y = x W^T (+ bias), shape and type of the layer's result. Nothing where x is on
 // another device than the prepared weight: the layer then prepares its weight there.
 OptionalTensor layer_forward(const torch::Tensor& prepared, const torch::Tensor& x, const OptionalTensor& bias, int64_t m,
@@ -140,7 +146,7 @@ OptionalTensor layer_forward(const torch::Tensor& prepared, const torch::Tensor&
   const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device);
   const LayerTypes types = layer_types(x.scalar_type(), out_dtype);
   // fp32 activations of a few tokens are rounded by the kernel that reads them, all others by a conversion in front of it
-  const bool read_f32 = x.scalar_type() == torch::kFloat32 && x.is_contiguous() &&
+  const bool read_f32 = x.scalar_type() == torch::kFloat32 && x.is_contiguous() && values_in_memory(x) &&
                         reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
                         onebit_sparse_linear_reads_f32((int)tokens, (int)m, (int)k);
   const torch::Tensor in = read_f32 ? x : kernel_input(x, types.in);

@@ -38,3 +38,27 @@ def test_a_failed_call_is_not_made_again():
     with pytest.raises(RuntimeError):
         layer(x)
     assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == 1  # the result, no converted copy of x
+
+
+class _Elsewhere(torch.Tensor):
+    """fp32 values that arrive with the conversion, none in the tensor's own memory"""
+
+    @staticmethod
+    def __new__(cls, values):
+        self = torch.Tensor._make_wrapper_subclass(cls, values.shape, dtype=torch.float32, device=values.device)
+        self.values = values
+        return self
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        assert func in (torch.ops.aten.to.dtype, torch.ops.aten._to_copy.default), func
+        return args[0].values.to(args[1] if len(args) > 1 else kwargs["dtype"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [1, 16])
+def test_values_that_are_not_what_lies_in_memory(tokens):
+    layer = _layer(128, 512)
+    x = torch.randn(tokens, 512, device="cuda")
+    assert torch.equal(layer(torch._neg_view(x)), layer(-x))
+    assert torch.equal(layer(_Elsewhere(x)), layer(x))
