@@ -9,8 +9,6 @@ host computation.
 import torch
 import torch.nn as nn
 
-from torch.nn.modules.module import _global_buffer_registration_hooks as _buffer_hooks
-
 from . import _native
 from ._semi_structured_conversions import (
     mask_creator,
@@ -162,12 +160,17 @@ class BinaryLinear_2_4(nn.Module):
                 weight = weight.clone()  # a view that starts inside a 16-byte unit
             a, meta = _binding().pack_weight(weight, True, _native.META_REFERENCE)
             buffers = self._buffers
-            if "packed_binary_sparse" in buffers and "meta" in buffers and not _buffer_hooks:
-                # where nn.Module.__setattr__ puts a registered buffer, without its 1.5 us per attribute
+            # where nn.Module.__setattr__ puts a registered buffer, without its 1.5 us per attribute: not for a class that sets
+            # attributes its own way, nor where a registration hook is to see the buffer (or torch keeps those elsewhere)
+            if (type(self).__setattr__ is nn.Module.__setattr__ and "packed_binary_sparse" in buffers and "meta" in buffers
+                    and getattr(nn.modules.module, "_global_buffer_registration_hooks", None) == {}):
                 buffers["packed_binary_sparse"], buffers["meta"] = a, meta
+                object.__setattr__(self, "vaild", True)
+                object.__setattr__(self, "_prepared", None)
             else:
                 self.packed_binary_sparse, self.meta = a, meta
-            self.__dict__.update(vaild=True, _prepared=None)
+                self.vaild = True
+                self._prepared = None
             return
         w = weight * mask_creator(weight).to(weight.dtype)
         if w.dtype not in (torch.half, torch.bfloat16, torch.int32):
