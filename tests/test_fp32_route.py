@@ -27,6 +27,29 @@ def test_few_tokens_through_the_kernel_that_is_on():
     assert reads(1, 4096, 4096) == 0
 
 
+@pytest.mark.parametrize("tokens,m,k,faster", [
+    (16, 4096, 9568, 1), (16, 4096, 9600, 0), (9, 4096, 12256, 1), (9, 4096, 12288, 0),  # one round of workgroups
+    (8, 4096, 28672, 1), (16, 4096, 28672, 1), (16, 8192, 28672, 0), (16, 11008, 28672, 0),  # K in four, in two, not split
+    (8, 7168, 18720, 1), (8, 7168, 18752, 0), (5, 11008, 28672, 1),                      # up to eight tokens
+    (16, 32768, 4096, 1), (16, 32768 + 64, 4096, 0), (16, 49152, 2048, 1), (8, 49152, 8192, 1), (8, 131072, 8192, 0),  # more rounds
+])
+def test_where_reading_fp32_is_faster(tokens, m, k, faster):
+    assert _native.lib().onebit_sparse_linear_reads_f32(tokens, m, k) == faster
+
+
+@pytest.mark.gpu
+def test_the_layer_converts_where_that_is_faster():
+    m, k = 11008, 28672
+    layer, x = _layer(m, k), torch.randn(16, k, device="cuda")
+    layer(x)
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    y = layer(x)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == 2  # the converted copy and the result
+    want = torch.empty_like(y)
+    _native.linear_prepared(layer._prepared.buffer, x.half(), want, m, k)
+    assert torch.equal(y, want)
+
+
 @pytest.mark.gpu
 def test_a_failed_call_is_not_made_again():
     """A refused call raises where it was refused: no conversion, no second attempt whose success or error would stand for it."""
