@@ -618,44 +618,48 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   }
 }
 
-// A kernel's arguments as three vectors. The hardware puts the first two, twelve dwords, into scalar registers before a
-// wavefront starts (the build asks for that); out of a struct they would have to be loaded, 0.2 us before the first address can
-// be formed. Vectors, because the host pays for every argument of a launch. us inside a HIP graph, weights from HBM, struct ->
-// this: 11008 x 4096 with 1 / 4 / 16 tokens 5.16 / 5.35 / 5.91 -> 5.00 / 5.02 / 5.63, 28672 x 8192 with one 12.5 -> 12.2,
-// 11008 x 3 x 4096 6.35 -> 6.08.
+// A kernel's arguments as three vectors of fourteen dwords in all, which the hardware puts into scalar registers before a wavefront
+// starts (the build asks for that); out of a struct they would have to be loaded, 0.2 us before the first address can be formed.
+// Vectors, because the host pays for every argument of a launch. us inside a HIP graph, weights from HBM, struct -> this: 11008 x
+// 4096 with 1 / 4 / 16 tokens 5.58 / 5.56 / 6.48 -> 5.10 / 5.10 / 6.27, 28672 x 8192 with one 13.2 -> 12.7, 11008 x 4 x 4096 6.25 ->
+// 5.94. With flags, alpha and beta in a fourth vector that is loaded where the results are stored, the smallest calls were slower than
+// with the struct: 512 x 2 x 512 2.93 | 3.09 | 2.87 as a struct | so | now, 512 x 4 x 512 2.84 | 2.86 | 2.78, 512 x 3 x 512 2.81 | 2.97 |
+// 2.88.
 enum ArgFlags : uint32_t { kArgD16 = 1, kArgC16 = 2, kArgBias = 4 };  // bits 3 and 4: type of the bias
 struct LaunchArgs {
-  u32x8_t operands;  // prep, b; n, k, m, chunks_per_split
+  u32x8_t operands;  // prep, b; n, k, m, chunks_per_split (chunks of 256 of an int K: 23 bits; what a kernel adds from bit 24 on)
   u32x4_t results;   // d, the bias (token-major form) or C: a call has one of them at most
-  u32x4_t epilogue;  // ArgFlags, alpha, beta
+  u32x2_t scale;     // alpha, beta
+  uint32_t flags;
 };
 static LaunchArgs pack_args(const SkinnyArgs& a) {
   const uint64_t prep = (uint64_t)a.prep, b = (uint64_t)a.b, d = (uint64_t)a.d, extra = (uint64_t)(a.bias ? a.bias : a.c);
-  const uint32_t flags = (a.d_f16 ? kArgD16 : 0) | (a.c_f16 ? kArgC16 : 0) | (a.bias ? kArgBias : 0) | (uint32_t)a.bias_type << 3;
   return LaunchArgs{u32x8_t{(uint32_t)prep, (uint32_t)(prep >> 32), (uint32_t)b, (uint32_t)(b >> 32), (uint32_t)a.n, (uint32_t)a.k,
                             (uint32_t)a.m, (uint32_t)a.chunks_per_split},
                     u32x4_t{(uint32_t)d, (uint32_t)(d >> 32), (uint32_t)extra, (uint32_t)(extra >> 32)},
-                    u32x4_t{flags, __builtin_bit_cast(uint32_t, a.alpha), __builtin_bit_cast(uint32_t, a.beta), 0u}};
+                    u32x2_t{__builtin_bit_cast(uint32_t, a.alpha), __builtin_bit_cast(uint32_t, a.beta)},
+                    (a.d_f16 ? kArgD16 : 0) | (a.c_f16 ? kArgC16 : 0) | (a.bias ? kArgBias : 0) | (uint32_t)a.bias_type << 3};
 }
-__device__ __forceinline__ SkinnyArgs unpack_args(u32x8_t operands, u32x4_t results, u32x4_t epilogue) {
+__device__ __forceinline__ SkinnyArgs unpack_args(u32x8_t operands, u32x4_t results, u32x2_t scale, uint32_t flags) {
   auto pointer = [](uint32_t low, uint32_t high) __attribute__((always_inline)) { return (uint64_t)high << 32 | low; };
   SkinnyArgs p{};
   p.prep = reinterpret_cast<const uint8_t*>(pointer(operands[0], operands[1]));
   p.b = reinterpret_cast<const _Float16*>(pointer(operands[2], operands[3]));
-  p.n = operands[4]; p.k = operands[5]; p.m = operands[6]; p.chunks_per_split = operands[7];
+  p.n = operands[4]; p.k = operands[5]; p.m = operands[6]; p.chunks_per_split = operands[7] & 0xFFFFFFu;
   p.kc_total = (p.k + kChunkK - 1) / kChunkK;
   p.d = reinterpret_cast<void*>(pointer(results[0], results[1]));
   p.c = reinterpret_cast<const void*>(pointer(results[2], results[3]));  // read where beta != 0 only: never with a bias
-  p.bias = epilogue[0] & kArgBias ? p.c : nullptr;
-  p.d_f16 = epilogue[0] & kArgD16; p.c_f16 = epilogue[0] & kArgC16; p.bias_type = epilogue[0] >> 3 & 3;
+  p.bias = flags & kArgBias ? p.c : nullptr;
+  p.d_f16 = flags & kArgD16; p.c_f16 = flags & kArgC16; p.bias_type = flags >> 3 & 3;
   // (values, not elements: the compiler casts the bits of a vector's first element where an element is named)
-  p.alpha = __builtin_bit_cast(float, (uint32_t)epilogue[1]); p.beta = __builtin_bit_cast(float, (uint32_t)epilogue[2]);
+  p.alpha = __builtin_bit_cast(float, (uint32_t)scale[0]); p.beta = __builtin_bit_cast(float, (uint32_t)scale[1]);
   return p;
 }
 
+// operands[7]: ArgFlags from bit 24 on
 template <int NW, int R, int MODE, int NC, bool BF16>
-__global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_kernel(u32x8_t operands, u32x4_t results, u32x4_t epilogue) {
-  const SkinnyArgs p = unpack_args(operands, results, epilogue);
+__global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_kernel(u32x8_t operands, u32x4_t results, u32x2_t scale) {
+  const SkinnyArgs p = unpack_args(operands, results, scale, operands[7] >> 24);
   skinny_body<NW, R, MODE, NC, BF16>(p, blockIdx.x, blockIdx.y);
 }
 
@@ -754,8 +758,9 @@ static hipError_t launch_skinny_mode(const SkinnyArgs& args, hipStream_t stream)
       return hipGetLastError();
     }
   if constexpr (!kPieces || NC == 16) {
-    const LaunchArgs a = pack_args(args);
-    hipLaunchKernelGGL((skinny_kernel<NW, R, MODE, NC, BF16>), grid, threads, 0, stream, a.operands, a.results, a.epilogue);
+    LaunchArgs a = pack_args(args);
+    a.operands[7] |= a.flags << 24;
+    hipLaunchKernelGGL((skinny_kernel<NW, R, MODE, NC, BF16>), grid, threads, 0, stream, a.operands, a.results, a.scale);
   }
   return hipGetLastError();
 }

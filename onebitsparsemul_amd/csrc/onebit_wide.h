@@ -421,8 +421,7 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
 template <int R, int COPIES, bool TOKENS, bool BF16>
 __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_kernel(u32x8_t operands, u32x4_t results, u32x2_t shape, u32x4_t rest) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  SkinnyArgs p = unpack_args(operands, results, u32x4_t{shape[0], rest[2], rest[3], 0u});
-  p.chunks_per_split = operands[7] & 0xFFFFFFu;
+  SkinnyArgs p = unpack_args(operands, results, u32x2_t{rest[2], rest[3]}, shape[0]);
   p.tokens_per_group = operands[7] >> 24;
   p.ldb = shape[1];
   int x = blockIdx.x, group = blockIdx.z;
@@ -460,8 +459,8 @@ static hipError_t launch_wide_kernel(const SkinnyArgs& args, hipStream_t stream)
   const bool strips = groups > 1 && (!TOKENS || args.n > kSkinnyMaxN);
   LaunchArgs a = pack_args(args);
   a.operands[7] |= (uint32_t)args.tokens_per_group << 24;  // chunks of 256 of an int K: 23 bits
-  const u32x2_t shape = {a.epilogue[0] | (strips ? (uint32_t)rows << 5 : 0u), (uint32_t)args.ldb};
-  const u32x4_t rest = {(uint32_t)((uint64_t(1) << 32) / (2 * rows) + 1), (uint32_t)(rows * groups), a.epilogue[1], a.epilogue[2]};
+  const u32x2_t shape = {a.flags | (strips ? (uint32_t)rows << 5 : 0u), (uint32_t)args.ldb};
+  const u32x4_t rest = {(uint32_t)((uint64_t(1) << 32) / (2 * rows) + 1), (uint32_t)(rows * groups), a.scale[0], a.scale[1]};
   const dim3 grid = strips ? dim3(rows * groups, args.splits) : dim3(rows, args.splits, groups);
   hipLaunchKernelGGL(kern, grid, dim3(64 * kWideWaves), lds, stream, a.operands, a.results, shape, rest);
   return hipGetLastError();
