@@ -1,5 +1,4 @@
-"""The split-K kernel's two argument forms, on either side of the line between them (sixteen chunks of K per split and fewer, or
-more), with all that a call can pass: C of either type, alpha, beta, results of either type, K split or not. Integer operands:
+"""The split-K kernel's two argument forms, on either side of the lines between them (eight and sixteen chunks of K per split), with all that a call can pass: C of either type, alpha, beta, results of either type, K split or not. Integer operands:
 bit-exact."""
 import numpy as np
 import pytest
@@ -22,7 +21,7 @@ def _defaults():
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 8, 13, 16, 18, 32, 41, 64])
 def test_every_argument_reaches_the_kernel(rows, n):
     _native.set_skinny_rows(rows)
-    for m, k, splits in ((192, 4096, 1), (192, 4128, 1), (64, 8192, 2), (64, 8224, 2)):
+    for m, k, splits in ((192, 2048, 1), (192, 2080, 1), (192, 4096, 1), (192, 4128, 1), (64, 8192, 2), (64, 8224, 2)):
         _native.set_split_k(splits)
         a, meta = synthetic.make_weight(m, k, seed=n + k)
         prepared = _native.prepare(a.cuda(), meta.cuda(), m, k)
