@@ -392,6 +392,23 @@ WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, 
   return best;
 }
 
+// Whether wide_kernel walks its grid in strips of two column groups. Dealt over the XCDs by row groups, every XCD fetches all of x
+// and, where their number is no multiple of eight, the same rows of the weight for several of the column groups; in strips it fetches
+// a few column groups of x and a part of the rows. That pays where all of x does not fit an XCD's L2 (4 MB), and where x and the
+// weight are large enough for the second fetch to show, the earlier the more XCDs repeat it. us inside HIP graphs, weights from HBM, dealt
+// | strips: x of 4 MB and more: 2048 x 256 x 8192 14.1 | 12.3, layers 1024 x 4096 with 1000 tokens 14.5 | 12.6, 6784 x 9984 with
+// 537 54.8 | 52.2; an odd number of row groups: layers 960 x 6528 with 415 10.5 | 8.0, 3456 x 4640 with 135 10.1 | 9.2, 1984 x 2784 with
+// 123 5.3 | 4.8; below: layers 512 x 1024 with 500 3.15 | 3.40, 4096 x 4096 with 200 8.0 | 8.7, products 4096 x 256 x 4096 9.4 |
+// 10.1, 1024 x 64 x 4096 5.0 | 5.35, 704 x 48 x 2976 4.75 | 4.55. On 700 calls in several column groups this rule is 3.8 % faster in
+// the mean than strips wherever there are several (with their parameters loaded); eight are more than 2 % slower.
+bool wide_in_strips(int m, int n, int k, const WidePlan& plan, bool plain, int compute_units) {
+  const int column_groups = (n + plan.tokens - 1) / plan.tokens, row_groups = (m + plan.rows - 1) / plan.rows;
+  // a layer's x of up to 64 tokens lies in every L2; the walk is made for eight XCDs of 32 compute units
+  if (column_groups < 2 || (!plain && n <= onebit::kSkinnyMaxN) || compute_units != 256) return false;
+  const double x = 2.0 * n * k, both = x + 0.1875 * m * k;
+  return x >= 4e6 || (row_groups % 2 ? both >= 1.5e6 : row_groups % 4 ? both >= 3.5e6 : false);
+}
+
 LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int compute_units, bool tokens = false) {
   LaunchPlan plan{};
   // 32 < n <= 64: every 64-row workgroup of the split-K kernel stages all of B, which the main kernel's tiles overtake
@@ -610,6 +627,7 @@ int matmul_prepared_impl(const void* prepared, const void* b, const void* c, voi
     args.c_f16 = c_dtype == ONEBIT_DTYPE_F16;
     args.d_f16 = d_dtype == ONEBIT_DTYPE_F16;
     args.tokens_per_group = wide.tokens;
+    args.strips = wide.rows && wide_in_strips(m, n, k, wide, true, compute_units);
     args.ldb = n;
     DeviceLock lock;
     if (int rc = setup_skinny_split(args, wide.rows ? wide.splits : plan.splits, plan.splits, stream, fixed, lock); rc != ONEBIT_OK)
@@ -650,6 +668,7 @@ int matmul_prepared_impl(const void* prepared, const void* b, const void* c, voi
     w.chunks_per_split = args.chunks_per_split;
     w.split_ws = args.split_ws;
     w.tokens_per_group = wide.tokens;
+    w.strips = wide_in_strips(m, n, k, wide, true, compute_units);
     w.ldb = n;
     if (pad_b) {
       if (hipError_t st = onebit::launch_pad_b(args.b, args.b_pad, k, n, stream); st != hipSuccess) return st;
@@ -728,7 +747,8 @@ int linear_prepared_impl(const void* prepared, const void* x, const void* bias, 
   if (!prepared || !x || !y) return fail(ONEBIT_ERR_ARGUMENT, "null operand pointer");
   if ((reinterpret_cast<uintptr_t>(x) & 15) != 0) return fail(ONEBIT_ERR_ARGUMENT, "x must be 16-byte aligned");
   const int kc_total = (k + onebit::kChunkK - 1) / onebit::kChunkK;
-  const LinearPlan linear = plan_linear(m, tokens, k, current_compute_units());
+  const int compute_units = current_compute_units();
+  const LinearPlan linear = plan_linear(m, tokens, k, compute_units);
   const LaunchPlan& plan = linear.launch;
   if ((size_t)k * 256 * 2 >= (size_t(1) << 32))
     return fail(ONEBIT_ERR_ARGUMENT, "the token-major form addresses x with 32-bit offsets inside a tile of 256 tokens: "
@@ -751,6 +771,7 @@ int linear_prepared_impl(const void* prepared, const void* x, const void* bias, 
         rc != ONEBIT_OK)
       return rc;
     args.tokens_per_group = linear.wide_plan.tokens;
+    args.strips = linear.wide && wide_in_strips(m, tokens, k, linear.wide_plan, false, compute_units);
     ONEBIT_HIP(linear.wide ? onebit::launch_wide_tokens(args, linear.wide_plan.rows, s)
                            : onebit::launch_skinny_tokens(args, plan.rows_or_tile, s));
     return ONEBIT_OK;

@@ -58,9 +58,10 @@ struct SkinnyArgs {
   float* split_ws;
   // launch_skinny_tokens only: b is x in fp32, rounded to fp16 as it is read (bf16 = 0)
   int x_f32;
-  // wide_kernel only: tokens (columns) a workgroup multiplies (at most 64), grid.z = ceil(n / tokens_per_group); ldb: elements
-  // between B rows in the plain form
+  // wide_kernel only: tokens (columns) a workgroup multiplies (at most 64); strips: the grid is walked in strips of two column
+  // groups, on a device of eight XCDs; ldb: elements between B rows in the plain form, n rounded up to eight
   int tokens_per_group;
+  int strips;
   int ldb;
 };
 

@@ -408,27 +408,24 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
   }
 }
 
-// Workgroups of several column groups walk the grid in strips of two of them: an XCD is given a contiguous range of the list
-// (workgroup b runs on XCD b % 8), so that what its workgroups read of x and of the weight meets in its L2. In the plain form the
-// column groups share the lines of B's rows, and with the row groups dealt over the XCDs each of those fetched every line (us,
-// row groups dealt -> strips: 2048 x 256 x 4096 9.0 -> 7.3, 4096 x 128 x 4096 7.7 -> 7.3; token-major 4096 x 11008 with 512 tokens
-// 31.2 -> 30.2).
-// Arguments as for skinny_kernel, but: operands[7] holds chunks_per_split and, from bit 24 on, the columns per workgroup; shape[0]
-// ArgFlags and, from bit 5 on, the row groups (0: the grid has the column groups as its third dimension); shape[1] is ldb; rest = 2^32 / (2 row groups) + 1,
-// workgroups, alpha, beta. All but `rest` is in registers from the start, and the token-major form of up to 64 tokens, where a load
-// at the start or in the epilogue would show most, does not need it: its x lies in every L2, strips gain nothing (1024 x 1024 with
-// 24 tokens 2.71 -> 2.81 us, 4096 x 4096 with 64 5.08 -> 5.18).
+// Arguments as for skinny_kernel, but: operands[7] holds the columns per workgroup from bit 24 on; shape[0] ArgFlags and, from bit 5
+// on, the column groups of a grid that is walked in strips (0: the grid has them as its third dimension), shape[1] 2^32 / (2 row
+// groups) + 1. `scale`, which the token-major form does not use, is the only argument that is not in registers from the start.
+// In strips of two column groups an XCD is given a contiguous range of the list (workgroup b runs on XCD b % 8, all eight are there:
+// the launcher's condition), so that what its workgroups read of x and of the weight meets in its L2; where that pays is the host's
+// rule (wide_in_strips).
 template <int R, int COPIES, bool TOKENS, bool BF16>
-__global__ __launch_bounds__(64 * kWideWaves, 2) void wide_kernel(u32x8_t operands, u32x4_t results, u32x2_t shape, u32x4_t rest) {
+__global__ __launch_bounds__(64 * kWideWaves, 2) void wide_kernel(u32x8_t operands, u32x4_t results, u32x2_t shape, u32x2_t scale) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  SkinnyArgs p = unpack_args(operands, results, u32x2_t{rest[2], rest[3]}, shape[0]);
+  SkinnyArgs p = unpack_args(operands, results, scale, shape[0]);
   p.tokens_per_group = operands[7] >> 24;
-  p.ldb = shape[1];
+  p.ldb = (p.n + 7) & ~7;  // the launcher's condition
   int x = blockIdx.x, group = blockIdx.z;
-  if (const int row_groups = shape[0] >> 5; row_groups > 0) {
-    const int total = rest[1], per = total / 8, rem = total % 8, xcd = x % 8;
+  if (const int groups = shape[0] >> 5; groups > 0) {
+    const int row_groups = (p.m + 32 * R - 1) / (32 * R);
+    const int total = row_groups * groups, per = total / 8, rem = total % 8, xcd = x % 8;
     const int v = xcd * per + (xcd < rem ? xcd : rem) + x / 8;
-    int strip = (int)__umulhi((uint32_t)v, rest[0]), w = v - strip * 2 * row_groups;
+    int strip = (int)__umulhi((uint32_t)v, shape[1]), w = v - strip * 2 * row_groups;
     if (w < 0) --strip, w += 2 * row_groups;  // the reciprocal is rounded up
     const bool pair = 2 * (strip + 1) * row_groups <= total;
     x = pair ? w >> 1 : w;
@@ -456,13 +453,11 @@ static hipError_t launch_wide_kernel(const SkinnyArgs& args, hipStream_t stream)
   const auto kern = wide_kernel<R, COPIES, TOKENS, BF16>;
   if (hipError_t st = wide_lds_limit(reinterpret_cast<const void*>(kern), lds, attr_done); st != hipSuccess) return st;
   const int rows = (args.m + 32 * R - 1) / (32 * R), groups = (args.n + args.tokens_per_group - 1) / args.tokens_per_group;
-  const bool strips = groups > 1 && (!TOKENS || args.n > kSkinnyMaxN);
   LaunchArgs a = pack_args(args);
-  a.operands[7] |= (uint32_t)args.tokens_per_group << 24;  // chunks of 256 of an int K: 23 bits
-  const u32x2_t shape = {a.flags | (strips ? (uint32_t)rows << 5 : 0u), (uint32_t)args.ldb};
-  const u32x4_t rest = {(uint32_t)((uint64_t(1) << 32) / (2 * rows) + 1), (uint32_t)(rows * groups), a.scale[0], a.scale[1]};
-  const dim3 grid = strips ? dim3(rows * groups, args.splits) : dim3(rows, args.splits, groups);
-  hipLaunchKernelGGL(kern, grid, dim3(64 * kWideWaves), lds, stream, a.operands, a.results, shape, rest);
+  a.operands[7] |= (uint32_t)args.tokens_per_group << 24;
+  const u32x2_t shape = {a.flags | (args.strips ? (uint32_t)groups << 5 : 0u), (uint32_t)((uint64_t(1) << 32) / (2 * rows) + 1)};
+  const dim3 grid = args.strips ? dim3(rows * groups, args.splits) : dim3(rows, args.splits, groups);
+  hipLaunchKernelGGL(kern, grid, dim3(64 * kWideWaves), lds, stream, a.operands, a.results, shape, a.scale);
   return hipGetLastError();
 }
 

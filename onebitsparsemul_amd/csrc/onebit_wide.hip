@@ -17,8 +17,7 @@ static hipError_t launch_wide_columns(const SkinnyArgs& args, hipStream_t stream
 hipError_t launch_wide(SkinnyArgs args, int rows_per_group, hipStream_t stream) {
   const int columns = args.tokens_per_group;
   // 16-byte copies of B's rows, 32-bit offsets inside an image
-  if (args.n < 1 || columns < 1 || columns > kSkinnyMaxN || columns % 8 != 0 || rows_per_group < 1 || args.ldb < args.n ||
-      args.ldb % 8 != 0 || (reinterpret_cast<uintptr_t>(args.b) & 15) != 0 || (size_t)args.ldb * 128 >= (size_t(1) << 32))
+  if (args.n < 1 || columns < 1 || columns > kSkinnyMaxN || columns % 8 != 0 || rows_per_group < 1 || args.ldb != (args.n + 7) / 8 * 8 || (reinterpret_cast<uintptr_t>(args.b) & 15) != 0 || (size_t)args.ldb * 128 >= (size_t(1) << 32))
     return hipErrorInvalidValue;
   SkinnyArgs pass;
   if (hipError_t st = skinny_split_setup(args, pass); st != hipSuccess) return st;

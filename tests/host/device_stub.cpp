@@ -39,7 +39,7 @@ uintptr_t allocate(size_t bytes) {
 }
 
 struct Record {
-  int kind, rows_or_tile, splits, columns_per_group, padded, m, n, k;
+  int kind, rows_or_tile, splits, columns_per_group, padded, m, n, k, strips;
 };
 Record g_last{};
 enum Kind { kMain = 0, kSkinny = 1, kWide = 2 };
@@ -89,7 +89,7 @@ Range weight_of(const Args& a) {
 }
 
 Record record_of(int kind, int rows_or_tile, const onebit::SkinnyArgs& a) {
-  return Record{kind, rows_or_tile, a.splits, kind == kWide ? a.tokens_per_group : 0, 0, a.m, a.n, a.k};
+  return Record{kind, rows_or_tile, a.splits, kind == kWide ? a.tokens_per_group : 0, 0, a.m, a.n, a.k, a.strips};
 }
 
 }  // namespace
@@ -156,6 +156,11 @@ void stub_last_launch(int* out) {
   out[2] = g_last.splits > 1 ? g_last.splits : 1;
   out[3] = g_last.padded;
   out[4] = g_last.columns_per_group;
+}
+// whether the last launch's grid is walked in strips of column groups
+int stub_last_strips() {
+  std::lock_guard<std::mutex> lock(g_mu);
+  return g_last.strips;
 }
 size_t stub_allocated_bytes() {
   std::lock_guard<std::mutex> lock(g_mu);

@@ -227,3 +227,15 @@ def test_description_is_what_is_launched(fresh):
             hook(-1)
     assert len(seen) >= 11, seen
     assert fresh.stub_violations() == 0, fresh.stub_violation().decode()
+
+
+@pytest.mark.parametrize("call,m,n,k,strips", [
+    (layer, 1024, 488, 4096, 0), (layer, 1024, 489, 4096, 1),    # sixteen row groups: from 4 MB of x on
+    (layer, 1984, 123, 2784, 1), (layer, 1984, 66, 1792, 0),     # 31 row groups: from 1.5 MB of x and weight on
+    (product, 1984, 184, 5536, 1), (product, 704, 48, 2976, 0), (product, 2688, 296, 2848, 0),
+    (product, 4096, 256, 4096, 0), (product, 2048, 256, 8192, 1), (product, 1024, 64, 4096, 0),
+    (layer, 4096, 64, 11008, 0), (layer, 28672, 48, 8192, 0),    # up to 64 tokens, one column group
+])
+def test_where_the_grid_is_walked_in_strips(fresh, call, m, n, k, strips):
+    assert call(fresh, m, n, k) == 0
+    assert last_launch(fresh)["kernel"] == "wide_kernel" and fresh.stub_last_strips() == strips
