@@ -55,6 +55,8 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
   // operand is used as it is stored (us: 28672 x 8192 with 32 tokens 16.7 -> 16.1, 8192 x 8192 with 128 15.9 -> 15.2, 16384 x 16384
   // with 64 27.7 -> 26.9; where every compute unit is busy and power sets the clock about 1 % the other way).
   constexpr bool S32 = CT % 2 == 0;
+  // a chunk of few column tiles is over before the next one's operand can come from HBM: it is requested a chunk earlier
+  constexpr bool FAR = CT == 1 || (CT == 3 && R <= 2);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rb_total = p.m / kRowBlock, rb_first = block_x * R;
@@ -280,6 +282,10 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
   // Requests return in order, and a wait names how many younger ones may be outstanding. Per chunk a wavefront requests its
   // image 2, the prepared operand of its next chunk, image 3 and the first two images of the next chunk; before the loop the
   // operand of the first chunk and its first two images. Nothing is requested past the last chunk (wave-uniform branches).
+  // FAR: the operand of the chunk after the next one at the end of a chunk, behind image 1 of the next, and before the loop that of the
+  // second chunk, last. us, weights from HBM, otherwise -> this: 4096 x 11008 with 24 / 40 / 64 tokens 8.7 / 10.5 / 10.7 -> 8.5 / 10.3 /
+  // 10.5 (as it was before the operand was requested inside the chunk), 7360 x 10880 with 77 16.4 -> 15.7, 11264 x 40 x 3072 8.1 -> 7.6;
+  // four row blocks with three tiles, whose chunks take longer, and whole 32-column tiles are no faster for it.
   // A compute unit takes 64 bytes of requests per clock, so what stands in front of the first SMFMAC is what all wavefronts
   // request before it: the second chunk's operand, requested up front too, held that up by 48 KB (28672 x 8192 with 48 tokens:
   // the first SMFMAC of a workgroup 6000 to 8000 clocks after its start). And the older four wavefronts are served first all the
@@ -297,6 +303,7 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
       __builtin_amdgcn_sched_barrier(0);
     }
     copy_image(first * kChunkK + kWideImageK, 1);
+    if (FAR && first + NW < kc_end) load_a(first + NW, next);
     __builtin_amdgcn_sched_barrier(0);
     if (wave >= NW / 2) __builtin_amdgcn_s_setprio(1);
     if constexpr (!S32) gather(raw);
@@ -307,12 +314,12 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
       auto stage = [&](auto s_tag) __attribute__((always_inline)) {
         constexpr int S = decltype(s_tag)::value;
         // all but the requests younger than image S
-        if (more) wait_vmcnt<(S == 1 || S == 2 ? COPIES + 2 * R : COPIES)>();
+        if (more) wait_vmcnt<((FAR ? S < 2 : S == 1 || S == 2) ? COPIES + 2 * R : COPIES)>();
         else wait_vmcnt<(S < 3 ? COPIES : 0)>();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         read_image(S & 1);
-        if constexpr (S == 3) {
+        if constexpr (S == (FAR ? 2 : 3)) {
           // the wait the compiler puts in front of the operand's first use counts its own loads only and so also waits for
           // every copy issued by then: here that is one image, which has had a stage's time
 #pragma unroll
@@ -326,7 +333,7 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
           __builtin_amdgcn_sched_barrier(0);
         }
         compute(s_tag);
-        if constexpr (S == 0) {
+        if constexpr (S == 0 && !FAR) {
           if (more) load_a(kc + NW, next);
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -340,6 +347,10 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
         for (int r = 0; r < R; ++r) raw[r] = next[r];
       } else {
         gather(next);
+        if constexpr (FAR) {
+          if (kc + 2 * NW < kc_end) load_a(kc + 2 * NW, next);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
       kc += NW;
     } while (kc < kc_end);
