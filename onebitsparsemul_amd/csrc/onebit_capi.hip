@@ -287,26 +287,24 @@ struct SkinnyPlan {
 // Weight rows per workgroup of the split-K kernel up to sixteen columns, from the workgroups that 32 and 64 rows give: the smallest
 // whose workgroups have a compute unit each. A workgroup more than that waits for a second round (us, 32 | 64 | 128 rows, both forms
 // alike: 9216 x 4096 with one token 6.0 | 4.6 | 6.6, with sixteen 7.3 | 5.4 | 7.2, with three columns 8.3 | 6.3 | 8.3; 17408 x
-// 4096 9.4 | 8.5 | 7.0, 11.2 | 10.2 | 7.6, 12.4 | 11.8 | 8.8; 18432 x 8192 with sixteen 15.9 | 14.6 | 11.5), and a larger group
+// 4096 9.4 | 8.5 | 7.0, 11.2 | 10.2 | 7.6, 12.4 | 11.8 | 8.8; 18432 x 8192 with sixteen 15.9 | 14.6 | 11.5; on short K 64 | 128
+// rows: 18688 x 1280 with one / four columns, three / sixteen tokens 6.6 | 5.4, 5.3 | 5.3, 6.5 | 5.3, 7.7 | 6.1, x 512 5.4 | 4.2, 4.5 |
+// 4.3, 5.4 | 4.2, 6.6 | 5.1), and a larger group
 // leaves compute units idle (8192 x 4096 with one token 3.9 | 4.6 | 6.6, 16384 x 4096 7.3 | 5.4 | 7.0).
 int single_round_rows(long groups_of_32, long groups_of_64, int compute_units) {
   return groups_of_32 <= compute_units ? 32 : groups_of_64 <= compute_units ? 64 : 128;
 }
 
-SkinnyPlan plan_skinny(int m, int n, int k, bool pieces, int compute_units) {
+SkinnyPlan plan_skinny(int m, int n, int k, int compute_units) {
   const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
   const int forced_rows = g_skinny_rows, forced_splits = g_split_k;
-  // up to sixteen columns: single_round_rows. (pieces: B in pieces at any alignment. The other modes keep 64-row groups on K of up
-  // to five chunks, a route that is pinned by a test; 128 rows are the faster ones there too, 17408 x 1024 with one token 4.3
-  // against 5.3 us)
+  // up to sixteen columns: single_round_rows
   // beyond: the largest row group that still gives about two workgroups per three compute units (measured: larger groups
   // re-read B less often, but idle compute units cost more)
   // (n > 32: two column fragments per row block, at most two row blocks per wavefront)
   const int enough = std::max(1, 160 * compute_units / 256);
   const int rows = forced_rows > 0 ? forced_rows
-                   : n <= 16       ? (m / 128 < enough && !pieces && chunks <= 5
-                                          ? std::min(64, single_round_rows((m + 31) / 32, (m + 63) / 64, compute_units))
-                                          : single_round_rows((m + 31) / 32, (m + 63) / 64, compute_units))
+                   : n <= 16       ? single_round_rows((m + 31) / 32, (m + 63) / 64, compute_units)
                    : (m / 128 >= enough && n <= 32) ? 128 : (m / 64 >= enough) ? 64 : 32;
   if (forced_splits >= 1) return SkinnyPlan{rows, forced_splits > chunks ? chunks : forced_splits};
   const double image_row_bytes = n <= 16 ? 32.0 : n <= 32 ? 64.0 : 128.0;
@@ -409,15 +407,14 @@ bool wide_in_strips(int m, int n, int k, const WidePlan& plan, bool plain, int c
   return x >= 4e6 || (row_groups % 2 ? both >= 1.5e6 : row_groups % 4 ? both >= 3.5e6 : false);
 }
 
-LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int compute_units, bool tokens = false) {
+LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int compute_units) {
   LaunchPlan plan{};
   // 32 < n <= 64: every 64-row workgroup of the split-K kernel stages all of B, which the main kernel's tiles overtake
   // from about 48k rows on (n = 64: 28672 x 8192 32 us against 42; 32768 x 4096 20 against 26; 49152 x 4096 32.5
   // against 34.4; 65536 x 8192 66 against 68, at n = 40 77 against 66; 131072 x 2048 51 against 35)
   const bool skinny_shape = n <= 32 || (n <= onebit::kSkinnyMaxN && m <= 40960);
   if (skinny_shape && g_skinny_enabled) {
-    const bool pieces = !tokens && n <= 16 && !(b_16_byte_aligned && (n == 1 || n == 2 || n == 4 || n == 16));
-    const SkinnyPlan sk = plan_skinny(m, n, k, pieces, compute_units);
+    const SkinnyPlan sk = plan_skinny(m, n, k, compute_units);
     plan.split_k_kernel = 1;
     plan.rows_or_tile = sk.rows;
     plan.splits = sk.splits;
@@ -489,7 +486,7 @@ struct LinearPlan {
 };
 LinearPlan plan_linear(int m, int tokens, int k, int compute_units) {
   LinearPlan plan{};
-  plan.launch = choose_launch(m, tokens, k, true, compute_units, true);
+  plan.launch = choose_launch(m, tokens, k, true, compute_units);
   if (tokens <= onebit::kSkinnyTokens || !g_skinny_enabled) return plan;
   const long groups[3] = {(m + 31) / 32, (m + 63) / 64, (m + 127) / 128};
   if (!plan.launch.split_k_kernel && g_tile_config >= 0) return plan;
@@ -1001,7 +998,7 @@ int onebit_sparse_linear_prepared_grouped_typed(const onebit_linear_problem* pro
     }
     return ONEBIT_OK;
   }
-  // Row group of the launch: as for one product with all the weight rows.
+  // Row group of the launch: as for one product with all the weight rows that does not split K.
   const int compute_units = current_compute_units();
   for (int first = 0; first < count; first += onebit::kSkinnyMaxGroup) {
     const int in_launch = std::min(count - first, onebit::kSkinnyMaxGroup);

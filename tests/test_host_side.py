@@ -171,9 +171,11 @@ def test_kernel_of_32_columns(fresh, m, k, kernel):
 
 
 @pytest.mark.parametrize("call,m,n,rows", [(product, 18688, 3, 128), (product, 16448, 12, 128), (product, 16384, 3, 64),
-                                           (product, 18688, 4, 64), (product, 18688, 1, 64), (layer, 18688, 3, 64)])
+                                           (product, 18688, 4, 128), (product, 18688, 1, 128), (layer, 18688, 3, 128)])
 def test_pieces_at_any_alignment_in_one_round(fresh, call, m, n, rows):
-    """64-row groups of that mode beyond one per compute unit took up to 22 % longer than the element copies before them."""
+    """64-row groups of that mode beyond one per compute unit took up to 22 % longer than the element copies before them. The other
+    modes' are no slower in one round either (18688 x 1280, 64- | 128-row groups: four columns 5.3 | 5.3 us, one 6.6 | 5.4, a layer of
+    three tokens 6.5 | 5.3)."""
     assert call(fresh, m, n, 1280) == 0
     assert last_launch(fresh)["rows_or_tile"] == rows
 
