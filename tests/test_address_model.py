@@ -3,8 +3,9 @@
 The kernels' addresses depend on shapes, launch plan and pointers only, never on operand contents, so their index
 arithmetic can be restated on the CPU (numpy, one array element per lane) and every access asserted to lie inside its
 operand: the prepared weight, B (or its padded copy), C / D, the K-split partial sums. The model restates the index
-arithmetic of onebitsparsemul_amd/csrc/: prepare_kernel and pack_kernel, skinny_kernel with its four B staging modes, wide_kernel
-in both forms, gemm_kernel's asynchronous copy pattern and epilogue ranges, splitk_reduce_kernel, pad_b_kernel. Where a load
+arithmetic of onebitsparsemul_amd/csrc/: prepare_kernel and pack_kernel, skinny_kernel with its five B staging modes, wide_kernel
+in both forms (its walk over the grid, the requests a wait names, both SMFMACs' reads of an image), gemm_kernel's asynchronous copy
+pattern, epilogue ranges and the turns of both epilogues through LDS, splitk_reduce_kernel, pad_b_kernel. Where a load
 deliberately reaches past a row (pieces at any alignment, padded copy) the elements that arrive are tracked too. The route of a call
 comes from the library itself (onebit_sparse_describe_call, host-only). It covers the benchmark configurations and the long-K shapes
 with 33 to 64 columns (8192 x 28672 with n = 40, 48, 64). No GPU is touched.
@@ -151,14 +152,14 @@ def check_pack(m, k, size):
 
 
 # ---------------------------------------------------------------------------------------------------------------
-def skinny_variant(n, rows, b_aligned=True, tokens=False):
+def skinny_variant(n, rows, b_aligned=True, tokens=False, x32=False):
     nw, r = {32: (16, 1), 64: (8, 2), 128: (8, 4)}[rows]
     nc = 64 if n > 32 else 32 if n > 16 else 16
     if nc == 64:
         r = min(r, 2)
     if tokens:
         assert n <= 16
-        mode = "tokens"
+        mode = "tokens32" if x32 else "tokens"
     elif n == nc and b_aligned:
         mode = "full"
     elif n == 1 and b_aligned:
@@ -206,12 +207,51 @@ def check_any_image(n, k, nc, k_base):
     assert np.array_equal(image[:, :n], np.where(k_base + row < k, (k_base + row) * n + col, -1))
 
 
-def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1):
-    nw, R, nc, mode = skinny_variant(n, rows, b_aligned, tokens)
+def token_image_16(n, k, k_base):
+    """The token-major image of 16-bit activations: byte offset of each eight values -> (token, first K), from the stores of the
+    pieces."""
+    image = {}
+    for i in range(8):
+        for lane in range(64):
+            piece, token = lane % 32, lane // 32 + 2 * i
+            swizzle = (lane // 32) & 15
+            at = ((lane // 32) * 512 + ((piece ^ swizzle) << 4) ^ (((2 * i) & 15) << 4)) + i * 1024
+            assert at not in image
+            image[at] = (token, k_base + 8 * piece)
+    return image
+
+
+def check_tokens32_image(n, k, k_base):
+    """One image of fp32 activations: every load inside x and what it brings where the 16-bit form has it (a token's K in pieces of
+    eight, a piece as two halves)."""
+    size, image = n * k * 4, token_image_16(n, k, k_base)
+    whole, seen = k_base + CHUNK_K <= k, set()
+    for first in (0, 8) if n > 8 else (0,):
+        for i in range(8):
+            token = first + i
+            if token < n:
+                offset = LANE * 16 + token * k * 4
+                if whole:
+                    lane_off, scalar_off = offset, k_base * 4
+                else:
+                    lane_off, scalar_off = np.where(k_base + 4 * LANE < k, offset + k_base * 4, 0xFFFFFF00), 0
+                accessed = lane_off + 16 <= size  # the descriptor's range check looks at the lane offset alone
+                assert lane_off.max() < (1 << 32) and np.array_equal(accessed, lane_off != 0xFFFFFF00)
+                inside(lane_off[accessed] + scalar_off, 16, size, "split-K kernel: fp32 x rows")
+                assert np.array_equal((lane_off + scalar_off)[accessed] // 4, (token * k + k_base + 4 * LANE)[accessed])
+            at = token * 512 + (((LANE >> 1) ^ (token & 15)) << 4) + (LANE & 1) * 8
+            for lane in range(64):
+                assert image[at[lane] // 16 * 16] == (token, k_base + 8 * (lane >> 1)) and at[lane] not in seen
+                seen.add(at[lane])
+    assert len(seen) == (1024 if n > 8 else 512) and max(seen) + 8 <= 8192
+
+
+def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1, x32=False):
+    nw, R, nc, mode = skinny_variant(n, rows, b_aligned, tokens, x32)
     kc_total, rb_total = (k + 255) // 256, m // 32
     img_rows = 8192 // (nc * 2)
     sub = CHUNK_K // img_rows
-    prep_size, b_size = prepared_bytes(m, k), k * n * 2
+    prep_size, b_size = prepared_bytes(m, k), k * n * (4 if x32 else 2)
     grid = (rb_total + R - 1) // R
     prefetch_b = nw <= 8 or mode == "run"
     images = set()
@@ -219,8 +259,8 @@ def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1
     splits = (kc_total + cps - 1) // cps
     assert (splits - 1) * cps < kc_total  # the launcher's check: no empty split
     b_fits = b_size < (1 << 32)
-    if mode == "tokens":
-        assert k * 64 * 2 < 0xFFFFFF00  # the launcher's check
+    if mode in ("tokens", "tokens32"):
+        assert k * 64 * (4 if x32 else 2) < 0xFFFFFF00  # the launcher's check
     if mode == "run":
         assert k * n * 2 < 0xFFFFFF00   # the launcher's check
     for wg, split in [(g, sp) for g in sorted({0, 1, grid // 2, grid - 1} & set(range(grid)))
@@ -269,6 +309,12 @@ def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1
                     kc += nw
             for k_base in k_bases:
                 rows_valid = min(max(k - k_base, 0), img_rows)
+                if mode == "tokens32":
+                    if k_base not in images:
+                        images.add(k_base)
+                        if len(images) <= 4 or k - k_base < 2 * CHUNK_K:
+                            check_tokens32_image(n, k, k_base)
+                    continue
                 if mode == "tokens":
                     # raw buffer loads: the descriptor (n * k * 2 bytes) checks the lane offset alone and returns zero
                     # without an access when it is out of range; the scalar offset is added afterwards
@@ -328,7 +374,7 @@ def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1
         elem = 4 if splits > 1 else d_size          # a split writes fp32 partial sums to its slice of the workspace
         slice0 = split * m * n * elem if splits > 1 else 0
         total = splits * m * n * elem
-        if mode == "tokens":  # (one column: the same element in both layouts)
+        if mode in ("tokens", "tokens32"):  # (one column: the same element in both layouts)
             inside(slice0 + (cols[None, :] * m + rows_out[:, None]) * elem, elem, total, "split-K kernel: y")
         else:
             inside(slice0 + (rows_out[:, None] * n + cols[None, :]) * elem, elem, total, "split-K kernel: D")
@@ -360,9 +406,75 @@ def wide_copies(tokens_form, copies, tokens, k, ldb, first_column):
     return out
 
 
+def wide_strip_walk(row_groups, groups):
+    """(row group, column group) of every workgroup of a grid that is walked in strips of two column groups, in the kernel's
+    arithmetic: 32-bit reciprocal, eight XCDs"""
+    total = row_groups * groups
+    reciprocal = ((1 << 32) // (2 * row_groups) + 1) & 0xFFFFFFFF
+    x = np.arange(total, dtype=np.int64)
+    per, rem, xcd = total // 8, total % 8, x % 8
+    v = xcd * per + np.minimum(xcd, rem) + x // 8
+    strip = (v * reciprocal) >> 32
+    w = v - strip * 2 * row_groups
+    strip, w = np.where(w < 0, strip - 1, strip), np.where(w < 0, w + 2 * row_groups, w)
+    pair = 2 * (strip + 1) * row_groups <= total
+    return np.where(pair, w >> 1, w), 2 * strip + np.where(pair, w & 1, 0)
+
+
+def check_wide_strips(row_groups, groups):
+    """every (row group, column group) once"""
+    rows, cols = wide_strip_walk(row_groups, groups)
+    assert rows.min() >= 0 and rows.max() < row_groups and cols.min() >= 0 and cols.max() < groups
+    assert len(set(rows * groups + cols)) == row_groups * groups
+
+
+def wide_requests(chunks, copies, R, far):
+    """The requests of a wavefront in order, and at each stage's wait how many of the youngest may be outstanding. Returns the prepared
+    operands and images in the order of their requests; asserts that a wait leaves nothing outstanding that the stage reads and does not
+    wait for anything younger than its image."""
+    issued, operands, images = [], [], []
+
+    def image(chunk, stage):
+        images.append(chunk * 4 + stage)
+        issued.extend([("image", chunk, stage)] * copies)
+
+    def operand(chunk):
+        operands.append(chunk)
+        issued.extend([("operand", chunk, 0)] * (2 * R))  # metadata and signs of each row block
+
+    if not chunks:
+        return [], []
+    operand(chunks[0])
+    image(chunks[0], 0)
+    image(chunks[0], 1)
+    if far and len(chunks) > 1:
+        operand(chunks[1])
+    for at, kc in enumerate(chunks):
+        more = at + 1 < len(chunks)
+        for stage in range(4):
+            if more:
+                allowed = copies + 2 * R if (stage < 2 if far else stage in (1, 2)) else copies
+            else:
+                allowed = copies if stage < 3 else 0
+            done = issued[:len(issued) - allowed]
+            assert done.count(("image", kc, stage)) == copies and done[-1] == ("image", kc, stage), (kc, stage)
+            if more and stage == (2 if far else 3):
+                # the next operand's first use: it has arrived, and the compiler's wait for it covers one image more
+                assert done.count(("operand", chunks[at + 1], 0)) == 2 * R and allowed == copies
+            if stage < 2:
+                image(kc, stage + 2)
+            elif more:
+                image(chunks[at + 1], stage - 2)
+            if stage == 0 and more and not far:
+                operand(chunks[at + 1])
+        if far and at + 2 < len(chunks):
+            operand(chunks[at + 2])
+    return operands, images
+
+
 def check_wide(m, n, k, rows, columns, splits, tokens=False, pad_b=False, d_size=2):
-    """wide_kernel, either form: the launcher's checks, the prepared operand, the copies of x or B into the ring of two images
-    (K tail, last column group), the fragment reads of an image, the results"""
+    """wide_kernel, either form: the launcher's checks, the walk over the grid, the prepared operand, the copies of x or B into the ring
+    of two images (K tail, last column group), the fragment reads of an image, the results"""
     R = rows // 32
     ldb = k if tokens else (n + 7) // 8 * 8 if pad_b else n
     copies = (columns + 7) // 8 if tokens else 2 * ((columns + 15) // 16)
@@ -387,8 +499,32 @@ def check_wide(m, n, k, rows, columns, splits, tokens=False, pad_b=False, d_size
             where = i * 64 + lane
             assert where * 16 + 16 <= image_bytes and where not in image
             image[where] = (k_at[lane], col[lane])  # eight K positions of a token, or eight columns of a K position
+    check_wide_strips(grid, col_groups)
     i16, g16 = LANE & 15, LANE >> 4
-    for ct in range(ct_count):
+    # whole 32-column tiles: the 32x32x32 SMFMAC, whose lane (column l % 32, half l / 32) holds K positions 8 half ... + 7 and
+    # 16 + 8 half ... + 7 of each 32-wide step
+    half, col32 = LANE >> 5, LANE & 31
+    for f in range(ct_count // 2 if ct_count % 2 == 0 else 0):
+        for ks in range(2):
+            if tokens:
+                base = col32 * 128 + ((half ^ ((col32 >> 1) & 7)) << 4)
+                for h in range(2):
+                    at = (base ^ ((4 * ks + 2 * h) << 4)) + f * 4096
+                    for lane in range(64):
+                        assert at[lane] % 16 == 0 and at[lane] + 16 <= image_bytes
+                        if 32 * f + col32[lane] < 8 * copies:
+                            assert image[at[lane] // 16] == (32 * ks + 16 * h + 8 * half[lane], 32 * f + col32[lane])
+            else:
+                row0 = 8 * half + (i16 >> 2)
+                c8 = (col32 >> 4) * 4 + (i16 & 3)
+                tile = row0 * pieces * 16 + (((4 * f + (c8 >> 1)) ^ row_swizzle(row0, pieces)) << 4) + (c8 & 1) * 8
+                for q in range(4):
+                    step = 32 * ks + 4 * (q & 1) + 16 * (q >> 1)
+                    at = tile + step * pieces * 16
+                    for lane in range(64):  # four columns of a K position per lane of the transpose read
+                        assert at[lane] + 8 <= image_bytes and at[lane] % 16 == 8 * (c8[lane] & 1)
+                        assert image[at[lane] // 16] == (row0[lane] + step, 32 * f + 8 * (c8[lane] >> 1))
+    for ct in range(ct_count if ct_count % 2 else 0):
         if tokens:
             base = i16 * 128 + (((4 * (g16 >> 1) + (g16 & 1)) ^ ((i16 >> 1) & 7)) << 4)
             for h in range(2):
@@ -420,21 +556,11 @@ def check_wide(m, n, k, rows, columns, splits, tokens=False, pad_b=False, d_size
             kc_begin = split * cps
             kc_end = min(kc_begin + cps, kc_total)
             for wave in range(WIDE_WAVES):
-                chunks, images, kc = [kc_begin + wave], [], kc_begin + wave
-                if kc < kc_end:
-                    images += [kc * 4, kc * 4 + 1]
-                    if kc + WIDE_WAVES < kc_end:
-                        chunks.append(kc + WIDE_WAVES)
-                while kc < kc_end:
-                    images += [kc * 4 + 2, kc * 4 + 3]
-                    if kc + WIDE_WAVES < kc_end:
-                        images += [(kc + WIDE_WAVES) * 4, (kc + WIDE_WAVES) * 4 + 1]
-                    if kc + 2 * WIDE_WAVES < kc_end:
-                        chunks.append(kc + 2 * WIDE_WAVES)
-                    kc += WIDE_WAVES
-                mine = range(kc_begin + wave, kc_end, WIDE_WAVES)
+                mine = list(range(kc_begin + wave, kc_end, WIDE_WAVES))
+                chunks, images = wide_requests(mine, copies, R, far=ct_count == 1 or (ct_count == 3 and R <= 2))
                 assert images == [c * 4 + s for c in mine for s in range(4)]  # every image of its chunks once, in order
-                assert len(mine) == 0 or chunks == list(mine)
+                assert chunks == mine
+                chunks = chunks or [kc_begin + wave]  # requested, clamped, by a wavefront without a chunk
                 for kc in chunks:
                     for wg in sorted({0, grid // 2, grid - 1}):
                         for r in range(R):
@@ -616,6 +742,9 @@ def check_gemm(m, n, k, tile, splits, pad_b, tokens=False, b_aligned=True, d_siz
             total = (splits if splits > 1 else 1) * m * n * elem
             if tokens:
                 inside(slice0 + (cols_out[None, :] * m + rows_out[:, None]) * elem, elem, total, "main kernel: y")
+                rows_tile = tile_m * BM + 4 * np.arange(BM // 4)  # the bias: four values, of row 0 past the end
+                for size in (2, 4):
+                    inside(np.where(rows_tile < m, rows_tile, 0) * size, 4 * size, m * size, "main kernel: bias")
             else:
                 inside(slice0 + (rows_out[:, None] * n + cols_out[None, :]) * elem, elem, total, "main kernel: D")
     if splits > 1:
@@ -628,6 +757,8 @@ def check_call(m, n, k, tokens=False, b_aligned=True):
     plan = _native.describe_launch(m, n, k, b_aligned=b_aligned or tokens, tokens=tokens)
     if plan["kernel"] == "skinny_kernel":
         check_skinny(m, n, k, plan["rows"], tokens=tokens, b_aligned=b_aligned, splits=plan["splits"])
+        if tokens:
+            check_skinny(m, n, k, plan["rows"], tokens=True, splits=plan["splits"], x32=True)
     elif plan["kernel"] == "wide_kernel":
         check_wide(m, n, k, plan["rows"], plan["columns"], plan["splits"], tokens=tokens, pad_b=plan["pad_b"])
     else:
@@ -869,6 +1000,107 @@ def test_epilogue_scratch_swizzle_avoids_bank_conflicts():
             sw = ((r & 1) << 2) ^ (((r >> 2) & 1) * 32)
             banks += [(r * wcols + (c8 ^ sw) + j) % 64 for j in range(4)]
         assert len(set(banks)) == 64
+
+
+# ---- the turns of the token-major epilogue through the LDS scratch ------------------------------------------------
+TOKEN_TILES = (4, 6, 9, 10, 11, 12, 13, 14, 15)
+
+
+@pytest.mark.parametrize("tile", TOKEN_TILES)
+def test_token_epilogue_16_bit_turns(tile):
+    """Every four rows of every token that a wavefront finishes are written once, inside its scratch, and read back as what they are; all
+    of them are stored; sixteen lanes meet in no bank."""
+    _, _, FM, FN, KG = TILES[tile]
+    m16 = tile == 15
+    wcols, split = FN * 32, KG == 2 and FM % 2 == 0
+    frags = FM // 2 if split else FM
+    pieces, turn = 4 * frags, 2 * wcols // frags if frags > 2 else wcols
+    groups = 2 if m16 else 4
+    assert turn * pieces <= wcols * 8 and wcols % turn == 0 and turn % (16 if m16 else 32) == 0
+
+    def slot_at(t, slot):
+        return t * (pieces * 16) + ((((slot >> 1) ^ ((t * pieces >> 4) & (pieces - 1))) << 4) | ((slot & 1) << 3))
+
+    for kg in range(2 if split else 1):
+        stored = set()
+        for first in range(0, wcols, turn):
+            scratch = {}
+            for fm in range(FM):
+                if split and (fm >= FM // 2) != (kg == 1):
+                    continue
+                for q in range(groups):
+                    tiles = range(first // 16, (first + turn) // 16) if m16 else range(first // 32, (first + turn) // 32)
+                    for part in tiles:
+                        at = []
+                        for lane in range(64):
+                            if m16:  # registers of tile (2 fm + q, ct): rows 16 q + 4 (lane / 16) on of token 16 ct + lane % 16
+                                slot, row, t = 4 * q + (lane >> 4), 16 * q + 4 * (lane >> 4), part * 16 - first + (lane & 15)
+                            else:    # registers 4 q ... 4 q + 3: rows 8 q + 4 (lane / 32) on of token 32 fn + lane % 32
+                                slot, row, t = 2 * q + (lane >> 5), 8 * q + 4 * (lane >> 5), part * 32 - first + (lane & 31)
+                            where = slot_at(t, 8 * (fm % frags) + slot)
+                            assert where not in scratch and where + 8 <= wcols * 128
+                            scratch[where] = ((fm % frags) * 32 + row, first + t)
+                            at.append(where)
+                        for sixteen in range(0, 64, 16):
+                            banks = [b % 64 for w in at[sixteen:sixteen + 16] for b in (w // 4, w // 4 + 1)]
+                            assert len(set(banks)) == 32
+            for it in range(turn * pieces // 64):
+                at = []
+                for lane in range(64):
+                    piece, t = lane % pieces, it * (64 // pieces) + lane // pieces
+                    where = slot_at(t, 2 * piece)
+                    assert where % 16 == 0
+                    assert scratch[where] == (8 * piece, first + t) and scratch[where + 8] == (8 * piece + 4, first + t)
+                    stored.add((8 * piece, first + t))
+                    at.append(where)
+                for sixteen in range(0, 64, 16):
+                    assert len({(w // 4 + j) % 64 for w in at[sixteen:sixteen + 16] for j in range(4)}) == 64
+        assert stored == {(8 * piece, t) for piece in range(pieces) for t in range(wcols)}
+
+
+@pytest.mark.parametrize("tile", TOKEN_TILES)
+def test_token_epilogue_fp32_turns(tile):
+    _, _, FM, FN, _ = TILES[tile]
+    wcols, scratch = FN * 32, {}
+    for lane in range(64):
+        if tile == 15:
+            parts = [(ct * 16 + (lane & 15), 4 * rh + (lane >> 4), lane & 15) for rh in range(2) for ct in range(2 * FN)]
+        else:
+            parts = [(fn * 32 + (lane & 31), 2 * q + (lane >> 5), lane & 31) for fn in range(FN) for q in range(4)]
+        for token, slot, low in parts:  # slot s: rows 4 s ... 4 s + 3 of the 32-row block
+            where = token * 128 + ((slot ^ ((low >> 1) & 7)) << 4)
+            assert where not in scratch and where + 16 <= wcols * 128
+            scratch[where] = (4 * slot, token)
+    read = set()
+    for it in range(wcols * 8 // 64):
+        for lane in range(64):
+            j, t = lane % 8, it * 8 + lane // 8
+            assert scratch[t * 128 + ((j ^ ((t >> 1) & 7)) << 4)] == (4 * j, t)
+            read.add((4 * j, t))
+    assert len(read) == 8 * wcols == len(scratch)
+
+
+@pytest.mark.parametrize("row_groups", [1, 2, 3, 7, 8, 11, 15, 31, 32, 53, 131, 1000])
+def test_strips_reach_every_workgroup_once(row_groups):
+    """odd and even numbers of column groups, fewer workgroups than XCDs, numbers that eight does not divide"""
+    for groups in (1, 2, 3, 4, 5, 8, 9, 19, 63):
+        check_wide_strips(row_groups, groups)
+
+
+@pytest.mark.parametrize("chunks", [1, 2, 3, 7])
+@pytest.mark.parametrize("R", [1, 2, 4])
+def test_waits_of_wide_kernel_name_the_requests_behind_an_image(chunks, R):
+    for copies in range(1, 9):
+        for far in (False, True):
+            wide_requests(list(range(0, 8 * chunks, 8)), copies, R, far)
+
+
+@pytest.mark.parametrize("m,k", [(64, 32), (192, 1056), (320, 4640), (1024, 8192), (128, 16416)])
+def test_fp32_activations_addresses(m, k):
+    for n in (1, 7, 8, 9, 16):
+        for rows in (32, 64, 128):
+            for splits in (1, 3):
+                check_skinny(m, n, k, rows, tokens=True, splits=min(splits, (k + 255) // 256), x32=True, d_size=4)
 
 
 # ---------------------------------------------------------------------------------------------------------------
