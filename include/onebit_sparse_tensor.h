@@ -153,9 +153,9 @@ int onebit_sparse_linear_prepared_f32(const void *prepared, const void *x, const
                                       int bias_dtype, int y_dtype, void *stream);
 /*
  * 1 where a layer call on fp32 activations of this size is taken by onebit_sparse_linear_prepared_f32, as the calling thread's hooks
- * stand, and faster there than converting them first on the current device; else 0.
+ * stand, and faster there than converting them first on the current device (captured into a graph or not, as `stream` is now); else 0.
  */
-int onebit_sparse_linear_reads_f32(int tokens, int m, int k);
+int onebit_sparse_linear_reads_f32(int tokens, int m, int k, void *stream);
 int onebit_sparse_linear_prepared_grouped_typed(const onebit_linear_problem *problems, int count, int tokens, int x_dtype,
                                                 int bias_dtype, int y_dtype, void *stream);
 

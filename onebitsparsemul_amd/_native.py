@@ -56,7 +56,7 @@ def lib():
         L.onebit_sparse_pack.restype = i32
         L.onebit_sparse_pack.argtypes = [vp, i32, i32, i32, vp, vp, i32, vp]
         L.onebit_sparse_linear_reads_f32.restype = i32
-        L.onebit_sparse_linear_reads_f32.argtypes = [i32, i32, i32]
+        L.onebit_sparse_linear_reads_f32.argtypes = [i32, i32, i32, vp]
         L.onebit_sparse_linear_prepared_f32.restype = i32
         L.onebit_sparse_linear_prepared_f32.argtypes = [vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]
         L.onebit_sparse_linear_prepared_typed.restype = i32

@@ -724,18 +724,27 @@ bool takes_f32(int tokens) { return tokens <= onebit::kSkinnyTokens && g_skinny_
 // Whether skinny_kernel on fp32 activations is faster than converting them and running it on fp16 ones. Every workgroup reads all of
 // x of its K range, so fp32 costs a compute unit half of these bytes more, and beyond eight tokens an image comes in two batches, the
 // second requested behind the first (as long as sixteen more tokens would take); both hide behind the weights until they are many.
-// The conversion costs about 2 us whatever the size. us inside HIP graphs, weights from HBM, converted | read as fp32: 4096 x 8192
-// with 16 tokens 9.3 | 9.1, x 11008 with 9 / 12 / 16 9.5 | 9.3, 10.1 | 10.1, 10.9 | 11.6; 8192 x 14336 with 8 / 9 11.9 | 11.4, 12.0 |
-// 12.6; 7168 x 20480 with 8 / 16 14.3 | 14.8, 18.3 | 21.4; 11008 x 28672 with 5 / 16 24.6 | 22.9, 28.8 | 35.6; two rounds of
-// workgroups: 49152 x 2048 with 16 16.2 | 15.3, x 4096 19.9 | 21.2. Of 384 calls of up to sixteen tokens one is more than 2.5 %
-// slower than the better of the two (12288 x 20480 with 8, 20.8 | 20.1).
-bool reading_f32_is_faster(int tokens, int m, int k, int compute_units) {
+// The conversion costs about 2 us whatever the size, and the host 4 us, which a call outside a graph hides behind its kernel only if
+// that takes 9 us. us inside HIP graphs, weights from HBM, converted | read as fp32: 4096 x 8192 with 16 tokens 9.3 | 9.1, x 11008 with
+// 9 / 12 / 16 9.5 | 9.3, 10.1 | 10.1, 10.9 | 11.6; 8192 x 14336 with 8 / 9 11.9 | 11.4, 12.0 | 12.6; 7168 x 20480 with 8 / 16 14.3 | 14.8,
+// 18.3 | 21.4; 11008 x 28672 with 5 / 16 24.6 | 22.9, 28.8 | 35.6; two rounds of workgroups: 49152 x 2048 with 16 16.2 | 15.3, x 4096
+// 19.9 | 21.2. Of 384 calls of up to sixteen tokens one is more than 2.5 % slower than the better of the two (12288 x 20480 with 8,
+// 20.8 | 20.1). Call after call without a graph: 4096 x 9600 with 16 8.9 | 8.2, x 11008 with 13 / 16 9.1 | 7.8, 9.1 | 8.8, 5120 x 13824
+// with 12 9.5 | 9.2, 8192 x 14336 with 9 9.8 | 9.8, 11008 x 28672 with 16 21.5 | 27.8.
+bool reading_f32_is_faster(int tokens, int m, int k, int compute_units, hipStream_t stream) {
+  // read whatever the plan: no row group is smaller than 32, a split reads less (spares a small call the second plan)
+  const long most_rounds = (m / 32 + compute_units - 1) / compute_units;
+  if ((double)k * most_rounds * (tokens + 16) < 150e3) return true;
   const LaunchPlan plan = plan_linear(m, tokens, k, compute_units).launch;
   const int splits = full_splits((k + onebit::kChunkK - 1) / onebit::kChunkK, plan.splits);
   const long workgroups = (long)((m + plan.rows_or_tile - 1) / plan.rows_or_tile) * splits;
   const long rounds = (workgroups + compute_units - 1) / compute_units;
   const double values = (double)k / splits * rounds;  // of a token that a compute unit reads
-  return tokens <= 8 ? values * tokens < 150e3 : values * (tokens + 16) < (rounds > 1 ? 150e3 : 307e3);
+  if (tokens <= 8) return values * tokens < 150e3;
+  const double work = values * (tokens + 16);
+  if (rounds > 1 || work < 307e3 || work >= 390e3) return work < (rounds > 1 ? 150e3 : 307e3);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
 }
 
 // The layer's product on 16-bit activations of either type, or up to sixteen tokens of fp32 ones (x_dtype).
@@ -962,9 +971,10 @@ int onebit_sparse_linear_prepared_f32(const void* prepared, const void* x, const
   return linear_prepared_impl(prepared, x, bias, y, tokens, m, k, ONEBIT_DTYPE_F32, bias_dtype, y_dtype, static_cast<hipStream_t>(stream));
 }
 
-int onebit_sparse_linear_reads_f32(int tokens, int m, int k) {
+int onebit_sparse_linear_reads_f32(int tokens, int m, int k, void* stream) {
   g_last_error.clear();
-  return check_shape(m, tokens, k) == ONEBIT_OK && takes_f32(tokens) && reading_f32_is_faster(tokens, m, k, current_compute_units());
+  return check_shape(m, tokens, k) == ONEBIT_OK && takes_f32(tokens) &&
+         reading_f32_is_faster(tokens, m, k, current_compute_units(), static_cast<hipStream_t>(stream));
 }
 
 int onebit_sparse_linear_prepared_grouped(const onebit_linear_problem* problems, int count, int tokens, int bias_dtype,

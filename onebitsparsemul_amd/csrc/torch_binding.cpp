@@ -148,7 +148,7 @@ OptionalTensor layer_forward(const torch::Tensor& prepared, const torch::Tensor&
   // fp32 activations of a few tokens are rounded by the kernel that reads them, all others by a conversion in front of it
   const bool read_f32 = x.scalar_type() == torch::kFloat32 && x.is_contiguous() && values_in_memory(x) &&
                         reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
-                        onebit_sparse_linear_reads_f32((int)tokens, (int)m, (int)k);
+                        onebit_sparse_linear_reads_f32((int)tokens, (int)m, (int)k, current_stream(device));
   const torch::Tensor in = read_f32 ? x : kernel_input(x, types.in);
   OptionalTensor b;
   if (bias.has_value()) b = kernel_bias(*bias, device, m);

@@ -20,7 +20,8 @@ def _layer(m, k):
 
 
 def test_few_tokens_through_the_kernel_that_is_on():
-    reads = _native.lib().onebit_sparse_linear_reads_f32
+    def reads(*size):
+        return _native.lib().onebit_sparse_linear_reads_f32(*size, None)
     assert reads(1, 4096, 4096) == 1 and reads(16, 4096, 4096) == 1 and reads(17, 4096, 4096) == 0
     assert reads(0, 4096, 4096) == 0 and reads(4, 100, 4096) == 0
     _native.set_skinny_enabled(False)
@@ -28,25 +29,47 @@ def test_few_tokens_through_the_kernel_that_is_on():
 
 
 @pytest.mark.parametrize("tokens,m,k,faster", [
-    (16, 4096, 9568, 1), (16, 4096, 9600, 0), (9, 4096, 12256, 1), (9, 4096, 12288, 0),  # one round of workgroups
+    (16, 4096, 9568, 1), (16, 4096, 12192, 0), (9, 8192, 12256, 1), (9, 8192, 15616, 0),  # one round of workgroups
     (8, 4096, 28672, 1), (16, 4096, 28672, 1), (16, 8192, 28672, 0), (16, 11008, 28672, 0),  # K in four, in two, not split
     (8, 7168, 18720, 1), (8, 7168, 18752, 0), (5, 11008, 28672, 1),                      # up to eight tokens
     (16, 32768, 4096, 1), (16, 32768 + 64, 4096, 0), (16, 49152, 2048, 1), (8, 49152, 8192, 1), (8, 131072, 8192, 0),  # more rounds
 ])
 def test_where_reading_fp32_is_faster(tokens, m, k, faster):
-    assert _native.lib().onebit_sparse_linear_reads_f32(tokens, m, k) == faster
+    assert _native.lib().onebit_sparse_linear_reads_f32(tokens, m, k, None) == faster
 
 
 @pytest.mark.gpu
 def test_the_layer_converts_where_that_is_faster():
-    m, k = 11008, 28672
+    for m, k, allocations in ((11008, 28672, 2), (4096, 11008, 1)):  # the converted copy and the result, or the result
+        layer, x = _layer(m, k), torch.randn(16, k, device="cuda")
+        layer(x)
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        y = layer(x)
+        assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == allocations
+        want = torch.empty_like(y)
+        _native.linear_prepared(layer._prepared.buffer, x.half(), want, m, k)
+        assert torch.equal(y, want)
+
+
+@pytest.mark.gpu
+def test_captured_where_the_host_decides_outside_a_graph():
+    """converted in a graph, read as fp32 outside of one: the same results on every replay"""
+    m, k = 4096, 11008
     layer, x = _layer(m, k), torch.randn(16, k, device="cuda")
-    layer(x)
-    before = torch.cuda.memory_stats()["allocation.all.allocated"]
-    y = layer(x)
-    assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == 2  # the converted copy and the result
-    want = torch.empty_like(y)
-    _native.linear_prepared(layer._prepared.buffer, x.half(), want, m, k)
+    want = layer(x)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        layer(x)
+    torch.cuda.current_stream().wait_stream(stream)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        y = layer(x)
+    for _ in range(4):
+        x.neg_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, layer(x))
     assert torch.equal(y, want)
 
 

@@ -241,3 +241,12 @@ def test_description_is_what_is_launched(fresh):
 def test_where_the_grid_is_walked_in_strips(fresh, call, m, n, k, strips):
     assert call(fresh, m, n, k) == 0
     assert last_launch(fresh)["kernel"] == "wide_kernel" and fresh.stub_last_strips() == strips
+
+
+@pytest.mark.parametrize("tokens,m,k,outside,captured", [(16, 4096, 9568, 1, 1), (16, 4096, 9600, 1, 0), (13, 4096, 11008, 1, 0),
+                                                         (16, 4096, 12192, 0, 0), (9, 8192, 15584, 1, 0), (9, 8192, 15616, 0, 0)])
+def test_fp32_activations_in_and_outside_a_graph(fresh, tokens, m, k, outside, captured):
+    """where the kernel's time does not cover the host's for a conversion in front of it, a captured call converts and another does not"""
+    assert fresh.onebit_sparse_linear_reads_f32(tokens, m, k, None) == outside
+    fresh.stub_set(0, 1)
+    assert fresh.onebit_sparse_linear_reads_f32(tokens, m, k, None) == captured
