@@ -744,7 +744,9 @@ bool reading_f32_is_faster(int tokens, int m, int k, int compute_units, hipStrea
   const double work = values * (tokens + 16);
   if (rounds > 1 || work < 307e3 || work >= 390e3) return work < (rounds > 1 ? 150e3 : 307e3);
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) == hipSuccess) return capture == hipStreamCaptureStatusNone;
+  (void)hipGetLastError();  // the default stream, another one being captured: the launch is not to report this
+  return false;
 }
 
 // The layer's product on 16-bit activations of either type, or up to sixteen tokens of fp32 ones (x_dtype).

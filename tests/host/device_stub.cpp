@@ -14,6 +14,7 @@
 #include <mutex>
 #include <string>
 #include <thread>
+#include <utility>
 
 namespace {
 
@@ -25,6 +26,9 @@ uintptr_t g_next = kFirstAddress;
 std::string g_violation;               // the first one
 int g_violations = 0, g_capturing = 0, g_launch_us = 0;
 size_t g_allocated_total = 0;
+thread_local hipError_t t_last_error = hipSuccess;  // of the thread's calls, until it is asked for, as in the HIP runtime
+
+hipError_t last_error() { return std::exchange(t_last_error, hipSuccess); }
 
 void violation(const char* what) {
   if (g_violations++ == 0) g_violation = what;
@@ -76,7 +80,7 @@ hipError_t launch(const Record& record, std::initializer_list<Range> ranges) {
   std::lock_guard<std::mutex> lock(g_mu);
   for (const Range& r : ranges)
     if (r.owned() && --g_in_use[reinterpret_cast<uintptr_t>(r.at)] == 0) g_in_use.erase(reinterpret_cast<uintptr_t>(r.at));
-  return hipSuccess;
+  return last_error();  // what the kernels' launchers return
 }
 
 template <class Args>
@@ -137,7 +141,7 @@ int stub_violations() {
   return g_violations;
 }
 const char* stub_violation() { return g_violation.c_str(); }
-void stub_set(int launch_us, int capturing) {
+void stub_set(int launch_us, int capturing) {  // capturing < 0: the question is refused
   std::lock_guard<std::mutex> lock(g_mu);
   g_launch_us = launch_us;
   g_capturing = capturing;
@@ -192,10 +196,12 @@ hipError_t hipDeviceGetAttribute(int* value, hipDeviceAttribute_t, int) {
 }
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* status) {
   std::lock_guard<std::mutex> lock(g_mu);
+  // the default stream while another one is captured
+  if (g_capturing < 0) return t_last_error = hipErrorStreamCaptureImplicit;
   *status = g_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
   return hipSuccess;
 }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() { return last_error(); }
 const char* hipGetErrorString(hipError_t) { return "stub"; }
 hipError_t hipGetSymbolAddress(void** address, const void*) {
   static const uintptr_t scratch = allocate(size_t(64) << 20);

@@ -250,3 +250,10 @@ def test_fp32_activations_in_and_outside_a_graph(fresh, tokens, m, k, outside, c
     assert fresh.onebit_sparse_linear_reads_f32(tokens, m, k, None) == outside
     fresh.stub_set(0, 1)
     assert fresh.onebit_sparse_linear_reads_f32(tokens, m, k, None) == captured
+
+
+def test_a_refused_question_does_not_fail_the_call_after_it(fresh):
+    """On the default stream the HIP runtime refuses to say whether it is captured while another stream is: no error of the layer's."""
+    fresh.stub_set(0, -1)
+    assert fresh.onebit_sparse_linear_reads_f32(13, 4096, 11008, None) == 0
+    assert layer(fresh, 4096, 13, 11008) == 0
