@@ -252,10 +252,11 @@ GemmPlan plan_gemm(int m, int n, int k, int compute_units) {
   if (best.tile == onebit::kTile512x128w8 && best.splits == 1) {
     const long tiles = (long)((m + 511) / 512) * ((n + 127) / 128);
     // From 85 % of a round on; on K from 43 chunks on, where the epilogue of its four wavefronts weighs less, from three quarters on.
-    // us, eight wavefronts | four (layers in fp16 with a bias, layers with fp32 results, products, products with C and fp32 results):
-    // 4096 x 11008 with 3072 125 | 120, 127 | 127, 124 | 120, 136 | 134; 8192 x 16384 with 1600 194 | 185, 195 | 186, 193 | 185, 204 |
-    // 197; bf16 layers 4096 x 11008 with 3072 118 | 114. On K = 8192 what is stored as fp32 or has C is slower (8192 x 8192 with 1408
-    // 94 | 97 and 102 | 104, fp16 layers 92 | 91).
+    // us, eight wavefronts | four (layers in fp16 with a bias, layers with fp32 results, products, products with fp32 C and results),
+    // 192, 200 and 208 tiles: 4096 x 11008 with 3072 127 | 120, 129 | 126, 126 | 121, 138 | 136; 5120 x 11008 with 2560 131 | 123,
+    // 133 | 129, 130 | 124, 142 | 139; 8192 x 16384 with 1600 194 | 183, 195 | 191, 193 | 186, 204 | 199. On shorter K the gain shrinks
+    // with the chunks, for fp32 results first: from 34 chunks on all four forms are still equal or faster (34: 4096 x 8704 with 3072 103 |
+    // 97, 104 | 103, 101 | 97, 115 | 114), at 32 fp32 results are equal (98.4 | 98.4, 109.2 | 109.6); the line is on the safe side.
     if (tiles * 20 >= 17L * compute_units || (chunks >= 43 && tiles * 4 >= 3L * compute_units)) best.tile = onebit::kTile512x128m16;
   }
   return best;
@@ -329,9 +330,10 @@ SkinnyPlan plan_skinny(int m, int n, int k, int compute_units) {
 // sixteen-token column tiles and grows with the share of compute units that load at the same time. Workgroups beyond one per
 // compute unit pay the rounds again, less where two fit a compute unit (up to two column tiles on up to 64 rows). A split
 // pays a second launch and the partial sums.
-// Fitted to m = 1024 ... 28672, k = 1024 ... 22176, 17 ... 1024 tokens inside HIP graphs. us of the chosen plan | of 64-token
-// workgroups on 32 rows, unsplit: 28672 x 8192 x 48 21.0 (128 rows) | 36.0; 4096 x 11008 x 32 9.0 (32 rows, 16 tokens) | 12.2;
-// 1024 x 4096 x 256 5.3 (32 rows, 32 tokens) | 7.1; 4096 x 4096 x 128 6.3 (64 rows, 32 tokens) | 7.8.
+// Fitted to m = 1024 ... 28672, k = 1024 ... 22176, 17 ... 1024 tokens inside HIP graphs, when the kernel was slower than it is: it
+// takes 0.78 to 0.96 of the modelled time now (median by class of plan, see wide_is_faster). us of the chosen plan | of all tokens, or
+// 64, per workgroup on 32 rows, unsplit: 28672 x 8192 x 48 22.3 (128 rows) | 40.4; 4096 x 11008 x 32 8.6 (32 rows, 16 tokens) | 12.0;
+// 1024 x 4096 x 256 4.6 (64 rows, 16 tokens) | 6.6; 4096 x 4096 x 128 5.6 (64 rows, 32 tokens) | 7.4.
 // total_groups: row groups of all products of the launch, for each of kWideRows.
 const int kWideRows[3] = {32, 64, 128};
 struct WidePlan {
@@ -355,8 +357,9 @@ WidePlan plan_wide(const long (&total_groups)[3], double results, int n, int k, 
   static const double kFurther[3] = {0.18, 0.06, 0.0};
   const bool cut_lines = n > onebit::kSkinnyMaxN && n % 64;
   // The row groups that multiply one token group run on different XCDs, and each XCD fetches its own copy of x: with more x
-  // than fits an XCD's L2 (4 MB) that is what a launch of few rows waits for (us measured | modelled without it:
-  // 896 x 24256 x 704 45 | 29, 1088 x 13888 x 1758 62 | 38, 640 x 17536 x 676 30 | 19; the main kernel takes 29, 41 and 21).
+  // than fits an XCD's L2 (4 MB) that is what a launch of few rows waits for (fitted to us measured | modelled without it: 896 x 24256
+  // x 704 45 | 29, 1088 x 13888 x 1758 62 | 38, 640 x 17536 x 676 30 | 19. In strips these take 42, 59 and 23 as products, the main
+  // kernel 34, 46 and 26, and 29, 59 and 21 as layers, the main kernel 35, 42 and 26).
   constexpr double kFetchBytesPerUs = 5.6e6;
   const double xcds = std::max(1, compute_units / 32);
   const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
@@ -431,21 +434,21 @@ LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int comput
   return plan;
 }
 
-// wide_kernel against the main kernel. Both models err, and by how much depends on the plans. Measured on 13000 calls of 512 to
-// 28672 rows, k = 512 to 28672 and 65 to 2048 columns (measured / modelled, median): the main kernel's 256 x 128 tile 0.80 for
-// layers and 0.90 for products, its others 0.91 to 1.05; wide_kernel 0.8 to 0.95 where K is one round of its wavefronts, 1.0 to
-// 1.1 on longer K, and 1.0 where it splits K. The lines lie where about as few calls are slower on either side: timed again on
-// 4000 other calls whose modelled times are 0.55 to 1.1 of one another, 25 are more than 5 % slower than on the main kernel, and
-// all are 1.23 times as fast in the mean. One line for all does worse: at 0.81 short K loses (3648 x 992 with 181 tokens 5.6 us,
-// 6.6 on the main kernel; 2176 x 512 with 184 3.8 and 5.2), at 0.88 2496 x 19648 with 197 tokens was 21 % slower than there, and
-// 20864 x 7616 with 152 columns 52 us against 48.
+// wide_kernel against the main kernel. Both models err, and by how much depends on the plans. The lines were drawn where about as few
+// calls were slower on either side, on an earlier wide_kernel. Timed on the kernels as they are (6789 calls of 512 to 28672 rows, k =
+// 512 to 28672 and 65 to 2048 columns whose modelled times are 0.55 to 1.1 of one another, weights from HBM) they lie too low, on the
+// main kernel's side: of the 4115 calls that go to wide_kernel ten are more than 5 % slower than on the main kernel (9 % at most, 2176 x
+// 2048 with 712 tokens 10.0 us, 8.9 there; 20864 x 7616 with 152 columns would be another, 51 and 48), and all 6789 are 1.30 times as
+// fast as there in the mean; 1718 of the other 2674 would be more than 5 % faster here (2496 x 19648 with 197 tokens 25.9 and 27.9). Median
+// of measured / modelled time, wide_kernel and the main kernel, by line: 0.81 0.94 and 0.82 for layers, 0.96 and 0.85 for products; 0.85
+// 0.83 and 0.93; 0.87 0.85 and 0.91; 0.88 0.78 and 0.88; 0.92 0.87 and 0.97 for layers, 0.89 and 0.97 for products.
 // Up to 64 columns the main kernel is the other plan beyond 40960 rows only, where a wavefront of wide_kernel has one short round
 // of work per workgroup and the workgroups come in many rounds, outside what its model was fitted to: the line is the length of
-// K, from which on wide_kernel is faster at 45056 to 262144 rows (us, wide | main, 48 and 64 tokens: 65536 x 1024 17.0 | 12.0 and
-// 19.0 | 12.4, x 4096 28.5 | 31.4 and 32.8 | 31.8, x 8192 44.1 | 60.2 and 50.1 | 60.5; 45056 x 3616 25.4 | 23.9, x 4096
-// 23.5 | 25.1). With k % 64 != 0, where every second token's pieces straddle two lines, it lies twice as far out (45056 x 4128
-// with 48 tokens 28.6 | 26.8, x 8224 43.4 | 47.9). Where the main kernel would split K,
-// wide_kernel in any case (41024 x 7936 and x 8160, 56 and 64 tokens: 46.6 to 49.6 against 53.8 to 56).
+// K, from which on wide_kernel is faster at 45056 to 262144 rows (us, wide | main, 48 and 64 tokens: 65536 x 1024 15.8 | 15.6 and
+// 16.2 | 16.9, x 4096 28.4 | 33.2 and 32.5 | 33.5, x 8192 44.7 | 61.5 and 51.5 | 62.8; 45056 x 3616 24.6 | 26.5 and 27.1 | 26.7,
+// x 4096 23.9 | 27.3 and 28.5 | 27.5). With k % 64 != 0, where every second token's pieces straddle two lines, it lies twice as far out
+// (45056 x 4128 with 48 tokens 30.3 | 28.7, x 8224 45.7 | 51.4). Where the main kernel would split K,
+// wide_kernel in any case (41024 x 7936 and x 8160, 56 and 64 tokens: 44.1 to 47.8 against 55.5 to 59.4).
 bool wide_is_faster(const WidePlan& wide, const LaunchPlan& launch, int n, int k, bool plain) {
   const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
   if (n <= onebit::kSkinnyMaxN) return launch.splits > 1 || chunks >= (n <= 48 ? 16 : 32) * (k % 64 ? 2 : 1);

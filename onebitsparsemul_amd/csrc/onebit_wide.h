@@ -16,14 +16,23 @@ namespace onebit {
 // all tokens, 2 KB per sixteen) in LDS that asynchronous copies fill. No registers hold x on its way, so the tile can be
 // 128 x 64 (R = 4), and with v_smfmac_f32_16x16x64 there are no idle columns at 16 or 48 tokens; one fragment read from LDS
 // serves 2 R SMFMACs (R of the 32x32x32 ones that whole 32-column tiles take).
-// Bound: with many tokens the bytes of x that pass through LDS. skinny_kernel's 64-row groups staged x through registers,
-// 16 KB of LDS writes and reads per 64 x 64 weights; a 128-row group halves that (28672 x 8192 with 48 tokens: 13 us of LDS
-// time, 12 of SMFMACs and 6 of sign expansion that hardly overlapped). With 128 x 64 per workgroup and every compute unit busy
-// it is the 64 bytes per clock that a compute unit takes in: 76 KB of x and weights per 64 K of its eight wavefronts, 1216 of
-// the 1310 clocks they need (60 KB, 960 of 1250, at 48 tokens). us inside a HIP graph, weights from HBM, skinny_kernel ->
-// now: 28672 x 8192 with 24 / 48 / 64 tokens 16.6 / 33.4 / 35.9 -> 14.3 / 19.4 / 21.4; 11008 x 4096 8.0 / 11.0 / 11.7 -> 5.5 /
-// 7.9 / 9.1; 4096 x 4096 5.7 / 8.4 / 8.7 -> 3.6 / 4.7 / 5.1; 1024 x 1024 with 56 5.0 -> 2.65. Up to sixteen tokens there is no
-// gain (11008 x 4096 with 16: 6.4 -> 6.1, with 4: 5.5 -> 5.8; 28672 x 8192 with 16: 13.5 -> 14.0): skinny_kernel keeps those.
+// Bound: no single resource. Stamps of every wavefront, launches back to back, weights from HBM (us after the first one's start,
+// wavefronts 0-3 | 4-7):
+//                                        28672 x 8192, 48 tokens   the same, 64   4096 x 11008, 500 tokens
+//   first operand and image there        2.6 | 3.3                 2.8 | 3.4      2.0 | 2.9
+//   first chunk multiplied               7.5 | 6.6                 8.3 | 7.1      6.9 | 6.3
+//   last chunk (of 4, 4, 6 or 5)         17.5 | 14.5               19.7 | 16.6    24.7 | 19.5
+//   all partial tiles in LDS             18.0                      20.5           25.9
+//   tiles added, stored                  21.9                      24.6           28.0
+// 2 to 3 us until the operands come; the first chunk, four memory latencies beside its work; a chunk of each of the eight wavefronts
+// from then on 5400 to 5900 clocks of those that go first, 6900 to 7200 of the others, against 5000 to 5200 of a full pipeline that a
+// compute unit's 64 bytes per clock set (76 KB of x and weights per 64 K at 64 tokens, 60 at 48); those that go first then wait 3 to 6
+// us; and 2 to 4 us of reduction. SMFMACs fill 30 % (48 tokens) and 47 % (500) of the time.
+// skinny_kernel's 64-row groups staged x through registers, 16 KB of LDS writes and reads per 64 x 64 weights; a 128-row group halves
+// that. us inside a HIP graph under load, weights from HBM, skinny_kernel -> now: 28672 x 8192 with 24 / 48 / 64 tokens 16.6 / 33.4 /
+// 35.9 -> 15.6 / 21.8 / 23.8; 11008 x 4096 8.0 / 11.0 / 11.7 -> 6.3 / 8.0 / 9.5; 4096 x 4096 5.7 / 8.4 / 8.7 -> 3.8 / 4.6 / 4.7; 1024 x
+// 1024 with 56 5.0 -> 2.55. Up to sixteen tokens there is no gain (11008 x 4096 with 16: 6.4 -> 6.1, with 4: 5.5 -> 5.8; 28672 x 8192
+// with 16: 13.5 -> 14.0): skinny_kernel keeps those.
 // Beyond 64 tokens, and for products, the host's plan compares it with the kernel it would replace (onebit_capi.hip).
 // =====================================================================================================
 // Source of zeros for the copies of K positions at or past K.
