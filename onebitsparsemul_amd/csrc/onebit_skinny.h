@@ -665,11 +665,13 @@ __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_kernel(u32x8
 
 // The same with its arguments as a struct: all of them loaded at the start, the compiler's schedule of the image's requests and
 // stores another one. Pieces at any alignment are the faster for it with images of 32 and 64 columns, and with those of sixteen where
-// a wavefront of a 128-row group has one or two chunks, or one of a 64-row group two (us inside a HIP graph, weights from HBM, vectors | struct: 4096 x 33 x
-// 4096 12.8 | 12.1, 1344 x 47 x 1376 6.6 | 6.2, 4096 x 18 x 4096 5.9 | 5.7, 832 x 18 x 6112 7.0 | 6.9; 24576 x 3 x 4096 10.6 | 9.8,
-// 17408 x 8 x 2048 6.0 | 5.7, 9216 x 3 x 4096 7.4 | 7.2). Elsewhere the vectors are (28672 x 8 x 8192 13.8 | 16.0, 18432
-// x 3 x 8192 14.4 | 16.0, 25280 x 11 x 4992 13.0 | 13.7; 64-row groups of one chunk: 8256 x 13 x 512 4.1 | 4.2, 10176 x 3 x 2048 4.7 |
-// 4.8; 32-row groups: 2048 x 8 x 3456 3.75 | 3.87, 8192 x 3 x 8192 8.4 | 8.7).
+// a wavefront of a 128-row group has one or two chunks, or one of a 64-row group two, and more where the pieces of ten to fourteen
+// columns start at whole words (us inside a HIP graph, weights from HBM, vectors | struct: 4096 x 33 x 4096 12.8 | 12.1, 1344 x 47 x 1376
+// 6.6 | 6.2, 4096 x 18 x 4096 5.9 | 5.7, 832 x 18 x 6112 7.0 | 6.9; 24576 x 3 x 4096 10.6 | 9.8, 17408 x 8 x 2048 6.0 | 5.7, 9216 x 3 x
+// 4096 7.4 | 7.2; 12672 x 12 x 6752 9.96 | 9.68, 13888 x 10 x 9952 13.65 | 13.16, 9344 x 14 x 24032 27.4 | 25.9). Elsewhere the vectors are
+// (28672 x 8 x 8192 13.8 | 16.0, 18432 x 3 x 8192 14.4 | 16.0, 25280 x 11 x 4992 13.0 | 13.7; 64-row groups of one chunk: 8256 x 13 x 512
+// 4.1 | 4.2, 10176 x 3 x 2048 4.7 | 4.8, of three and more 1 to 3 % where a piece may start at any half, none from the sixth on; 32-row
+// groups: 2048 x 8 x 3456 3.75 | 3.87, 8192 x 3 x 8192 8.4 | 8.7).
 template <int NW, int R, int MODE, int NC, bool BF16>
 __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_struct_kernel(SkinnyArgs p) {
   skinny_body<NW, R, MODE, NC, BF16>(p, blockIdx.x, blockIdx.y);
@@ -753,11 +755,13 @@ template <int NW, int R, int MODE, int NC, bool BF16 = false>
 static hipError_t launch_skinny_mode(const SkinnyArgs& args, hipStream_t stream) {
   const dim3 grid((args.m / kRowBlock + R - 1) / R, args.splits), threads(64 * NW);
   constexpr bool kPieces = MODE == kSkinnyBAny;
-  if constexpr (kPieces && (NC > 16 || NW <= 8))
-    if (NC > 16 || (args.chunks_per_split > (R == 2 ? NW : 0) && args.chunks_per_split <= 2 * NW)) {  // see skinny_struct_kernel
+  if constexpr (kPieces && (NC > 16 || NW <= 8)) {  // see skinny_struct_kernel
+    const bool words = R == 2 && args.n >= 10 && args.n <= 14 && args.n % 2 == 0 && (reinterpret_cast<uintptr_t>(args.b) & 3) == 0;
+    if (NC > 16 || (args.chunks_per_split > (R == 2 ? NW : 0) && (words || args.chunks_per_split <= 2 * NW))) {
       hipLaunchKernelGGL((skinny_struct_kernel<NW, R, MODE, NC, BF16>), grid, threads, 0, stream, args);
       return hipGetLastError();
     }
+  }
   if constexpr (!kPieces || NC == 16) {
     LaunchArgs a = pack_args(args);
     a.operands[7] |= a.flags << 24;

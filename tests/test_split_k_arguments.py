@@ -1,4 +1,6 @@
-"""The split-K kernel's two argument forms, on either side of the lines between them (eight and sixteen chunks of K per split), with all that a call can pass: C of either type, alpha, beta, results of either type, K split or not. Integer operands:
+"""The split-K kernel's two argument forms, on either side of the lines between them (eight and sixteen chunks of K per split, ten to
+fourteen columns in whole words or not), with all that a call can pass: C of either type, alpha, beta, results of either type, K split or
+not. Integer operands:
 bit-exact."""
 import numpy as np
 import pytest
@@ -18,7 +20,7 @@ def _defaults():
 
 
 @pytest.mark.parametrize("rows", [32, 64, 128])
-@pytest.mark.parametrize("n", [1, 2, 3, 4, 8, 13, 16, 18, 32, 41, 64])
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 8, 10, 13, 14, 16, 18, 32, 41, 64])
 def test_every_argument_reaches_the_kernel(rows, n):
     _native.set_skinny_rows(rows)
     for m, k, splits in ((192, 2048, 1), (192, 2080, 1), (192, 4096, 1), (192, 4128, 1), (64, 8192, 2), (64, 8224, 2)):
