@@ -24,7 +24,7 @@ namespace onebit {
 //   last chunk (of 4, 4, 6 or 5)         17.5 | 14.5               19.7 | 16.6    24.7 | 19.5
 //   all partial tiles in LDS             18.0                      20.5           25.9
 //   tiles added, stored                  21.9                      24.6           28.0
-// 2 to 3 us until the operands come; the first chunk, four memory latencies beside its work; a chunk of each of the eight wavefronts
+// 2 to 3 us until the operands come; the first chunk, up to 1.7 us longer than a later one; a chunk of each of the eight wavefronts
 // from then on 5400 to 5900 clocks of those that go first, 6900 to 7200 of the others, against 5000 to 5200 of a full pipeline that a
 // compute unit's 64 bytes per clock set (76 KB of x and weights per 64 K at 64 tokens, 60 at 48); those that go first then wait 3 to 6
 // us; and 2 to 4 us of reduction. SMFMACs fill 30 % (48 tokens) and 47 % (500) of the time.
