@@ -54,7 +54,10 @@ struct WideShape {
 // TOKENS = false is the plain form, D = alpha A B + beta C, a column of B in the place of a token: B's rows start 16-byte
 // aligned (ldb % 8 == 0, first_token % 8 == 0), an image is 64 of them as they lie, COPIES 16-byte pieces each, read through
 // transpose reads; COPIES is even.
-template <int R, int COPIES, bool TOKENS, bool BF16>
+// PARTS: the chunks that are left after whole rounds of eight, up to four of them, are dealt over the wavefronts in parts
+// of 64 or 128 K values, where otherwise some wavefronts have a chunk more and the others wait for them: 9 chunks are five
+// images in a row instead of eight, 43 are 22 instead of 24.
+template <int R, int COPIES, bool TOKENS, bool BF16, bool PARTS>
 __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x, const int block_y, const int first_token,
                                           char* const smem) {
   using Shape = WideShape<R, COPIES>;
@@ -302,6 +305,14 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
   // here on. us, weights from HBM, both: 28672 x 8192 with 64 23.7 -> 22.9, 16384 x 16384 with 64 26.9 -> 25.6, 4096 x 4096 with
   // 32 3.93 -> 3.72, 2048 x 8192 with 256 10.4 -> 9.8.
   if (first < kc_end) {
+    // parts: the remainder's chunks in halves, up to two of them in quarters
+    static_assert((NW & (NW - 1)) == 0, "a round is a power of two");
+    const int left = (kc_end - kc_begin) & (NW - 1);
+    const int halvings = !PARTS || left > 4 || kc_end - kc_begin < NW ? 0 : left > 2 ? 1 : 2;
+    const int whole_end = halvings ? kc_end - left : kc_end;
+    const int part_kc = whole_end + (wave >> halvings), part_images = 4 >> halvings;
+    const int part_image = (wave & ((1 << halvings) - 1)) * part_images;  // first image of the part, of four
+    const bool has_part = PARTS && part_kc < kc_end;
     copy_image(first * kChunkK, 0);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (S32) {
@@ -312,14 +323,17 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
       __builtin_amdgcn_sched_barrier(0);
     }
     copy_image(first * kChunkK + kWideImageK, 1);
-    if (FAR && first + NW < kc_end) load_a(first + NW, next);
+    if (FAR && first + NW < whole_end) load_a(first + NW, next);
+    else if (FAR && PARTS && has_part) load_a(part_kc, next);
     __builtin_amdgcn_sched_barrier(0);
     if (wave >= NW / 2) __builtin_amdgcn_s_setprio(1);
     if constexpr (!S32) gather(raw);
     int kc = first;
 #pragma unroll 1
     do {
-      const bool more = kc + NW < kc_end;
+      const bool whole = kc + NW < whole_end, more = whole || has_part;  // what follows: a chunk, a part or nothing
+      const int next_kc = !PARTS || whole ? kc + NW : part_kc;
+      const int next_k0 = next_kc * kChunkK + (!PARTS || whole ? 0 : part_image * kWideImageK);
       auto stage = [&](auto s_tag) __attribute__((always_inline)) {
         constexpr int S = decltype(s_tag)::value;
         // all but the requests younger than image S
@@ -334,16 +348,16 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
 #pragma unroll
           for (int r = 0; r < R; ++r) asm volatile("" : "+v"(next[r].meta), "+v"(next[r].sign));
         }
-        if (S < 2 || more) {
+        if (S < 2 || (S == 2 ? more : whole || (has_part && part_images > 1))) {
           wait_vmcnt_lgkm0<63>();  // the image is in registers: its place is free
           asm volatile("" ::: "memory");
           __builtin_amdgcn_sched_barrier(0);
-          copy_image(S < 2 ? kc * kChunkK + (S + 2) * kWideImageK : (kc + NW) * kChunkK + (S - 2) * kWideImageK, S & 1);
+          copy_image(S < 2 ? kc * kChunkK + (S + 2) * kWideImageK : next_k0 + (S - 2) * kWideImageK, S & 1);
           __builtin_amdgcn_sched_barrier(0);
         }
         compute(s_tag);
         if constexpr (S == 0 && !FAR) {
-          if (more) load_a(kc + NW, next);
+          if (more) load_a(next_kc, next);
           __builtin_amdgcn_sched_barrier(0);
         }
       };
@@ -351,18 +365,41 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
       stage(std::integral_constant<int, 1>{});
       stage(std::integral_constant<int, 2>{});
       stage(std::integral_constant<int, 3>{});
+      if (PARTS && !whole && has_part) {  // the operand of the part's images to the front
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          if (part_image & 2) next[r].meta.x = next[r].meta.z, next[r].meta.y = next[r].meta.w, next[r].sign.x = next[r].sign.y;
+          if (part_image & 1) next[r].meta.x = next[r].meta.y, next[r].sign.x <<= 8;
+        }
+      }
       if constexpr (S32) {
 #pragma unroll
         for (int r = 0; r < R; ++r) raw[r] = next[r];
       } else {
         gather(next);
         if constexpr (FAR) {
-          if (kc + 2 * NW < kc_end) load_a(kc + 2 * NW, next);
+          if (whole && kc + 2 * NW < whole_end) load_a(kc + 2 * NW, next);
+          else if (PARTS && whole && has_part) load_a(part_kc, next);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
       kc += NW;
-    } while (kc < kc_end);
+    } while (kc < whole_end);
+    if (PARTS && has_part) {
+      if (part_images > 1) wait_vmcnt<COPIES>();
+      else wait_vmcnt<0>();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      read_image(0);
+      compute(std::integral_constant<int, 0>{});
+      if (part_images > 1) {
+        wait_vmcnt<0>();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        read_image(1);
+        compute(std::integral_constant<int, 1>{});
+      }
+    }
   }
 
   // ---- add the eight partial tiles, RT row blocks per round: a token's rows as 16-byte slots of four rows, slot s at
@@ -434,7 +471,7 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
 // In strips of two column groups an XCD is given a contiguous range of the list (workgroup b runs on XCD b % 8, all eight are there:
 // the launcher's condition), so that what its workgroups read of x and of the weight meets in its L2; where that pays is the host's
 // rule (wide_in_strips).
-template <int R, int COPIES, bool TOKENS, bool BF16>
+template <int R, int COPIES, bool TOKENS, bool BF16, bool PARTS>
 __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_kernel(u32x8_t operands, u32x4_t results, u32x2_t shape, u32x2_t scale) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   SkinnyArgs p = unpack_args(operands, results, scale, shape[0]);
@@ -451,7 +488,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_kernel(u32x8_t operan
     x = pair ? w >> 1 : w;
     group = 2 * strip + (pair ? w & 1 : 0);
   }
-  wide_body<R, COPIES, TOKENS, BF16>(p, x, blockIdx.y, group * p.tokens_per_group, smem);
+  wide_body<R, COPIES, TOKENS, BF16, PARTS>(p, x, blockIdx.y, group * p.tokens_per_group, smem);
 }
 
 // The dynamic-LDS limit of a kernel, a per-device attribute; threads that race here set the same value.
@@ -466,11 +503,19 @@ static hipError_t wide_lds_limit(const void* kern, int lds, std::atomic<bool> (&
   return hipSuccess;
 }
 
-template <int R, int COPIES, bool TOKENS, bool BF16>
-static hipError_t launch_wide_kernel(const SkinnyArgs& args, hipStream_t stream) {
+// Whether a workgroup that multiplies `chunks` chunks deals a remainder in parts. us inside HIP graphs, weights from HBM, a chunk to a
+// wavefront | parts: one or two chunks left of two rounds, layers 5760 x 2272 with 54 tokens 5.76 | 5.37, 2752 x 2368 with 62 5.26 | 4.73,
+// 5568 x 2496 with 21 5.20 | 4.63, 10048 x 2464 with 43 8.42 | 7.74, 1472 x 2496 with 128 5.46 | 4.92; of more rounds 28672 x 8448 with
+// 48 23.6 | 23.0, 6720 x 8352 with 17 9.45 | 8.89, 1280 x 10592 with 153 10.4 | 10.0; three chunks of six rounds equal (4096 x 11008
+// with 32 / 500 8.55 | 8.38, 30.8 | 30.6). From five chunks on a part is a chunk, and below a round the calls wait for the host. The build
+// of the kernel without parts is 1 to 4 % faster where there are none (4096 x 4096 with 48 5.2 | 5.4).
+static bool wide_has_parts(int chunks) { return chunks >= kWideWaves && chunks % kWideWaves >= 1 && chunks % kWideWaves <= 4; }
+
+template <int R, int COPIES, bool TOKENS, bool BF16, bool PARTS>
+static hipError_t launch_wide_parts(const SkinnyArgs& args, hipStream_t stream) {
   static std::atomic<bool> attr_done[64] = {};
   constexpr int lds = WideShape<R, COPIES>::LDS_BYTES;
-  const auto kern = wide_kernel<R, COPIES, TOKENS, BF16>;
+  const auto kern = wide_kernel<R, COPIES, TOKENS, BF16, PARTS>;
   if (hipError_t st = wide_lds_limit(reinterpret_cast<const void*>(kern), lds, attr_done); st != hipSuccess) return st;
   const int rows = (args.m + 32 * R - 1) / (32 * R), groups = (args.n + args.tokens_per_group - 1) / args.tokens_per_group;
   LaunchArgs a = pack_args(args);
@@ -479,6 +524,13 @@ static hipError_t launch_wide_kernel(const SkinnyArgs& args, hipStream_t stream)
   const dim3 grid = args.strips ? dim3(rows * groups, args.splits) : dim3(rows, args.splits, groups);
   hipLaunchKernelGGL(kern, grid, dim3(64 * kWideWaves), lds, stream, a.operands, a.results, shape, a.scale);
   return hipGetLastError();
+}
+
+template <int R, int COPIES, bool TOKENS, bool BF16>
+static hipError_t launch_wide_kernel(const SkinnyArgs& args, hipStream_t stream) {
+  if (wide_has_parts(args.chunks_per_split))  // of all splits but perhaps the last
+    return launch_wide_parts<R, COPIES, TOKENS, BF16, true>(args, stream);
+  return launch_wide_parts<R, COPIES, TOKENS, BF16, false>(args, stream);
 }
 
 }  // namespace onebit
