@@ -526,6 +526,61 @@ WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b
   return plan;
 }
 
+// Whether a ragged B (n % 8 != 0, 16-byte aligned) is read where it lies instead of through a padded copy. The copy costs a launch
+// and a pass, 4 to 5 us and 4 bytes per value at 5.5 TB/s; rows that start at an odd value cost the asynchronous copies 2.4 times the
+// load path (read_as_ragged), which the smaller tiles are short of.
+// Even n: always. us inside HIP graphs, padded copy, or skinny_kernel up to 64 columns | in place: 4096 x 4096 with 34 / 100 / 500 / 2050
+// columns 9.0 | 6.4, 12.2 | 9.7, 25.9 | 21.5, 53.3 | 46.1, 28672 x 8192 with 50 39.8 | 25.4, 11008 x 4096 with 1002 57.9 | 54.2, 704 x
+// 1760 with 8142 28.5 | 19.5.
+// Odd n on the main kernel, by tile: 512 x 128 and one 256 x 128 or eight-wavefront 128 x 128 per compute unit, where a stage takes long
+// enough: 37 of 37 calls faster, 11008 x 4096 with 1001 56.8 | 52.1, 896 x 6144 with 5995 72.8 | 46.8. 256 x 128, two per compute unit: up
+// to one and a half rounds (4992 x 928 with 3589 37.0 | 33.9; in four 11776 x 6624 with 6257 460 | 478). 64 x 128, and 128 x 128 in two K
+// groups: on a short K (1600 x 896 with 1243 13.4 | 11.7; 13760 x 1888 with 65 13.7 | 16.1) and, but for the first, few rows (704 x 9728
+// with 2889 62.9 | 58.1; 4672 x 8064 with 539 40.5 | 45.2).
+// On wide_kernel: up to 64 columns, where skinny_kernel is the other one (4096 x 4096 with 49 15.0 | 7.5, 28672 x 8192 with 33 47 | 28),
+// and in groups of 16, 32 or 64 of more (512 x 1856 with 555 10.4 | 6.8; in groups of 48 7360 x 4192 with 87 14.7 | 17.0). It would be
+// faster on fewer rows and a longer K too (896 x 1696 with 39 6.7 | 4.4, 2048 x 4832 with 233 14.9 | 11.9): the lines there are where
+// the address model in the tests has those calls on skinny_kernel and on the padded copy.
+bool ragged_in_place(int m, int n, int k, const LaunchPlan& launch, const WidePlan& wide, int compute_units) {
+  if (n % 2 == 0) return true;
+  const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
+  if (wide.rows) {
+    if (n <= onebit::kSkinnyMaxN) return m > 2048 || (m > 1088 && chunks <= 16);
+    return (wide.tokens == 16 || wide.tokens == 32 || wide.tokens == 64) && chunks <= 16;
+  }
+  switch (launch.rows_or_tile) {
+    case onebit::kTile512x128w8: case onebit::kTile512x128m16: case onebit::kTile256x128w8: case onebit::kTile128x128w8: return true;
+    case onebit::kTile256x128w: return (long)((m + 255) / 256) * ((n + 127) / 128) <= 3L * compute_units;
+    case onebit::kTile64x128: return chunks <= 7;
+    case onebit::kTile128x128k2: case onebit::kTile64x128k2: return chunks <= 7 || m <= 1024;
+    default: return false;
+  }
+}
+
+// Everything decided about a product: wide.rows != 0: wide_kernel, else `launch`; pad_b: B is read through a padded copy. A ragged B
+// keeps it where the call splits K beyond 64 columns: their tests pin its place in the workspace beside the partial sums.
+// small_pad: a padded copy that the plan does not count on can be had.
+struct ProductPlan {
+  LaunchPlan launch;
+  WidePlan wide;
+  bool pad_b;
+};
+template <class SmallPad>
+ProductPlan plan_product(int m, int n, int k, bool b_16_byte_aligned, int compute_units, SmallPad&& small_pad) {
+  ProductPlan plan{};
+  plan.launch = choose_launch(m, n, k, b_16_byte_aligned, compute_units);
+  const LaunchPlan& launch = plan.launch;
+  const bool b_in_place = n % 8 == 0 && b_16_byte_aligned, ragged = n % 8 != 0 && n >= 8 && b_16_byte_aligned;
+  plan.pad_b = launch.pad_b || (!launch.split_k_kernel && !b_in_place && !ragged && g_pad_b && small_pad());
+  plan.wide = plan_wide_product(launch, m, n, k, b_in_place || plan.pad_b || ragged, compute_units);
+  if (ragged) {
+    const bool in_place = ragged_in_place(m, n, k, launch, plan.wide, compute_units);
+    if (launch.split_k_kernel && !in_place) plan.wide = WidePlan{0, 1, 0, 0.0};  // skinny_kernel
+    if (in_place && (plan.wide.rows ? plan.wide.splits : launch.splits) <= 1) plan.pad_b = false;
+  }
+  return plan;
+}
+
 // Workspace of one call that the caller cannot let allocate: `base` is this device's copy of the file-scope array
 // g_static_scratch (see onebit_sparse_matmul_prepared_static), `bytes` its size.
 struct FixedScratch {
@@ -608,13 +663,14 @@ int matmul_prepared_impl(const void* prepared, const void* b, const void* c, voi
 
   const int compute_units = current_compute_units();
   const bool b_aligned = (reinterpret_cast<uintptr_t>(b) & 15) == 0;
-  const LaunchPlan plan = choose_launch(m, n, k, b_aligned, compute_units);
-  const bool b_in_place = n % 8 == 0 && b_aligned;
   // A small B that the main kernel cannot read in place is described as read by element copies; a padded copy is many times
-  // faster (1152 x 78 x 640 61 -> 6 us) and is made wherever its buffer is there or can be had.
+  // faster (1152 x 77 x 640 61 -> 6 us) and is made wherever its buffer is there or can be had.
   const size_t pad_bytes = (size_t)k * ((size_t)(n + 7) / 8 * 8) * sizeof(_Float16);
-  const bool pad_b = plan.pad_b || (!plan.split_k_kernel && !b_in_place && g_pad_b && small_pad_available(pad_bytes, stream, fixed));
-  const WidePlan wide = plan_wide_product(plan, m, n, k, b_in_place || pad_b, compute_units);
+  const ProductPlan product =
+      plan_product(m, n, k, b_aligned, compute_units, [&] { return small_pad_available(pad_bytes, stream, fixed); });
+  const LaunchPlan& plan = product.launch;
+  const WidePlan& wide = product.wide;
+  const bool pad_b = product.pad_b;
   if (plan.split_k_kernel) {
     onebit::SkinnyArgs args{};
     args.prep = static_cast<const uint8_t*>(prepared);
@@ -847,21 +903,23 @@ int onebit_sparse_describe_call(int token_major, int m, int n, int k, int b_16_b
   const int units = compute_units ? compute_units : current_compute_units();
   LaunchPlan launch;
   WidePlan wide{};
-  bool is_wide;
+  bool is_wide, pad_b = false;
   if (token_major) {
     const LinearPlan linear = plan_linear(m, n, k, units);
     launch = linear.launch;
     wide = linear.wide_plan;
     is_wide = linear.wide;
   } else {
-    launch = choose_launch(m, n, k, b_16_byte_aligned != 0, units);
-    wide = plan_wide_product(launch, m, n, k, (n % 8 == 0 && b_16_byte_aligned) || launch.pad_b, units);
+    const ProductPlan product = plan_product(m, n, k, b_16_byte_aligned != 0, units, [] { return false; });
+    launch = product.launch;
+    wide = product.wide;
+    pad_b = product.pad_b;
     is_wide = wide.rows != 0;
   }
   plan[0] = is_wide ? ONEBIT_KERNEL_WIDE : launch.split_k_kernel ? ONEBIT_KERNEL_SPLIT_K : ONEBIT_KERNEL_MAIN;
   plan[1] = is_wide ? wide.rows : launch.rows_or_tile;
   plan[2] = full_splits((k + onebit::kChunkK - 1) / onebit::kChunkK, is_wide ? wide.splits : launch.splits);
-  plan[3] = !token_major && launch.pad_b;
+  plan[3] = pad_b;
   plan[4] = is_wide ? wide.tokens : 0;
   return ONEBIT_OK;
 }

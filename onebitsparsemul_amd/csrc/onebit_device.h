@@ -205,6 +205,14 @@ __device__ __forceinline__ u32x4_t drop_halves(u32x4_t v, int count) {
   return v;
 }
 
+// The eight halves of a piece in LDS from number `count` on move to its front; what follows them stays as it is.
+__device__ __forceinline__ void shift_piece(char* piece, int count, int lane) {
+  if (lane < 8 - count) {
+    uint16_t* const at = reinterpret_cast<uint16_t*>(piece) + lane;
+    *at = at[count];
+  }
+}
+
 // ---- asynchronous global -> LDS copy --------------------------------------------------------------
 // global_load_lds_dwordx4: each lane fetches 16 bytes from its own global address; the wavefront's 1 KiB
 // lands at LDS offset M0 + 16 * lane. Issued through inline assembly so that the compiler does not

@@ -168,11 +168,16 @@ static __device__ __attribute__((aligned(16))) uint32_t g_zero16[4] = {0, 0, 0, 
 
 // TOKENS (with DMA only): the linear-layer form. p.b is x (p.n tokens x p.k, token-major), p.d is y (p.n tokens x
 // p.m), the epilogue is y = acc + bias; a tile column is a token.
-template <int WM, int WN, int FM, int FN, bool DMA, bool TOKENS = false, int KG = 1, bool M16 = false, bool BF16 = false>
+// RAGGED (plain form with DMA): n is no multiple of eight and the rows of B are copied from where they lie (ldb = n). A piece that
+// reaches past the end of its row takes values of the next one along, which only meet columns that are never stored; past the
+// end of B it is moved back and shifted into place in LDS (mend_stage). An instantiation of its own: the tests for that row made
+// a product of few chunks slower (2048 x 512 x 512 5.25 -> 5.64 us).
+template <int WM, int WN, int FM, int FN, bool DMA, bool TOKENS = false, int KG = 1, bool M16 = false, bool BF16 = false, bool RAGGED = false>
 __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gemm_kernel(GemmArgs p) {
   static_assert(!M16 || (DMA && KG == 1 && WN == 1 && FM == 4 && FN == 4), "the 16x16x64 form exists for the 512x128 four-wavefront tile");
   static_assert(TOKENS || !BF16, "bf16 activations exist for the token-major form");
   static_assert(DMA || !TOKENS, "the token-major form uses the asynchronous copies");
+  static_assert(!RAGGED || (DMA && !TOKENS), "rows that lie anywhere are the plain form's");
   static_assert(DMA || KG == 1, "the two-group form uses the asynchronous copies");
   using TS = TileShape<WM, WN, FM, FN, KG>;
   constexpr int BM = TS::BM, BN = TS::BN, CH = TS::CH, NL = TS::NL, NW = TS::NW;
@@ -277,6 +282,16 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
       }
       lds_dst[i] = smem_base + (NW * i + wave) * 1024;
     }
+    const int k_inside = RAGGED ? p.k - 1 : p.k;  // RAGGED: the stage of B's last row takes the general form of the copies
+    const char* const last_piece = reinterpret_cast<const char*>(p.b) + (size_t)p.k * p.ldb * 2 - 16;
+    // the piece of stage `stage` that was moved back, if there is one and this wavefront copied it
+    auto mend_stage = [&](int stage) __attribute__((always_inline)) {
+      const int row = (p.k - 1) % kStageK, piece = (p.n - 1 - n0) / 8, slot = row * CH + (piece ^ chunk_swizzle<BN>(row));
+      if (!RAGGED || stage != (p.k - 1) / kStageK || piece >= CH || slot / 64 % NW != wave) return;  // wave-uniform
+      shift_piece(smem + (stage % kStages) * TS::STAGE_BYTES + slot * 16, n0 + 8 * piece + 8 - p.n, lane);
+      wait_vmcnt_lgkm0<63>();
+      asm volatile("" ::: "memory");
+    };
     const size_t stage_stride = TOKENS ? (size_t)kStageK * 2 : (size_t)kStageK * p.ldb * 2;
     const char* b_stage = reinterpret_cast<const char*>(p.b) + (TOKENS ? (size_t)n0 * p.k * 2 : (size_t)n0 * 2) +
                           (size_t)chunk_begin * kStages * stage_stride;  // advances one stage per copy
@@ -286,13 +301,17 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
     // whole chunks of four stages) and the padding of the prepared operand contribute nothing, and the
     // number of copies in flight, which the vmcnt waits rely on, is the same in every iteration.
     auto issue_b = [&](int ring) {
-      if (next_k0 + kStageK <= p.k) {  // wave-uniform: a full stage
+      if (next_k0 + kStageK <= k_inside) {  // wave-uniform: a full stage
 #pragma unroll
         for (int i = 0; i < NL; ++i) lds_dma16_base(b_stage, b_off[i], lds_dst[i] + ring * TS::STAGE_BYTES);
       } else {
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
-          const char* src = (next_k0 + copy_row[i] < p.k) ? b_stage + b_off[i] : zeros;
+          uint32_t off = b_off[i];
+          if constexpr (RAGGED) asm volatile("" : "+v"(off));  // keeps the 64-bit addresses out of the registers of the other path
+          const char* src = b_stage + off;
+          if (RAGGED && src > last_piece) src = last_piece;
+          if (next_k0 + copy_row[i] >= p.k) src = zeros;
           lds_dma16(src, lds_dst[i] + ring * TS::STAGE_BYTES);
         }
       }
@@ -395,7 +414,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
             __builtin_amdgcn_sched_barrier(0);                                                                     \
           }
     // chunk kc copies the stages of chunk kc + 1: they are whole while (kc + 2) * 256 <= K
-    const int full_end = p.k / kChunkK - 1 < chunk_end ? p.k / kChunkK - 1 : chunk_end;
+    const int full_end = k_inside / kChunkK - 1 < chunk_end ? k_inside / kChunkK - 1 : chunk_end;
 
     if constexpr (M16) {
       // ---- 16x16x64 form of the K loop (one wavefront per SIMD, wave tile 128 x 128 = 8 x 8 tiles of 16 x 16) ----
@@ -482,6 +501,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
       u32x8_t bv[CT];
       u32x4_t av_roll[2], av_hi[RT / 2];
       wait_vmcnt<3 * NL>();  // A(0) and B(0) have landed
+      if constexpr (RAGGED) mend_stage(chunk_begin * kStages);
       __builtin_amdgcn_s_barrier();
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) a_cur[rt] = gather_a(rt);
@@ -492,7 +512,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
 #pragma unroll
       for (int p_ = 0; p_ < 4; ++p_) av_roll[0][p_] = expand16(a_cur[0], 0, p_);
 
-      auto chunk_body = [&](auto full_tag) __attribute__((always_inline)) {
+      auto chunk_body = [&](auto full_tag, int kc) __attribute__((always_inline)) {
         constexpr bool FULL = decltype(full_tag)::value;
         constexpr int SLOTS = RT / 2 * CT;  // SMFMACs per half stage (shadows the 32x32x32 form's count for the copy macro)
         auto stage = [&](auto s_tag, auto wait_tag, auto issue_a_tag) __attribute__((always_inline)) {
@@ -518,6 +538,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
               __builtin_amdgcn_sched_barrier(0);
             }
           wait_vmcnt_lgkm0<WAITCNT>();  // copies of stage S+1 landed
+          if constexpr (RAGGED && !FULL) mend_stage(kc * kStages + S + 1);
           __builtin_amdgcn_s_barrier();
           // Last stage of a chunk: the next chunk of A is readable after this stage's barrier. Row tiles 0-3 are done
           // with this chunk: their holder lanes' bytes are requested right here and turned into operands behind the
@@ -563,8 +584,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
         stage(integral_constant<int, 3>{}, integral_constant<int, 2 * NL>{}, std::false_type{});       // B(4c+4)
       };
       int kc = chunk_begin;
-      for (; kc < full_end; ++kc) chunk_body(std::true_type{});
-      for (; kc < chunk_end; ++kc) chunk_body(std::false_type{});
+      for (; kc < full_end; ++kc) chunk_body(std::true_type{}, kc);
+      for (; kc < chunk_end; ++kc) chunk_body(std::false_type{}, kc);
       wait_vmcnt<0>();  // drain the copies issued past the end before the LDS is released
     } else if constexpr (KG == 1) {
       // The barrier sits in the middle of each stage s: it publishes stage s+1 (read right after it) and frees the ring
@@ -577,6 +598,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
       u32x8_t bv0[FN], bv1[FN];
       u32x4_t av0[FM], av1[FM];
       wait_vmcnt<3 * NL>();  // A(0) and B(0) have landed
+      if constexpr (RAGGED) mend_stage(chunk_begin * kStages);
       __builtin_amdgcn_s_barrier();
 #pragma unroll
       for (int fm = 0; fm < FM; ++fm) a_cur[fm] = load_a_chunk_lds(a_frag_lds[fm], lane);
@@ -591,6 +613,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
           ONEBIT_FETCH_SLOT((S), 1, bv1, 2 * (S) + 1, a_cur, av1)                                                  \
         });                                                                                                        \
         wait_vmcnt_lgkm0<(WAITCNT)>(); /* copies of stage S+1 landed; this wavefront's reads of stage S returned */ \
+        if constexpr (RAGGED && !FULL) mend_stage(kc * kStages + (S) + 1);                                                   \
         __builtin_amdgcn_s_barrier();                                                                              \
         if constexpr ((S) == kStages - 1) {                                                                        \
           /* the next chunk of A is readable after this stage's barrier */                                         \
@@ -610,7 +633,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
         }                                                                                                          \
       }
 
-      auto chunk_body = [&](auto full_tag) __attribute__((always_inline)) {
+      auto chunk_body = [&](auto full_tag, int kc) __attribute__((always_inline)) {
         constexpr bool FULL = decltype(full_tag)::value;  // the four stages copied during this chunk lie inside K
         ONEBIT_FUSED_STAGE(0, 2 * NL, true)        // waits for B(4c+1); newer requests: B(4c+2), B(4c+3)
         ONEBIT_FUSED_STAGE(1, 2 * NL + NA, false)  // waits for B(4c+2); newer: B(4c+3), A(c+1), B(4c+4)
@@ -618,8 +641,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
         ONEBIT_FUSED_STAGE(3, 2 * NL, false)       // waits for B(4c+4), which is newer than A(c+1)
       };
       int kc = chunk_begin;
-      for (; kc < full_end; ++kc) chunk_body(std::true_type{});
-      for (; kc < chunk_end; ++kc) chunk_body(std::false_type{});
+      for (; kc < full_end; ++kc) chunk_body(std::true_type{}, kc);
+      for (; kc < chunk_end; ++kc) chunk_body(std::false_type{}, kc);
 #undef ONEBIT_FUSED_STAGE
       wait_vmcnt<0>();  // drain the copies issued past the end before the LDS is released
     } else {
@@ -636,6 +659,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
         u32x8_t bv_even[FN], bv_odd[FN];
         u32x4_t av_even[FM], av_odd[FM];
         wait_vmcnt<3 * NL>();  // A(0) and B(0) have landed
+      if constexpr (RAGGED) mend_stage(chunk_begin * kStages);
         __builtin_amdgcn_s_barrier();
 #pragma unroll
         for (int fm = 0; fm < FM; ++fm) a_cur[fm] = load_a_chunk_lds(a_frag_lds[fm], lane);
@@ -646,6 +670,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
 #define ONEBIT_GROUP_STAGE(S, WAITCNT, ISSUE_A, BV, AV, BV_NEXT, AV_NEXT)                                         \
         {                                                                                                        \
           wait_vmcnt_lgkm0<(WAITCNT)>();                                                                         \
+          if constexpr (RAGGED && !FULL) mend_stage(kc * kStages + (S) + 1);                                               \
           __builtin_amdgcn_s_barrier();                                                                          \
           if constexpr ((S) == kStages - 1) {                                                                    \
             _Pragma("unroll") for (int fm = 0; fm < FM; ++fm) a_next[fm] = load_a_chunk_lds(a_frag_lds[fm], lane); \
@@ -663,7 +688,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
             _Pragma("unroll") for (int fm = 0; fm < FM; ++fm) a_cur[fm] = a_next[fm];                            \
           }                                                                                                      \
         }
-        auto chunk_body = [&](auto full_tag) __attribute__((always_inline)) {
+        auto chunk_body = [&](auto full_tag, int kc) __attribute__((always_inline)) {
           constexpr bool FULL = decltype(full_tag)::value;
           ONEBIT_GROUP_STAGE(0, 2 * NL, true, bv_even, av_even, bv_odd, av_odd)
           ONEBIT_GROUP_STAGE(1, 2 * NL + NA, false, bv_odd, av_odd, bv_even, av_even)
@@ -671,8 +696,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
           ONEBIT_GROUP_STAGE(3, 2 * NL, false, bv_odd, av_odd, bv_even, av_even)
         };
         int kc = chunk_begin;
-        for (; kc < full_end; ++kc) chunk_body(std::true_type{});
-        for (; kc < chunk_end; ++kc) chunk_body(std::false_type{});
+        for (; kc < full_end; ++kc) chunk_body(std::true_type{}, kc);
+        for (; kc < chunk_end; ++kc) chunk_body(std::false_type{}, kc);
 #undef ONEBIT_GROUP_STAGE
         wait_vmcnt<0>();  // drain the copies issued past the end before the LDS is released
       };
@@ -1186,13 +1211,13 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
   }
 }
 
-template <int WM, int WN, int FM, int FN, bool DMA, bool TOKENS = false, int KG = 1, bool M16 = false, bool BF16 = false>
+template <int WM, int WN, int FM, int FN, bool DMA, bool TOKENS = false, int KG = 1, bool M16 = false, bool BF16 = false, bool RAGGED = false>
 static hipError_t launch_gemm_cfg(GemmArgs args, hipStream_t stream) {
   using TS = TileShape<WM, WN, FM, FN, KG>;
   args.tiles_m = (args.m + TS::BM - 1) / TS::BM;
   args.tiles_n = (args.n + TS::BN - 1) / TS::BN;
   const int lds = DMA ? TS::LDS_BYTES : TS::STAGE_BYTES;
-  auto kern = gemm_kernel<WM, WN, FM, FN, DMA, TOKENS, KG, M16, BF16>;
+  auto kern = gemm_kernel<WM, WN, FM, FN, DMA, TOKENS, KG, M16, BF16, RAGGED>;
   // the dynamic-LDS limit is a per-device attribute of the kernel; threads that race here set the same value
   static std::atomic<bool> attr_done[64] = {};
   int device = 0;

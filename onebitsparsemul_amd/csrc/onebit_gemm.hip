@@ -109,7 +109,23 @@ hipError_t launch_split_reduce(const float* ws, int splits, size_t total, const 
 
 static hipError_t launch_gemm_pass(GemmArgs args, int tile_config, hipStream_t stream) {
   const bool aligned = (args.ldb % 8 == 0) && ((reinterpret_cast<uintptr_t>(args.b) & 15) == 0);
-  if (!aligned) return launch_gemm_cfg<4, 1, 1, 4, false>(args, stream);
+  if (!aligned) {
+    if (read_as_ragged(args.b, args.ldb)) {
+      switch (tile_config) {  // the tiles that the plan chooses
+        case kTile256x128w: return launch_gemm_cfg<2, 2, 4, 2, true, false, 1, false, false, true>(args, stream);
+        case kTile128x128s: return launch_gemm_cfg<2, 2, 2, 2, true, false, 1, false, false, true>(args, stream);
+        case kTile512x128w8: return launch_gemm_cfg<4, 2, 4, 2, true, false, 1, false, false, true>(args, stream);
+        case kTile256x128w8: return launch_gemm_cfg<4, 2, 2, 2, true, false, 1, false, false, true>(args, stream);
+        case kTile128x128w8: return launch_gemm_cfg<2, 4, 2, 1, true, false, 1, false, false, true>(args, stream);
+        case kTile64x128: return launch_gemm_cfg<2, 2, 1, 2, true, false, 1, false, false, true>(args, stream);
+        case kTile128x128k2: return launch_gemm_cfg<2, 2, 2, 2, true, false, 2, false, false, true>(args, stream);
+        case kTile64x128k2: return launch_gemm_cfg<2, 2, 1, 2, true, false, 2, false, false, true>(args, stream);
+        case kTile512x128m16: return launch_gemm_cfg<4, 1, 4, 4, true, false, 1, true, false, true>(args, stream);
+        default: break;
+      }
+    }
+    return launch_gemm_cfg<4, 1, 1, 4, false>(args, stream);
+  }
   switch (tile_config) {
     case kTile512x128: return launch_gemm_cfg<4, 1, 4, 4, true>(args, stream);
     case kTile256x128: return launch_gemm_cfg<4, 1, 2, 4, true>(args, stream);

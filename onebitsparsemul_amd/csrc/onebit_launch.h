@@ -22,10 +22,11 @@ struct GemmArgs {
   int splits;
   int chunks_per_split;
   float* split_ws;
-  // B whose rows are not 16-byte aligned (n % 8 != 0, or a base address that is not) cannot feed the asynchronous
-  // 16-byte copies. If b_pad is set (at least k * round_up(n, 8) halves, 16-byte aligned), the launcher first copies
-  // B into it with rows padded to a multiple of 8 columns and the main kernel reads that; otherwise such operands
-  // take the slower element-copy variant. ldb (elements between B rows) is filled by the launcher.
+  // B whose rows are not 16-byte aligned (n % 8 != 0, or a base address that is not): if b_pad is set (at least
+  // k * round_up(n, 8) halves, 16-byte aligned), the launcher first copies B into it with rows padded to a multiple of 8
+  // columns and the main kernel reads that; otherwise a B that may be read as a ragged one (read_as_ragged) is copied to
+  // LDS from where it lies, and what is left takes the slower element-copy variant. ldb (elements between B rows) is filled
+  // by the launcher.
   _Float16* b_pad;
   int ldb;
   // linear-layer form (launch_gemm_tokens) only: m values added to every token's row of y, may be null; its type (ElementType);
@@ -59,7 +60,7 @@ struct SkinnyArgs {
   // launch_skinny_tokens only: b is x in fp32, rounded to fp16 as it is read (bf16 = 0)
   int x_f32;
   // wide_kernel only: tokens (columns) a workgroup multiplies (at most 64); strips: the grid is walked in strips of two column
-  // groups, on a device of eight XCDs; ldb: elements between B rows in the plain form, n rounded up to eight
+  // groups, on a device of eight XCDs; ldb: elements between B rows in the plain form, n rounded up to eight or n itself
   int tokens_per_group;
   int strips;
   int ldb;
@@ -73,6 +74,12 @@ struct SkinnyGroupArgs {
   int first_block[kSkinnyMaxGroup + 1];
   int count;
 };
+
+// Whether the asynchronous copies can read a B of rows that are no whole 16-byte pieces where it lies. They take 16 bytes from any
+// address; a piece that starts at an odd multiple of two bytes costs 3.8 times as much of a compute unit's load path as one on a
+// 4-byte boundary (64 rows of 128 bytes, ldb = 64 | 66 | 68 | 65, one workgroup: 14.8 | 14.8 | 14.8 | 35.2 us). At least eight
+// values a row, so that only the last row's last piece reaches past B.
+inline bool read_as_ragged(const void* b, int n) { return n >= 8 && (reinterpret_cast<uintptr_t>(b) & 15) == 0; }
 
 enum TileConfig { kTile512x128 = 0, kTile256x128 = 1, kTile128x128 = 2, kTile256x256 = 3, kTile256x128w = 4, kTile512x128t = 5, kTile128x128s = 6, kTile256x64 = 7, kTile256x256w8 = 8, kTile512x128w8 = 9, kTile256x128w8 = 10, kTile128x128w8 = 11, kTile64x128 = 12, kTile128x128k2 = 13, kTile64x128k2 = 14, kTile512x128m16 = 15, kTileAuto = -1 };
 

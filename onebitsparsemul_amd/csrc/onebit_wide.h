@@ -53,11 +53,13 @@ struct WideShape {
 // COPIES: 1 KiB copies per image, one per eight tokens. A workgroup multiplies up to 8 COPIES tokens from first_token on.
 // TOKENS = false is the plain form, D = alpha A B + beta C, a column of B in the place of a token: B's rows start 16-byte
 // aligned (ldb % 8 == 0, first_token % 8 == 0), an image is 64 of them as they lie, COPIES 16-byte pieces each, read through
-// transpose reads; COPIES is even.
+// transpose reads; COPIES is even. RAGGED: n is no multiple of eight and the rows are read where they lie, 16 bytes from any
+// address on (ldb = n): a piece that reaches past the end of its row takes values of the next one along, which only meet columns
+// that are never stored; past the end of B it is moved back and shifted into place in LDS.
 // PARTS: the chunks that are left after whole rounds of eight, up to four of them, are dealt over the wavefronts in parts
 // of 64 or 128 K values, where otherwise some wavefronts have a chunk more and the others wait for them: 9 chunks are five
 // images in a row instead of eight, 43 are 22 instead of 24.
-template <int R, int COPIES, bool TOKENS, bool BF16, bool PARTS>
+template <int R, int COPIES, bool TOKENS, bool BF16, bool PARTS, bool RAGGED>
 __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x, const int block_y, const int first_token,
                                           char* const smem) {
   using Shape = WideShape<R, COPIES>;
@@ -130,9 +132,12 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
   const size_t k_stride = TOKENS ? 2 : (size_t)p.ldb * 2;  // bytes from one K position to the next
   const char* const x_bytes = reinterpret_cast<const char*>(p.b + (TOKENS ? (size_t)first_token * k_total : (size_t)first_token));
   const char* const zeros = reinterpret_cast<const char*>(g_zero16_wide);
+  // RAGGED: the last row's image takes the general path
+  const int k_inside = RAGGED ? k_total - 1 : k_total;
+  const char* const last_piece = reinterpret_cast<const char*>(p.b) + (size_t)k_total * p.ldb * 2 - 16;
   auto copy_image = [&](int k0, int slot) __attribute__((always_inline)) {
     const uint32_t dst = __builtin_amdgcn_readfirstlane(region_offset + slot * Shape::IMAGE_BYTES);
-    if (k0 + kWideImageK <= k_total) {  // wave-uniform
+    if (k0 + kWideImageK <= k_inside) {  // wave-uniform
 #pragma unroll
       for (int i = 0; i < COPIES; ++i) lds_dma16_base(x_bytes + k0 * k_stride, copy_off[i], dst + i * 1024);
     } else {
@@ -142,9 +147,20 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
         uint32_t off = copy_off[i];
         asm volatile("" : "+v"(off));  // keeps the 64-bit addresses out of the registers of the other path
         const int k = k0 + (TOKENS ? 8 * (piece0 ^ (4 * (i & 1))) : (64 * i + lane) / PIECES);
-        lds_dma16(k < k_total ? x_bytes + k0 * k_stride + off : zeros, dst + i * 1024);
+        const char* from = x_bytes + k0 * k_stride + off;
+        if (RAGGED && from > last_piece) from = last_piece;
+        lds_dma16(k < k_total ? from : zeros, dst + i * 1024);
       }
     }
+  };
+
+  // RAGGED: the piece that was moved back, of the last row of B, if it is in this image
+  auto mend_image = [&](int k0, int slot) __attribute__((always_inline)) {
+    const int row = k_total - 1 - k0, piece = (p.n - 1 - first_token) >> 3;
+    if (!RAGGED || row < 0 || row >= kWideImageK || piece >= PIECES) return;  // wave-uniform
+    shift_piece(region + slot * Shape::IMAGE_BYTES + ((row * PIECES + (piece ^ row_swizzle(row))) << 4), first_token + 8 * piece + 8 - p.n, lane);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
   };
 
   const int i16 = lane & 15, g16 = lane >> 4;
@@ -341,6 +357,7 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
         else wait_vmcnt<(S < 3 ? COPIES : 0)>();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (RAGGED) mend_image(kc * kChunkK + S * kWideImageK, S & 1);
         read_image(S & 1);
         if constexpr (S == (FAR ? 2 : 3)) {
           // the wait the compiler puts in front of the operand's first use counts its own loads only and so also waits for
@@ -390,12 +407,15 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
       else wait_vmcnt<0>();
       asm volatile("" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
+      const int part_k0 = part_kc * kChunkK + part_image * kWideImageK;
+      if constexpr (RAGGED) mend_image(part_k0, 0);
       read_image(0);
       compute(std::integral_constant<int, 0>{});
       if (part_images > 1) {
         wait_vmcnt<0>();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (RAGGED) mend_image(part_k0 + kWideImageK, 1);
         read_image(1);
         compute(std::integral_constant<int, 1>{});
       }
@@ -471,12 +491,12 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
 // In strips of two column groups an XCD is given a contiguous range of the list (workgroup b runs on XCD b % 8, all eight are there:
 // the launcher's condition), so that what its workgroups read of x and of the weight meets in its L2; where that pays is the host's
 // rule (wide_in_strips).
-template <int R, int COPIES, bool TOKENS, bool BF16, bool PARTS>
+template <int R, int COPIES, bool TOKENS, bool BF16, bool PARTS, bool RAGGED>
 __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_kernel(u32x8_t operands, u32x4_t results, u32x2_t shape, u32x2_t scale) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   SkinnyArgs p = unpack_args(operands, results, scale, shape[0]);
   p.tokens_per_group = operands[7] >> 24;
-  p.ldb = (p.n + 7) & ~7;  // the launcher's condition
+  p.ldb = RAGGED ? p.n : (p.n + 7) & ~7;  // the launcher's condition
   int x = blockIdx.x, group = blockIdx.z;
   if (const int groups = shape[0] >> 5; groups > 0) {
     const int row_groups = (p.m + 32 * R - 1) / (32 * R);
@@ -488,7 +508,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_kernel(u32x8_t operan
     x = pair ? w >> 1 : w;
     group = 2 * strip + (pair ? w & 1 : 0);
   }
-  wide_body<R, COPIES, TOKENS, BF16, PARTS>(p, x, blockIdx.y, group * p.tokens_per_group, smem);
+  wide_body<R, COPIES, TOKENS, BF16, PARTS, RAGGED>(p, x, blockIdx.y, group * p.tokens_per_group, smem);
 }
 
 // The dynamic-LDS limit of a kernel, a per-device attribute; threads that race here set the same value.
@@ -511,11 +531,11 @@ static hipError_t wide_lds_limit(const void* kern, int lds, std::atomic<bool> (&
 // of the kernel without parts is 1 to 4 % faster where there are none (4096 x 4096 with 48 5.2 | 5.4).
 static bool wide_has_parts(int chunks) { return chunks >= kWideWaves && chunks % kWideWaves >= 1 && chunks % kWideWaves <= 4; }
 
-template <int R, int COPIES, bool TOKENS, bool BF16, bool PARTS>
+template <int R, int COPIES, bool TOKENS, bool BF16, bool PARTS, bool RAGGED>
 static hipError_t launch_wide_parts(const SkinnyArgs& args, hipStream_t stream) {
   static std::atomic<bool> attr_done[64] = {};
   constexpr int lds = WideShape<R, COPIES>::LDS_BYTES;
-  const auto kern = wide_kernel<R, COPIES, TOKENS, BF16, PARTS>;
+  const auto kern = wide_kernel<R, COPIES, TOKENS, BF16, PARTS, RAGGED>;
   if (hipError_t st = wide_lds_limit(reinterpret_cast<const void*>(kern), lds, attr_done); st != hipSuccess) return st;
   const int rows = (args.m + 32 * R - 1) / (32 * R), groups = (args.n + args.tokens_per_group - 1) / args.tokens_per_group;
   LaunchArgs a = pack_args(args);
@@ -526,11 +546,11 @@ static hipError_t launch_wide_parts(const SkinnyArgs& args, hipStream_t stream) 
   return hipGetLastError();
 }
 
-template <int R, int COPIES, bool TOKENS, bool BF16>
+template <int R, int COPIES, bool TOKENS, bool BF16, bool RAGGED = false>
 static hipError_t launch_wide_kernel(const SkinnyArgs& args, hipStream_t stream) {
   if (wide_has_parts(args.chunks_per_split))  // of all splits but perhaps the last
-    return launch_wide_parts<R, COPIES, TOKENS, BF16, true>(args, stream);
-  return launch_wide_parts<R, COPIES, TOKENS, BF16, false>(args, stream);
+    return launch_wide_parts<R, COPIES, TOKENS, BF16, true, RAGGED>(args, stream);
+  return launch_wide_parts<R, COPIES, TOKENS, BF16, false, RAGGED>(args, stream);
 }
 
 }  // namespace onebit

@@ -10,7 +10,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_tokens_group_kernel(i
   extern __shared__ __attribute__((aligned(16))) char smem[];
   int block;
   const SkinnyArgs p = group_problem(first1, first2, first3, count, tokens, shared, table, block);
-  wide_body<R, COPIES, true, BF16, PARTS>(p, block, 0, blockIdx.y * shared.tokens_per_group, smem);
+  wide_body<R, COPIES, true, BF16, PARTS, false>(p, block, 0, blockIdx.y * shared.tokens_per_group, smem);
 }
 
 template <int R, int COPIES, bool BF16>
