@@ -34,15 +34,16 @@ constexpr int kSkinnyRegion = 8192;  // bytes of one B image
 // the image's K range of token t in 16-byte pieces, piece p stored at position p ^ token_swizzle(t) so that lanes
 // which read the same piece of consecutive tokens fall into different banks; a lane's SMFMAC operand is two plain
 // 16-byte reads (K consecutive inside a piece), no transpose. Up to sixteen tokens; more go to wide_kernel.
-// kSkinnyBRun: n = 2 or 4 with B 16-byte aligned. The 256 rows of a chunk are one run of 512 n consecutive bytes,
-// loaded in 16-byte pieces (32 n of them: at most two load instructions per wavefront and chunk, where the row-wise
-// modes issue eight; the split-K kernel's time is set by the number of load instructions it issues) and spread over the image rows
-// by LDS stores of 2 n bytes.
+// kSkinnyBTokens + l: l load instructions take an image, two tokens each. How many is known to the compiler, and none is in a branch,
+// because its waits for an earlier load count only what is requested behind it on every path.
+// kSkinnyBColumns + n: n = 2 ... 8 columns, B 16-byte aligned. Four rows of B are 8 n consecutive bytes that begin at a multiple of
+// eight: each lane loads those of four K positions, n / 2 instructions per chunk, and stores them as n columns of four K values into
+// an image that is token-major, read as such; the tiles' reduction turns them back.
 // kSkinnyBTokens32: the token-major form on fp32 activations, rounded to fp16 (nearest even) on their way into the image. One load
 // instruction takes a token's 256 K, whole lines, so there are as many as tokens. A conversion in front of the kernel costs a
 // launch and an allocation (us per layer call, conversion in front -> here: 4096 x 4096 with 1 / 16 tokens 9.2 / 9.0 -> 4.8 / 4.9,
 // 28672 x 8192 with 8 / 16 14.0 / 15.5 -> 11.8 / 14.8, 4096 x 11008 with 16 9.0 -> 8.7).
-enum SkinnyBMode { kSkinnyBFull = 0, kSkinnyBAny = 1, kSkinnyBTokens = 2, kSkinnyBRun = 3, kSkinnyBTokens32 = 4 };
+enum SkinnyBMode { kSkinnyBFull = 0, kSkinnyBAny = 1, kSkinnyBColumns = 16, kSkinnyBTokens = 32, kSkinnyBTokens32 = 48 };
 
 // The body of the split-K kernel for workgroup (block_x, block_y) of problem p: block_x = row group, block_y = K split.
 template <int NW, int R, int MODE, int NC, bool BF16 = false>
@@ -55,11 +56,14 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   constexpr int NF = NC <= 32 ? 1 : NC / 32;           // 32-column fragments per image row
   constexpr int TILE_BYTES = kRowBlock * NC * 4;       // one fp32 partial tile
   static_assert(NC == 16 || NC == 32 || NC == 64, "image width");
-  static_assert((MODE != kSkinnyBRun && MODE != kSkinnyBTokens && MODE != kSkinnyBTokens32) || NC == 16, "the run and token modes are for 16 columns");
+  static_assert(MODE == kSkinnyBFull || MODE == kSkinnyBAny || NC == 16, "the column and token modes are for 16 columns");
   // the partial tiles reuse the wavefront's image memory, RT row blocks per round of the final reduction
   constexpr int RT = R * TILE_BYTES <= kSkinnyRegion ? R : kSkinnyRegion / TILE_BYTES;
   static_assert(RT >= 1 && R % RT == 0, "the row blocks must divide into whole reduction rounds");
-  constexpr bool X32 = MODE == kSkinnyBTokens32, TOKENS = MODE == kSkinnyBTokens || X32;
+  constexpr bool X32 = MODE > kSkinnyBTokens32, TOKENS = MODE > kSkinnyBTokens;
+  constexpr int COLUMNS = MODE > kSkinnyBColumns && !TOKENS ? MODE - kSkinnyBColumns : 0;
+  static_assert(COLUMNS <= 8, "two to eight columns");
+  constexpr bool TOKEN_IMAGE = TOKENS || COLUMNS > 0;
   static_assert(!X32 || !BF16, "fp32 activations are multiplied as fp16");
   // Sixteen columns fill half of the 32x32x32 SMFMAC's result tile; v_smfmac_f32_16x16x64_f16 has no idle half and
   // multiplies a row block's chunk in half the matrix-pipe time (eight instructions of four passes).
@@ -67,6 +71,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   constexpr int PPT = IMG_ROWS / 8;                    // token-major image: 16-byte pieces per token row
   constexpr int TPI = 64 / PPT;                        // ... and tokens covered by the 64 pieces of one wavefront load
   constexpr int TOKEN_ROW_BYTES = IMG_ROWS * 2;
+  constexpr int TOKEN_LOADS = X32 ? MODE - kSkinnyBTokens32 : TOKENS ? MODE - kSkinnyBTokens : 8;
   __shared__ __attribute__((aligned(16))) char bs[NW * kSkinnyRegion];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -139,8 +144,6 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   const uint32_t token_load_step = (uint32_t)TPI * (uint32_t)k_rows * 2u;
   const uint32_t token_store_base =
       (uint32_t)token_lane * TOKEN_ROW_BYTES + (uint32_t)((piece_lane ^ token_swizzle<TOKEN_ROW_BYTES>(token_lane)) << 4);
-  // run mode: piece q = lane + 64 i of the image's run; pieces at or past 32 n are sent outside the descriptor (zero)
-  const uint32_t run_pieces = 32u * (uint32_t)n_cols;
   // fp32 activations, eight tokens from first_token on. Load i: the image's K range of one token, four values per lane; K positions
   // at or past k: outside the descriptor, as below (the launcher checks that 64 * k * 4 stays well below 2^32). Tokens 8 to 15
   // are requested when the first eight have been stored: 64 registers of loads in flight do not fit beside the rest.
@@ -148,17 +151,15 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
     const bool whole = k_base + IMG_ROWS <= k_rows;  // wave-uniform
     const bool inside = k_base + 4 * lane < k_rows;
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (first_token + i < n_cols) {
-        const uint32_t offset = meta_off + (uint32_t)(first_token + i) * (uint32_t)k_rows * 4u;
-        v[i] = buffer_load16(b_buffer, whole ? offset : inside ? offset + (uint32_t)k_base * 4u : 0xFFFFFF00u, whole ? (uint32_t)k_base * 4u : 0u);
-      } else {
-        v[i] = u32x4_t{0, 0, 0, 0};
-      }
+    for (int i = 0; i < TOKEN_LOADS; ++i) {
+      const uint32_t offset = meta_off + (uint32_t)(first_token + i) * (uint32_t)k_rows * 4u;
+      // tokens past the last: outside the descriptor, as in load_b
+      v[i] = buffer_load16(b_buffer, whole ? offset : inside ? offset + (uint32_t)k_base * 4u : 0xFFFFFF00u, whole ? (uint32_t)k_base * 4u : 0u);
+    }
   };
   auto store_b32 = [&](int first_token, const u32x4_t (&v)[8]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < TOKEN_LOADS; ++i) {
       const float4v_t f = __builtin_bit_cast(float4v_t, v[i]);
       const int token = first_token + i;
       *reinterpret_cast<u32x2_t*>(region + token * TOKEN_ROW_BYTES + (((lane >> 1) ^ token_swizzle<TOKEN_ROW_BYTES>(token)) << 4) +
@@ -166,23 +167,18 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
     }
   };
   auto load_b = [&](int k_base, u32x4_t (&v)[8]) __attribute__((always_inline)) {
-    if (MODE == kSkinnyBRun) {
-      const uint32_t run_base = (uint32_t)k_base * (uint32_t)n_cols * 2u;  // the launcher checks k n 2 < 2^32
-      if (k_base + IMG_ROWS <= k_rows) {
+    if constexpr (COLUMNS > 0) {
+      // four K positions of a lane: all of them inside K or none (k % 32 == 0); those past its end are sent outside the
+      // descriptor, which reads zeros (the launcher checks k n 2 < 2^32)
+      const uint32_t image = (uint32_t)k_base * (COLUMNS * 2), at = (uint32_t)lane * (COLUMNS * 8);
+      const bool whole = k_base + IMG_ROWS <= k_rows;  // wave-uniform
+      const uint32_t lane_at = whole ? at : k_base + 4 * lane < k_rows ? at + image : 0xFFFFFF00u, image_at = whole ? image : 0u;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-          if (64u * i < run_pieces)
-            v[i] = buffer_load16(b_buffer, lane + 64u * i < run_pieces ? meta_off + 1024u * i : 0xFFFFFF00u, run_base);
-        return;
+      for (int i = 0; i < COLUMNS / 2; ++i) v[i] = buffer_load16(b_buffer, lane_at + 16u * i, image_at);
+      if constexpr (COLUMNS % 2 != 0) {
+        const u32x2_t rest = buffer_load8(b_buffer, lane_at + 8u * (COLUMNS - 1), image_at);
+        v[COLUMNS / 2].x = rest.x; v[COLUMNS / 2].y = rest.y;
       }
-      // last image of a K that is no multiple of 256 (or an image past the end that is loaded but never multiplied):
-      // pieces inside B as they are, zeros past its end. K is a multiple of 32, so the valid bytes are a multiple of 16 n
-      // and no piece straddles the end.
-      const uint32_t valid_bytes = (uint32_t)rows_valid_of(k_base) * (uint32_t)n_cols * 2u;
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        if (64u * i < run_pieces)
-          v[i] = buffer_load16(b_buffer, meta_off + 1024u * i + 16u <= valid_bytes ? run_base + meta_off + 1024u * i : 0xFFFFFF00u, 0);
       return;
     }
     if (X32) {
@@ -190,26 +186,15 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
       return;
     }
     if (TOKENS) {
-      // offsets at or past n * k * 2 (tokens >= n) fall outside the descriptor and read as zero; K positions at or
-      // past k are sent there too (the launcher checks that 64 * k * 2 stays well below 2^32)
-      if (k_base + IMG_ROWS <= k_rows) {
-        // the image's whole K range exists (wave-uniform test): lane offsets that do not change from image to image
-        // plus a scalar offset; the range check looks at the lane offset alone, which is what sends tokens >= n to zero
-        // (load i covers tokens TPI i ... TPI i + TPI - 1: nothing to fetch past the last token)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          if (TPI * i < n_cols) v[i] = buffer_load16(b_buffer, token_load_base + i * token_load_step, (uint32_t)k_base * 2u);
-          else v[i] = u32x4_t{0, 0, 0, 0};
-        }
-        return;
-      }
+      // offsets at or past n * k * 2 (tokens >= n) fall outside the descriptor and read as zero; K positions at or past k are sent
+      // there too (the launcher checks that 64 * k * 2 stays well below 2^32). Where the image's whole K range exists, the lane
+      // offsets do not change from image to image and a scalar offset is added, which the range check does not look at.
+      const bool whole = k_base + IMG_ROWS <= k_rows;  // wave-uniform
       const bool inside = k_base + 8 * piece_lane < k_rows;
-      const uint32_t first = token_load_base + (uint32_t)k_base * 2u;
+      const uint32_t lane_at = whole ? token_load_base : token_load_base + (uint32_t)k_base * 2u, image_at = whole ? (uint32_t)k_base * 2u : 0u;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if (TPI * i < n_cols) v[i] = buffer_load16(b_buffer, inside ? first + i * token_load_step : 0xFFFFFF00u, 0);
-        else v[i] = u32x4_t{0, 0, 0, 0};
-      }
+      for (int i = 0; i < TOKEN_LOADS; ++i)
+        v[i] = buffer_load16(b_buffer, whole || inside ? lane_at + i * token_load_step : 0xFFFFFF00u, image_at);
       return;
     }
     if (MODE == kSkinnyBFull) {
@@ -264,7 +249,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   auto store_b = [&](int k_base, const u32x4_t (&v)[8]) __attribute__((always_inline)) {
     if (X32) {
       store_b32(0, v);
-      if (n_cols > 8) {
+      if (TOKEN_LOADS == 8 && n_cols > 8) {
         u32x4_t w[8];
         load_b32(k_base, 8, w);
         store_b32(8, w);
@@ -278,28 +263,23 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
           *reinterpret_cast<u32x4_t*>(region + any_store + i * any_rows * ROW_BYTES) = v[i];
       return;
     }
-    if (MODE == kSkinnyBRun) {
-      // piece q holds the n columns of rows 8 q / n ... : 2 n bytes to each row's start; columns n ... 15 keep the zeros the
-      // image was cleared to
+    if constexpr (COLUMNS > 0) {
+      auto value = [&](int row, int col) __attribute__((always_inline)) { return row * COLUMNS + col; };
+      auto pair = [&](int low, int high) __attribute__((always_inline)) {  // halves `low` and `high` of the lane's 4 n as one word
+        const uint32_t from_low = low & 1 ? 0x0302u : 0x0100u, from_high = high & 1 ? 0x07060000u : 0x05040000u;
+        return __builtin_amdgcn_perm(v[high / 8][high / 2 % 4], v[low / 8][low / 2 % 4], from_low | from_high);
+      };
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const uint32_t q = lane + 64u * i;
-        if (q >= run_pieces) continue;
-        if (n_cols == 4) {
-          *reinterpret_cast<u32x2_t*>(region + (2 * q) * ROW_BYTES) = u32x2_t{v[i].x, v[i].y};
-          *reinterpret_cast<u32x2_t*>(region + (2 * q + 1) * ROW_BYTES) = u32x2_t{v[i].z, v[i].w};
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) *reinterpret_cast<uint32_t*>(region + (4 * q + j) * ROW_BYTES) = v[i][j];
-        }
-      }
+      for (int c = 0; c < COLUMNS; ++c)
+        *reinterpret_cast<u32x2_t*>(region + c * TOKEN_ROW_BYTES + (((lane >> 1) ^ token_swizzle<TOKEN_ROW_BYTES>(c)) << 4) + (lane & 1) * 8) =
+            u32x2_t{pair(value(0, c), value(1, c)), pair(value(2, c), value(3, c))};
       return;
     }
     if (TOKENS) {
       // token = token_lane + TPI i with token_lane < TPI (a power of two): the two terms share no bits, so the swizzle of
       // piece i differs from that of piece 0 by a compile-time XOR
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < TOKEN_LOADS; ++i)
         *reinterpret_cast<u32x4_t*>(region + (token_store_base ^ (uint32_t)(token_swizzle<TOKEN_ROW_BYTES>(TPI * i) << 4)) + i * 1024) = v[i];
       return;
     }
@@ -363,7 +343,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   // B operand of instruction F = 2 P + abid
   auto frag16 = [&](int F) __attribute__((always_inline)) {
     u32x8_t raw;
-    if (TOKENS) {
+    if (TOKEN_IMAGE) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const u32x4_t t = *reinterpret_cast<const u32x4_t*>(
@@ -478,14 +458,9 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
 
   // The next image is requested while this one is multiplied. Sixteen wavefronts have 128 registers each: no room for an image
   // of 32 registers with wide columns, and with sixteen its requests crowd out the ones for the weights (4096 x 11008 with 16
-  // tokens 8.45 -> 8.9 us, with 7 columns 9.9 -> 10.3). The two requests of the run mode pay (us inside a HIP graph, weights
-  // from HBM): 4096 x 11008 with 2 / 4 columns 9.6 / 7.45 -> 9.35 / 7.35, 5120 x 13824 11.65 / 9.0 -> 11.2 / 8.6, 8192 x 8192
-  // 8.5 / 6.75 -> 8.2 / 6.75, 4096 x 4096 5.3 / 4.5 -> 5.25 / 4.4.
-  constexpr bool kPrefetchB = NW <= 8 || MODE == kSkinnyBRun;
-  if (MODE == kSkinnyBRun) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) *reinterpret_cast<u32x4_t*>(region + (lane + i * 64) * 16) = u32x4_t{0, 0, 0, 0};
-  }
+  // tokens 8.45 -> 8.9 us).
+  constexpr bool kFewLoads = (TOKENS && !X32 && TOKEN_LOADS <= 2) || COLUMNS > 0;
+  constexpr bool kPrefetchB = NW <= 8 || kFewLoads;
   u32x4_t breg[8];
   char* const d_out = reinterpret_cast<char*>(p.d) + (size_t)block_y * p.m * p.n * (p.d_f16 ? 2 : 4);
   if (short_k) {
@@ -504,9 +479,38 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
       compute(a_next, std::integral_constant<int, 0>{});
     }
   }
+  // Two or three chunks for each of sixteen wavefronts: as in the short form, everything is requested at once. What a wavefront without
+  // a last chunk requests is zeros that it does not multiply. (us, one chunk after the other | this: 4096 x 11008 with 1 / 4 tokens 6.03 |
+  // 4.97, 6.22 | 5.22; images of four loads are no faster for it, 2048 x 5120 with five tokens 3.65 | 4.11.)
+  const bool at_once = NW == 16 && kFewLoads && kc_end - kc_begin > NW && kc_end - kc_begin <= 3 * NW;
+  if constexpr (NW == 16 && kFewLoads) {
+    auto rounds_at_once = [&](auto rounds_tag) __attribute__((always_inline)) {
+      constexpr int ROUNDS = decltype(rounds_tag)::value;
+      u32x4_t b[ROUNDS][8];
+      AChunk a[ROUNDS - 1][R];
+      load_b(first * kChunkK, b[0]);
+#pragma unroll
+      for (int i = 1; i < ROUNDS; ++i) {
+        load_a(first + i * NW, a[i - 1]);
+        load_b((first + i * NW) * kChunkK, b[i]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < ROUNDS; ++i) {
+        if (i == ROUNDS - 1 && first + i * NW >= kc_end) break;  // wave-uniform
+        store_b((first + i * NW) * kChunkK, b[i]);
+        if (i == 0) compute(a_cur, std::integral_constant<int, 0>{});
+        else compute(a[i - 1], std::integral_constant<int, 0>{});
+      }
+    };
+    if (at_once) {
+      if (kc_end - kc_begin > 2 * NW) rounds_at_once(std::integral_constant<int, 3>{});
+      else rounds_at_once(std::integral_constant<int, 2>{});
+    }
+  }
   // (of sixteen wavefronts a short K leaves some without a chunk: no request for those)
-  if (kPrefetchB && !short_k && (NW <= 8 || first < kc_end)) load_b(first * kChunkK, breg);
-  for (int kc = short_k ? kc_end : first; kc < kc_end; kc += NW) {
+  if (kPrefetchB && !short_k && !at_once && (NW <= 8 || first < kc_end)) load_b(first * kChunkK, breg);
+  for (int kc = short_k || at_once ? kc_end : first; kc < kc_end; kc += NW) {
     const int k_base = kc * kChunkK;
     // this wavefront has another chunk after this one (wave-uniform): only then is the next chunk requested; a load
     // past the last chunk would be one more instruction for the memory pipeline, a third of them when a wavefront
@@ -558,7 +562,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
               const float value = acc16[round * RT + rr][h][v];
               // token-major: [token][weight row of the round], the row index XOR-swizzled by the token so that neither
               // these stores (16 tokens, one row) nor the reads below (one token, consecutive rows) collide in a bank
-              if (TOKENS) tile[i16 * ROUND_ROWS + ((rr * 32 + row) ^ i16)] = value;
+              if (TOKEN_IMAGE) tile[i16 * ROUND_ROWS + ((rr * 32 + row) ^ i16)] = value;
               else tile[(rr * 32 + row) * NC + i16] = value;
             }
       } else if (col < NC) {
@@ -576,9 +580,11 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
     }
     __syncthreads();
     const int round_row0 = rb_first * kRowBlock + round * ROUND_ROWS;
-    if (TOKENS) {
-      for (int idx = tid; idx < ROUND_ROWS * NC; idx += NT) {
-        const int local = idx % ROUND_ROWS, token = idx / ROUND_ROWS;
+    if (TOKEN_IMAGE) {
+      // (plain form: neighbouring threads take neighbouring results, and there are no others than its columns')
+      for (int idx = tid; idx < ROUND_ROWS * (COLUMNS > 0 ? COLUMNS : NC); idx += NT) {
+        const int local = COLUMNS > 0 ? idx / (COLUMNS + (COLUMNS == 0)) : idx % ROUND_ROWS;
+        const int token = COLUMNS > 0 ? idx - local * COLUMNS : idx / ROUND_ROWS;
         const int pos = token * ROUND_ROWS + (local ^ (token & 31));
         float sum = 0.f;
 #pragma unroll
@@ -586,7 +592,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
         const int row = round_row0 + local;
         if (token < p.n && row < p.m) {
           if (p.bias) sum += load_element(p.bias, p.bias_type, row);
-          const size_t o = (size_t)token * p.m + row;
+          const size_t o = COLUMNS > 0 ? (size_t)row * COLUMNS + token : (size_t)token * p.m + row;
           // a B of one column is a token-major x of one token and its result column is y: the launcher sends such calls
           // here with their alpha, beta and C (element o of C in both layouts); the linear layer passes 1, 0, null
           sum = p.alpha * sum;
@@ -721,12 +727,12 @@ __device__ __forceinline__ SkinnyArgs group_problem(int first1, int first2, int 
   return p;
 }
 
-template <int NW, int R, int NC, bool BF16>
+template <int NW, int R, int MODE, bool BF16>
 __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_group_kernel(int first1, int first2, int first3, int count,
                                                                                  int tokens, GroupShared shared, GroupTable table) {
   int block;
   const SkinnyArgs p = group_problem(first1, first2, first3, count, tokens, shared, table, block);
-  skinny_body<NW, R, kSkinnyBTokens, NC, BF16>(p, block, 0);
+  skinny_body<NW, R, MODE, 16, BF16>(p, block, 0);
 }
 
 static bool same_group_types(const SkinnyArgs& a, const SkinnyArgs& b) {
@@ -768,6 +774,23 @@ static hipError_t launch_skinny_mode(const SkinnyArgs& args, hipStream_t stream)
     hipLaunchKernelGGL((skinny_kernel<NW, R, MODE, NC, BF16>), grid, threads, 0, stream, a.operands, a.results, a.scale);
   }
   return hipGetLastError();
+}
+
+// Load instructions per image of the token-major form on 16-bit activations, of those that there are kernels for. us inside HIP
+// graphs, weights from HBM, eight conditional ones | this: 4096 x 11008 with 1 / 4 / 8 / 16 tokens 6.03 | 4.97, 6.22 | 5.22, 6.41 | 5.75,
+// 7.26 | 7.08, 4096 x 4096 3.73 | 3.29, 3.79 | 3.37, 3.94 | 3.60, 4.33 | 4.08, 11008 x 4096 5.00 | 4.89, 5.05 | 4.60, 5.25 | 4.66, 5.87 |
+// 5.58, 28672 x 8192 with 1 / 8 / 16 12.1 | 11.5, 12.5 | 12.3, 13.8 | 13.8; on fp32 activations 4096 x 4096 with 1 / 4 4.00 | 3.31, 4.12 |
+// 3.58. More loads than tokens cost their place in the load path (8192 x 8192 with 9 tokens 6.16 with six, 6.68 with eight).
+static int token_loads(int tokens) { return tokens <= 2 ? 1 : tokens <= 4 ? 2 : tokens <= 8 ? 4 : tokens <= 12 ? 6 : 8; }
+template <int NW, int R, bool BF16>
+static hipError_t launch_skinny_token_loads(const SkinnyArgs& args, hipStream_t stream) {
+  switch (token_loads(args.n)) {
+    case 1: return launch_skinny_mode<NW, R, kSkinnyBTokens + 1, 16, BF16>(args, stream);
+    case 2: return launch_skinny_mode<NW, R, kSkinnyBTokens + 2, 16, BF16>(args, stream);
+    case 4: return launch_skinny_mode<NW, R, kSkinnyBTokens + 4, 16, BF16>(args, stream);
+    case 6: return launch_skinny_mode<NW, R, kSkinnyBTokens + 6, 16, BF16>(args, stream);
+    default: return launch_skinny_mode<NW, R, kSkinnyBTokens + 8, 16, BF16>(args, stream);
+  }
 }
 
 // Fills in the K split of a split-K kernel launch: splits <= 1 = one pass straight into d.

@@ -5,12 +5,18 @@ namespace onebit {
 
 template <int NW, int R, bool BF16>
 static hipError_t launch_skinny_tokens_type(const SkinnyArgs& args, hipStream_t stream) {
-  return launch_skinny_mode<NW, R, kSkinnyBTokens, 16, BF16>(args, stream);
+  return launch_skinny_token_loads<NW, R, BF16>(args, stream);
 }
 
 template <int NW, int R>
 static hipError_t launch_skinny_tokens_cfg(const SkinnyArgs& args, hipStream_t stream) {
-  if (args.x_f32) return launch_skinny_mode<NW, R, kSkinnyBTokens32, 16>(args, stream);
+  if (args.x_f32) {  // one token per load instruction, eight at once
+    if (args.n == 1) return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 1, 16>(args, stream);
+    if (args.n == 2) return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 2, 16>(args, stream);
+    if (args.n <= 4) return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 4, 16>(args, stream);
+    if (args.n <= 6) return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 6, 16>(args, stream);
+    return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 8, 16>(args, stream);
+  }
   return args.bf16 ? launch_skinny_tokens_type<NW, R, true>(args, stream) : launch_skinny_tokens_type<NW, R, false>(args, stream);
 }
 
@@ -33,13 +39,24 @@ hipError_t launch_skinny_tokens(SkinnyArgs args, int rows_per_group, hipStream_t
                              args.d_f16 && args.bf16 ? kBF16 : args.d_f16, args.bias, args.bias_type, args.m, stream);
 }
 
-template <int NW, int R, bool BF16>
-static hipError_t launch_skinny_group_type(const SkinnyGroupArgs& g, int blocks, hipStream_t stream) {
+template <int NW, int R, int MODE, bool BF16>
+static hipError_t launch_skinny_group_mode(const SkinnyGroupArgs& g, int blocks, hipStream_t stream) {
   const dim3 grid(blocks), threads(64 * NW);
   const GroupLaunch l = group_launch(g);
-  hipLaunchKernelGGL((skinny_group_kernel<NW, R, 16, BF16>), grid, threads, 0, stream, l.first[1], l.first[2], l.first[3], g.count,
+  hipLaunchKernelGGL((skinny_group_kernel<NW, R, MODE, BF16>), grid, threads, 0, stream, l.first[1], l.first[2], l.first[3], g.count,
                      g.problem[0].n, l.shared, l.table);
   return hipGetLastError();
+}
+
+template <int NW, int R, bool BF16>
+static hipError_t launch_skinny_group_type(const SkinnyGroupArgs& g, int blocks, hipStream_t stream) {
+  switch (token_loads(g.problem[0].n)) {
+    case 1: return launch_skinny_group_mode<NW, R, kSkinnyBTokens + 1, BF16>(g, blocks, stream);
+    case 2: return launch_skinny_group_mode<NW, R, kSkinnyBTokens + 2, BF16>(g, blocks, stream);
+    case 4: return launch_skinny_group_mode<NW, R, kSkinnyBTokens + 4, BF16>(g, blocks, stream);
+    case 6: return launch_skinny_group_mode<NW, R, kSkinnyBTokens + 6, BF16>(g, blocks, stream);
+    default: return launch_skinny_group_mode<NW, R, kSkinnyBTokens + 8, BF16>(g, blocks, stream);
+  }
 }
 
 template <int NW, int R>
