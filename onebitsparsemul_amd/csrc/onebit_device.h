@@ -141,9 +141,12 @@ __device__ __forceinline__ half8_t expand_signs(const AChunk& a, uint32_t packed
 // allocation mixes the two register files and then copies whole accumulator tiles between them behind the SMFMAC
 // that produced them, which serialises the matrix pipe. Consecutive SMFMACs never share an accumulator, so no
 // wait states are needed between them.
-template <int STEP, bool PINNED = true, bool BF16 = false>
+// A vector instruction's result may be an operand of an SMFMAC two instructions later at the earliest, which the compiler does not know of
+// inline assembly: SETTLE puts the wait states in front, for the first SMFMAC behind a loop's register copies.
+template <int STEP, bool PINNED = true, bool BF16 = false, bool SETTLE = false>
 __device__ __forceinline__ float16_t smfmac_step(const AChunk& a, half8_t av, half16_t bv, float16_t acc) {
   const int idx = (int)a.meta[STEP / 2];
+  if constexpr (PINNED && SETTLE) asm volatile("s_nop 1" : "+v"(av), "+v"(bv) : "v"(idx));
   // Kernels whose consecutive SMFMACs update the same accumulator use the builtin, so that the compiler inserts
   // the wait states that dependency needs.
   if constexpr (!PINNED && BF16)

@@ -55,25 +55,30 @@ struct TileShape {
 // four-wavefront tiles with two workgroups per CU; 32 for the tiles with one per CU), which then form one block: every B column
 // panel it streams is shared by GROUP_M workgroups and every A row panel by 4 in that XCD's L2, and the whole
 // range of one XCD covers few column strips, so B is fetched into few L2s.
+// strip_reciprocal = 2^32 / (4 tiles_m) + 1. The other two quotients are of a divisor from 1 to 4 and below 4: no division in front of the
+// first copy (measured at GemmResult).
+constexpr int kStripTiles = 4;
 template <int GROUP_M>
-__device__ __forceinline__ void tile_of_block(int b, int tiles_m, int tiles_n, int xcds, int& tm, int& tn) {
+__device__ __forceinline__ void tile_of_block(int b, int tiles_m, int tiles_n, int xcds, uint32_t strip_reciprocal, int& tm, int& tn) {
+  static_assert(GROUP_M == 8 || GROUP_M == 16, "a power of two");
   const int total = tiles_m * tiles_n;
   int per, rem, x, local;
   if (xcds == 8) {  // the usual case with constant divisors
-    per = total / 8, rem = total % 8, x = b % 8, local = b / 8;
+    per = total >> 3, rem = total & 7, x = b & 7, local = b >> 3;
   } else {
     per = total / xcds, rem = total % xcds, x = b % xcds, local = b / xcds;
   }
   const int v = x * per + (x < rem ? x : rem) + local;
-  constexpr int STRIP_N = 4;
-  const int strip = v / (tiles_m * STRIP_N);
-  const int strip_w = (tiles_n - strip * STRIP_N) < STRIP_N ? (tiles_n - strip * STRIP_N) : STRIP_N;
-  const int w = v - strip * STRIP_N * tiles_m;
-  const int group = w / (GROUP_M * strip_w);
+  int strip = (int)__umulhi((uint32_t)v, strip_reciprocal), w = v - strip * kStripTiles * tiles_m;
+  if (w < 0) --strip, w += kStripTiles * tiles_m;  // the reciprocal is rounded up
+  const int strip_w = (tiles_n - strip * kStripTiles) < kStripTiles ? (tiles_n - strip * kStripTiles) : kStripTiles;
+  const uint32_t rows = (uint32_t)w / GROUP_M;  // of tiles, in units of a group's height
+  const int group = strip_w == 4 ? rows >> 2 : strip_w == 3 ? rows / 3 : strip_w == 2 ? rows >> 1 : rows;
   const int group_h = (tiles_m - group * GROUP_M) < GROUP_M ? (tiles_m - group * GROUP_M) : GROUP_M;
   const int u = w - group * GROUP_M * strip_w;
-  tm = group * GROUP_M + u % group_h;
-  tn = strip * STRIP_N + u / group_h;
+  const int column = (u >= group_h) + (u >= 2 * group_h) + (u >= 3 * group_h);
+  tm = group * GROUP_M + u - column * group_h;
+  tn = strip * kStripTiles + column;
 }
 
 // One stage (64 K = two SMFMAC K steps) of a wavefront's FM x FN tile.
@@ -154,14 +159,29 @@ __device__ __forceinline__ void mfma_frags_fused(const AChunk (&a)[FM], const u3
 #pragma unroll
     for (int fn = 0; fn < FN; ++fn) {
       __builtin_amdgcn_s_setprio(1);  // the wavefront that is about to issue an SMFMAC wins the arbitration on its SIMD
-      acc[fm][fn] = smfmac_step<STEP, PINNED, BF16>(a[fm], __builtin_bit_cast(half8_t, av[fm]),
-                                              __builtin_bit_cast(half16_t, bv[fn]), acc[fm][fn]);
+      const half8_t a8 = __builtin_bit_cast(half8_t, av[fm]);
+      const half16_t b16 = __builtin_bit_cast(half16_t, bv[fn]);
+      acc[fm][fn] = fm == 0 && fn == 0 ? smfmac_step<STEP, PINNED, BF16, true>(a[fm], a8, b16, acc[fm][fn])
+                                       : smfmac_step<STEP, PINNED, BF16>(a[fm], a8, b16, acc[fm][fn]);
       __builtin_amdgcn_s_setprio(0);
       __builtin_amdgcn_sched_barrier(0);
       fetch(fm * FN + fn);
       __builtin_amdgcn_sched_barrier(0);
     }
 }
+
+// us inside HIP graphs, arguments as one struct and three divisions by run-time values in front of the first copy | this: 512^3 5.12 |
+// 4.78, 1024^3 7.11 | 6.47, 2048^3 15.2 | 14.8, 11008 x 256 x 4096 20.8 | 20.0, 640 x 816 x 576 7.64 | 7.08, 4096^3 62.6 | 61.6; large
+// products within 1 %.
+// A launch's arguments: eight dwords of operands (prep, b; m, n, k, ldb), four of the grid (tiles_m, tiles_n, reciprocal of a strip,
+// chunks_per_split with the XCDs from bit 24 on) and what the epilogue takes.
+struct GemmResult {
+  void* d;
+  const void* c;
+  const void* bias;
+  float alpha, beta;
+  int c_f16, d_f16, bias_type;
+};
 
 // Source of zeros for the asynchronous copies of B rows at or past K.
 static __device__ __attribute__((aligned(16))) uint32_t g_zero16[4] = {0, 0, 0, 0};
@@ -173,7 +193,7 @@ static __device__ __attribute__((aligned(16))) uint32_t g_zero16[4] = {0, 0, 0, 
 // end of B it is moved back and shifted into place in LDS (mend_stage). An instantiation of its own: the tests for that row made
 // a product of few chunks slower (2048 x 512 x 512 5.25 -> 5.64 us).
 template <int WM, int WN, int FM, int FN, bool DMA, bool TOKENS = false, int KG = 1, bool M16 = false, bool BF16 = false, bool RAGGED = false>
-__global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gemm_kernel(GemmArgs p) {
+__global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gemm_kernel(u32x8_t operands, u32x4_t tiles, GemmResult result) {
   static_assert(!M16 || (DMA && KG == 1 && WN == 1 && FM == 4 && FN == 4), "the 16x16x64 form exists for the 512x128 four-wavefront tile");
   static_assert(TOKENS || !BF16, "bf16 activations exist for the token-major form");
   static_assert(DMA || !TOKENS, "the token-major form uses the asynchronous copies");
@@ -183,6 +203,15 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
   constexpr int BM = TS::BM, BN = TS::BN, CH = TS::CH, NL = TS::NL, NW = TS::NW;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
+  // What the first copies need is in scalar registers when a wavefront starts (see LaunchArgs); the rest is loaded under them.
+  GemmArgs p{};
+  p.prep = reinterpret_cast<const uint8_t*>((uint64_t)operands[1] << 32 | operands[0]);
+  p.b = reinterpret_cast<const _Float16*>((uint64_t)operands[3] << 32 | operands[2]);
+  p.m = operands[4]; p.n = operands[5]; p.k = operands[6]; p.ldb = operands[7];
+  p.kc_total = (p.k + kChunkK - 1) / kChunkK;
+  p.tiles_m = tiles[0]; p.tiles_n = tiles[1]; p.chunks_per_split = tiles[3] & 0xFFFFFFu; p.xcds = tiles[3] >> 24;
+  p.d = result.d; p.c = result.c; p.alpha = result.alpha; p.beta = result.beta; p.c_f16 = result.c_f16; p.d_f16 = result.d_f16;
+  p.bias = result.bias; p.bias_type = result.bias_type;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, kept in a scalar register
   const int kg = KG == 2 ? wave / (WM * WN) : 0;   // K group of this wavefront
@@ -190,7 +219,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
   const int wm = wave_in_group / WN, wn = wave_in_group % WN;
   int tile_m, tile_n;
   // one workgroup per compute unit (eight wavefronts, or four that use all the registers): 32 resident on an XCD
-  tile_of_block<(NW == 8 || FM * FN > 8 ? 8 : 16)>(blockIdx.x, p.tiles_m, p.tiles_n, p.xcds, tile_m, tile_n);
+  tile_of_block<(NW == 8 || FM * FN > 8 ? 8 : 16)>(blockIdx.x, p.tiles_m, p.tiles_n, p.xcds, tiles[2], tile_m, tile_n);
   const int row0 = tile_m * BM + wm * FM * 32;  // first row of this wavefront
   const int n0 = tile_n * BN;                   // first column of the workgroup
   const int col0 = n0 + wn * FN * 32;           // first column of this wavefront
@@ -308,7 +337,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
           uint32_t off = b_off[i];
-          if constexpr (RAGGED) asm volatile("" : "+v"(off));  // keeps the 64-bit addresses out of the registers of the other path
+          asm volatile("" : "+v"(off));  // keeps the 64-bit addresses out of the registers of the other path
           const char* src = b_stage + off;
           if (RAGGED && src > last_piece) src = last_piece;
           if (next_k0 + copy_row[i] >= p.k) src = zeros;
@@ -494,6 +523,11 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
         else asm("v_smfmac_f32_16x16x64_f16 %0, %1, %2, %3 abid:1" : "+a"(c) : "v"(a8), "v"(b16), "v"(idx));
       };
 
+      // wait states behind what a loop copies between registers, see smfmac_step
+      auto settle16 = [&](u32x4_t& av, u32x8_t& bv, const ATile& t) __attribute__((always_inline)) {
+        asm volatile("s_nop 1" : "+v"(av), "+v"(bv) : "v"(t.idx01));
+      };
+
       issue_a();
 #pragma unroll
       for (int s = 0; s < kStages; ++s) issue_b(s);
@@ -524,6 +558,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, (FM * FN <= 8 ? 2 : 1)) void gem
           for (int rt = 0; rt < RT / 2; ++rt)
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) {
+              if (S == 0 && rt == 0 && ct == 0) settle16(av_roll[0], bv[0], a_cur[0]);
               mma16(acc16[rt][ct], av_roll[rt & 1], bv[ct], a_cur[rt], S);
               __builtin_amdgcn_sched_barrier(0);
               // this slot's share of the eight registers to expand: the next row tile's four, then row tile 4 + rt's four
@@ -1240,7 +1275,14 @@ static hipError_t launch_gemm_cfg(GemmArgs args, hipStream_t stream) {
     xcds_of[device].store(xcds, std::memory_order_relaxed);
   }
   args.xcds = xcds;
-  hipLaunchKernelGGL(kern, dim3(args.tiles_m * args.tiles_n, args.splits), dim3(64 * TS::NW), lds, stream, args);
+  const uint64_t prep = (uint64_t)args.prep, b = (uint64_t)args.b;
+  const u32x8_t operands = {(uint32_t)prep, (uint32_t)(prep >> 32), (uint32_t)b, (uint32_t)(b >> 32), (uint32_t)args.m, (uint32_t)args.n,
+                            (uint32_t)args.k, (uint32_t)args.ldb};
+  const u32x4_t tiles = {(uint32_t)args.tiles_m, (uint32_t)args.tiles_n,
+                         (uint32_t)((uint64_t(1) << 32) / ((uint64_t)kStripTiles * args.tiles_m) + 1),
+                         (uint32_t)args.chunks_per_split | (uint32_t)args.xcds << 24};  // (chunks of 256 of an int K: 23 bits)
+  const GemmResult result{args.d, args.c, args.bias, args.alpha, args.beta, args.c_f16, args.d_f16, args.bias_type};
+  hipLaunchKernelGGL(kern, dim3(args.tiles_m * args.tiles_n, args.splits), dim3(64 * TS::NW), lds, stream, operands, tiles, result);
   return hipGetLastError();
 }
 
