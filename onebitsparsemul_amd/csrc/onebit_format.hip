@@ -375,28 +375,26 @@ hipError_t launch_prepare(const void* a, const void* e, void* prep, int m, int k
   const dim3 grid(kc_total * kPrepareStrip * ((m / 64 + kStripPairs - 1) / kStripPairs));
   // the dword form of the metadata loads needs e on a 4-byte boundary
   const auto kernel = layout == 0 && (reinterpret_cast<uintptr_t>(e) & 3) == 0 ? prepare_kernel<true> : prepare_kernel<false>;
-  hipLaunchKernelGGL(kernel, grid, dim3(64 * kPreparePairs), 0, stream, (const uint8_t*)a, (const uint16_t*)e,
-                     (uint8_t*)prep, m, k, kc_total, layout);
-  return hipGetLastError();
+  return launch_kernel(kernel, grid, dim3(64 * kPreparePairs), 0, stream, (const uint8_t*)a, (const uint16_t*)e, (uint8_t*)prep, m, k,
+                       kc_total, layout);
 }
 
 template <int DTYPE>
-static void launch_pack_type(const void* w, void* a, void* e, int m, int k, int prune, int layout, hipStream_t stream) {
+static hipError_t launch_pack_type(const void* w, void* a, void* e, int m, int k, int prune, int layout, hipStream_t stream) {
   const int k_tiles = (k / 16 + 3) / 4;
   constexpr int kStripTiles = kPackTiles * kPackStrip;
   const dim3 grid(k_tiles * kPackStrip * ((m / 64 + kStripTiles - 1) / kStripTiles));
-  hipLaunchKernelGGL(pack_kernel<DTYPE>, grid, dim3(64 * kPackTiles), 0, stream,
-                     (const typename PackType<DTYPE>::type*)w, (uint8_t*)a, (uint16_t*)e, m, k, prune, layout, k_tiles);
+  return launch_kernel(pack_kernel<DTYPE>, grid, dim3(64 * kPackTiles), 0, stream, (const typename PackType<DTYPE>::type*)w, (uint8_t*)a,
+                       (uint16_t*)e, m, k, prune, layout, k_tiles);
 }
 
 hipError_t launch_pack(const void* w, int dtype, void* a, void* e, int m, int k, int prune, int layout, hipStream_t stream) {
   switch (dtype) {
-    case kPackF32: launch_pack_type<kPackF32>(w, a, e, m, k, prune, layout, stream); break;
-    case kPackF16: launch_pack_type<kPackF16>(w, a, e, m, k, prune, layout, stream); break;
-    case kPackBF16: launch_pack_type<kPackBF16>(w, a, e, m, k, prune, layout, stream); break;
+    case kPackF32: return launch_pack_type<kPackF32>(w, a, e, m, k, prune, layout, stream);
+    case kPackF16: return launch_pack_type<kPackF16>(w, a, e, m, k, prune, layout, stream);
+    case kPackBF16: return launch_pack_type<kPackBF16>(w, a, e, m, k, prune, layout, stream);
     default: return hipErrorInvalidValue;
   }
-  return hipGetLastError();
 }
 
 }  // namespace onebit

@@ -1282,8 +1282,7 @@ static hipError_t launch_gemm_cfg(GemmArgs args, hipStream_t stream) {
                          (uint32_t)((uint64_t(1) << 32) / ((uint64_t)kStripTiles * args.tiles_m) + 1),
                          (uint32_t)args.chunks_per_split | (uint32_t)args.xcds << 24};  // (chunks of 256 of an int K: 23 bits)
   const GemmResult result{args.d, args.c, args.bias, args.alpha, args.beta, args.c_f16, args.d_f16, args.bias_type};
-  hipLaunchKernelGGL(kern, dim3(args.tiles_m * args.tiles_n, args.splits), dim3(64 * TS::NW), lds, stream, operands, tiles, result);
-  return hipGetLastError();
+  return launch_kernel(kern, dim3(args.tiles_m * args.tiles_n, args.splits), dim3(64 * TS::NW), lds, stream, operands, tiles, result);
 }
 
 }  // namespace onebit

@@ -99,12 +99,10 @@ hipError_t launch_split_reduce(const float* ws, int splits, size_t total, const 
   const bool vec = total % 4 == 0 && (reinterpret_cast<uintptr_t>(d) & 15) == 0 &&
                    (beta == 0.f || (reinterpret_cast<uintptr_t>(c) & 15) == 0) && (!bias || row_length % 4 == 0);
   if (vec)
-    hipLaunchKernelGGL(splitk_reduce_kernel<4>, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream, ws,
-                       splits, total, c, d, total, alpha, beta, c_f16, d_type, bias, bias_type, row_length);
-  else
-    hipLaunchKernelGGL(splitk_reduce_kernel<1>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, ws,
-                       splits, total, c, d, total, alpha, beta, c_f16, d_type, bias, bias_type, row_length);
-  return hipGetLastError();
+    return launch_kernel(splitk_reduce_kernel<4>, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream, ws, splits, total, c, d,
+                         total, alpha, beta, c_f16, d_type, bias, bias_type, row_length);
+  return launch_kernel(splitk_reduce_kernel<1>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, ws, splits, total, c, d, total,
+                       alpha, beta, c_f16, d_type, bias, bias_type, row_length);
 }
 
 static hipError_t launch_gemm_pass(GemmArgs args, int tile_config, hipStream_t stream) {
@@ -149,9 +147,8 @@ static hipError_t launch_gemm_pass(GemmArgs args, int tile_config, hipStream_t s
 
 hipError_t launch_pad_b(const _Float16* b, _Float16* dst, int k, int n, hipStream_t stream) {
   const int per_row = (n + 7) / 8, rows = per_row > 1 && per_row < kPadPieces ? kPadPieces / per_row : 1;
-  hipLaunchKernelGGL(pad_b_kernel, dim3((k + rows - 1) / rows, (per_row + kPadPieces - 1) / kPadPieces), dim3(256), 0, stream, b,
-                     dst, k, n, 8 * per_row, rows, (uint32_t)((uint64_t(1) << 32) / per_row + 1));
-  return hipGetLastError();
+  return launch_kernel(pad_b_kernel, dim3((k + rows - 1) / rows, (per_row + kPadPieces - 1) / kPadPieces), dim3(256), 0, stream, b, dst, k, n,
+                       8 * per_row, rows, (uint32_t)((uint64_t(1) << 32) / per_row + 1));
 }
 
 hipError_t launch_gemm(GemmArgs args, int tile_config, hipStream_t stream) {

@@ -699,9 +699,17 @@ struct GroupProblem {
   const void* bias;
   int m, k;
 };
+// Up to MOST problems. The host pays for the bytes of a launch's arguments (64 | 192 | 384 | 720 bytes: 2.5 | 3.0 | 3.4 | 3.5 us), so
+// there are kernels for up to four, whose first workgroups are arguments of their own.
+template <int MOST>
 struct GroupTable {
-  GroupProblem problem[kSkinnyMaxGroup];
-  int first_block[kSkinnyMaxGroup];
+  GroupProblem problem[MOST];
+  int first_block[MOST];
+};
+constexpr int kGroupFew = 4;
+template <>
+struct GroupTable<kGroupFew> {
+  GroupProblem problem[kGroupFew];
 };
 struct GroupShared {  // the same for all problems (same_group_types)
   int d_f16, bias_type, tokens_per_group;
@@ -709,13 +717,15 @@ struct GroupShared {  // the same for all problems (same_group_types)
 
 // First workgroups of problems 1, 2 and 3 (INT_MAX where there is none), the number of problems, the token count; `problem`: of
 // this workgroup, `block`: its number among that problem's.
+template <int MOST>
 __device__ __forceinline__ SkinnyArgs group_problem(int first1, int first2, int first3, int count, int tokens, const GroupShared& shared,
-                                                    const GroupTable& table, int& block) {
+                                                    const GroupTable<MOST>& table, int& block) {
   block = blockIdx.x;
   int which = (block >= first1) + (block >= first2) + (block >= first3);
   int first = block >= first3 ? first3 : block >= first2 ? first2 : block >= first1 ? first1 : 0;
-  for (int i = 4; i < count; ++i)
-    if (block >= table.first_block[i]) which = i, first = table.first_block[i];
+  if constexpr (MOST > kGroupFew)
+    for (int i = kGroupFew; i < count; ++i)
+      if (block >= table.first_block[i]) which = i, first = table.first_block[i];
   const GroupProblem& q = table.problem[which];
   SkinnyArgs p{};
   p.prep = q.prep; p.b = q.b; p.d = q.d; p.bias = q.bias;
@@ -727,9 +737,9 @@ __device__ __forceinline__ SkinnyArgs group_problem(int first1, int first2, int 
   return p;
 }
 
-template <int NW, int R, int MODE, bool BF16>
+template <int NW, int R, int MODE, bool BF16, int MOST>
 __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void skinny_group_kernel(int first1, int first2, int first3, int count,
-                                                                                 int tokens, GroupShared shared, GroupTable table) {
+                                                                                 int tokens, GroupShared shared, GroupTable<MOST> table) {
   int block;
   const SkinnyArgs p = group_problem(first1, first2, first3, count, tokens, shared, table, block);
   skinny_body<NW, R, MODE, 16, BF16>(p, block, 0);
@@ -740,19 +750,21 @@ static bool same_group_types(const SkinnyArgs& a, const SkinnyArgs& b) {
 }
 
 // The arguments of a grouped launch from the launcher's (first_block filled in).
+template <int MOST>
 struct GroupLaunch {
   int first[4];
   GroupShared shared;
-  GroupTable table;
+  GroupTable<MOST> table;
 };
-static GroupLaunch group_launch(const SkinnyGroupArgs& g) {
-  GroupLaunch l{};
+template <int MOST>
+static GroupLaunch<MOST> group_launch(const SkinnyGroupArgs& g) {
+  GroupLaunch<MOST> l{};
   for (int i = 0; i < 4; ++i) l.first[i] = i < g.count ? g.first_block[i] : INT_MAX;
   l.shared = GroupShared{g.problem[0].d_f16, g.problem[0].bias_type, g.problem[0].tokens_per_group};
   for (int i = 0; i < g.count; ++i) {
     const SkinnyArgs& p = g.problem[i];
     l.table.problem[i] = GroupProblem{p.prep, p.b, p.d, p.bias, p.m, p.k};
-    l.table.first_block[i] = g.first_block[i];
+    if constexpr (MOST > kGroupFew) l.table.first_block[i] = g.first_block[i];
   }
   return l;
 }
@@ -763,17 +775,15 @@ static hipError_t launch_skinny_mode(const SkinnyArgs& args, hipStream_t stream)
   constexpr bool kPieces = MODE == kSkinnyBAny;
   if constexpr (kPieces && (NC > 16 || NW <= 8)) {  // see skinny_struct_kernel
     const bool words = R == 2 && args.n >= 10 && args.n <= 14 && args.n % 2 == 0 && (reinterpret_cast<uintptr_t>(args.b) & 3) == 0;
-    if (NC > 16 || (args.chunks_per_split > (R == 2 ? NW : 0) && (words || args.chunks_per_split <= 2 * NW))) {
-      hipLaunchKernelGGL((skinny_struct_kernel<NW, R, MODE, NC, BF16>), grid, threads, 0, stream, args);
-      return hipGetLastError();
-    }
+    if (NC > 16 || (args.chunks_per_split > (R == 2 ? NW : 0) && (words || args.chunks_per_split <= 2 * NW)))
+      return launch_kernel(skinny_struct_kernel<NW, R, MODE, NC, BF16>, grid, threads, 0, stream, args);
   }
   if constexpr (!kPieces || NC == 16) {
     LaunchArgs a = pack_args(args);
     a.operands[7] |= a.flags << 24;
-    hipLaunchKernelGGL((skinny_kernel<NW, R, MODE, NC, BF16>), grid, threads, 0, stream, a.operands, a.results, a.scale);
+    return launch_kernel(skinny_kernel<NW, R, MODE, NC, BF16>, grid, threads, 0, stream, a.operands, a.results, a.scale);
   }
-  return hipGetLastError();
+  return hipErrorInvalidValue;  // not reached: wide images of pieces went the other way
 }
 
 // Load instructions per image of the token-major form on 16-bit activations, of those that there are kernels for. us inside HIP

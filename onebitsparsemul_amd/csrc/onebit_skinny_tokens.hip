@@ -39,13 +39,17 @@ hipError_t launch_skinny_tokens(SkinnyArgs args, int rows_per_group, hipStream_t
                              args.d_f16 && args.bf16 ? kBF16 : args.d_f16, args.bias, args.bias_type, args.m, stream);
 }
 
+template <int NW, int R, int MODE, bool BF16, int MOST>
+static hipError_t launch_skinny_group_most(const SkinnyGroupArgs& g, int blocks, hipStream_t stream) {
+  const dim3 grid(blocks), threads(64 * NW);
+  const auto l = group_launch<MOST>(g);
+  return launch_kernel(skinny_group_kernel<NW, R, MODE, BF16, MOST>, grid, threads, 0, stream, l.first[1], l.first[2], l.first[3], g.count,
+                       g.problem[0].n, l.shared, l.table);
+}
 template <int NW, int R, int MODE, bool BF16>
 static hipError_t launch_skinny_group_mode(const SkinnyGroupArgs& g, int blocks, hipStream_t stream) {
-  const dim3 grid(blocks), threads(64 * NW);
-  const GroupLaunch l = group_launch(g);
-  hipLaunchKernelGGL((skinny_group_kernel<NW, R, MODE, BF16>), grid, threads, 0, stream, l.first[1], l.first[2], l.first[3], g.count,
-                     g.problem[0].n, l.shared, l.table);
-  return hipGetLastError();
+  return g.count <= kGroupFew ? launch_skinny_group_most<NW, R, MODE, BF16, kGroupFew>(g, blocks, stream)
+                              : launch_skinny_group_most<NW, R, MODE, BF16, kSkinnyMaxGroup>(g, blocks, stream);
 }
 
 template <int NW, int R, bool BF16>

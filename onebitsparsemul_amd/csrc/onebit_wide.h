@@ -542,8 +542,7 @@ static hipError_t launch_wide_parts(const SkinnyArgs& args, hipStream_t stream) 
   a.operands[7] |= (uint32_t)args.tokens_per_group << 24;
   const u32x2_t shape = {a.flags | (args.strips ? (uint32_t)groups << 5 : 0u), (uint32_t)((uint64_t(1) << 32) / (2 * rows) + 1)};
   const dim3 grid = args.strips ? dim3(rows * groups, args.splits) : dim3(rows, args.splits, groups);
-  hipLaunchKernelGGL(kern, grid, dim3(64 * kWideWaves), lds, stream, a.operands, a.results, shape, a.scale);
-  return hipGetLastError();
+  return launch_kernel(kern, grid, dim3(64 * kWideWaves), lds, stream, a.operands, a.results, shape, a.scale);
 }
 
 template <int R, int COPIES, bool TOKENS, bool BF16, bool RAGGED = false>

@@ -4,9 +4,9 @@
 namespace onebit {
 
 // Several products that share the token count, workgroups numbered over their row groups as in skinny_group_kernel.
-template <int R, int COPIES, bool BF16, bool PARTS>
+template <int R, int COPIES, bool BF16, bool PARTS, int MOST>
 __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_tokens_group_kernel(int first1, int first2, int first3, int count, int tokens,
-                                                                               GroupShared shared, GroupTable table) {
+                                                                               GroupShared shared, GroupTable<MOST> table) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   int block;
   const SkinnyArgs p = group_problem(first1, first2, first3, count, tokens, shared, table, block);
@@ -17,23 +17,24 @@ template <int R, int COPIES, bool BF16>
 static hipError_t launch_wide_one(const SkinnyArgs& args, int, hipStream_t stream) {
   return launch_wide_kernel<R, COPIES, true, BF16>(args, stream);
 }
-template <int R, int COPIES, bool BF16, bool PARTS>
+template <int R, int COPIES, bool BF16, bool PARTS, int MOST>
 static hipError_t launch_wide_group(const SkinnyGroupArgs& g, int blocks, hipStream_t stream) {
   static std::atomic<bool> attr_done[64] = {};
   constexpr int lds = WideShape<R, COPIES>::LDS_BYTES;
-  const auto kern = wide_tokens_group_kernel<R, COPIES, BF16, PARTS>;
+  const auto kern = wide_tokens_group_kernel<R, COPIES, BF16, PARTS, MOST>;
   if (hipError_t st = wide_lds_limit(reinterpret_cast<const void*>(kern), lds, attr_done); st != hipSuccess) return st;
   const int n = g.problem[0].n, tokens = g.problem[0].tokens_per_group;
-  const GroupLaunch l = group_launch(g);
-  hipLaunchKernelGGL(kern, dim3(blocks, (n + tokens - 1) / tokens), dim3(64 * kWideWaves), lds, stream, l.first[1], l.first[2],
-                     l.first[3], g.count, n, l.shared, l.table);
-  return hipGetLastError();
+  const auto l = group_launch<MOST>(g);
+  return launch_kernel(kern, dim3(blocks, (n + tokens - 1) / tokens), dim3(64 * kWideWaves), lds, stream, l.first[1], l.first[2], l.first[3],
+                       g.count, n, l.shared, l.table);
 }
 template <int R, int COPIES, bool BF16>
 static hipError_t launch_wide_one(const SkinnyGroupArgs& g, int blocks, hipStream_t stream) {
+  // more than four: the rare call that is not worth a build without parts
+  if (g.count > kGroupFew) return launch_wide_group<R, COPIES, BF16, true, kSkinnyMaxGroup>(g, blocks, stream);
   for (int i = 0; i < g.count; ++i)
-    if (wide_has_parts(g.problem[i].kc_total)) return launch_wide_group<R, COPIES, BF16, true>(g, blocks, stream);
-  return launch_wide_group<R, COPIES, BF16, false>(g, blocks, stream);
+    if (wide_has_parts(g.problem[i].kc_total)) return launch_wide_group<R, COPIES, BF16, true, kGroupFew>(g, blocks, stream);
+  return launch_wide_group<R, COPIES, BF16, false, kGroupFew>(g, blocks, stream);
 }
 
 // One instantiation per copy, not per pair of copies (a column tile of sixteen tokens): the eight tokens that an odd count leaves
