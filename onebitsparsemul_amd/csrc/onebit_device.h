@@ -104,6 +104,13 @@ __device__ __forceinline__ float load_element(const void* p, int type, size_t at
   const uint16_t bits = reinterpret_cast<const uint16_t*>(p)[at];
   return type == kF16 ? (float)__builtin_bit_cast(_Float16, bits) : __builtin_bit_cast(float, (uint32_t)bits << 16);
 }
+// Four consecutive elements from `at` on as they lie, one load (16-bit types: the first two words), and their values.
+__device__ __forceinline__ u32x4_t load_four(const void* p, int type, size_t at) {
+  if (type == kF32) return *reinterpret_cast<const u32x4_any_t*>(reinterpret_cast<const float*>(p) + at);
+  const u32x2_t v = *reinterpret_cast<const u32x2_any_t*>(reinterpret_cast<const uint16_t*>(p) + at);
+  return u32x4_t{v.x, v.y, 0, 0};
+}
+
 // the two values of a packed word, fp16 or bf16
 __device__ __forceinline__ float2v_t unpack_pair(uint32_t word, int type) {
   if (type == kF16) {
@@ -111,6 +118,12 @@ __device__ __forceinline__ float2v_t unpack_pair(uint32_t word, int type) {
     return float2v_t{(float)h.x, (float)h.y};
   }
   return float2v_t{__builtin_bit_cast(float, word << 16), __builtin_bit_cast(float, word & 0xFFFF0000u)};
+}
+
+__device__ __forceinline__ float4v_t values_of_four(u32x4_t raw, int type) {
+  if (type == kF32) return __builtin_bit_cast(float4v_t, raw);
+  const float2v_t a = unpack_pair(raw.x, type), b = unpack_pair(raw.y, type);
+  return float4v_t{a.x, a.y, b.x, b.y};
 }
 
 // 1.0 in both halves, held in a vector register: v_and_or_b32 can then take the sign mask as its only
