@@ -86,8 +86,8 @@ int onebit_sparse_matmul_prepared(const void *prepared, const void *b, const voi
  * The prepared product for callers that cannot allocate device memory: code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc. It has no counterpart in the reference. Same arguments, kernels and results
  * as onebit_sparse_matmul_prepared; the only difference is where the two internal buffers live that some shapes need
- * (fp32 partial sums when K is split over workgroups, a copy of B with padded rows when B's rows are not 16-byte
- * aligned): in a fixed array of ONEBIT_STATIC_SCRATCH_BYTES bytes that is part of the library's device code, of
+ * (fp32 partial sums when K is split over workgroups, a copy of B with padded rows for some B whose rows are not
+ * 16-byte aligned): in a fixed array of ONEBIT_STATIC_SCRATCH_BYTES bytes that is part of the library's device code, of
  * which every GPU the library runs on holds one copy until the process ends. The call never calls hipMalloc, hipFree
  * or any allocating routine. A shape whose buffers do not fit is refused with ONEBIT_ERR_ARGUMENT and a message
  * that names the sizes (onebit_sparse_describe_launch of the tuning header tells which shapes need buffers: plan[2] > 1 or plan[3] = 1).

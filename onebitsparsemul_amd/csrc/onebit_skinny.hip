@@ -6,7 +6,7 @@ namespace onebit {
 template <int NW, int R>
 static hipError_t launch_skinny_cfg(const SkinnyArgs& args, hipStream_t stream) {
   const bool aligned = (reinterpret_cast<uintptr_t>(args.b) & 15) == 0;
-  // Beyond sixteen columns what wide_kernel leaves: B that is not read in 16-byte pieces in place, some products of 32 columns,
+  // Beyond sixteen columns what wide_kernel leaves: B at an unaligned base, an odd n on few rows, some products of 32 columns,
   // and more rows than give its grid two workgroups per compute unit (65536 on the whole GPU, where the main kernel takes 33
   // columns or more; 8192 on a partition of 32 compute units).
   if (args.n > 32) {  // 64-column images, two column fragments: at most two row blocks fit the registers
