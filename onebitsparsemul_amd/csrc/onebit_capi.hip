@@ -434,14 +434,19 @@ LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int comput
   return plan;
 }
 
-// wide_kernel against the main kernel. Both models err, and by how much depends on the plans. The lines were drawn where about as few
-// calls were slower on either side, on an earlier wide_kernel. Timed on the kernels as they are (6789 calls of 512 to 28672 rows, k =
-// 512 to 28672 and 65 to 2048 columns whose modelled times are 0.55 to 1.1 of one another, weights from HBM) they lie too low, on the
-// main kernel's side: of the 4115 calls that go to wide_kernel ten are more than 5 % slower than on the main kernel (9 % at most, 2176 x
-// 2048 with 712 tokens 10.0 us, 8.9 there; 20864 x 7616 with 152 columns would be another, 51 and 48), and all 6789 are 1.30 times as
-// fast as there in the mean; 1718 of the other 2674 would be more than 5 % faster here (2496 x 19648 with 197 tokens 25.9 and 27.9). Median
-// of measured / modelled time, wide_kernel and the main kernel, by line: 0.81 0.94 and 0.82 for layers, 0.96 and 0.85 for products; 0.85
-// 0.83 and 0.93; 0.87 0.85 and 0.91; 0.88 0.78 and 0.88; 0.92 0.87 and 0.97 for layers, 0.89 and 0.97 for products.
+// wide_kernel against the main kernel. Both models err, and by how much depends on the plans. A line of 0.81 to 0.88 was drawn where
+// about as few calls were slower on either side, on an earlier wide_kernel, whose model has it too slow now wherever its workgroups
+// have a compute unit each (in several rounds it is right: 64-row groups of 4992 x 1024 with 270 tokens, 468 of them, 8.7 us, 6.7 on
+// the main kernel at 1.17 of its modelled time). There the line is 1.05; main kernel | wide_kernel, us inside HIP graphs, weights from
+// HBM, random calls that it moves: 22 layers of one whole tile per K range 0.70 to 0.98 of the time, median 0.84 (3520 x 1248 with 206
+// tokens 8.6 | 6.0, 2624 x 7584 with 630 33.9 | 24.0), 44 products 0.51 to 1.03, median 0.79 (1088 x 672 with 416 columns 6.9 | 4.3, 3840 x
+// 7136 with 512 29.0 | 23.0, 1856 x 2400 with 471 17.4 | 10.9), 22 layers where the main kernel splits K 0.70 to 1.02, median 0.85 (704 x
+// 7456 with 985 19.3 | 13.5). Not moved: products where the main kernel splits K (768 x 8192 with 616 16.3 | 17.4) or has
+// the 256 x 128 tile (5440 x 13120 with 168 30.9 | 34.4); and layers in groups of other than 32 or 64 tokens where it splits K, products
+// with a workgroup for every compute unit or 32-row groups, which tests hold on the main kernel, some of which would gain (4096 x 4096
+// with 512 20.3 | 16.9, 512^3 4.8 | 3.6; 1024^3 6.5 | 6.5).
+// Where wide_kernel splits K the line is 0.96 for layers (0.78 to 1.03, median 0.88) and, with three splits or more, for products (0.73
+// to 1.03, median 0.87; in two splits 0.95 to 1.13, in few rows on 64-row groups up to 1.05).
 // Up to 64 columns the main kernel is the other plan beyond 40960 rows only, where a wavefront of wide_kernel has one short round
 // of work per workgroup and the workgroups come in many rounds, outside what its model was fitted to: the line is the length of
 // K, from which on wide_kernel is faster at 45056 to 262144 rows (us, wide | main, 48 and 64 tokens: 65536 x 1024 15.8 | 15.6 and
@@ -449,14 +454,23 @@ LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int comput
 // x 4096 23.9 | 27.3 and 28.5 | 27.5). With k % 64 != 0, where every second token's pieces straddle two lines, it lies twice as far out
 // (45056 x 4128 with 48 tokens 30.3 | 28.7, x 8224 45.7 | 51.4). Where the main kernel would split K,
 // wide_kernel in any case (41024 x 7936 and x 8160, 56 and 64 tokens: 44.1 to 47.8 against 55.5 to 59.4).
-bool wide_is_faster(const WidePlan& wide, const LaunchPlan& launch, int n, int k, bool plain) {
+bool wide_is_faster(const WidePlan& wide, const LaunchPlan& launch, int m, int n, int k, bool plain, int compute_units) {
   const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
   if (n <= onebit::kSkinnyMaxN) return launch.splits > 1 || chunks >= (n <= 48 ? 16 : 32) * (k % 64 ? 2 : 1);
-  const double line = wide.splits > 1                                 ? 0.92
-                      : launch.rows_or_tile == onebit::kTile256x128w8 ? 0.81
-                      : plain                                         ? 0.85
-                      : launch.splits > 1                             ? 0.87
-                                                                      : 0.88;
+  const long workgroups = (long)((m + wide.rows - 1) / wide.rows) * ((n + wide.tokens - 1) / wide.tokens);
+  const bool many_splits = !plain || (wide.splits >= 3 && (wide.rows == 128 || m >= 1024));
+  double line = wide.splits > 1                                 ? (many_splits ? 0.96 : 0.92)
+                : launch.rows_or_tile == onebit::kTile256x128w8 ? 0.81
+                : plain                                         ? 0.85
+                : launch.splits > 1                             ? 0.87
+                                                                : 0.88;
+  if (wide.splits == 1 && workgroups <= compute_units) {
+    if (plain) {
+      if (launch.rows_or_tile != onebit::kTile256x128w8 && launch.splits <= 1 && wide.rows >= 64 && workgroups < compute_units) line = 1.05;
+    } else if (launch.splits <= 1 || wide.tokens == 32 || wide.tokens == 64) {
+      line = 1.05;
+    }
+  }
   return wide.us < line * launch.model_us;
 }
 
@@ -496,7 +510,7 @@ LinearPlan plan_linear(int m, int tokens, int k, int compute_units) {
   if (tokens > onebit::kSkinnyMaxN && groups[2] * ((tokens + 63) / 64) > 2L * compute_units) return plan;
   plan.wide_plan = plan_wide(groups, (double)m * tokens, tokens, k, false, wide_least_splits(plan.launch, tokens, k, false),
                              plan.launch.splits, compute_units);
-  plan.wide = plan.launch.split_k_kernel || wide_is_faster(plan.wide_plan, plan.launch, tokens, k, false);
+  plan.wide = plan.launch.split_k_kernel || wide_is_faster(plan.wide_plan, plan.launch, m, tokens, k, false, compute_units);
   return plan;
 }
 
@@ -522,7 +536,7 @@ WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b
   if (!b_readable) return none;
   const WidePlan plan = plan_wide(groups, (double)m * n, n, k, true, wide_least_splits(launch, n, k, true), launch.splits,
                                   compute_units);
-  if (plan.us == 1e30 || (!launch.split_k_kernel && !wide_is_faster(plan, launch, n, k, true))) return none;
+  if (plan.us == 1e30 || (!launch.split_k_kernel && !wide_is_faster(plan, launch, m, n, k, true, compute_units))) return none;
   return plan;
 }
 
