@@ -331,7 +331,7 @@ SkinnyPlan plan_skinny(int m, int n, int k, int compute_units) {
 // compute unit pay the rounds again, less where two fit a compute unit (up to two column tiles on up to 64 rows). A split
 // pays a second launch and the partial sums.
 // Fitted to m = 1024 ... 28672, k = 1024 ... 22176, 17 ... 1024 tokens inside HIP graphs, when the kernel was slower than it is: it
-// takes 0.78 to 0.96 of the modelled time now (median by class of plan, see wide_is_faster). us of the chosen plan | of all tokens, or
+// takes 0.78 to 0.96 of the modelled time now (median by class of plan). us of the chosen plan | of all tokens, or
 // 64, per workgroup on 32 rows, unsplit: 28672 x 8192 x 48 22.3 (128 rows) | 40.4; 4096 x 11008 x 32 8.6 (32 rows, 16 tokens) | 12.0;
 // 1024 x 4096 x 256 4.6 (64 rows, 16 tokens) | 6.6; 4096 x 4096 x 128 5.6 (64 rows, 32 tokens) | 7.4.
 // total_groups: row groups of all products of the launch, for each of kWideRows.
