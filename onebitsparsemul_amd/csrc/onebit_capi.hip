@@ -796,14 +796,15 @@ bool takes_f32(int tokens) { return tokens <= onebit::kSkinnyTokens && g_skinny_
 
 // Whether skinny_kernel on fp32 activations is faster than converting them and running it on fp16 ones. Every workgroup reads all of
 // x of its K range, so fp32 costs a compute unit half of these bytes more, and beyond eight tokens an image comes in two batches, the
-// second requested behind the first (as long as sixteen more tokens would take); both hide behind the weights until they are many.
-// The conversion costs about 2 us whatever the size, and the host 4 us, which a call outside a graph hides behind its kernel only if
-// that takes 9 us. us inside HIP graphs, weights from HBM, converted | read as fp32: 4096 x 8192 with 16 tokens 9.3 | 9.1, x 11008 with
-// 9 / 12 / 16 9.5 | 9.3, 10.1 | 10.1, 10.9 | 11.6; 8192 x 14336 with 8 / 9 11.9 | 11.4, 12.0 | 12.6; 7168 x 20480 with 8 / 16 14.3 | 14.8,
-// 18.3 | 21.4; 11008 x 28672 with 5 / 16 24.6 | 22.9, 28.8 | 35.6; two rounds of workgroups: 49152 x 2048 with 16 16.2 | 15.3, x 4096
-// 19.9 | 21.2. Of 384 calls of up to sixteen tokens one is more than 2.5 % slower than the better of the two (12288 x 20480 with 8,
-// 20.8 | 20.1). Call after call without a graph: 4096 x 9600 with 16 8.9 | 8.2, x 11008 with 13 / 16 9.1 | 7.8, 9.1 | 8.8, 5120 x 13824
-// with 12 9.5 | 9.2, 8192 x 14336 with 9 9.8 | 9.8, 11008 x 28672 with 16 21.5 | 27.8.
+// second requested behind the first; both hide behind the weights until they are many. The conversion costs about 2 us whatever the
+// size, and the host 4 us, which a call outside a graph hides behind its kernel only if that takes 9 us. us inside HIP graphs, weights
+// from HBM, converted | read as fp32: 4096 x 8192 with 16 tokens 8.5 | 7.9, x 11008 with 9 / 12 / 16 8.6 | 7.4, 9.1 | 8.3, 9.2 | 9.7;
+// 8192 x 14336 with 8 / 9 10.0 | 9.0, 10.3 | 9.4; 7168 x 20480 with 8 / 16 11.0 | 11.0, 16.7 | 19.7; 11008 x 28672 with 5 / 16 20.1 |
+// 19.1, 26.1 | 32.7; two rounds of workgroups: 49152 x 2048 with 16 13.7 | 13.8, x 4096 18.1 | 19.4. Of 170 calls near the lines one that
+// is read is more than 5 % slower than converted (832 x 9088 with 16, 8.2 | 8.7). The lines were drawn when nine to fifteen tokens took
+// the loads of sixteen in branches: 20 calls that are converted would be 5 to 22 % faster read, most of nine to thirteen tokens (4608 x
+// 12448 with 10 10.2 | 8.3). Call after call without a graph: 4096 x 9600 with 16 10.1 | 8.9, x 11008 with 13 / 16 10.2 | 8.6, 10.2 |
+// 9.5, 5120 x 13824 with 12 10.2 | 9.8, 8192 x 14336 with 9 10.2 | 9.2, 11008 x 28672 with 16 26.9 | 34.0.
 bool reading_f32_is_faster(int tokens, int m, int k, int compute_units, hipStream_t stream) {
   // read whatever the plan: no row group is smaller than 32, a split reads less (spares a small call the second plan)
   const long most_rounds = (m / 32 + compute_units - 1) / compute_units;

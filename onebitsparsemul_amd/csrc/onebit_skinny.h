@@ -43,6 +43,10 @@ constexpr int kSkinnyRegion = 8192;  // bytes of one B image
 // instruction takes a token's 256 K, whole lines, so there are as many as tokens. A conversion in front of the kernel costs a
 // launch and an allocation (us per layer call, conversion in front -> here: 4096 x 4096 with 1 / 16 tokens 9.2 / 9.0 -> 4.8 / 4.9,
 // 28672 x 8192 with 8 / 16 14.0 / 15.5 -> 11.8 / 14.8, 4096 x 11008 with 16 9.0 -> 8.7).
+// kSkinnyBTokens32 + l: l load instructions take an image, the ninth and later ones in a second batch. No more than one past the last
+// token: a surplus one costs its place in the load path (us inside HIP graphs, weights from HBM, each load in a branch of its own | eight
+// and eight for nine tokens and more | this: 8192 x 8192 with 9 / 13 tokens 7.5 | 8.8 | 7.3, 8.4 | 9.0 | 8.5, 4096 x 11008 with 9 8.3 |
+// 9.4 | 7.6, 4096 x 4096 with 9 / 16 5.0 | 5.4 | 4.5, 5.8 | 5.7 | 5.4, 28672 x 8192 with 10 15.5 | 16.0 | 14.4).
 enum SkinnyBMode { kSkinnyBFull = 0, kSkinnyBAny = 1, kSkinnyBColumns = 16, kSkinnyBTokens = 32, kSkinnyBTokens32 = 48 };
 
 // The body of the split-K kernel for workgroup (block_x, block_y) of problem p: block_x = row group, block_y = K split.
@@ -71,7 +75,8 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   constexpr int PPT = IMG_ROWS / 8;                    // token-major image: 16-byte pieces per token row
   constexpr int TPI = 64 / PPT;                        // ... and tokens covered by the 64 pieces of one wavefront load
   constexpr int TOKEN_ROW_BYTES = IMG_ROWS * 2;
-  constexpr int TOKEN_LOADS = X32 ? MODE - kSkinnyBTokens32 : TOKENS ? MODE - kSkinnyBTokens : 8;
+  constexpr int LOADS32 = X32 ? MODE - kSkinnyBTokens32 : 0, SECOND_LOADS = LOADS32 > 8 ? LOADS32 - 8 : 0;
+  constexpr int TOKEN_LOADS = X32 ? LOADS32 - SECOND_LOADS : TOKENS ? MODE - kSkinnyBTokens : 8;
   __shared__ __attribute__((aligned(16))) char bs[NW * kSkinnyRegion];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -144,22 +149,26 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   const uint32_t token_load_step = (uint32_t)TPI * (uint32_t)k_rows * 2u;
   const uint32_t token_store_base =
       (uint32_t)token_lane * TOKEN_ROW_BYTES + (uint32_t)((piece_lane ^ token_swizzle<TOKEN_ROW_BYTES>(token_lane)) << 4);
-  // fp32 activations, eight tokens from first_token on. Load i: the image's K range of one token, four values per lane; K positions
+  // fp32 activations, up to eight tokens from first_token on. Load i: the image's K range of one token, four values per lane; K positions
   // at or past k: outside the descriptor, as below (the launcher checks that 64 * k * 4 stays well below 2^32). Tokens 8 to 15
   // are requested when the first eight have been stored: 64 registers of loads in flight do not fit beside the rest.
-  auto load_b32 = [&](int k_base, int first_token, u32x4_t (&v)[8]) __attribute__((always_inline)) {
+  auto load_b32 = [&](int k_base, int first_token, auto loads_tag, u32x4_t (&v)[8]) __attribute__((always_inline)) {
     const bool whole = k_base + IMG_ROWS <= k_rows;  // wave-uniform
     const bool inside = k_base + 4 * lane < k_rows;
 #pragma unroll
-    for (int i = 0; i < TOKEN_LOADS; ++i) {
+    for (int i = 0; i < decltype(loads_tag)::value; ++i) {
       const uint32_t offset = meta_off + (uint32_t)(first_token + i) * (uint32_t)k_rows * 4u;
+      // Sixteen wavefronts with six loads or more at a time: one per sixteen clocks, as many as the load path takes. All at once they
+      // keep out the other wavefronts' (8192 x 8192 with 6 / 8 tokens 6.08 / 6.50 us with a branch around each, 6.32 / 6.77 at once, 5.98 /
+      // 6.40 so; 2048 x 8192 with 8 5.63, 5.70, 5.42; one per 48 clocks 6.02)
+      if (NW == 16 && LOADS32 >= 6 && LOADS32 <= 8 && i > 0) asm volatile("s_nop 15" ::: "memory");
       // tokens past the last: outside the descriptor, as in load_b
       v[i] = buffer_load16(b_buffer, whole ? offset : inside ? offset + (uint32_t)k_base * 4u : 0xFFFFFF00u, whole ? (uint32_t)k_base * 4u : 0u);
     }
   };
-  auto store_b32 = [&](int first_token, const u32x4_t (&v)[8]) __attribute__((always_inline)) {
+  auto store_b32 = [&](int first_token, auto loads_tag, const u32x4_t (&v)[8]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < TOKEN_LOADS; ++i) {
+    for (int i = 0; i < decltype(loads_tag)::value; ++i) {
       const float4v_t f = __builtin_bit_cast(float4v_t, v[i]);
       const int token = first_token + i;
       *reinterpret_cast<u32x2_t*>(region + token * TOKEN_ROW_BYTES + (((lane >> 1) ^ token_swizzle<TOKEN_ROW_BYTES>(token)) << 4) +
@@ -182,7 +191,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
       return;
     }
     if (X32) {
-      load_b32(k_base, 0, v);
+      load_b32(k_base, 0, std::integral_constant<int, TOKEN_LOADS>{}, v);
       return;
     }
     if (TOKENS) {
@@ -248,11 +257,11 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
   };
   auto store_b = [&](int k_base, const u32x4_t (&v)[8]) __attribute__((always_inline)) {
     if (X32) {
-      store_b32(0, v);
-      if (TOKEN_LOADS == 8 && n_cols > 8) {
+      store_b32(0, std::integral_constant<int, TOKEN_LOADS>{}, v);
+      if constexpr (SECOND_LOADS > 0) {
         u32x4_t w[8];
-        load_b32(k_base, 8, w);
-        store_b32(8, w);
+        load_b32(k_base, 8, std::integral_constant<int, SECOND_LOADS>{}, w);
+        store_b32(8, std::integral_constant<int, SECOND_LOADS>{}, w);
       }
       return;
     }

@@ -11,11 +11,19 @@ static hipError_t launch_skinny_tokens_type(const SkinnyArgs& args, hipStream_t 
 template <int NW, int R>
 static hipError_t launch_skinny_tokens_cfg(const SkinnyArgs& args, hipStream_t stream) {
   if (args.x_f32) {  // one token per load instruction, eight at once
-    if (args.n == 1) return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 1, 16>(args, stream);
-    if (args.n == 2) return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 2, 16>(args, stream);
-    if (args.n <= 4) return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 4, 16>(args, stream);
-    if (args.n <= 6) return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 6, 16>(args, stream);
-    return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 8, 16>(args, stream);
+    switch (args.n) {
+      case 1: return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 1, 16>(args, stream);
+      case 2: return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 2, 16>(args, stream);
+      case 3: case 4: return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 4, 16>(args, stream);
+      case 5: return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 5, 16>(args, stream);
+      case 6: return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 6, 16>(args, stream);
+      case 7: return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 7, 16>(args, stream);
+      case 8: return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 8, 16>(args, stream);
+      case 9: case 10: return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 10, 16>(args, stream);
+      case 11: case 12: return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 12, 16>(args, stream);
+      case 13: case 14: return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 14, 16>(args, stream);
+      default: return launch_skinny_mode<NW, R, kSkinnyBTokens32 + 16, 16>(args, stream);
+    }
   }
   return args.bf16 ? launch_skinny_tokens_type<NW, R, true>(args, stream) : launch_skinny_tokens_type<NW, R, false>(args, stream);
 }

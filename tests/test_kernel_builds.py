@@ -1,0 +1,53 @@
+"""Which build of a kernel a call launches, without a GPU: the library is linked against tests/host/launch_stub.cpp, which stands in for
+the HIP runtime and records the kernels' names."""
+import ctypes
+import os
+import re
+import subprocess
+
+import pytest
+
+from onebitsparsemul_amd import build as native_build
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+vp, i32, f32 = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("host")
+    obj, out = str(folder / "launch_stub.o"), str(folder / "libhost.so")
+    subprocess.run([os.path.join(os.path.dirname(native_build.HIPCC), "..", "llvm", "bin", "clang++"), "-O1", "-std=c++17", "-fPIC",
+                    "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-c", os.path.join(HERE, "host", "launch_stub.cpp"), "-o", obj],
+                   check=True)
+    # -Bsymbolic: the stand-ins, not the HIP runtime that torch has loaded
+    subprocess.run(["g++", "-shared", "-Wl,-Bsymbolic", "-o", out, obj, "-Wl,-u,onebit_sparse_prepare", native_build.STATIC_LIB,
+                    "-lpthread"], check=True)
+    lib = ctypes.CDLL(out)
+    lib.stub_launched.restype = ctypes.c_char_p
+    lib.onebit_sparse_last_error.restype = ctypes.c_char_p
+    lib.onebit_sparse_linear_prepared_f32.argtypes = [vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]
+    return lib
+
+
+def launched(lib, call, *args):
+    """[(kernel, template arguments)] of a call's launches"""
+    lib.stub_reset()
+    assert call(*args) == 0, lib.onebit_sparse_last_error()
+    names = lib.stub_launched().decode().splitlines()
+    return [(m[1], m[2].split(", ")) for m in (re.match(r"(?:void )?onebit::(\w+)<([^>]*)>", name) for name in names)]
+
+
+@pytest.mark.parametrize("rows", [32, 64, 128])
+def test_fp32_activations_take_no_more_than_one_surplus_load(host, rows):
+    """One load instruction per token and image: a surplus one costs its place in the load path (8192 x 8192 with nine tokens 7.3 us, 8.8
+    with sixteen loads)."""
+    host.onebit_sparse_set_skinny_rows(rows)
+    try:
+        for tokens in range(1, 17):
+            (kernel, arguments), = launched(host, host.onebit_sparse_linear_prepared_f32, 0x1000, 0x2000, None, 0x3000, tokens, 8192, 8192, 1,
+                                            0, None)
+            loads = int(arguments[2]) - 48  # kSkinnyBTokens32
+            assert kernel == "skinny_kernel" and tokens <= loads <= tokens + 1, (tokens, loads)
+    finally:
+        host.onebit_sparse_set_skinny_rows(-1)
