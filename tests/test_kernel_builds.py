@@ -7,6 +7,7 @@ import subprocess
 
 import pytest
 
+from onebitsparsemul_amd import _native
 from onebitsparsemul_amd import build as native_build
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -27,6 +28,7 @@ def host(tmp_path_factory):
     lib.stub_launched.restype = ctypes.c_char_p
     lib.onebit_sparse_last_error.restype = ctypes.c_char_p
     lib.onebit_sparse_linear_prepared_f32.argtypes = [vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]
+    lib.onebit_sparse_linear_prepared_grouped.argtypes = [ctypes.POINTER(_native.LinearProblem), i32, i32, i32, i32, vp]
     return lib
 
 
@@ -51,3 +53,17 @@ def test_fp32_activations_take_no_more_than_one_surplus_load(host, rows):
             assert kernel == "skinny_kernel" and tokens <= loads <= tokens + 1, (tokens, loads)
     finally:
         host.onebit_sparse_set_skinny_rows(-1)
+
+
+@pytest.mark.parametrize("count", [1, 2, 4, 5, 16])
+@pytest.mark.parametrize("k,parts", [(4096, False), (5120, True), (4096 + 1792, False)])  # 16, 20 and 23 chunks of 256
+def test_groups_take_the_build_with_parts_where_a_remainder_is_dealt_in_parts(host, count, k, parts):
+    """The build with parts is 1 to 4 % slower where there are none."""
+    problems = (_native.LinearProblem * count)(*[_native.LinearProblem(0x1000, 0x2000, None, 0x3000, 512, k)] * count)
+    for tokens in (17, 64):
+        (kernel, arguments), = launched(host, host.onebit_sparse_linear_prepared_grouped, problems, count, tokens, 1, 1, None)
+        if kernel == "wide_kernel":  # R, COPIES, TOKENS, BF16, PARTS, RAGGED
+            assert arguments[4] == str(parts).lower()
+        else:                        # R, COPIES, BF16, PARTS, MOST
+            assert kernel == "wide_tokens_group_kernel" and arguments[3] == str(parts).lower()
+            assert int(arguments[4]) == (4 if count <= 4 else 16)
