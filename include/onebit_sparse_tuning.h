@@ -30,7 +30,7 @@ void onebit_sparse_set_skinny_rows(int rows);
 void onebit_sparse_set_split_k(int splits);
 /* B whose rows are not 16-byte aligned and n beyond the split-K kernel's range. With an aligned base and n % 8 != 0 the kernels
  * mostly read B where it lies; with an unaligned base, beyond 64 columns when K is split, and for an odd n where its rows would
- * cost more than a copy: 1 (default) = the kernel reads a copy of B with rows padded to a multiple of 8 columns, made by one extra
+ * cost more than a copy, and with a forced tile that the plan never chooses: 1 (default) = the kernel reads a copy of B with rows padded to a multiple of 8 columns, made by one extra
  * pass into a library-owned buffer kept per device and stream (same rules as the K-split buffer); 0 = B is read in place all the
  * same, with an unaligned base by the main kernel's element-copy variant (much slower). With k * n < 65536 the copy is made where its buffer is there
  * or can be allocated: not by the non-allocating entry point, and in a stream capture only after a warm-up. */

@@ -584,7 +584,9 @@ ProductPlan plan_product(int m, int n, int k, bool b_16_byte_aligned, int comput
   ProductPlan plan{};
   plan.launch = choose_launch(m, n, k, b_16_byte_aligned, compute_units);
   const LaunchPlan& launch = plan.launch;
-  const bool b_in_place = n % 8 == 0 && b_16_byte_aligned, ragged = n % 8 != 0 && n >= 8 && b_16_byte_aligned;
+  const bool b_in_place = n % 8 == 0 && b_16_byte_aligned;
+  // (a forced tile without a build for it reads the padded copy: 4096 x 1002 x 4096 in element copies more than ten times as long)
+  const bool ragged = n % 8 != 0 && n >= 8 && b_16_byte_aligned && (launch.split_k_kernel || onebit::tile_reads_ragged(launch.rows_or_tile));
   plan.pad_b = launch.pad_b || (!launch.split_k_kernel && !b_in_place && !ragged && g_pad_b && small_pad());
   plan.wide = plan_wide_product(launch, m, n, k, b_in_place || plan.pad_b || ragged, compute_units);
   if (ragged) {

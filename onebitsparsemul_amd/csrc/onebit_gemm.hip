@@ -109,7 +109,7 @@ static hipError_t launch_gemm_pass(GemmArgs args, int tile_config, hipStream_t s
   const bool aligned = (args.ldb % 8 == 0) && ((reinterpret_cast<uintptr_t>(args.b) & 15) == 0);
   if (!aligned) {
     if (read_as_ragged(args.b, args.ldb)) {
-      switch (tile_config) {  // the tiles that the plan chooses
+      switch (tile_config) {  // tile_reads_ragged
         case kTile256x128w: return launch_gemm_cfg<2, 2, 4, 2, true, false, 1, false, false, true>(args, stream);
         case kTile128x128s: return launch_gemm_cfg<2, 2, 2, 2, true, false, 1, false, false, true>(args, stream);
         case kTile512x128w8: return launch_gemm_cfg<4, 2, 4, 2, true, false, 1, false, false, true>(args, stream);

@@ -93,6 +93,15 @@ inline bool read_as_ragged(const void* b, int n) { return n >= 8 && (reinterpret
 
 enum TileConfig { kTile512x128 = 0, kTile256x128 = 1, kTile128x128 = 2, kTile256x256 = 3, kTile256x128w = 4, kTile512x128t = 5, kTile128x128s = 6, kTile256x64 = 7, kTile256x256w8 = 8, kTile512x128w8 = 9, kTile256x128w8 = 10, kTile128x128w8 = 11, kTile64x128 = 12, kTile128x128k2 = 13, kTile64x128k2 = 14, kTile512x128m16 = 15, kTileAuto = -1 };
 
+// Whether the main kernel's tile has a build that reads a ragged B: those that the plan chooses.
+inline bool tile_reads_ragged(int tile) {
+  switch (tile) {
+    case kTile256x128w: case kTile128x128s: case kTile512x128w8: case kTile256x128w8: case kTile128x128w8: case kTile64x128:
+    case kTile128x128k2: case kTile64x128k2: case kTile512x128m16: return true;
+    default: return false;
+  }
+}
+
 hipError_t launch_prepare(const void* a, const void* e, void* prep, int m, int k, int layout, hipStream_t stream);
 hipError_t launch_gemm(GemmArgs args, int tile_config, hipStream_t stream);
 // The linear layer's form of the main kernel: b is x (n tokens x k, token-major, 16-byte aligned), d is y (n tokens x

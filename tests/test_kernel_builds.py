@@ -28,6 +28,7 @@ def host(tmp_path_factory):
     lib.stub_launched.restype = ctypes.c_char_p
     lib.onebit_sparse_last_error.restype = ctypes.c_char_p
     lib.onebit_sparse_linear_prepared_f32.argtypes = [vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]
+    lib.onebit_sparse_matmul_prepared.argtypes = [vp, vp, vp, vp, i32, i32, i32, f32, f32, i32, i32, vp]
     lib.onebit_sparse_linear_prepared_grouped.argtypes = [ctypes.POINTER(_native.LinearProblem), i32, i32, i32, i32, vp]
     return lib
 
@@ -36,8 +37,10 @@ def launched(lib, call, *args):
     """[(kernel, template arguments)] of a call's launches"""
     lib.stub_reset()
     assert call(*args) == 0, lib.onebit_sparse_last_error()
-    names = lib.stub_launched().decode().splitlines()
-    return [(m[1], m[2].split(", ")) for m in (re.match(r"(?:void )?onebit::(\w+)<([^>]*)>", name) for name in names)]
+    # (a name with _Float16 among its parameters stays mangled)
+    found = [re.search(r"(\w+)<([^>]*)>\(", name) or re.match(r"_ZN6onebit\d+([a-z_]+)(E)", name)
+             for name in lib.stub_launched().decode().splitlines()]
+    return [(m[1], m[2].split(", ")) for m in found]
 
 
 @pytest.mark.parametrize("rows", [32, 64, 128])
@@ -67,3 +70,19 @@ def test_groups_take_the_build_with_parts_where_a_remainder_is_dealt_in_parts(ho
         else:                        # R, COPIES, BF16, PARTS, MOST
             assert kernel == "wide_tokens_group_kernel" and arguments[3] == str(parts).lower()
             assert int(arguments[4]) == (4 if count <= 4 else 16)
+
+
+@pytest.mark.parametrize("tile", [-1, *range(16)])
+@pytest.mark.parametrize("n,k", [(1002, 4096), (1001, 4096), (102, 512), (12, 4096), (9, 512)])
+def test_no_ragged_product_takes_the_element_copies(host, tile, n, k):
+    """A tile, forced by the hook too, that has no build for rows that lie anywhere reads the padded copy: more than ten times faster."""
+    host.onebit_sparse_set_tile_config(tile)
+    host.onebit_sparse_set_skinny_enabled(0)
+    try:
+        kernels = launched(host, host.onebit_sparse_matmul_prepared, 0x1000, 0x2000, None, 0x3000, 4096, n, k, 1.0, 0.0, 0, 1, None)
+    finally:
+        host.onebit_sparse_set_tile_config(-1)
+        host.onebit_sparse_set_skinny_enabled(1)
+    gemm = [arguments for kernel, arguments in kernels if kernel == "gemm_kernel"]  # WM, WN, FM, FN, DMA, TOKENS, KG, M16, BF16, RAGGED
+    padded = kernels[0][0] == "pad_b_kernel"
+    assert len(gemm) == 1 and gemm[0][4] == "true" and (gemm[0][9] == "false") == padded
