@@ -130,6 +130,16 @@ def test_fewer_columns_never_replace_the_partial_sum_buffer(fresh, call, m, k):
         assert call(fresh, m, n, k) == 0, (n, fresh.onebit_sparse_last_error())
 
 
+def test_small_unaligned_b_never_replaces_the_padded_copy_of_another(fresh):
+    """The copy of 992 x 66 values is the larger in bytes than that of 576 x 119: made into the same buffer, and captured after it
+    without a warm-up."""
+    assert product(fresh, 256, 119, 576, b=0x2002) == 0 and last_launch(fresh)["padded"]
+    before = fresh.stub_allocated_bytes()
+    fresh.stub_set(0, 1)
+    assert product(fresh, 256, 66, 992, b=0x2002) == 0 and last_launch(fresh)["padded"]
+    assert fresh.stub_allocated_bytes() == before
+
+
 @pytest.mark.parametrize("call,m,n,k", [(layer, 896, 704, 24256), (layer, 1088, 1758, 13888), (layer, 704, 1920, 14816),
                                         (layer, 640, 676, 17536), (layer, 1088, 1694, 5696), (layer, 1344, 969, 9216),
                                         (layer, 2496, 197, 19648), (product, 20864, 152, 7616), (product, 768, 616, 8192),

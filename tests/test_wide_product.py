@@ -51,16 +51,17 @@ def test_result_over_c(n, dtype):
     assert torch.equal(d.cpu(), (dense @ b.double() + c.double()).to(dtype))
 
 
-def test_small_ragged_b_leaves_the_buffer_of_a_captured_graph():
+def test_small_unaligned_b_leaves_the_buffer_of_a_captured_graph():
     """The padded copy of B (576 x 119, the larger in values) is the smaller in bytes: the second call must not replace the
-    buffer that the graph reads."""
+    buffer that the graph reads. Both start at an odd value, where a copy is made whatever kernel reads it."""
+    assert _native.describe_launch(256, 119, 576, b_aligned=False, compute_units=None)["pad_b"]
     stream = torch.cuda.Stream()
     weights = {k: synthetic.make_weight(256, k, k, device="cuda") for k in (576, 992)}
     prepared = {k: PreparedWeight(*w) for k, w in weights.items()}
     dense = {k: dequant_desparse_tile(w[0].cpu(), w[1].cpu()).double() for k, w in weights.items()}
     g = torch.Generator().manual_seed(1)
     large, small = (torch.randint(-4, 5, shape, generator=g).half() for shape in ((576, 119), (992, 66)))
-    large_gpu, small_gpu = large.cuda(), small.cuda()
+    large_gpu, small_gpu = (torch.empty(b.numel() + 1, dtype=b.dtype, device="cuda")[1:].view(b.shape).copy_(b) for b in (large, small))
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.stream(stream):
