@@ -154,8 +154,10 @@ __device__ __forceinline__ half8_t expand_signs(const AChunk& a, uint32_t packed
 // allocation mixes the two register files and then copies whole accumulator tiles between them behind the SMFMAC
 // that produced them, which serialises the matrix pipe. Consecutive SMFMACs never share an accumulator, so no
 // wait states are needed between them.
-// A vector instruction's result may be an operand of an SMFMAC two instructions later at the earliest, which the compiler does not know of
-// inline assembly: SETTLE puts the wait states in front, for the first SMFMAC behind a loop's register copies.
+// From a vector instruction that writes an operand to the SMFMAC two wait states must pass, which the compiler does not know of inline
+// assembly: SETTLE puts them in front, for the first SMFMAC behind a loop's register copies (without it one tile's build has a copy one
+// wait state ahead). The other SMFMACs' operands are read and expanded a K step ahead; that no copy comes between is not given by the
+// source, tests/test_wait_states.py checks it on the machine code of every build.
 template <int STEP, bool PINNED = true, bool BF16 = false, bool SETTLE = false>
 __device__ __forceinline__ float16_t smfmac_step(const AChunk& a, half8_t av, half16_t bv, float16_t acc) {
   const int idx = (int)a.meta[STEP / 2];

@@ -1,0 +1,79 @@
+"""The compiler counts no wait states in front of an SMFMAC in inline assembly. On the machine code of the built library: no vector
+instruction writes an operand of one of gemm_kernel's SMFMACs less than two wait states in front of it."""
+import os
+import re
+import subprocess
+
+import pytest
+
+from onebitsparsemul_amd import build as native_build
+
+NEEDED = 2  # wait states from a vector instruction's write to an SMFMAC's read of the register
+REGISTER = re.compile(r"\b([av])(?:\[(\d+):(\d+)\]|(\d+))")
+
+
+def registers(text):
+    return {(kind, i) for kind, low, high, one in REGISTER.findall(text) for i in range(int(low or one), int(high or one) + 1)}
+
+
+def too_close(code):
+    """(SMFMAC, write) line pairs of one function's code, [(address, instruction, operands, branch target or None)]"""
+    at = {line[0]: i for i, line in enumerate(code)}
+    jumps = {}
+    for i, (_, _, _, target) in enumerate(code):
+        if target in at:
+            jumps.setdefault(at[target], []).append(i)
+
+    def writes(i, operands, states):
+        """vector instructions that write one of `operands` and reach instruction i within less than `states` wait states"""
+        falls = [i - 1] if i > 0 and code[i - 1][1] not in ("s_branch", "s_endpgm") else []
+        for j in falls + jumps.get(i, []):
+            _, name, rest, _ = code[j]
+            if name.startswith("v_") and "mfma" not in name and "smfmac" not in name:
+                if registers(rest if "swap" in name else rest.split(",")[0]) & operands:
+                    yield j
+                    continue
+            passed = int(rest, 0) + 1 if name == "s_nop" else 1
+            if passed < states:
+                yield from writes(j, operands, states - passed)
+
+    return [(code[i][1:3], code[j][1:3]) for i, line in enumerate(code) if "smfmac" in line[1]
+            for j in writes(i, registers(line[2]), NEEDED)]
+
+
+def functions(text):
+    """name and code of each function of a disassembly"""
+    for part in re.split(r"^(?=[0-9a-f]{16} <)", text, flags=re.M)[1:]:
+        head, *lines = part.splitlines()
+        start, code = int(head[:16], 16), []
+        for line in lines:
+            found = re.match(r"\s+(\w+)(.*?)\s*// ([0-9A-F]{12}): [0-9A-F ]+(?:<[^+>]+(?:\+0x([0-9a-f]+))?>)?", line)
+            if found:
+                branch = found[1].startswith(("s_cbranch", "s_branch"))
+                code.append((int(found[3], 16), found[1], found[2], start + int(found[4] or "0", 16) if branch else None))
+        yield head[18:-2], code
+
+
+def test_the_check_finds_a_write_that_is_too_close():
+    smfmac = (12, "v_smfmac_f32_32x32x32_f16", " a[0:15], v[6:9], v[10:17], v5", None)
+    for write in ((0, "v_mov_b64_e32", " v[4:5], v[2:3]", None), (0, "v_accvgpr_write_b32", " a15, v1", None)):
+        wait = (4, "s_setprio", " 1", None)
+        assert too_close([write, smfmac]) and too_close([write, wait, smfmac])
+        assert not too_close([write, wait, (8, "s_nop", " 0", None), smfmac]) and not too_close([write, (4, "s_nop", " 1", None), smfmac])
+        # around a loop
+        assert too_close([(8, "s_nop", " 3", None), smfmac, write, (20, "s_cbranch_scc1", " 1", 12)])
+    assert not too_close([(0, "v_mov_b32_e32", " v4, v5", None), smfmac])
+
+
+@pytest.mark.parametrize("source", ["onebit_gemm.o", "onebit_gemm_tokens.o"])
+def test_operands_of_inline_smfmacs_are_written_early_enough(source, tmp_path):
+    llvm = os.path.join(os.path.dirname(native_build.HIPCC), "..", "llvm", "bin")
+    subprocess.run(["ar", "x", native_build.STATIC_LIB, source], cwd=tmp_path, check=True)
+    subprocess.run([os.path.join(llvm, "llvm-objdump"), "--offloading", source], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL)
+    (device,) = [name for name in os.listdir(tmp_path) if name.endswith("gfx950")]
+    text = subprocess.run([os.path.join(llvm, "llvm-objdump"), "-d", device], cwd=tmp_path, check=True, capture_output=True, text=True).stdout
+    kernels = {name: code for name, code in functions(text) if "gemm_kernel" in name}
+    assert len(kernels) >= 18 and sum("smfmac" in line[1] for code in kernels.values() for line in code) > 2000
+    assert sum(line[3] is not None for code in kernels.values() for line in code) > 100  # branches with their targets
+    for name, code in kernels.items():
+        assert not too_close(code), name
