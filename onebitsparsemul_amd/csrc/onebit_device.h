@@ -98,16 +98,21 @@ __device__ __forceinline__ uint16_t round_one(float x) {
   if constexpr (BF16) return __builtin_bit_cast(uint16_t, (__bf16)x);
   else return __builtin_bit_cast(uint16_t, (_Float16)x);
 }
+// Memory that is known to be global: a load through a pointer put together from arguments counts as one that may be LDS, and while one is
+// outstanding the compiler waits for all LDS reads instead of some.
+template <class T>
+using global_t = const __attribute__((address_space(1))) T;
+
 // element `at` of an array whose type is known at run time
 __device__ __forceinline__ float load_element(const void* p, int type, size_t at) {
-  if (type == kF32) return reinterpret_cast<const float*>(p)[at];
-  const uint16_t bits = reinterpret_cast<const uint16_t*>(p)[at];
+  if (type == kF32) return ((global_t<float>*)p)[at];
+  const uint16_t bits = ((global_t<uint16_t>*)p)[at];
   return type == kF16 ? (float)__builtin_bit_cast(_Float16, bits) : __builtin_bit_cast(float, (uint32_t)bits << 16);
 }
 // Four consecutive elements from `at` on as they lie, one load (16-bit types: the first two words), and their values.
 __device__ __forceinline__ u32x4_t load_four(const void* p, int type, size_t at) {
-  if (type == kF32) return *reinterpret_cast<const u32x4_any_t*>(reinterpret_cast<const float*>(p) + at);
-  const u32x2_t v = *reinterpret_cast<const u32x2_any_t*>(reinterpret_cast<const uint16_t*>(p) + at);
+  if (type == kF32) return *(global_t<u32x4_any_t>*)((global_t<float>*)p + at);
+  const u32x2_t v = *(global_t<u32x2_any_t>*)((global_t<uint16_t>*)p + at);
   return u32x4_t{v.x, v.y, 0, 0};
 }
 
@@ -157,7 +162,7 @@ __device__ __forceinline__ half8_t expand_signs(const AChunk& a, uint32_t packed
 // From a vector instruction that writes an operand to the SMFMAC two wait states must pass, which the compiler does not know of inline
 // assembly: SETTLE puts them in front, for the first SMFMAC behind a loop's register copies (without it one tile's build has a copy one
 // wait state ahead). The other SMFMACs' operands are read and expanded a K step ahead; that no copy comes between is not given by the
-// source, tests/test_wait_states.py checks it on the machine code of every build.
+// source, tests/test_machine_code.py checks it on the machine code of every build.
 template <int STEP, bool PINNED = true, bool BF16 = false, bool SETTLE = false>
 __device__ __forceinline__ float16_t smfmac_step(const AChunk& a, half8_t av, half16_t bv, float16_t acc) {
   const int idx = (int)a.meta[STEP / 2];

@@ -426,17 +426,13 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
   // position s ^ (token % slots)
   constexpr int SLOTS = RT * 8;
   char* const y_out = reinterpret_cast<char*>(p.d) + (size_t)block_y * p.m * p.n * 4;  // a K split's slice: fp32 sums
-  // A thread's results of a round are four rows of several tokens: their bias is requested in front of the first barrier, not behind
-  // the sums, where its latency came once per four rows (us, so | this: 28672 x 8192 with 48 tokens 23.4 | 22.4, 11008 x 4096 with 64
-  // 10.5 | 9.6, 16704 x 1056 with 44 9.7 | 8.3; requested ahead of the K loop no less, and calls without a bias 1 to 2 % more).
+  // A thread's results of a round are four rows of several tokens: their bias is requested in front of the sums, once. The calls without
+  // one have a form of their own behind the barrier: what selects or skips a bias in theirs, and whatever stands in front of the barrier
+  // (a wait for the operands that a wavefront without a chunk has requested, too), is 2 to 5 % of a call of few chunks. us, bias of each
+  // row loaded behind the sums | requested in front of the barrier, one form | this: with a bias 28672 x 8192 with 48 tokens 23.5 | 21.9 |
+  // 22.3, 11008 x 4096 with 64 9.27 | 8.64 | 8.81, 16384 x 1024 with 64 5.72 | 5.36 | 5.27; without 16384 x 1024 with 64 5.03 | 5.25 |
+  // 5.01, 11520 x 1312 with 53 5.42 | 5.64 | 5.37, 1152 x 960 with 175 3.14 | 3.27 | 3.16, 18304 x 768 with 64 6.23 | 6.45 | 6.35.
   static_assert(64 * NW % SLOTS == 0, "a thread's rows of a round");
-  u32x4_t bias_raw[R / RT];
-  if (TOKENS && p.bias)
-#pragma unroll
-    for (int round = 0; round < R / RT; ++round) {
-      const int row = (rb_first + round * RT) * kRowBlock + 4 * (tid % SLOTS);
-      bias_raw[round] = load_four(p.bias, p.bias_type, row < p.m ? row : 0);
-    }
 #pragma unroll
   for (int round = 0; round < R / RT; ++round) {
     if (round > 0) __syncthreads();
@@ -464,33 +460,43 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
               acc[2 * (round * RT + rr) + h][ct];
         }
     __syncthreads();
-    for (int idx = tid; idx < SLOTS * 16 * CT; idx += 64 * NW) {
-      const int slot = TOKENS ? idx % SLOTS : idx / (16 * CT), token = TOKENS ? idx / SLOTS : idx % (16 * CT);
-      const int at = (token * SLOTS + (slot ^ (token & (SLOTS - 1)))) * 16;
-      float4v_t sum = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int w = 0; w < NW; ++w) sum += *reinterpret_cast<const float4v_t*>(smem + w * Shape::REGION + at);
-      const int row = (rb_first + round * RT) * kRowBlock + 4 * slot;
-      if (token >= tokens || row >= p.m) continue;
-      if constexpr (!TOKENS) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const size_t o = (size_t)(row + e) * p.n + first_token + token;
-          float x = p.alpha * sum[e];
-          if (p.beta != 0.f)
-            x = x + p.beta * (p.c_f16 ? (float)reinterpret_cast<const _Float16*>(p.c)[o] : reinterpret_cast<const float*>(p.c)[o]);
-          if (p.d_f16) reinterpret_cast<_Float16*>(y_out)[o] = (_Float16)x;
-          else reinterpret_cast<float*>(y_out)[o] = x;
-        }
-        continue;
+    auto finish = [&](auto bias_tag) __attribute__((always_inline)) {
+      constexpr bool BIAS = decltype(bias_tag)::value;
+      u32x4_t bias_raw = {};
+      if constexpr (BIAS) {
+        const int row = (rb_first + round * RT) * kRowBlock + 4 * (tid % SLOTS);
+        bias_raw = load_four(p.bias, p.bias_type, row < p.m ? row : 0);
       }
-      if (p.bias) sum += values_of_four(bias_raw[round], p.bias_type);
-      const size_t o = (size_t)(first_token + token) * p.m + row;
-      if (p.d_f16)
-        *reinterpret_cast<u32x2_any_t*>(y_out + o * 2) = u32x2_t{round_pair<BF16>(sum[0], sum[1]), round_pair<BF16>(sum[2], sum[3])};
-      else
-        *reinterpret_cast<u32x4_any_t*>(y_out + o * 4) = __builtin_bit_cast(u32x4_t, sum);
-    }
+      for (int idx = tid; idx < SLOTS * 16 * CT; idx += 64 * NW) {
+        const int slot = TOKENS ? idx % SLOTS : idx / (16 * CT), token = TOKENS ? idx / SLOTS : idx % (16 * CT);
+        const int at = (token * SLOTS + (slot ^ (token & (SLOTS - 1)))) * 16;
+        float4v_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < NW; ++w) sum += *reinterpret_cast<const float4v_t*>(smem + w * Shape::REGION + at);
+        const int row = (rb_first + round * RT) * kRowBlock + 4 * slot;
+        if (token >= tokens || row >= p.m) continue;
+        if constexpr (!TOKENS) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const size_t o = (size_t)(row + e) * p.n + first_token + token;
+            float x = p.alpha * sum[e];
+            if (p.beta != 0.f)
+              x = x + p.beta * (p.c_f16 ? (float)reinterpret_cast<const _Float16*>(p.c)[o] : reinterpret_cast<const float*>(p.c)[o]);
+            if (p.d_f16) reinterpret_cast<_Float16*>(y_out)[o] = (_Float16)x;
+            else reinterpret_cast<float*>(y_out)[o] = x;
+          }
+          continue;
+        }
+        if constexpr (BIAS) sum += values_of_four(bias_raw, p.bias_type);
+        const size_t o = (size_t)(first_token + token) * p.m + row;
+        if (p.d_f16)
+          *reinterpret_cast<u32x2_any_t*>(y_out + o * 2) = u32x2_t{round_pair<BF16>(sum[0], sum[1]), round_pair<BF16>(sum[2], sum[3])};
+        else
+          *reinterpret_cast<u32x4_any_t*>(y_out + o * 4) = __builtin_bit_cast(u32x4_t, sum);
+      }
+    };
+    if (!TOKENS || __builtin_expect(p.bias == nullptr, 1)) finish(std::false_type{});
+    else finish(std::bool_constant<TOKENS>{});
   }
 }
 

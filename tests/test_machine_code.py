@@ -1,5 +1,6 @@
-"""The compiler counts no wait states in front of an SMFMAC in inline assembly. On the machine code of the built library: no vector
-instruction writes an operand of one of gemm_kernel's SMFMACs less than two wait states in front of it."""
+"""What the source does not give by itself, checked on the machine code of the built library. The compiler counts no wait states in front
+of an SMFMAC in inline assembly: no vector instruction writes an operand of one of gemm_kernel's less than two wait states in front of
+it. Layers without a bias pass none of a bias's code in front of wide_kernel's barrier."""
 import os
 import re
 import subprocess
@@ -65,15 +66,31 @@ def test_the_check_finds_a_write_that_is_too_close():
     assert not too_close([(0, "v_mov_b32_e32", " v4, v5", None), smfmac])
 
 
+def disassembly(source, folder):
+    """functions() of one object of the built library"""
+    llvm = os.path.join(os.path.dirname(native_build.HIPCC), "..", "llvm", "bin")
+    subprocess.run(["ar", "x", native_build.STATIC_LIB, source], cwd=folder, check=True)
+    subprocess.run([os.path.join(llvm, "llvm-objdump"), "--offloading", source], cwd=folder, check=True, stdout=subprocess.DEVNULL)
+    (device,) = [name for name in os.listdir(folder) if name.endswith("gfx950")]
+    return functions(subprocess.run([os.path.join(llvm, "llvm-objdump"), "-d", device], cwd=folder, check=True, capture_output=True,
+                                    text=True).stdout)
+
+
 @pytest.mark.parametrize("source", ["onebit_gemm.o", "onebit_gemm_tokens.o"])
 def test_operands_of_inline_smfmacs_are_written_early_enough(source, tmp_path):
-    llvm = os.path.join(os.path.dirname(native_build.HIPCC), "..", "llvm", "bin")
-    subprocess.run(["ar", "x", native_build.STATIC_LIB, source], cwd=tmp_path, check=True)
-    subprocess.run([os.path.join(llvm, "llvm-objdump"), "--offloading", source], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL)
-    (device,) = [name for name in os.listdir(tmp_path) if name.endswith("gfx950")]
-    text = subprocess.run([os.path.join(llvm, "llvm-objdump"), "-d", device], cwd=tmp_path, check=True, capture_output=True, text=True).stdout
-    kernels = {name: code for name, code in functions(text) if "gemm_kernel" in name}
+    kernels = {name: code for name, code in disassembly(source, tmp_path) if "gemm_kernel" in name}
     assert len(kernels) >= 18 and sum("smfmac" in line[1] for code in kernels.values() for line in code) > 2000
     assert sum(line[3] is not None for code in kernels.values() for line in code) > 100  # branches with their targets
     for name, code in kernels.items():
         assert not too_close(code), name
+
+
+def test_layers_without_a_bias_pass_none_of_its_code_in_front_of_the_barrier(tmp_path):
+    """wide_kernel's token-major form: a bias is read behind the reduction's barrier, by loads that are not taken for LDS reads"""
+    kernels = [(name, code) for name, code in disassembly("onebit_wide_tokens.o", tmp_path) if "wide_kernel" in name]
+    assert len(kernels) >= 24
+    for name, code in kernels:
+        names = [line[1] for line in code]
+        # (the copies of x go to LDS: global_load_lds_...)
+        bias = [i for i, n in enumerate(names) if n.startswith(("flat_load", "global_load_dword", "global_load_ushort"))]
+        assert bias and not any(names[i].startswith("flat") for i in bias) and min(bias) > names.index("s_barrier"), name
