@@ -440,8 +440,11 @@ LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int comput
 // the main kernel at 1.17 of its modelled time). There the line is 1.05; main kernel | wide_kernel, us inside HIP graphs, weights from
 // HBM, random calls that it moves: 22 layers of one whole tile per K range 0.70 to 0.98 of the time, median 0.84 (3520 x 1248 with 206
 // tokens 8.6 | 6.0, 2624 x 7584 with 630 33.9 | 24.0), 44 products 0.51 to 1.03, median 0.79 (1088 x 672 with 416 columns 6.9 | 4.3, 3840 x
-// 7136 with 512 29.0 | 23.0, 1856 x 2400 with 471 17.4 | 10.9), 22 layers where the main kernel splits K 0.70 to 1.02, median 0.85 (704 x
-// 7456 with 985 19.3 | 13.5). Not moved: products where the main kernel splits K (768 x 8192 with 616 16.3 | 17.4) or has
+// 7136 with 512 29.0 | 23.0, 1856 x 2400 with 471 17.4 | 10.9), 135 layers where the main kernel splits K 0.54 to 1.08, median 0.86 (704 x
+// 7456 with 985 19.3 | 13.5). A long K is where both models' errors grow: 38 more such layers, from 60 chunks on in groups of 64 tokens
+// against the 256 x 128 tile and from 71 on in groups of 32 and 64 rows, are 0.91 to 1.14 of the time, mean 1.00 (2048 x 27552 with 846
+// 61.6 | 70.2, 3776 x 26336 with 496 61.9 | 67.0, 1280 x 22304 with 295 24.4 | 26.4; 1344 x 24448 with 345 25.9 | 24.0), and stay, on 64
+// rows but for what is below 0.9 of the modelled time (0.86 to 0.94 but for two of 1.01 and 1.07). Not moved: products where the main kernel splits K (768 x 8192 with 616 16.3 | 17.4) or has
 // the 256 x 128 tile (5440 x 13120 with 168 30.9 | 34.4); and layers in groups of other than 32 or 64 tokens where it splits K, products
 // with a workgroup for every compute unit or 32-row groups, which tests hold on the main kernel, some of which would gain (4096 x 4096
 // with 512 20.3 | 16.9, 512^3 4.8 | 3.6; 1024^3 6.5 | 6.5).
@@ -467,8 +470,13 @@ bool wide_is_faster(const WidePlan& wide, const LaunchPlan& launch, int m, int n
   if (wide.splits == 1 && workgroups <= compute_units) {
     if (plain) {
       if (launch.rows_or_tile != onebit::kTile256x128w8 && launch.splits <= 1 && wide.rows >= 64 && workgroups < compute_units) line = 1.05;
-    } else if (launch.splits <= 1 || wide.tokens == 32 || wide.tokens == 64) {
+    } else if (launch.splits <= 1) {
       line = 1.05;
+    } else if (wide.tokens == 32 || wide.tokens == 64) {
+      const bool main_256x128 = launch.rows_or_tile == onebit::kTile256x128w8;
+      const bool long_k = wide.tokens == 64 ? main_256x128 && chunks >= 60 : wide.rows == 64 && chunks > 70;
+      if (!long_k) line = 1.05;
+      else if (!main_256x128) line = 0.9;
     }
   }
   return wide.us < line * launch.model_us;

@@ -27,6 +27,16 @@ def test_more_rounds_and_split_products_stay_on_the_main_kernel(tokens, m, n, k)
     assert _native.describe_launch(m, n, k, tokens=tokens)["kernel"] == "gemm_kernel"
 
 
+# long K, the main kernel in splits of it: on either side of the lines by chunks, tile and rows of a group
+@pytest.mark.parametrize("m,n,k,wide", [(2048, 846, 27552, False), (3776, 496, 26336, False), (2240, 679, 16224, False),
+                                        (1280, 295, 22304, False), (2048, 1001, 15648, True), (3328, 465, 17440, True),
+                                        (3712, 228, 17984, True), (960, 329, 17696, True)])
+def test_long_k_of_layers(m, n, k, wide):
+    """us on the main kernel | on wide_kernel: 61.6 | 70.2, 61.9 | 67.0, 39.7 | 42.5, 24.4 | 26.4; the others are 0.85 to 0.88 of the time"""
+    plan = _native.describe_launch(m, n, k, tokens=True)
+    assert (plan["kernel"] == "wide_kernel") == wide and (wide or plan["splits"] > 1)
+
+
 @pytest.mark.parametrize("tokens,m,n,k", SPLIT_CALLS)
 def test_split_plans(tokens, m, n, k):
     plan = _native.describe_launch(m, n, k, tokens=tokens)
