@@ -556,9 +556,12 @@ WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b
 // 1760 with 8142 28.5 | 19.5.
 // Odd n on the main kernel, by tile: 512 x 128 and one 256 x 128 or eight-wavefront 128 x 128 per compute unit, where a stage takes long
 // enough: 37 of 37 calls faster, 11008 x 4096 with 1001 56.8 | 52.1, 896 x 6144 with 5995 72.8 | 46.8. 256 x 128, two per compute unit: up
-// to one and a half rounds (4992 x 928 with 3589 37.0 | 33.9; in four 11776 x 6624 with 6257 460 | 478). 64 x 128, and 128 x 128 in two K
-// groups: on a short K (1600 x 896 with 1243 13.4 | 11.7; 13760 x 1888 with 65 13.7 | 16.1) and, but for the first, few rows (704 x 9728
-// with 2889 62.9 | 58.1; 4672 x 8064 with 539 40.5 | 45.2).
+// to one and a half rounds (in four 11776 x 6624 with 6257 460 | 478) of up to 15 chunks (109 calls 0.86 to 1.04 of the time, mean 0.95,
+// 4992 x 928 with 3589 37.0 | 33.9; of 41 longer ones 0.93 to 1.09, mean 1.01, 21312 x 3872 with 969 96.4 | 100.3). 64 x 128, and 128 x 128
+// in two K groups: on a short K, shorter where a copy of few columns is soon made (218 calls 0.68 to 1.00, mean 0.84, 1600 x 896 with 1243
+// 13.4 | 11.7; 13760 x 1888 with 65 13.7 | 16.1, 26112 x 1536 with 85 14.1 | 14.9) and, but for the first, few rows (212 calls 0.63 to
+// 1.07, median 0.83, 704 x 9728 with 2889 62.9 | 58.1; six are more than 3 % slower, where the copy's row length suits the caches: 640 x
+// 7008 with 1977 34.6 | 36.9, with 2197 43.4 | 37.2; 4672 x 8064 with 539 40.5 | 45.2).
 // On wide_kernel: up to 64 columns, where skinny_kernel is the other one (4096 x 4096 with 49 15.0 | 7.5, 28672 x 8192 with 33 47 | 28),
 // and in groups of 16, 32 or 64 of more (512 x 1856 with 555 10.4 | 6.8; in groups of 48 7360 x 4192 with 87 14.7 | 17.0). It would be
 // faster on fewer rows and a longer K too (896 x 1696 with 39 6.7 | 4.4, 2048 x 4832 with 233 14.9 | 11.9): the lines there are where
@@ -570,11 +573,12 @@ bool ragged_in_place(int m, int n, int k, const LaunchPlan& launch, const WidePl
     if (n <= onebit::kSkinnyMaxN) return m > 2048 || (m > 1088 && chunks <= 16);
     return (wide.tokens == 16 || wide.tokens == 32 || wide.tokens == 64) && chunks <= 16;
   }
+  const bool short_k = chunks <= (n <= 224 ? 5 : 7);
   switch (launch.rows_or_tile) {
     case onebit::kTile512x128w8: case onebit::kTile512x128m16: case onebit::kTile256x128w8: case onebit::kTile128x128w8: return true;
-    case onebit::kTile256x128w: return (long)((m + 255) / 256) * ((n + 127) / 128) <= 3L * compute_units;
-    case onebit::kTile64x128: return chunks <= 7;
-    case onebit::kTile128x128k2: case onebit::kTile64x128k2: return chunks <= 7 || m <= 1024;
+    case onebit::kTile256x128w: return chunks <= 15 && (long)((m + 255) / 256) * ((n + 127) / 128) <= 3L * compute_units;
+    case onebit::kTile64x128: return short_k;
+    case onebit::kTile128x128k2: case onebit::kTile64x128k2: return short_k || m <= 1024;
     default: return false;
   }
 }

@@ -44,6 +44,17 @@ def test_which_calls_read_b_where_it_lies():
     assert split["splits"] > 1 and split["pad_b"] is True
 
 
+# an odd n on either side of the lines by chunks, of the 256 x 128, the 128 x 128 tile in two K groups and the 64 x 128 one
+@pytest.mark.parametrize("m,n,k,tile,padded", [(21312, 969, 3872, 4, True), (21312, 969, 3840, 4, False), (26112, 85, 1536, 13, True),
+                                               (26112, 85, 1280, 13, False), (9728, 333, 1696, 13, False), (12480, 73, 1600, 12, True),
+                                               (12480, 83, 1120, 12, False), (6272, 225, 1568, 12, False)])
+def test_odd_counts_are_copied_where_that_is_faster(m, n, k, tile, padded):
+    """us through the copy | in place: 21312 x 3872 with 969 columns 96.4 | 100.3, 26112 x 1536 with 85 14.1 | 14.9, 12480 x 1600 with 73
+    12.5 | 13.7"""
+    plan = _native.describe_launch(m, n, k)
+    assert (plan["tile"], plan["pad_b"]) == (tile, padded)
+
+
 @pytest.fixture
 def hooks():
     def reset():
