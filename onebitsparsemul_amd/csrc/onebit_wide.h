@@ -541,10 +541,14 @@ static hipError_t wide_lds_limit(const void* kern, int lds, std::atomic<bool> (&
 // Whether a workgroup that multiplies `chunks` chunks deals a remainder in parts. us inside HIP graphs, weights from HBM, a chunk to a
 // wavefront | parts: one or two chunks left of two rounds, layers 5760 x 2272 with 54 tokens 5.76 | 5.37, 2752 x 2368 with 62 5.26 | 4.73,
 // 5568 x 2496 with 21 5.20 | 4.63, 10048 x 2464 with 43 8.42 | 7.74, 1472 x 2496 with 128 5.46 | 4.92; of more rounds 28672 x 8448 with
-// 48 23.6 | 23.0, 6720 x 8352 with 17 9.45 | 8.89, 1280 x 10592 with 153 10.4 | 10.0; three chunks of six rounds equal (4096 x 11008
-// with 32 / 500 8.55 | 8.38, 30.8 | 30.6). From five chunks on a part is a chunk, and below a round the calls wait for the host. The build
+// 48 23.6 | 23.0, 6720 x 8352 with 17 9.45 | 8.89, 1280 x 10592 with 153 10.4 | 10.0; three or four chunks of up to five rounds 0.98 of the
+// time in the mean of 111 calls (4096 x 11008 with 32 / 500 8.55 | 8.38, 30.8 | 30.6), of more 1.00 of 71 (three layers of 1536 x 15168 with
+// 20 11.65 | 12.19, eight of 576 x 21120 with 22 17.1 | 17.7): a chunk to a wavefront. From five chunks on a part is a chunk, and below a round the calls wait for the host. The build
 // of the kernel without parts is 1 to 4 % faster where there are none (4096 x 4096 with 48 5.2 | 5.4).
-static bool wide_has_parts(int chunks) { return chunks >= kWideWaves && chunks % kWideWaves >= 1 && chunks % kWideWaves <= 4; }
+static bool wide_has_parts(int chunks) {
+  const int left = chunks % kWideWaves;
+  return chunks >= kWideWaves && left >= 1 && left <= (chunks < 6 * kWideWaves ? 4 : 2);
+}
 
 template <int R, int COPIES, bool TOKENS, bool BF16, bool PARTS, bool RAGGED>
 static hipError_t launch_wide_parts(const SkinnyArgs& args, hipStream_t stream) {

@@ -59,7 +59,8 @@ def test_fp32_activations_take_no_more_than_one_surplus_load(host, rows):
 
 
 @pytest.mark.parametrize("count", [1, 2, 4, 5, 16])
-@pytest.mark.parametrize("k,parts", [(4096, False), (5120, True), (4096 + 1792, False)])  # 16, 20 and 23 chunks of 256
+@pytest.mark.parametrize("k,parts", [(4096, False), (5120, True), (4096 + 1792, False),  # 16, 20 and 23 chunks of 256
+                                     (11776, False), (11008, True), (12800, True), (13056, False)])  # 46, 43, 50 and 51
 def test_groups_take_the_build_with_parts_where_a_remainder_is_dealt_in_parts(host, count, k, parts):
     """The build with parts is 1 to 4 % slower where there are none."""
     problems = (_native.LinearProblem * count)(*[_native.LinearProblem(0x1000, 0x2000, None, 0x3000, 512, k)] * count)
