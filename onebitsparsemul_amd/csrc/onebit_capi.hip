@@ -551,9 +551,10 @@ WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b
 // Whether a ragged B (n % 8 != 0, 16-byte aligned) is read where it lies instead of through a padded copy. The copy costs a launch
 // and a pass, 4 to 5 us and 4 bytes per value at 5.5 TB/s; rows that start at an odd value cost the asynchronous copies 2.4 times the
 // load path (read_as_ragged), which the smaller tiles are short of.
-// Even n: always. us inside HIP graphs, padded copy, or skinny_kernel up to 64 columns | in place: 4096 x 4096 with 34 / 100 / 500 / 2050
-// columns 9.0 | 6.4, 12.2 | 9.7, 25.9 | 21.5, 53.3 | 46.1, 28672 x 8192 with 50 39.8 | 25.4, 11008 x 4096 with 1002 57.9 | 54.2, 704 x
-// 1760 with 8142 28.5 | 19.5.
+// Even n: always but on few rows and a short K up to 32 columns, where skinny_kernel has as little to read: 10 calls 0.94 to 1.03 of
+// its time, with a C 16 of 0.96 to 1.09 (1600 x 320 with 22 3.8 | 4.2; 9600 x 320 with 28 6.7 | 4.7). us inside HIP graphs, padded
+// copy, or skinny_kernel up to 64 columns | in place: 4096 x 4096 with 34 / 100 / 500 / 2050 columns 9.0 | 6.4, 12.2 | 9.7, 25.9 | 21.5,
+// 53.3 | 46.1, 28672 x 8192 with 50 39.8 | 25.4, 11008 x 4096 with 1002 57.9 | 54.2, 704 x 1760 with 8142 28.5 | 19.5.
 // Odd n on the main kernel, by tile: 512 x 128 and one 256 x 128 or eight-wavefront 128 x 128 per compute unit, where a stage takes long
 // enough: 37 of 37 calls faster, 11008 x 4096 with 1001 56.8 | 52.1, 896 x 6144 with 5995 72.8 | 46.8. 256 x 128, two per compute unit: up
 // to one and a half rounds (in four 11776 x 6624 with 6257 460 | 478) of up to 15 chunks (109 calls 0.86 to 1.04 of the time, mean 0.95,
@@ -562,14 +563,17 @@ WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b
 // 13.4 | 11.7; 13760 x 1888 with 65 13.7 | 16.1, 26112 x 1536 with 85 14.1 | 14.9) and, but for the first, few rows (212 calls 0.63 to
 // 1.07, median 0.83, 704 x 9728 with 2889 62.9 | 58.1; six are more than 3 % slower, where the copy's row length suits the caches: 640 x
 // 7008 with 1977 34.6 | 36.9, with 2197 43.4 | 37.2; 4672 x 8064 with 539 40.5 | 45.2).
-// On wide_kernel: up to 64 columns, where skinny_kernel is the other one (4096 x 4096 with 49 15.0 | 7.5, 28672 x 8192 with 33 47 | 28),
-// and in groups of 16, 32 or 64 of more (512 x 1856 with 555 10.4 | 6.8; in groups of 48 7360 x 4192 with 87 14.7 | 17.0). It would be
-// faster on fewer rows and a longer K too (896 x 1696 with 39 6.7 | 4.4, 2048 x 4832 with 233 14.9 | 11.9): the lines there are where
-// the address model in the tests has those calls on skinny_kernel and on the padded copy.
+// Odd n on wide_kernel: up to 64 columns, where skinny_kernel is the other one (4096 x 4096 with 49 15.0 | 7.5, 28672 x 8192 with 33 47 |
+// 28), but not where that splits K and 32-row groups of 24, 40 or 48 columns do not (K of 32 chunks, 4160 x 8192 with 35 14.3 | 18.7,
+// 2368 x 8192 with 17 9.4 | 11.5, all of 46 calls 1.04 to 1.31 of the time); in groups of 16, 32 or 64 of more columns (512 x 1856 with 555
+// 10.4 | 6.8; in groups of 48 7360 x 4192 with 87 14.7 | 17.0). It would be faster on fewer rows and a longer K too (896 x 1696 with 39
+// 6.7 | 4.4, 2048 x 4832 with 233 14.9 | 11.9): the lines there are where the address model in the tests has those calls on
+// skinny_kernel and on the padded copy.
 bool ragged_in_place(int m, int n, int k, const LaunchPlan& launch, const WidePlan& wide, int compute_units) {
-  if (n % 2 == 0) return true;
   const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
+  if (n % 2 == 0) return !launch.split_k_kernel || n > 32 || m > 8192 || chunks > 4;
   if (wide.rows) {
+    if (launch.splits > 1 && wide.splits == 1 && wide.rows == 32 && wide.tokens % 32 != 0) return false;
     if (n <= onebit::kSkinnyMaxN) return m > 2048 || (m > 1088 && chunks <= 16);
     return (wide.tokens == 16 || wide.tokens == 32 || wide.tokens == 64) && chunks <= 16;
   }

@@ -55,6 +55,15 @@ def test_odd_counts_are_copied_where_that_is_faster(m, n, k, tile, padded):
     assert (plan["tile"], plan["pad_b"]) == (tile, padded)
 
 
+@pytest.mark.parametrize("m,n,k,wide", [(1600, 22, 320, False), (8192, 30, 1024, False), (8256, 30, 1024, True), (8192, 30, 1056, True),
+                                        (8192, 34, 1024, True), (4160, 35, 8192, False), (2368, 17, 8192, False), (5376, 45, 8096, False),
+                                        (4096, 35, 7936, True), (4096, 35, 8224, True), (4096, 35, 8192, True), (4096, 49, 8192, True), (4096, 36, 8192, True)])
+def test_up_to_64_columns_go_where_they_are_faster(m, n, k, wide):
+    """us, skinny_kernel | wide_kernel in place: 1600 x 320 with 22 columns and a C 3.8 | 4.2, 4160 x 8192 with 35 14.3 | 18.7, 2368 x 8192
+    with 17 9.4 | 11.5, 5376 x 8096 with 45 15.4 | 18.9"""
+    assert (_native.describe_launch(m, n, k)["kernel"] == "wide_kernel") == wide
+
+
 @pytest.fixture
 def hooks():
     def reset():
