@@ -4,10 +4,11 @@ The kernels' addresses depend on shapes, launch plan and pointers only, never on
 arithmetic can be restated on the CPU (numpy, one array element per lane) and every access asserted to lie inside its
 operand: the prepared weight, B (or its padded copy), C / D, the K-split partial sums. The model restates the index
 arithmetic of onebitsparsemul_amd/csrc/: prepare_kernel and pack_kernel, skinny_kernel with its five B staging modes, wide_kernel
-in both forms (its walk over the grid, the requests a wait names, both SMFMACs' reads of an image), gemm_kernel's asynchronous copy
-pattern, epilogue ranges and the turns of both epilogues through LDS, splitk_reduce_kernel, pad_b_kernel. Where a load
-deliberately reaches past a row (pieces at any alignment, padded copy) the elements that arrive are tracked too. The route of a call
-comes from the library itself (onebit_sparse_describe_call, host-only). It covers the benchmark configurations and the long-K shapes
+in both forms (its walk over the grid, a remainder in parts, the requests a wait names, both SMFMACs' reads of an image), gemm_kernel's
+asynchronous copy pattern, epilogue ranges and the turns of both epilogues through LDS, splitk_reduce_kernel, pad_b_kernel. Where a load
+deliberately reaches past a row (pieces at any alignment, rows read where they lie, padded copy) the elements that arrive are tracked
+too. The route of a call comes from the library itself (onebit_sparse_describe_call, host-only); that the build which the library
+launches is the one modelled here is checked in test_kernel_builds.py. It covers the benchmark configurations and the long-K shapes
 with 33 to 64 columns (8192 x 28672 with n = 40, 48, 64). No GPU is touched.
 """
 import numpy as np
@@ -152,23 +153,29 @@ def check_pack(m, k, size):
 
 
 # ---------------------------------------------------------------------------------------------------------------
-def skinny_variant(n, rows, b_aligned=True, tokens=False, x32=False):
+def token_loads(n, x32=False):
+    """load instructions per image of the token-major form: of two tokens each on 16-bit activations, of one on fp32"""
+    if x32:
+        return n if n <= 2 or 5 <= n <= 8 else n + n % 2
+    return 1 if n <= 2 else 2 if n <= 4 else 4 if n <= 8 else 6 if n <= 12 else 8
+
+
+def skinny_variant(n, rows, chunks, b_aligned=True, tokens=False, x32=False):
+    """(wavefronts, row blocks, image columns, mode, loads per image where the build names them); chunks: of a K split"""
     nw, r = {32: (16, 1), 64: (8, 2), 128: (8, 4)}[rows]
     nc = 64 if n > 32 else 32 if n > 16 else 16
     if nc == 64:
         r = min(r, 2)
     if tokens:
         assert n <= 16
-        mode = "tokens32" if x32 else "tokens"
-    elif n == nc and b_aligned:
-        mode = "full"
-    elif n == 1 and b_aligned:
-        mode = "tokens"   # a k x 1 B is a token-major x of one token
-    elif n in (2, 4) and b_aligned:
-        mode = "run"      # a chunk's 256 rows as one run of 16-byte pieces
-    else:
-        mode = "any"      # 16-byte pieces wherever the rows start
-    return nw, r, nc, mode
+        return nw, r, nc, "tokens32" if x32 else "tokens", token_loads(n, x32)
+    if n == nc and b_aligned:
+        return nw, r, nc, "full", 8
+    if n == 1 and b_aligned:
+        return nw, r, nc, "tokens", 1   # a k x 1 B is a token-major x of one token
+    if 2 <= n <= 8 and b_aligned and not (n == 8 and r != 2 and chunks < (32 if nw == 16 else 16)):
+        return nw, r, nc, "columns", (n + 1) // 2   # four K positions per lane
+    return nw, r, nc, "any", 8          # 16-byte pieces wherever the rows start
 
 
 def drop_halves(values, count):
@@ -223,45 +230,77 @@ def token_image_16(n, k, k_base):
 
 def check_tokens32_image(n, k, k_base):
     """One image of fp32 activations: every load inside x and what it brings where the 16-bit form has it (a token's K in pieces of
-    eight, a piece as two halves)."""
+    eight, a piece as two halves). The loads of a token past the last one fall outside the descriptor."""
     size, image = n * k * 4, token_image_16(n, k, k_base)
     whole, seen = k_base + CHUNK_K <= k, set()
-    for first in (0, 8) if n > 8 else (0,):
-        for i in range(8):
-            token = first + i
-            if token < n:
-                offset = LANE * 16 + token * k * 4
-                if whole:
-                    lane_off, scalar_off = offset, k_base * 4
-                else:
-                    lane_off, scalar_off = np.where(k_base + 4 * LANE < k, offset + k_base * 4, 0xFFFFFF00), 0
-                accessed = lane_off + 16 <= size  # the descriptor's range check looks at the lane offset alone
-                assert lane_off.max() < (1 << 32) and np.array_equal(accessed, lane_off != 0xFFFFFF00)
-                inside(lane_off[accessed] + scalar_off, 16, size, "split-K kernel: fp32 x rows")
-                assert np.array_equal((lane_off + scalar_off)[accessed] // 4, (token * k + k_base + 4 * LANE)[accessed])
-            at = token * 512 + (((LANE >> 1) ^ (token & 15)) << 4) + (LANE & 1) * 8
-            for lane in range(64):
-                assert image[at[lane] // 16 * 16] == (token, k_base + 8 * (lane >> 1)) and at[lane] not in seen
-                seen.add(at[lane])
-    assert len(seen) == (1024 if n > 8 else 512) and max(seen) + 8 <= 8192
+    loads = token_loads(n, x32=True)
+    assert n <= loads <= n + 1
+    for token in range(loads):
+        offset = LANE * 16 + token * k * 4
+        if whole:
+            lane_off, scalar_off = offset, k_base * 4
+        else:
+            lane_off, scalar_off = np.where(k_base + 4 * LANE < k, offset + k_base * 4, 0xFFFFFF00), 0
+        accessed = lane_off + 16 <= size  # the descriptor's range check looks at the lane offset alone
+        assert lane_off.max() < (1 << 32) and np.array_equal(accessed, (lane_off != 0xFFFFFF00) & (token < n))
+        inside(lane_off[accessed] + scalar_off, 16, size, "split-K kernel: fp32 x rows")
+        assert np.array_equal((lane_off + scalar_off)[accessed] // 4, (token * k + k_base + 4 * LANE)[accessed])
+        at = token * 512 + (((LANE >> 1) ^ (token & 15)) << 4) + (LANE & 1) * 8
+        for lane in range(64):
+            assert image[at[lane] // 16 * 16] == (token, k_base + 8 * (lane >> 1)) and at[lane] not in seen
+            seen.add(at[lane])
+    assert len(seen) == 64 * loads and max(seen) + 8 <= 8192
+
+
+def check_columns_image(n, k, k_base):
+    """One image of two to eight columns: a lane loads the 4 n values of four K positions and stores them as n columns of four K values,
+    where the token-major reads look for them. An element of B is tracked by its number, zeros as -1."""
+    size, image = k * n * 2, token_image_16(n, k, k_base)
+    base, at = k_base * n * 2, LANE * n * 8
+    if k_base + CHUNK_K <= k:
+        lane_at, image_at = at, base
+    else:
+        lane_at, image_at = np.where(k_base + 4 * LANE < k, at + base, 0xFFFFFF00), 0
+    halves = np.full((64, 32), -2, dtype=np.int64)  # the lane's v[i]: eight values each
+    loads = [(16 * i, 16) for i in range(n // 2)] + ([(8 * (n - 1), 8)] if n % 2 else [])
+    for i, (start, width) in enumerate(loads):
+        offset = lane_at + start
+        assert offset.max() + width <= (1 << 32)
+        accessed = offset + width <= size  # the descriptor's range check looks at the lane offset alone
+        assert np.array_equal(accessed, lane_at != 0xFFFFFF00)
+        inside(offset[accessed] + image_at, width, size, "split-K kernel: fours of K positions")
+        assert (offset[accessed] % 8 == 0).all()
+        for j in range(width // 2):
+            halves[:, 8 * i + j] = np.where(accessed, (offset + image_at) // 2 + j, -1)
+    seen = set()
+    for c in range(n):
+        where = c * 512 + (((LANE >> 1) ^ (c & 15)) << 4) + (LANE & 1) * 8
+        for lane in range(64):
+            assert image[where[lane] // 16 * 16] == (c, k_base + 8 * (lane >> 1)) and where[lane] not in seen
+            seen.add(where[lane])
+        for j in range(4):  # half j of the lane's eight bytes: K position 4 lane + j
+            row = k_base + 4 * LANE + j
+            assert np.array_equal(halves[:, j * n + c], np.where(row < k, row * n + c, -1))
+    assert len(seen) == 64 * n and max(seen) + 8 <= 8192
 
 
 def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1, x32=False):
-    nw, R, nc, mode = skinny_variant(n, rows, b_aligned, tokens, x32)
     kc_total, rb_total = (k + 255) // 256, m // 32
+    cps = (kc_total + splits - 1) // splits if splits > 1 else kc_total
+    nw, R, nc, mode, loads = skinny_variant(n, rows, cps, b_aligned, tokens, x32)
     img_rows = 8192 // (nc * 2)
     sub = CHUNK_K // img_rows
     prep_size, b_size = prepared_bytes(m, k), k * n * (4 if x32 else 2)
     grid = (rb_total + R - 1) // R
-    prefetch_b = nw <= 8 or mode == "run"
+    few_loads = mode == "columns" or (mode == "tokens" and loads <= 2)
+    prefetch_b = nw <= 8 or few_loads
     images = set()
-    cps = (kc_total + splits - 1) // splits if splits > 1 else kc_total
     splits = (kc_total + cps - 1) // cps
     assert (splits - 1) * cps < kc_total  # the launcher's check: no empty split
     b_fits = b_size < (1 << 32)
     if mode in ("tokens", "tokens32"):
         assert k * 64 * (4 if x32 else 2) < 0xFFFFFF00  # the launcher's check
-    if mode == "run":
+    if mode == "columns":
         assert k * n * 2 < 0xFFFFFF00   # the launcher's check
     for wg, split in [(g, sp) for g in sorted({0, 1, grid // 2, grid - 1} & set(range(grid)))
                       for sp in sorted({0, splits // 2, splits - 1})]:
@@ -269,12 +308,19 @@ def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1
         kc_begin = split * cps
         kc_end = min(kc_begin + cps, kc_total)
         short_k = nw <= 8 and sub == 1 and kc_end - kc_begin <= 2 * nw
+        at_once = nw == 16 and few_loads and nw < kc_end - kc_begin <= 3 * nw
+        rounds = 3 if kc_end - kc_begin > 2 * nw else 2  # of a wavefront that requests everything at once
         for wave in range(nw):
             first = kc_begin + wave
             # --- prepared operand through one descriptor per row block
             chunks = []
             if short_k:
                 chunks += [first, first + nw]
+            elif at_once:
+                chunks += [first + i * nw for i in range(rounds)]
+                # multiplied: all but the last where there is none left for this wavefront
+                multiplied = chunks[:-1] if chunks[-1] >= kc_end else chunks
+                assert multiplied == list(range(first, kc_end, nw))
             else:
                 chunks.append(first)   # requested before the loop (clamped to the last chunk when past it)
                 kc = first
@@ -297,6 +343,8 @@ def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1
                 k_bases.append(first * CHUNK_K)
                 if mode != "any" or first + nw < kc_end:
                     k_bases.append((first + nw) * CHUNK_K)
+            elif at_once:
+                k_bases += [kc * CHUNK_K for kc in chunks]
             else:
                 kc = first
                 if prefetch_b and (nw <= 8 or first < kc_end):
@@ -321,9 +369,8 @@ def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1
                     ppt = img_rows // 8
                     tpi = 64 // ppt
                     piece_lane, token_lane = LANE % ppt, LANE // ppt
-                    for i in range(8):
-                        if tpi * i >= n:
-                            continue  # token groups past the last token are not requested
+                    assert n <= tpi * loads
+                    for i in range(loads):
                         if k_base + img_rows <= k:
                             lane_off = (token_lane * k + 8 * piece_lane) * 2 + i * tpi * k * 2
                             scalar_off = k_base * 2
@@ -337,24 +384,11 @@ def check_skinny(m, n, k, rows, tokens=False, b_aligned=True, d_size=2, splits=1
                         assert np.array_equal(accessed, (token_lane + tpi * i < n) & (lane_off != 0xFFFFFF00))
                         inside(lane_off[accessed] + scalar_off, 16, b_size, "split-K kernel: x rows")
                     continue
-                if mode == "run":
-                    # raw buffer loads of 16-byte pieces q = lane + 64 i < 32 n of the run that starts at k_base * n * 2
-                    pieces = 32 * n
-                    for i in range(2):
-                        if 64 * i >= pieces:
-                            continue
-                        at = LANE * 16 + 1024 * i
-                        if k_base + img_rows <= k:
-                            lane_off = np.where(LANE + 64 * i < pieces, at, 0xFFFFFF00)
-                            scalar_off = k_base * n * 2
-                        else:
-                            valid_bytes = rows_valid * n * 2
-                            assert valid_bytes % 16 == 0  # K is a multiple of 32: no piece straddles the end of B
-                            lane_off = np.where(at + 16 <= valid_bytes, k_base * n * 2 + at, 0xFFFFFF00)
-                            scalar_off = 0
-                        accessed = lane_off + 16 <= b_size  # the descriptor's range check looks at the lane offset alone
-                        assert not accessed[lane_off == 0xFFFFFF00].any()
-                        inside(lane_off[accessed] + scalar_off, 16, b_size, "split-K kernel: B run pieces")
+                if mode == "columns":
+                    if k_base not in images:
+                        images.add(k_base)
+                        if len(images) <= 4 or k - k_base < 2 * CHUNK_K:
+                            check_columns_image(n, k, k_base)
                     continue
                 if mode == "full":
                     if b_fits and k_base + img_rows <= k:
@@ -428,10 +462,26 @@ def check_wide_strips(row_groups, groups):
     assert len(set(rows * groups + cols)) == row_groups * groups
 
 
-def wide_requests(chunks, copies, R, far):
+def wide_has_parts(chunks):
+    """whether the launcher takes the build that deals a remainder in parts"""
+    left = chunks % WIDE_WAVES
+    return chunks >= WIDE_WAVES and 1 <= left <= (4 if chunks < 6 * WIDE_WAVES else 2)
+
+
+def wide_deal(kc_begin, kc_end, wave, parts):
+    """(whole chunks, part) of a wavefront: part = (chunk, first image, images) or None"""
+    left = (kc_end - kc_begin) & (WIDE_WAVES - 1)
+    halvings = 0 if not parts or left > 4 or kc_end - kc_begin < WIDE_WAVES else 1 if left > 2 else 2
+    whole_end = kc_end - left if halvings else kc_end
+    chunk, images = whole_end + (wave >> halvings), 4 >> halvings
+    part = (chunk, (wave & ((1 << halvings) - 1)) * images, images) if parts and chunk < kc_end else None
+    return list(range(kc_begin + wave, whole_end, WIDE_WAVES)), part
+
+
+def wide_requests(chunks, part, copies, R, far):
     """The requests of a wavefront in order, and at each stage's wait how many of the youngest may be outstanding. Returns the prepared
     operands and images in the order of their requests; asserts that a wait leaves nothing outstanding that the stage reads and does not
-    wait for anything younger than its image."""
+    wait for anything younger than its image, and that what is multiplied as image S of an operand is that image's."""
     issued, operands, images = [], [], []
 
     def image(chunk, stage):
@@ -442,6 +492,11 @@ def wide_requests(chunks, copies, R, far):
         operands.append(chunk)
         issued.extend([("operand", chunk, 0)] * (2 * R))  # metadata and signs of each row block
 
+    def wait(allowed, chunk, stage):
+        done = issued[:len(issued) - allowed]
+        assert done.count(("image", chunk, stage)) == copies and done[-1] == ("image", chunk, stage), (chunk, stage)
+        return done
+
     if not chunks:
         return [], []
     operand(chunks[0])
@@ -449,32 +504,63 @@ def wide_requests(chunks, copies, R, far):
     image(chunks[0], 1)
     if far and len(chunks) > 1:
         operand(chunks[1])
+    elif far and part:
+        operand(part[0])
     for at, kc in enumerate(chunks):
-        more = at + 1 < len(chunks)
+        whole = at + 1 < len(chunks)
+        more = whole or part is not None
+        next_kc = chunks[at + 1] if whole else part[0] if part else None
+        next_first = 0 if whole else part[1] if part else None
         for stage in range(4):
             if more:
                 allowed = copies + 2 * R if (stage < 2 if far else stage in (1, 2)) else copies
             else:
                 allowed = copies if stage < 3 else 0
-            done = issued[:len(issued) - allowed]
-            assert done.count(("image", kc, stage)) == copies and done[-1] == ("image", kc, stage), (kc, stage)
+            done = wait(allowed, kc, stage)
             if more and stage == (2 if far else 3):
                 # the next operand's first use: it has arrived, and the compiler's wait for it covers one image more
-                assert done.count(("operand", chunks[at + 1], 0)) == 2 * R and allowed == copies
+                assert done.count(("operand", next_kc, 0)) == 2 * R and allowed == copies
             if stage < 2:
                 image(kc, stage + 2)
-            elif more:
-                image(chunks[at + 1], stage - 2)
+            elif more if stage == 2 else whole or (part is not None and part[2] > 1):
+                image(next_kc, next_first + stage - 2)
             if stage == 0 and more and not far:
-                operand(chunks[at + 1])
+                operand(next_kc)
         if far and at + 2 < len(chunks):
             operand(chunks[at + 2])
+        elif far and whole and part:
+            operand(part[0])
+    if part:
+        chunk, first, count = part
+        # the operand's words, moved to the front: image S is multiplied with metadata word S and sign word S / 2 shifted by 8 (S % 2)
+        meta, sign = [0, 1, 2, 3], [(0, 0), (1, 0)]
+        if first & 2:
+            meta[0], meta[1], sign[0] = meta[2], meta[3], sign[1]
+        if first & 1:
+            meta[0], sign[0] = meta[1], (sign[0][0], sign[0][1] + 8)
+        wait(copies if count > 1 else 0, chunk, first)
+        for stage in range(count):
+            assert meta[stage] == first + stage
+            assert (sign[0][0], sign[0][1] + 8 * stage) == ((first + stage) // 2, 8 * ((first + stage) % 2))
+        if count > 1:
+            wait(0, chunk, first + 1)
     return operands, images
+
+
+def check_moved_piece(moved, row, col, start, n, k):
+    """The pieces of a ragged B that would reach past its end (start: byte where they would begin, of values that are used): of the last
+    row the last one alone, which holds behind the shift the values that it stands for."""
+    assert moved.sum() <= 1
+    for j in np.flatnonzero(moved):
+        shift = (start[j] - (k * n * 2 - 16)) // 2
+        assert row[j] == k - 1 and col[j] // 8 == (n - 1) // 8 and shift == col[j] + 8 - n and 0 < shift < 8
+        values = drop_halves([k * n - 8 + e for e in range(8)], shift)
+        assert all(values[e] == row[j] * n + col[j] + e for e in range(n - col[j]))
 
 
 def check_wide(m, n, k, rows, columns, splits, tokens=False, pad_b=False, d_size=2):
     """wide_kernel, either form: the launcher's checks, the walk over the grid, the prepared operand, the copies of x or B into the ring
-    of two images (K tail, last column group), the fragment reads of an image, the results"""
+    of two images (K tail, last column group, a ragged B where it lies), the fragment reads of an image, the results"""
     R = rows // 32
     ldb = k if tokens else (n + 7) // 8 * 8 if pad_b else n
     copies = (columns + 7) // 8 if tokens else 2 * ((columns + 15) // 16)
@@ -483,7 +569,8 @@ def check_wide(m, n, k, rows, columns, splits, tokens=False, pad_b=False, d_size
     image_bytes = 16 * ct_count * WIDE_IMAGE_K * 2
     lds = WIDE_WAVES * 2 * image_bytes
     assert 1 <= columns <= 64 and columns % 8 == 0 and lds <= 160 * 1024
-    assert (k * 64 * 2 if tokens else ldb * 128) < (1 << 32) and (tokens or (ldb % 8 == 0 and ldb >= n))
+    ragged = not tokens and ldb % 8 != 0  # rows that start anywhere, copied from where they lie
+    assert (k * 64 * 2 if tokens else ldb * 128) < (1 << 32) and (tokens or (ldb == n >= 8 if ragged else ldb >= n))
     # the reduction's tiles take the place of the ring: min(R, 2) row blocks of 32 rows, sixteen columns per tile, fp32
     assert min(R, 2) * 32 * 16 * ct_count * 4 <= 2 * image_bytes
     kc_total, rb_total = (k + 255) // 256, m // 32
@@ -555,11 +642,15 @@ def check_wide(m, n, k, rows, columns, splits, tokens=False, pad_b=False, d_size
         for split in sorted({0, splits // 2, splits - 1}):
             kc_begin = split * cps
             kc_end = min(kc_begin + cps, kc_total)
+            dealt = []
             for wave in range(WIDE_WAVES):
-                mine = list(range(kc_begin + wave, kc_end, WIDE_WAVES))
-                chunks, images = wide_requests(mine, copies, R, far=ct_count == 1 or (ct_count == 3 and R <= 2))
-                assert images == [c * 4 + s for c in mine for s in range(4)]  # every image of its chunks once, in order
-                assert chunks == mine
+                mine, part = wide_deal(kc_begin, kc_end, wave, wide_has_parts(cps))
+                chunks, images = wide_requests(mine, part, copies, R, far=ct_count == 1 or (ct_count == 3 and R <= 2))
+                # every image of its chunks once, in order, and of its part
+                assert images == [c * 4 + s for c in mine for s in range(4)] + (
+                    [part[0] * 4 + part[1] + s for s in range(part[2])] if part else [])
+                assert chunks == mine + ([part[0]] if part else [])
+                dealt += images
                 chunks = chunks or [kc_begin + wave]  # requested, clamped, by a wavefront without a chunk
                 for kc in chunks:
                     for wg in sorted({0, grid // 2, grid - 1}):
@@ -571,10 +662,23 @@ def check_wide(m, n, k, rows, columns, splits, tokens=False, pad_b=False, d_size
                                 inside(rb * kc_total * BLOCK + block + off, width, prep_size, "wide_kernel: prepared operand")
                 for at in images:
                     k0 = at * WIDE_IMAGE_K
-                    for lane_off, k_at, _ in plan:
+                    for i, (lane_off, k_at, col) in enumerate(plan):
                         real = k0 + k_at < k  # the others are copied from the block of zeros
                         assert real.all() or k0 + WIDE_IMAGE_K > k
-                        inside(base0 + k0 * (2 if tokens else ldb * 2) + lane_off[real], 16, b_size, "wide_kernel: copies")
+                        start = base0 + k0 * (2 if tokens else ldb * 2) + lane_off
+                        if ragged and k0 + WIDE_IMAGE_K > k - 1:  # the general path moves pieces past the end of B back
+                            moved = real & (start > b_size - 16) & (first_column + col < n)
+                            check_moved_piece(moved, k0 + k_at, first_column + col, start, n, k)
+                            # mend_image: the one place in the image that is shifted
+                            row, piece = k - 1 - k0, (n - 1 - first_column) // 8
+                            if 0 <= row < WIDE_IMAGE_K and piece < pieces:
+                                slot = row * pieces + (piece ^ int(row_swizzle(np.int64(row), pieces)))
+                                assert np.array_equal(moved, 64 * i + LANE == slot)
+                            else:
+                                assert not moved.any()
+                            start = np.minimum(start, b_size - 16)
+                        inside(start[real], 16, b_size, "wide_kernel: copies")
+            assert sorted(dealt) == list(range(4 * kc_begin, 4 * kc_end))
         # ---- results of the group: rows below m, this group's columns and no other's
         cols = first_column + np.arange(here)
         assert cols.max() < n and (group == col_groups - 1 or here == columns)
@@ -637,22 +741,33 @@ def check_reduce(m, n, splits, d_size):
 
 # ---------------------------------------------------------------------------------------------------------------
 def tile_of_block(b, tiles_m, tiles_n, group_m, xcds=8):
+    """in the kernel's arithmetic: a 32-bit reciprocal in the place of the division by a strip's tiles"""
     total = tiles_m * tiles_n
     per, rem = total // xcds, total % xcds
     x, local = b % xcds, b // xcds
     v = x * per + min(x, rem) + local
-    strip = v // (tiles_m * 4)
-    strip_w = min(tiles_n - strip * 4, 4)
+    reciprocal = ((1 << 32) // (4 * tiles_m) + 1) & 0xFFFFFFFF
+    strip = (v * reciprocal) >> 32
     w = v - strip * 4 * tiles_m
-    group = w // (group_m * strip_w)
+    if w < 0:
+        strip, w = strip - 1, w + 4 * tiles_m
+    strip_w = min(tiles_n - strip * 4, 4)
+    rows = w // group_m
+    group = {4: rows >> 2, 3: rows // 3, 2: rows >> 1, 1: rows}[strip_w]
     group_h = min(tiles_m - group * group_m, group_m)
     u = w - group * group_m * strip_w
-    return group * group_m + u % group_h, strip * 4 + u // group_h
+    column = (u >= group_h) + (u >= 2 * group_h) + (u >= 3 * group_h)
+    return group * group_m + u - column * group_h, strip * 4 + column
+
+
+RAGGED_TILES = (4, 6, 9, 10, 11, 12, 13, 14, 15)  # with a build that copies a ragged B from where it lies
 
 
 def check_gemm(m, n, k, tile, splits, pad_b, tokens=False, b_aligned=True, d_size=2):
     WM, WN, FM, FN, KG = TILES[tile]
-    aligned = tokens or pad_b or (n % 8 == 0 and b_aligned)
+    whole_rows = tokens or pad_b or (n % 8 == 0 and b_aligned)
+    ragged = not whole_rows and b_aligned and n >= 8 and tile in RAGGED_TILES
+    aligned = whole_rows or ragged
     if not aligned:
         WM, WN, FM, FN, KG = 4, 1, 1, 4, 1  # the element-copy variant
     BM, BN, NW = WM * FM * 32, WN * FN * 32, WM * WN * KG
@@ -683,6 +798,14 @@ def check_gemm(m, n, k, tile, splits, pad_b, tokens=False, b_aligned=True, d_siz
         for tile_m, tile_n in corner_tiles:
             n0 = tile_n * BN
             if aligned:
+                k_inside = k - 1 if ragged else k
+                # a chunk of the loop copies the next one's stages; where those lie inside K it has no test for the last row
+                full_end = min(k_inside // CHUNK_K - 1, chunk_end)
+                mended = {chunk_begin * STAGES} | {kc * STAGES + s + 1 for kc in range(max(full_end, chunk_begin), chunk_end) for s in range(STAGES)}
+                last_stage = (k - 1) // STAGE_K
+                if ragged and chunk_begin * STAGES <= last_stage < chunk_end * STAGES:
+                    assert last_stage in mended
+                found = []
                 for wave in range(NW):
                     for i in range(NL):
                         slot = (NW * i + wave) * 64 + LANE
@@ -707,11 +830,18 @@ def check_gemm(m, n, k, tile, splits, pad_b, tokens=False, b_aligned=True, d_siz
                         for stage in range(chunk_begin * STAGES, chunk_end * STAGES + STAGES):
                             next_k0 = stage * STAGE_K
                             base = stage0 + stage * stage_stride
-                            if next_k0 + STAGE_K <= k:
+                            if next_k0 + STAGE_K <= k_inside:
                                 inside(base + b_off, 16, b_size, "main kernel: B stage copy")
                             else:
+                                assert full_end <= chunk_begin or stage // STAGES > full_end
                                 real = next_k0 + copy_row < k  # the other lanes copy from the block of zeros
-                                inside(base + b_off[real], 16, b_size, "main kernel: B stage copy (K tail)")
+                                start = base + b_off
+                                if ragged:  # pieces past the end of B are moved back
+                                    moved = real & (start > b_size - 16) & (n0 + 8 * lc < n)
+                                    check_moved_piece(moved, next_k0 + copy_row, n0 + 8 * lc, start, n, k)
+                                    found += [(stage, slot[j], wave) for j in np.flatnonzero(moved)]
+                                    start = np.minimum(start, b_size - 16)
+                                inside(start[real], 16, b_size, "main kernel: B stage copy (K tail)")
                     rb0 = tile_m * (BM // 32)
                     for j in range(NA):
                         byte = (NW * j + wave) * 1024 + LANE * 16
@@ -722,6 +852,12 @@ def check_gemm(m, n, k, tile, splits, pad_b, tokens=False, b_aligned=True, d_siz
                         # the chunk pointer advances while next_chunk + 1 < chunks: it never passes the last chunk
                         for chunk in range(chunk_begin, min(chunk_end + 1, chunks_total)):
                             inside(chunk * BLOCK + a_off, 16, prep_size, "main kernel: prepared block copy")
+                if ragged:  # mend_stage: the one place that is shifted, in the stage of the last row, by the wavefront that copied it
+                    row, piece = (k - 1) % STAGE_K, (n - 1 - n0) // 8
+                    sw = (((row & 3) << 2) | (((row >> 3) & 1) << 1)) if BN >= 128 else (((row >> 1) & 1) << 2)
+                    copied = chunk_begin * STAGES <= last_stage < (chunk_end + 1) * STAGES
+                    place = row * CH + (piece ^ sw)
+                    assert found == ([(last_stage, place, place // 64 % NW)] if piece < CH and copied else [])
             else:
                 rows_k = np.arange(k)
                 cols = n0 + np.arange(BN)
@@ -805,16 +941,19 @@ def test_padded_copy_addresses(n, k):
     check_pad_b(n, k)
 
 
-@pytest.mark.parametrize("n", [17, 24, 40, 56, 65, 72, 104, 257])
-@pytest.mark.parametrize("m,k", [(64, 32), (192, 1056), (320, 4640), (1024, 8192)])
+@pytest.mark.parametrize("n", [17, 24, 34, 40, 56, 65, 66, 72, 104, 257])
+@pytest.mark.parametrize("m,k", [(64, 32), (192, 1056), (64, 2336), (128, 2848), (320, 4640), (1024, 8192)])
 def test_wide_kernel_addresses(n, m, k):
-    """every width of the column groups the plan can choose, each row group, K splits; B in place and through its padded copy"""
+    """every width of the column groups the plan can choose, each row group, K splits, remainders with and without parts; B in place,
+    a ragged one too, and through its padded copy"""
     for rows in (32, 64, 128):
         for columns in {8 * ((min(n, 16 * width) + 7) // 8) for width in (1, 2, 3, 4)}:
             for splits in (1, 3):
                 splits = min(splits, (k + 255) // 256)
                 check_wide(m, n, k, rows, columns, splits, tokens=True)
-                check_wide(m, n, k, rows, columns, splits, pad_b=n % 8 != 0)
+                check_wide(m, n, k, rows, columns, splits)
+                if n % 8:
+                    check_wide(m, n, k, rows, columns, splits, pad_b=True)
 
 
 @pytest.mark.parametrize("n", [40, 48, 64])
@@ -850,7 +989,8 @@ def test_benchmark_configurations(hooks, m, n, k):
                                              (1088, 63, 2208, True), (2048, 32, 20480, True), (4096, 16, 16384, True),
                                              (576, 200, 352, True), (640, 1001, 160, True), (4096, 1001, 4096, True),
                                              (256, 264, 512, False), (1024, 203, 4128, True), (128, 1000, 4128, True),
-                                             (28672, 40, 512, True), (20480, 64, 1024, True), (4096, 384, 11008, True),
+                                             (4096, 50, 4096, True), (4096, 49, 4096, True), (11008, 1001, 4096, True),
+                                             (4096, 1002, 4096, True), (512, 555, 1856, True), (28672, 40, 512, True), (20480, 64, 1024, True), (4096, 384, 11008, True),
                                              (64, 72, 64, False), (2112, 1032, 64, True), (4096, 16, 16384, True),
                                              (2048, 33, 28672, True), (11008, 32, 28672, True), (192, 5, 12320, True),
                                              (320, 2, 4128, True), (320, 4, 4128, True), (2240, 1, 8224, True),
@@ -886,6 +1026,25 @@ def test_every_tile_configuration(hooks, tile):
         check_call(m, n, k)
         if tile in (4, 6, 9, 10, 11, 12, 13, 14, 15):
             check_call(m, n, k, tokens=True)
+
+
+@pytest.mark.parametrize("tile", RAGGED_TILES)
+@pytest.mark.parametrize("k", [32, 64, 256, 288, 544, 1056, 2272])
+def test_main_kernel_on_rows_that_lie_anywhere(tile, k):
+    for n in (9, 65, 66, 127, 130, 1001):
+        for splits in (1, 2, 3):
+            check_gemm(576, n, k, tile, min(splits, (k + 255) // 256), False)
+
+
+@pytest.mark.parametrize("rows", [32, 64, 128])
+@pytest.mark.parametrize("k", [256, 2048, 4128, 8192, 11008, 12288, 12320])
+def test_few_columns_and_tokens(rows, k):
+    """one chunk per wavefront, two and three (requested at once on sixteen of them) and more, the last of them without a last one"""
+    for splits in (1, 2):
+        splits = min(splits, (k + 255) // 256)
+        for n in range(1, 17):
+            check_skinny(192, n, k, rows, splits=splits)
+            check_skinny(192, n, k, rows, tokens=True, splits=splits)
 
 
 def test_the_model_catches_an_out_of_range_access():
@@ -1092,7 +1251,9 @@ def test_strips_reach_every_workgroup_once(row_groups):
 def test_waits_of_wide_kernel_name_the_requests_behind_an_image(chunks, R):
     for copies in range(1, 9):
         for far in (False, True):
-            wide_requests(list(range(0, 8 * chunks, 8)), copies, R, far)
+            for part in (None, (8 * chunks, 0, 1), (8 * chunks, 1, 1), (8 * chunks, 2, 1), (8 * chunks, 3, 1), (8 * chunks, 0, 2),
+                         (8 * chunks + 1, 2, 2)):
+                wide_requests(list(range(0, 8 * chunks, 8)), part, copies, R, far)
 
 
 @pytest.mark.parametrize("m,k", [(64, 32), (192, 1056), (320, 4640), (1024, 8192), (128, 16416)])

@@ -5,26 +5,18 @@ import pytest
 import torch
 
 from onebitsparsemul_amd import PreparedWeight, _native, dequant_desparse_tile, synthetic
+from test_address_model import check_columns_image
 
 KS = [32, 256, 288, 2080, 4128, 8224, 11008, 12288, 12320]  # 1, 1, 2, 9, 17, 33, 43, 48 and 49 chunks
 
 
 @pytest.mark.parametrize("n", range(2, 9))
 def test_fours_of_k_positions(n):
-    """the loads of a lane stay inside B and the words that it stores are the columns of its four K positions"""
-    for k in (32, 288, 512):
-        for k_base in range(0, (k + 255) // 256 * 256, 256):
-            for lane in range(64):
-                if k_base + 256 > k and k_base + 4 * lane >= k:
-                    continue  # outside the descriptor
-                start = (k_base * n * 2 + lane * 8 * n) // 2
-                assert start % 4 == 0 and start + 4 * n <= k * n
-                words = [(start + 2 * i, start + 2 * i + 1) for i in range(2 * n)]  # n / 2 loads of 16 bytes, one of eight
-                for c in range(n):
-                    for low, high in ((0, 1), (2, 3)):
-                        for row in (low, high):
-                            at = row * n + c
-                            assert words[at // 2][at % 2] == (k_base + 4 * lane + row) * n + c
+    """the loads of a lane stay inside B and what it stores is found by the reads as the columns of its four K positions; K that ends inside
+    an image, at its end and before it"""
+    for k in (32, 96, 256, 288, 512):
+        for k_base in range(0, k + 512, 256):
+            check_columns_image(n, k, k_base)
 
 
 @pytest.fixture

@@ -112,11 +112,18 @@ def test_main_kernel(hooks, tile, m, k):
 @pytest.mark.parametrize("rows", [32, 64, 128])
 def test_wide_kernel(hooks, rows, k):
     _native.set_skinny_rows(rows)
-    m = 2112  # from there on odd counts up to 64 columns are multiplied by wide_kernel
-    a, meta = synthetic.make_weight(m, k, seed=rows + k)
-    prepared = _native.prepare(a.cuda(), meta.cuda(), m, k)
-    dense = dequant_desparse_tile(a, meta).double()
+    weights = {}
+    for m in (2112, 576, 8256):
+        a, meta = synthetic.make_weight(m, k, seed=rows + k)
+        weights[m] = _native.prepare(a.cuda(), meta.cuda(), m, k), dequant_desparse_tile(a, meta).double()
     for n in (17, 18, 20, 22, 23, 26, 34, 39, 42, 46, 50, 57, 58, 62, 63, 66, 98, 114, 127):
+        # rows from which on wide_kernel multiplies these columns; beyond 64 few rows, and not on the shortest K
+        m = 576 if n > 64 else 8256 if n % 2 == 0 and n <= 32 and k <= 1024 else 2112
         for splits in (1, 2) if k >= 1056 else (1,):
+            if n > 64 and k < splits * (1024 if rows == 128 else 256):
+                continue
             _native.set_split_k(splits)
-            check(m, n, k, n + k, prepared, dense)
+            _native.set_pad_b(False)
+            plan = _native.describe_launch(m, n, k)
+            assert (plan["kernel"], plan["rows"], plan["pad_b"]) == ("wide_kernel", rows, False), (m, n, splits)
+            check(m, n, k, n + k, *weights[m])

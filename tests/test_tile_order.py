@@ -3,6 +3,8 @@ import random
 
 import pytest
 
+from test_address_model import tile_of_block
+
 
 def by_division(v, tiles_m, tiles_n, group_m):
     strip = v // (tiles_m * 4)
@@ -15,17 +17,7 @@ def by_division(v, tiles_m, tiles_n, group_m):
 
 
 def as_in_the_kernel(v, tiles_m, tiles_n, group_m):
-    strip = (v * ((1 << 32) // (4 * tiles_m) + 1) & ((1 << 64) - 1)) >> 32
-    w = v - strip * 4 * tiles_m
-    if w < 0:
-        strip, w = strip - 1, w + 4 * tiles_m
-    strip_w = min(tiles_n - strip * 4, 4)
-    rows = w // group_m
-    group = rows >> 2 if strip_w == 4 else rows // 3 if strip_w == 3 else rows >> 1 if strip_w == 2 else rows
-    group_h = min(tiles_m - group * group_m, group_m)
-    u = w - group * group_m * strip_w
-    column = (u >= group_h) + (u >= 2 * group_h) + (u >= 3 * group_h)
-    return group * group_m + u - column * group_h, strip * 4 + column
+    return tile_of_block(v, tiles_m, tiles_n, group_m, xcds=1)  # (one XCD: workgroup v is place v of the list)
 
 
 @pytest.mark.parametrize("group_m", [8, 16])

@@ -4,28 +4,21 @@ import pytest
 import torch
 
 from onebitsparsemul_amd import PreparedWeight, _native, dequant_desparse_tile, synthetic
-
-
-def deal(kc_begin, kc_end, wave):
-    """images (of 64 K values, four a chunk) of a wavefront in order, as the kernel's index arithmetic has them"""
-    left = (kc_end - kc_begin) & 7
-    halvings = 0 if left > 4 or kc_end - kc_begin < 8 else 1 if left > 2 else 2
-    whole_end = kc_end - left if halvings else kc_end
-    images = [4 * kc + s for kc in range(kc_begin + wave, whole_end, 8) for s in range(4)]
-    part_kc, part_images = whole_end + (wave >> halvings), 4 >> halvings
-    if kc_begin + wave < kc_end and halvings and part_kc < kc_end:
-        first = 4 * part_kc + (wave & ((1 << halvings) - 1)) * part_images
-        images += range(first, first + part_images)
-    return images
+from test_address_model import wide_deal, wide_has_parts
 
 
 @pytest.mark.parametrize("kc_begin", [0, 13])
 def test_every_image_goes_to_one_wavefront(kc_begin):
+    """in both builds, for every number of chunks that either may be launched with"""
     for chunks in range(1, 60):
-        dealt = [deal(kc_begin, kc_begin + chunks, wave) for wave in range(8)]
-        assert sorted(i for images in dealt for i in images) == list(range(4 * kc_begin, 4 * (kc_begin + chunks)))
-        if chunks >= 8 and 1 <= chunks % 8 <= 4:
-            assert max(len(images) for images in dealt) == chunks // 8 * 4 + (1 if chunks % 8 <= 2 else 2)
+        for parts in (False, True):
+            dealt = []
+            for wave in range(8):
+                mine, part = wide_deal(kc_begin, kc_begin + chunks, wave, parts)
+                dealt.append([4 * kc + s for kc in mine for s in range(4)] + ([4 * part[0] + part[1] + s for s in range(part[2])] if part else []))
+            assert sorted(i for images in dealt for i in images) == list(range(4 * kc_begin, 4 * (kc_begin + chunks)))
+            if parts and wide_has_parts(chunks):
+                assert max(len(images) for images in dealt) == chunks // 8 * 4 + (1 if chunks % 8 <= 2 else 2)
 
 
 @pytest.fixture
