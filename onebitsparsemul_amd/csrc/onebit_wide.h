@@ -426,12 +426,13 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
   // position s ^ (token % slots)
   constexpr int SLOTS = RT * 8;
   char* const y_out = reinterpret_cast<char*>(p.d) + (size_t)block_y * p.m * p.n * 4;  // a K split's slice: fp32 sums
-  // A thread's results of a round are four rows of several tokens: their bias is requested in front of the sums, once. The calls without
-  // one have a form of their own behind the barrier: what selects or skips a bias in theirs, and whatever stands in front of the barrier
-  // (a wait for the operands that a wavefront without a chunk has requested, too), is 2 to 5 % of a call of few chunks. us, bias of each
-  // row loaded behind the sums | requested in front of the barrier, one form | this: with a bias 28672 x 8192 with 48 tokens 23.5 | 21.9 |
-  // 22.3, 11008 x 4096 with 64 9.27 | 8.64 | 8.81, 16384 x 1024 with 64 5.72 | 5.36 | 5.27; without 16384 x 1024 with 64 5.03 | 5.25 |
-  // 5.01, 11520 x 1312 with 53 5.42 | 5.64 | 5.37, 1152 x 960 with 175 3.14 | 3.27 | 3.16, 18304 x 768 with 64 6.23 | 6.45 | 6.35.
+  // A thread's results of a round are four rows of several tokens: their bias is requested once, in front of the reduction's barrier, which
+  // hides its latency. The calls without one have a barrier and sums of their own: what selects or skips a bias, and whatever stands in
+  // front of the barrier (a wait for the operands that a wavefront without a chunk has requested, too), is 2 to 5 % of a call of few
+  // chunks. us, bias of each row loaded behind the sums | requested in front of one barrier for both | behind it, sums of their own | this:
+  // with a bias 28672 x 8192 with 48 tokens 22.5 | 21.1 | 21.5 | 21.0, 11008 x 4096 with 64 10.2 | 9.6 | 9.8 | 9.7, 16384 x 1024 with 64 5.64 |
+  // 5.35 | 5.22 | 5.07, 16704 x 1056 with 44 9.25 | 8.10 | 8.23 | 8.10; without 16384 x 1024 with 64 4.98 | 5.22 | 4.93 | 4.93, 11520 x
+  // 1312 with 53 5.43 | 5.62 | 5.38 | 5.40, 1152 x 960 with 175 2.96 | 3.02 | 2.97 | 2.95, 18304 x 768 with 64 6.17 | 6.31 | 6.20 | 6.13.
   static_assert(64 * NW % SLOTS == 0, "a thread's rows of a round");
 #pragma unroll
   for (int round = 0; round < R / RT; ++round) {
@@ -459,7 +460,6 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
           *reinterpret_cast<float4v_t*>(region + (token * SLOTS + (slot ^ (token & (SLOTS - 1)))) * 16) =
               acc[2 * (round * RT + rr) + h][ct];
         }
-    __syncthreads();
     auto finish = [&](auto bias_tag) __attribute__((always_inline)) {
       constexpr bool BIAS = decltype(bias_tag)::value;
       u32x4_t bias_raw = {};
@@ -467,6 +467,7 @@ __device__ __forceinline__ void wide_body(const SkinnyArgs& p, const int block_x
         const int row = (rb_first + round * RT) * kRowBlock + 4 * (tid % SLOTS);
         bias_raw = load_four(p.bias, p.bias_type, row < p.m ? row : 0);
       }
+      __syncthreads();
       for (int idx = tid; idx < SLOTS * 16 * CT; idx += 64 * NW) {
         const int slot = TOKENS ? idx % SLOTS : idx / (16 * CT), token = TOKENS ? idx / SLOTS : idx % (16 * CT);
         const int at = (token * SLOTS + (slot ^ (token & (SLOTS - 1)))) * 16;

@@ -86,7 +86,8 @@ def test_operands_of_inline_smfmacs_are_written_early_enough(source, tmp_path):
 
 
 def test_layers_without_a_bias_pass_none_of_its_code_in_front_of_the_barrier(tmp_path):
-    """wide_kernel's token-major form: a bias is read behind the reduction's barrier, by loads that are not taken for LDS reads"""
+    """wide_kernel's token-major form: a bias is read by loads that are not taken for LDS reads, on a path of its own: behind the barrier
+    that calls without one pass, in front of its own, where the reads of the sums do not wait for it"""
     kernels = [(name, code) for name, code in disassembly("onebit_wide_tokens.o", tmp_path) if "wide_kernel" in name]
     assert len(kernels) >= 24
     for name, code in kernels:
@@ -94,3 +95,5 @@ def test_layers_without_a_bias_pass_none_of_its_code_in_front_of_the_barrier(tmp
         # (the copies of x go to LDS: global_load_lds_...)
         bias = [i for i, n in enumerate(names) if n.startswith(("flat_load", "global_load_dword", "global_load_ushort"))]
         assert bias and not any(names[i].startswith("flat") for i in bias) and min(bias) > names.index("s_barrier"), name
+        behind = [n for n in names[min(bias):] if n == "s_barrier" or n.startswith("ds_read")]
+        assert behind[0] == "s_barrier", name
