@@ -444,10 +444,14 @@ LaunchPlan choose_launch(int m, int n, int k, bool b_16_byte_aligned, int comput
 // 7456 with 985 19.3 | 13.5). A long K is where both models' errors grow: 38 more such layers, from 60 chunks on in groups of 64 tokens
 // against the 256 x 128 tile and from 71 on in groups of 32 and 64 rows, are 0.91 to 1.14 of the time, mean 1.00 (2048 x 27552 with 846
 // 61.6 | 70.2, 3776 x 26336 with 496 61.9 | 67.0, 1280 x 22304 with 295 24.4 | 26.4; 1344 x 24448 with 345 25.9 | 24.0), and stay, on 64
-// rows but for what is below 0.9 of the modelled time (0.86 to 0.94 but for two of 1.01 and 1.07). Not moved: products where the main kernel splits K (768 x 8192 with 616 16.3 | 17.4) or has
-// the 256 x 128 tile (5440 x 13120 with 168 30.9 | 34.4); and layers in groups of other than 32 or 64 tokens where it splits K, products
-// with a workgroup for every compute unit or 32-row groups, which tests hold on the main kernel, some of which would gain (4096 x 4096
-// with 512 20.3 | 16.9, 512^3 4.8 | 3.6; 1024^3 6.5 | 6.5).
+// rows but for what is below 0.9 of the modelled time (0.86 to 0.94 but for two of 1.01 and 1.07). Not moved: products where the main
+// kernel splits K (768 x 8192 with 616 16.3 | 17.4) or has the 256 x 128 tile (5440 x 13120 with 168 30.9 | 34.4); and layers in groups
+// of other than 32 or 64 tokens where it splits K, products with a workgroup for every compute unit or 32-row groups. Those lines are not
+// where the measurements end: some calls beyond would gain (4096 x 4096 with 512 20.3 | 16.9, 512^3 4.8 | 3.6; 1024^3 6.5 | 6.5), others
+// not (layers of 1344 x 9216 with 969 and of 640 x 17536 with 676), and they have not been timed over the ranges.
+// The sums are fp32 on both sides and in another order. Their relative error against 64 bits, main kernel | wide_kernel, 1e-8: layers that
+// it splits 704 x 7456 with 985 6.0 | 6.7, 960 x 17696 with 329 7.4 | 8.0, 3328 x 17440 with 465 8.9 | 8.0, 576 x 10848 with 484 7.3 |
+// 6.5; others 5.8 | 5.6 (1216 x 3808 with 1077); products 4.8 | 4.7, 7.7 | 6.9, 2.8 | 2.5.
 // Where wide_kernel splits K the line is 0.96 for layers (0.78 to 1.03, median 0.88) and, with three splits or more, for products (0.73
 // to 1.03, median 0.87; in two splits 0.95 to 1.13, in few rows on 64-row groups up to 1.05).
 // Up to 64 columns the main kernel is the other plan beyond 40960 rows only, where a wavefront of wide_kernel has one short round
@@ -567,8 +571,8 @@ WidePlan plan_wide_product(const LaunchPlan& launch, int m, int n, int k, bool b
 // 28), but not where that splits K and 32-row groups of 24, 40 or 48 columns do not (K of 32 chunks, 4160 x 8192 with 35 14.3 | 18.7,
 // 2368 x 8192 with 17 9.4 | 11.5, all of 46 calls 1.04 to 1.31 of the time); in groups of 16, 32 or 64 of more columns (512 x 1856 with 555
 // 10.4 | 6.8; in groups of 48 7360 x 4192 with 87 14.7 | 17.0). It would be faster on fewer rows and a longer K too (896 x 1696 with 39
-// 6.7 | 4.4, 2048 x 4832 with 233 14.9 | 11.9): the lines there are where the address model in the tests has those calls on
-// skinny_kernel and on the padded copy.
+// 6.7 | 4.4, 2048 x 4832 with 233 14.9 | 11.9): these two lines, by m and chunks, are not where the measurements end, the calls beyond
+// them have not been timed over the ranges.
 bool ragged_in_place(int m, int n, int k, const LaunchPlan& launch, const WidePlan& wide, int compute_units) {
   const int chunks = (k + onebit::kChunkK - 1) / onebit::kChunkK;
   if (n % 2 == 0) return !launch.split_k_kernel || n > 32 || m > 8192 || chunks > 4;

@@ -488,9 +488,12 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
       compute(a_next, std::integral_constant<int, 0>{});
     }
   }
-  // Two or three chunks for each of sixteen wavefronts: as in the short form, everything is requested at once. What a wavefront without
-  // a last chunk requests is zeros that it does not multiply. (us, one chunk after the other | this: 4096 x 11008 with 1 / 4 tokens 6.03 |
-  // 4.97, 6.22 | 5.22; images of four loads are no faster for it, 2048 x 5120 with five tokens 3.65 | 4.11.)
+  // Two or three chunks for each of sixteen wavefronts: as in the short form, everything is requested at once. A wavefront without a
+  // last chunk requests one too, which it does not multiply: past the weight's end the weight's last one and zeros of B, in a K split
+  // the next split's. None stands in a branch, where the compiler could not count it (see kSkinnyBTokens); 17 chunks, 32 requested, are
+  // faster so, too. us, one chunk after the other | this: 4096 x 11008 with 1 / 4 tokens 6.03 | 4.97, 6.22 | 5.22; 4096 x 4352 with 1 / 4 4.04 | 3.66,
+  // 4.23 | 3.94; 33 chunks, 8192 x 8448 6.09 | 5.44, 6.08 | 5.55. Images of four loads are no faster for it, 2048 x 5120 with five tokens
+  // 3.65 | 4.11.
   const bool at_once = NW == 16 && kFewLoads && kc_end - kc_begin > NW && kc_end - kc_begin <= 3 * NW;
   if constexpr (NW == 16 && kFewLoads) {
     auto rounds_at_once = [&](auto rounds_tag) __attribute__((always_inline)) {
