@@ -175,7 +175,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
                                   (lane & 1) * 8) = u32x2_t{round_pair<false>(f[0], f[1]), round_pair<false>(f[2], f[3])};
     }
   };
-  auto load_b = [&](int k_base, u32x4_t (&v)[8]) __attribute__((always_inline)) {
+  auto load_b = [&](int k_base, u32x4_t (&v)[8], bool spaced = false) __attribute__((always_inline)) {
     if constexpr (COLUMNS > 0) {
       // four K positions of a lane: all of them inside K or none (k % 32 == 0); those past its end are sent outside the
       // descriptor, which reads zeros (the launcher checks k n 2 < 2^32)
@@ -202,8 +202,10 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
       const bool inside = k_base + 8 * piece_lane < k_rows;
       const uint32_t lane_at = whole ? token_load_base : token_load_base + (uint32_t)k_base * 2u, image_at = whole ? (uint32_t)k_base * 2u : 0u;
 #pragma unroll
-      for (int i = 0; i < TOKEN_LOADS; ++i)
+      for (int i = 0; i < TOKEN_LOADS; ++i) {
+        if (spaced && i > 0) asm volatile("s_nop 15" ::: "memory");
         v[i] = buffer_load16(b_buffer, whole || inside ? lane_at + i * token_load_step : 0xFFFFFF00u, image_at);
+      }
       return;
     }
     if (MODE == kSkinnyBFull) {
@@ -521,7 +523,11 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs& p, const int block
     }
   }
   // (of sixteen wavefronts a short K leaves some without a chunk: no request for those)
-  if (kPrefetchB && !short_k && !at_once && (NW <= 8 || first < kc_end)) load_b(first * kChunkK, breg);
+  // Eight loads of tokens: the first image's one per sixteen clocks. All at once, behind the requests for the weights, they keep out the
+  // other wavefronts' (us, a branch around each | at once | this: 10624 x 5024 with 16 tokens 6.69 | 6.91 | 6.63, 8256 x 4992 with 14 6.42 |
+  // 6.64 | 6.37, 8768 x 8096 with 15 8.67 | 8.89 | 8.64, 4608 x 20320 with 15 10.7 | 10.9 | 10.6; the loop's spaced as well, no better)
+  constexpr bool kSpaced = TOKENS && !X32 && TOKEN_LOADS == 8 && NW == 8;
+  if (kPrefetchB && !short_k && !at_once && (NW <= 8 || first < kc_end)) load_b(first * kChunkK, breg, kSpaced);
   for (int kc = short_k || at_once ? kc_end : first; kc < kc_end; kc += NW) {
     const int k_base = kc * kChunkK;
     // this wavefront has another chunk after this one (wave-uniform): only then is the next chunk requested; a load
